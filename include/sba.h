@@ -51,6 +51,8 @@ extern "C" {
 
 /* Size of the static device scratch behind sba_fwd_static. */
 #define SBA_STATIC_SCRATCH_BYTES ((size_t)1 << 20)
+/* Largest token stride (in elements) of q, k, v and d_o with SBA_F32: the kernels address 32 rows with 32-bit byte offsets. */
+#define SBA_F32_MAX_TOKEN_STRIDE (1 << 24)
 
 typedef enum SbaDtype { SBA_BF16 = 0, SBA_F32 = 1, SBA_F16 = 2 } SbaDtype;
 
@@ -59,8 +61,9 @@ typedef enum SbaStatus {
   SBA_ERR_NULL = -1,        /* a required pointer is NULL */
   SBA_ERR_DTYPE = -2,       /* dtype not supported by this build */
   SBA_ERR_HEAD_DIM = -3,    /* head_dim outside 1..128 */
-  SBA_ERR_STRIDE = -4,      /* a negative stride (any non-negative head/token/batch stride is accepted; strides and
-                               base pointers that are multiples of 16 bytes select the fast kernels) */
+  SBA_ERR_STRIDE = -4,      /* a negative stride, or with SBA_F32 a token stride beyond SBA_F32_MAX_TOKEN_STRIDE (any other
+                               head/token/batch stride is accepted; strides and base pointers that are multiples of 16 bytes
+                               select the fast kernels) */
   SBA_ERR_ALIGN = -5,       /* a tensor base pointer is not aligned to its element size */
   SBA_ERR_SHAPE = -6,       /* non-positive sizes, total_tokens > 2^30, a negative carry_slots or a flag outside {0, 1} */
   SBA_ERR_WORKSPACE = -7,   /* workspace missing, not 256-byte aligned, or too small (sba_bwd: smaller than one head needs) */
@@ -219,9 +222,8 @@ int sba_fwd_static(const SbaArgs* args);
 
 /*
  * Backward: fills dq, dk, dv from q, k, v, carry, d_o, d_rem (and row_stat when add_remainder is set).
- * 16-bit dtypes: every element of dq, dk, dv is written exactly once (no zero-fill needed, no atomics,
- * no locks; bit-reproducible).  SBA_F32: dk and dv are zero-filled by the call and summed with fp32
- * atomics, so their last bits depend on the execution order.
+ * Every element of dq, dk, dv is written exactly once (no zero-fill needed, no atomics, no locks;
+ * bit-reproducible).
  * Replaces `_compileable_backward` (stickbreaking_attention/sb_varlen/sb_varlen_bwd.py:541-640,
  * custom op "varlen_bwd") and (stickbreaking_attention/sb_attn/sb_bwd.py:207-296, custom op
  * "attn_bwd"), and the `locked_add` accumulation (sb_varlen_bwd.py:11-53).

@@ -16,7 +16,7 @@ int dkv_key_tile(const BwdParams& p);
 bool chain_supported(const BwdParams& p);
 hipError_t launch_bwd_chain(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
 hipError_t launch_fwd_f32(const FwdParams& p, int max_tiles, hipStream_t stream);
-hipError_t launch_bwd_f32(const BwdParams& p, int batches, int64_t tokens, int max_q_tiles, hipStream_t stream);
+hipError_t launch_bwd_f32(const BwdParams& p, int max_q_tiles, int max_k_tiles, hipStream_t stream);
 }  // namespace sba
 
 namespace {
@@ -137,6 +137,12 @@ int check_tensor(const SbaTensor& t, bool required, bool fixed) {
   if (!t.ptr) return required ? SBA_ERR_NULL : SBA_OK;
   if (t.stride_token < 0 || t.stride_head < 0 || (fixed && t.stride_batch < 0)) return SBA_ERR_STRIDE;
   return SBA_OK;
+}
+// The fp32 kernels address 32 rows at a time with 32-bit byte offsets.
+bool f32_stride_ok(const SbaArgs* a) {
+  for (const SbaTensor* t : {&a->q, &a->k, &a->v, &a->d_o})
+    if (t->stride_token > (int64_t)SBA_F32_MAX_TOKEN_STRIDE) return false;
+  return true;
 }
 sba::TensorRef ref(const SbaTensor& t, bool fixed) { return sba::TensorRef{t.ptr, fixed ? t.stride_batch : 0, t.stride_head, t.stride_token}; }
 sba::VectorRef vref(const SbaVector& t, bool fixed) { return sba::VectorRef{t.ptr, fixed ? t.stride_batch : 0, t.stride_head, t.stride_token}; }
@@ -262,6 +268,7 @@ int fwd_on(const SbaArgs* a, char* ws, size_t ws_bytes, bool ws_is_static) {
       (st = check_tensor(a->v, true, fixed)) || (st = check_tensor(a->o, true, fixed)))
     return st;
   if (!a->rem.ptr || !a->row_stat) return SBA_ERR_NULL;
+  if (a->dtype == SBA_F32 && !f32_stride_ok(a)) return SBA_ERR_STRIDE;
   for (const SbaTensor* t : {&a->q, &a->k, &a->v, &a->o})
     if (t->ptr && ((uintptr_t)t->ptr % es)) return SBA_ERR_ALIGN;
   if (ws_is_static && ws_bytes < L.fwd_bytes) return SBA_ERR_TOO_LARGE;
@@ -358,6 +365,7 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last) {
       (st = check_tensor(a->dv, true, fixed)))
     return st;
   if (!a->carry && !a->recompute_carry) return SBA_ERR_NULL;
+  if (a->dtype == SBA_F32 && !f32_stride_ok(a)) return SBA_ERR_STRIDE;
   if (a->add_remainder && !a->row_stat) return SBA_ERR_NULL;
   for (const SbaTensor* t : {&a->q, &a->k, &a->v, &a->d_o, &a->dq, &a->dk, &a->dv})
     if (t->ptr && ((uintptr_t)t->ptr % es)) return SBA_ERR_ALIGN;
@@ -404,13 +412,13 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last) {
     p.chain_sb = fixed ? a->total_tokens : 0;
     p.chain_tile_cap = (int32_t)L.max_k_tiles;
   }
-  // The key-tile list is built for the dK/dV kernel that will run (the fp32 kernels do not use it).
+  // The key-tile list is built for the dK/dV kernel that will run.
   const int key_tile = a->dtype == SBA_F32 ? kBlockK : sba::dkv_key_tile(p);
   if ((st = run_sched(a, ws, L, true, true, key_tile, stream, chain)) != SBA_OK) return st;
   hipEvent_t* ev = (hipEvent_t*)a->trace_events;
   if (ev && first && hipEventRecord(ev[0], stream) != hipSuccess) return SBA_ERR_LAUNCH;
   if (a->dtype == SBA_F32) {
-    if (sba::launch_bwd_f32(p, fixed ? a->num_seqs : 1, a->total_tokens, (int)L.max_q_tiles, stream) != hipSuccess) return SBA_ERR_LAUNCH;
+    if (sba::launch_bwd_f32(p, (int)L.max_q_tiles, (int)L.max_k_tiles, stream) != hipSuccess) return SBA_ERR_LAUNCH;
     if (ev && last && (hipEventRecord(ev[1], stream) != hipSuccess || hipEventRecord(ev[2], stream) != hipSuccess)) return SBA_ERR_LAUNCH;
     return SBA_OK;
   }

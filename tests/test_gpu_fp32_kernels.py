@@ -1,0 +1,31 @@
+"""The fp32 kernels at the edges of their tiles: head_dims around the multiples of 32 (exact and padded variants), lengths
+around the 32-key sub-tiles, the 128-key steps of the four waves and the 128-row query tiles, against the float64 oracle."""
+import pytest
+import torch
+
+from oracle import sb_oracle as orc
+from test_gpu_parity import NAMES, run_varlen, small_case
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("qk_std,attend_current,add_remainder", [(1.0, False, True), (6.0, True, False)])
+@pytest.mark.parametrize("D", [1, 31, 32, 33, 64, 66, 96, 97, 127, 128])
+def test_fp32_tile_edges_against_oracle(gpu_device, D, qk_std, attend_current, add_remainder):
+    lengths = [1, 31, 32, 33, 127, 128, 129, 161, 255, 257, 2, 385]
+    (q, k, v, do, drem), dev, cu = small_case(3, D, lengths, torch.float32, seed=D, qk_std=qk_std)
+    outs = run_varlen(dev[0], dev[1], dev[2], cu.to(gpu_device), lengths, False, attend_current, dev[3], dev[4],
+                      add_remainder=add_remainder)
+    again = run_varlen(dev[0], dev[1], dev[2], cu.to(gpu_device), lengths, False, attend_current, dev[3], dev[4],
+                       add_remainder=add_remainder)
+    d = [t.double() for t in (q, k, v, do, drem)]
+    if add_remainder:
+        d[4] = orc.remainder_drem(d[3], d[4], d[2])
+    ref = orc.varlen_stream(d[0], d[1], d[2], cu, attend_current=attend_current, do=d[3], drem=d[4], dtype=torch.float64)
+    if add_remainder:
+        ref = orc.with_remainder(ref, d[2], d[3])
+    for n, a, b, r in zip(NAMES, outs, again, ref):
+        rel = (a.detach().double().cpu() - r).norm() / r.norm()
+        print(f"D={D} {n}: relative error {rel.item():.2e}", flush=True)
+        assert rel < 1e-5, f"{n}: {rel.item():.2e}"
+        assert torch.equal(a, b), f"{n}: two runs differ"

@@ -1,7 +1,8 @@
-"""ctypes binding of libsba.so (the C ABI declared in include/sba.h).
+"""Bindings of the native code: the torch host layer _sba_torch.so, which eager calls of the operators go through, and the C ABI
+of libsba.so (include/sba.h) by ctypes, which the operators registered for torch.compile, traced calls and tools use.
 
-This is the only place that touches the shared library.  There is no fallback: if the library has not
-been built, or a call reports an error, the operators raise.
+This is the only place that touches the shared libraries.  There is no fallback: if they have not been built, or a call
+reports an error, the operators raise.
 """
 from __future__ import annotations
 
@@ -109,6 +110,36 @@ def lib():
             raise RuntimeError(f"{path}: ABI version {handle.sba_version()} != {ABI_VERSION}")
         _lib = handle
     return _lib
+
+
+_ext = None
+
+
+def ext():
+    """The torch host layer (csrc/sba_torch.cpp), loaded once."""
+    global _ext
+    if _ext is None:
+        lib()
+        try:
+            from . import _sba_torch as module
+        except ImportError as e:
+            raise RuntimeError(f"_sba_torch.so is missing or does not load ({e}): build it with `make -C "
+                               "stickbreaking-attention_amd/csrc`; stick-breaking attention has no fallback path") from e
+        if module.version() != ABI_VERSION:
+            raise RuntimeError(f"_sba_torch.so: ABI version {module.version()} != {ABI_VERSION}")
+        module.set_backward_workspace_limit(BWD_WORKSPACE_LIMIT)
+        _ext = module
+    return _ext
+
+
+def use_ext() -> bool:
+    """Whether a call goes through the torch host layer: eager calls do, unless their kernels are traced."""
+    return TRACE_EVENTS is None and not torch.compiler.is_compiling()
+
+
+def flags() -> int:
+    """The debugging options in force, as the torch host layer takes them."""
+    return (1 if POISON else 0) | (2 if DEBUG_CHECK else 0) | (BACKWARD_KERNELS << 2)
 
 
 def _check(status: int, what: str):
@@ -233,6 +264,8 @@ BWD_WORKSPACE_LIMIT: Optional[int] = None
 def set_backward_workspace_limit(nbytes: Optional[int]):
     global BWD_WORKSPACE_LIMIT
     BWD_WORKSPACE_LIMIT = None if nbytes is None else int(nbytes)
+    if _ext is not None:
+        _ext.set_backward_workspace_limit(BWD_WORKSPACE_LIMIT)
 
 
 def _poison(t: torch.Tensor):

@@ -13,6 +13,8 @@ from .. import _native
 
 
 class StickBreakingAttention(torch.autograd.Function):
+    """The operator under torch.compile; eager calls take the node of the same form in csrc/sba_torch.cpp."""
+
     @staticmethod
     def forward(ctx, q, k, v, inv_temp, attend_current=False, add_remainder=False, save_carry=True):
         need_grad = any(ctx.needs_input_grad[:3]) and (save_carry or q.dtype == torch.float32)   # fp32 always keeps them
@@ -36,10 +38,14 @@ def sb_attn(q, k, v, inv_temp=None, zero_start=True, attend_current=False, add_r
     """``add_remainder=True`` returns ``(o + rem[..., None] * v, rem)`` (what tests/test_attn.py:67 forms from the
     reference's outputs), fused into the kernels' epilogues.  ``save_carry=False`` keeps only q, k, v for the backward,
     which then rebuilds the forward's per-(row, sub-tile) products itself."""
+    if _native.use_ext():
+        return _native.ext().fixed(q, k, v, inv_temp, attend_current, add_remainder, save_carry, _native.flags())
     if inv_temp is None:
         inv_temp = 1 / math.sqrt(q.size(-1))
     return sb_attn_(q, k, v, inv_temp, attend_current=attend_current, add_remainder=add_remainder, save_carry=save_carry)
 
 
 def sb_attn_(q, k, v, inv_temp, attend_current, add_remainder=False, save_carry=True):
+    if _native.use_ext():
+        return _native.ext().fixed(q, k, v, inv_temp, attend_current, add_remainder, save_carry, _native.flags())
     return StickBreakingAttention.apply(q, k, v, inv_temp, attend_current, bool(add_remainder), bool(save_carry))

@@ -15,7 +15,8 @@ from .. import _native
 
 class StickBreakingAttention(torch.autograd.Function):
     """Counterpart of sb_varlen/__init__.py:23-67.  ``cu_seqlens`` here still carries its leading zero when
-    ``zero_start`` was requested; the scheduler kernel skips it instead of the host slicing the tensor."""
+    ``zero_start`` was requested; the scheduler kernel skips it instead of the host slicing the tensor.  The operator under
+    torch.compile; eager calls take the node of the same form in csrc/sba_torch.cpp."""
 
     @staticmethod
     def forward(ctx, q, k, v, cu_seqlens, max_seqlens, inv_temp, attend_current, leading_zero=False, add_remainder=False,
@@ -57,6 +58,9 @@ def sb_attn_varlen(q, k, v, cu_seqlens, max_seqlens=None, inv_temp=None, zero_st
     unchecked and would run out of bounds, sb_varlen_fwd.py:283-288).  Set ``SBA_DEBUG_CHECK=1`` to have every launch
     followed by a read of the scheduler's status word (one synchronisation per call) and a ``ValueError`` that says
     which check failed; never understate ``max_seqlens``."""
+    if _native.use_ext():
+        return _native.ext().varlen(q, k, v, cu_seqlens, int(max_seqlens) if max_seqlens else None, inv_temp, zero_start,
+                                    attend_current, add_remainder, save_carry, _native.flags())
     # The lengths are on the host when cu_seqlens was given as a CPU tensor, or after the one device-to-host copy that
     # stands in for the reference's `assert cu_seqlens[0] == 0` (sb_varlen/__init__.py:71-73, the same host sync).
     # They are then validated there and the carry buffer is sized exactly; a device-only cu_seqlens is validated by
@@ -83,4 +87,7 @@ def sb_attn_varlen(q, k, v, cu_seqlens, max_seqlens=None, inv_temp=None, zero_st
 def sb_attn_varlen_(q, k, v, inv_temp, cu_seqlens, max_seqlens, attend_current):
     """Positional form of sb_varlen/__init__.py:80-81: ``cu_seqlens`` holds sequence ends, no leading zero."""
     cu_seqlens = _native.prepare_cu_seqlens(cu_seqlens, q.device)
+    if _native.use_ext():
+        return _native.ext().varlen(q, k, v, cu_seqlens, int(max_seqlens) if max_seqlens else None, inv_temp, False,
+                                    attend_current, False, True, _native.flags())
     return StickBreakingAttention.apply(q, k, v, cu_seqlens, max_seqlens, inv_temp, attend_current, False)

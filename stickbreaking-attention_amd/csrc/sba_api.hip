@@ -123,15 +123,25 @@ int plan(const SbaArgs* a, Layout* out) {
 
 size_t elem_size(int dtype) { return dtype == SBA_F32 ? 4 : 2; }
 
-// A tensor is usable with 16-byte buffer accesses when its base and its row/head/batch strides are 16-byte
-// multiples and the rows of one sequence span less than 2 GiB (32-bit offsets from the sequence's first row).
-bool vec16(const SbaTensor& t, size_t es, bool fixed, int64_t max_rows) {
-  const int64_t per = 16 / (int64_t)es;
-  if (max_rows * t.stride_token * (int64_t)es >= ((int64_t)1 << 31)) return false;
-  if (((uintptr_t)t.ptr & 15) != 0) return false;
-  if (t.stride_token % per || t.stride_head % per) return false;
-  if (fixed && (t.stride_batch % per)) return false;
-  return true;
+// How the 16-bit kernels may read (and write) the rows of these tensors.  Buffer accesses need the rows of one sequence, and
+// the rows of the last tiles beyond it, within 2 GiB (32-bit offsets from the sequence's first row); the aligned form also
+// base pointers and row/head/batch strides that are 16-byte multiples, and a head_dim that fills the kernel.
+template <size_t N>
+int row_load(const SbaArgs* a, const SbaTensor* const (&tensors)[N]) {
+  if (a->dtype == SBA_F32 || a->head_dim < 8) return sba::kLoadScalar;
+  const bool fixed = a->cu_seqlens == nullptr;
+  const int64_t max_rows = (a->max_seqlen > 0 && a->max_seqlen < a->total_tokens) ? a->max_seqlen : a->total_tokens;
+  int load = a->head_dim == 64 || a->head_dim == 128 ? sba::kLoadAligned : sba::kLoadPadded;
+  for (const SbaTensor* t : tensors) {
+    if (!t->ptr) continue;
+    const int64_t row_bytes = t->stride_token * 2;
+    if (load == sba::kLoadAligned) {
+      if (((uintptr_t)t->ptr & 15) || ((t->stride_token | t->stride_head | (fixed ? t->stride_batch : 0)) & 7)) load = sba::kLoadPadded;
+      else if (max_rows * row_bytes >= ((int64_t)1 << 31)) return sba::kLoadScalar;
+    }
+    if (load == sba::kLoadPadded && (max_rows + 256) * row_bytes >= ((int64_t)1 << 31)) return sba::kLoadScalar;
+  }
+  return load;
 }
 int check_tensor(const SbaTensor& t, bool required, bool fixed) {
   if (!t.ptr) return required ? SBA_ERR_NULL : SBA_OK;
@@ -296,10 +306,7 @@ int fwd_on(const SbaArgs* a, char* ws, size_t ws_bytes, bool ws_is_static) {
   p.add_rem = a->add_remainder ? 1 : 0;
   p.max_tiles = (int32_t)L.max_q_tiles;
   p.total_tokens = a->total_tokens;
-  const int64_t max_rows = (a->max_seqlen > 0 && a->max_seqlen < a->total_tokens) ? a->max_seqlen : a->total_tokens;
-  bool v16 = (a->head_dim % (16 / (int)es)) == 0;
-  for (const SbaTensor* t : {&a->q, &a->k, &a->v, &a->o}) v16 = v16 && vec16(*t, es, fixed, max_rows);
-  p.vec_ok = v16 ? 1 : 0;
+  p.load = row_load(a, {&a->q, &a->k, &a->v, &a->o});
   hipEvent_t* ev = (hipEvent_t*)a->trace_events;
   if (ev && hipEventRecord(ev[0], stream) != hipSuccess) return SBA_ERR_LAUNCH;
   hipError_t e = (a->dtype == SBA_F32) ? sba::launch_fwd_f32(p, (int)L.max_q_tiles, stream)
@@ -330,21 +337,12 @@ int sba_fwd_static(const SbaArgs* a) {
 
 namespace {
 
-// Whether every tensor of the backward allows 16-byte accesses.
-bool bwd_vec_ok(const SbaArgs* a) {
-  const bool fixed = a->cu_seqlens == nullptr;
-  const size_t es = elem_size(a->dtype);
-  const int64_t max_rows = (a->max_seqlen > 0 && a->max_seqlen < a->total_tokens) ? a->max_seqlen : a->total_tokens;
-  bool v16 = (a->head_dim % (16 / (int)es)) == 0;
-  for (const SbaTensor* t : {&a->q, &a->k, &a->v, &a->d_o, &a->dq, &a->dk, &a->dv})
-    if (t->ptr) v16 = v16 && vec16(*t, es, fixed, max_rows);
-  return v16;
-}
+int bwd_load(const SbaArgs* a) { return row_load(a, {&a->q, &a->k, &a->v, &a->d_o, &a->dq, &a->dk, &a->dv}); }
 // Whether one pass over the heads `a` describes runs the one-kernel backward (its buffers are laid out and the
 // tensors and the device allow it).
 bool bwd_is_chained(const SbaArgs* a, const Layout& L) {
   sba::BwdParams p{};
-  p.vec_ok = bwd_vec_ok(a) ? 1 : 0;
+  p.load = bwd_load(a);
   p.head_dim = a->head_dim;
   p.num_heads = a->num_heads;
   p.add_rem = a->add_remainder ? 1 : 0;
@@ -399,7 +397,7 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last) {
   p.head_queue = (int32_t*)(ws + L.off_queue);
   p.max_tiles = (int32_t)L.max_q_tiles;
   p.total_tokens = a->total_tokens;
-  p.vec_ok = bwd_vec_ok(a) ? 1 : 0;
+  p.load = bwd_load(a);
   // One kernel (the key tiles of a sequence hand C and partial dQ to each other) where it applies, else dQ then dK/dV.
   const bool chain = bwd_is_chained(a, L);
   if (chain) {
@@ -438,10 +436,7 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last) {
     f.attend_current = p.attend_current;
     f.max_tiles = (int32_t)L.max_q_tiles;
     f.total_tokens = a->total_tokens;
-    const int64_t max_rows = (a->max_seqlen > 0 && a->max_seqlen < a->total_tokens) ? a->max_seqlen : a->total_tokens;
-    bool fv16 = (a->head_dim % (16 / (int)es)) == 0;
-    for (const SbaTensor* t : {&a->q, &a->k}) fv16 = fv16 && vec16(*t, es, fixed, max_rows);
-    f.vec_ok = fv16 ? 1 : 0;
+    f.load = row_load(a, {&a->q, &a->k});
     if (sba::launch_fwd_carry_only(f, a->dtype == SBA_F16, (int)L.max_q_tiles, stream) != hipSuccess) return SBA_ERR_LAUNCH;
   }
   if (chain) {

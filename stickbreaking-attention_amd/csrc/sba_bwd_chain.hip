@@ -220,7 +220,7 @@ __global__ __launch_bounds__(kChThreads) void bwd_chain_kernel(BwdParams p) {
       const T* kb = (const T*)p.k.ptr + tl.seq_id * p.k.sb + head * p.k.sh + (int64_t)tl.seq_start * p.k.st;
       const T* vb = (const T*)p.v.ptr + tl.seq_id * p.v.sb + head * p.v.sh + (int64_t)tl.seq_start * p.v.st;
       const int key = tl.origin + 32 * g + mfma_row_to_key32(col);
-      const RowSource<T> ks = make_row_source<T, true>(kb, p.k.st, tl.seq_len, DH), vs = make_row_source<T, true>(vb, p.v.st, tl.seq_len, DH);
+      const RowSource<T> ks = make_row_source<T, kLoadAligned>(kb, p.k.st, tl.seq_len, DH), vs = make_row_source<T, kLoadAligned>(vb, p.v.st, tl.seq_len, DH);
 #pragma unroll
       for (int kk = 0; kk < kSteps; kk++) {       // keys beyond the sequence are outside the buffer and read as zero
         kf[kk] = as_vec8<T>(__builtin_amdgcn_raw_buffer_load_b128(ks.rsrc, key * ks.stride_bytes + (16 * kk + 8 * half) * (int)sizeof(T), 0, 0));
@@ -495,7 +495,7 @@ __global__ __launch_bounds__(kChThreads) void bwd_chain_kernel(BwdParams p) {
       const Facts ft = facts_of(tl);
       const T* qb = (const T*)p.q.ptr + tl.seq_id * p.q.sb + head * p.q.sh + (int64_t)tl.seq_start * p.q.st;
       const T* dob = (const T*)p.d_o.ptr + tl.seq_id * p.d_o.sb + head * p.d_o.sh + (int64_t)tl.seq_start * p.d_o.st;
-      const RowSource<T> qs = make_row_source<T, true>(qb, p.q.st, ft.L, DH), ds = make_row_source<T, true>(dob, p.d_o.st, ft.L, DH);
+      const RowSource<T> qs = make_row_source<T, kLoadAligned>(qb, p.q.st, ft.L, DH), ds = make_row_source<T, kLoadAligned>(dob, p.d_o.st, ft.L, DH);
       rq_q = qs.rsrc; rq_do = ds.rsrc; rq_qsb = qs.stride_bytes; rq_dosb = ds.stride_bytes;
       rq_block = ft.nb - 1; rq_left = ft.n;
     };
@@ -575,7 +575,7 @@ __global__ __launch_bounds__(kChThreads) void bwd_chain_kernel(BwdParams p) {
           // K^T of this tile for the dQ contraction, through the wave's scratch: [32 keys][32 columns] at a time,
           // gathered down the keys by the transpose read.  The previous tile's results leave first (same scratch).
           const T* kb = (const T*)p.k.ptr + tile.seq_id * p.k.sb + head * p.k.sh + f.tok0 * p.k.st;
-          const RowSource<T> ksrc = make_row_source<T, true>(kb, p.k.st, L, DH);
+          const RowSource<T> ksrc = make_row_source<T, kLoadAligned>(kb, p.k.st, L, DH);
           u32x4 kr[8];
 #pragma unroll
           for (int q = 0; q < 4; q++)
@@ -790,7 +790,7 @@ static hipError_t launch_chain_t(const BwdParams& p_in, int max_tiles, hipStream
 bool chain_supported(const BwdParams& p) {
   int dev = 0, cus = 0;
   if (device_cus(&dev, &cus) != hipSuccess) return false;
-  return p.vec_ok && p.head_dim == 128 && (p.num_heads & 7) == 0 && cus / p.num_heads >= 1 && !p.add_rem;
+  return p.load == kLoadAligned && p.head_dim == 128 && (p.num_heads & 7) == 0 && cus / p.num_heads >= 1 && !p.add_rem;
 }
 
 hipError_t launch_bwd_chain(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream) {

@@ -30,8 +30,9 @@ template <int DH> struct DkvLds {
   static constexpr int kElems = kDz + kBlockQ * kPStride;
 };
 
-template <typename T, int DH, bool kFast>
+template <typename T, int DH>
 __global__ __launch_bounds__(kThreads) void bwd_dkv_kernel(BwdParams p) {
+  constexpr int kLoad = kLoadScalar;
   typedef typename Elem<T>::vec8 vec8;
   typedef DkvLds<DH> Lds;
   constexpr int kRowStride = Lds::kRowStride, kPStride = Lds::kPStride;
@@ -76,8 +77,8 @@ __global__ __launch_bounds__(kThreads) void bwd_dkv_kernel(BwdParams p) {
     const int key = j0 + mfma_row_to_key(mt, col);
 #pragma unroll
     for (int kk = 0; kk < kSteps; kk++) {
-      kf[mt][kk] = as_vec8<T>(load_row8<T, kFast>(kb + (int64_t)key * p.k.st, 16 * kk + 8 * half, D, key < L));
-      vf[mt][kk] = as_vec8<T>(load_row8<T, kFast>(vb + (int64_t)key * p.v.st, 16 * kk + 8 * half, D, key < L));
+      kf[mt][kk] = as_vec8<T>(load_row8<T, kLoad>(kb + (int64_t)key * p.k.st, 16 * kk + 8 * half, D, key < L));
+      vf[mt][kk] = as_vec8<T>(load_row8<T, kLoad>(vb + (int64_t)key * p.v.st, 16 * kk + 8 * half, D, key < L));
     }
   }
 
@@ -89,8 +90,8 @@ __global__ __launch_bounds__(kThreads) void bwd_dkv_kernel(BwdParams p) {
   const float* carry = p.carry + seq0 + carry_offset(2 * jt + 1, n_qt);      // + row
   const float* prefix = p.prefix + seq0 + carry_offset(2 * jt, n_qt);
 
-  const RowSource<T> qsrc = make_row_source<T, kFast>(qb, p.q.st, L, D), dosrc = make_row_source<T, kFast>(dob, p.d_o.st, L, D);
-  TileCopy<T, DH, kBlockQ, kFast> cq, cdo;
+  const RowSource<T> qsrc = make_row_source<T, kLoad>(qb, p.q.st, L, D), dosrc = make_row_source<T, kLoad>(dob, p.d_o.st, L, D);
+  TileCopy<T, DH, kBlockQ, kLoad> cq, cdo;
   if (qt_begin < n_qt) {
     cq.load(qsrc, qt_begin * kBlockQ);
     cdo.load(dosrc, qt_begin * kBlockQ);
@@ -189,6 +190,14 @@ __global__ __launch_bounds__(kThreads) void bwd_dkv_kernel(BwdParams p) {
   }
 }
 
+// Results in 16-byte stores where rows are 16-byte aligned and full, element by element otherwise.
+template <typename T, int kLoad>
+__device__ __forceinline__ void store_result_tile(const RowSink<T>& sink, const f32x16& acc, float scale, int row0, int col0, int half,
+                                                  int col, int lane, T* scratch, int d) {
+  if (kLoad == kLoadPadded) store_acc_tile<T>(sink, acc, scale, row0, col0, half, col, d);
+  else store_acc_tile_wide<T>(sink, acc, scale, row0, col0, half, col, lane, scratch);
+}
+
 // ---------------------------------------------------------------------------------------------------------
 // Fast path, producer / consumer waves (runs head_dim 64; head_dim 128 runs the software-pipelined kernel below).
 //
@@ -212,7 +221,7 @@ template <int DH> struct Dkv3Lds {
   static constexpr int kElems = kP + 4 * kPTile;
 };
 
-template <typename T, int DH>
+template <typename T, int DH, int kLoad>
 __global__ __launch_bounds__(kDkv3Threads) void bwd_dkv3_kernel(BwdParams p) {
   typedef typename Elem<T>::vec8 vec8;
   typedef Dkv3Lds<DH> Lds;
@@ -229,7 +238,7 @@ __global__ __launch_bounds__(kDkv3Threads) void bwd_dkv3_kernel(BwdParams p) {
   const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) & 3;
   const bool producer = threadIdx.x < 256;
   const int half = lane >> 5, col = lane & 31;
-  const int ac = p.attend_current;
+  const int ac = p.attend_current, D = kLoad == kLoadPadded ? p.head_dim : DH;
   // The `wph` workgroups of a head start with the head's first wph tiles (the list is heaviest first) and then take
   // the next tile from a per-head cursor whenever they finish one, so the load balances itself.  The cursor is read
   // a tile ahead: thread 0 takes the slot after next before a tile's start-up barrier and publishes it through LDS.
@@ -251,14 +260,14 @@ __global__ __launch_bounds__(kDkv3Threads) void bwd_dkv3_kernel(BwdParams p) {
   // The tile record of the next round is fetched a round ahead; the consumers also request the first query rows
   // of the next tile before they store the results of the current one.
   Tile next_tile = p.k_tiles[w < n_tiles ? w : 0];
-  TileCopy<T, DH, kDkvRows, true> cq, cdo;                   // staging registers (consumer waves)
+  TileCopy<T, DH, kDkvRows, kLoad> cq, cdo;                   // staging registers (consumer waves)
   auto stage_first = [&](const Tile& tl) {
     const T* qb = (const T*)p.q.ptr + tl.seq_id * p.q.sb + head * p.q.sh + (int64_t)tl.seq_start * p.q.st;
     const T* dob = (const T*)p.d_o.ptr + tl.seq_id * p.d_o.sb + head * p.d_o.sh + (int64_t)tl.seq_start * p.d_o.st;
     const int rb = first_row_block(tl);
     if (rb < tl.seq_len) {
-      cq.load(make_row_source<T, true>(qb, p.q.st, tl.seq_len, DH), rb);
-      cdo.load(make_row_source<T, true>(dob, p.d_o.st, tl.seq_len, DH), rb);
+      cq.load(make_row_source<T, kLoad>(qb, p.q.st, tl.seq_len, D), rb);
+      cdo.load(make_row_source<T, kLoad>(dob, p.d_o.st, tl.seq_len, D), rb);
     }
   };
   // Producer waves: the K and V operands of the next tile's 32-key sub-tile are requested a tile ahead as well.
@@ -267,12 +276,9 @@ __global__ __launch_bounds__(kDkv3Threads) void bwd_dkv3_kernel(BwdParams p) {
     const T* kb = (const T*)p.k.ptr + tl.seq_id * p.k.sb + head * p.k.sh + (int64_t)tl.seq_start * p.k.st;
     const T* vb = (const T*)p.v.ptr + tl.seq_id * p.v.sb + head * p.v.sh + (int64_t)tl.seq_start * p.v.st;
     const int key = tl.origin + 32 * (wave & 1) + mfma_row_to_key32(col);
-    const RowSource<T> ks = make_row_source<T, true>(kb, p.k.st, tl.seq_len, DH), vs = make_row_source<T, true>(vb, p.v.st, tl.seq_len, DH);
-#pragma unroll
-    for (int kk = 0; kk < kSteps; kk++) {       // keys beyond the sequence are outside the buffer and read as zero
-      kf_next[kk] = as_vec8<T>(__builtin_amdgcn_raw_buffer_load_b128(ks.rsrc, key * ks.stride_bytes + (16 * kk + 8 * half) * (int)sizeof(T), 0, 0));
-      vf_next[kk] = as_vec8<T>(__builtin_amdgcn_raw_buffer_load_b128(vs.rsrc, key * vs.stride_bytes + (16 * kk + 8 * half) * (int)sizeof(T), 0, 0));
-    }
+    const RowSource<T> ks = make_row_source<T, kLoad>(kb, p.k.st, tl.seq_len, D), vs = make_row_source<T, kLoad>(vb, p.v.st, tl.seq_len, D);
+    request_operand<T, kLoad>(kf_next, ks, key, half);
+    request_operand<T, kLoad>(vf_next, vs, key, half);
   };
   // Each role runs its own walk over the same rounds (same tiles, same number of barriers), so that what one role
   // carries from tile to tile does not occupy registers in the other role's code.
@@ -305,6 +311,8 @@ __global__ __launch_bounds__(kDkv3Threads) void bwd_dkv3_kernel(BwdParams p) {
     vec8 kf[kSteps], vf[kSteps];
 #pragma unroll
     for (int kk = 0; kk < kSteps; kk++) { kf[kk] = kf_next[kk]; vf[kk] = vf_next[kk]; }
+    place_operand<T, kLoad>(kf, D, half);
+    place_operand<T, kLoad>(vf, D, half);
     // Per-row scalars (drem, product above the sub-tile, C below it), fetched one step ahead.
     const float* drem_eff = p.drem_eff + tile.seq_id * p.drem_sb + head * p.stat_sh + tok0;
     float n_drem = 0.f, n_prod = 1.f, n_prefix = 0.f;
@@ -408,24 +416,24 @@ __global__ __launch_bounds__(kDkv3Threads) void bwd_dkv3_kernel(BwdParams p) {
 #pragma unroll
           for (int r = 0; r < 16; r++) {
             const int key = tl_j0 + 32 * (mt0 + mt) + 8 * (r >> 2) + 4 * half + (r & 3);
-            if (key < tl_len)
+            if (key < tl_len && d < D)
               dvacc[mt][r] += fast_exp2(p.row_stat[tl.seq_id * p.stat_sb + head * p.stat_sh + tl_tok0 + key]) *
                               (float)dob[(int64_t)key * p.d_o.st + d];
           }
       }
-      const RowSink<T> dk_sink = make_row_sink<T>(dkb, p.dk.st, tl_len, DH), dv_sink = make_row_sink<T>(dvb, p.dv.st, tl_len, DH);
+      const RowSink<T> dk_sink = make_row_sink<T>(dkb, p.dk.st, tl_len, D), dv_sink = make_row_sink<T>(dvb, p.dv.st, tl_len, D);
       // Wave-private transposition scratch in the third Q/dO buffer: free during a tile's first step and after the
       // last one.
       T* scratch = lds + Lds::kQ + 4 * Lds::kQdoTile + wave * (32 * lds_stride<32>());
 #pragma unroll
       for (int mt = 0; mt < kMT; mt++) {
-        store_acc_tile_wide<T>(dk_sink, dkacc[mt], p.logit_scale, tl_j0 + 32 * (mt0 + mt), 32 * ct, half, col, lane, scratch);
-        store_acc_tile_wide<T>(dv_sink, dvacc[mt], 1.f, tl_j0 + 32 * (mt0 + mt), 32 * ct, half, col, lane, scratch);
+        store_result_tile<T, kLoad>(dk_sink, dkacc[mt], p.logit_scale, tl_j0 + 32 * (mt0 + mt), 32 * ct, half, col, lane, scratch, D);
+        store_result_tile<T, kLoad>(dv_sink, dvacc[mt], 1.f, tl_j0 + 32 * (mt0 + mt), 32 * ct, half, col, lane, scratch, D);
       }
     };
   for (int slot = w; slot < n_tiles;) {
   const Tile tile = next_tile;
-  const int L = tile.seq_len, j0 = tile.origin, ac = p.attend_current, D = DH;
+  const int L = tile.seq_len, j0 = tile.origin;
   const int64_t tok0 = tile.seq_start;
 
   const int first_row = j0 + 1 - ac;                         // first row that sees key j0
@@ -437,7 +445,7 @@ __global__ __launch_bounds__(kDkv3Threads) void bwd_dkv3_kernel(BwdParams p) {
     // the barrier that ends a step is the only point that waits for those loads.
     [[maybe_unused]] const T* qb = (const T*)p.q.ptr + tile.seq_id * p.q.sb + head * p.q.sh + tok0 * p.q.st;
     [[maybe_unused]] const T* dob = (const T*)p.d_o.ptr + tile.seq_id * p.d_o.sb + head * p.d_o.sh + tok0 * p.d_o.st;
-    const RowSource<T> qsrc = make_row_source<T, true>(qb, p.q.st, L, D), dosrc = make_row_source<T, true>(dob, p.d_o.st, L, D);
+    const RowSource<T> qsrc = make_row_source<T, kLoad>(qb, p.q.st, L, D), dosrc = make_row_source<T, kLoad>(dob, p.d_o.st, L, D);
     if (n_steps > 0) {                                       // rows of step 0 were requested a tile ago
       cq.store(lds + Lds::kQ);
       cdo.store(lds + Lds::kQ + Lds::kQdoTile);
@@ -503,7 +511,7 @@ __global__ __launch_bounds__(kDkv3Threads) void bwd_dkv3_kernel(BwdParams p) {
   }
 }
 
-template <typename T, int DH>
+template <typename T, int DH, int kLoad>
 static hipError_t launch_dkv3(const BwdParams& p_in, int max_tiles, hipStream_t stream) {
   const size_t lds_bytes = (size_t)Dkv3Lds<DH>::kElems * sizeof(T) + 256;      // + the published queue slot
   // The tile set exceeds the default 64 KB dynamic-LDS cap: the limit is raised once per device.
@@ -511,14 +519,14 @@ static hipError_t launch_dkv3(const BwdParams& p_in, int max_tiles, hipStream_t 
   int dev = 0, cus = 0;
   hipError_t e = device_cus(&dev, &cus);
   if (e != hipSuccess) return e;
-  if ((e = raise_lds_limit(&bwd_dkv3_kernel<T, DH>, lds_done, dev, lds_bytes)) != hipSuccess) return e;
+  if ((e = raise_lds_limit(&bwd_dkv3_kernel<T, DH, kLoad>, lds_done, dev, lds_bytes)) != hipSuccess) return e;
   BwdParams p = p_in;
   // One workgroup per CU: the same number of workgroups for every head, and with a head count that is a multiple of
   // 8 the workgroups of a head share an XCD (workgroup ids are dealt round-robin to the 8 XCDs).
   p.wgs_per_head = cus / p.num_heads > 0 ? cus / p.num_heads : 1;
   if (p.wgs_per_head > max_tiles) p.wgs_per_head = max_tiles;
   const dim3 grid((unsigned)(p.wgs_per_head * p.num_heads)), block(kDkv3Threads);
-  hipLaunchKernelGGL((bwd_dkv3_kernel<T, DH>), grid, block, lds_bytes, stream, p);
+  hipLaunchKernelGGL((bwd_dkv3_kernel<T, DH, kLoad>), grid, block, lds_bytes, stream, p);
   return hipGetLastError();
 }
 
@@ -553,7 +561,7 @@ template <int DH> struct Dkv4Lds {
 };
 
 
-template <typename T, int DH>
+template <typename T, int DH, int kLoad>
 __global__ __launch_bounds__(kDkv4Threads) void bwd_dkv4_kernel(BwdParams p) {
   typedef typename Elem<T>::vec8 vec8;
   typedef Dkv4Lds<DH> Lds;
@@ -568,7 +576,7 @@ __global__ __launch_bounds__(kDkv4Threads) void bwd_dkv4_kernel(BwdParams p) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
   const bool producer = threadIdx.x < 256;
   const int half = lane >> 5, col = lane & 31;
-  const int ac = p.attend_current;
+  const int ac = p.attend_current, D = kLoad == kLoadPadded ? p.head_dim : DH;
   const int wph = p.wgs_per_head;
   int head, w;
   if ((p.num_heads & 7) == 0) {
@@ -595,12 +603,9 @@ __global__ __launch_bounds__(kDkv4Threads) void bwd_dkv4_kernel(BwdParams p) {
       const T* kb = (const T*)p.k.ptr + tl.seq_id * p.k.sb + head * p.k.sh + (int64_t)tl.seq_start * p.k.st;
       const T* vb = (const T*)p.v.ptr + tl.seq_id * p.v.sb + head * p.v.sh + (int64_t)tl.seq_start * p.v.st;
       const int key = tl.origin + 32 * g + mfma_row_to_key32(col);
-      const RowSource<T> ks = make_row_source<T, true>(kb, p.k.st, tl.seq_len, DH), vs = make_row_source<T, true>(vb, p.v.st, tl.seq_len, DH);
-#pragma unroll
-      for (int kk = 0; kk < kSteps; kk++) {       // keys beyond the sequence are outside the buffer and read as zero
-        kf[kk] = as_vec8<T>(__builtin_amdgcn_raw_buffer_load_b128(ks.rsrc, key * ks.stride_bytes + (16 * kk + 8 * half) * (int)sizeof(T), 0, 0));
-        vf[kk] = as_vec8<T>(__builtin_amdgcn_raw_buffer_load_b128(vs.rsrc, key * vs.stride_bytes + (16 * kk + 8 * half) * (int)sizeof(T), 0, 0));
-      }
+      const RowSource<T> ks = make_row_source<T, kLoad>(kb, p.k.st, tl.seq_len, D), vs = make_row_source<T, kLoad>(vb, p.v.st, tl.seq_len, D);
+      request_operand<T, kLoad>(kf, ks, key, half);
+      request_operand<T, kLoad>(vf, vs, key, half);
     };
     if (w < n_tiles) load_kv(next_tile);
     for (int slot = w; slot < n_tiles;) {
@@ -740,6 +745,8 @@ __global__ __launch_bounds__(kDkv4Threads) void bwd_dkv4_kernel(BwdParams p) {
         }
         if (t == n_steps - 1 && have_next) load_kv(next_tile);   // kf / vf have fed their last MFMAs of this tile
       };
+      place_operand<T, kLoad>(kf, D, half);
+      place_operand<T, kLoad>(vf, D, half);
       f32x16 s_a, dp_a, s_b, dp_b;
       if (n_steps > 0) scores(0, s_a, dp_a);
       else if (have_next) load_kv(next_tile);
@@ -759,11 +766,11 @@ __global__ __launch_bounds__(kDkv4Threads) void bwd_dkv4_kernel(BwdParams p) {
     f32x16 acc[4][kCT];
     // Two sets of staging registers, used alternately: a step's rows are requested two steps before they are
     // written to LDS (a step is shorter than a global load).
-    TileCopy<T, DH, kRows, true> cq[2], cdo[2];
+    TileCopy<T, DH, kRows, kLoad> cq[2], cdo[2];
     auto stage_first = [&](const Tile& tl) {                 // rows of steps 0 and 1 of a tile
       const T* qb = (const T*)p.q.ptr + tl.seq_id * p.q.sb + head * p.q.sh + (int64_t)tl.seq_start * p.q.st;
       const T* dob = (const T*)p.d_o.ptr + tl.seq_id * p.d_o.sb + head * p.d_o.sh + (int64_t)tl.seq_start * p.d_o.st;
-      const RowSource<T> qs = make_row_source<T, true>(qb, p.q.st, tl.seq_len, DH), ds = make_row_source<T, true>(dob, p.d_o.st, tl.seq_len, DH);
+      const RowSource<T> qs = make_row_source<T, kLoad>(qb, p.q.st, tl.seq_len, D), ds = make_row_source<T, kLoad>(dob, p.d_o.st, tl.seq_len, D);
       const int rb = first_row_block(tl);
 #pragma unroll
       for (int i = 0; i < 2; i++)                            // rows beyond the sequence read as zero
@@ -796,18 +803,19 @@ __global__ __launch_bounds__(kDkv4Threads) void bwd_dkv4_kernel(BwdParams p) {
               const float rem = fast_exp2(p.row_stat[tl.seq_id * p.stat_sb + head * p.stat_sh + tl_tok0 + key]);
 #pragma unroll
               for (int n = 0; n < kCT; n++)
-                acc[m][n][r] += rem * (float)dob[(int64_t)key * p.d_o.st + 32 * (kCT * cp + n) + col];
+                if (32 * (kCT * cp + n) + col < D)
+                  acc[m][n][r] += rem * (float)dob[(int64_t)key * p.d_o.st + 32 * (kCT * cp + n) + col];
             }
           }
       }
-      const RowSink<T> sink = make_row_sink<T>(outb, out_st, tl_len, DH);
+      const RowSink<T> sink = make_row_sink<T>(outb, out_st, tl_len, D);
       const float scale = out ? p.logit_scale : 1.f;
       T* scratch = lds + Lds::kScratch + wave * (32 * lds_stride<32>());
 #pragma unroll
       for (int m = 0; m < 4; m++)
 #pragma unroll
         for (int n = 0; n < kCT; n++)
-          store_acc_tile_wide<T>(sink, acc[m][n], scale, tl_j0 + 32 * m, 32 * (kCT * cp + n), half, col, lane, scratch);
+          store_result_tile<T, kLoad>(sink, acc[m][n], scale, tl_j0 + 32 * m, 32 * (kCT * cp + n), half, col, lane, scratch, D);
     };
     for (int slot = w; slot < n_tiles;) {
       const Tile tile = next_tile;
@@ -818,7 +826,7 @@ __global__ __launch_bounds__(kDkv4Threads) void bwd_dkv4_kernel(BwdParams p) {
       const int n_steps = (L - row_begin + kRows - 1) / kRows;
       const T* qb = (const T*)p.q.ptr + tile.seq_id * p.q.sb + head * p.q.sh + tok0 * p.q.st;
       const T* dob = (const T*)p.d_o.ptr + tile.seq_id * p.d_o.sb + head * p.d_o.sh + tok0 * p.d_o.st;
-      const RowSource<T> qsrc = make_row_source<T, true>(qb, p.q.st, L, DH), dosrc = make_row_source<T, true>(dob, p.d_o.st, L, DH);
+      const RowSource<T> qsrc = make_row_source<T, kLoad>(qb, p.q.st, L, D), dosrc = make_row_source<T, kLoad>(dob, p.d_o.st, L, D);
       // Rows of step r into stage r%4 from register set r%2, then the rows of step r+2 requested into that set.
       auto stage_rows = [&](int r) {
         T* q_lds = lds + Lds::kQ + (r & 3) * 2 * Lds::kQdoTile;
@@ -881,46 +889,47 @@ __global__ __launch_bounds__(kDkv4Threads) void bwd_dkv4_kernel(BwdParams p) {
   }
 }
 
-template <typename T, int DH>
+template <typename T, int DH, int kLoad>
 static hipError_t launch_dkv4(const BwdParams& p_in, int max_tiles, hipStream_t stream) {
   const size_t lds_bytes = (size_t)Dkv4Lds<DH>::kElems * sizeof(T) + 256;      // + the published queue slot
   static std::atomic<uint64_t> lds_done{0};
   int dev = 0, cus = 0;
   hipError_t e = device_cus(&dev, &cus);
   if (e != hipSuccess) return e;
-  if ((e = raise_lds_limit(&bwd_dkv4_kernel<T, DH>, lds_done, dev, lds_bytes)) != hipSuccess) return e;
+  if ((e = raise_lds_limit(&bwd_dkv4_kernel<T, DH, kLoad>, lds_done, dev, lds_bytes)) != hipSuccess) return e;
   BwdParams p = p_in;
   p.wgs_per_head = cus / p.num_heads > 0 ? cus / p.num_heads : 1;
   if (p.wgs_per_head > max_tiles) p.wgs_per_head = max_tiles;
   const dim3 grid((unsigned)(p.wgs_per_head * p.num_heads)), block(kDkv4Threads);
-  hipLaunchKernelGGL((bwd_dkv4_kernel<T, DH>), grid, block, lds_bytes, stream, p);
+  hipLaunchKernelGGL((bwd_dkv4_kernel<T, DH, kLoad>), grid, block, lds_bytes, stream, p);
   return hipGetLastError();
 }
 
-template <typename T, int DH, bool kFast>
+template <typename T, int DH>
 static hipError_t launch_one(const BwdParams& p, int max_tiles, hipStream_t stream) {
   const size_t lds_bytes = (size_t)DkvLds<DH>::kElems * sizeof(T);
   static std::atomic<uint64_t> lds_done{0};
   int dev = 0, cus = 0;
   hipError_t e = device_cus(&dev, &cus);
   if (e != hipSuccess) return e;
-  if ((e = raise_lds_limit(&bwd_dkv_kernel<T, DH, kFast>, lds_done, dev, lds_bytes)) != hipSuccess) return e;
+  if ((e = raise_lds_limit(&bwd_dkv_kernel<T, DH>, lds_done, dev, lds_bytes)) != hipSuccess) return e;
   const dim3 grid((unsigned)(max_tiles * p.num_heads)), block(kThreads);
-  hipLaunchKernelGGL((bwd_dkv_kernel<T, DH, kFast>), grid, block, lds_bytes, stream, p);
+  hipLaunchKernelGGL((bwd_dkv_kernel<T, DH>), grid, block, lds_bytes, stream, p);
   return hipGetLastError();
 }
 
 template <typename T>
 static hipError_t launch_t(const BwdParams& p, int max_tiles, hipStream_t stream) {
   // head_dim 64 measures slightly faster on the 64-key kernel (its steps are already short).
-  if (p.vec_ok && p.head_dim == 128) return launch_dkv4<T, 128>(p, max_tiles, stream);
-  if (p.vec_ok && p.head_dim == 64) return launch_dkv3<T, 64>(p, max_tiles, stream);
-  return p.head_dim <= 64 ? launch_one<T, 64, false>(p, max_tiles, stream) : launch_one<T, 128, false>(p, max_tiles, stream);
+  const bool wide = p.head_dim > 64;
+  if (p.load == kLoadAligned) return wide ? launch_dkv4<T, 128, kLoadAligned>(p, max_tiles, stream) : launch_dkv3<T, 64, kLoadAligned>(p, max_tiles, stream);
+  if (p.load == kLoadPadded) return wide ? launch_dkv4<T, 128, kLoadPadded>(p, max_tiles, stream) : launch_dkv3<T, 64, kLoadPadded>(p, max_tiles, stream);
+  return wide ? launch_one<T, 128>(p, max_tiles, stream) : launch_one<T, 64>(p, max_tiles, stream);
 }
 
 // Keys per key tile of the kernel launch_bwd_dkv will pick for these parameters.
 int dkv_key_tile(const BwdParams& p) {
-  return (p.vec_ok && p.head_dim == 128) ? kDkv4Keys : kBlockK;
+  return p.load != kLoadScalar && p.head_dim > 64 ? kDkv4Keys : kBlockK;
 }
 
 hipError_t launch_bwd_dkv(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream) {

@@ -21,8 +21,9 @@
 
 namespace sba {
 
-template <typename T, int DH, bool kFast, int KT>
+template <typename T, int DH, int kLoad, int KT>
 __global__ __launch_bounds__(kThreads, KT == 32 ? 2 : 1) void bwd_dq_kernel(BwdParams p) {
+  constexpr bool kFast = kLoad != kLoadScalar;
   constexpr int NT = KT / 32;         // MFMA row tiles per key tile: a lane owns 16*NT consecutive keys
   typedef typename Elem<T>::vec8 vec8;
   constexpr int kRowStride = lds_stride<DH>();
@@ -58,8 +59,8 @@ __global__ __launch_bounds__(kThreads, KT == 32 ? 2 : 1) void bwd_dq_kernel(BwdP
 #pragma unroll
   for (int kk = 0; kk < kSteps; kk++) {
     const int d0 = 16 * kk + 8 * half;
-    qf[kk] = as_vec8<T>(load_row8<T, kFast>(qb + (int64_t)qi * p.q.st, d0, D, row_ok));
-    dof[kk] = as_vec8<T>(load_row8<T, kFast>(dob + (int64_t)qi * p.d_o.st, d0, D, row_ok));
+    qf[kk] = as_vec8<T>(load_row8<T, kLoad>(qb + (int64_t)qi * p.q.st, d0, D, row_ok));
+    dof[kk] = as_vec8<T>(load_row8<T, kLoad>(dob + (int64_t)qi * p.d_o.st, d0, D, row_ok));
   }
   float drem = 0.f;
   if (row_ok && p.d_rem.ptr)
@@ -69,7 +70,7 @@ __global__ __launch_bounds__(kThreads, KT == 32 ? 2 : 1) void bwd_dq_kernel(BwdP
     float dot = 0.f;
 #pragma unroll
     for (int kk = 0; kk < kSteps; kk++) {
-      const vec8 vv = as_vec8<T>(load_row8<T, kFast>(vb + (int64_t)qi * p.v.st, 16 * kk + 8 * half, D, row_ok));
+      const vec8 vv = as_vec8<T>(load_row8<T, kLoad>(vb + (int64_t)qi * p.v.st, 16 * kk + 8 * half, D, row_ok));
 #pragma unroll
       for (int t = 0; t < 8; t++) dot = fmaf((float)dof[kk][t], (float)vv[t], dot);
     }
@@ -101,8 +102,8 @@ __global__ __launch_bounds__(kThreads, KT == 32 ? 2 : 1) void bwd_dq_kernel(BwdP
     return carry_offset(u, n_qt) + (qi - kBlockQ * (u >> 2));
   };
   float n_prod = 1.f;
-  const RowSource<T> ksrc = make_row_source<T, kFast>(kb, p.k.st, L, D), vsrc = make_row_source<T, kFast>(vb, p.v.st, L, D);
-  TileCopy<T, DH, KT, kFast> ck, cv;
+  const RowSource<T> ksrc = make_row_source<T, kLoad>(kb, p.k.st, L, D), vsrc = make_row_source<T, kLoad>(vb, p.v.st, L, D);
+  TileCopy<T, DH, KT, kLoad> ck, cv;
   if (n_kt > 0) {
     ck.load(ksrc, 0);
     cv.load(vsrc, 0);
@@ -200,7 +201,7 @@ __global__ __launch_bounds__(kThreads, KT == 32 ? 2 : 1) void bwd_dq_kernel(BwdP
   if (kFast) {
     const RowSink<T> sink = make_row_sink<T>(dqb, p.dq.st, L, D);
 #pragma unroll
-    for (int dt = 0; dt < kDTiles; dt++) store_acc_tile<T>(sink, dqacc[dt], p.logit_scale, w_first, 32 * dt, half, col);
+    for (int dt = 0; dt < kDTiles; dt++) store_acc_tile<T>(sink, dqacc[dt], p.logit_scale, w_first, 32 * dt, half, col, kLoad == kLoadPadded ? D : DH);
     return;
   }
 #pragma unroll
@@ -217,14 +218,15 @@ __global__ __launch_bounds__(kThreads, KT == 32 ? 2 : 1) void bwd_dq_kernel(BwdP
 template <typename T>
 static hipError_t launch_t(const BwdParams& p, int max_tiles, hipStream_t stream) {
   const dim3 grid((unsigned)(max_tiles * p.num_heads)), block(kThreads);
-  if (p.vec_ok && p.head_dim == 128) {
-    hipLaunchKernelGGL((bwd_dq_kernel<T, 128, true, 32>), grid, block, 0, stream, p);
-  } else if (p.vec_ok && p.head_dim == 64) {
-    hipLaunchKernelGGL((bwd_dq_kernel<T, 64, true, 32>), grid, block, 0, stream, p);
-  } else if (p.head_dim <= 64) {
-    hipLaunchKernelGGL((bwd_dq_kernel<T, 64, false, 64>), grid, block, 0, stream, p);
+  if (p.load == kLoadAligned) {
+    if (p.head_dim == 128) hipLaunchKernelGGL((bwd_dq_kernel<T, 128, kLoadAligned, 32>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((bwd_dq_kernel<T, 64, kLoadAligned, 32>), grid, block, 0, stream, p);
+  } else if (p.load == kLoadPadded) {
+    if (p.head_dim > 64) hipLaunchKernelGGL((bwd_dq_kernel<T, 128, kLoadPadded, 32>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((bwd_dq_kernel<T, 64, kLoadPadded, 32>), grid, block, 0, stream, p);
   } else {
-    hipLaunchKernelGGL((bwd_dq_kernel<T, 128, false, 64>), grid, block, 0, stream, p);
+    if (p.head_dim > 64) hipLaunchKernelGGL((bwd_dq_kernel<T, 128, kLoadScalar, 64>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((bwd_dq_kernel<T, 64, kLoadScalar, 64>), grid, block, 0, stream, p);
   }
   return hipGetLastError();
 }

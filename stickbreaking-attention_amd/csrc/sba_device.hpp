@@ -122,6 +122,20 @@ __device__ __forceinline__ int mfma_row_to_key(int mt, int m) {
 // Same for a 32-key sub-tile handled as ONE row tile: register r of half-wave h holds key 16*h + r.
 __device__ __forceinline__ int mfma_row_to_key32(int m) { return ((m >> 2) & 1) * 16 + (m >> 3) * 4 + (m & 3); }
 
+constexpr int kOutside = (int)0x80000000;      // byte offset beyond every buffer (they span less than 2 GiB)
+
+// The 8 elements of v moved down by n elements (0..7), zeros from above.
+__device__ __forceinline__ u32x4 shift_down(u32x4 v, int n) {
+  const uint32_t bits = (n & 1) * 16;
+  uint32_t t[4] = {__builtin_amdgcn_alignbit(v[1], v[0], bits), __builtin_amdgcn_alignbit(v[2], v[1], bits),
+                   __builtin_amdgcn_alignbit(v[3], v[2], bits), v[3] >> bits};
+  const bool one = n & 2, two = n & 4;
+  t[0] = one ? t[1] : t[0]; t[1] = one ? t[2] : t[1]; t[2] = one ? t[3] : t[2]; t[3] = one ? 0u : t[3];
+  return u32x4{two ? t[2] : t[0], two ? t[3] : t[1], two ? 0u : t[2], two ? 0u : t[3]};
+}
+// Columns a chunk at column `col` has to be moved down by after a padded load (0 where it is loaded in place).
+__device__ __forceinline__ int padded_shift(int col, int d) { return col < d && col > d - 8 ? col - (d - 8) : 0; }
+
 // The rows of one (head, sequence) of a [.., token, head_dim] tensor, as the tile copies see them.  The fast path
 // addresses them through a raw buffer resource: scalar base, out-of-range rows read as zero for free, and one
 // loop-invariant 32-bit lane offset instead of 64-bit pointer arithmetic per chunk.
@@ -133,33 +147,55 @@ struct RowSource {
   __amdgpu_buffer_rsrc_t rsrc;    // base .. last valid element (fast path only)
   int stride_bytes;
 };
-template <typename T, bool kFast>
+template <typename T, int kLoad>
 __device__ __forceinline__ RowSource<T> make_row_source(const T* base, int64_t stride, int rows, int d) {
   RowSource<T> r;
   r.base = base; r.stride = stride; r.rows = rows; r.d = d;
   r.stride_bytes = (int)(stride * (int64_t)sizeof(T));
-  if (kFast) {
+  if (kLoad != kLoadScalar) {
     const int bytes = rows > 0 ? (rows - 1) * r.stride_bytes + d * (int)sizeof(T) : 0;
     r.rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes, 0x00020000);
   }
   return r;
 }
 
+// Byte offset of the 8 elements at column `col` of row `row`.
+template <typename T, int kLoad>
+__device__ __forceinline__ int chunk_offset(const RowSource<T>& src, int row, int col) {
+  if (kLoad == kLoadPadded && col >= src.d) return kOutside;
+  return row * src.stride_bytes + (kLoad == kLoadPadded ? col - padded_shift(col, src.d) : col) * (int)sizeof(T);
+}
+// An MFMA operand of kSteps such chunks (columns 16 kk + 8 half), requested and, once it is here, put into place.
+template <typename T, int kLoad, int kSteps>
+__device__ __forceinline__ void request_operand(typename Elem<T>::vec8 (&x)[kSteps], const RowSource<T>& src, int row, int half) {
+#pragma unroll
+  for (int kk = 0; kk < kSteps; kk++)       // rows beyond the sequence are outside the buffer and read as zero
+    x[kk] = as_vec8<T>(__builtin_amdgcn_raw_buffer_load_b128(src.rsrc, chunk_offset<T, kLoad>(src, row, 16 * kk + 8 * half), 0, 0));
+}
+template <typename T, int kLoad, int kSteps>
+__device__ __forceinline__ void place_operand(typename Elem<T>::vec8 (&x)[kSteps], int d, int half) {
+  if (kLoad != kLoadPadded || (d & 7) == 0) return;
+#pragma unroll
+  for (int kk = 0; kk < kSteps; kk++)
+    if (kk == (d >> 4)) x[kk] = as_vec8<T>(shift_down(__builtin_bit_cast(u32x4, x[kk]), padded_shift(16 * kk + 8 * half, d)));
+}
+
 // Cooperative global -> register -> LDS copy of a [kRows x DH] tile of 16-bit elements, 16 bytes per access.
-// Rows beyond the source and columns at or beyond head_dim are zero-filled.  kFast: head_dim == DH, every row
-// start 16-byte aligned and the sequence's rows span < 2 GiB, so the copy is straight-line buffer loads.
-template <typename T, int DH, int kRows, bool kFast, int kNumThreads = kThreads>
+// Rows beyond the source and columns at or beyond head_dim are zero-filled.
+template <typename T, int DH, int kRows, int kLoad, int kNumThreads = kThreads>
 struct TileCopy {
   static constexpr int kChunksPerRow = DH / 8;
   static constexpr int kRowsPerPass = kNumThreads / kChunksPerRow;
   static constexpr int kPerThread = kRows / kRowsPerPass;
   static_assert(kRows % kRowsPerPass == 0, "tile must divide evenly over the workgroup");
   u32x4 regs[kPerThread];
+  int shift;      // padded loads only
 
   __device__ __forceinline__ void load(const RowSource<T>& src, int row0) {
     const int tr = (threadIdx.x % kNumThreads) / kChunksPerRow, col = ((threadIdx.x % kNumThreads) % kChunksPerRow) * 8;
-    if (kFast) {
-      const int voff = tr * src.stride_bytes + col * (int)sizeof(T);
+    if (kLoad != kLoadScalar) {
+      const int voff = chunk_offset<T, kLoad>(src, tr, col);
+      if (kLoad == kLoadPadded) shift = padded_shift(col, src.d);
 #pragma unroll
       for (int i = 0; i < kPerThread; i++)
         regs[i] = __builtin_amdgcn_raw_buffer_load_b128(src.rsrc, voff, (row0 + i * kRowsPerPass) * src.stride_bytes, 0);
@@ -184,17 +220,24 @@ struct TileCopy {
     const int tr = (threadIdx.x % kNumThreads) / kChunksPerRow, col = ((threadIdx.x % kNumThreads) % kChunksPerRow) * 8;
 #pragma unroll
     for (int i = 0; i < kPerThread; i++)
-      *reinterpret_cast<u32x4*>(tile + (tr + i * kRowsPerPass) * lds_stride<DH>() + col) = regs[i];
+      *reinterpret_cast<u32x4*>(tile + (tr + i * kRowsPerPass) * lds_stride<DH>() + col) =
+          kLoad == kLoadPadded && __any(shift) ? shift_down(regs[i], shift) : regs[i];
   }
 };
 
 // Load 8 consecutive head_dim elements of one token row from global memory (zero beyond head_dim / when !valid).
-template <typename T, bool kFast>
+template <typename T, int kLoad>
 __device__ __forceinline__ u32x4 load_row8(const T* row, int d0, int d_valid, bool valid) {
   u32x4 v = {0, 0, 0, 0};
   if (valid) {
-    if (kFast) {
+    if (kLoad == kLoadAligned) {
       v = *reinterpret_cast<const u32x4*>(row + d0);
+    } else if (kLoad == kLoadPadded) {
+      if (d0 < d_valid) {
+        typedef __attribute__((ext_vector_type(4), aligned(2))) uint32_t u32x4_any;
+        const int n = padded_shift(d0, d_valid);
+        v = shift_down(*reinterpret_cast<const u32x4_any*>(row + d0 - n), n);
+      }
     } else {
       uint16_t e[8];
 #pragma unroll
@@ -305,11 +348,12 @@ __device__ __forceinline__ RowSink<T> make_row_sink(T* base, int64_t stride, int
   r.rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes, 0x00020000);
   return r;
 }
-// acc[r] -> row (row0 + 8*(r/4) + 4*half + r%4), column col0 + (lane % 32), scaled; row0 and col0 wave-uniform.
+// acc[r] -> row (row0 + 8*(r/4) + 4*half + r%4), column col0 + (lane % 32), scaled; row0 and col0 wave-uniform; columns at or
+// beyond `d` are dropped.
 template <typename T>
 __device__ __forceinline__ void store_acc_tile(const RowSink<T>& sink, const f32x16& acc, float scale, int row0, int col0,
-                                               int half, int col) {
-  const int voff = 4 * half * sink.stride_bytes + col * (int)sizeof(T);
+                                               int half, int col, int d) {
+  const int voff = col0 + col < d ? 4 * half * sink.stride_bytes + col * (int)sizeof(T) : kOutside;
   const int sbase = __builtin_amdgcn_readfirstlane(row0 * sink.stride_bytes + col0 * (int)sizeof(T));
 #pragma unroll
   for (int r = 0; r < 16; r++) {

@@ -93,7 +93,7 @@ struct Operand {
     } else {
 #pragma unroll
       for (int j = 0; j < P::NC; j++) {
-        const uint32_t vo = kExact || part * P::C + P::NC * col + j < D ? voff + 4 * (part * P::C + j) : 0xfffffff0u;
+        const uint32_t vo = kExact || part * P::C + P::NC * col + j < D ? voff + 4 * (part * P::C + j) : (uint32_t)kOutside;
         y[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(src.rsrc, vo, soff, 0));
       }
     }
@@ -211,7 +211,7 @@ __device__ __forceinline__ void stage_rows(float* lds, const Rows32& s, int D) {
   } else {
     for (int idx = threadIdx.x; idx < 32 * DH; idx += kThreads) {
       const int row = idx / DH, d = idx % DH;
-      const uint32_t v = __builtin_amdgcn_raw_buffer_load_b32(s.rsrc, d < D ? (uint32_t)row * s.stride_bytes + 4 * d : 0xfffffff0u, 0, 0);
+      const uint32_t v = __builtin_amdgcn_raw_buffer_load_b32(s.rsrc, d < D ? (uint32_t)row * s.stride_bytes + 4 * d : (uint32_t)kOutside, 0, 0);
       lds[row * (DH + 4) + d] = __builtin_bit_cast(float, v);
     }
   }

@@ -19,8 +19,9 @@ namespace sba {
 
 // kCarryOnly: only the products of (1 - sigma) above every sub-tile are rebuilt (into `carry`), for a backward whose
 // forward did not keep them: no V, no P V, no outputs.
-template <typename T, int DH, bool kFast, int KT, int kMinWaves, bool kCarryOnly = false>
+template <typename T, int DH, int kLoad, int KT, int kMinWaves, bool kCarryOnly = false>
 __global__ __launch_bounds__(kThreads, kMinWaves) void fwd_kernel(FwdParams p) {
+  constexpr bool kFast = kLoad != kLoadScalar;
   constexpr int NT = KT / 32;         // MFMA row tiles per key tile: a lane owns N = 16*NT consecutive keys
   constexpr int N = 16 * NT;
   typedef typename Elem<T>::vec8 vec8;
@@ -56,7 +57,7 @@ __global__ __launch_bounds__(kThreads, kMinWaves) void fwd_kernel(FwdParams p) {
   vec8 qf[kSteps];
 #pragma unroll
   for (int kk = 0; kk < kSteps; kk++)
-    qf[kk] = as_vec8<T>(load_row8<T, kFast>(qb + (int64_t)qi * p.q.st, 16 * kk + 8 * half, D, qi < L));
+    qf[kk] = as_vec8<T>(load_row8<T, kLoad>(qb + (int64_t)qi * p.q.st, 16 * kk + 8 * half, D, qi < L));
 
   const int last_row = min(q0 + kBlockQ, L) - 1;
   const int last_key = last_row - 1 + ac;                    // last key any row of this tile can see
@@ -72,8 +73,8 @@ __global__ __launch_bounds__(kThreads, kMinWaves) void fwd_kernel(FwdParams p) {
   const int64_t n_qt = (L + kBlockQ - 1) / kBlockQ;
   float* carry = p.carry ? p.carry + (int64_t)head * p.carry_head_stride + tile.carry_base : nullptr;
 
-  const RowSource<T> ksrc = make_row_source<T, kFast>(kb, p.k.st, L, D), vsrc = make_row_source<T, kFast>(vb, p.v.st, L, D);
-  TileCopy<T, DH, KT, kFast> ck, cv;
+  const RowSource<T> ksrc = make_row_source<T, kLoad>(kb, p.k.st, L, D), vsrc = make_row_source<T, kLoad>(vb, p.v.st, L, D);
+  TileCopy<T, DH, KT, kLoad> ck, cv;
   if (n_kt > 0) {
     ck.load(ksrc, (n_kt - 1) * KT);
     if (!kCarryOnly) cv.load(vsrc, (n_kt - 1) * KT);
@@ -207,7 +208,7 @@ __global__ __launch_bounds__(kThreads, kMinWaves) void fwd_kernel(FwdParams p) {
   } else if (kFast) {
     const RowSink<T> sink = make_row_sink<T>(ob, p.o.st, L, D);
 #pragma unroll
-    for (int dt = 0; dt < kDTiles; dt++) store_acc_tile<T>(sink, oacc[dt], 1.f, w_first, 32 * dt, half, col);
+    for (int dt = 0; dt < kDTiles; dt++) store_acc_tile<T>(sink, oacc[dt], 1.f, w_first, 32 * dt, half, col, kLoad == kLoadPadded ? D : DH);
   } else {
 #pragma unroll
     for (int dt = 0; dt < kDTiles; dt++) {
@@ -229,14 +230,15 @@ __global__ __launch_bounds__(kThreads, kMinWaves) void fwd_kernel(FwdParams p) {
 template <typename T, bool kCarryOnly>
 static hipError_t launch_fwd_t(const FwdParams& p, int max_tiles, hipStream_t stream) {
   const dim3 grid((unsigned)(max_tiles * p.num_heads)), block(kThreads);
-  if (p.vec_ok && p.head_dim == 128) {
-    hipLaunchKernelGGL((fwd_kernel<T, 128, true, 32, 3, kCarryOnly>), grid, block, 0, stream, p);
-  } else if (p.vec_ok && p.head_dim == 64) {
-    hipLaunchKernelGGL((fwd_kernel<T, 64, true, 64, 2, kCarryOnly>), grid, block, 0, stream, p);
-  } else if (p.head_dim <= 64) {
-    hipLaunchKernelGGL((fwd_kernel<T, 64, false, 64, 2, kCarryOnly>), grid, block, 0, stream, p);
+  if (p.load == kLoadAligned) {
+    if (p.head_dim == 128) hipLaunchKernelGGL((fwd_kernel<T, 128, kLoadAligned, 32, 3, kCarryOnly>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((fwd_kernel<T, 64, kLoadAligned, 64, 2, kCarryOnly>), grid, block, 0, stream, p);
+  } else if (p.load == kLoadPadded) {
+    if (p.head_dim > 64) hipLaunchKernelGGL((fwd_kernel<T, 128, kLoadPadded, 32, 2, kCarryOnly>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((fwd_kernel<T, 64, kLoadPadded, 64, 2, kCarryOnly>), grid, block, 0, stream, p);
   } else {
-    hipLaunchKernelGGL((fwd_kernel<T, 128, false, 64, 2, kCarryOnly>), grid, block, 0, stream, p);
+    if (p.head_dim > 64) hipLaunchKernelGGL((fwd_kernel<T, 128, kLoadScalar, 64, 2, kCarryOnly>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((fwd_kernel<T, 64, kLoadScalar, 64, 2, kCarryOnly>), grid, block, 0, stream, p);
   }
   return hipGetLastError();
 }

@@ -22,6 +22,15 @@ struct Tile {
   int64_t carry_base;  // first carry slot of the sequence within a head's plane (0 when no carries are laid out)
 };
 
+// How the 16-bit kernels read rows of head_dim elements, by what the tensors allow:
+//   kLoadAligned : head_dim is the kernel's width (64 or 128) and every row starts on a 16-byte boundary: 16-byte loads.
+//   kLoadPadded  : any head_dim from 8 on, any alignment: 16-byte loads all the same (the memory pipe takes them at any
+//                  element's address).  A chunk of 8 columns that head_dim cuts is loaded from column head_dim - 8 and shifted
+//                  into place, so that no load leaves its row; chunks beyond head_dim ask for an address outside the buffer.
+//                  The shift costs 12 vector-ALU instructions per 16 bytes where head_dim is no multiple of 8.
+//   kLoadScalar  : what is left (head_dim below 8, or a sequence whose rows span 2 GiB): element by element.
+enum : int { kLoadScalar = 0, kLoadAligned = 1, kLoadPadded = 2 };
+
 // Slots of the scheduler's `counts` array.
 enum : int { kCountQ = 0, kCountK = 1, kCountStatus = 2, kCountCovered = 3 };
 // Values of counts[kCountStatus].
@@ -62,7 +71,7 @@ struct FwdParams {
   int32_t num_heads, head_dim;
   float scale_log2;            // logit_scale * log2(e)
   int32_t attend_current;
-  int32_t vec_ok;              // all row strides / base pointers allow 16-byte accesses and head_dim % 8 == 0
+  int32_t load;                // kLoadAligned, kLoadPadded or kLoadScalar: how rows are read
   int32_t add_rem;             // write o + rem * v
   int32_t max_tiles;           // query-tile slots the launch provides per head (>= counts[kCountQ])
   int64_t total_tokens;        // packed mode: rows of the token axis; rows no sequence covers are zero-filled
@@ -82,7 +91,7 @@ struct BwdParams {
   float scale_log2;
   float logit_scale;
   int32_t attend_current;
-  int32_t vec_ok;
+  int32_t load;                // as in FwdParams
   // Fused remainder term (the forward wrote o + rem * v): d_rem_eff = d_rem + d_o . v per row, dv += rem * d_o.
   int32_t add_rem;
   const float* row_stat;       // log2(rem), fp32 [batch][head][token]

@@ -4,10 +4,11 @@
 #include <atomic>
 
 #include "../../include/sba.h"
+#include "sba_internal.hpp"
 #include "sba_params.hpp"
 
 namespace sba {
-hipError_t launch_sched(const SchedParams& p, hipStream_t stream);
+hipError_t launch_sched(const SchedParams& p, int clear_wgs, hipStream_t stream);
 hipError_t launch_fwd(const FwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
 hipError_t launch_fwd_carry_only(const FwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
 hipError_t launch_bwd_dq(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
@@ -29,13 +30,16 @@ inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 struct Layout {
   int64_t max_q_tiles, max_k_tiles, carry_slots_per_head;
-  size_t off_counts, off_q_tiles, off_k_tiles, off_carry_base, off_prefix, off_drem, off_queue, off_carry;
+  // Offsets in the schedule, which a forward can prepare for the backward that follows it ...
+  size_t off_counts, off_q_tiles, off_k_tiles, off_carry_base, off_queue, sched_bytes;
+  // ... and in the rest of a backward's workspace, which starts behind it.
+  size_t off_prefix, off_drem, off_carry, rest_bytes;
   size_t fwd_bytes, bwd_bytes, carry_bytes;
   size_t pass_bytes;                        // what ONE pass over these heads needs (bwd_bytes: what sba_bwd wants, see split_heads)
-  // One-kernel backward: its buffers share the prefix plane's region (only one of the two backwards runs).
+  // One-kernel backward: its partial sums share the prefix plane's region (only one of the two backwards runs).
   int64_t chain_rows;                       // rows per head
-  size_t off_chain_zero, chain_zero_bytes;  // {C, tag} per row, the flags and the heads' XCC ids: cleared by every launch
-  size_t off_chain_c, off_chain_flags, off_chain_xcc, off_chain_dq;
+  size_t off_chain_zero, chain_zero_bytes;  // {C, tag} per row, the flags and the heads' XCC ids: cleared with the schedule
+  size_t off_chain_c, off_chain_flags, off_chain_xcc;
   int32_t split_heads;                      // > 0: sba_bwd takes this many heads (a multiple of 8) through the one-kernel
                                             // backward and the rest through the two kernels
 };
@@ -71,6 +75,7 @@ int plan(const SbaArgs* a, Layout* out) {
   L.off_carry_base = off;  off = align_up(off + (size_t)B * sizeof(int64_t), 256);
   L.fwd_bytes = off;
   L.off_k_tiles = off;     off = align_up(off + (size_t)L.max_k_tiles * sizeof(sba::Tile), 256);
+  L.off_queue = off;       off = align_up(off + (size_t)a->num_heads * sizeof(int32_t), 256);      // per-head tile cursors
   L.carry_bytes = align_up((size_t)L.carry_slots_per_head * a->num_heads * sizeof(float), 256);
   size_t chain_bytes = 0;
   L.chain_rows = fixed ? B * T : T;
@@ -86,22 +91,22 @@ int plan(const SbaArgs* a, Layout* out) {
   const bool chain_pays = max_len <= 256 ||
                           (a->num_heads <= 32 && mean_len * a->num_heads >= 32768 && max_len * a->num_heads <= (int64_t)512 * 256);
   if (chain_shape && (a->backward_kernels == 2 || (a->backward_kernels == 0 && chain_pays))) {
-    size_t c = off;
-    L.off_chain_zero = c;
-    L.off_chain_c = c;      c = align_up(c + (size_t)a->num_heads * L.chain_rows * 8, 256);
-    L.off_chain_flags = c;  c = align_up(c + (size_t)a->num_heads * L.max_k_tiles * 32, 256);
-    L.off_chain_xcc = c;    c = align_up(c + (size_t)a->num_heads * 4, 256);
-    L.chain_zero_bytes = c - L.off_chain_zero;
-    L.off_chain_dq = c;     c += (size_t)a->num_heads * L.chain_rows * 128 * sizeof(float);
-    chain_bytes = align_up(c - off, 256);
+    L.off_chain_zero = off;
+    L.off_chain_c = off;      off = align_up(off + (size_t)a->num_heads * L.chain_rows * 8, 256);
+    L.off_chain_flags = off;  off = align_up(off + (size_t)a->num_heads * L.max_k_tiles * 32, 256);
+    L.off_chain_xcc = off;    off = align_up(off + (size_t)a->num_heads * 4, 256);
+    L.chain_zero_bytes = off - L.off_chain_zero;
+    chain_bytes = align_up((size_t)a->num_heads * L.chain_rows * 128 * sizeof(float), 256);
   }
+  L.sched_bytes = off;
+  off = 0;
   L.off_prefix = off;      off += L.carry_bytes > chain_bytes ? L.carry_bytes : chain_bytes;
   // d_rem + d_o . v per row (fp32), used when the remainder term is fused
   L.off_drem = off;        off = align_up(off + (size_t)a->num_heads * (size_t)T * (fixed ? (size_t)B : 1) * sizeof(float), 256);
-  L.off_queue = off;       off = align_up(off + (size_t)a->num_heads * sizeof(int32_t), 256);      // per-head tile cursors
   // the forward's products, rebuilt inside the backward when the caller did not keep them
   L.off_carry = off;       if (a->recompute_carry) off += L.carry_bytes;
-  L.bwd_bytes = L.pass_bytes = off;
+  L.rest_bytes = off;
+  L.bwd_bytes = L.pass_bytes = L.sched_bytes + L.rest_bytes;
   // A head count that is not a multiple of 8 (the reference's own benchmarks use 12) cannot run the one-kernel backward,
   // whose workgroups of a head must share an XCD.  Left to choose, sba_bwd then takes the largest multiple of 8 through
   // it and the remaining heads through the two kernels, one pass after the other on the stream -- where that pays: two
@@ -157,10 +162,11 @@ bool f32_stride_ok(const SbaArgs* a) {
 sba::TensorRef ref(const SbaTensor& t, bool fixed) { return sba::TensorRef{t.ptr, fixed ? t.stride_batch : 0, t.stride_head, t.stride_token}; }
 sba::VectorRef vref(const SbaVector& t, bool fixed) { return sba::VectorRef{t.ptr, fixed ? t.stride_batch : 0, t.stride_head, t.stride_token}; }
 
-int run_sched(const SbaArgs* a, char* ws, const Layout& L, bool want_key_tiles, bool want_carry_base, int key_tile, hipStream_t stream,
-              bool clear_chain = false) {
+// What the scheduler is asked for: always the query tiles; `for_backward`: the key tiles as well, the tile cursors at zero and
+// what the one-kernel backward needs cleared.
+sba::SchedParams sched_params(const SbaArgs* a, char* ws, const Layout& L, bool for_backward, bool want_carry_base, int key_tile) {
   sba::SchedParams sp{};
-  if (clear_chain) {
+  if (for_backward && L.chain_zero_bytes > 0) {
     sp.zero_fill = (uint32_t*)(ws + L.off_chain_zero);
     sp.zero_bytes = (int64_t)L.chain_zero_bytes;
   }
@@ -171,8 +177,7 @@ int run_sched(const SbaArgs* a, char* ws, const Layout& L, bool want_key_tiles, 
   sp.fixed_len = (int32_t)a->total_tokens;
   sp.total_tokens = a->total_tokens;
   sp.carry_capacity = L.carry_slots_per_head;
-  sp.attend_current = a->attend_current ? 1 : 0;
-  sp.want_key_tiles = want_key_tiles ? 1 : 0;
+  sp.want_key_tiles = for_backward ? 1 : 0;
   sp.want_carry_base = want_carry_base ? 1 : 0;
   sp.q_tiles = (sba::Tile*)(ws + L.off_q_tiles);
   sp.k_tiles = (sba::Tile*)(ws + L.off_k_tiles);
@@ -181,7 +186,22 @@ int run_sched(const SbaArgs* a, char* ws, const Layout& L, bool want_key_tiles, 
   sp.head_queue = (int32_t*)(ws + L.off_queue);
   sp.num_heads = a->num_heads;
   sp.key_tile = key_tile;
-  return sba::launch_sched(sp, stream) == hipSuccess ? SBA_OK : SBA_ERR_LAUNCH;
+  return sp;
+}
+
+// Workgroups that clear the region a schedule is asked to clear: one per 256 KiB, at most 64.
+int clear_wgs(const sba::SchedParams& sp) {
+  const int64_t n = (sp.zero_bytes + (256 << 10) - 1) / (256 << 10);
+  return (int)(n > 64 ? 64 : n);
+}
+
+// Keys per key tile of the backward that will follow a forward, as far as the forward's tensors tell.
+int expected_key_tile(const SbaArgs* a) {
+  if (a->dtype == SBA_F32) return kBlockK;
+  sba::BwdParams p{};
+  p.head_dim = a->head_dim;
+  p.load = row_load(a, {&a->q, &a->k, &a->v});
+  return sba::dkv_key_tile(p);
 }
 
 }  // namespace
@@ -267,8 +287,9 @@ int static_scratch(char** out) {
   return SBA_OK;
 }
 
-// The forward on a given workspace (the caller's, or the library's static scratch).
-int fwd_on(const SbaArgs* a, char* ws, size_t ws_bytes, bool ws_is_static) {
+// The forward on a given workspace (the caller's, or the library's static scratch).  `for_backward`: the workspace holds
+// sched_bytes and keeps the schedule of the backward that will follow.
+int fwd_on(const SbaArgs* a, char* ws, size_t ws_bytes, bool ws_is_static, bool for_backward) {
   Layout L;
   int st = plan(a, &L);
   if (st != SBA_OK) return st;
@@ -282,13 +303,18 @@ int fwd_on(const SbaArgs* a, char* ws, size_t ws_bytes, bool ws_is_static) {
   for (const SbaTensor* t : {&a->q, &a->k, &a->v, &a->o})
     if (t->ptr && ((uintptr_t)t->ptr % es)) return SBA_ERR_ALIGN;
   if (ws_is_static && ws_bytes < L.fwd_bytes) return SBA_ERR_TOO_LARGE;
-  if (!ws || ((uintptr_t)ws & 255) || ws_bytes < L.fwd_bytes) return SBA_ERR_WORKSPACE;
+  if (!ws || ((uintptr_t)ws & 255) || ws_bytes < (for_backward ? L.sched_bytes : L.fwd_bytes)) return SBA_ERR_WORKSPACE;
   hipStream_t stream = (hipStream_t)a->stream;
   // The carry offsets are laid out (and the capacity checked) when products are recorded, and also when the backward
   // will rebuild them: both passes then agree on whether the schedule stands.
-  if ((st = run_sched(a, ws, L, false, a->carry != nullptr || a->recompute_carry, kBlockK, stream)) != SBA_OK) return st;
-
   sba::FwdParams p{};
+  p.sched = sched_params(a, ws, L, for_backward, a->carry != nullptr || a->recompute_carry, for_backward ? expected_key_tile(a) : kBlockK);
+  if (fixed || a->num_seqs <= sba::kInlineSeqs) {
+    p.sched.service = 1 + clear_wgs(p.sched);
+  } else {
+    if (sba::launch_sched(p.sched, clear_wgs(p.sched), stream) != hipSuccess) return SBA_ERR_LAUNCH;
+    p.tiles = (const sba::Tile*)(ws + L.off_q_tiles);
+  }
   p.q = ref(a->q, fixed); p.k = ref(a->k, fixed); p.v = ref(a->v, fixed); p.o = ref(a->o, fixed);
   p.rem = vref(a->rem, fixed);
   p.row_stat = a->row_stat;
@@ -297,7 +323,6 @@ int fwd_on(const SbaArgs* a, char* ws, size_t ws_bytes, bool ws_is_static) {
   p.carry_head_stride = L.carry_slots_per_head;
   p.stat_sb = fixed ? (int64_t)a->num_heads * a->total_tokens : 0;
   p.stat_sh = a->total_tokens;
-  p.tiles = (const sba::Tile*)(ws + L.off_q_tiles);
   p.counts = (const int32_t*)(ws + L.off_counts);
   p.num_heads = a->num_heads;
   p.head_dim = a->head_dim;
@@ -322,7 +347,7 @@ extern "C" {
 
 int sba_fwd(const SbaArgs* a) {
   if (!a) return SBA_ERR_NULL;
-  return fwd_on(a, (char*)a->workspace, a->workspace_bytes, false);
+  return fwd_on(a, (char*)a->workspace, a->workspace_bytes, false, false);
 }
 
 int sba_fwd_static(const SbaArgs* a) {
@@ -330,7 +355,7 @@ int sba_fwd_static(const SbaArgs* a) {
   char* ws = nullptr;
   const int st = static_scratch(&ws);
   if (st != SBA_OK) return st;
-  return fwd_on(a, ws, kStaticScratchBytes, true);
+  return fwd_on(a, ws, kStaticScratchBytes, true, false);
 }
 
 }  // extern "C"
@@ -350,8 +375,10 @@ bool bwd_is_chained(const SbaArgs* a, const Layout& L) {
 }
 
 // One pass of the backward over the heads `a` describes (all of them, or one group of a larger call: `stat_heads` is
-// the head count of the caller's row_stat array, `first`/`last` say which trace events this pass records).
-int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last) {
+// the head count of the caller's row_stat array, `first`/`last` say which trace events this pass records).  `sched`: the
+// schedule a forward left (the workspace is then the rest), or NULL to run the
+// scheduler here.
+int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* sched = nullptr) {
   Layout L;
   int st = plan(a, &L);
   if (st != SBA_OK) return st;
@@ -367,10 +394,11 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last) {
   if (a->add_remainder && !a->row_stat) return SBA_ERR_NULL;
   for (const SbaTensor* t : {&a->q, &a->k, &a->v, &a->d_o, &a->dq, &a->dk, &a->dv})
     if (t->ptr && ((uintptr_t)t->ptr % es)) return SBA_ERR_ALIGN;
-  if (!a->workspace || ((uintptr_t)a->workspace & 255) || a->workspace_bytes < L.pass_bytes) return SBA_ERR_WORKSPACE;
+  if (!a->workspace || ((uintptr_t)a->workspace & 255) || a->workspace_bytes < (sched ? L.rest_bytes : L.pass_bytes)) return SBA_ERR_WORKSPACE;
   hipStream_t stream = (hipStream_t)a->stream;
 
-  char* ws = (char*)a->workspace;
+  char* const ws = sched ? sched : (char*)a->workspace;
+  char* const rest = sched ? (char*)a->workspace : ws + L.sched_bytes;
   sba::BwdParams p{};
   p.q = ref(a->q, fixed); p.k = ref(a->k, fixed); p.v = ref(a->v, fixed);
   p.d_o = ref(a->d_o, fixed);
@@ -380,8 +408,8 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last) {
   p.k_tiles = (const sba::Tile*)(ws + L.off_k_tiles);
   p.counts = (const int32_t*)(ws + L.off_counts);
   p.carry_base = (const int64_t*)(ws + L.off_carry_base);
-  p.carry = a->recompute_carry ? (const float*)(ws + L.off_carry) : a->carry;
-  p.prefix = (float*)(ws + L.off_prefix);
+  p.carry = a->recompute_carry ? (const float*)(rest + L.off_carry) : a->carry;
+  p.prefix = (float*)(rest + L.off_prefix);
   p.carry_head_stride = L.carry_slots_per_head;
   p.num_heads = a->num_heads;
   p.head_dim = a->head_dim;
@@ -393,7 +421,7 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last) {
   p.stat_sb = fixed ? stat_heads * a->total_tokens : 0;
   p.stat_sh = a->total_tokens;
   p.drem_sb = fixed ? (int64_t)a->num_heads * a->total_tokens : 0;
-  p.drem_eff = (float*)(ws + L.off_drem);
+  p.drem_eff = (float*)(rest + L.off_drem);
   p.head_queue = (int32_t*)(ws + L.off_queue);
   p.max_tiles = (int32_t)L.max_q_tiles;
   p.total_tokens = a->total_tokens;
@@ -404,7 +432,7 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last) {
     p.chain_c = (uint32_t*)(ws + L.off_chain_c);
     p.chain_flags = (int32_t*)(ws + L.off_chain_flags);
     p.chain_head_xcc = (int32_t*)(ws + L.off_chain_xcc);
-    p.chain_dq = (float*)(ws + L.off_chain_dq);
+    p.chain_dq = (float*)(rest + L.off_prefix);
     p.status = (int32_t*)(ws + L.off_counts) + sba::kCountStatus;
     p.chain_rows = L.chain_rows;
     p.chain_sb = fixed ? a->total_tokens : 0;
@@ -412,7 +440,10 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last) {
   }
   // The key-tile list is built for the dK/dV kernel that will run.
   const int key_tile = a->dtype == SBA_F32 ? kBlockK : sba::dkv_key_tile(p);
-  if ((st = run_sched(a, ws, L, true, true, key_tile, stream, chain)) != SBA_OK) return st;
+  if (!sched) {
+    const sba::SchedParams sp = sched_params(a, ws, L, true, true, key_tile);
+    if (sba::launch_sched(sp, clear_wgs(sp), stream) != hipSuccess) return SBA_ERR_LAUNCH;
+  }
   hipEvent_t* ev = (hipEvent_t*)a->trace_events;
   if (ev && first && hipEventRecord(ev[0], stream) != hipSuccess) return SBA_ERR_LAUNCH;
   if (a->dtype == SBA_F32) {
@@ -425,7 +456,7 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last) {
     // forward kernel stripped of everything else (timed with the dQ kernel by trace_events).
     sba::FwdParams f{};
     f.q = p.q; f.k = p.k; f.v = p.v; f.o = p.q;
-    f.carry = (float*)(ws + L.off_carry);
+    f.carry = (float*)(rest + L.off_carry);
     f.carry_base = p.carry_base;
     f.carry_head_stride = L.carry_slots_per_head;
     f.tiles = p.q_tiles;
@@ -520,3 +551,28 @@ int sba_bwd(const SbaArgs* a) {
 }
 
 }  // extern "C"
+
+namespace sba {
+
+int prepared_bytes(const SbaArgs* a, size_t* sched_bytes, size_t* rest_bytes, size_t* carry_bytes) {
+  Layout L;
+  const int st = plan(a, &L);
+  if (st != SBA_OK) return st;
+  *sched_bytes = L.sched_bytes; *rest_bytes = L.rest_bytes; *carry_bytes = L.carry_bytes;
+  return SBA_OK;
+}
+
+int forward_prepared(const SbaArgs* a) { return fwd_on(a, (char*)a->workspace, a->workspace_bytes, false, true); }
+
+bool prepared_fits(const SbaArgs* a) {
+  Layout L;
+  if (plan(a, &L) != SBA_OK || L.split_heads > 0) return false;
+  BwdParams p{};
+  p.head_dim = a->head_dim;
+  p.load = bwd_load(a);
+  return a->dtype == SBA_F32 || dkv_key_tile(p) == expected_key_tile(a);
+}
+
+int backward_prepared(const SbaArgs* a, void* sched) { return bwd_pass(a, a->num_heads, true, true, (char*)sched); }
+
+}  // namespace sba

@@ -75,11 +75,8 @@ __global__ __launch_bounds__(kThreads) void bwd_dkv_kernel(BwdParams p) {
 #pragma unroll
   for (int mt = 0; mt < 2; mt++) {
     const int key = j0 + mfma_row_to_key(mt, col);
-#pragma unroll
-    for (int kk = 0; kk < kSteps; kk++) {
-      kf[mt][kk] = as_vec8<T>(load_row8<T, kLoad>(kb + (int64_t)key * p.k.st, 16 * kk + 8 * half, D, key < L));
-      vf[mt][kk] = as_vec8<T>(load_row8<T, kLoad>(vb + (int64_t)key * p.v.st, 16 * kk + 8 * half, D, key < L));
-    }
+    load_operand<T, kLoad>(kf[mt], make_row_source<T, kLoad>(kb, p.k.st, L, D), key, half);
+    load_operand<T, kLoad>(vf[mt], make_row_source<T, kLoad>(vb, p.v.st, L, D), key, half);
   }
 
   const int first_row = j0 + 1 - ac;                                  // first row that sees key j0

@@ -56,24 +56,20 @@ __global__ __launch_bounds__(kThreads, KT == 32 ? 2 : 1) void bwd_dq_kernel(BwdP
   const int qi = q0 + wave * 32 + col;
   const bool row_ok = qi < L;
   vec8 qf[kSteps], dof[kSteps];
-#pragma unroll
-  for (int kk = 0; kk < kSteps; kk++) {
-    const int d0 = 16 * kk + 8 * half;
-    qf[kk] = as_vec8<T>(load_row8<T, kLoad>(qb + (int64_t)qi * p.q.st, d0, D, row_ok));
-    dof[kk] = as_vec8<T>(load_row8<T, kLoad>(dob + (int64_t)qi * p.d_o.st, d0, D, row_ok));
-  }
+  load_operand<T, kLoad>(qf, make_row_source<T, kLoad>(qb, p.q.st, L, D), qi, half);
+  load_operand<T, kLoad>(dof, make_row_source<T, kLoad>(dob, p.d_o.st, L, D), qi, half);
   float drem = 0.f;
   if (row_ok && p.d_rem.ptr)
     drem = (float)((const T*)p.d_rem.ptr)[tile.seq_id * p.d_rem.sb + head * p.d_rem.sh + (tok0 + qi) * p.d_rem.st];
   if (p.add_rem) {
     // The forward wrote o + rem * v: the gradient reaching rem is d_rem + d_o . v_i.
     float dot = 0.f;
+    vec8 vf[kSteps];
+    load_operand<T, kLoad>(vf, make_row_source<T, kLoad>(vb, p.v.st, L, D), qi, half);
 #pragma unroll
-    for (int kk = 0; kk < kSteps; kk++) {
-      const vec8 vv = as_vec8<T>(load_row8<T, kLoad>(vb + (int64_t)qi * p.v.st, 16 * kk + 8 * half, D, row_ok));
+    for (int kk = 0; kk < kSteps; kk++)
 #pragma unroll
-      for (int t = 0; t < 8; t++) dot = fmaf((float)dof[kk][t], (float)vv[t], dot);
-    }
+      for (int t = 0; t < 8; t++) dot = fmaf((float)dof[kk][t], (float)vf[kk][t], dot);
     drem += dot + other_half(dot, half);
   }
   // The dK/dV kernel reads the gradient of rem back from this fp32 plane (one value per row).
@@ -95,19 +91,18 @@ __global__ __launch_bounds__(kThreads, KT == 32 ? 2 : 1) void bwd_dq_kernel(BwdP
 #pragma unroll
     for (int r = 0; r < 16; r++) dqacc[dt][r] = 0.f;
 
+  // Slots of sub-tile u in either plane: a uniform offset, then this lane's row within the tile.
+  auto slot_row = [&](int u) { return carry_offset(u, n_qt) + (q0 - kBlockQ * (u >> 2)); };
+  const uint32_t lrow = wave * 32 + col;
   // The forward's product above the next key tile (above its upper sub-tile), fetched one tile ahead.
-  // sub-tile whose upper edge is the upper edge of key tile t, and the first row that owns slots for tile t
-  auto carry_slot = [&](int t) {
-    const int u = NT == 2 ? 2 * t + 1 : t;
-    return carry_offset(u, n_qt) + (qi - kBlockQ * (u >> 2));
-  };
+  auto product_above = [&](int t) { return (carry + slot_row(NT == 2 ? 2 * t + 1 : t))[lrow]; };
   float n_prod = 1.f;
   const RowSource<T> ksrc = make_row_source<T, kLoad>(kb, p.k.st, L, D), vsrc = make_row_source<T, kLoad>(vb, p.v.st, L, D);
   TileCopy<T, DH, KT, kLoad> ck, cv;
   if (n_kt > 0) {
     ck.load(ksrc, 0);
     cv.load(vsrc, 0);
-    n_prod = carry[carry_slot(0)];
+    n_prod = product_above(0);
   }
   for (int jt = 0; jt < n_kt; ++jt) {
     const int j0 = jt * KT;
@@ -120,15 +115,13 @@ __global__ __launch_bounds__(kThreads, KT == 32 ? 2 : 1) void bwd_dq_kernel(BwdP
       const int jn = j0 + KT;
       ck.load(ksrc, jn);
       cv.load(vsrc, jn);
-      n_prod = carry[carry_slot(jt + 1)];
+      n_prod = product_above(jt + 1);
     }
     // For the key-stationary kernel: C just below each 32-key sub-tile, for every row of the tile.
     const int u_lo = NT == 2 ? 2 * jt : jt;
-    const int64_t slot_lo = carry_offset(u_lo, n_qt) + (qi - kBlockQ * (u_lo >> 2));
-    const int64_t slot_hi = carry_offset(u_lo + 1, n_qt) + (qi - kBlockQ * (u_lo >> 2));     // NT == 2 only
-    if (half == 0) prefix_out[slot_lo] = prefix;
+    if (half == 0) (prefix_out + slot_row(u_lo))[lrow] = prefix;
     if (j0 > w_last - 1 + ac) {
-      if (NT == 2 && half == 0) prefix_out[slot_hi] = prefix;
+      if (NT == 2 && half == 0) (prefix_out + slot_row(u_lo + 1))[lrow] = prefix;
       continue;
     }
     const bool diagonal = (j0 + KT - 1) > (w_first - 1 + ac) || w_last >= L;
@@ -182,7 +175,7 @@ __global__ __launch_bounds__(kThreads, KT == 32 ? 2 : 1) void bwd_dq_kernel(BwdP
       bwd_tile_math<T, NT, false>(s, dp, p.scale_log2, diagonal, lim, half, drem, prod_in, prefix, pk, dzk, prod_lower,
                            prefix_upper, prefix);
     }
-    if (NT == 2 && half == 0) prefix_out[slot_hi] = prefix_upper;
+    if (NT == 2 && half == 0) (prefix_out + slot_row(u_lo + 1))[lrow] = prefix_upper;
 
     // dQ += dZ K: A = dZ from registers, B = K gathered down the keys.
 #pragma unroll

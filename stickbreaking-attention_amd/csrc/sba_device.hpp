@@ -177,7 +177,30 @@ __device__ __forceinline__ void place_operand(typename Elem<T>::vec8 (&x)[kSteps
   if (kLoad != kLoadPadded || (d & 7) == 0) return;
 #pragma unroll
   for (int kk = 0; kk < kSteps; kk++)
-    if (kk == (d >> 4)) x[kk] = as_vec8<T>(shift_down(__builtin_bit_cast(u32x4, x[kk]), padded_shift(16 * kk + 8 * half, d)));
+    x[kk] = as_vec8<T>(shift_down(__builtin_bit_cast(u32x4, x[kk]), padded_shift(16 * kk + 8 * half, d)));
+}
+
+// The same at once, in any of the three ways.
+template <typename T, int kLoad, int kSteps>
+__device__ __forceinline__ void load_operand(typename Elem<T>::vec8 (&x)[kSteps], const RowSource<T>& src, int row, int half) {
+  if (kLoad != kLoadScalar) {
+    request_operand<T, kLoad>(x, src, row, half);
+    place_operand<T, kLoad>(x, src.d, half);
+    return;
+  }
+#pragma unroll
+  for (int kk = 0; kk < kSteps; kk++) {
+    u32x4 v = {0, 0, 0, 0};
+    if (row < src.rows) {
+      const uint16_t* p = reinterpret_cast<const uint16_t*>(src.base + row * src.stride);
+#pragma unroll
+      for (int t = 0; t < 8; t++) {
+        const int d = 16 * kk + 8 * half + t;
+        if (d < src.d) v[t >> 1] |= (uint32_t)p[d] << (16 * (t & 1));
+      }
+    }
+    x[kk] = as_vec8<T>(v);
+  }
 }
 
 // Cooperative global -> register -> LDS copy of a [kRows x DH] tile of 16-bit elements, 16 bytes per access.
@@ -224,31 +247,6 @@ struct TileCopy {
           kLoad == kLoadPadded && __any(shift) ? shift_down(regs[i], shift) : regs[i];
   }
 };
-
-// Load 8 consecutive head_dim elements of one token row from global memory (zero beyond head_dim / when !valid).
-template <typename T, int kLoad>
-__device__ __forceinline__ u32x4 load_row8(const T* row, int d0, int d_valid, bool valid) {
-  u32x4 v = {0, 0, 0, 0};
-  if (valid) {
-    if (kLoad == kLoadAligned) {
-      v = *reinterpret_cast<const u32x4*>(row + d0);
-    } else if (kLoad == kLoadPadded) {
-      if (d0 < d_valid) {
-        typedef __attribute__((ext_vector_type(4), aligned(2))) uint32_t u32x4_any;
-        const int n = padded_shift(d0, d_valid);
-        v = shift_down(*reinterpret_cast<const u32x4_any*>(row + d0 - n), n);
-      }
-    } else {
-      uint16_t e[8];
-#pragma unroll
-      for (int t = 0; t < 8; t++) e[t] = (d0 + t < d_valid) ? reinterpret_cast<const uint16_t*>(row + d0)[t] : (uint16_t)0;
-      v[0] = e[0] | ((uint32_t)e[1] << 16); v[1] = e[2] | ((uint32_t)e[3] << 16);
-      v[2] = e[4] | ((uint32_t)e[5] << 16); v[3] = e[6] | ((uint32_t)e[7] << 16);
-    }
-  }
-  return v;
-}
-
 
 // Element-wise backward math of one 64-key tile for the 32 keys this lane owns (see the conventions above).
 //   s, dp     : S^T = K Q^T and dP^T = V dO^T accumulators (row tile mt, register r  <->  key 32*half + 16*mt + r)

@@ -30,6 +30,7 @@
 #include "sba_device.hpp"
 #include "sba_host.hpp"
 #include "sba_params.hpp"
+#include "sba_sched.hpp"
 
 #include <type_traits>
 
@@ -288,12 +289,17 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_f32_kernel(FwdParams p) {
   __shared__ __attribute__((aligned(16))) float lds[RowsF32Lds<DH, 1>::kFloats];      // Q rows and the waves' scratch, then the final sums
   __shared__ float xch[2][kWaves][32];
   __shared__ float rem_lds[32];
+  if ((int)blockIdx.x < p.sched.service) {
+    forward_service(p.sched, blockIdx.x);
+    return;
+  }
+  const int wg = blockIdx.x - p.sched.service, sub = wg % kF32Split;
   int head, slot;
-  xcd_head_tile(blockIdx.x / kF32Split, p.num_heads, &head, &slot);
-  const int sub = blockIdx.x % kF32Split;
-  if (slot >= p.counts[kCountQ]) {
-    int64_t r0, r1;
-    if (uncovered_rows(p.counts, slot, p.total_tokens, sub, kF32Rows, &r0, &r1)) {
+  xcd_head_tile(wg / kF32Split, p.num_heads, &head, &slot);
+  Tile tile;
+  int64_t r0, r1;
+  if (!forward_tile(p, slot, sub, kF32Rows, &tile, &r0, &r1)) {
+    if (r0 < r1) {
       zero_rows<float>(p.o, head, r0, r1, p.head_dim);      // rows of no sequence: o = rem = 0
       for (int64_t r = r0 + threadIdx.x; r < r1; r += kThreads) {
         ((float*)p.rem.ptr)[head * p.rem.sh + r * p.rem.st] = 0.f;
@@ -302,7 +308,6 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_f32_kernel(FwdParams p) {
     }
     return;
   }
-  const Tile tile = p.tiles[slot];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = lane >> 5, col = lane & 31;
   const int L = tile.seq_len, ac = p.attend_current, D = p.head_dim;
   const int q0 = tile.origin + sub * kF32Rows;
@@ -597,7 +602,7 @@ static hipError_t by_head_dim(int D, F&& f) {
 
 hipError_t launch_fwd_f32(const FwdParams& p, int max_tiles, hipStream_t stream) {
   return by_head_dim(p.head_dim, [&](auto dh, auto exact) {
-    hipLaunchKernelGGL((fwd_f32_kernel<decltype(dh)::value, decltype(exact)::value>), dim3((unsigned)(max_tiles * p.num_heads * kF32Split)),
+    hipLaunchKernelGGL((fwd_f32_kernel<decltype(dh)::value, decltype(exact)::value>), dim3((unsigned)(max_tiles * p.num_heads * kF32Split + p.sched.service)),
                        dim3(kThreads), 0, stream, p);
     return hipGetLastError();
   });

@@ -14,6 +14,7 @@
 // below 2^-126, and row_stat = log2(prod) is taken once per row at the end.
 #include "sba_device.hpp"
 #include "sba_params.hpp"
+#include "sba_sched.hpp"
 
 namespace sba {
 
@@ -31,11 +32,16 @@ __global__ __launch_bounds__(kThreads, kMinWaves) void fwd_kernel(FwdParams p) {
   __shared__ __attribute__((aligned(16))) T k_lds[KT * kRowStride];
   __shared__ __attribute__((aligned(16))) T v_lds[KT * kRowStride];
 
+  if (!kCarryOnly && (int)blockIdx.x < p.sched.service) {
+    forward_service(p.sched, blockIdx.x);
+    return;
+  }
   int head, slot;
-  xcd_head_tile(blockIdx.x, p.num_heads, &head, &slot);
-  if (slot >= p.counts[kCountQ]) {
-    int64_t r0, r1;
-    if (!kCarryOnly && uncovered_rows(p.counts, slot, p.total_tokens, 0, kBlockQ, &r0, &r1)) {      // rows of no sequence: o = rem = 0
+  xcd_head_tile(blockIdx.x - p.sched.service, p.num_heads, &head, &slot);
+  Tile tile;
+  int64_t r0, r1;
+  if (!forward_tile(p, slot, 0, kBlockQ, &tile, &r0, &r1)) {
+    if (!kCarryOnly && r0 < r1) {      // rows of no sequence: o = rem = 0
       zero_rows<T>(p.o, head, r0, r1, p.head_dim);
       for (int64_t r = r0 + threadIdx.x; r < r1; r += kThreads) {
         ((T*)p.rem.ptr)[head * p.rem.sh + r * p.rem.st] = (T)0;
@@ -44,7 +50,6 @@ __global__ __launch_bounds__(kThreads, kMinWaves) void fwd_kernel(FwdParams p) {
     }
     return;
   }
-  const Tile tile = p.tiles[slot];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, half = lane >> 5, col = lane & 31;
   const int L = tile.seq_len, q0 = tile.origin, ac = p.attend_current, D = p.head_dim;
 
@@ -55,9 +60,7 @@ __global__ __launch_bounds__(kThreads, kMinWaves) void fwd_kernel(FwdParams p) {
   // This lane's query row as the B operand of S^T = K Q^T: 8 consecutive head_dim elements per k-step.
   const int qi = q0 + wave * 32 + col;
   vec8 qf[kSteps];
-#pragma unroll
-  for (int kk = 0; kk < kSteps; kk++)
-    qf[kk] = as_vec8<T>(load_row8<T, kLoad>(qb + (int64_t)qi * p.q.st, 16 * kk + 8 * half, D, qi < L));
+  load_operand<T, kLoad>(qf, make_row_source<T, kLoad>(qb, p.q.st, L, D), qi, half);
 
   const int last_row = min(q0 + kBlockQ, L) - 1;
   const int last_key = last_row - 1 + ac;                    // last key any row of this tile can see
@@ -82,7 +85,10 @@ __global__ __launch_bounds__(kThreads, kMinWaves) void fwd_kernel(FwdParams p) {
   // The recorded products are read per 64-key tile by the backward kernels that sweep 64 keys at a time, whichever
   // forward variant ran: a 32-key sweep that ends on the lower half of such a tile also records the (empty) product
   // above the upper half.
-  if (NT == 1 && carry && half == 0 && (n_kt & 1)) carry[carry_offset(n_kt, n_qt) + (qi - kBlockQ * (n_kt >> 2))] = 1.f;
+  // Slots of sub-tile u: a uniform base and this lane's row within the tile.
+  const uint32_t lrow = wave * 32 + col;
+  auto carry_row = [&](int u) { return carry + carry_offset(u, n_qt) + (q0 - kBlockQ * (u >> 2)); };
+  if (NT == 1 && carry && half == 0 && (n_kt & 1)) carry_row(n_kt)[lrow] = 1.f;
   for (int jt = n_kt - 1; jt >= 0; --jt) {
     const int j0 = jt * KT;
     __syncthreads();
@@ -97,10 +103,9 @@ __global__ __launch_bounds__(kThreads, kMinWaves) void fwd_kernel(FwdParams p) {
     // For the backward: the product over the keys between the upper 32-key sub-tile and the row, for every row
     // of the tile (the lower sub-tile's value follows once this tile's upper half is known).
     const int u_hi = NT == 2 ? 2 * jt + 1 : jt;                // sub-tile at the upper edge of this tile
-    const int64_t cslot = qi - kBlockQ * (u_hi >> 2);
-    if (carry && half == 0) carry[carry_offset(u_hi, n_qt) + cslot] = prod;
+    if (carry && half == 0) carry_row(u_hi)[lrow] = prod;
     if (j0 > w_last - 1 + ac) {                               // nothing visible to this wave yet
-      if (NT == 2 && carry && half == 0) carry[carry_offset(u_hi - 1, n_qt) + cslot] = prod;
+      if (NT == 2 && carry && half == 0) carry_row(u_hi - 1)[lrow] = prod;
       continue;
     }
     const bool diagonal = (j0 + KT - 1) > (w_first - 1 + ac);
@@ -166,7 +171,7 @@ __global__ __launch_bounds__(kThreads, kMinWaves) void fwd_kernel(FwdParams p) {
     const float oth = other_half(run, half);
     // The upper half-wave holds the higher keys, which come first in the sweep.
     const float seed = half ? prod : prod * oth;
-    if (NT == 2 && carry && half == 0) carry[carry_offset(u_hi - 1, n_qt) + cslot] = seed;   // product above the lower sub-tile
+    if (NT == 2 && carry && half == 0) carry_row(u_hi - 1)[lrow] = seed;   // product above the lower sub-tile
     prod = (prod * oth) * run;
     if (kCarryOnly) continue;
 
@@ -229,12 +234,12 @@ __global__ __launch_bounds__(kThreads, kMinWaves) void fwd_kernel(FwdParams p) {
 
 template <typename T, bool kCarryOnly>
 static hipError_t launch_fwd_t(const FwdParams& p, int max_tiles, hipStream_t stream) {
-  const dim3 grid((unsigned)(max_tiles * p.num_heads)), block(kThreads);
+  const dim3 grid((unsigned)(max_tiles * p.num_heads + p.sched.service)), block(kThreads);
   if (p.load == kLoadAligned) {
     if (p.head_dim == 128) hipLaunchKernelGGL((fwd_kernel<T, 128, kLoadAligned, 32, 3, kCarryOnly>), grid, block, 0, stream, p);
     else hipLaunchKernelGGL((fwd_kernel<T, 64, kLoadAligned, 64, 2, kCarryOnly>), grid, block, 0, stream, p);
   } else if (p.load == kLoadPadded) {
-    if (p.head_dim > 64) hipLaunchKernelGGL((fwd_kernel<T, 128, kLoadPadded, 32, 2, kCarryOnly>), grid, block, 0, stream, p);
+    if (p.head_dim > 64) hipLaunchKernelGGL((fwd_kernel<T, 128, kLoadPadded, 32, 3, kCarryOnly>), grid, block, 0, stream, p);
     else hipLaunchKernelGGL((fwd_kernel<T, 64, kLoadPadded, 64, 2, kCarryOnly>), grid, block, 0, stream, p);
   } else {
     if (p.head_dim > 64) hipLaunchKernelGGL((fwd_kernel<T, 128, kLoadScalar, 64, 2, kCarryOnly>), grid, block, 0, stream, p);

@@ -1,0 +1,17 @@
+// What the torch host layer uses of libsba.so besides the C ABI: a forward that prepares the schedule of the backward that
+// follows it (tile lists, cursors, cleared flags), so that the backward needs no scheduler launch of its own.
+#pragma once
+#include "../../include/sba.h"
+
+namespace sba {
+
+// Sizes: of the schedule, of the backward's workspace besides it, and of `carry`.
+int prepared_bytes(const SbaArgs* a, size_t* sched_bytes, size_t* rest_bytes, size_t* carry_bytes);
+// sba_fwd with the schedule in a->workspace (sched_bytes of it).
+int forward_prepared(const SbaArgs* a);
+// Whether the backward these arguments describe can run on the schedule its forward prepared.
+bool prepared_fits(const SbaArgs* a);
+// sba_bwd on that schedule, with the rest in a->workspace.  The schedule serves ONE backward: its cursors are used up.
+int backward_prepared(const SbaArgs* a, void* sched);
+
+}  // namespace sba

@@ -43,7 +43,6 @@ struct SchedParams {
   int32_t fixed_len;       // L in fixed-length mode
   int64_t total_tokens;    // T: rows of the packed token axis (L in fixed-length mode)
   int64_t carry_capacity;  // carry slots reserved per head
-  int32_t attend_current;
   int32_t want_key_tiles;  // backward: also build the key-tile list
   int32_t want_carry_base; // also lay out the per-sequence carry offsets
   Tile* q_tiles;           // query tiles (kBlockQ rows), heaviest first
@@ -56,7 +55,11 @@ struct SchedParams {
   int32_t key_tile;        // keys per key tile (a multiple of 32; what the dK/dV kernel that will run sweeps)
   uint32_t* zero_fill;     // optional: 16-byte aligned region cleared by the launch (the one-kernel backward's flags
   int64_t zero_bytes;      // and tags start every call at zero), a multiple of 16 bytes
+  int32_t service;         // workgroups at the head of a forward launch that schedule and clear (0: a scheduler launch did)
 };
+// Most sequences of a packed batch whose tiles the forward's workgroups derive themselves (one lane each).  The derivation
+// takes 12 vector-ALU instructions per sequence and wave, 1.5 us at 64, and replaces a launch of 8 us in front of the forward.
+constexpr int kInlineSeqs = 64;
 
 struct FwdParams {
   TensorRef q, k, v, o;
@@ -66,8 +69,9 @@ struct FwdParams {
   float* carry;                // optional [head][slot]: running product per (row, key tile)
   const int64_t* carry_base;
   int64_t carry_head_stride;
-  const Tile* tiles;
+  const Tile* tiles;           // NULL: the workgroups derive their tiles from `sched`
   const int32_t* counts;
+  SchedParams sched;
   int32_t num_heads, head_dim;
   float scale_log2;            // logit_scale * log2(e)
   int32_t attend_current;

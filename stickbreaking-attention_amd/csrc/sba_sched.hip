@@ -10,17 +10,12 @@
 // the cheap tiles of the short sequences.  It also lays out the per-(row, 32-key sub-tile) carries per sequence.
 #include "sba_device.hpp"
 #include "sba_params.hpp"
+#include "sba_sched.hpp"
 
 namespace sba {
 
 constexpr int kBins = 4096;          // sequence length classes (query tiles per sequence, saturating)
 constexpr int kSchedThreads = 1024;
-
-// Returns false for an unusable cu_seqlens entry (see seq_span); the span is then empty.
-__device__ __forceinline__ bool seq_bounds(const SchedParams& p, int s, int* start, int* len) {
-  if (p.cu == nullptr) { *start = 0; *len = p.fixed_len; return true; }
-  return seq_span(p.cu, p.cu_is_int64, p.cu_has_leading_zero, s, p.total_tokens, start, len);
-}
 
 // Exclusive prefix sum over bins taken from the heaviest bin downwards; bins[] becomes the start offsets.
 __device__ void descending_offsets(int* bins, int* scratch) {
@@ -156,14 +151,9 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
 
 }
 
-hipError_t launch_sched(const SchedParams& p, hipStream_t stream) {
-  // One workgroup schedules; with a region to clear, one more per 256 KiB of it (at most 64) clears alongside.
-  int helpers = 0;
-  if (p.zero_fill && p.zero_bytes > 0) {
-    helpers = (int)((p.zero_bytes + (256 << 10) - 1) / (256 << 10));
-    if (helpers > 64) helpers = 64;
-  }
-  hipLaunchKernelGGL(sched_kernel, dim3(1 + helpers), dim3(kSchedThreads), 0, stream, p);
+// One workgroup schedules; `clear_wgs` more clear p.zero_fill alongside.
+hipError_t launch_sched(const SchedParams& p, int clear_wgs, hipStream_t stream) {
+  hipLaunchKernelGGL(sched_kernel, dim3(1 + clear_wgs), dim3(kSchedThreads), 0, stream, p);
   return hipGetLastError();
 }
 

@@ -11,6 +11,7 @@
 #include <ATen/ops/empty_like.h>
 #include <ATen/ops/zeros_like.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 
 #include <atomic>
@@ -18,6 +19,7 @@
 #include <optional>
 
 #include "../../include/sba.h"
+#include "sba_internal.hpp"
 
 namespace {
 
@@ -119,41 +121,46 @@ SbaArgs base_args(const Call& c, const Tensor& q) {
 
 Tensor bytes(size_t n, const Tensor& like) { return at::empty({(int64_t)n}, like.options().dtype(at::kByte)); }
 
-struct Outputs { Tensor o, rem, row_stat, carry; };
+struct Outputs {
+  Tensor o, rem;
+  Tensor state;      // one allocation: {schedule, row_stat, carry}; kept for the backward
+};
+size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
+size_t row_stat_bytes(const Tensor& q) { return align256(q.numel() / q.size(-1) * 4); }
 
-Outputs run_forward(const Call& c, const Tensor& q, const Tensor& k, const Tensor& v, bool want_carry) {
+// `for_backward`: a backward will follow; `want_carry`: it starts from recorded products instead of rebuilding them.
+Outputs run_forward(const Call& c, const Tensor& q, const Tensor& k, const Tensor& v, bool for_backward, bool want_carry) {
   const c10::DeviceGuard guard(q.device());
   SbaArgs a = base_args(c, q);
   Outputs out;
   out.o = at::empty_like(q);
   if (out.o.stride(-1) != 1) out.o = at::empty(q.sizes(), q.options());
   out.rem = at::empty(q.sizes().slice(0, q.dim() - 1), q.options());
-  out.row_stat = at::empty(out.rem.sizes(), q.options().dtype(at::kFloat));
   // No products kept: a backward, if one follows, rebuilds them, and the forward's scheduler checks their capacity as that
   // backward's will (both passes void, or neither).
   a.recompute_carry = !want_carry && a.dtype != SBA_F32;
-  size_t ws_bytes = 0, carry_bytes = 0;
-  check(sba_workspace_bytes(&a, &ws_bytes, nullptr, &carry_bytes), "sba_workspace_bytes");
-  const Tensor ws = bytes(ws_bytes, q);
-  if (want_carry) out.carry = bytes(carry_bytes, q);
-  if (c.flags & kPoison) {
-    poison(ws);
-    if (want_carry) poison(out.carry);
-  }
+  size_t sched = 0, rest = 0, carry = 0;
+  if (for_backward) check(sba::prepared_bytes(&a, &sched, &rest, &carry), "sba_workspace_bytes");
+  else check(sba_workspace_bytes(&a, &sched, nullptr, nullptr), "sba_workspace_bytes");
+  const size_t stat = row_stat_bytes(q);
+  out.state = bytes(sched + stat + (want_carry ? carry : 0), q);
+  if (c.flags & kPoison) poison(out.state);
+  char* const base = (char*)out.state.data_ptr();
   a.q = ref<SbaTensor>(q, c.fixed); a.k = ref<SbaTensor>(k, c.fixed); a.v = ref<SbaTensor>(v, c.fixed);
   a.o = ref<SbaTensor>(out.o, c.fixed);
   a.rem = ref<SbaVector>(out.rem, c.fixed);
-  a.row_stat = (float*)out.row_stat.data_ptr();
-  a.carry = want_carry ? (float*)out.carry.data_ptr() : nullptr;
-  a.workspace = ws.data_ptr();
-  a.workspace_bytes = ws_bytes;
-  check(sba_fwd(&a), "sba_fwd");
-  if (c.flags & kDebugCheck) check_status(ws, "sba_fwd");
+  a.row_stat = (float*)(base + sched);
+  a.carry = want_carry ? (float*)(base + sched + stat) : nullptr;
+  a.workspace = base;
+  a.workspace_bytes = sched;
+  check(for_backward ? sba::forward_prepared(&a) : sba_fwd(&a), "sba_fwd");
+  if (c.flags & kDebugCheck) check_status(out.state, "sba_fwd");
   return out;
 }
 
+// `state` as the forward left it; `fresh`: no backward has run on its schedule yet.
 variable_list run_backward(const Call& c, Tensor d_o, Tensor d_rem, const Tensor& q, const Tensor& k, const Tensor& v,
-                           const Tensor& carry, const Tensor& row_stat) {
+                           const Tensor& state, bool have_carry, bool fresh) {
   const c10::DeviceGuard guard(q.device());
   if (!d_o.defined()) d_o = at::zeros_like(q);
   require_gpu(d_o);
@@ -169,25 +176,33 @@ variable_list run_backward(const Call& c, Tensor d_o, Tensor d_rem, const Tensor
   a.d_o = ref<SbaTensor>(d_o, c.fixed);
   a.d_rem = ref<SbaVector>(d_rem, c.fixed);
   a.dq = ref<SbaTensor>(dq, c.fixed); a.dk = ref<SbaTensor>(dk, c.fixed); a.dv = ref<SbaTensor>(dv, c.fixed);
-  a.row_stat = row_stat.defined() ? (float*)row_stat.data_ptr() : nullptr;
-  a.carry = carry.defined() ? (float*)carry.data_ptr() : nullptr;
-  a.recompute_carry = !carry.defined();      // the forward kept no products: rebuild them in the backward's workspace
-  size_t ws_bytes = 0;
-  check(sba_workspace_bytes(&a, nullptr, &ws_bytes, nullptr), "sba_workspace_bytes");
+  a.recompute_carry = !have_carry;      // the forward kept no products: rebuild them in the backward's workspace
+  size_t sched_bytes = 0, rest_bytes = 0, carry_bytes = 0;
+  check(sba::prepared_bytes(&a, &sched_bytes, &rest_bytes, &carry_bytes), "sba_workspace_bytes");
+  char* const base = (char*)state.data_ptr();
+  a.row_stat = (float*)(base + sched_bytes);
+  a.carry = have_carry ? (float*)(base + sched_bytes + row_stat_bytes(q)) : nullptr;
   const int64_t limit = g_bwd_limit.load(std::memory_order_relaxed);
-  if (limit >= 0 && ws_bytes > (size_t)limit) {
-    SbaArgs one = a;                          // the smallest workspace the library accepts is the one of a single head
-    one.num_heads = 1;
-    size_t one_bytes = 0;
-    check(sba_workspace_bytes(&one, nullptr, &one_bytes, nullptr), "sba_workspace_bytes");
-    ws_bytes = std::max((size_t)limit, one_bytes);
+  // The forward's schedule serves one backward.  Under graph capture it may be replayed more often than the forward.
+  const bool prepared = fresh && limit < 0 && sba::prepared_fits(&a) &&
+                        c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None;
+  size_t ws_bytes = rest_bytes;
+  if (!prepared) {
+    check(sba_workspace_bytes(&a, nullptr, &ws_bytes, nullptr), "sba_workspace_bytes");
+    if (limit >= 0 && ws_bytes > (size_t)limit) {
+      SbaArgs one = a;                        // the smallest workspace the library accepts is the one of a single head
+      one.num_heads = 1;
+      size_t one_bytes = 0;
+      check(sba_workspace_bytes(&one, nullptr, &one_bytes, nullptr), "sba_workspace_bytes");
+      ws_bytes = std::max((size_t)limit, one_bytes);
+    }
   }
   const Tensor ws = bytes(ws_bytes, q);
   if (c.flags & kPoison) poison(ws);
   a.workspace = ws.data_ptr();
   a.workspace_bytes = ws_bytes;
-  check(sba_bwd(&a), "sba_bwd");
-  if (c.flags & kDebugCheck) check_status(ws, "sba_bwd");
+  check(prepared ? sba::backward_prepared(&a, base) : sba_bwd(&a), "sba_bwd");
+  if (c.flags & kDebugCheck) check_status(prepared ? state : ws, "sba_bwd");
   return {dq, dk, dv};
 }
 
@@ -195,11 +210,12 @@ struct StickBreaking : torch::autograd::Function<StickBreaking> {
   static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Call* call,
                                bool save_carry) {
     const Call& c = *call;
-    const Outputs out = run_forward(c, q, k, v, save_carry);
+    const Outputs out = run_forward(c, q, k, v, true, save_carry);
     ctx->set_materialize_grads(false);
-    ctx->save_for_backward({q, k, v, c.cu, out.carry, c.add_remainder ? out.row_stat : Tensor()});
+    ctx->save_for_backward({q, k, v, c.cu, out.state});
+    ctx->saved_data["fresh"] = true;
     ctx->saved_data["call"] = c10::IValue(std::vector<int64_t>{c.fixed, c.leading_zero, c.attend_current, c.add_remainder,
-                                                               c.max_seqlen, c.carry_slots, c.flags});
+                                                               c.max_seqlen, c.carry_slots, c.flags, save_carry});
     ctx->saved_data["scale"] = c.logit_scale;
     return {out.o, out.rem};
   }
@@ -211,7 +227,9 @@ struct StickBreaking : torch::autograd::Function<StickBreaking> {
     c.max_seqlen = n[4]; c.carry_slots = n[5]; c.flags = n[6];
     c.logit_scale = ctx->saved_data["scale"].toDouble();
     c.cu = s[3];
-    variable_list g = run_backward(c, grads[0], grads[1], s[0], s[1], s[2], s[4], s[5]);
+    c10::IValue& fresh = ctx->saved_data["fresh"];
+    variable_list g = run_backward(c, grads[0], grads[1], s[0], s[1], s[2], s[4], n[7], fresh.toBool());
+    fresh = false;
     g.resize(5);      // call, save_carry
     return g;
   }
@@ -228,7 +246,7 @@ std::tuple<Tensor, Tensor> attention(const Call& c, Tensor q, Tensor k, Tensor v
     const variable_list out = StickBreaking::apply(q, k, v, &c, save_carry || q.scalar_type() == at::kFloat);
     return {out[0], out[1]};
   }
-  const Outputs out = run_forward(c, q, k, v, false);
+  const Outputs out = run_forward(c, q, k, v, false, false);
   return {out.o, out.rem};
 }
 

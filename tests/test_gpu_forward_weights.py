@@ -1,0 +1,30 @@
+"""The forward's two ways through a tile's weights: groups of keys whose odds multiply up to any size (the wave then takes them
+one by one), next to tame ones in the same wave, against the float64 oracle."""
+import pytest
+import torch
+
+from oracle import sb_oracle as orc
+from test_gpu_parity import NAMES, run_varlen, tol_check
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("D", [64, 80, 128])
+@pytest.mark.parametrize("low,high", [(-20.0, 20.0), (15.0, 30.0), (-200.0, 200.0), (50.0, 400.0)])
+def test_logits_of_any_size(gpu_device, D, low, high):
+    lengths = [33, 200]
+    T, H = sum(lengths), 2
+    g = torch.Generator().manual_seed(int(high) + D)
+    # one column carries the logits: z_ij = k_j for every row, so that every size of odds meets every other
+    q, k, v, do = (torch.zeros(H, T, D), 0.01 * torch.randn(H, T, D, generator=g), *(torch.randn(H, T, D, generator=g) for _ in range(2)))
+    q[..., 0] = 1
+    k[..., 0] = low + (high - low) * torch.rand(H, T, generator=g)
+    drem = torch.randn(H, T, generator=g)
+    host = [t.bfloat16() for t in (q, k, v, do, drem)]
+    cu = torch.tensor([33, 233], dtype=torch.int32)
+    ref = orc.varlen_stream(*host[:3], cu, do=host[3], drem=host[4], dtype=torch.float64, scale=1.0)
+    dev = [t.to(gpu_device) for t in host]
+    got = run_varlen(dev[0], dev[1], dev[2], cu.to(gpu_device), lengths, False, False, dev[3], dev[4], scale=1.0)
+    for n, a, b in list(zip(NAMES, got, ref))[:2]:
+        tol_check(n, a, b, torch.bfloat16, f"logits {low}..{high}")
+    assert all(torch.isfinite(t).all() for t in got)

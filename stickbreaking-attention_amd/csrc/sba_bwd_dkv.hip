@@ -670,7 +670,7 @@ __global__ __launch_bounds__(kDkv4Threads) void bwd_dkv4_kernel(BwdParams p) {
         // Vector-ALU instructions per MFMA.  The group solver is greedy: with a budget a little below the block's
         // instruction count it puts the last MFMAs back to back and the rest of the math behind them, so the values
         // were checked in the generated code (both element types, both copies of the unrolled step).
-        constexpr int kGap = (kDiag ? 270 : 240) / (2 * kSteps);
+        constexpr int kGap = kDiag ? 14 : 12;                  // (255 and 220 instructions)
         constexpr int kAlu = 0x402;                            // scheduling-group mask: vector ALU incl. transcendentals
         const T* q_lds = lds + Lds::kQ + st * 2 * Lds::kQdoTile;
         const T* do_lds = q_lds + Lds::kQdoTile;

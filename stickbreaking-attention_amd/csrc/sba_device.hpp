@@ -275,40 +275,45 @@ __device__ __forceinline__ void bwd_tile_math_impl(const f32x16 (&s)[NT], const 
     if (kDiagonal) x = (R < lim) ? x : -INFINITY;
     const float omb = fast_rcp(1.f + fast_exp2(x));
     beta[R] = 1.f - omb;
-    pe[R] = run;           // product over this lane's higher keys
     run *= omb;
+    pe[R] = run;           // product over this key and this lane's higher keys
   }
   const float oth = other_half(run, half);
   prod_lower = prod_in * (half ? run : oth);               // product above the lower half-wave's keys
   const float seed = half ? prod_in : prod_lower;           // the upper half-wave holds the higher keys
-  // Running C as if this lane's keys were preceded only by the keys below the tile; the upper half-wave's
-  // share of the lower half-wave's total is added afterwards (fixup).
-  float acc = prefix_in;
-  float dz[N];
-  const float neg_drem_seed = -drem * seed;
+  // Let D = drem + (sum of g over this lane's keys up to j) / (product above key j).  Then, with u_j = dP_j - D_{j-1},
+  //   D_j = D_{j-1} + sigma_j u_j        g_j - sigma_j (sum of g over the lane's keys up to j) = sigma_j (product below key j) u_j
+  // (D is a running weighted mean of drem and dP, so it neither grows nor cancels), and with C0 = C below the lane's keys
+  //   dz_j = sigma_j (seed pe_j u_j - C0)
+  // which is 4 instructions per key where summing g and correcting by sigma C takes 6.  The vector ALU is what bounds the
+  // backward kernels (87 % busy in dQ at head_dim 64): dQ 32 heads x 2 x 4096 x 64 345 -> 320 us, see the kernels for the rest.
+  float u[N];
+  float D = kNeedP ? drem : drem * seed;                    // (kNeedP: P wants seed * pe anyway; else D is kept times seed)
+  const float D0 = D;
 #pragma unroll
   for (int R = 0; R < N; R++) {
-    float g;
-    if (kNeedP) {
-      const float a = beta[R] * (pe[R] * seed);
-      g = a * (dp[R >> 4][R & 15] - drem);
-      pe[R] = a;
-    } else {
-      // A is not wanted for itself: the seed goes into (dP - drem) with one fma instead of a multiply of its own
-      g = (beta[R] * pe[R]) * fmaf(dp[R >> 4][R & 15], seed, neg_drem_seed);
-    }
-    acc += g;
-    dz[R] = g - beta[R] * acc;
+    u[R] = kNeedP ? dp[R >> 4][R & 15] - D : fmaf(dp[R >> 4][R & 15], seed, -D);
+    D = fmaf(beta[R], u[R], D);
   }
-  const float tot = acc - prefix_in;
+  const float tot = kNeedP ? (D - D0) * seed : D - D0;
   const float oth_g = other_half(tot, half);
-  const float fixup = half ? oth_g : 0.f;                   // the lower half-wave holds the lower keys
+  const float below = prefix_in + (half ? oth_g : 0.f);     // the lower half-wave holds the lower keys
   prefix_upper = prefix_in + (half ? oth_g : tot);          // C just below the upper half-wave's keys
-  prefix_out = acc + oth_g;
+  prefix_out = prefix_in + (tot + oth_g);
+  float a[N];
+  if (kNeedP) {
+    float above = seed;
+#pragma unroll
+    for (int R = N - 1; R >= 0; --R) {
+      a[R] = beta[R] * above;
+      above = pe[R] * seed;
+      pe[R] = above;
+    }
+  }
 #pragma unroll
   for (int R = 0; R < N; R += 2) {
-    pk[R >> 1] = kNeedP ? pack2<T>(pe[R], pe[R + 1]) : 0u;
-    dzk[R >> 1] = pack2<T>(dz[R] - beta[R] * fixup, dz[R + 1] - beta[R + 1] * fixup);
+    pk[R >> 1] = kNeedP ? pack2<T>(a[R], a[R + 1]) : 0u;
+    dzk[R >> 1] = pack2<T>(beta[R] * fmaf(pe[R], u[R], -below), beta[R + 1] * fmaf(pe[R + 1], u[R + 1], -below));
   }
 }
 

@@ -277,7 +277,7 @@ static hipError_t launch_fwd_t(const FwdParams& p, int max_tiles, hipStream_t st
     if (p.head_dim == 128) hipLaunchKernelGGL((fwd_kernel<T, 128, kLoadAligned, 32, 3, kCarryOnly>), grid, block, 0, stream, p);
     else hipLaunchKernelGGL((fwd_kernel<T, 64, kLoadAligned, 64, 2, kCarryOnly>), grid, block, 0, stream, p);
   } else if (p.load == kLoadPadded) {
-    if (p.head_dim > 64) hipLaunchKernelGGL((fwd_kernel<T, 128, kLoadPadded, 32, 2, kCarryOnly>), grid, block, 0, stream, p);
+    if (p.head_dim > 64) hipLaunchKernelGGL((fwd_kernel<T, 128, kLoadPadded, 32, 3, kCarryOnly>), grid, block, 0, stream, p);
     else hipLaunchKernelGGL((fwd_kernel<T, 64, kLoadPadded, 64, 2, kCarryOnly>), grid, block, 0, stream, p);
   } else {
     if (p.head_dim > 64) hipLaunchKernelGGL((fwd_kernel<T, 128, kLoadScalar, 64, 2, kCarryOnly>), grid, block, 0, stream, p);

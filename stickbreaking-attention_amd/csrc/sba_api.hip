@@ -16,6 +16,9 @@ hipError_t launch_bwd_dkv(const BwdParams& p, int dtype_is_f16, int max_tiles, h
 int dkv_key_tile(const BwdParams& p);
 bool chain_supported(const BwdParams& p);
 hipError_t launch_bwd_chain(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
+hipError_t launch_fwd_split(const FwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
+hipError_t launch_bwd_dq_split(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
+hipError_t launch_bwd_dkv_split(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
 hipError_t launch_fwd_f32(const FwdParams& p, int max_tiles, hipStream_t stream);
 hipError_t launch_bwd_f32(const BwdParams& p, int max_q_tiles, int max_k_tiles, hipStream_t stream);
 }  // namespace sba
@@ -148,6 +151,26 @@ int row_load(const SbaArgs* a, const SbaTensor* const (&tensors)[N]) {
   }
   return load;
 }
+// Whether a call is too small to fill the chip with tiles of 128 query rows (and key tiles): its kernels then split the keys
+// (rows) of a workgroup's rows (keys) over the waves.  By rows times heads, at which the time of the longest row in an unsplit
+// workgroup (a third of which remains when it is split) meets the throughput of the split kernels, which stage K and V four
+// times as often.  Measured on 256 compute units, split / unsplit us:
+//   rows x heads          8 K         16 K        32 K        64 K
+//   head_dim 64   fwd   23.5 / 43.8  24.8 / 44.4  30 / 46    52 / 50     (2048 tokens; 8192: 83 / 162 up to 16 K, 162 / 176 at 64 K)
+//                 dQ    28.8 / 61    29.9 / 62    43 / 63    78 / 69
+//   head_dim 128  fwd   34.7 / 61    39 / 62      60 / 64   112 / 73     (8192: 128 / 230, 131 / 236, 189 / 238, 325 / 262)
+//                 dQ    39 / 79      47 / 80      91 / 84   185 / 94
+bool few_tiles(const SbaArgs* a, int load) {
+  if (a->dtype == SBA_F32 || load == sba::kLoadScalar) return false;
+  const int64_t rows = a->total_tokens * (a->cu_seqlens ? 1 : a->num_seqs) * a->num_heads;
+  return rows < (a->head_dim > 64 ? 30 << 10 : 60 << 10);
+}
+// The same for dK/dV: below, head_dim up to 64 splits the rows over the waves (130 K rows x heads: 542 / 565 us at 8192
+// tokens), wider ones take key tiles of 64 instead of 128 (64 K: 113 / 119 at 2048, 354 / 410 at 8192; 130 K: 672 / 657).
+bool few_key_tiles(const SbaArgs* a, int load) {
+  if (a->dtype == SBA_F32 || load == sba::kLoadScalar) return false;
+  return a->total_tokens * (a->cu_seqlens ? 1 : a->num_seqs) * a->num_heads < 100 << 10;
+}
 int check_tensor(const SbaTensor& t, bool required, bool fixed) {
   if (!t.ptr) return required ? SBA_ERR_NULL : SBA_OK;
   if (t.stride_token < 0 || t.stride_head < 0 || (fixed && t.stride_batch < 0)) return SBA_ERR_STRIDE;
@@ -196,11 +219,12 @@ int clear_wgs(const sba::SchedParams& sp) {
 }
 
 // Keys per key tile of the backward that will follow a forward, as far as the forward's tensors tell.
-int expected_key_tile(const SbaArgs* a) {
+int expected_key_tile(const SbaArgs* a, const Layout& L) {
   if (a->dtype == SBA_F32) return kBlockK;
   sba::BwdParams p{};
   p.head_dim = a->head_dim;
   p.load = row_load(a, {&a->q, &a->k, &a->v});
+  p.split = L.chain_zero_bytes == 0 && few_key_tiles(a, p.load);
   return sba::dkv_key_tile(p);
 }
 
@@ -308,7 +332,7 @@ int fwd_on(const SbaArgs* a, char* ws, size_t ws_bytes, bool ws_is_static, bool 
   // The carry offsets are laid out (and the capacity checked) when products are recorded, and also when the backward
   // will rebuild them: both passes then agree on whether the schedule stands.
   sba::FwdParams p{};
-  p.sched = sched_params(a, ws, L, for_backward, a->carry != nullptr || a->recompute_carry, for_backward ? expected_key_tile(a) : kBlockK);
+  p.sched = sched_params(a, ws, L, for_backward, a->carry != nullptr || a->recompute_carry, for_backward ? expected_key_tile(a, L) : kBlockK);
   if (fixed || a->num_seqs <= sba::kInlineSeqs) {
     p.sched.service = 1 + clear_wgs(p.sched);
   } else {
@@ -335,7 +359,8 @@ int fwd_on(const SbaArgs* a, char* ws, size_t ws_bytes, bool ws_is_static, bool 
   hipEvent_t* ev = (hipEvent_t*)a->trace_events;
   if (ev && hipEventRecord(ev[0], stream) != hipSuccess) return SBA_ERR_LAUNCH;
   hipError_t e = (a->dtype == SBA_F32) ? sba::launch_fwd_f32(p, (int)L.max_q_tiles, stream)
-                                       : sba::launch_fwd(p, a->dtype == SBA_F16, (int)L.max_q_tiles, stream);
+                 : few_tiles(a, p.load)  ? sba::launch_fwd_split(p, a->dtype == SBA_F16, (int)L.max_q_tiles, stream)
+                                         : sba::launch_fwd(p, a->dtype == SBA_F16, (int)L.max_q_tiles, stream);
   if (e != hipSuccess) return SBA_ERR_LAUNCH;
   if (ev && hipEventRecord(ev[1], stream) != hipSuccess) return SBA_ERR_LAUNCH;
   return SBA_OK;
@@ -426,6 +451,7 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* 
   p.max_tiles = (int32_t)L.max_q_tiles;
   p.total_tokens = a->total_tokens;
   p.load = bwd_load(a);
+  p.split = L.chain_zero_bytes == 0 && few_key_tiles(a, p.load);
   // One kernel (the key tiles of a sequence hand C and partial dQ to each other) where it applies, else dQ then dK/dV.
   const bool chain = bwd_is_chained(a, L);
   if (chain) {
@@ -476,9 +502,13 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* 
     if (ev && last && hipEventRecord(ev[2], stream) != hipSuccess) return SBA_ERR_LAUNCH;
     return SBA_OK;
   }
-  if (sba::launch_bwd_dq(p, a->dtype == SBA_F16, (int)L.max_q_tiles, stream) != hipSuccess) return SBA_ERR_LAUNCH;
+  const bool f16 = a->dtype == SBA_F16;
+  if ((few_tiles(a, p.load) ? sba::launch_bwd_dq_split(p, f16, (int)L.max_q_tiles, stream) : sba::launch_bwd_dq(p, f16, (int)L.max_q_tiles, stream)) != hipSuccess)
+    return SBA_ERR_LAUNCH;
   if (ev && last && hipEventRecord(ev[1], stream) != hipSuccess) return SBA_ERR_LAUNCH;
-  if (sba::launch_bwd_dkv(p, a->dtype == SBA_F16, (int)L.max_k_tiles, stream) != hipSuccess) return SBA_ERR_LAUNCH;
+  if ((p.split && a->head_dim <= 64 ? sba::launch_bwd_dkv_split(p, f16, (int)L.max_k_tiles, stream)
+                                    : sba::launch_bwd_dkv(p, f16, (int)L.max_k_tiles, stream)) != hipSuccess)
+    return SBA_ERR_LAUNCH;
   if (ev && last && hipEventRecord(ev[2], stream) != hipSuccess) return SBA_ERR_LAUNCH;
   return SBA_OK;
 }
@@ -570,7 +600,8 @@ bool prepared_fits(const SbaArgs* a) {
   BwdParams p{};
   p.head_dim = a->head_dim;
   p.load = bwd_load(a);
-  return a->dtype == SBA_F32 || dkv_key_tile(p) == expected_key_tile(a);
+  p.split = L.chain_zero_bytes == 0 && few_key_tiles(a, p.load);
+  return a->dtype == SBA_F32 || dkv_key_tile(p) == expected_key_tile(a, L);
 }
 
 int backward_prepared(const SbaArgs* a, void* sched) { return bwd_pass(a, a->num_heads, true, true, (char*)sched); }

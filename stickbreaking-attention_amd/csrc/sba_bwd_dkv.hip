@@ -109,7 +109,7 @@ __global__ __launch_bounds__(kThreads) void bwd_dkv_kernel(BwdParams p) {
     const int qi = w_first + col;
     const bool row_ok = qi < L;
     uint32_t pk[16], dzk[16];
-    if (j0 > min(w_last, L - 1) - 1 + ac) {
+    if (w_first >= L || j0 > min(w_last, L - 1) - 1 + ac) {
       // no row of this wave that belongs to the sequence sees the tile: contributes zeros
 #pragma unroll
       for (int i = 0; i < 16; i++) { pk[i] = 0; dzk[i] = 0; }
@@ -343,7 +343,7 @@ __global__ __launch_bounds__(kDkv3Threads) void bwd_dkv3_kernel(BwdParams p) {
         // Skipped unless a row of the SEQUENCE sees the sub-tile: the forward and the dQ kernel record the per-row
         // scalars only for sub-tiles that hold a key visible to the last row of their query tile, so a sub-tile that
         // merely lies below rows beyond the sequence's end has no recorded values to start from.
-        if (jb > min(w_last, L - 1) - 1 + ac) {
+        if (w_first >= L || jb > min(w_last, L - 1) - 1 + ac) {
 #pragma unroll
           for (int i = 0; i < 8; i++) { pk[i] = 0; dzk[i] = 0; }
         } else {
@@ -919,6 +919,8 @@ template <typename T>
 static hipError_t launch_t(const BwdParams& p, int max_tiles, hipStream_t stream) {
   // head_dim 64 measures slightly faster on the 64-key kernel (its steps are already short).
   const bool wide = p.head_dim > 64;
+  if (p.split && wide)
+    return p.load == kLoadAligned ? launch_dkv3<T, 128, kLoadAligned>(p, max_tiles, stream) : launch_dkv3<T, 128, kLoadPadded>(p, max_tiles, stream);
   if (p.load == kLoadAligned) return wide ? launch_dkv4<T, 128, kLoadAligned>(p, max_tiles, stream) : launch_dkv3<T, 64, kLoadAligned>(p, max_tiles, stream);
   if (p.load == kLoadPadded) return wide ? launch_dkv4<T, 128, kLoadPadded>(p, max_tiles, stream) : launch_dkv3<T, 64, kLoadPadded>(p, max_tiles, stream);
   return wide ? launch_one<T, 128>(p, max_tiles, stream) : launch_one<T, 64>(p, max_tiles, stream);
@@ -926,7 +928,7 @@ static hipError_t launch_t(const BwdParams& p, int max_tiles, hipStream_t stream
 
 // Keys per key tile of the kernel launch_bwd_dkv will pick for these parameters.
 int dkv_key_tile(const BwdParams& p) {
-  return p.load != kLoadScalar && p.head_dim > 64 ? kDkv4Keys : kBlockK;
+  return p.load != kLoadScalar && p.head_dim > 64 && !p.split ? kDkv4Keys : kBlockK;
 }
 
 hipError_t launch_bwd_dkv(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream) {

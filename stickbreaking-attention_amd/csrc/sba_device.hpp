@@ -248,6 +248,78 @@ struct TileCopy {
   }
 };
 
+// The forward's weights of this lane's N keys R (ascending; register R & 15 of score tile R >> 4).  With r[R] the running product below key R (so r[R+1] is above it),
+//   weight of key R = sigma[R] r[R+1] = e[R] r[R]        r[R+1] = r[R] + e[R] r[R]
+// so, taken upwards from the product below a group of keys, a weight costs one multiplication and one addition, carries
+// the product above the tile without one of its own, and loses nothing to cancellation.  The products below come from
+// one reciprocal of prod(1 + e) per kGroup keys: 20 transcendentals per 16 keys instead of 32, 5.5 instructions per key
+// besides instead of 7.5.  Vector-ALU issue is what bounds this kernel (75 % busy at head_dim 64, 60 % at 128): 32 heads
+// x 8192 x 128 653 -> 606 us, 32 heads x 2 x 4096 x 64 227 -> 188 us.  The product of a group has to stay far from
+// overflow; where it does not (four keys whose logits add up to 100 octaves), the wave takes the weights downwards as
+// differences of the running product, one reciprocal per key, where e = inf gives a factor 0 and the whole remaining stick.
+// Hidden keys (diagonal tiles only) get e = 0: factor 1, weight 0.
+template <int N>
+struct Weights {
+  static constexpr int kGroup = 4;
+  float t[N];                   // e, then the weights
+  float below[N / kGroup];      // 1 / prod(1 + e) of a group, then the running product below it
+  float run;                    // product over all N keys
+  bool tame;
+
+  // Up to the product over the keys; key R is visible iff R < lim.
+  template <bool kDiagonal, int NT>
+  __device__ __forceinline__ void front(const f32x16 (&s)[NT], float scale_log2, int lim) {
+    static_assert(N == 16 * NT, "");
+#pragma unroll
+    for (int R = 0; R < N; ++R) {
+      const float x = s[R >> 4][R & 15] * scale_log2;
+      t[R] = fast_exp2(!kDiagonal || R < lim ? x : -INFINITY);
+    }
+    float most = 0.f;      // (a sum, so that a NaN of inf * 0 shows)
+#pragma unroll
+    for (int g = 0; g < N / kGroup; g++) {
+      float prod_g = 1.f + t[kGroup * g];
+#pragma unroll
+      for (int i = 1; i < kGroup; i++) prod_g = fmaf(prod_g, t[kGroup * g + i], prod_g);
+      below[g] = prod_g;
+      most += prod_g;
+    }
+    tame = !__any(!(most < 0x1p100f));
+    run = 1.f;
+    if (tame) {
+#pragma unroll
+      for (int g = N / kGroup - 1; g >= 0; --g) {
+        run *= fast_rcp(below[g]);
+        below[g] = run;
+      }
+    } else {
+#pragma unroll
+      for (int R = N - 1; R >= 0; --R) {
+        const float before = run;
+        run *= fast_rcp(1.f + t[R]);
+        t[R] = before - run;
+      }
+    }
+  }
+  // The weights; `seed`: the product above the N keys.
+  __device__ __forceinline__ void back(float seed) {
+    if (tame) {
+#pragma unroll
+      for (int g = 0; g < N / kGroup; g++) {
+        float r = below[g] * seed;
+#pragma unroll
+        for (int i = 0; i < kGroup; i++) {
+          t[kGroup * g + i] *= r;
+          if (i + 1 < kGroup) r += t[kGroup * g + i];
+        }
+      }
+    } else {
+#pragma unroll
+      for (int R = 0; R < N; R++) t[R] *= seed;
+    }
+  }
+};
+
 // Element-wise backward math of one 64-key tile for the 32 keys this lane owns (see the conventions above).
 //   s, dp     : S^T = K Q^T and dP^T = V dO^T accumulators (row tile mt, register r  <->  key 32*half + 16*mt + r)
 //   lim       : key R of this lane is visible iff R < lim (only consulted when `diagonal`)
@@ -259,62 +331,80 @@ struct TileCopy {
 // Produces P (pk) and dZ = g - sigma * C (dzk), C_ij = sum_{j' <= j} g_ij', packed to 16 bit two keys per
 // word, and the prefix sum for the next tile up.  (The reference evaluates the same quantities tile by tile at
 // stickbreaking_attention/sb_varlen/sb_varlen_bwd.py:438-447.)
-template <typename T, int NT, bool kDiagonal, bool kNeedP = true>
-__device__ __forceinline__ void bwd_tile_math_impl(const f32x16 (&s)[NT], const f32x16 (&dp)[NT], float scale_log2, int lim,
-                                                   int half, float drem, float prod_in, float prefix_in,
-                                                   uint32_t (&pk)[8 * NT], uint32_t (&dzk)[8 * NT], float& prod_lower,
-                                                   float& prefix_upper, float& prefix_out) {
+template <int N>
+struct BwdMath {
+  float beta[N], pe[N], u[N];      // sigma, the product below each key (times `seed` with kNeedP), u (times `seed` without)
+  float seed;                      // product above this lane's keys
+  float run, oth;                  // product over this lane's keys, and over the other half-wave's
+  float tot, oth_g;                // sum of g over this lane's keys, and over the other half-wave's
+};
+// Up to the sums of g.  What may be known only afterwards is C below this lane's keys.
+template <int NT, bool kDiagonal, bool kNeedP>
+__device__ __forceinline__ void bwd_math_front(BwdMath<16 * NT>& m, const f32x16 (&s)[NT], const f32x16 (&dp)[NT], float scale_log2, int lim,
+                                               int half, float drem, float prod_in) {
   constexpr int N = 16 * NT;      // keys per lane
   // sigma = 1 - 1/(1+e) needs no clamp on e: e = inf gives 1/(1+e) = 0 and sigma = 1 exactly, and the absolute
   // error of the subtraction (6e-8) is far below the 16-bit rounding of P and dZ.
-  float beta[N], pe[N];
   float run = 1.f;
 #pragma unroll
   for (int R = N - 1; R >= 0; --R) {
     float x = s[R >> 4][R & 15] * scale_log2;
     if (kDiagonal) x = (R < lim) ? x : -INFINITY;
     const float omb = fast_rcp(1.f + fast_exp2(x));
-    beta[R] = 1.f - omb;
+    m.beta[R] = 1.f - omb;
     run *= omb;
-    pe[R] = run;           // product over this key and this lane's higher keys
+    m.pe[R] = run;           // product over this key and this lane's higher keys
   }
-  const float oth = other_half(run, half);
-  prod_lower = prod_in * (half ? run : oth);               // product above the lower half-wave's keys
-  const float seed = half ? prod_in : prod_lower;           // the upper half-wave holds the higher keys
+  m.run = run;
+  m.oth = other_half(run, half);
+  const float seed = m.seed = half ? prod_in : prod_in * m.oth;      // the upper half-wave holds the higher keys
   // Let D = drem + (sum of g over this lane's keys up to j) / (product above key j).  Then, with u_j = dP_j - D_{j-1},
   //   D_j = D_{j-1} + sigma_j u_j        g_j - sigma_j (sum of g over the lane's keys up to j) = sigma_j (product below key j) u_j
   // (D is a running weighted mean of drem and dP, so it neither grows nor cancels), and with C0 = C below the lane's keys
   //   dz_j = sigma_j (seed pe_j u_j - C0)
   // which is 4 instructions per key where summing g and correcting by sigma C takes 6.  The vector ALU is what bounds the
   // backward kernels (87 % busy in dQ at head_dim 64): dQ 32 heads x 2 x 4096 x 64 345 -> 320 us, see the kernels for the rest.
-  float u[N];
   float D = kNeedP ? drem : drem * seed;                    // (kNeedP: P wants seed * pe anyway; else D is kept times seed)
   const float D0 = D;
 #pragma unroll
   for (int R = 0; R < N; R++) {
-    u[R] = kNeedP ? dp[R >> 4][R & 15] - D : fmaf(dp[R >> 4][R & 15], seed, -D);
-    D = fmaf(beta[R], u[R], D);
+    m.u[R] = kNeedP ? dp[R >> 4][R & 15] - D : fmaf(dp[R >> 4][R & 15], seed, -D);
+    D = fmaf(m.beta[R], m.u[R], D);
   }
-  const float tot = kNeedP ? (D - D0) * seed : D - D0;
-  const float oth_g = other_half(tot, half);
-  const float below = prefix_in + (half ? oth_g : 0.f);     // the lower half-wave holds the lower keys
-  prefix_upper = prefix_in + (half ? oth_g : tot);          // C just below the upper half-wave's keys
-  prefix_out = prefix_in + (tot + oth_g);
+  m.tot = kNeedP ? (D - D0) * seed : D - D0;
+  m.oth_g = other_half(m.tot, half);
+}
+// P and dZ, packed.  `below`: C below this lane's keys (prefix below the tile, plus the lower half-wave's sum in the upper one).
+template <typename T, int N, bool kNeedP>
+__device__ __forceinline__ void bwd_math_back(BwdMath<N>& m, float below, uint32_t (&pk)[N / 2], uint32_t (&dzk)[N / 2]) {
   float a[N];
   if (kNeedP) {
-    float above = seed;
+    float above = m.seed;
 #pragma unroll
     for (int R = N - 1; R >= 0; --R) {
-      a[R] = beta[R] * above;
-      above = pe[R] * seed;
-      pe[R] = above;
+      a[R] = m.beta[R] * above;
+      above = m.pe[R] * m.seed;
+      m.pe[R] = above;
     }
   }
 #pragma unroll
   for (int R = 0; R < N; R += 2) {
     pk[R >> 1] = kNeedP ? pack2<T>(a[R], a[R + 1]) : 0u;
-    dzk[R >> 1] = pack2<T>(beta[R] * fmaf(pe[R], u[R], -below), beta[R + 1] * fmaf(pe[R + 1], u[R + 1], -below));
+    dzk[R >> 1] = pack2<T>(m.beta[R] * fmaf(m.pe[R], m.u[R], -below), m.beta[R + 1] * fmaf(m.pe[R + 1], m.u[R + 1], -below));
   }
+}
+
+template <typename T, int NT, bool kDiagonal, bool kNeedP = true>
+__device__ __forceinline__ void bwd_tile_math_impl(const f32x16 (&s)[NT], const f32x16 (&dp)[NT], float scale_log2, int lim,
+                                                   int half, float drem, float prod_in, float prefix_in,
+                                                   uint32_t (&pk)[8 * NT], uint32_t (&dzk)[8 * NT], float& prod_lower,
+                                                   float& prefix_upper, float& prefix_out) {
+  BwdMath<16 * NT> m;
+  bwd_math_front<NT, kDiagonal, kNeedP>(m, s, dp, scale_log2, lim, half, drem, prod_in);
+  prod_lower = prod_in * (half ? m.run : m.oth);            // product above the lower half-wave's keys
+  prefix_upper = prefix_in + (half ? m.oth_g : m.tot);      // C just below the upper half-wave's keys
+  prefix_out = prefix_in + (m.tot + m.oth_g);
+  bwd_math_back<T, 16 * NT, kNeedP>(m, prefix_in + (half ? m.oth_g : 0.f), pk, dzk);
 }
 
 // prod_lower / prefix_upper: the same two carries at the boundary between the two half-waves' keys (the middle of

@@ -142,84 +142,26 @@ __global__ __launch_bounds__(kThreads, kMinWaves) void fwd_kernel(FwdParams p) {
       }
     }
 
-    // This lane's N keys are j0 + N*half + R, R = 16*mt + r.  With r[R] the running product below key R (so r[R+1] is above it),
-    //   weight of key R = sigma[R] r[R+1] = e[R] r[R]        r[R+1] = r[R] + e[R] r[R]
-    // so, taken upwards from the product below a group of keys, a weight costs one multiplication and one addition, carries
-    // the product above the tile without one of its own, and loses nothing to cancellation.  The products below come from
-    // one reciprocal of prod(1 + e) per kGroup keys: 20 transcendentals per 16 keys instead of 32, 5.5 instructions per key
-    // besides instead of 7.5.  Vector-ALU issue is what bounds this kernel (75 % busy at head_dim 64, 60 % at 128): 32 heads
-    // x 8192 x 128 653 -> 606 us, 32 heads x 2 x 4096 x 64 227 -> 188 us.  The product of a group has to stay far from
-    // overflow; where it does not (four keys whose logits add up to 100 octaves), the wave takes the weights downwards as
-    // differences of the running product, one reciprocal per key, where e = inf gives a factor 0 and the whole remaining stick.
-    // Hidden keys (diagonal tiles only) get e = 0: factor 1, weight 0.
+    // This lane's N keys are j0 + N*half + R, R = 16*mt + r.
     __builtin_amdgcn_s_setprio(0);
-    constexpr int kGroup = 4;
-    float t[N];      // e, then the weights
-    if (diagonal) {
-      const int lim = qi + ac - j0 - N * half;                // key R is visible iff R < lim
-#pragma unroll
-      for (int R = 0; R < N; ++R) {
-        const float x = s[R >> 4][R & 15] * p.scale_log2;
-        t[R] = fast_exp2((R < lim) ? x : -INFINITY);
-      }
-    } else {
-#pragma unroll
-      for (int R = 0; R < N; ++R) t[R] = fast_exp2(s[R >> 4][R & 15] * p.scale_log2);
-    }
-    float below[N / kGroup];      // 1 / prod(1 + e) of a group, then the running product below it
-    float most = 0.f;      // (a sum, so that a NaN of inf * 0 shows)
-#pragma unroll
-    for (int g = 0; g < N / kGroup; g++) {
-      float prod_g = 1.f + t[kGroup * g];
-#pragma unroll
-      for (int i = 1; i < kGroup; i++) prod_g = fmaf(prod_g, t[kGroup * g + i], prod_g);
-      below[g] = prod_g;
-      most += prod_g;
-    }
-    const bool tame = !__any(!(most < 0x1p100f));
-    float run = 1.f;
-    if (tame) {
-#pragma unroll
-      for (int g = N / kGroup - 1; g >= 0; --g) {
-        run *= fast_rcp(below[g]);
-        below[g] = run;
-      }
-    } else {
-#pragma unroll
-      for (int R = N - 1; R >= 0; --R) {
-        const float before = run;
-        run *= fast_rcp(1.f + t[R]);
-        t[R] = before - run;
-      }
-    }
+    Weights<N> w;
+    const int lim = qi + ac - j0 - N * half;                  // key R is visible iff R < lim
+    if (diagonal) w.template front<true>(s, p.scale_log2, lim); else w.template front<false>(s, p.scale_log2, lim);
+    const float run = w.run;
     const float oth = other_half(run, half);
     // The upper half-wave holds the higher keys, which come first in the sweep.
     const float seed = half ? prod : prod * oth;
     if (NT == 2 && carry && half == 0) carry_row(u_hi - 1)[lrow] = seed;   // product above the lower sub-tile
     prod = (prod * oth) * run;
     if (kCarryOnly) continue;
-    if (tame) {
-#pragma unroll
-      for (int g = 0; g < N / kGroup; g++) {
-        float r = below[g] * seed;
-#pragma unroll
-        for (int i = 0; i < kGroup; i++) {
-          t[kGroup * g + i] *= r;
-          if (i + 1 < kGroup) r += t[kGroup * g + i];
-        }
-      }
-    } else {
-#pragma unroll
-      for (int R = 0; R < N; R++) t[R] *= seed;
-    }
-
+    w.back(seed);
     __builtin_amdgcn_s_setprio(3);
     // O += P V: A = P from registers (k index <-> key 32*half + 8c + t), B = V gathered down the keys.
 #pragma unroll
     for (int c = 0; c < KT / 16; c++) {
       u32x4 av;
 #pragma unroll
-      for (int i = 0; i < 4; i++) av[i] = pack2<T>(t[8 * c + 2 * i], t[8 * c + 2 * i + 1]);
+      for (int i = 0; i < 4; i++) av[i] = pack2<T>(w.t[8 * c + 2 * i], w.t[8 * c + 2 * i + 1]);
       vec8 a = as_vec8<T>(av);
 #pragma unroll
       for (int dt = 0; dt < kDTiles; dt++) {

@@ -96,6 +96,7 @@ struct BwdParams {
   float logit_scale;
   int32_t attend_current;
   int32_t load;                // as in FwdParams
+  int32_t split;               // dK/dV: too few key tiles to fill the chip
   // Fused remainder term (the forward wrote o + rem * v): d_rem_eff = d_rem + d_o . v per row, dv += rem * d_o.
   int32_t add_rem;
   const float* row_stat;       // log2(rem), fp32 [batch][head][token]

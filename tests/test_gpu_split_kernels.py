@@ -1,0 +1,39 @@
+"""The kernels of problems too small to fill the chip (keys split over the waves): lengths around their 32-row blocks and
+128-key steps, rows no sequence covers, both directions, against the float64 oracle; and both kinds of kernel on the two sides
+of the size from which on the wide ones run."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import sb_oracle as orc
+from stickbreaking_attention import sb_attn_varlen
+from test_gpu_parity import NAMES, tol_check
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("attend_current,add_remainder,save_carry", [(False, False, True), (True, True, False)])
+@pytest.mark.parametrize("H,D", [(2, 24), (3, 64), (2, 100), (3, 128), (40, 64), (25, 128)])
+def test_lengths_around_the_steps(gpu_device, H, D, attend_current, add_remainder, save_carry):
+    lengths, pad = [1, 31, 32, 33, 95, 127, 128, 129, 160, 257, 300], 50
+    dtype = torch.bfloat16
+    T = sum(lengths)
+    g = torch.Generator().manual_seed(H * D)
+    host = [torch.randn(H, T + pad, D, generator=g).to(dtype) for _ in range(4)] + [torch.randn(H, T + pad, generator=g).to(dtype)]
+    q, k, v, do, drem = (t.to(gpu_device) for t in host)
+    for t in (q, k, v):
+        t.requires_grad_()
+    cu = torch.tensor(np.cumsum(lengths), dtype=torch.int32)
+    o, rem = sb_attn_varlen(q, k, v, cu, max(lengths), zero_start=False, attend_current=attend_current, add_remainder=add_remainder,
+                            save_carry=save_carry)
+    got = (o, rem, *torch.autograd.grad([o, rem], [q, k, v], [do, drem]))
+    heads = sorted({0, H - 1})
+    d = [t[heads, :T].double() for t in host]
+    if add_remainder:
+        d[4] = orc.remainder_drem(d[3], d[4], d[2])
+    ref = orc.varlen_stream(d[0], d[1], d[2], cu, attend_current=attend_current, do=d[3], drem=d[4], dtype=torch.float64)
+    if add_remainder:
+        ref = orc.with_remainder(ref, d[2], d[3])
+    for n, a, b in zip(NAMES, got, ref):
+        tol_check(n, a[heads, :T], b, dtype, f"H={H} D={D}")
+        assert (a[:, T:] == 0).all(), f"{n}: rows no sequence covers must be zero"

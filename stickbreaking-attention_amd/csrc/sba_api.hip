@@ -17,6 +17,7 @@ int dkv_key_tile(const BwdParams& p);
 bool chain_supported(const BwdParams& p);
 hipError_t launch_bwd_chain(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
 hipError_t launch_fwd_split(const FwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
+hipError_t launch_fwd_split_carry_only(const FwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
 hipError_t launch_bwd_dq_split(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
 hipError_t launch_bwd_dkv_split(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
 hipError_t launch_fwd_f32(const FwdParams& p, int max_tiles, hipStream_t stream);
@@ -160,16 +161,18 @@ int row_load(const SbaArgs* a, const SbaTensor* const (&tensors)[N]) {
 //                 dQ    28.8 / 61    29.9 / 62    43 / 63    78 / 69
 //   head_dim 128  fwd   34.7 / 61    39 / 62      60 / 64   112 / 73     (8192: 128 / 230, 131 / 236, 189 / 238, 325 / 262)
 //                 dQ    39 / 79      47 / 80      91 / 84   185 / 94
-bool few_tiles(const SbaArgs* a, int load) {
+// `heads` is the head count of the caller's call, also where the backward takes them through in groups: the groups then run the
+// kernels, and give the bits, of one pass, and products are rebuilt by the kernel whose forward would have kept them.
+bool few_tiles(const SbaArgs* a, int64_t heads, int load) {
   if (a->dtype == SBA_F32 || load == sba::kLoadScalar) return false;
-  const int64_t rows = a->total_tokens * (a->cu_seqlens ? 1 : a->num_seqs) * a->num_heads;
+  const int64_t rows = a->total_tokens * (a->cu_seqlens ? 1 : a->num_seqs) * heads;
   return rows < (a->head_dim > 64 ? 30 << 10 : 60 << 10);
 }
 // The same for dK/dV: below, head_dim up to 64 splits the rows over the waves (130 K rows x heads: 542 / 565 us at 8192
 // tokens), wider ones take key tiles of 64 instead of 128 (64 K: 113 / 119 at 2048, 354 / 410 at 8192; 130 K: 672 / 657).
-bool few_key_tiles(const SbaArgs* a, int load) {
+bool few_key_tiles(const SbaArgs* a, int64_t heads, int load) {
   if (a->dtype == SBA_F32 || load == sba::kLoadScalar) return false;
-  return a->total_tokens * (a->cu_seqlens ? 1 : a->num_seqs) * a->num_heads < 100 << 10;
+  return a->total_tokens * (a->cu_seqlens ? 1 : a->num_seqs) * heads < 100 << 10;
 }
 int check_tensor(const SbaTensor& t, bool required, bool fixed) {
   if (!t.ptr) return required ? SBA_ERR_NULL : SBA_OK;
@@ -224,7 +227,7 @@ int expected_key_tile(const SbaArgs* a, const Layout& L) {
   sba::BwdParams p{};
   p.head_dim = a->head_dim;
   p.load = row_load(a, {&a->q, &a->k, &a->v});
-  p.split = L.chain_zero_bytes == 0 && few_key_tiles(a, p.load);
+  p.split = L.chain_zero_bytes == 0 && few_key_tiles(a, a->num_heads, p.load);
   return sba::dkv_key_tile(p);
 }
 
@@ -359,7 +362,7 @@ int fwd_on(const SbaArgs* a, char* ws, size_t ws_bytes, bool ws_is_static, bool 
   hipEvent_t* ev = (hipEvent_t*)a->trace_events;
   if (ev && hipEventRecord(ev[0], stream) != hipSuccess) return SBA_ERR_LAUNCH;
   hipError_t e = (a->dtype == SBA_F32) ? sba::launch_fwd_f32(p, (int)L.max_q_tiles, stream)
-                 : few_tiles(a, p.load)  ? sba::launch_fwd_split(p, a->dtype == SBA_F16, (int)L.max_q_tiles, stream)
+                 : few_tiles(a, a->num_heads, p.load) ? sba::launch_fwd_split(p, a->dtype == SBA_F16, (int)L.max_q_tiles, stream)
                                          : sba::launch_fwd(p, a->dtype == SBA_F16, (int)L.max_q_tiles, stream);
   if (e != hipSuccess) return SBA_ERR_LAUNCH;
   if (ev && hipEventRecord(ev[1], stream) != hipSuccess) return SBA_ERR_LAUNCH;
@@ -451,7 +454,7 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* 
   p.max_tiles = (int32_t)L.max_q_tiles;
   p.total_tokens = a->total_tokens;
   p.load = bwd_load(a);
-  p.split = L.chain_zero_bytes == 0 && few_key_tiles(a, p.load);
+  p.split = L.chain_zero_bytes == 0 && few_key_tiles(a, stat_heads, p.load);
   // One kernel (the key tiles of a sequence hand C and partial dQ to each other) where it applies, else dQ then dK/dV.
   const bool chain = bwd_is_chained(a, L);
   if (chain) {
@@ -494,7 +497,9 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* 
     f.max_tiles = (int32_t)L.max_q_tiles;
     f.total_tokens = a->total_tokens;
     f.load = row_load(a, {&a->q, &a->k});
-    if (sba::launch_fwd_carry_only(f, a->dtype == SBA_F16, (int)L.max_q_tiles, stream) != hipSuccess) return SBA_ERR_LAUNCH;
+    if ((few_tiles(a, stat_heads, f.load) ? sba::launch_fwd_split_carry_only(f, a->dtype == SBA_F16, (int)L.max_q_tiles, stream)
+                                          : sba::launch_fwd_carry_only(f, a->dtype == SBA_F16, (int)L.max_q_tiles, stream)) != hipSuccess)
+      return SBA_ERR_LAUNCH;
   }
   if (chain) {
     if (ev && last && hipEventRecord(ev[1], stream) != hipSuccess) return SBA_ERR_LAUNCH;
@@ -503,7 +508,7 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* 
     return SBA_OK;
   }
   const bool f16 = a->dtype == SBA_F16;
-  if ((few_tiles(a, p.load) ? sba::launch_bwd_dq_split(p, f16, (int)L.max_q_tiles, stream) : sba::launch_bwd_dq(p, f16, (int)L.max_q_tiles, stream)) != hipSuccess)
+  if ((few_tiles(a, stat_heads, p.load) ? sba::launch_bwd_dq_split(p, f16, (int)L.max_q_tiles, stream) : sba::launch_bwd_dq(p, f16, (int)L.max_q_tiles, stream)) != hipSuccess)
     return SBA_ERR_LAUNCH;
   if (ev && last && hipEventRecord(ev[1], stream) != hipSuccess) return SBA_ERR_LAUNCH;
   if ((p.split && a->head_dim <= 64 ? sba::launch_bwd_dkv_split(p, f16, (int)L.max_k_tiles, stream)
@@ -600,7 +605,7 @@ bool prepared_fits(const SbaArgs* a) {
   BwdParams p{};
   p.head_dim = a->head_dim;
   p.load = bwd_load(a);
-  p.split = L.chain_zero_bytes == 0 && few_key_tiles(a, p.load);
+  p.split = L.chain_zero_bytes == 0 && few_key_tiles(a, a->num_heads, p.load);
   return a->dtype == SBA_F32 || dkv_key_tile(p) == expected_key_tile(a, L);
 }
 

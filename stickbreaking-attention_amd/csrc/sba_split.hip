@@ -99,14 +99,15 @@ __device__ __forceinline__ void contract32(f32x16 (&acc)[DH / 32], const uint32_
   }
 }
 
-template <typename T, int DH, int kLoad>
+// kCarryOnly: as in fwd_kernel, and with this kernel's products bit for bit.
+template <typename T, int DH, int kLoad, bool kCarryOnly>
 __global__ __launch_bounds__(kThreads, 2) void fwd_split_kernel(FwdParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   __shared__ float xch[2][kWaves][32];
   __shared__ float rem_lds[32];
   T* const k_lds = reinterpret_cast<T*>(lds_raw);
   T* const v_lds = k_lds + SplitLds<DH>::kTile;
-  if ((int)blockIdx.x < p.sched.service) {
+  if (!kCarryOnly && (int)blockIdx.x < p.sched.service) {
     forward_service(p.sched, blockIdx.x);
     return;
   }
@@ -116,7 +117,7 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_split_kernel(FwdParams p) {
   Tile tile;
   int64_t r0, r1;
   if (!forward_tile(p, slot, sub, kSplitRows, &tile, &r0, &r1)) {
-    if (r0 < r1) {      // rows of no sequence: o = rem = 0
+    if (!kCarryOnly && r0 < r1) {      // rows of no sequence: o = rem = 0
       zero_rows<T>(p.o, head, r0, r1, p.head_dim);
       for (int64_t r = r0 + threadIdx.x; r < r1; r += kThreads) {
         ((T*)p.rem.ptr)[head * p.rem.sh + r * p.rem.st] = (T)0;
@@ -143,7 +144,7 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_split_kernel(FwdParams p) {
   TileCopy<T, DH, kStep, kLoad> ck, cv;
   if (n_kt > 0) {
     ck.load(ksrc, (n_kt - 1) * kStep);
-    cv.load(vsrc, (n_kt - 1) * kStep);
+    if (!kCarryOnly) cv.load(vsrc, (n_kt - 1) * kStep);
   }
   typename Elem<T>::vec8 qf[DH / 16];
   load_operand<T, kLoad>(qf, make_row_source<T, kLoad>(qb, p.q.st, L, D), qi, half);
@@ -158,11 +159,11 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_split_kernel(FwdParams p) {
     const bool active = j0 <= last_key;
     lds_barrier();
     ck.store(k_lds);
-    cv.store(v_lds);
+    if (!kCarryOnly) cv.store(v_lds);
     lds_barrier();
     if (jt > 0) {
       ck.load(ksrc, (jt - 1) * kStep);
-      cv.load(vsrc, (jt - 1) * kStep);
+      if (!kCarryOnly) cv.load(vsrc, (jt - 1) * kStep);
     }
     Weights<16> w;
     w.run = 1.f;
@@ -185,7 +186,7 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_split_kernel(FwdParams p) {
     }
     // (every sub-tile of the step is recorded: the kernels that sweep 64 keys read the upper of a pair)
     if (carry && half == 0) (carry + carry_offset(u, n_qt) + (tile.origin - kBlockQ * (u >> 2)))[col] = above;
-    if (active) {
+    if (!kCarryOnly && active) {
       w.back(half ? above : above * oth);                     // the upper half-wave holds the higher keys
       uint32_t pk[8];
 #pragma unroll
@@ -193,6 +194,7 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_split_kernel(FwdParams p) {
       contract32<T, DH>(oacc, pk, v_lds + 32 * wave * lds_stride<DH>(), half, lane);
     }
   }
+  if (kCarryOnly) return;
   if (wave == 0 && half == 0) {
     rem_lds[col] = prod;
     if (qi < L) {
@@ -457,12 +459,19 @@ static hipError_t launch_split(Kernel kernel, std::atomic<uint64_t>& lds_done, s
   return hipGetLastError();
 }
 
-hipError_t launch_fwd_split(const FwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream) {
+template <bool kCarryOnly>
+static hipError_t launch_fwd_split_t(const FwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream) {
   return by_shape(dtype_is_f16, p.head_dim, p.load, [&](auto t, auto dh, auto load) {
     static std::atomic<uint64_t> lds_done{0};
-    return launch_split(&fwd_split_kernel<decltype(t), decltype(dh)::value, decltype(load)::value>, lds_done, SplitLds<decltype(dh)::value>::kBytes,
-                        (unsigned)(max_tiles * p.num_heads * kSplitSubs + p.sched.service), p, stream);
+    return launch_split(&fwd_split_kernel<decltype(t), decltype(dh)::value, decltype(load)::value, kCarryOnly>, lds_done,
+                        SplitLds<decltype(dh)::value>::kBytes, (unsigned)(max_tiles * p.num_heads * kSplitSubs + p.sched.service), p, stream);
   });
+}
+hipError_t launch_fwd_split(const FwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream) {
+  return launch_fwd_split_t<false>(p, dtype_is_f16, max_tiles, stream);
+}
+hipError_t launch_fwd_split_carry_only(const FwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream) {
+  return launch_fwd_split_t<true>(p, dtype_is_f16, max_tiles, stream);
 }
 hipError_t launch_bwd_dq_split(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream) {
   return by_shape(dtype_is_f16, p.head_dim, p.load, [&](auto t, auto dh, auto load) {

@@ -11,8 +11,11 @@
 #include <ATen/ops/empty_like.h>
 #include <ATen/ops/zeros_like.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <atomic>
 #include <cmath>
@@ -228,8 +231,9 @@ struct StickBreaking : torch::autograd::Function<StickBreaking> {
     c.logit_scale = ctx->saved_data["scale"].toDouble();
     c.cu = s[3];
     c10::IValue& fresh = ctx->saved_data["fresh"];
-    variable_list g = run_backward(c, grads[0], grads[1], s[0], s[1], s[2], s[4], n[7], fresh.toBool());
-    fresh = false;
+    const bool first = fresh.toBool();
+    fresh = false;      // (also where the call fails half way through the schedule)
+    variable_list g = run_backward(c, grads[0], grads[1], s[0], s[1], s[2], s[4], n[7], first);
     g.resize(5);      // call, save_carry
     return g;
   }
@@ -250,12 +254,34 @@ std::tuple<Tensor, Tensor> attention(const Call& c, Tensor q, Tensor k, Tensor v
   return {out.o, out.rem};
 }
 
+// Whether a call on these tensors is ordinary eager work.  What records, transforms or replaces operations (a jit trace,
+// dispatch modes, torch.func transforms, tensor subclasses and wrappers) and forward-mode derivatives see nothing of what
+// happens here: such calls take the Python operators, which record themselves or refuse.
+bool ordinary(py::handle q, py::handle k, py::handle v) {
+  using c10::DispatchKey;
+  static const c10::DispatchKeySet wrapped({DispatchKey::Python, DispatchKey::Functionalize, DispatchKey::FuncTorchBatched,
+                                            DispatchKey::FuncTorchGradWrapper, DispatchKey::Batched, DispatchKey::Conjugate,
+                                            DispatchKey::Negative, DispatchKey::ZeroTensor});
+  if (torch::jit::tracer::isTracing() || c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+      c10::impl::tls_is_dispatch_key_included(DispatchKey::FuncTorchDynamicLayerFrontMode))
+    return false;
+  for (const py::handle h : {q, k, v}) {
+    if (!THPVariable_CheckExact(h.ptr())) return false;      // (a tensor or a parameter, and no subclass)
+    const Tensor& t = THPVariable_Unpack(h.ptr());
+    if (t.key_set().has_any(wrapped) || t._fw_grad(0).defined()) return false;
+  }
+  return true;
+}
+
 double scale_of(const std::optional<double>& inv_temp, const Tensor& q) {
   return inv_temp ? *inv_temp : 1.0 / std::sqrt((double)q.size(-1));
 }
 
-std::tuple<Tensor, Tensor> fixed(const Tensor& q, const Tensor& k, const Tensor& v, std::optional<double> inv_temp,
-                                 bool attend_current, bool add_remainder, bool save_carry, int64_t flags) {
+// None where the call is not ordinary.
+std::optional<std::tuple<Tensor, Tensor>> fixed(py::handle hq, py::handle hk, py::handle hv, std::optional<double> inv_temp,
+                                                bool attend_current, bool add_remainder, bool save_carry, int64_t flags) {
+  if (!ordinary(hq, hk, hv)) return std::nullopt;
+  const Tensor &q = THPVariable_Unpack(hq.ptr()), &k = THPVariable_Unpack(hk.ptr()), &v = THPVariable_Unpack(hv.ptr());
   require_gpu(q); require_gpu(k); require_gpu(v);
   Call c;
   c.fixed = true;
@@ -266,9 +292,11 @@ std::tuple<Tensor, Tensor> fixed(const Tensor& q, const Tensor& k, const Tensor&
   return attention(c, q, k, v, save_carry);
 }
 
-std::tuple<Tensor, Tensor> varlen(const Tensor& q, const Tensor& k, const Tensor& v, Tensor cu, std::optional<int64_t> max_seqlens,
-                                  std::optional<double> inv_temp, bool zero_start, bool attend_current, bool add_remainder,
-                                  bool save_carry, int64_t flags) {
+std::optional<std::tuple<Tensor, Tensor>> varlen(py::handle hq, py::handle hk, py::handle hv, Tensor cu,
+                                                 std::optional<int64_t> max_seqlens, std::optional<double> inv_temp, bool zero_start,
+                                                 bool attend_current, bool add_remainder, bool save_carry, int64_t flags) {
+  if (!ordinary(hq, hk, hv)) return std::nullopt;
+  const Tensor &q = THPVariable_Unpack(hq.ptr()), &k = THPVariable_Unpack(hk.ptr()), &v = THPVariable_Unpack(hv.ptr());
   Call c;
   c.leading_zero = zero_start;
   c.attend_current = attend_current; c.add_remainder = add_remainder;
@@ -308,6 +336,7 @@ std::tuple<Tensor, Tensor> varlen(const Tensor& q, const Tensor& k, const Tensor
 }  // namespace
 
 PYBIND11_MODULE(_sba_torch, m) {
+  m.def("ordinary", &ordinary);
   m.def("fixed", &fixed);
   m.def("varlen", &varlen);
   m.def("set_backward_workspace_limit", [](std::optional<int64_t> n) { g_bwd_limit.store(n ? std::max<int64_t>(*n, 0) : -1); });

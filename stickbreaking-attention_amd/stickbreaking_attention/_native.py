@@ -133,7 +133,8 @@ def ext():
 
 
 def use_ext() -> bool:
-    """Whether a call goes through the torch host layer: eager calls do, unless their kernels are traced."""
+    """Whether a call is offered to the torch host layer: eager calls are, unless their kernels are timed.  It declines (None) what
+    is not ordinary eager work on plain tensors (``ordinary`` in csrc/sba_torch.cpp)."""
     return TRACE_EVENTS is None and not torch.compiler.is_compiling()
 
 

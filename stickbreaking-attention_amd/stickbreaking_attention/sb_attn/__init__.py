@@ -39,7 +39,9 @@ def sb_attn(q, k, v, inv_temp=None, zero_start=True, attend_current=False, add_r
     reference's outputs), fused into the kernels' epilogues.  ``save_carry=False`` keeps only q, k, v for the backward,
     which then rebuilds the forward's per-(row, sub-tile) products itself."""
     if _native.use_ext():
-        return _native.ext().fixed(q, k, v, inv_temp, attend_current, add_remainder, save_carry, _native.flags())
+        out = _native.ext().fixed(q, k, v, inv_temp, attend_current, add_remainder, save_carry, _native.flags())
+        if out is not None:
+            return out
     if inv_temp is None:
         inv_temp = 1 / math.sqrt(q.size(-1))
     return sb_attn_(q, k, v, inv_temp, attend_current=attend_current, add_remainder=add_remainder, save_carry=save_carry)
@@ -47,5 +49,7 @@ def sb_attn(q, k, v, inv_temp=None, zero_start=True, attend_current=False, add_r
 
 def sb_attn_(q, k, v, inv_temp, attend_current, add_remainder=False, save_carry=True):
     if _native.use_ext():
-        return _native.ext().fixed(q, k, v, inv_temp, attend_current, add_remainder, save_carry, _native.flags())
+        out = _native.ext().fixed(q, k, v, inv_temp, attend_current, add_remainder, save_carry, _native.flags())
+        if out is not None:
+            return out
     return StickBreakingAttention.apply(q, k, v, inv_temp, attend_current, bool(add_remainder), bool(save_carry))

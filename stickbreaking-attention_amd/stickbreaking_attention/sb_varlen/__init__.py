@@ -59,8 +59,10 @@ def sb_attn_varlen(q, k, v, cu_seqlens, max_seqlens=None, inv_temp=None, zero_st
     followed by a read of the scheduler's status word (one synchronisation per call) and a ``ValueError`` that says
     which check failed; never understate ``max_seqlens``."""
     if _native.use_ext():
-        return _native.ext().varlen(q, k, v, cu_seqlens, int(max_seqlens) if max_seqlens else None, inv_temp, zero_start,
-                                    attend_current, add_remainder, save_carry, _native.flags())
+        out = _native.ext().varlen(q, k, v, cu_seqlens, int(max_seqlens) if max_seqlens else None, inv_temp, zero_start,
+                                   attend_current, add_remainder, save_carry, _native.flags())
+        if out is not None:
+            return out
     # The lengths are on the host when cu_seqlens was given as a CPU tensor, or after the one device-to-host copy that
     # stands in for the reference's `assert cu_seqlens[0] == 0` (sb_varlen/__init__.py:71-73, the same host sync).
     # They are then validated there and the carry buffer is sized exactly; a device-only cu_seqlens is validated by
@@ -88,6 +90,8 @@ def sb_attn_varlen_(q, k, v, inv_temp, cu_seqlens, max_seqlens, attend_current):
     """Positional form of sb_varlen/__init__.py:80-81: ``cu_seqlens`` holds sequence ends, no leading zero."""
     cu_seqlens = _native.prepare_cu_seqlens(cu_seqlens, q.device)
     if _native.use_ext():
-        return _native.ext().varlen(q, k, v, cu_seqlens, int(max_seqlens) if max_seqlens else None, inv_temp, False,
-                                    attend_current, False, True, _native.flags())
+        out = _native.ext().varlen(q, k, v, cu_seqlens, int(max_seqlens) if max_seqlens else None, inv_temp, False,
+                                   attend_current, False, True, _native.flags())
+        if out is not None:
+            return out
     return StickBreakingAttention.apply(q, k, v, cu_seqlens, max_seqlens, inv_temp, attend_current, False)

@@ -147,10 +147,12 @@ typedef struct SbaArgs {
                                   (head_dim 128, 16-bit, 16-byte aligned rows, a head count that is a multiple of 8, no
                                   add_remainder) ONE kernel in which the key tiles of a sequence hand the row prefix
                                   sums and the partial dQ to each other through the L2; the two kernels otherwise.
-                                  0: the one kernel where it applies AND was measured to be the faster one: no
-                                  sequence longer than 256 tokens, or at most 32 heads with (total_tokens / num_seqs) *
-                                  num_heads >= 32768 and max_seqlen * num_heads <= 131072 (in packed mode an overstated
-                                  max_seqlen only costs the faster choice).  A head count above 8 that is not a multiple
+                                  0: the one kernel where it applies AND was measured to be the faster one.  Up to 64 K
+                                  rows * heads: no sequence longer than 256 tokens, or at most 32 heads with
+                                  (total_tokens / num_seqs) * num_heads >= 16 K and rows * heads >= 20 K.  Beyond: no
+                                  sequence longer than 128 tokens and more than 96 on average, or at most 32 heads with
+                                  (total_tokens / num_seqs) * num_heads >= 32 K and max_seqlen * num_heads <= 192 K (in
+                                  packed mode an overstated max_seqlen only costs the faster choice).  A head count above 8 that is not a multiple
                                   of 8 is then split where that pays (long sequences): the largest multiple of 8 through
                                   the one kernel, the remaining heads through the two, one pass after the other (with
                                   trace_events, [1] and [2] then bracket the last pass's kernels only).  Must be the

@@ -83,17 +83,27 @@ int plan(const SbaArgs* a, Layout* out) {
   L.carry_bytes = align_up((size_t)L.carry_slots_per_head * a->num_heads * sizeof(float), 256);
   size_t chain_bytes = 0;
   L.chain_rows = fixed ? B * T : T;
-  // The one-kernel backward is laid out when it is asked for, or (backward_kernels 0) where it is the faster one.
-  // Measured on 256 compute units with the two backwards alternating in one process (uniform lengths and log-normal
-  // mixes, 8 to 64 heads): it wins by 9-13 % when no sequence exceeds two key tiles (nothing is handed over then), and
-  // by 2-6 % while the sequences give each of a head's workgroups between one and four key tiles of 128 (mean length
-  // x heads >= 32768, longest x heads <= 131072) at up to 32 heads; it loses 2-10 % on sequences of 512-1024 tokens
-  // (two more slots per tile than the dK/dV kernel) and 6-20 % beyond four tiles per workgroup (the partial dQ a
-  // tile finds was written too long ago to still be in the L2).
+  // The one-kernel backward is laid out when it is asked for, or (backward_kernels 0) where it is the faster one.  Measured on
+  // 256 compute units, training passes of equal sequences, both backwards in turn, its time over the two kernels':
+  //   rows x heads                       8 heads       16 heads      32 heads
+  //   < 20 K, up to 256 tokens        0.97          0.93 .. 0.97  0.95 .. 0.97
+  //   < 20 K, 1024 to 2048 tokens     1.16 .. 1.25  1.10             -              (a chain of tiles against the split kernels)
+  //   20 K .. 64 K, up to 256 tokens  0.97          0.91 .. 0.97  0.96
+  //   20 K .. 64 K, length x heads
+  //     from 16 K on                  0.79 .. 0.93  0.82 .. 0.92  0.84 .. 0.87
+  //   more, 64 tokens                    -          1.14          1.10 .. 1.17
+  //   more, 128 tokens                   -          0.98          0.91 .. 0.99      (nothing is handed over)
+  //   more, 256 to 1024 tokens        1.04 .. 1.14  1.02 .. 1.09  0.97 .. 1.09
+  //   more, length x heads 32 K       0.96          0.97          1.00
+  //   ... 64 K to 128 K               0.93 .. 0.99  0.93 .. 0.95  0.92 .. 0.96
+  //   ... 192 K                          -          0.96, 0.99    0.96, 0.99
+  //   ... 256 K                          -          1.01, 1.04    1.00, 1.10        (the partial dQ a tile finds has left the L2)
   const bool chain_shape = a->dtype != SBA_F32 && a->head_dim == 128 && (a->num_heads & 7) == 0 && !a->add_remainder;
-  const int64_t mean_len = fixed ? T : T / B;
-  const bool chain_pays = max_len <= 256 ||
-                          (a->num_heads <= 32 && mean_len * a->num_heads >= 32768 && max_len * a->num_heads <= (int64_t)512 * 256);
+  const int64_t mean_len = fixed ? T : T / B, rows_heads = L.chain_rows * a->num_heads, mean_heads = mean_len * a->num_heads;
+  const bool chain_pays = rows_heads <= 64 << 10
+                              ? max_len <= 256 || (a->num_heads <= 32 && rows_heads >= 20 << 10 && mean_heads >= 16 << 10)
+                              : (max_len <= 128 && mean_len > 96) ||
+                                    (a->num_heads <= 32 && mean_heads >= 32 << 10 && max_len * a->num_heads <= 192 << 10);
   if (chain_shape && (a->backward_kernels == 2 || (a->backward_kernels == 0 && chain_pays))) {
     L.off_chain_zero = off;
     L.off_chain_c = off;      off = align_up(off + (size_t)a->num_heads * L.chain_rows * 8, 256);

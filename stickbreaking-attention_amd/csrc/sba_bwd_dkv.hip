@@ -196,7 +196,160 @@ __device__ __forceinline__ void store_result_tile(const RowSink<T>& sink, const 
 }
 
 // ---------------------------------------------------------------------------------------------------------
-// Fast path, producer / consumer waves (runs head_dim 64; head_dim 128 runs the software-pipelined kernel below).
+// head_dim up to 64: a wave per 32 keys that does everything.
+//
+// One workgroup = 4 waves = 128 keys, swept by steps of 32 query rows, one step ahead in LDS.  Wave w keeps the K and V
+// operands of keys 32w..32w+31 and the 32 x 64 blocks of their dK and dV in registers (64 of each), recomputes P^T and dZ^T of
+// its 32 x 32 block, turns them round through a scratch of its own and contracts them.  The waves meet only where rows are
+// staged, once per step, so that the two workgroups of a CU drift apart and one's matrix and LDS phases run under the other's
+// vector ALU, which is what bounds the pass; the dP^T MFMAs are dealt among the math as in the dQ kernel.  Training passes, us,
+// against the producer/consumer kernel below, which this one replaced at head_dim 64 (in brackets: without the dealing):
+// 32 heads x 2 x 4096 1039 -> 945 (975), 12 heads x 16384 2960 -> 2620 (2725), 12 heads, 16384 tokens in sequences of
+// 256..4096 596 -> 535 (545).  Measured and not kept: 64 rows per step (+-1 %), raised priority for the MFMA phases (+-1 %), the
+// contraction a step late under the math (39 spills, +2 %), three waves per SIMD with V in LDS (77 spills, twice the time).
+// (At head_dim 128 the accumulators leave room for one wave per SIMD, and the producer/consumer kernels are the better ones.)
+constexpr int kDkv5Rows = 32, kDkv5PzStride = lds_stride<32>();
+template <typename T, int kLoad>
+__global__ __launch_bounds__(kThreads, 2) void bwd_dkv5_kernel(BwdParams p) {
+  constexpr int DH = 64, kSteps = DH / 16, kDTiles = DH / 32, kRowStride = lds_stride<DH>(), kTile = kDkv5Rows * kRowStride;
+  typedef typename Elem<T>::vec8 vec8;
+  __shared__ __attribute__((aligned(16))) T rows_lds[2][2][kTile];                            // two stages of {Q, dO}
+  __shared__ __attribute__((aligned(16))) T pz_lds[kWaves][2][32 * kDkv5PzStride];            // per wave {P, dZ}: [row][key]
+  int head, slot;
+  xcd_head_tile(blockIdx.x, p.num_heads, &head, &slot);
+  if (slot >= p.counts[kCountK]) return;
+  const Tile tile = p.k_tiles[slot];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = lane >> 5, col = lane & 31;
+  const int L = tile.seq_len, ac = p.attend_current, D = kLoad == kLoadPadded ? p.head_dim : DH;
+  const int64_t tok0 = tile.seq_start;
+  const int k0 = tile.origin + 32 * wave, u = k0 >> 5;       // this wave's keys
+  const int64_t n_qt = (L + kBlockQ - 1) / kBlockQ;
+  const T* qb = (const T*)p.q.ptr + tile.seq_id * p.q.sb + head * p.q.sh + tok0 * p.q.st;
+  const T* kb = (const T*)p.k.ptr + tile.seq_id * p.k.sb + head * p.k.sh + tok0 * p.k.st;
+  const T* vb = (const T*)p.v.ptr + tile.seq_id * p.v.sb + head * p.v.sh + tok0 * p.v.st;
+  const T* dob = (const T*)p.d_o.ptr + tile.seq_id * p.d_o.sb + head * p.d_o.sh + tok0 * p.d_o.st;
+  const int64_t slot0 = (int64_t)head * p.carry_head_stride + tile.carry_base + carry_offset(u, n_qt) - kBlockQ * (u >> 2);
+  const float* carry = p.carry + slot0;                      // + row
+  const float* prefix = p.prefix + slot0;
+  const float* drem_plane = p.drem_eff + tile.seq_id * p.drem_sb + head * p.stat_sh + tok0;
+  const int first_row = tile.origin + 1 - ac;                // first row that sees a key of the tile
+  const int t_begin = first_row < L ? first_row / kDkv5Rows : 0, t_end = first_row < L ? (L + kDkv5Rows - 1) / kDkv5Rows : 0;
+
+  const RowSource<T> qsrc = make_row_source<T, kLoad>(qb, p.q.st, L, D), dosrc = make_row_source<T, kLoad>(dob, p.d_o.st, L, D);
+  TileCopy<T, DH, kDkv5Rows, kLoad> cq, cdo;
+  // No row of the SEQUENCE in step t sees this wave's keys (nothing is recorded for rows beyond it).
+  auto unseen = [&](int t) { return k0 > min(kDkv5Rows * t + 31, L - 1) - 1 + ac; };
+  float n_prod = 1.f, n_prefix = 0.f, n_drem = 0.f;
+  auto fetch_row_scalars = [&](int t) {
+    if (unseen(t)) return;
+    const int qi = kDkv5Rows * t + col;
+    n_prod = carry[qi];
+    n_prefix = prefix[qi];
+    n_drem = qi < L ? drem_plane[qi] : 0.f;
+  };
+  if (t_begin < t_end) {
+    cq.load(qsrc, t_begin * kDkv5Rows);
+    cdo.load(dosrc, t_begin * kDkv5Rows);
+    fetch_row_scalars(t_begin);
+  }
+  vec8 kf[kSteps], vf[kSteps];
+  const int key = k0 + mfma_row_to_key32(col);
+  load_operand<T, kLoad>(kf, make_row_source<T, kLoad>(kb, p.k.st, L, D), key, half);
+  load_operand<T, kLoad>(vf, make_row_source<T, kLoad>(vb, p.v.st, L, D), key, half);
+  f32x16 dkacc[kDTiles], dvacc[kDTiles];
+#pragma unroll
+  for (int dt = 0; dt < kDTiles; dt++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) { dkacc[dt][r] = 0.f; dvacc[dt][r] = 0.f; }
+  T* const p_rows = pz_lds[wave][0];
+  T* const z_rows = pz_lds[wave][1];
+  for (int t = t_begin; t < t_end; ++t) {
+    // This stage was last read two steps ago, and every wave has passed the barrier of the step between.
+    T* const q_rows = rows_lds[t & 1][0];
+    T* const do_rows = rows_lds[t & 1][1];
+    cq.store(q_rows);
+    cdo.store(do_rows);
+    lds_barrier();
+    const float prod_in = n_prod, prefix_in = n_prefix, drem = n_drem;
+    if (t + 1 < t_end) {
+      cq.load(qsrc, (t + 1) * kDkv5Rows);
+      cdo.load(dosrc, (t + 1) * kDkv5Rows);
+      fetch_row_scalars(t + 1);
+    }
+    if (unseen(t)) continue;
+    const int w_first = kDkv5Rows * t, w_last = w_first + 31, qi = w_first + col;
+    f32x16 s[1], dp[1];
+#pragma unroll
+    for (int r = 0; r < 16; r++) { s[0][r] = 0.f; dp[0][r] = 0.f; }
+    vec8 b[kSteps];
+#pragma unroll
+    for (int kk = 0; kk < kSteps; kk++) b[kk] = lds_row8<T>(q_rows, kRowStride, col, 16 * kk + 8 * half);
+#pragma unroll
+    for (int kk = 0; kk < kSteps; kk++) s[0] = Elem<T>::mfma(kf[kk], b[kk], s[0]);
+    uint32_t pk[8], dzk[8];
+    float prod_lower, prefix_upper, prefix_next;
+    const int lim = qi < L ? qi + ac - k0 - 16 * half : 0;
+    auto math = [&](auto diag_tag) {
+      constexpr bool kDiag = decltype(diag_tag)::value;
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int kk = 0; kk < kSteps; kk++) dp[0] = Elem<T>::mfma(vf[kk], lds_row8<T>(do_rows, kRowStride, col, 16 * kk + 8 * half), dp[0]);
+      bwd_tile_math_impl<T, 1, kDiag, true>(s, dp, p.scale_log2, lim, half, drem, prod_in, prefix_in, pk, dzk, prod_lower, prefix_upper, prefix_next);
+      __builtin_amdgcn_sched_group_barrier(0x100, kSteps, 0);
+      __builtin_amdgcn_sched_group_barrier(0x402, 8, 0);
+#pragma unroll
+      for (int kk = 0; kk < kSteps; kk++) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x402, 14, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    if (k0 + 31 > w_first - 1 + ac || w_last >= L) math(std::true_type{}); else math(std::false_type{});
+#pragma unroll
+    for (int c = 0; c < 2; c++) {      // this lane's 16 consecutive keys of row `col`
+      *reinterpret_cast<u32x4*>(p_rows + col * kDkv5PzStride + 16 * half + 8 * c) = u32x4{pk[4 * c], pk[4 * c + 1], pk[4 * c + 2], pk[4 * c + 3]};
+      *reinterpret_cast<u32x4*>(z_rows + col * kDkv5PzStride + 16 * half + 8 * c) = u32x4{dzk[4 * c], dzk[4 * c + 1], dzk[4 * c + 2], dzk[4 * c + 3]};
+    }
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      const int row0 = 16 * c + 8 * half;
+      const vec8 ap = lds_col8<T>(p_rows, kDkv5PzStride, row0, 0, lane), az = lds_col8<T>(z_rows, kDkv5PzStride, row0, 0, lane);
+#pragma unroll
+      for (int dt = 0; dt < kDTiles; dt++) {
+        dvacc[dt] = Elem<T>::mfma(ap, lds_col8<T>(do_rows, kRowStride, row0, 32 * dt, lane), dvacc[dt]);
+        dkacc[dt] = Elem<T>::mfma(az, lds_col8<T>(q_rows, kRowStride, row0, 32 * dt, lane), dkacc[dt]);
+      }
+    }
+  }
+  if (k0 >= L) return;
+  if (p.add_rem) {      // the forward wrote o + rem * v: dv_j gains rem_j * d_o_j
+    const float* stat = p.row_stat + tile.seq_id * p.stat_sb + head * p.stat_sh + tok0;
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const int j = k0 + 8 * (r >> 2) + 4 * half + (r & 3);
+      const float rem = j < L ? fast_exp2(stat[j]) : 0.f;
+#pragma unroll
+      for (int dt = 0; dt < kDTiles; dt++)
+        if (j < L && 32 * dt + col < D) dvacc[dt][r] += rem * (float)dob[(int64_t)j * p.d_o.st + 32 * dt + col];
+    }
+  }
+  const RowSink<T> dk_sink = make_row_sink<T>((T*)p.dk.ptr + tile.seq_id * p.dk.sb + head * p.dk.sh + tok0 * p.dk.st, p.dk.st, L, D);
+  const RowSink<T> dv_sink = make_row_sink<T>((T*)p.dv.ptr + tile.seq_id * p.dv.sb + head * p.dv.sh + tok0 * p.dv.st, p.dv.st, L, D);
+#pragma unroll
+  for (int dt = 0; dt < kDTiles; dt++) {
+    store_result_tile<T, kLoad>(dk_sink, dkacc[dt], p.logit_scale, k0, 32 * dt, half, col, lane, p_rows, D);
+    store_result_tile<T, kLoad>(dv_sink, dvacc[dt], 1.f, k0, 32 * dt, half, col, lane, z_rows, D);
+  }
+}
+
+template <typename T, int kLoad>
+static hipError_t launch_dkv5(const BwdParams& p, hipStream_t stream) {      // (a sequence has as many tiles of 128 keys as of 128 rows)
+  hipLaunchKernelGGL((bwd_dkv5_kernel<T, kLoad>), dim3((unsigned)(p.max_tiles * p.num_heads)), dim3(kThreads), 0, stream, p);
+  return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------------------------------------
+// Producer / consumer waves on 64-key tiles (head_dim beyond 64, calls with too few tiles for the 128-key kernel below).
 //
 // One workgroup = 8 waves = one 64-key tile, swept by query tiles of 64 rows.  Waves 0-3 are PRODUCERS: wave
 // (rg, g) takes rows 32*rg .. +31 against the 32-key sub-tile g (one MFMA row tile, 16 keys per lane, that
@@ -389,13 +542,12 @@ __global__ __launch_bounds__(kDkv3Threads) void bwd_dkv3_kernel(BwdParams p) {
     }  // rounds of the tile walk (producers)
   } else {
     if (w < n_tiles) stage_first(next_tile);
-    // Output blocks of this consumer wave.  head_dim 128: both 32-key row tiles x columns 32*wave .. +31;
-    // head_dim 64: row tile wave/2 x columns 32*(wave%2) .. +31.
-    constexpr int kMT = DH == 128 ? 2 : 1;
-    const int mt0 = DH == 128 ? 0 : wave >> 1, ct = DH == 128 ? wave : wave & 1;
+    // Output blocks of this consumer wave: both 32-key row tiles x columns 32*wave .. +31.
+    constexpr int kMT = 2;
+    const int ct = wave;
     f32x16 dkacc[kMT], dvacc[kMT];
     // The results of a tile are stored during the first step of the NEXT tile, when the consumers have nothing to
-    // contract yet (and after the last tile): acc[mt][r] is key origin + 32*(mt0 + mt) + 8*(r/4) + 4*half + r%4,
+    // contract yet (and after the last tile): acc[mt][r] is key origin + 32*mt + 8*(r/4) + 4*half + r%4,
     // column 32*ct + col.
     bool pending = false;
     Tile done_tile = next_tile;
@@ -412,7 +564,7 @@ __global__ __launch_bounds__(kDkv3Threads) void bwd_dkv3_kernel(BwdParams p) {
         for (int mt = 0; mt < kMT; mt++)
 #pragma unroll
           for (int r = 0; r < 16; r++) {
-            const int key = tl_j0 + 32 * (mt0 + mt) + 8 * (r >> 2) + 4 * half + (r & 3);
+            const int key = tl_j0 + 32 * mt + 8 * (r >> 2) + 4 * half + (r & 3);
             if (key < tl_len && d < D)
               dvacc[mt][r] += fast_exp2(p.row_stat[tl.seq_id * p.stat_sb + head * p.stat_sh + tl_tok0 + key]) *
                               (float)dob[(int64_t)key * p.d_o.st + d];
@@ -424,8 +576,8 @@ __global__ __launch_bounds__(kDkv3Threads) void bwd_dkv3_kernel(BwdParams p) {
       T* scratch = lds + Lds::kQ + 4 * Lds::kQdoTile + wave * (32 * lds_stride<32>());
 #pragma unroll
       for (int mt = 0; mt < kMT; mt++) {
-        store_result_tile<T, kLoad>(dk_sink, dkacc[mt], p.logit_scale, tl_j0 + 32 * (mt0 + mt), 32 * ct, half, col, lane, scratch, D);
-        store_result_tile<T, kLoad>(dv_sink, dvacc[mt], 1.f, tl_j0 + 32 * (mt0 + mt), 32 * ct, half, col, lane, scratch, D);
+        store_result_tile<T, kLoad>(dk_sink, dkacc[mt], p.logit_scale, tl_j0 + 32 * mt, 32 * ct, half, col, lane, scratch, D);
+        store_result_tile<T, kLoad>(dv_sink, dvacc[mt], 1.f, tl_j0 + 32 * mt, 32 * ct, half, col, lane, scratch, D);
       }
     };
   for (int slot = w; slot < n_tiles;) {
@@ -491,9 +643,9 @@ __global__ __launch_bounds__(kDkv3Threads) void bwd_dkv3_kernel(BwdParams p) {
           vec8 bq = lds_col8<T>(q_lds, kRowStride, row0, 32 * ct, lane);
 #pragma unroll
           for (int mt = 0; mt < kMT; mt++) {
-            vec8 ap = lds_col8<T>(p_lds, kPStride, row0, 32 * (mt0 + mt), lane);
+            vec8 ap = lds_col8<T>(p_lds, kPStride, row0, 32 * mt, lane);
             dvacc[mt] = Elem<T>::mfma(ap, bd, dvacc[mt]);
-            vec8 az = lds_col8<T>(dz_lds, kPStride, row0, 32 * (mt0 + mt), lane);
+            vec8 az = lds_col8<T>(dz_lds, kPStride, row0, 32 * mt, lane);
             dkacc[mt] = Elem<T>::mfma(az, bq, dkacc[mt]);
           }
         }
@@ -917,18 +1069,17 @@ static hipError_t launch_one(const BwdParams& p, int max_tiles, hipStream_t stre
 
 template <typename T>
 static hipError_t launch_t(const BwdParams& p, int max_tiles, hipStream_t stream) {
-  // head_dim 64 measures slightly faster on the 64-key kernel (its steps are already short).
   const bool wide = p.head_dim > 64;
   if (p.split && wide)
     return p.load == kLoadAligned ? launch_dkv3<T, 128, kLoadAligned>(p, max_tiles, stream) : launch_dkv3<T, 128, kLoadPadded>(p, max_tiles, stream);
-  if (p.load == kLoadAligned) return wide ? launch_dkv4<T, 128, kLoadAligned>(p, max_tiles, stream) : launch_dkv3<T, 64, kLoadAligned>(p, max_tiles, stream);
-  if (p.load == kLoadPadded) return wide ? launch_dkv4<T, 128, kLoadPadded>(p, max_tiles, stream) : launch_dkv3<T, 64, kLoadPadded>(p, max_tiles, stream);
+  if (p.load == kLoadAligned) return wide ? launch_dkv4<T, 128, kLoadAligned>(p, max_tiles, stream) : launch_dkv5<T, kLoadAligned>(p, stream);
+  if (p.load == kLoadPadded) return wide ? launch_dkv4<T, 128, kLoadPadded>(p, max_tiles, stream) : launch_dkv5<T, kLoadPadded>(p, stream);
   return wide ? launch_one<T, 128>(p, max_tiles, stream) : launch_one<T, 64>(p, max_tiles, stream);
 }
 
 // Keys per key tile of the kernel launch_bwd_dkv will pick for these parameters.
 int dkv_key_tile(const BwdParams& p) {
-  return p.load != kLoadScalar && p.head_dim > 64 && !p.split ? kDkv4Keys : kBlockK;
+  return p.load != kLoadScalar && !p.split ? kDkv4Keys : kBlockK;
 }
 
 hipError_t launch_bwd_dkv(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream) {

@@ -231,13 +231,19 @@ int clear_wgs(const sba::SchedParams& sp) {
   return (int)(n > 64 ? 64 : n);
 }
 
+// Whether the dK/dV kernel of a call with few key tiles runs: the one-kernel backward, where it is laid out and the rows allow
+// it, takes such calls itself.
+bool split_keys(const SbaArgs* a, const Layout& L, int64_t heads, int load) {
+  return !(L.chain_zero_bytes > 0 && load == sba::kLoadAligned) && few_key_tiles(a, heads, load);
+}
+
 // Keys per key tile of the backward that will follow a forward, as far as the forward's tensors tell.
 int expected_key_tile(const SbaArgs* a, const Layout& L) {
   if (a->dtype == SBA_F32) return kBlockK;
   sba::BwdParams p{};
   p.head_dim = a->head_dim;
   p.load = row_load(a, {&a->q, &a->k, &a->v});
-  p.split = L.chain_zero_bytes == 0 && few_key_tiles(a, a->num_heads, p.load);
+  p.split = split_keys(a, L, a->num_heads, p.load);
   return sba::dkv_key_tile(p);
 }
 
@@ -464,7 +470,7 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* 
   p.max_tiles = (int32_t)L.max_q_tiles;
   p.total_tokens = a->total_tokens;
   p.load = bwd_load(a);
-  p.split = L.chain_zero_bytes == 0 && few_key_tiles(a, stat_heads, p.load);
+  p.split = split_keys(a, L, stat_heads, p.load);
   // One kernel (the key tiles of a sequence hand C and partial dQ to each other) where it applies, else dQ then dK/dV.
   const bool chain = bwd_is_chained(a, L);
   if (chain) {
@@ -615,7 +621,7 @@ bool prepared_fits(const SbaArgs* a) {
   BwdParams p{};
   p.head_dim = a->head_dim;
   p.load = bwd_load(a);
-  p.split = L.chain_zero_bytes == 0 && few_key_tiles(a, a->num_heads, p.load);
+  p.split = split_keys(a, L, a->num_heads, p.load);
   return a->dtype == SBA_F32 || dkv_key_tile(p) == expected_key_tile(a, L);
 }
 

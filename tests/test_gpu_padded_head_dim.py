@@ -38,3 +38,28 @@ def test_head_dim_between_nans_against_oracle(gpu_device, D, dtype, pad, add_rem
         ref = orc.with_remainder(ref, d[2], d[3])
     for n, a, b in zip(NAMES, got, ref):
         tol_check(n, a, b, dtype, f"D={D}")
+
+
+@pytest.mark.parametrize("odd", ["none", "do", "all"])
+def test_rows_off_16_bytes_where_the_one_kernel_backward_is_laid_out(gpu_device, odd):
+    """A call the one-kernel backward takes if its rows allow it: with a gradient, or everything, at odd addresses the two kernels
+    do (and the schedule the forward prepared fits, or is made again)."""
+    lengths, H, D, dtype = [2600, 130], 8, 128, torch.bfloat16
+    T = sum(lengths)
+    g = torch.Generator().manual_seed(7)
+    host = [torch.randn(H, T, D, generator=g).to(dtype) for _ in range(4)] + [torch.randn(H, T, generator=g).to(dtype)]
+
+    def placed(t, shift):
+        buf = torch.zeros(t.numel() + shift, dtype=dtype, device=gpu_device)
+        buf[shift:] = t.to(gpu_device).flatten()
+        return buf[shift:].view(t.shape)
+
+    q, k, v = (placed(t, 1 if odd == "all" else 0).requires_grad_() for t in host[:3])
+    do = placed(host[3], 0 if odd == "none" else 1)
+    cu = torch.tensor(np.cumsum(lengths), dtype=torch.int32)
+    o, rem = sb_attn_varlen(q, k, v, cu, max(lengths), zero_start=False)
+    got = (o, rem, *torch.autograd.grad([o, rem], [q, k, v], [do, host[4].to(gpu_device)]))
+    d = [t[[0, 7]].double() for t in host]
+    ref = orc.varlen_stream(d[0], d[1], d[2], cu, do=d[3], drem=d[4], dtype=torch.float64)
+    for n, a, b in zip(NAMES, got, ref):
+        tol_check(n, a[[0, 7]], b, dtype, f"odd: {odd}")

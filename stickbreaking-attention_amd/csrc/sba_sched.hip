@@ -111,29 +111,38 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
   }
   __syncthreads();
 
-  // Pass 2: each sequence takes a contiguous range of slots in its class; one wave per sequence.
-  for (int s = wave; s < p.num_seqs; s += nwaves) {
-    int start, len;
-    seq_bounds(p, s, &start, &len);
-    const int nq = (len + kBlockQ - 1) / kBlockQ, nk = (len + p.key_tile - 1) / p.key_tile;
+  // Pass 2: each sequence takes a contiguous range of slots in its class.  A wave holds `group` sequences, one per lane; a lane
+  // writes the tiles of a short sequence itself, the wave those of a long one together.  (A wave per sequence took 1.1 us of
+  // dependent loads for each: 151 us for 2049 sequences.)
+  constexpr int kOwnTiles = 4;
+  const int group = min(64, (p.num_seqs + nwaves - 1) / nwaves);
+  for (int s0 = wave * group; s0 < p.num_seqs; s0 += nwaves * group) {
+    const int s = s0 + lane;
+    int start = 0, len = 0, qbase = 0, kbase = 0;
+    int64_t cbase = 0;
+    const bool mine = lane < group && s < p.num_seqs;
+    if (mine) {
+      seq_bounds(p, s, &start, &len);
+      if (p.want_carry_base) cbase = p.carry_base[s];      // written above by this workgroup
+    }
+    const int nq = (len + kBlockQ - 1) / kBlockQ, nk = p.want_key_tiles ? (len + p.key_tile - 1) / p.key_tile : 0;
     const int cls = min(nq, kBins - 1);
-    int qbase = 0, kbase = 0;
-    if (lane == 0) {
-      if (nq) qbase = atomicAdd(&qbins[cls], nq);
-      if (nk && p.want_key_tiles) kbase = atomicAdd(&kbins[cls], nk);
+    if (nq) qbase = atomicAdd(&qbins[cls], nq);
+    if (nk) kbase = atomicAdd(&kbins[cls], nk);
+    Tile d;
+    d.seq_start = start; d.seq_len = len; d.seq_id = s; d.carry_base = cbase;
+    if (nq <= kOwnTiles) {
+      for (int t = 0; t < nq; t++) { d.origin = (nq - 1 - t) * kBlockQ; p.q_tiles[qbase + t] = d; }      // heaviest first: the last one
+      for (int t = 0; t < nk; t++) { d.origin = t * p.key_tile; p.k_tiles[kbase + t] = d; }             // ... and the first one
     }
-    qbase = __shfl(qbase, 0);
-    kbase = __shfl(kbase, 0);
-    const int64_t cbase = p.want_carry_base ? p.carry_base[s] : 0;      // written above by this workgroup
-    for (int t = lane; t < nq; t += 64) {        // heaviest query tile (the last one) first
-      Tile d; d.seq_start = start; d.seq_len = len; d.origin = (nq - 1 - t) * kBlockQ; d.seq_id = s; d.carry_base = cbase;
-      p.q_tiles[qbase + t] = d;
-    }
-    if (p.want_key_tiles) {
-      for (int t = lane; t < nk; t += 64) {      // heaviest key tile (the first one) first
-        Tile d; d.seq_start = start; d.seq_len = len; d.origin = t * p.key_tile; d.seq_id = s; d.carry_base = cbase;
-        p.k_tiles[kbase + t] = d;
-      }
+    for (uint64_t left = __ballot(nq > kOwnTiles); left; left &= left - 1) {
+      const int j = __builtin_ctzll(left);
+      const int nq_j = __shfl(nq, j), nk_j = __shfl(nk, j), qbase_j = __shfl(qbase, j), kbase_j = __shfl(kbase, j);
+      Tile e;
+      e.seq_start = __shfl(start, j); e.seq_len = __shfl(len, j); e.seq_id = __shfl(s, j);
+      e.carry_base = (int64_t)(uint32_t)__shfl((int)cbase, j) | (int64_t)__shfl((int)(cbase >> 32), j) << 32;
+      for (int t = lane; t < nq_j; t += 64) { e.origin = (nq_j - 1 - t) * kBlockQ; p.q_tiles[qbase_j + t] = e; }
+      for (int t = lane; t < nk_j; t += 64) { e.origin = t * p.key_tile; p.k_tiles[kbase_j + t] = e; }
     }
   }
   __syncthreads();

@@ -175,14 +175,14 @@ int row_load(const SbaArgs* a, const SbaTensor* const (&tensors)[N]) {
 // the lines lie lower; training passes: head_dim 128, 21 K (6 x 1740) 205 / 210, 28 K (7 x 1024, 8 x 1740, 14 x 512)
 // 166 / 149, 249 / 226, 128 / 111; head_dim 64, 33 K to 41 K (16 x 2048, 10 x 1740, 9 x 1024, 10 x 4096) 201 / 195, 168 / 177, 129 / 136,
 // 356 / 397, 51 K (12 x 512, 13 x 1024, 15 x 1740, 26 x 2048) 114 / 110, 164 / 154, 222 / 206, 284 / 253.
-// (Several: none holds more than a quarter of the rows.  7 heads x 50, 8191 tokens of which one sequence has 4001: 185 / 207.)
+// (Several: none holds more than a sixth of the rows.  7 heads x 50, 8191 tokens, a log-normal mix: 185 / 207.)
 // `heads` is the head count of the caller's call, also where the backward takes them through in groups: the groups then run the
 // kernels, and give the bits, of one pass, and products are rebuilt by the kernel whose forward would have kept them.
 bool few_tiles(const SbaArgs* a, int64_t heads, int load) {
   if (a->dtype == SBA_F32 || load == sba::kLoadScalar) return false;
   const int64_t seq_rows = a->total_tokens * (a->cu_seqlens ? 1 : a->num_seqs), rows = seq_rows * heads;
   const int64_t longest = a->max_seqlen > 0 && a->max_seqlen < a->total_tokens ? a->max_seqlen : a->total_tokens;
-  const bool several = 4 * longest <= seq_rows;
+  const bool several = 6 * longest <= seq_rows;
   return rows < (a->head_dim > 64 ? (several ? 20 << 10 : 30 << 10) : several ? 40 << 10 : 60 << 10);
 }
 // The same for dK/dV: below, head_dim up to 64 splits the rows over the waves (130 K rows x heads: 542 / 565 us at 8192

@@ -277,11 +277,14 @@ double scale_of(const std::optional<double>& inv_temp, const Tensor& q) {
   return inv_temp ? *inv_temp : 1.0 / std::sqrt((double)q.size(-1));
 }
 
-// None where the call is not ordinary.
+// None where the call is not ordinary.  From the first tensor operation on, the interpreter's lock is given up: a device-to-host
+// copy of cu_seqlens, a copy of host lengths to the device and an allocator that has to wait all wait for the stream, and another
+// Python thread may be the one that what the stream waits for depends on.
 std::optional<std::tuple<Tensor, Tensor>> fixed(py::handle hq, py::handle hk, py::handle hv, std::optional<double> inv_temp,
                                                 bool attend_current, bool add_remainder, bool save_carry, int64_t flags) {
   if (!ordinary(hq, hk, hv)) return std::nullopt;
-  const Tensor &q = THPVariable_Unpack(hq.ptr()), &k = THPVariable_Unpack(hk.ptr()), &v = THPVariable_Unpack(hv.ptr());
+  const Tensor q = THPVariable_Unpack(hq.ptr()), k = THPVariable_Unpack(hk.ptr()), v = THPVariable_Unpack(hv.ptr());
+  const py::gil_scoped_release unlocked;
   require_gpu(q); require_gpu(k); require_gpu(v);
   Call c;
   c.fixed = true;
@@ -296,7 +299,8 @@ std::optional<std::tuple<Tensor, Tensor>> varlen(py::handle hq, py::handle hk, p
                                                  std::optional<int64_t> max_seqlens, std::optional<double> inv_temp, bool zero_start,
                                                  bool attend_current, bool add_remainder, bool save_carry, int64_t flags) {
   if (!ordinary(hq, hk, hv)) return std::nullopt;
-  const Tensor &q = THPVariable_Unpack(hq.ptr()), &k = THPVariable_Unpack(hk.ptr()), &v = THPVariable_Unpack(hv.ptr());
+  const Tensor q = THPVariable_Unpack(hq.ptr()), k = THPVariable_Unpack(hk.ptr()), v = THPVariable_Unpack(hv.ptr());
+  const py::gil_scoped_release unlocked;
   Call c;
   c.leading_zero = zero_start;
   c.attend_current = attend_current; c.add_remainder = add_remainder;
@@ -311,6 +315,7 @@ std::optional<std::tuple<Tensor, Tensor>> varlen(py::handle hq, py::handle hk, p
   if (zero_start) {
     const int64_t first = host.scalar_type() == at::kLong ? *host.const_data_ptr<int64_t>() : *host.const_data_ptr<int32_t>();
     if (first != 0) {
+      const py::gil_scoped_acquire locked;
       PyErr_SetString(PyExc_AssertionError, "cu_seqlens[0] must be 0");
       throw py::error_already_set();
     }

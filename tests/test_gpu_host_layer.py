@@ -1,5 +1,8 @@
 """The torch host layer of eager calls: gradients arriving through only one of the two outputs, and graphs kept for a second
-backward, against the same call with both gradients given."""
+backward, against the same call with both gradients given; other Python threads while a call waits for the GPU."""
+import threading
+import time
+
 import pytest
 import torch
 
@@ -27,3 +30,38 @@ def test_gradient_through_either_output_and_a_second_backward(gpu_device, throug
     for got, want in zip(torch.autograd.grad(outs, [q, k, v], grads), both):
         assert torch.equal(got, want)
     assert all(t.abs().max() > 0 for t in both[:2])
+
+
+@pytest.mark.parametrize("where", ["device", "host"])
+def test_other_threads_run_while_a_call_waits_for_the_gpu(gpu_device, where):
+    """Reading the lengths back (or sending them) waits for everything the stream holds; the interpreter is not held meanwhile."""
+    q, k, v = (torch.randn(2, 200, 64, device=gpu_device, dtype=torch.bfloat16) for _ in range(3))
+    cu = torch.tensor([0, 70, 200], dtype=torch.int32, device=gpu_device if where == "device" else "cpu")
+    sb_attn_varlen(q, k, v, cu, 130)
+    start, end = torch.cuda.Event(True), torch.cuda.Event(True)
+    torch.cuda._sleep(1 << 20)
+    start.record()
+    torch.cuda._sleep(1 << 20)
+    end.record()
+    torch.cuda.synchronize()
+    cycles = int((1 << 20) * 150 / start.elapsed_time(end))      # of a kernel of 150 ms
+    ticks, stop = [], threading.Event()
+
+    def tick():
+        while not stop.wait(0.0005):
+            ticks.append(time.perf_counter())
+
+    thread = threading.Thread(target=tick)
+    thread.start()
+    try:
+        time.sleep(0.01)
+        torch.cuda._sleep(cycles)
+        t0 = time.perf_counter()
+        sb_attn_varlen(q, k, v, cu, 130)
+        t1 = time.perf_counter()
+    finally:
+        stop.set()
+        thread.join()
+    print(f"{where}: the call took {1e3 * (t1 - t0):.1f} ms", flush=True)
+    assert where == "host" or t1 - t0 > 0.04
+    assert t1 - t0 < 0.04 or sum(t0 < t < t1 for t in ticks) > (t1 - t0) / 0.02

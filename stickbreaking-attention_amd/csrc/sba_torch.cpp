@@ -161,10 +161,20 @@ Outputs run_forward(const Call& c, const Tensor& q, const Tensor& k, const Tenso
   return out;
 }
 
-// `state` as the forward left it; `fresh`: no backward has run on its schedule yet.
-variable_list run_backward(const Call& c, Tensor d_o, Tensor d_rem, const Tensor& q, const Tensor& k, const Tensor& v,
-                           const Tensor& state, bool have_carry, bool fresh) {
+// `state` as the forward left it; `fresh`: no backward has run on its schedule yet.  What a saved-tensor hook hands back may lie
+// in another place, and in another layout, than what the forward saved.
+variable_list run_backward(Call c, Tensor d_o, Tensor d_rem, Tensor q, Tensor k, Tensor v, Tensor state, bool have_carry,
+                           bool fresh) {
+  for (const Tensor* t : {&q, &k, &v, &state}) require_gpu(*t);
+  same_dtype(q, k, "k");
+  same_dtype(q, v, "v");
   const c10::DeviceGuard guard(q.device());
+  q = rows_contiguous(q); k = rows_contiguous(k); v = rows_contiguous(v);
+  if (!c.fixed) {
+    require_gpu(c.cu);
+    c.cu = c.cu.contiguous();
+  }
+  if (!state.is_contiguous() || ((uintptr_t)state.data_ptr() & 255)) state = state.clone(at::MemoryFormat::Contiguous);
   if (!d_o.defined()) d_o = at::zeros_like(q);
   require_gpu(d_o);
   same_dtype(q, d_o, "do");
@@ -182,6 +192,7 @@ variable_list run_backward(const Call& c, Tensor d_o, Tensor d_rem, const Tensor
   a.recompute_carry = !have_carry;      // the forward kept no products: rebuild them in the backward's workspace
   size_t sched_bytes = 0, rest_bytes = 0, carry_bytes = 0;
   check(sba::prepared_bytes(&a, &sched_bytes, &rest_bytes, &carry_bytes), "sba_workspace_bytes");
+  TORCH_CHECK((size_t)state.numel() == sched_bytes + row_stat_bytes(q) + (have_carry ? carry_bytes : 0), "saved state of another size");
   char* const base = (char*)state.data_ptr();
   a.row_stat = (float*)(base + sched_bytes);
   a.carry = have_carry ? (float*)(base + sched_bytes + row_stat_bytes(q)) : nullptr;

@@ -1,10 +1,12 @@
 """The torch host layer of eager calls: gradients arriving through only one of the two outputs, and graphs kept for a second
-backward, against the same call with both gradients given; other Python threads while a call waits for the GPU."""
+backward, against the same call with both gradients given; other Python threads while a call waits for the GPU;
+what saved-tensor hooks and checkpointing hand back to the backward."""
 import threading
 import time
 
 import pytest
 import torch
+from torch.utils.checkpoint import checkpoint
 
 from stickbreaking_attention import sb_attn, sb_attn_varlen
 
@@ -65,3 +67,51 @@ def test_other_threads_run_while_a_call_waits_for_the_gpu(gpu_device, where):
     print(f"{where}: the call took {1e3 * (t1 - t0):.1f} ms", flush=True)
     assert where == "host" or t1 - t0 > 0.04
     assert t1 - t0 < 0.04 or sum(t0 < t < t1 for t in ticks) > (t1 - t0) / 0.02
+
+
+def moved_by_a_byte(t):
+    if t.dtype != torch.uint8:
+        return t
+    buf = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    buf[1:] = t
+    return buf[1:]
+
+
+def other_strides(t):
+    return t.transpose(-1, -2).contiguous().transpose(-1, -2) if t.dim() >= 3 else t
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("how", ["host and back", "by a byte", "other strides", "left on the host", "checkpoint", "reentrant checkpoint"])
+def test_saved_tensors_that_come_back_different(gpu_device, how, packed, dtype):
+    H, L, D = 8, 200, 128
+    shape = (H, L, D) if packed else (1, H, L, D)
+    q, k, v, do = (torch.randn(shape, device=gpu_device).to(dtype) for _ in range(4))
+    drem = torch.randn(shape[:-1], device=gpu_device).to(dtype)
+    for t in (q, k, v):
+        t.requires_grad_()
+    cu = torch.tensor([70, L], dtype=torch.int32, device=gpu_device)
+
+    def call(q, k, v):
+        return sb_attn_varlen(q, k, v, cu, 130, zero_start=False) if packed else sb_attn(q, k, v)
+
+    def grads(out):
+        return torch.autograd.grad(out, [q, k, v], [do, drem])
+
+    want = grads(call(q, k, v))
+    if "checkpoint" in how:
+        leaves = [t.detach().requires_grad_() for t in (q, k, v)]      # (a reentrant one needs .backward())
+        torch.autograd.backward(checkpoint(call, *leaves, use_reentrant=how.startswith("re")), [do, drem])
+        got = [t.grad for t in leaves]
+    else:
+        pack, unpack = {"host and back": (lambda t: t.cpu(), lambda t: t.to(gpu_device)), "by a byte": (lambda t: t, moved_by_a_byte),
+                        "other strides": (lambda t: t, other_strides), "left on the host": (lambda t: t.cpu(), lambda t: t)}[how]
+        with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
+            out = call(q, k, v)
+        if how == "left on the host":
+            with pytest.raises(RuntimeError, match="GPU only"):
+                grads(out)
+            return
+        got = grads(out)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))

@@ -255,8 +255,11 @@ struct TileCopy {
 // one reciprocal of prod(1 + e) per kGroup keys: 20 transcendentals per 16 keys instead of 32, 5.5 instructions per key
 // besides instead of 7.5.  Vector-ALU issue is what bounds this kernel (75 % busy at head_dim 64, 60 % at 128): 32 heads
 // x 8192 x 128 653 -> 606 us, 32 heads x 2 x 4096 x 64 227 -> 188 us.  The product of a group has to stay far from
-// overflow; where it does not (four keys whose logits add up to 100 octaves), the wave takes the weights downwards as
-// differences of the running product, one reciprocal per key, where e = inf gives a factor 0 and the whole remaining stick.
+// overflow; where it does not (keys whose logits add up to 100 octaves in one group of a lane), that lane takes the weights
+// downwards as differences of the running product, one reciprocal per key, where e = inf gives a factor 0 and the whole
+// remaining stick.  A wave with such a lane does both and every lane keeps its own: a row's bits depend on no other row.  Below
+// 100 octaves a product below a group can still underflow where the stick above it is shorter than 2^-26; what is then lost
+// is less than one rounding of the row's sum of weights.
 // Hidden keys (diagonal tiles only) get e = 0: factor 1, weight 0.
 template <int N>
 struct Weights {
@@ -264,7 +267,7 @@ struct Weights {
   float t[N];                   // e, then the weights
   float below[N / kGroup];      // 1 / prod(1 + e) of a group, then the running product below it
   float run;                    // product over all N keys
-  bool tame;
+  bool mine, tame;              // whether the products of this lane's groups are far from overflow; whether every lane's are
 
   // Up to the product over the keys; key R is visible iff R < lim.
   template <bool kDiagonal, int NT>
@@ -284,7 +287,8 @@ struct Weights {
       below[g] = prod_g;
       most += prod_g;
     }
-    tame = !__any(!(most < 0x1p100f));
+    mine = most < 0x1p100f;
+    tame = !__any(!mine);
     run = 1.f;
     if (tame) {
 #pragma unroll
@@ -292,13 +296,13 @@ struct Weights {
         run *= fast_rcp(below[g]);
         below[g] = run;
       }
-    } else {
+    } else {      // lanes of both kinds, each by the way it would take among lanes like itself
+      float odd = 1.f;
 #pragma unroll
-      for (int R = N - 1; R >= 0; --R) {
-        const float before = run;
-        run *= fast_rcp(1.f + t[R]);
-        t[R] = before - run;
-      }
+      for (int R = N - 1; R >= 0; --R) { odd *= fast_rcp(1.f + t[R]); __builtin_amdgcn_sched_barrier(0); }
+#pragma unroll
+      for (int g = N / kGroup - 1; g >= 0; --g) run *= fast_rcp(below[g]);
+      run = mine ? run : odd;
     }
   }
   // The weights; `seed`: the product above the N keys.
@@ -309,13 +313,39 @@ struct Weights {
         float r = below[g] * seed;
 #pragma unroll
         for (int i = 0; i < kGroup; i++) {
-          t[kGroup * g + i] *= r;
-          if (i + 1 < kGroup) r += t[kGroup * g + i];
+          const float e = t[kGroup * g + i];
+          t[kGroup * g + i] = e * r;
+          r = fmaf(e, r, r);
         }
       }
-    } else {
+    } else {      // (taken from t again: nothing but t and `mine` is kept for it)
+      float b[N / kGroup];
+      float r = 1.f;
 #pragma unroll
-      for (int R = 0; R < N; R++) t[R] *= seed;
+      for (int g = N / kGroup - 1; g >= 0; --g) {
+        float prod_g = 1.f + t[kGroup * g];
+#pragma unroll
+        for (int i = 1; i < kGroup; i++) prod_g = fmaf(prod_g, t[kGroup * g + i], prod_g);
+        r *= fast_rcp(prod_g);
+        b[g] = r;
+      }
+#pragma unroll
+      for (int g = 0; g < N / kGroup; g++) {
+        r = b[g] * seed;
+#pragma unroll
+        for (int i = 0; i < kGroup; i++) {
+          const float e = t[kGroup * g + i];
+          t[kGroup * g + i] = mine ? e * r : e;
+          r = fmaf(e, r, r);
+        }
+      }
+      float odd = 1.f;
+#pragma unroll
+      for (int R = N - 1; R >= 0; --R) {
+        const float before = odd, omb = fast_rcp(1.f + t[R]);
+        odd *= omb;
+        t[R] = mine ? t[R] : fmaf(-before, omb, before) * seed;
+      }
     }
   }
 };

@@ -1,9 +1,10 @@
-"""The forward's two ways through a tile's weights: groups of keys whose odds multiply up to any size (the wave then takes them
-one by one), next to tame ones in the same wave, against the float64 oracle."""
+"""The forward's two ways through a tile's weights: groups of keys whose odds multiply up to any size (the lane then takes them
+one by one), next to tame ones in the same wave, against the float64 oracle; and that neither way shows in another row's bits."""
 import pytest
 import torch
 
 from oracle import sb_oracle as orc
+from stickbreaking_attention import sb_attn_varlen
 from test_gpu_parity import NAMES, run_varlen, tol_check
 
 pytestmark = pytest.mark.gpu
@@ -28,3 +29,24 @@ def test_logits_of_any_size(gpu_device, D, low, high):
     for n, a, b in list(zip(NAMES, got, ref))[:2]:
         tol_check(n, a, b, torch.bfloat16, f"logits {low}..{high}")
     assert all(torch.isfinite(t).all() for t in got)
+
+
+@pytest.mark.parametrize("H,D", [(2, 64), (2, 80), (2, 128), (100, 64), (100, 50), (100, 96), (100, 128)])
+def test_a_rows_bits_depend_on_no_other_row(gpu_device, H, D):
+    """Few and many heads: the kernels that split the keys over the waves, and those that do not."""
+    T, odd = 700, [3, 40, 131, 699]
+    g = torch.Generator(device=gpu_device).manual_seed(D)
+    q, k, v, do = (torch.randn(H, T, D, generator=g, device=gpu_device).bfloat16() for _ in range(4))
+    cu = torch.tensor([T], dtype=torch.int32, device=gpu_device)
+    saturated = q.clone()
+    saturated[:, odd] *= 100
+
+    def run(q):
+        q = q.requires_grad_()
+        o, rem = sb_attn_varlen(q, k, v, cu, T, zero_start=False)
+        return o, rem, torch.autograd.grad(o, q, do)[0]
+
+    others = [i for i in range(T) if i not in odd]
+    for n, a, b in zip(("o", "rem", "dq"), run(q), run(saturated)):
+        assert torch.equal(a[:, others], b[:, others]), n
+        assert not torch.equal(a[:, odd], b[:, odd]), n

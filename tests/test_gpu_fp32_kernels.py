@@ -1,5 +1,5 @@
 """The fp32 kernels at the edges of their tiles: head_dims around the multiples of 32 (exact and padded variants), lengths
-around the 32-key sub-tiles, the 128-key steps of the four waves and the 128-row query tiles, against the float64 oracle."""
+around the 32-key sub-tiles, the 128-key steps of the four waves and the 128-row query tiles, and odds around the smallest normal number, against the float64 oracle."""
 import pytest
 import torch
 
@@ -29,3 +29,25 @@ def test_fp32_tile_edges_against_oracle(gpu_device, D, qk_std, attend_current, a
         print(f"D={D} {n}: relative error {rel.item():.2e}", flush=True)
         assert rel < 1e-5, f"{n}: {rel.item():.2e}"
         assert torch.equal(a, b), f"{n}: two runs differ"
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_odds_below_the_smallest_normal_number(gpu_device, D):
+    """Logits of -92 to -86, odds of 2^-133 to 2^-124.  A logit in octaves has an error of up to 2^-17.9 (133 octaves, two
+    roundings), which is 3e-6 of the odds at most and the same again where they are multiplied; the odds' own last place lies
+    at 2^-149, 4e-6 of the mean of 2^-128."""
+    H, T = 2, 300
+    g = torch.Generator().manual_seed(D)
+    q, k = torch.zeros(H, T, D), torch.zeros(H, T, D)
+    q[..., 0] = 1
+    k[..., 0] = -92 + 6 * torch.rand(H, T, generator=g)
+    v, do = (2.0 ** 20 * torch.randn(H, T, D, generator=g) for _ in range(2))
+    drem = torch.randn(H, T, generator=g)
+    cu = torch.tensor([T], dtype=torch.int32)
+    ref = orc.varlen_stream(*(t.double() for t in (q, k, v)), cu, do=do.double(), drem=drem.double(), dtype=torch.float64, scale=1.0)
+    dev = [t.to(gpu_device) for t in (q, k, v, do, drem)]
+    got = run_varlen(dev[0], dev[1], dev[2], cu.to(gpu_device), [T], False, False, dev[3], dev[4], scale=1.0)
+    for n, a, b in zip(NAMES, got, ref):
+        rel = (a.detach().double().cpu() - b).norm() / b.norm()
+        print(f"D={D} {n}: relative error {rel.item():.2e}", flush=True)
+        assert rel < 1e-5, f"{n}: {rel.item():.2e}"

@@ -51,8 +51,6 @@ extern "C" {
 
 /* Size of the static device scratch behind sba_fwd_static. */
 #define SBA_STATIC_SCRATCH_BYTES ((size_t)1 << 20)
-/* Largest token stride (in elements) of q, k, v and d_o with SBA_F32: the kernels address 32 rows with 32-bit byte offsets. */
-#define SBA_F32_MAX_TOKEN_STRIDE (1 << 24)
 
 typedef enum SbaDtype { SBA_BF16 = 0, SBA_F32 = 1, SBA_F16 = 2 } SbaDtype;
 
@@ -61,9 +59,8 @@ typedef enum SbaStatus {
   SBA_ERR_NULL = -1,        /* a required pointer is NULL */
   SBA_ERR_DTYPE = -2,       /* dtype not supported by this build */
   SBA_ERR_HEAD_DIM = -3,    /* head_dim outside 1..128 */
-  SBA_ERR_STRIDE = -4,      /* a negative stride, or with SBA_F32 a token stride beyond SBA_F32_MAX_TOKEN_STRIDE (any other
-                               head/token/batch stride is accepted; strides and base pointers that are multiples of 16 bytes
-                               select the fast kernels) */
+  SBA_ERR_STRIDE = -4,      /* a negative stride (any other head/token/batch stride is accepted; 16-bit strides and base
+                               pointers that are multiples of 16 bytes select the fastest kernels) */
   SBA_ERR_ALIGN = -5,       /* a tensor base pointer is not aligned to its element size */
   SBA_ERR_SHAPE = -6,       /* non-positive sizes, total_tokens > 2^30, a negative carry_slots or a flag outside {0, 1} */
   SBA_ERR_WORKSPACE = -7,   /* workspace missing, not 256-byte aligned, or too small (sba_bwd: smaller than one head needs) */

@@ -142,12 +142,18 @@ int plan(const SbaArgs* a, Layout* out) {
 
 size_t elem_size(int dtype) { return dtype == SBA_F32 ? 4 : 2; }
 
-// How the 16-bit kernels may read (and write) the rows of these tensors.  Buffer accesses need the rows of one sequence, and
+// How the kernels may read (and write) the rows of these tensors.  The fp32 ones address 32 rows at a time, which must span less
+// than 2 GiB, or else go through pointers (kLoadScalar).  16-bit: buffer accesses need the rows of one sequence, and
 // the rows of the last tiles beyond it, within 2 GiB (32-bit offsets from the sequence's first row); the aligned form also
 // base pointers and row/head/batch strides that are 16-byte multiples, and a head_dim that fills the kernel.
 template <size_t N>
 int row_load(const SbaArgs* a, const SbaTensor* const (&tensors)[N]) {
-  if (a->dtype == SBA_F32 || a->head_dim < 8) return sba::kLoadScalar;
+  if (a->dtype == SBA_F32) {
+    for (const SbaTensor* t : tensors)
+      if (t->ptr && t->stride_token > (int64_t)1 << 24) return sba::kLoadScalar;
+    return sba::kLoadPadded;
+  }
+  if (a->head_dim < 8) return sba::kLoadScalar;
   const bool fixed = a->cu_seqlens == nullptr;
   const int64_t max_rows = (a->max_seqlen > 0 && a->max_seqlen < a->total_tokens) ? a->max_seqlen : a->total_tokens;
   int load = a->head_dim == 64 || a->head_dim == 128 ? sba::kLoadAligned : sba::kLoadPadded;
@@ -195,12 +201,6 @@ int check_tensor(const SbaTensor& t, bool required, bool fixed) {
   if (!t.ptr) return required ? SBA_ERR_NULL : SBA_OK;
   if (t.stride_token < 0 || t.stride_head < 0 || (fixed && t.stride_batch < 0)) return SBA_ERR_STRIDE;
   return SBA_OK;
-}
-// The fp32 kernels address 32 rows at a time with 32-bit byte offsets.
-bool f32_stride_ok(const SbaArgs* a) {
-  for (const SbaTensor* t : {&a->q, &a->k, &a->v, &a->d_o})
-    if (t->stride_token > (int64_t)SBA_F32_MAX_TOKEN_STRIDE) return false;
-  return true;
 }
 sba::TensorRef ref(const SbaTensor& t, bool fixed) { return sba::TensorRef{t.ptr, fixed ? t.stride_batch : 0, t.stride_head, t.stride_token}; }
 sba::VectorRef vref(const SbaVector& t, bool fixed) { return sba::VectorRef{t.ptr, fixed ? t.stride_batch : 0, t.stride_head, t.stride_token}; }
@@ -349,7 +349,6 @@ int fwd_on(const SbaArgs* a, char* ws, size_t ws_bytes, bool ws_is_static, bool 
       (st = check_tensor(a->v, true, fixed)) || (st = check_tensor(a->o, true, fixed)))
     return st;
   if (!a->rem.ptr || !a->row_stat) return SBA_ERR_NULL;
-  if (a->dtype == SBA_F32 && !f32_stride_ok(a)) return SBA_ERR_STRIDE;
   for (const SbaTensor* t : {&a->q, &a->k, &a->v, &a->o})
     if (t->ptr && ((uintptr_t)t->ptr % es)) return SBA_ERR_ALIGN;
   if (ws_is_static && ws_bytes < L.fwd_bytes) return SBA_ERR_TOO_LARGE;
@@ -441,7 +440,6 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* 
       (st = check_tensor(a->dv, true, fixed)))
     return st;
   if (!a->carry && !a->recompute_carry) return SBA_ERR_NULL;
-  if (a->dtype == SBA_F32 && !f32_stride_ok(a)) return SBA_ERR_STRIDE;
   if (a->add_remainder && !a->row_stat) return SBA_ERR_NULL;
   for (const SbaTensor* t : {&a->q, &a->k, &a->v, &a->d_o, &a->dq, &a->dk, &a->dv})
     if (t->ptr && ((uintptr_t)t->ptr % es)) return SBA_ERR_ALIGN;

@@ -41,6 +41,8 @@ constexpr int kF32Split = kBlockQ / kF32Rows;      // workgroups per 128-row que
 constexpr int kF32KeySplit = kBlockK / kF32Rows;   // workgroups per 64-key tile of the schedule
 constexpr int kF32TrStride = 36;                   // floats per row of the transposition buffers
 
+enum : int { kF32Padded = 0, kF32Exact = 1, kF32Far = 2 };      // how rows are read, see Operand
+
 __device__ __forceinline__ f32x16 mfma_f32(float a, float b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
 __device__ __forceinline__ f32x16 zero16() {
   f32x16 z;
@@ -52,15 +54,20 @@ typedef __attribute__((ext_vector_type(4), aligned(4))) float f32x4_u;      // r
 
 // 32 consecutive rows of a [.., token, head_dim] tensor as the source of one operand.  A raw buffer resource per 32 rows:
 // rows at or beyond `last + 1` read as zero, and offsets stay small whatever the length of the sequence.
+// (Rows more than 2^24 elements apart, of which 32 span more than 32-bit offsets reach, are read through pointers: `p`.)
 struct Rows32 {
   __amdgpu_buffer_rsrc_t rsrc;
   uint32_t stride_bytes;
+  const float* p;
+  int64_t stride;
+  int n;
 };
 __device__ __forceinline__ Rows32 rows32(const float* base, int64_t stride, int first, int rows_total, int D) {
   Rows32 r;
   r.stride_bytes = (uint32_t)stride * 4u;
   const int n = min(rows_total - first, 32);
   const float* p = base + (int64_t)first * stride;
+  r.p = p; r.stride = stride; r.n = n;
   r.rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, n > 0 ? (int)((uint32_t)(n - 1) * r.stride_bytes + 4u * (uint32_t)D) : 0, 0x00020000);
   return r;
 }
@@ -70,7 +77,8 @@ __device__ __forceinline__ Rows32 rows32(const float* base, int64_t stride, int 
 // rows as it stands, and 64 lanes read two runs of C*4 contiguous bytes per instruction.  (A lane per row, what a
 // contraction over head_dim wants, costs a cache access per lane when loaded like that: measured 1024 instead of 290 per
 // 32 x 128 operand, and the kernels were bound by them.  Those operands go through LDS, a part at a time.)
-// kExact: head_dim == DH; otherwise an element beyond head_dim is asked for outside the buffer and reads as zero.
+// kF32Exact: head_dim == DH.  kF32Padded: an element beyond head_dim is asked for outside the buffer and reads as zero.
+// kF32Far: any head_dim, rows at any distance.
 template <int DH> struct Parts {
   static constexpr int C = DH == 128 ? 64 : 32, N = DH / C, NC = C / 32;
   static constexpr int kTurn = 32 * (C + 4);      // floats of a wave's scratch: [32 rows][C + 4]
@@ -79,22 +87,26 @@ template <int DH> __device__ __forceinline__ int out_col(int dt, int col) {
   typedef Parts<DH> P;
   return (dt / P::NC) * P::C + P::NC * col + dt % P::NC;
 }
-template <int DH, bool kExact>
+template <int DH, int kMode>
 struct Operand {
   typedef Parts<DH> P;
   Rows32 src;
   uint32_t voff;      // 16 * half rows, this lane's first column
-  int col, D;
+  int col, D, half16;
   __device__ __forceinline__ void fill_piece(float (&x)[DH / 2], int part, int r) const {
     const uint32_t soff = (uint32_t)r * src.stride_bytes;
     float* y = x + (part * 16 + r) * P::NC;
-    if (kExact && P::NC == 2) {
+    if (kMode == kF32Exact && P::NC == 2) {
       const f32x2 v = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(src.rsrc, voff + 4 * part * P::C, soff, 0));
       y[0] = v[0]; y[P::NC - 1] = v[1];
+    } else if (kMode == kF32Far) {
+      const int row = half16 + r, d = part * P::C + P::NC * col;
+#pragma unroll
+      for (int j = 0; j < P::NC; j++) y[j] = row < src.n && d + j < D ? src.p[row * src.stride + d + j] : 0.f;
     } else {
 #pragma unroll
       for (int j = 0; j < P::NC; j++) {
-        const uint32_t vo = kExact || part * P::C + P::NC * col + j < D ? voff + 4 * (part * P::C + j) : (uint32_t)kOutside;
+        const uint32_t vo = kMode == kF32Exact || part * P::C + P::NC * col + j < D ? voff + 4 * (part * P::C + j) : (uint32_t)kOutside;
         y[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(src.rsrc, vo, soff, 0));
       }
     }
@@ -108,10 +120,10 @@ struct Operand {
     for (int part = 0; part < P::N; part++) fill_part(x, part);
   }
 };
-template <int DH, bool kExact>
-__device__ __forceinline__ Operand<DH, kExact> operand(const float* base, int64_t stride, int first, int rows_total, int half, int col, int D) {
+template <int DH, int kMode>
+__device__ __forceinline__ Operand<DH, kMode> operand(const float* base, int64_t stride, int first, int rows_total, int half, int col, int D) {
   const Rows32 s = rows32(base, stride, first, rows_total, D);
-  return Operand<DH, kExact>{s, 16u * (uint32_t)half * s.stride_bytes + 4u * (uint32_t)out_col<DH>(0, col), col, D};
+  return Operand<DH, kMode>{s, 16u * (uint32_t)half * s.stride_bytes + 4u * (uint32_t)out_col<DH>(0, col), col, D, 16 * half};
 }
 
 // The phases.  Each consumes what x holds, part by part, and refills a part's registers for the phase that follows once
@@ -122,9 +134,9 @@ __device__ __forceinline__ Operand<DH, kExact> operand(const float* base, int64_
 // acc = (rows in x) . (rows in LDS, stride DH + 4), contracted over head_dim; row `xrow` of x and the LDS row `lds_row`
 // are this lane's.  kLdsIsA: the LDS rows are the A operand (output rows).  x goes through the wave's scratch; the
 // operands of four MFMAs are read one group ahead.
-template <int DH, bool kExact, bool kLdsIsA>
+template <int DH, int kMode, bool kLdsIsA>
 __device__ __forceinline__ f32x16 score_phase(float (&x)[DH / 2], float* turn, int xrow, const float* lds_row, int half, int col,
-                                              const Operand<DH, kExact>& next, const Operand<DH, kExact>& late, bool has_late) {
+                                              const Operand<DH, kMode>& next, const Operand<DH, kMode>& late, bool has_late) {
   typedef Parts<DH> P;
   constexpr int S = P::C + 4, G = P::C / 8;      // groups of four MFMAs per part
   f32x16 acc = zero16();
@@ -176,9 +188,9 @@ __device__ __forceinline__ f32x16 score_phase(float (&x)[DH / 2], float* turn, i
 }
 
 // acc[dt] += a . x, contraction over 32 rows.
-template <int DH, bool kExact>
+template <int DH, int kMode>
 __device__ __forceinline__ void contract_phase(f32x16 (&acc)[DH / 32], const float (&a)[16], float (&x)[DH / 2],
-                                               const Operand<DH, kExact>& next, bool refill, const Operand<DH, kExact>& late,
+                                               const Operand<DH, kMode>& next, bool refill, const Operand<DH, kMode>& late,
                                                bool has_late) {
   typedef Parts<DH> P;
 #pragma unroll
@@ -200,14 +212,19 @@ __device__ __forceinline__ void contract_phase(f32x16 (&acc)[DH / 32], const flo
 }
 
 // 32 rows into LDS, [row][DH + 4] floats, zeros beyond the last row and beyond head_dim; all threads take part.
-template <int DH, bool kExact>
+template <int DH, int kMode>
 __device__ __forceinline__ void stage_rows(float* lds, const Rows32& s, int D) {
-  if (kExact) {
+  if (kMode == kF32Exact) {
 #pragma unroll
     for (int i = 0; i < 32 * (DH / 4) / kThreads; i++) {
       const int idx = threadIdx.x + kThreads * i, row = idx / (DH / 4), d = (idx % (DH / 4)) * 4;
       const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(s.rsrc, (uint32_t)row * s.stride_bytes + 4 * d, 0, 0);
       *reinterpret_cast<u32x4*>(lds + row * (DH + 4) + d) = v;
+    }
+  } else if (kMode == kF32Far) {
+    for (int idx = threadIdx.x; idx < 32 * DH; idx += kThreads) {
+      const int row = idx / DH, d = idx % DH;
+      lds[row * (DH + 4) + d] = row < s.n && d < D ? s.p[row * s.stride + d] : 0.f;
     }
   } else {
     for (int idx = threadIdx.x; idx < 32 * DH; idx += kThreads) {
@@ -258,7 +275,7 @@ __device__ __forceinline__ float sticks_f32(const f32x16& s, float scale_log2, i
 
 // Sum the four waves' partial [32 rows][DH] results through LDS and store them (times `scale`, plus add_scale[row] *
 // add[row] when `add` is given).  acc[dt][r]: row 8*(r/4) + 4*half + r%4, column out_col(dt).  All waves take part.
-template <int DH, bool kExact>
+template <int DH, int kMode>
 __device__ __forceinline__ void reduce_store_f32(float* lds, const f32x16 (&acc)[DH / 32], float scale, float* out, int64_t stride,
                                                  int rows, int D, const float* add = nullptr, int64_t add_stride = 0,
                                                  const float* add_scale = nullptr) {
@@ -282,7 +299,7 @@ __device__ __forceinline__ void reduce_store_f32(float* lds, const f32x16 (&acc)
     float* o = out + (int64_t)row * stride + d0;
     const float* a = add ? add + (int64_t)row * add_stride + d0 : nullptr;
     const float as = add ? add_scale[row] : 0.f;
-    if (kExact) {
+    if (kMode == kF32Exact) {
       if (a) { const f32x4_u w = *reinterpret_cast<const f32x4_u*>(a); v += as * (f32x4){w[0], w[1], w[2], w[3]}; }
       *reinterpret_cast<f32x4_u*>(o) = f32x4_u{v[0], v[1], v[2], v[3]};
     } else {
@@ -300,7 +317,7 @@ struct RowsF32Lds {
   static constexpr int kFloats = kLoop > kRed ? kLoop : kRed;
 };
 
-template <int DH, bool kExact>
+template <int DH, int kMode>
 __global__ __launch_bounds__(kThreads, 2) void fwd_f32_kernel(FwdParams p) {
   constexpr int NB = DH / 32;
   __shared__ __attribute__((aligned(16))) float lds[RowsF32Lds<DH, 1>::kFloats];      // Q rows and the waves' scratch, then the final sums
@@ -340,13 +357,13 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_f32_kernel(FwdParams p) {
   const int last_key = min(q0 + kF32Rows, L) - 2 + ac;
   const int n_sub = last_key < 0 ? 0 : last_key / 32 + 1, n_steps = (n_sub + kWaves - 1) / kWaves;
   const int krow = mfma_row_to_key32(col);
-  auto k_of = [&](int u) { return operand<DH, kExact>(kb, p.k.st, 32 * u, L, half, col, D); };
-  auto v_of = [&](int u) { return operand<DH, kExact>(vb, p.v.st, 32 * u, L, half, col, D); };
+  auto k_of = [&](int u) { return operand<DH, kMode>(kb, p.k.st, 32 * u, L, half, col, D); };
+  auto v_of = [&](int u) { return operand<DH, kMode>(vb, p.v.st, 32 * u, L, half, col, D); };
   float x[DH / 2];
   // Wave w takes sub-tile n_sub - 1 - (4 t + w) in step t.
   int U = n_sub - 1 - wave;
   if (U >= 0) k_of(U).fill(x);
-  stage_rows<DH, kExact>(lds, rows32(qb, p.q.st, q0, L, D), D);
+  stage_rows<DH, kMode>(lds, rows32(qb, p.q.st, q0, L, D), D);
   const float* q_lds = lds + col * (DH + 4);
   float* turn = lds + 32 * (DH + 4) + wave * Parts<DH>::kTurn;
   f32x16 oacc[NB];
@@ -358,7 +375,7 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_f32_kernel(FwdParams p) {
     float beta[16], pe[16];
     float run = 1.f, oth = 1.f;
     if (U >= 0) {
-      const f32x16 s = score_phase<DH, kExact, false>(x, turn, krow, q_lds, half, col, v_of(U), k_of(U), t > 0);
+      const f32x16 s = score_phase<DH, kMode, false>(x, turn, krow, q_lds, half, col, v_of(U), k_of(U), t > 0);
       run = sticks_f32(s, p.scale_log2, qi + ac - 32 * U - 16 * half, beta, pe);
       oth = other_half(run, half);
     }
@@ -376,7 +393,7 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_f32_kernel(FwdParams p) {
       const float seed = half ? above : above * oth;        // the upper half-wave holds the higher keys
 #pragma unroll
       for (int r = 0; r < 16; r++) pe[r] = beta[r] * (pe[r] * seed);
-      contract_phase<DH, kExact>(oacc, pe, x, k_of(U - kWaves), U >= kWaves, k_of(U), false);
+      contract_phase<DH, kMode>(oacc, pe, x, k_of(U - kWaves), U >= kWaves, k_of(U), false);
     }
   }
   if (wave == 0 && half == 0) {
@@ -387,10 +404,10 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_f32_kernel(FwdParams p) {
     }
   }
   float* ob = (float*)p.o.ptr + tile.seq_id * p.o.sb + head * p.o.sh + (tok0 + q0) * p.o.st;
-  reduce_store_f32<DH, kExact>(lds, oacc, 1.f, ob, p.o.st, L - q0, D, p.add_rem ? vb + (int64_t)q0 * p.v.st : nullptr, p.v.st, rem_lds);
+  reduce_store_f32<DH, kMode>(lds, oacc, 1.f, ob, p.o.st, L - q0, D, p.add_rem ? vb + (int64_t)q0 * p.v.st : nullptr, p.v.st, rem_lds);
 }
 
-template <int DH, bool kExact>
+template <int DH, int kMode>
 __global__ __launch_bounds__(kThreads, 2) void bwd_dq_f32_kernel(BwdParams p) {
   constexpr int NB = DH / 32;
   __shared__ __attribute__((aligned(16))) float lds[RowsF32Lds<DH, 2>::kFloats];      // Q and dO rows and the waves' scratch, then the final sums
@@ -426,13 +443,13 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dq_f32_kernel(BwdParams p) {
   const int last_key = min(q0 + kF32Rows, L) - 2 + ac;
   const int n_sub = last_key < 0 ? 0 : last_key / 32 + 1, n_steps = (n_sub + kWaves - 1) / kWaves;
   const int krow = mfma_row_to_key32(col);
-  auto k_of = [&](int u) { return operand<DH, kExact>(kb, p.k.st, 32 * u, L, half, col, D); };
-  auto v_of = [&](int u) { return operand<DH, kExact>(vb, p.v.st, 32 * u, L, half, col, D); };
+  auto k_of = [&](int u) { return operand<DH, kMode>(kb, p.k.st, 32 * u, L, half, col, D); };
+  auto v_of = [&](int u) { return operand<DH, kMode>(vb, p.v.st, 32 * u, L, half, col, D); };
   float x[DH / 2];
   int U = wave;            // wave w takes sub-tile 4 t + w in step t
   if (U < n_sub) k_of(U).fill(x);
-  stage_rows<DH, kExact>(lds, rows32(qb, p.q.st, q0, L, D), D);
-  stage_rows<DH, kExact>(lds + 32 * (DH + 4), rows32(dob, p.d_o.st, q0, L, D), D);
+  stage_rows<DH, kMode>(lds, rows32(qb, p.q.st, q0, L, D), D);
+  stage_rows<DH, kMode>(lds + 32 * (DH + 4), rows32(dob, p.d_o.st, q0, L, D), D);
   const float* q_lds = lds + col * (DH + 4);
   const float* do_lds = q_lds + 32 * (DH + 4);
   float* turn = lds + 64 * (DH + 4) + wave * Parts<DH>::kTurn;
@@ -459,8 +476,8 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dq_f32_kernel(BwdParams p) {
     const bool active = U < n_sub;
     if (active) {
       const float prod_in = carry[cslot];
-      const f32x16 s = score_phase<DH, kExact, false>(x, turn, krow, q_lds, half, col, v_of(U), k_of(U), t > 0);
-      const f32x16 dp = score_phase<DH, kExact, false>(x, turn, krow, do_lds, half, col, k_of(U), k_of(U), false);
+      const f32x16 s = score_phase<DH, kMode, false>(x, turn, krow, q_lds, half, col, v_of(U), k_of(U), t > 0);
+      const f32x16 dp = score_phase<DH, kMode, false>(x, turn, krow, do_lds, half, col, k_of(U), k_of(U), false);
       float pe[16];
       const float run = sticks_f32(s, p.scale_log2, qi < L ? qi + ac - 32 * U - 16 * half : 0, beta, pe);
       const float oth = other_half(run, half);
@@ -490,11 +507,11 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dq_f32_kernel(BwdParams p) {
       const float fixup = below + fix;
 #pragma unroll
       for (int r = 0; r < 16; r++) dz[r] -= beta[r] * fixup;
-      contract_phase<DH, kExact>(dqacc, dz, x, k_of(U + kWaves), U + kWaves < n_sub, k_of(U), false);
+      contract_phase<DH, kMode>(dqacc, dz, x, k_of(U + kWaves), U + kWaves < n_sub, k_of(U), false);
     }
   }
   float* dqb = (float*)p.dq.ptr + tile.seq_id * p.dq.sb + head * p.dq.sh + (tok0 + q0) * p.dq.st;
-  reduce_store_f32<DH, kExact>(lds, dqacc, p.logit_scale, dqb, p.dq.st, L - q0, D);
+  reduce_store_f32<DH, kMode>(lds, dqacc, p.logit_scale, dqb, p.dq.st, L - q0, D);
 }
 
 template <int DH>
@@ -508,7 +525,7 @@ struct DkvF32Lds {
   static constexpr int kFloats = (kLoop > kRed ? kLoop : kRed) + 32;                  // + rem of 32 rows
 };
 
-template <int DH, bool kExact>
+template <int DH, int kMode>
 __global__ __launch_bounds__(kThreads, 2) void bwd_dkv_f32_kernel(BwdParams p) {
   constexpr int NB = DH / 32;
   typedef DkvF32Lds<DH> Lds;
@@ -533,8 +550,8 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dkv_f32_kernel(BwdParams p) {
   const float* prefix = p.prefix + slot0;
   const float* drem_plane = p.drem_eff + tile.seq_id * p.drem_sb + head * p.stat_sh + tok0;
 
-  auto q_of = [&](int b) { return operand<DH, kExact>(qb, p.q.st, 32 * b, L, half, col, D); };
-  auto do_of = [&](int b) { return operand<DH, kExact>(dob, p.d_o.st, 32 * b, L, half, col, D); };
+  auto q_of = [&](int b) { return operand<DH, kMode>(qb, p.q.st, 32 * b, L, half, col, D); };
+  auto do_of = [&](int b) { return operand<DH, kMode>(dob, p.d_o.st, 32 * b, L, half, col, D); };
   // Row blocks of 32 that see these keys: from the last one down to the one that holds the keys' own rows; wave w takes every
   // fourth.  (Downwards the loop needs one bound fewer in registers: 20 instead of 64 of them spilled at head_dim 128, 2 % of
   // the pass.)
@@ -543,8 +560,8 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dkv_f32_kernel(BwdParams p) {
   float x[DH / 2];
   if (b >= U) q_of(b).fill(x);
   // K and V of the 32 keys stay in LDS for the A operands of S^T and dP^T.
-  stage_rows<DH, kExact>(lds + Lds::kK, rows32(kb, p.k.st, k0, L, D), D);
-  stage_rows<DH, kExact>(lds + Lds::kV, rows32(vb, p.v.st, k0, L, D), D);
+  stage_rows<DH, kMode>(lds + Lds::kK, rows32(kb, p.k.st, k0, L, D), D);
+  stage_rows<DH, kMode>(lds + Lds::kV, rows32(vb, p.v.st, k0, L, D), D);
   const int krow = mfma_row_to_key32(col);
   const float* k_lds = lds + Lds::kK + krow * Lds::kRowStride;
   const float* v_lds = lds + Lds::kV + krow * Lds::kRowStride;
@@ -561,8 +578,8 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dkv_f32_kernel(BwdParams p) {
     const bool row_ok = qi < L;
     const float prod_in = carry[qi], prefix_in = prefix[qi];
     const float drem = row_ok ? drem_plane[qi] : 0.f;
-    const f32x16 s = score_phase<DH, kExact, true>(x, turn, col, k_lds, half, col, do_of(b), q_of(b), b < nb - kWaves);
-    const f32x16 dp = score_phase<DH, kExact, true>(x, turn, col, v_lds, half, col, do_of(b), do_of(b), false);
+    const f32x16 s = score_phase<DH, kMode, true>(x, turn, col, k_lds, half, col, do_of(b), q_of(b), b < nb - kWaves);
+    const f32x16 dp = score_phase<DH, kMode, true>(x, turn, col, v_lds, half, col, do_of(b), do_of(b), false);
     {
       float beta[16], pe[16];
       const float run = sticks_f32(s, p.scale_log2, row_ok ? qi + ac - k0 - 16 * half : 0, beta, pe);
@@ -593,35 +610,41 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dkv_f32_kernel(BwdParams p) {
     };
     float y[16];
     transposed(tp, y);
-    contract_phase<DH, kExact>(dvacc, y, x, q_of(b), true, q_of(b), false);
+    contract_phase<DH, kMode>(dvacc, y, x, q_of(b), true, q_of(b), false);
     transposed(tz, y);
-    contract_phase<DH, kExact>(dkacc, y, x, q_of(b - kWaves), b - kWaves >= U, q_of(b), true);
+    contract_phase<DH, kMode>(dkacc, y, x, q_of(b - kWaves), b - kWaves >= U, q_of(b), true);
   }
   float* rem_lds = lds + Lds::kFloats - 32;
   if (p.add_rem && threadIdx.x < 32 && k0 + (int)threadIdx.x < L)      // the forward wrote o + rem * v: dv_i gains rem_i * d_o_i
     rem_lds[threadIdx.x] = exp2f(p.row_stat[tile.seq_id * p.stat_sb + head * p.stat_sh + tok0 + k0 + threadIdx.x]);
   float* dvb = (float*)p.dv.ptr + tile.seq_id * p.dv.sb + head * p.dv.sh + (tok0 + k0) * p.dv.st;
   float* dkb = (float*)p.dk.ptr + tile.seq_id * p.dk.sb + head * p.dk.sh + (tok0 + k0) * p.dk.st;
-  reduce_store_f32<DH, kExact>(lds, dvacc, 1.f, dvb, p.dv.st, L - k0, D, p.add_rem ? dob + (int64_t)k0 * p.d_o.st : nullptr,
+  reduce_store_f32<DH, kMode>(lds, dvacc, 1.f, dvb, p.dv.st, L - k0, D, p.add_rem ? dob + (int64_t)k0 * p.d_o.st : nullptr,
                                p.d_o.st, rem_lds);
-  reduce_store_f32<DH, kExact>(lds, dkacc, p.logit_scale, dkb, p.dk.st, L - k0, D);
+  reduce_store_f32<DH, kMode>(lds, dkacc, p.logit_scale, dkb, p.dk.st, L - k0, D);
 }
 
 // head_dim is rounded up to a multiple of 32 (the matrix cycles go by that); the exact variants skip every test of a
 // column against head_dim and load 16 bytes where the others load 4.
+template <int DH, typename F>
+static hipError_t by_mode(int D, int load, F&& f) {
+  std::integral_constant<int, DH> dh;
+  if (load == kLoadScalar) return f(dh, std::integral_constant<int, kF32Far>());
+  return D == DH ? f(dh, std::integral_constant<int, kF32Exact>()) : f(dh, std::integral_constant<int, kF32Padded>());
+}
 template <typename F>
-static hipError_t by_head_dim(int D, F&& f) {
+static hipError_t by_head_dim(int D, int load, F&& f) {
   switch ((D + 31) / 32) {
-    case 1: return D == 32 ? f(std::integral_constant<int, 32>(), std::true_type()) : f(std::integral_constant<int, 32>(), std::false_type());
-    case 2: return D == 64 ? f(std::integral_constant<int, 64>(), std::true_type()) : f(std::integral_constant<int, 64>(), std::false_type());
-    case 3: return D == 96 ? f(std::integral_constant<int, 96>(), std::true_type()) : f(std::integral_constant<int, 96>(), std::false_type());
-    default: return D == 128 ? f(std::integral_constant<int, 128>(), std::true_type()) : f(std::integral_constant<int, 128>(), std::false_type());
+    case 1: return by_mode<32>(D, load, f);
+    case 2: return by_mode<64>(D, load, f);
+    case 3: return by_mode<96>(D, load, f);
+    default: return by_mode<128>(D, load, f);
   }
 }
 
 hipError_t launch_fwd_f32(const FwdParams& p, int max_tiles, hipStream_t stream) {
-  return by_head_dim(p.head_dim, [&](auto dh, auto exact) {
-    hipLaunchKernelGGL((fwd_f32_kernel<decltype(dh)::value, decltype(exact)::value>), dim3((unsigned)(max_tiles * p.num_heads * kF32Split + p.sched.service)),
+  return by_head_dim(p.head_dim, p.load, [&](auto dh, auto mode) {
+    hipLaunchKernelGGL((fwd_f32_kernel<decltype(dh)::value, decltype(mode)::value>), dim3((unsigned)(max_tiles * p.num_heads * kF32Split + p.sched.service)),
                        dim3(kThreads), 0, stream, p);
     return hipGetLastError();
   });
@@ -631,15 +654,15 @@ hipError_t launch_bwd_f32(const BwdParams& p, int max_q_tiles, int max_k_tiles, 
   int dev = 0, cus = 0;
   const hipError_t e = device_cus(&dev, &cus);
   if (e != hipSuccess) return e;
-  return by_head_dim(p.head_dim, [&](auto dh, auto exact) {
+  return by_head_dim(p.head_dim, p.load, [&](auto dh, auto mode) {
     constexpr int DH = decltype(dh)::value;
-    constexpr bool kExact = decltype(exact)::value;
+    constexpr int kMode = decltype(mode)::value;
     constexpr size_t lds_bytes = DkvF32Lds<DH>::kFloats * sizeof(float);
     static std::atomic<uint64_t> lds_done{0};
-    const hipError_t r = raise_lds_limit(&bwd_dkv_f32_kernel<DH, kExact>, lds_done, dev, lds_bytes);
+    const hipError_t r = raise_lds_limit(&bwd_dkv_f32_kernel<DH, kMode>, lds_done, dev, lds_bytes);
     if (r != hipSuccess) return r;
-    hipLaunchKernelGGL((bwd_dq_f32_kernel<DH, kExact>), dim3((unsigned)(max_q_tiles * p.num_heads * kF32Split)), dim3(kThreads), 0, stream, p);
-    hipLaunchKernelGGL((bwd_dkv_f32_kernel<DH, kExact>), dim3((unsigned)(max_k_tiles * p.num_heads * kF32KeySplit)), dim3(kThreads), lds_bytes, stream, p);
+    hipLaunchKernelGGL((bwd_dq_f32_kernel<DH, kMode>), dim3((unsigned)(max_q_tiles * p.num_heads * kF32Split)), dim3(kThreads), 0, stream, p);
+    hipLaunchKernelGGL((bwd_dkv_f32_kernel<DH, kMode>), dim3((unsigned)(max_k_tiles * p.num_heads * kF32KeySplit)), dim3(kThreads), lds_bytes, stream, p);
     return hipGetLastError();
   });
 }

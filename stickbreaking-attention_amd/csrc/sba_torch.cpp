@@ -54,11 +54,8 @@ void require_gpu(const Tensor& t) {
   TORCH_CHECK(t.is_cuda(), "stick-breaking attention runs on the GPU only (got a CPU tensor); there is no CPU path");
 }
 
-// The kernels need unit stride along head_dim; the fp32 ones also a token stride their 32-bit offsets reach.
-Tensor rows_contiguous(const Tensor& t) {
-  const bool far = t.scalar_type() == at::kFloat && t.stride(-2) > SBA_F32_MAX_TOKEN_STRIDE;
-  return t.stride(-1) == 1 && !far ? t : t.contiguous();
-}
+// The kernels need unit stride along head_dim.
+Tensor rows_contiguous(const Tensor& t) { return t.stride(-1) == 1 ? t : t.contiguous(); }
 
 void same_dtype(const Tensor& q, const Tensor& t, const char* name) {
   TORCH_CHECK_TYPE(t.scalar_type() == q.scalar_type(), name, " has dtype ", t.dtype(), ", q has ", q.dtype(),

@@ -165,11 +165,8 @@ def _vector(t: Optional[torch.Tensor], fixed: bool) -> SbaVector:
 
 
 def rows_contiguous(t: torch.Tensor) -> torch.Tensor:
-    """The kernels need unit stride along head_dim (as the reference does, sb_varlen_fwd.py:235); the fp32 ones also a
-    token stride their 32-bit offsets reach (SBA_F32_MAX_TOKEN_STRIDE of include/sba.h)."""
-    if t.stride(-1) != 1 or (t.stride(-2) > 1 << 24 and t.dtype == torch.float32):
-        return t.contiguous()
-    return t
+    """The kernels need unit stride along head_dim (as the reference does, sb_varlen_fwd.py:235)."""
+    return t if t.stride(-1) == 1 else t.contiguous()
 
 
 def _require_gpu(*tensors):

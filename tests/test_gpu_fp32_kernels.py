@@ -1,9 +1,11 @@
 """The fp32 kernels at the edges of their tiles: head_dims around the multiples of 32 (exact and padded variants), lengths
-around the 32-key sub-tiles, the 128-key steps of the four waves and the 128-row query tiles, and odds around the smallest normal number, against the float64 oracle."""
+around the 32-key sub-tiles, the 128-key steps of the four waves and the 128-row query tiles, and odds around the smallest normal number, against the float64
+oracle; and rows further apart than 32-bit offsets reach."""
 import pytest
 import torch
 
 from oracle import sb_oracle as orc
+from stickbreaking_attention import sb_attn_varlen
 from test_gpu_parity import NAMES, run_varlen, small_case
 
 pytestmark = pytest.mark.gpu
@@ -51,3 +53,27 @@ def test_odds_below_the_smallest_normal_number(gpu_device, D):
         rel = (a.detach().double().cpu() - b).norm() / b.norm()
         print(f"D={D} {n}: relative error {rel.item():.2e}", flush=True)
         assert rel < 1e-5, f"{n}: {rel.item():.2e}"
+
+
+@pytest.mark.parametrize("D", [128, 50, 9])
+@pytest.mark.parametrize("far", ["all", "do"])
+def test_rows_further_apart_than_32_bit_offsets_reach(gpu_device, far, D):
+    H, T, stride = 2, 40, (1 << 24) + 8
+    buf = torch.empty(T * stride, device=gpu_device)
+    near = [torch.randn(H, T, D, device=gpu_device) for _ in range(4)]
+    drem = torch.randn(H, T, device=gpu_device)
+    cu = torch.tensor([7, T], dtype=torch.int32)
+    views = [buf.as_strided((H, T, D), (D, stride, 1), 2 * i * D) for i in range(4)]
+    for view, t in zip(views, near):
+        view.copy_(t)
+    if far == "do":
+        views[:3] = near[:3]
+
+    def run(q, k, v, do):      # (without the copies run_varlen makes)
+        for t in (q, k, v):
+            t.requires_grad_()
+        o, rem = sb_attn_varlen(q, k, v, cu, T - 7, zero_start=False, attend_current=True, add_remainder=True)
+        return o, rem, *torch.autograd.grad([o, rem], [q, k, v], [do, drem])
+
+    for n, a, b in zip(NAMES, run(*views), run(*near)):
+        assert (a - b).norm() < 1e-6 * b.norm(), n

@@ -316,7 +316,8 @@ std::optional<std::tuple<Tensor, Tensor>> varlen(py::handle hq, py::handle hk, p
   c.flags = flags;
   if (cu.scalar_type() != at::kInt && cu.scalar_type() != at::kLong) cu = cu.to(at::kLong);
   // The lengths are on the host when cu_seqlens was given there, or after the one device-to-host copy that stands in for
-  // the reference's `assert cu_seqlens[0] == 0`: they are then validated here and the carry buffer is sized exactly.
+  // the reference's `assert cu_seqlens[0] == 0`: they are then validated here, the carry buffer is sized exactly, and the
+  // longest of them is what the kernels are chosen by, whatever the caller's max_seqlens says.
   Tensor host;
   if (!cu.is_cuda()) host = cu.contiguous();
   else if (zero_start) host = cu.cpu().contiguous();
@@ -339,6 +340,7 @@ std::optional<std::tuple<Tensor, Tensor>> varlen(py::handle hq, py::handle hk, p
     check(sba_plan_host(&a, host.const_data_ptr(), &plan), "sba_plan_host");
     TORCH_CHECK_VALUE(plan.status == 0, "cu_seqlens must be non-decreasing sequence ends within [0, total_tokens]");
     c.carry_slots = plan.carry_slots;
+    c.max_seqlen = std::max(plan.longest, 1);
   }
   if (cu.device() != q.device()) cu = cu.to(q.device());
   c.cu = cu.contiguous();

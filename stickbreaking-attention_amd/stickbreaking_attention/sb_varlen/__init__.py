@@ -3,8 +3,8 @@
 Same call surface as the reference's stickbreaking_attention/sb_varlen/__init__.py:23-81:
 ``sb_attn_varlen(q, k, v, cu_seqlens, max_seqlens, inv_temp=None, zero_start=True, attend_current=False)``
 returns ``(o, rem)`` for ``q, k, v`` of shape (num_heads, total_tokens, head_dim).  ``max_seqlens`` may be
-omitted (the reference's README calls the function without it); it only bounds scratch memory here, the
-tile schedule is derived from ``cu_seqlens`` on the device.
+omitted (the reference's README calls the function without it): it bounds scratch memory and takes part in the choice of
+the kernels where the lengths are not on the host; the tile schedule is derived from ``cu_seqlens`` on the device.
 """
 import math
 
@@ -65,8 +65,9 @@ def sb_attn_varlen(q, k, v, cu_seqlens, max_seqlens=None, inv_temp=None, zero_st
             return out
     # The lengths are on the host when cu_seqlens was given as a CPU tensor, or after the one device-to-host copy that
     # stands in for the reference's `assert cu_seqlens[0] == 0` (sb_varlen/__init__.py:71-73, the same host sync).
-    # They are then validated there and the carry buffer is sized exactly; a device-only cu_seqlens is validated by
-    # the scheduler kernel and the buffer is sized from the bound total_tokens * max_seqlens / 64.
+    # They are then validated there, the carry buffer is sized exactly, and the longest of them is what the kernels are
+    # chosen by; a device-only cu_seqlens is validated by the scheduler kernel and the buffer is sized from the bound
+    # total_tokens * max_seqlens / 64.
     cu_host = cu_seqlens if cu_seqlens.device.type == "cpu" else None
     if zero_start:
         if cu_host is None and not torch.compiler.is_compiling():
@@ -78,7 +79,7 @@ def sb_attn_varlen(q, k, v, cu_seqlens, max_seqlens=None, inv_temp=None, zero_st
         plan = _native.plan_host(cu_host, bool(zero_start), q.size(1))
         if plan.status != 0:
             raise ValueError("cu_seqlens must be non-decreasing sequence ends within [0, total_tokens]")
-        carry_slots = int(plan.carry_slots)
+        carry_slots, max_seqlens = int(plan.carry_slots), max(int(plan.longest), 1)
     cu_seqlens = _native.prepare_cu_seqlens(cu_seqlens, q.device)
     if inv_temp is None:
         inv_temp = 1 / math.sqrt(q.size(-1))

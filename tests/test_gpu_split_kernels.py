@@ -1,9 +1,10 @@
 """The kernels of problems too small to fill the chip (keys split over the waves): lengths around their 32-row blocks and
 128-key steps, rows no sequence covers, both directions, against the float64 oracle; and both kinds of kernel on the two sides
-of the size from which on the wide ones run."""
+of the size from which on the wide ones run; and which of them runs when the lengths are known but max_seqlens is not given."""
 import numpy as np
 import pytest
 import torch
+from torch.utils._python_dispatch import TorchDispatchMode
 
 from oracle import sb_oracle as orc
 from stickbreaking_attention import sb_attn_varlen
@@ -37,3 +38,33 @@ def test_lengths_around_the_steps(gpu_device, H, D, attend_current, add_remainde
     for n, a, b in zip(NAMES, got, ref):
         tol_check(n, a[heads, :T], b, dtype, f"H={H} D={D}")
         assert (a[:, T:] == 0).all(), f"{n}: rows no sequence covers must be zero"
+
+
+class Passing(TorchDispatchMode):
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("where", ["host", "device with a leading zero", "host, Python operators"])
+def test_known_lengths_choose_the_kernels_without_max_seqlens(gpu_device, where):
+    """24 heads of 8 x 300 tokens: too many rows to split the keys of sequences this short, few enough if they were one.  The bits
+    tell the kernels apart."""
+    H, D, lengths = 24, 64, [300] * 8
+    q, k, v, do = (torch.randn(H, sum(lengths), D, device=gpu_device).bfloat16() for _ in range(4))
+    for t in (q, k, v):
+        t.requires_grad_()
+    zero = "zero" in where
+    cu = torch.tensor(np.cumsum([0] * zero + lengths), dtype=torch.int32, device=gpu_device if zero else "cpu")
+
+    def run(max_seqlens):
+        o, rem = sb_attn_varlen(q, k, v, cu, max_seqlens, zero_start=zero)
+        return o, rem, *torch.autograd.grad(o, [q, k, v], do)
+
+    want = run(300)
+    for hint in (None, 2000):
+        if "operators" in where:
+            with Passing():
+                got = run(hint)
+        else:
+            got = run(hint)
+        assert all(torch.equal(a, b) for a, b in zip(got, want)), hint

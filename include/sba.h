@@ -90,7 +90,9 @@ typedef struct SbaArgs {
   int32_t num_heads;           /* H */
   int32_t num_seqs;            /* number of sequences (varlen) or batch size B (fixed) */
   int64_t total_tokens;        /* T (varlen) or L (fixed) */
-  int64_t max_seqlen;          /* upper bound on the longest sequence; <= 0 means "unknown" (T is assumed) */
+  int64_t max_seqlen;          /* upper bound on the longest sequence; <= 0 means "unknown" (T is assumed).  Sizes scratch and takes
+                                  part in the choice of the kernels, which an overstated bound may make the slower ones: a
+                                  caller with the lengths on the host passes SbaPlan.longest.  The same in both passes. */
   float logit_scale;           /* z = logit_scale * q.k  (the operator's inv_temp) */
   int32_t attend_current;      /* 0: keys j < i are visible; 1: keys j <= i */
 

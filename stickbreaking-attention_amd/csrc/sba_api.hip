@@ -177,19 +177,31 @@ int row_load(const SbaArgs* a, const SbaTensor* const (&tensors)[N]) {
 //                 dQ    28.8 / 61    29.9 / 62    43 / 63    78 / 69
 //   head_dim 128  fwd   34.7 / 61    39 / 62      60 / 64   112 / 73     (8192: 128 / 230, 131 / 236, 189 / 238, 325 / 262)
 //                 dQ    39 / 79      47 / 80      91 / 84   185 / 94
-// That is for one sequence, whose tiles run longest first.  Several follow one another, the last one's longest rows start late, and
-// the lines lie lower; training passes: head_dim 128, 21 K (6 x 1740) 205 / 210, 28 K (7 x 1024, 8 x 1740, 14 x 512)
-// 166 / 149, 249 / 226, 128 / 111; head_dim 64, 33 K to 41 K (16 x 2048, 10 x 1740, 9 x 1024, 10 x 4096) 201 / 195, 168 / 177, 129 / 136,
-// 356 / 397, 51 K (12 x 512, 13 x 1024, 15 x 1740, 26 x 2048) 114 / 110, 164 / 154, 222 / 206, 284 / 253.
-// (Several: none holds more than a sixth of the rows.  7 heads x 50, 8191 tokens, a log-normal mix: 185 / 207.)
+// An unsplit workgroup's longest row costs what it does however many rows there are, so the line rises with the longest sequence; the
+// tiles of long sequences run first, so short ones beside them fill the gaps, and rows count for less the shorter the mean is.
+// Training passes, split / unsplit us, by rows x heads:
+//   head_dim 128   2 x  768   15 K  78 /  85   18 K  86 /  92   22 K 103 /  96      (line at 19 K)
+//                  4 x 1024   16 K  96 / 105   20 K 122 / 119   24 K 132 / 125      (21 K)
+//                  1 x 1740   19 K 149 / 171   24 K 161 / 178   31 K 190 / 185      (27 K)
+//                  2 x 2900   17 K 212 / 263   28 K 297 / 306   34 K 324 / 318      (30 K)
+//    7 of 222 to 1568 (mean 699)   33 K 169 / 171   5 of 568 down (mean 417)   18 K  84 /  77      (29 K; 19 K)
+//   head_dim 64    4 x  768   27 K  76 /  78   36 K  82 /  81   45 K  99 /  95      (32 K)
+//                  8 x 1024   32 K 101 /  98   40 K 118 / 112   48 K 129 / 117      (36 K)
+//                  1 x 2900   34 K 160 / 218   42 K 206 / 236   51 K 224 / 248      (60 K)
+//                 12 x 2900   34 K 223 / 245   68 K 344 / 325                       (60 K)
+//   28 of 1660 down (mean 473)     65 K 160 / 155  51 of 1324 down (mean 320)  48 K 125 / 125      (56 K; 50 K)
+// Over 877 batches of 1 to 146 sequences of up to 8000 tokens (equal, uniform, log-normal, one long among short ones) and
+// head_dims 50 to 128, the rule loses 0.3 % against the faster kind of each batch, 14 % at most.
 // `heads` is the head count of the caller's call, also where the backward takes them through in groups: the groups then run the
 // kernels, and give the bits, of one pass, and products are rebuilt by the kernel whose forward would have kept them.
 bool few_tiles(const SbaArgs* a, int64_t heads, int load) {
   if (a->dtype == SBA_F32 || load == sba::kLoadScalar) return false;
   const int64_t seq_rows = a->total_tokens * (a->cu_seqlens ? 1 : a->num_seqs), rows = seq_rows * heads;
   const int64_t longest = a->max_seqlen > 0 && a->max_seqlen < a->total_tokens ? a->max_seqlen : a->total_tokens;
-  const bool several = 6 * longest <= seq_rows;
-  return rows < (a->head_dim > 64 ? (several ? 20 << 10 : 30 << 10) : several ? 40 << 10 : 60 << 10);
+  const int64_t mean = a->cu_seqlens ? a->total_tokens / a->num_seqs : a->total_tokens;
+  const int64_t cap = a->head_dim > 64 ? 30 << 10 : 60 << 10, line = a->head_dim > 64 ? (13 << 10) + 8 * longest : (20 << 10) + 16 * longest;
+  if (rows >= 2 * cap) return false;
+  return rows * (mean + 3 * longest) < 4 * longest * (line < cap ? line : cap);
 }
 // The same for dK/dV: below, head_dim up to 64 splits the rows over the waves (130 K rows x heads: 542 / 565 us at 8192
 // tokens), wider ones take key tiles of 64 instead of 128 (64 K: 113 / 119 at 2048, 354 / 410 at 8192; 130 K: 672 / 657).

@@ -622,11 +622,11 @@ int sba_bwd(const SbaArgs* a) {
 
 namespace sba {
 
-int prepared_bytes(const SbaArgs* a, size_t* sched_bytes, size_t* rest_bytes, size_t* carry_bytes) {
+int prepared_bytes(const SbaArgs* a, Prepared* out) {
   Layout L;
   const int st = plan(a, &L);
   if (st != SBA_OK) return st;
-  *sched_bytes = L.sched_bytes; *rest_bytes = L.rest_bytes; *carry_bytes = L.carry_bytes;
+  *out = Prepared{L.sched_bytes, L.rest_bytes, L.carry_bytes, L.chain_zero_bytes > 0};
   return SBA_OK;
 }
 

@@ -5,9 +5,14 @@
 
 namespace sba {
 
-// Sizes: of the schedule, of the backward's workspace besides it, and of `carry`.
-int prepared_bytes(const SbaArgs* a, size_t* sched_bytes, size_t* rest_bytes, size_t* carry_bytes);
-// sba_fwd with the schedule in a->workspace (sched_bytes of it).
+// Sizes: of the schedule, of the backward's workspace besides it, and of `carry`; whether the schedule has parts per row and
+// head (and not only per tile).
+struct Prepared {
+  size_t schedule, rest, carry;
+  bool row_parts;
+};
+int prepared_bytes(const SbaArgs* a, Prepared* out);
+// sba_fwd with the schedule in a->workspace (`schedule` bytes of it).
 int forward_prepared(const SbaArgs* a);
 // Whether the backward these arguments describe can run on the schedule its forward prepared.
 bool prepared_fits(const SbaArgs* a);

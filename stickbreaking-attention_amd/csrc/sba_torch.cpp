@@ -123,12 +123,16 @@ Tensor bytes(size_t n, const Tensor& like) { return at::empty({(int64_t)n}, like
 
 struct Outputs {
   Tensor o, rem;
-  Tensor state;      // one allocation: {schedule, row_stat, carry}; kept for the backward
+  // Kept for the backward: {schedule (kept_schedule bytes, or none), row_stat, carry}, as far as the backward wants them.
+  Tensor state;
+  int64_t kept_schedule = 0;
 };
 size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 size_t row_stat_bytes(const Tensor& q) { return align256(q.numel() / q.size(-1) * 4); }
 
 // `for_backward`: a backward will follow; `want_carry`: it starts from recorded products instead of rebuilding them.
+// The schedule of that backward is prepared (and kept) unless it would go unused, under a workspace limit, or is asked to keep
+// little and the schedule has parts per row (the one-kernel backward's tags); tile lists alone are half a byte per token.
 Outputs run_forward(const Call& c, const Tensor& q, const Tensor& k, const Tensor& v, bool for_backward, bool want_carry) {
   const c10::DeviceGuard guard(q.device());
   SbaArgs a = base_args(c, q);
@@ -139,29 +143,43 @@ Outputs run_forward(const Call& c, const Tensor& q, const Tensor& k, const Tenso
   // No products kept: a backward, if one follows, rebuilds them, and the forward's scheduler checks their capacity as that
   // backward's will (both passes void, or neither).
   a.recompute_carry = !want_carry && a.dtype != SBA_F32;
-  size_t sched = 0, rest = 0, carry = 0;
-  if (for_backward) check(sba::prepared_bytes(&a, &sched, &rest, &carry), "sba_workspace_bytes");
-  else check(sba_workspace_bytes(&a, &sched, nullptr, nullptr), "sba_workspace_bytes");
+  sba::Prepared size{};
+  bool prepare = for_backward && g_bwd_limit.load(std::memory_order_relaxed) < 0;
+  if (for_backward) check(sba::prepared_bytes(&a, &size), "sba_workspace_bytes");
+  if (size.row_parts && !want_carry) prepare = false;
+  size_t sched = size.schedule;
+  if (!prepare) check(sba_workspace_bytes(&a, &sched, nullptr, nullptr), "sba_workspace_bytes");
   const size_t stat = row_stat_bytes(q);
-  out.state = bytes(sched + stat + (want_carry ? carry : 0), q);
-  if (c.flags & kPoison) poison(out.state);
-  char* const base = (char*)out.state.data_ptr();
+  const bool keep_stat = for_backward && (want_carry || c.add_remainder);
+  Tensor scratch;
+  size_t kept = 0, used = 0;      // bytes of `state` and of `scratch` so far
+  (prepare ? kept : used) += sched;
+  (keep_stat ? kept : used) += stat;
+  if (used > 0) scratch = bytes(used, q);
+  if (for_backward) out.state = bytes(kept + (want_carry ? size.carry : 0), q);
+  out.kept_schedule = prepare ? sched : 0;
+  if (c.flags & kPoison) {
+    if (for_backward) poison(out.state);
+    if (used > 0) poison(scratch);
+  }
+  char* const state = for_backward ? (char*)out.state.data_ptr() : nullptr;
+  char* const other = used > 0 ? (char*)scratch.data_ptr() : nullptr;
   a.q = ref<SbaTensor>(q, c.fixed); a.k = ref<SbaTensor>(k, c.fixed); a.v = ref<SbaTensor>(v, c.fixed);
   a.o = ref<SbaTensor>(out.o, c.fixed);
   a.rem = ref<SbaVector>(out.rem, c.fixed);
-  a.row_stat = (float*)(base + sched);
-  a.carry = want_carry ? (float*)(base + sched + stat) : nullptr;
-  a.workspace = base;
+  a.row_stat = (float*)(keep_stat ? state + out.kept_schedule : other + (prepare ? 0 : sched));
+  a.carry = want_carry ? (float*)(state + kept) : nullptr;
+  a.workspace = prepare ? state : other;
   a.workspace_bytes = sched;
-  check(for_backward ? sba::forward_prepared(&a) : sba_fwd(&a), "sba_fwd");
-  if (c.flags & kDebugCheck) check_status(out.state, "sba_fwd");
+  check(prepare ? sba::forward_prepared(&a) : sba_fwd(&a), "sba_fwd");
+  if (c.flags & kDebugCheck) check_status(prepare ? out.state : scratch, "sba_fwd");
   return out;
 }
 
 // `state` as the forward left it; `fresh`: no backward has run on its schedule yet.  What a saved-tensor hook hands back may lie
 // in another place, and in another layout, than what the forward saved.
-variable_list run_backward(Call c, Tensor d_o, Tensor d_rem, Tensor q, Tensor k, Tensor v, Tensor state, bool have_carry,
-                           bool fresh) {
+variable_list run_backward(Call c, Tensor d_o, Tensor d_rem, Tensor q, Tensor k, Tensor v, Tensor state, int64_t kept_schedule,
+                           bool have_carry, bool fresh) {
   for (const Tensor* t : {&q, &k, &v, &state}) require_gpu(*t);
   same_dtype(q, k, "k");
   same_dtype(q, v, "v");
@@ -187,17 +205,20 @@ variable_list run_backward(Call c, Tensor d_o, Tensor d_rem, Tensor q, Tensor k,
   a.d_rem = ref<SbaVector>(d_rem, c.fixed);
   a.dq = ref<SbaTensor>(dq, c.fixed); a.dk = ref<SbaTensor>(dk, c.fixed); a.dv = ref<SbaTensor>(dv, c.fixed);
   a.recompute_carry = !have_carry;      // the forward kept no products: rebuild them in the backward's workspace
-  size_t sched_bytes = 0, rest_bytes = 0, carry_bytes = 0;
-  check(sba::prepared_bytes(&a, &sched_bytes, &rest_bytes, &carry_bytes), "sba_workspace_bytes");
-  TORCH_CHECK((size_t)state.numel() == sched_bytes + row_stat_bytes(q) + (have_carry ? carry_bytes : 0), "saved state of another size");
+  sba::Prepared size{};
+  check(sba::prepared_bytes(&a, &size), "sba_workspace_bytes");
+  const size_t stat = have_carry || c.add_remainder ? row_stat_bytes(q) : 0;
+  TORCH_CHECK((size_t)state.numel() == kept_schedule + stat + (have_carry ? size.carry : 0) &&
+                  (kept_schedule == 0 || (size_t)kept_schedule == size.schedule),
+              "saved state of another size");
   char* const base = (char*)state.data_ptr();
-  a.row_stat = (float*)(base + sched_bytes);
-  a.carry = have_carry ? (float*)(base + sched_bytes + row_stat_bytes(q)) : nullptr;
+  a.row_stat = stat > 0 ? (float*)(base + kept_schedule) : nullptr;
+  a.carry = have_carry ? (float*)(base + kept_schedule + stat) : nullptr;
   const int64_t limit = g_bwd_limit.load(std::memory_order_relaxed);
   // The forward's schedule serves one backward.  Under graph capture it may be replayed more often than the forward.
-  const bool prepared = fresh && limit < 0 && sba::prepared_fits(&a) &&
+  const bool prepared = kept_schedule > 0 && fresh && limit < 0 && sba::prepared_fits(&a) &&
                         c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None;
-  size_t ws_bytes = rest_bytes;
+  size_t ws_bytes = size.rest;
   if (!prepared) {
     check(sba_workspace_bytes(&a, nullptr, &ws_bytes, nullptr), "sba_workspace_bytes");
     if (limit >= 0 && ws_bytes > (size_t)limit) {
@@ -226,7 +247,7 @@ struct StickBreaking : torch::autograd::Function<StickBreaking> {
     ctx->save_for_backward({q, k, v, c.cu, out.state});
     ctx->saved_data["fresh"] = true;
     ctx->saved_data["call"] = c10::IValue(std::vector<int64_t>{c.fixed, c.leading_zero, c.attend_current, c.add_remainder,
-                                                               c.max_seqlen, c.carry_slots, c.flags, save_carry});
+                                                               c.max_seqlen, c.carry_slots, c.flags, save_carry, out.kept_schedule});
     ctx->saved_data["scale"] = c.logit_scale;
     return {out.o, out.rem};
   }
@@ -241,7 +262,7 @@ struct StickBreaking : torch::autograd::Function<StickBreaking> {
     c10::IValue& fresh = ctx->saved_data["fresh"];
     const bool first = fresh.toBool();
     fresh = false;      // (also where the call fails half way through the schedule)
-    variable_list g = run_backward(c, grads[0], grads[1], s[0], s[1], s[2], s[4], n[7], first);
+    variable_list g = run_backward(c, grads[0], grads[1], s[0], s[1], s[2], s[4], n[8], n[7], first);
     g.resize(5);      // call, save_carry
     return g;
   }

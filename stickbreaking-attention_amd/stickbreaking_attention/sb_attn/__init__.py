@@ -36,8 +36,8 @@ class StickBreakingAttention(torch.autograd.Function):
 
 def sb_attn(q, k, v, inv_temp=None, zero_start=True, attend_current=False, add_remainder=False, save_carry=True):
     """``add_remainder=True`` returns ``(o + rem[..., None] * v, rem)`` (what tests/test_attn.py:67 forms from the
-    reference's outputs), fused into the kernels' epilogues.  ``save_carry=False`` keeps only q, k, v for the backward,
-    which then rebuilds the forward's per-(row, sub-tile) products itself."""
+    reference's outputs), fused into the kernels' epilogues.  ``save_carry=False`` keeps only q, k, v and the tile lists
+    for the backward, which then rebuilds the forward's per-(row, sub-tile) products itself (see ``sb_attn_varlen``)."""
     if _native.use_ext():
         out = _native.ext().fixed(q, k, v, inv_temp, attend_current, add_remainder, save_carry, _native.flags())
         if out is not None:

@@ -47,9 +47,11 @@ def sb_attn_varlen(q, k, v, cu_seqlens, max_seqlens=None, inv_temp=None, zero_st
                    add_remainder=False, save_carry=True):
     """``add_remainder=True`` returns ``(o + rem[..., None] * v, rem)``: the combination every caller of the
     reference forms from its outputs (tests/test_varlen.py:103), fused into the kernels' epilogues.
-    ``save_carry=False`` keeps only q, k, v between the forward and the backward, as the reference does, instead of
-    the per-(row, 32-key sub-tile) products (L^2 / 16 bytes per head and sequence); the backward rebuilds them with one
-    more kernel.  Gradients are bit-identical either way.
+    ``save_carry=False`` keeps only q, k, v between the forward and the backward, as the reference does, and the tile lists
+    (32 bytes per 128 rows and per key tile; with ``add_remainder`` also 4 bytes per row and head), instead of the
+    per-(row, 32-key sub-tile) products (L^2 / 16 bytes per head and sequence) and, in eager calls, the prepared schedule of
+    the backward (up to 12 bytes per row and head); the backward rebuilds the products with one more kernel.  Gradients are
+    bit-identical either way.
 
     A ``cu_seqlens`` that exists only on the device (a GPU tensor with ``zero_start=False``, or any call under
     ``torch.compile``) cannot be validated on the host.  The scheduler kernel validates it instead, and also checks

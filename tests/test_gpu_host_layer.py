@@ -1,6 +1,6 @@
 """The torch host layer of eager calls: gradients arriving through only one of the two outputs, and graphs kept for a second
 backward, against the same call with both gradients given; other Python threads while a call waits for the GPU;
-what saved-tensor hooks and checkpointing hand back to the backward."""
+what saved-tensor hooks and checkpointing hand back to the backward; what is held between the passes."""
 import threading
 import time
 
@@ -8,7 +8,7 @@ import pytest
 import torch
 from torch.utils.checkpoint import checkpoint
 
-from stickbreaking_attention import sb_attn, sb_attn_varlen
+from stickbreaking_attention import _native, sb_attn, sb_attn_varlen
 
 pytestmark = pytest.mark.gpu
 
@@ -115,3 +115,41 @@ def test_saved_tensors_that_come_back_different(gpu_device, how, packed, dtype):
             return
         got = grads(out)
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("limit", [False, True])
+@pytest.mark.parametrize("add_remainder", [False, True])
+@pytest.mark.parametrize("save_carry", [False, True])
+@pytest.mark.parametrize("H,L", [(32, 2048), (12, 2048)])
+def test_what_is_held_between_the_passes(gpu_device, H, L, save_carry, add_remainder, limit):
+    """save_carry=False holds no more than tile lists (32 bytes per 128 rows and per 64 keys), and with the remainder term a
+    number per row; save_carry=True the products and, where a schedule is prepared, up to 13 bytes per row and head.  Either backward
+    is the same with a workspace limit, under which nothing is prepared."""
+    D, rows = 128, H * L
+    q, k, v, do = (torch.randn(H, L, D, device=gpu_device).bfloat16() for _ in range(4))
+    for t in (q, k, v):
+        t.requires_grad_()
+    cu = torch.tensor([L], dtype=torch.int32)
+    options = dict(zero_start=False, add_remainder=add_remainder, save_carry=save_carry)
+    want = torch.autograd.grad(sb_attn_varlen(q, k, v, cu, L, **options)[0], [q, k, v], do)
+    saved = []
+
+    def note(t):
+        saved.append(t.nbytes)
+        return t
+
+    try:
+        if limit:
+            _native.set_backward_workspace_limit(1 << 40)
+        with torch.autograd.graph.saved_tensors_hooks(note, lambda t: t):
+            o, rem = sb_attn_varlen(q, k, v, cu, L, **options)
+        held = sum(saved) - 3 * q.nbytes
+        got = torch.autograd.grad(o, [q, k, v], do)
+    finally:
+        _native.set_backward_workspace_limit(None)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    lists = 4096 + 32 * (L // 128 + L // 64 + 2)
+    products = 4 * H * _native.plan_host(cu, False, L).carry_slots
+    allowed = lists + (products + (4 if limit else 13) * rows if save_carry else 4 * rows * add_remainder)
+    print(f"held {held} bytes, allowed {allowed}", flush=True)
+    assert held <= allowed + 2048

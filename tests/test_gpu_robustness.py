@@ -20,49 +20,63 @@ def poisoned(monkeypatch):
     monkeypatch.setattr(_native, "POISON", True)
 
 
+# Few heads take the kernels that split the keys or rows over the waves, many the wide ones (80 x 1349 rows: 105 K).
+@pytest.mark.parametrize("H", [2, 80])
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("attend_current", [False, True])
-def test_poisoned_buffers_lengths_one_past_a_sub_tile(gpu_device, poisoned, D, attend_current):
+def test_poisoned_buffers_lengths_one_past_a_sub_tile(gpu_device, poisoned, D, attend_current, H):
     # L - 1 a multiple of 32 but not of 128: the last key opens a 32-key sub-tile that only rows beyond the
     # sequence's end would sweep; its per-row scalars are never recorded and must never be used.
     lengths = [33, 65, 97, 161, 193, 225, 289, 34, 1, 96, 128, 129]
-    host, dev, cu = small_case(2, D, lengths, torch.bfloat16, seed=41)
-    ref = orc.varlen_stream(*host[:3], cu, attend_current=attend_current, do=host[3], drem=host[4], dtype=torch.float64)
+    host, dev, cu = small_case(H, D, lengths, torch.bfloat16, seed=41)
+    heads = [0, H - 1]
+    ref = orc.varlen_stream(*(t[heads] for t in host[:3]), cu, attend_current=attend_current, do=host[3][heads], drem=host[4][heads],
+                            dtype=torch.float64)
     got = run_varlen(*dev[:3], cu.to(gpu_device), lengths, False, attend_current, dev[3], dev[4])
     for n, a, b in zip(NAMES, got, ref):
-        tol_check(n, a, b, torch.bfloat16, f"poisoned D={D}")
+        assert torch.isfinite(a).all(), n
+        tol_check(n, a[heads], b, torch.bfloat16, f"poisoned H={H} D={D}")
 
 
-@pytest.mark.parametrize("which", ["do", "q"])
-def test_poisoned_buffers_forward_and_backward_on_different_kernel_variants(gpu_device, poisoned, which):
-    # head_dim 128: a tensor at an 8-byte offset sends one pass to the generic 64-key kernels while the other runs the
-    # aligned 32-key kernels; the recorded products must serve both.
-    lengths = [74, 33, 200, 1, 161]
-    host, dev, cu = small_case(2, 128, lengths, torch.bfloat16, seed=42)
-    ref = orc.varlen_stream(*host[:3], cu, do=host[3], drem=host[4], dtype=torch.float64)
+# How the rows of one tensor send its pass to another variant of the kernels: at an 8-byte offset, to the padded loads;
+# so far apart that a sequence's rows span 2 GiB, to the element-by-element kernels, which sweep 64 keys a step.
+@pytest.mark.parametrize("H", [2, 80])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("which,how", [("do", "odd"), ("q", "odd"), ("do", "far"), ("q", "far")])
+def test_poisoned_buffers_forward_and_backward_on_different_kernel_variants(gpu_device, poisoned, which, how, D, H):
+    # the products one variant of the forward records must serve any variant of the backward
+    lengths = [74, 33, 200, 1, 161, 831]
+    host, dev, cu = small_case(H, D, lengths, torch.bfloat16, seed=42)
+    heads = [0, H - 1]
+    ref = orc.varlen_stream(*(t[heads] for t in host[:3]), cu, do=host[3][heads], drem=host[4][heads], dtype=torch.float64)
 
-    def misaligned(t):
-        buf = torch.empty(t.numel() + 4, dtype=t.dtype, device=t.device)
-        view = buf[4:].view(t.shape)
+    def moved(t):
+        if how == "odd":
+            buf = torch.empty(t.numel() + 4, dtype=t.dtype, device=t.device)
+            view = buf[4:].view(t.shape)
+            assert view.data_ptr() % 16 == 8
+        else:
+            stride = 1 << 20
+            assert (max(lengths) + 256) * stride * 2 >= 1 << 31
+            view = torch.empty(t.size(1) * stride, dtype=t.dtype, device=t.device).as_strided(t.shape, (D, stride, 1))
         view.copy_(t)
-        assert view.data_ptr() % 16 == 8
         return view
 
     q, k, v, do, drem = dev
-    if which == "do":
-        do = misaligned(do)          # forward aligned, backward generic
-        got = run_varlen(q, k, v, cu.to(gpu_device), lengths, False, False, do, drem)
+    if which == "do":                # the backward alone takes the other variant
+        got = run_varlen(q, k, v, cu.to(gpu_device), lengths, False, False, moved(do), drem)
     else:
         from stickbreaking_attention import _native
 
-        # forward generic (q misaligned), backward aligned: drive the two launches directly
-        scale = 128 ** -0.5
+        # the forward alone: drive the two launches directly
+        scale = D ** -0.5
         cu_d = cu.to(gpu_device)
-        o, rem, stat, carry = _native.forward(misaligned(q), k, v, cu_d, False, max(lengths), scale, False, want_carry=True)
+        o, rem, stat, carry = _native.forward(moved(q), k, v, cu_d, False, max(lengths), scale, False, want_carry=True)
         got = [o, rem, *_native.backward(do, drem, q, k, v, carry, cu_d, False, max(lengths), scale, False)]
         torch.cuda.synchronize()
     for n, a, b in zip(NAMES, got, ref):
-        tol_check(n, a, b, torch.bfloat16, f"mixed variants ({which} misaligned)")
+        assert torch.isfinite(a).all(), n
+        tol_check(n, a[heads], b, torch.bfloat16, f"mixed variants ({which} {how}) H={H} D={D}")
 
 
 @pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 128), (torch.bfloat16, 64), (torch.bfloat16, 50), (torch.float32, 64)])

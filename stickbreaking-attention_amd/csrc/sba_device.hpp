@@ -253,13 +253,14 @@ struct TileCopy {
 // so, taken upwards from the product below a group of keys, a weight costs one multiplication and one addition, carries
 // the product above the tile without one of its own, and loses nothing to cancellation.  The products below come from
 // one reciprocal of prod(1 + e) per kGroup keys: 20 transcendentals per 16 keys instead of 32, 5.5 instructions per key
-// besides instead of 7.5.  Vector-ALU issue is what bounds this kernel (75 % busy at head_dim 64, 60 % at 128): 32 heads
+// besides instead of 7.5.  Vector-ALU issue is what bounds this kernel (70 % busy at head_dim 64, 55 % at 128): 32 heads
 // x 8192 x 128 653 -> 606 us, 32 heads x 2 x 4096 x 64 227 -> 188 us.  The product of a group has to stay far from
 // overflow; where it does not (keys whose logits add up to 100 octaves in one group of a lane), that lane takes the weights
 // downwards as differences of the running product, one reciprocal per key, where e = inf gives a factor 0 and the whole
-// remaining stick.  A wave with such a lane does both and every lane keeps its own: a row's bits depend on no other row.  Below
-// 100 octaves a product below a group can still underflow where the stick above it is shorter than 2^-26; what is then lost
-// is less than one rounding of the row's sum of weights.
+// remaining stick.  Each lane decides for itself, so a row's bits depend on no other row; that every lane of the wave is tame is
+// asked first only because a uniform branch is the cheaper one (divergent ones alone: +1 to 2 % of the kernel).  Below 100
+// octaves a product below a group can still underflow where the stick above it is shorter than 2^-26; what is then lost is
+// less than one rounding of the row's sum of weights.
 // Hidden keys (diagonal tiles only) get e = 0: factor 1, weight 0.
 template <int N>
 struct Weights {
@@ -267,7 +268,7 @@ struct Weights {
   float t[N];                   // e, then the weights
   float below[N / kGroup];      // 1 / prod(1 + e) of a group, then the running product below it
   float run;                    // product over all N keys
-  bool mine, tame;              // whether the products of this lane's groups are far from overflow; whether every lane's are
+  bool mine, tame;              // whether this lane's groups are far from overflow; whether every lane's are
 
   // Up to the product over the keys; key R is visible iff R < lim.
   template <bool kDiagonal, int NT>
@@ -290,61 +291,41 @@ struct Weights {
     mine = most < 0x1p100f;
     tame = !__any(!mine);
     run = 1.f;
-    if (tame) {
 #pragma unroll
-      for (int g = N / kGroup - 1; g >= 0; --g) {
-        run *= fast_rcp(below[g]);
-        below[g] = run;
+    for (int g = N / kGroup - 1; g >= 0; --g) {
+      run *= fast_rcp(below[g]);
+      below[g] = run;
+    }
+    if (!tame && !mine) {
+      run = 1.f;
+#pragma unroll
+      for (int R = N - 1; R >= 0; --R) {
+        const float before = run, omb = fast_rcp(1.f + t[R]);
+        run *= omb;
+        t[R] = fmaf(-before, omb, before);
       }
-    } else {      // lanes of both kinds, each by the way it would take among lanes like itself
-      float odd = 1.f;
-#pragma unroll
-      for (int R = N - 1; R >= 0; --R) { odd *= fast_rcp(1.f + t[R]); __builtin_amdgcn_sched_barrier(0); }
-#pragma unroll
-      for (int g = N / kGroup - 1; g >= 0; --g) run *= fast_rcp(below[g]);
-      run = mine ? run : odd;
     }
   }
   // The weights; `seed`: the product above the N keys.
   __device__ __forceinline__ void back(float seed) {
     if (tame) {
+      upwards(seed);
+    } else if (mine) {
+      upwards(seed);
+    } else {
 #pragma unroll
-      for (int g = 0; g < N / kGroup; g++) {
-        float r = below[g] * seed;
+      for (int R = 0; R < N; R++) t[R] *= seed;
+    }
+  }
+  __device__ __forceinline__ void upwards(float seed) {
 #pragma unroll
-        for (int i = 0; i < kGroup; i++) {
-          const float e = t[kGroup * g + i];
-          t[kGroup * g + i] = e * r;
-          r = fmaf(e, r, r);
-        }
-      }
-    } else {      // (taken from t again: nothing but t and `mine` is kept for it)
-      float b[N / kGroup];
-      float r = 1.f;
+    for (int g = 0; g < N / kGroup; g++) {
+      float r = below[g] * seed;
 #pragma unroll
-      for (int g = N / kGroup - 1; g >= 0; --g) {
-        float prod_g = 1.f + t[kGroup * g];
-#pragma unroll
-        for (int i = 1; i < kGroup; i++) prod_g = fmaf(prod_g, t[kGroup * g + i], prod_g);
-        r *= fast_rcp(prod_g);
-        b[g] = r;
-      }
-#pragma unroll
-      for (int g = 0; g < N / kGroup; g++) {
-        r = b[g] * seed;
-#pragma unroll
-        for (int i = 0; i < kGroup; i++) {
-          const float e = t[kGroup * g + i];
-          t[kGroup * g + i] = mine ? e * r : e;
-          r = fmaf(e, r, r);
-        }
-      }
-      float odd = 1.f;
-#pragma unroll
-      for (int R = N - 1; R >= 0; --R) {
-        const float before = odd, omb = fast_rcp(1.f + t[R]);
-        odd *= omb;
-        t[R] = mine ? t[R] : fmaf(-before, omb, before) * seed;
+      for (int i = 0; i < kGroup; i++) {
+        const float e = t[kGroup * g + i];
+        t[kGroup * g + i] = e * r;
+        r = fmaf(e, r, r);
       }
     }
   }
@@ -393,7 +374,7 @@ __device__ __forceinline__ void bwd_math_front(BwdMath<16 * NT>& m, const f32x16
   // (D is a running weighted mean of drem and dP, so it neither grows nor cancels), and with C0 = C below the lane's keys
   //   dz_j = sigma_j (seed pe_j u_j - C0)
   // which is 4 instructions per key where summing g and correcting by sigma C takes 6.  The vector ALU is what bounds the
-  // backward kernels (87 % busy in dQ at head_dim 64): dQ 32 heads x 2 x 4096 x 64 345 -> 320 us, see the kernels for the rest.
+  // backward kernels (81 % busy in dQ at head_dim 64): dQ 32 heads x 2 x 4096 x 64 345 -> 320 us, see the kernels for the rest.
   float D = kNeedP ? drem : drem * seed;                    // (kNeedP: P wants seed * pe anyway; else D is kept times seed)
   const float D0 = D;
 #pragma unroll

@@ -13,8 +13,8 @@
 //     of dQ (sub-tiles of 32 dealt round robin, one scalar per row exchanged per step) and the ROWS of dK/dV (nothing
 //     exchanged), and add their partial results through LDS at the end, in a fixed order: bit-reproducible.
 // Measured: 12 heads x 128, 6143 tokens in sequences of up to 2048, forward + backward 0.99 ms; 86.7 ms on the vector ALU
-// with one wave per query row and fp32 atomics for dK/dV.  32 heads x 2048 tokens: forward 0.37, dQ 0.52, dK/dV 0.69 ms =
-// 94, 99 and 100 TFLOP/s of products, where a large fp32 matrix product reaches 154 on this chip.
+// with one wave per query row and fp32 atomics for dK/dV.  32 heads x 2048 tokens: forward 0.34, dQ 0.49, dK/dV 0.67 ms =
+// 100, 104 and 102 TFLOP/s of products, where a large fp32 matrix product reaches 154 on this chip.
 //
 //   fwd_f32_kernel     : keys swept in reverse from the diagonal (as sb_varlen_fwd.py:155-165), running product per row;
 //                        records the product above every 32-key sub-tile in `carry`.
@@ -246,7 +246,8 @@ __device__ __forceinline__ float rcp_f32(float x) {
 // The hardware's exponential flushes results below 2^-126; a wave that holds such a logit takes the library's, which does not
 // and gives the same bits elsewhere (5 instructions more per key: taken always, 12 heads x 6 x 1024 x 128, forward and
 // backward, 970 -> 996 us; taken so, 970).  sigma is the quotient e / (1 + e) with its rounding error taken out, not a multiple
-// of the rounded reciprocal: +0.9 % of the pass, and 2 to 5 % off the error of every output.
+// of the rounded reciprocal, which takes 2 to 5 % off the error of every output.  Both together cost 0.9 % of a pass at head_dim 128,
+// 1.8 % at 64 and 96 and 2.7 % at 32 (12 heads, 6143 tokens: 980 -> 989, 515 -> 525, 740 -> 753, 298 -> 307 us).
 __device__ __forceinline__ float sticks_f32(const f32x16& s, float scale_log2, int lim, float (&beta)[16], float (&pe)[16]) {
   float x[16], lowest = 0.f;
 #pragma unroll
@@ -317,8 +318,9 @@ struct RowsF32Lds {
   static constexpr int kFloats = kLoop > kRed ? kLoop : kRed;
 };
 
+// (Width 96 keeps three waves per SIMD by spilling four registers; 177 registers and two waves take 4 % of a pass more.)
 template <int DH, int kMode>
-__global__ __launch_bounds__(kThreads, 2) void fwd_f32_kernel(FwdParams p) {
+__global__ __launch_bounds__(kThreads, DH == 96 ? 3 : 2) void fwd_f32_kernel(FwdParams p) {
   constexpr int NB = DH / 32;
   __shared__ __attribute__((aligned(16))) float lds[RowsF32Lds<DH, 1>::kFloats];      // Q rows and the waves' scratch, then the final sums
   __shared__ float xch[2][kWaves][32];

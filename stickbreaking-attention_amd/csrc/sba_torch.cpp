@@ -3,8 +3,9 @@
 // backward) it took in Python, which is more than the kernels of a short sequence need.  The backward runs in the autograd
 // thread without the interpreter.  No kernels here; libsba.so has no torch types.
 //
-// Measured per pass, Python before -> now: 12 heads x 64 tokens, forward 31.7 -> 11.3 us; 24 heads x 64, 4 x 256 tokens, forward
-// and backward 197 -> 78 us (its kernels take 54).
+// Measured per pass, Python before -> now: 12 heads x 64 tokens, forward 32 -> 8.1 us; 24 heads x 64, 4 x 256 tokens, forward and
+// backward 195 -> 75 us, or 43 in one process of four (its kernels take 40, and 51 replayed from a graph: the host is what
+// such a pass waits for).
 #include <torch/extension.h>
 
 #include <ATen/ops/empty.h>

@@ -153,3 +153,13 @@ def test_what_is_held_between_the_passes(gpu_device, H, L, save_carry, add_remai
     allowed = lists + (products + (4 if limit else 13) * rows if save_carry else 4 * rows * add_remainder)
     print(f"held {held} bytes, allowed {allowed}", flush=True)
     assert held <= allowed + 2048
+
+
+def test_anomaly_detection(gpu_device):
+    """The node's forward runs without the interpreter's lock; anomaly detection records a Python traceback there."""
+    q, k, v = (torch.randn(2, 100, 64, device=gpu_device).bfloat16().requires_grad_() for _ in range(3))
+    cu = torch.tensor([100], dtype=torch.int32)
+    want = torch.autograd.grad(sb_attn_varlen(q, k, v, cu, 100, zero_start=False)[0].sum(), [q, k, v])
+    with torch.autograd.set_detect_anomaly(True):
+        got = torch.autograd.grad(sb_attn_varlen(q, k, v, cu, 100, zero_start=False)[0].sum(), [q, k, v])
+    assert all(torch.equal(a, b) for a, b in zip(got, want))

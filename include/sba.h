@@ -144,17 +144,20 @@ typedef struct SbaArgs {
                                   exact count follows from the shape. */
   int32_t backward_kernels;    /* How sba_bwd computes dq, dk, dv.  1: a dQ kernel and a dK/dV kernel.  2: where it applies
                                   (head_dim 128, 16-bit, 16-byte aligned rows, a head count that is a multiple of 8, no
-                                  add_remainder) ONE kernel in which the key tiles of a sequence hand the row prefix
-                                  sums and the partial dQ to each other through the L2; the two kernels otherwise.
-                                  0: the one kernel where it applies AND was measured to be the faster one.  Up to 64 K
-                                  rows * heads: no sequence longer than 256 tokens, or at most 32 heads with
-                                  (total_tokens / num_seqs) * num_heads >= 16 K and rows * heads >= 20 K.  Beyond: no
-                                  sequence longer than 128 tokens and more than 96 on average, or at most 32 heads with
-                                  (total_tokens / num_seqs) * num_heads >= 32 K and max_seqlen * num_heads <= 192 K (in
-                                  packed mode an overstated max_seqlen only costs the faster choice).  A head count above 8 that is not a multiple
-                                  of 8 is then split where that pays (long sequences): the largest multiple of 8 through
-                                  the one kernel, the remaining heads through the two, one pass after the other (with
-                                  trace_events, [1] and [2] then bracket the last pass's kernels only).  Must be the
+                                  add_remainder) ONE kernel in which the tiles of a sequence hand partial sums to each
+                                  other through the L2: key tiles (partial dQ) below 64 K rows * heads, row tiles (partial
+                                  dK and dV) from there on; the two kernels otherwise.
+                                  0: what was measured to be the fastest.  Below 64 K rows * heads the one kernel where it
+                                  applies and no sequence is longer than 256 tokens, or at most 32 heads have
+                                  (total_tokens / num_seqs) * num_heads >= 16 K and rows * heads >= 20 K.  From 64 K on the
+                                  kernel on row tiles, with any head count whose heads and sequences spread over the 8 XCDs
+                                  within a seventh, and with add_remainder: as the one kernel where no sequence is
+                                  longer than 128 tokens and the mean is above 96, or at most 32 heads have (total_tokens /
+                                  num_seqs) * num_heads >= 32 K and max_seqlen * num_heads <= 192 K, and else behind a
+                                  kernel that clears what its tiles hand over.  Any other head count above 8 that is
+                                  not a multiple of 8 is split where that pays (long sequences): the largest multiple of 8
+                                  through the one kernel, the remaining heads through the two, one pass after the other
+                                  (with trace_events, [1] and [2] then bracket the last pass's kernels only).  Must be the
                                   same in sba_workspace_bytes and sba_bwd. */
   int32_t reserved0;
 } SbaArgs;
@@ -239,9 +242,10 @@ int sba_fwd_static(const SbaArgs* args);
 int sba_bwd(const SbaArgs* args);
 
 /*
- * How many attention kernels sba_bwd runs for these arguments on the current device when the workspace holds all
- * heads: 1 (the chained kernel, see SbaArgs.backward_kernels) or 2 (dQ, then dK/dV; also for a call whose heads are
- * split between the two forms); a negative SBA_ERR_* for arguments sba_bwd would refuse.  Launches nothing.  For callers that attribute the time between trace_events.
+ * How many kernels sba_bwd runs behind its schedule for these arguments on the current device when the workspace holds
+ * all heads: 1 (see SbaArgs.backward_kernels) or 2 (dQ, then dK/dV; the clearing kernel, then the one on row tiles;
+ * also for a call whose heads are split between two forms); a negative SBA_ERR_* for arguments sba_bwd would refuse.
+ * Launches nothing.  For callers that attribute the time between trace_events.
  * No counterpart in the reference (it always runs one kernel with atomics and locks, sb_varlen_bwd.py:541-640).
  */
 int sba_bwd_kernels(const SbaArgs* args);

@@ -16,6 +16,9 @@ hipError_t launch_bwd_dkv(const BwdParams& p, int dtype_is_f16, int max_tiles, h
 int dkv_key_tile(const BwdParams& p);
 bool chain_supported(const BwdParams& p);
 hipError_t launch_bwd_chain(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
+bool row_supported(const BwdParams& p);
+hipError_t launch_row_clear(uint32_t* region, int64_t bytes, hipStream_t stream);
+hipError_t launch_bwd_row(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
 hipError_t launch_fwd_split(const FwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
 hipError_t launch_fwd_split_carry_only(const FwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
 hipError_t launch_bwd_dq_split(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
@@ -40,15 +43,36 @@ struct Layout {
   size_t off_prefix, off_drem, off_carry, rest_bytes;
   size_t fwd_bytes, bwd_bytes, carry_bytes;
   size_t pass_bytes;                        // what ONE pass over these heads needs (bwd_bytes: what sba_bwd wants, see split_heads)
-  // One-kernel backward: its partial sums share the prefix plane's region (only one of the two backwards runs).
-  int64_t chain_rows;                       // rows per head
-  size_t off_chain_zero, chain_zero_bytes;  // {C, tag} per row, the flags and the heads' XCC ids: cleared with the schedule
+  // The backwards in which tiles hand partial sums to each other; these share the prefix plane's region (only one backward runs).
+  enum Chain { kNone, kKeyTiles, kRowTiles };
+  Chain chain;
+  bool one_kernel;                          // what has to be cleared is cleared with the schedule (else by a kernel in front)
+  int64_t chain_rows;                       // rows per head (key tiles), key blocks per head (row tiles)
+  size_t off_chain_zero, chain_zero_bytes;  // {C, tag} per row or the queues, the flags and the XCC ids: cleared for every call
   size_t off_chain_c, off_chain_flags, off_chain_xcc;
+  int64_t row_group;                        // row tiles: heads per launch (see plan), of which there are row_launches(heads)
+  int64_t row_launches(int64_t heads) const { return cdiv(heads, row_group); }
   int32_t split_heads;                      // > 0: sba_bwd takes this many heads (a multiple of 8) through the one-kernel
                                             // backward and the rest through the two kernels
 };
 
-int plan(const SbaArgs* a, Layout* out) {
+constexpr int64_t kRowTilesFrom = 64 << 10;      // rows x heads from which the backward on row tiles runs (see plan)
+
+// Whether the 8 queues of the backward on row tiles, each fed to one XCD, hold about the same work: (head, sequence) goes to queue
+// (head + heads x sequence) % 8.  With a head count that is a multiple of 8 they do; else a queue may hold one head of a sequence more
+// than another, which evens out over the sequences if none is much longer than the rest.
+bool queues_even(int64_t heads, int64_t seqs, int64_t mean_len, int64_t max_len) {
+  if ((heads & 7) == 0) return true;
+  int64_t units[8] = {0}, most = 0;
+  const int64_t n = seqs < 8 ? seqs : 8;      // (the pattern repeats)
+  for (int64_t s = 0; s < n; s++)
+    for (int64_t q = 0; q < 8; q++) units[(q + heads * s) & 7] += heads / 8 + (q < (heads & 7));
+  for (int64_t u : units) most = u > most ? u : most;
+  return most * 7 <= heads * n && (max_len <= 2 * mean_len || cdiv(heads, 8) * 7 <= heads);      // within 8/7 of the mean
+}
+
+// `row_tiles`: a group of the heads of a call that runs the backward on row tiles, which the group then runs as well.
+int plan(const SbaArgs* a, Layout* out, bool row_tiles = false) {
   if (a->num_heads <= 0 || a->num_seqs <= 0 || a->total_tokens <= 0) return SBA_ERR_SHAPE;
   if (a->head_dim < 1 || a->head_dim > 128) return SBA_ERR_HEAD_DIM;
   if (a->dtype != SBA_BF16 && a->dtype != SBA_F16 && a->dtype != SBA_F32) return SBA_ERR_DTYPE;
@@ -82,35 +106,64 @@ int plan(const SbaArgs* a, Layout* out) {
   L.off_queue = off;       off = align_up(off + (size_t)a->num_heads * sizeof(int32_t), 256);      // per-head tile cursors
   L.carry_bytes = align_up((size_t)L.carry_slots_per_head * a->num_heads * sizeof(float), 256);
   size_t chain_bytes = 0;
-  L.chain_rows = fixed ? B * T : T;
-  // The one-kernel backward is laid out when it is asked for, or (backward_kernels 0) where it is the faster one.  Measured on
-  // 256 compute units, training passes of equal sequences, both backwards in turn, its time over the two kernels':
-  //   rows x heads                       8 heads       16 heads      32 heads
-  //   < 20 K, up to 256 tokens        0.97          0.93 .. 0.97  0.95 .. 0.97
-  //   < 20 K, 1024 to 2048 tokens     1.16 .. 1.25  1.10             -              (a chain of tiles against the split kernels)
-  //   20 K .. 64 K, up to 256 tokens  0.97          0.91 .. 0.97  0.96
-  //   20 K .. 64 K, length x heads
-  //     from 16 K on                  0.79 .. 0.93  0.82 .. 0.92  0.84 .. 0.87
-  //   more, 64 tokens                    -          1.14          1.10 .. 1.17
-  //   more, 128 tokens                   -          0.98          0.91 .. 0.99      (nothing is handed over)
-  //   more, 256 to 1024 tokens        1.04 .. 1.14  1.02 .. 1.09  0.97 .. 1.09
-  //   more, length x heads 32 K       0.96          0.97          1.00
-  //   ... 64 K to 128 K               0.93 .. 0.99  0.93 .. 0.95  0.92 .. 0.96
-  //   ... 192 K                          -          0.96, 0.99    0.96, 0.99
-  //   ... 256 K                          -          1.01, 1.04    1.00, 1.10        (the partial dQ a tile finds has left the L2)
+  const int64_t rows = fixed ? B * T : T;
+  // Left to choose (backward_kernels 0), a backward whose tiles hand partial sums to each other runs where it is the faster one.
+  // Training passes at head_dim 128 on 256 compute units.  Row tiles (sba_bwd_row.hip) over the better of key tiles and the two
+  // kernels, equal sequences of 32768 tokens in all:
+  //   length     64           128          192, 256     384          512          768 .. 4096   8192, 16384
+  //              0.98 .. 1.01 0.92 .. 0.96 0.80 .. 0.86 0.93 .. 0.96 0.82 .. 0.85 0.79 .. 0.85  0.77 .. 0.85    (8 to 32 heads)
+  // A tile is 256 rows, so 64 K rows x heads give a tile to each compute unit.  Down there, by rows x heads:
+  //   64 K       512 .. 1024 tokens 0.77 .. 0.96     2048 tokens 0.86 (4 sequences), 0.97 (2), 1.04 (1)
+  //   32 K       512 tokens 0.82 .. 0.97             1024 tokens 0.97 (4 sequences), 1.22 (2 and 1)     2048 tokens 1.25
+  // where a tile's sweep over its keys is the time of the call, and key tiles of 128 keys are the better ones of long sequences:
+  // key tiles over the two kernels
+  //   20 K .. 64 K, length x heads from 16 K on      0.79 .. 0.93        up to 256 tokens  0.91 .. 0.97
+  //   < 20 K        1024 to 2048 tokens              1.10 .. 1.25        up to 256 tokens  0.93 .. 0.97
+  const int64_t mean_len = fixed ? T : T / B, rows_heads = rows * a->num_heads, mean_heads = mean_len * a->num_heads;
   const bool chain_shape = a->dtype != SBA_F32 && a->head_dim == 128 && (a->num_heads & 7) == 0 && !a->add_remainder;
-  const int64_t mean_len = fixed ? T : T / B, rows_heads = L.chain_rows * a->num_heads, mean_heads = mean_len * a->num_heads;
-  const bool chain_pays = rows_heads <= 64 << 10
-                              ? max_len <= 256 || (a->num_heads <= 32 && rows_heads >= 20 << 10 && mean_heads >= 16 << 10)
-                              : (max_len <= 128 && mean_len > 96) ||
-                                    (a->num_heads <= 32 && mean_heads >= 32 << 10 && max_len * a->num_heads <= 192 << 10);
-  if (chain_shape && (a->backward_kernels == 2 || (a->backward_kernels == 0 && chain_pays))) {
+  if (row_tiles) {
+    L.chain = Layout::kRowTiles;
+  } else if (rows_heads >= kRowTilesFrom && a->dtype != SBA_F32 && a->head_dim == 128 && a->backward_kernels != 1 && (chain_shape || a->backward_kernels == 0)) {
+    // One kernel where its flags were cleared with the schedule ...
+    L.one_kernel = chain_shape && (a->backward_kernels == 2 || (max_len <= 128 && mean_len > 96) ||
+                                   (a->num_heads <= 32 && mean_heads >= 32 << 10 && max_len * a->num_heads <= 192 << 10));
+    if (L.one_kernel || queues_even(a->num_heads, B, mean_len, max_len)) L.chain = Layout::kRowTiles;
+  } else if (chain_shape && (a->backward_kernels == 2 ||
+                             (a->backward_kernels == 0 &&
+                              (max_len <= 256 || (a->num_heads <= 32 && rows_heads >= 20 << 10 && mean_heads >= 16 << 10))))) {
+    L.chain = Layout::kKeyTiles;
+    L.one_kernel = true;
+  }
+  if (L.chain == Layout::kKeyTiles) {
+    L.chain_rows = rows;
     L.off_chain_zero = off;
     L.off_chain_c = off;      off = align_up(off + (size_t)a->num_heads * L.chain_rows * 8, 256);
     L.off_chain_flags = off;  off = align_up(off + (size_t)a->num_heads * L.max_k_tiles * 32, 256);
     L.off_chain_xcc = off;    off = align_up(off + (size_t)a->num_heads * 4, 256);
     L.chain_zero_bytes = off - L.off_chain_zero;
     chain_bytes = align_up((size_t)a->num_heads * L.chain_rows * 128 * sizeof(float), 256);
+  }
+  // Row tiles: the region that is cleared lies in the schedule, or (two kernels) in the rest.
+  auto row_region = [&]() {
+    L.off_chain_zero = off;
+    L.off_chain_c = off;      off = align_up(off + L.row_launches(a->num_heads) * 32, 256);      // the queues
+    L.off_chain_xcc = off;    off = align_up(off + L.row_launches(a->num_heads) * 32, 256);
+    L.off_chain_flags = off;  off = align_up(off + (size_t)a->num_heads * L.max_k_tiles * 32, 256);
+    L.chain_zero_bytes = off - L.off_chain_zero;
+  };
+  if (L.chain == Layout::kRowTiles) {
+    L.chain_rows = rows * 9 / 256 + 2;      // (key blocks of 32: every sequence that hands any over is longer than 256)
+    L.row_group = a->num_heads;
+    // What is handed over lies at its key blocks' places, also where most rows are in sequences that hand nothing over: 1152 bytes
+    // per row and head.  The heads of such a batch go through in several launches, multiples of 8 (an equal share for each
+    // queue), that keep this within 1.15 times the carry plane as long as each still fills the chip twice.
+    if (mean_len < sba::kRowTileRows && max_len > sba::kRowTileRows) {
+      const int64_t least = align_up(cdiv(2 * kRowTilesFrom, rows), 8), fit = (int64_t)L.carry_bytes / 20 * 23 / (L.chain_rows * 32768) & ~7;
+      const int64_t group = fit > least ? fit : least;
+      if (group < a->num_heads) L.row_group = group;
+    }
+    chain_bytes = (size_t)L.row_group * L.chain_rows * 32768;
+    if (L.one_kernel) row_region();
   }
   L.sched_bytes = off;
   off = 0;
@@ -119,6 +172,7 @@ int plan(const SbaArgs* a, Layout* out) {
   L.off_drem = off;        off = align_up(off + (size_t)a->num_heads * (size_t)T * (fixed ? (size_t)B : 1) * sizeof(float), 256);
   // the forward's products, rebuilt inside the backward when the caller did not keep them
   L.off_carry = off;       if (a->recompute_carry) off += L.carry_bytes;
+  if (L.chain == Layout::kRowTiles && !L.one_kernel) row_region();
   L.rest_bytes = off;
   L.bwd_bytes = L.pass_bytes = L.sched_bytes + L.rest_bytes;
   // A head count that is not a multiple of 8 (the reference's own benchmarks use 12) cannot run the one-kernel backward,
@@ -126,12 +180,12 @@ int plan(const SbaArgs* a, Layout* out) {
   // it and the remaining heads through the two kernels, one pass after the other on the stream -- where that pays: two
   // passes have two tails and two schedules, and on the reference's sweep (12 heads, 4 sequences) the split costs 12 %
   // at 4096 tokens and 2 % at 8192 and gains 4 % at 12288 and 16384.  The workspace must hold either pass.
-  if (a->backward_kernels == 0 && (a->num_heads & 7) != 0 && a->num_heads > 8 &&
+  if (!row_tiles && a->backward_kernels == 0 && (a->num_heads & 7) != 0 && a->num_heads > 8 &&
       mean_len * (a->num_heads & ~7) >= (int64_t)12288 * 8) {
     SbaArgs c = *a;
     c.num_heads = a->num_heads & ~7;
     Layout L8;
-    if (plan(&c, &L8) == SBA_OK && L8.chain_zero_bytes > 0) {
+    if (L.chain == Layout::kNone && plan(&c, &L8) == SBA_OK && L8.one_kernel) {
       L.split_heads = c.num_heads;
       if (L8.bwd_bytes > L.bwd_bytes) L.bwd_bytes = L8.bwd_bytes;
     }
@@ -209,6 +263,13 @@ bool few_key_tiles(const SbaArgs* a, int64_t heads, int load) {
   if (a->dtype == SBA_F32 || load == sba::kLoadScalar) return false;
   return a->total_tokens * (a->cu_seqlens ? 1 : a->num_seqs) * heads < 100 << 10;
 }
+// Row strides from 4 MiB on: the offsets of a row tile's rows beyond the sequence would not stay within 32 bits.
+template <size_t N>
+bool wide_rows(const SbaTensor* const (&tensors)[N]) {
+  for (const SbaTensor* t : tensors)
+    if (t->ptr && t->stride_token >= (int64_t)2 << 20) return true;
+  return false;
+}
 int check_tensor(const SbaTensor& t, bool required, bool fixed) {
   if (!t.ptr) return required ? SBA_ERR_NULL : SBA_OK;
   if (t.stride_token < 0 || t.stride_head < 0 || (fixed && t.stride_batch < 0)) return SBA_ERR_STRIDE;
@@ -221,7 +282,7 @@ sba::VectorRef vref(const SbaVector& t, bool fixed) { return sba::VectorRef{t.pt
 // what the one-kernel backward needs cleared.
 sba::SchedParams sched_params(const SbaArgs* a, char* ws, const Layout& L, bool for_backward, bool want_carry_base, int key_tile) {
   sba::SchedParams sp{};
-  if (for_backward && L.chain_zero_bytes > 0) {
+  if (for_backward && L.one_kernel) {
     sp.zero_fill = (uint32_t*)(ws + L.off_chain_zero);
     sp.zero_bytes = (int64_t)L.chain_zero_bytes;
   }
@@ -253,7 +314,18 @@ int clear_wgs(const sba::SchedParams& sp) {
 // Whether the dK/dV kernel of a call with few key tiles runs: the one-kernel backward, where it is laid out and the rows allow
 // it, takes such calls itself.
 bool split_keys(const SbaArgs* a, const Layout& L, int64_t heads, int load) {
-  return !(L.chain_zero_bytes > 0 && load == sba::kLoadAligned) && few_key_tiles(a, heads, load);
+  return !(L.chain != Layout::kNone && load == sba::kLoadAligned) && few_key_tiles(a, heads, load);
+}
+
+// Which of the chained backwards a pass runs: the one that is laid out, if the tensors and the device allow it.
+Layout::Chain chain_of(const Layout& L, const sba::BwdParams& p) {
+  if (L.chain == Layout::kKeyTiles && sba::chain_supported(p)) return L.chain;
+  if (L.chain == Layout::kRowTiles && sba::row_supported(p)) return L.chain;
+  return Layout::kNone;
+}
+// Keys per key tile (row tiles: rows per tile) of the schedule such a pass wants.
+int key_tile_of(const Layout& L, const sba::BwdParams& p) {
+  return chain_of(L, p) == Layout::kRowTiles ? sba::kRowTileRows : sba::dkv_key_tile(p);
 }
 
 // Keys per key tile of the backward that will follow a forward, as far as the forward's tensors tell.
@@ -262,8 +334,11 @@ int expected_key_tile(const SbaArgs* a, const Layout& L) {
   sba::BwdParams p{};
   p.head_dim = a->head_dim;
   p.load = row_load(a, {&a->q, &a->k, &a->v});
+  p.wide_rows = wide_rows({&a->q, &a->k, &a->v});
+  p.num_heads = a->num_heads;
+  p.add_rem = a->add_remainder ? 1 : 0;
   p.split = split_keys(a, L, a->num_heads, p.load);
-  return sba::dkv_key_tile(p);
+  return key_tile_of(L, p);
 }
 
 }  // namespace
@@ -425,24 +500,45 @@ int sba_fwd_static(const SbaArgs* a) {
 namespace {
 
 int bwd_load(const SbaArgs* a) { return row_load(a, {&a->q, &a->k, &a->v, &a->d_o, &a->dq, &a->dk, &a->dv}); }
-// Whether one pass over the heads `a` describes runs the one-kernel backward (its buffers are laid out and the
-// tensors and the device allow it).
-bool bwd_is_chained(const SbaArgs* a, const Layout& L) {
+bool bwd_wide_rows(const SbaArgs* a) { return wide_rows({&a->q, &a->k, &a->v, &a->d_o, &a->dq, &a->dk, &a->dv}); }
+// Whether one pass over the heads `a` describes runs one kernel.
+bool bwd_is_one_kernel(const SbaArgs* a, const Layout& L) {
   sba::BwdParams p{};
   p.load = bwd_load(a);
+  p.wide_rows = bwd_wide_rows(a);
   p.head_dim = a->head_dim;
   p.num_heads = a->num_heads;
   p.add_rem = a->add_remainder ? 1 : 0;
-  return a->dtype != SBA_F32 && L.chain_zero_bytes > 0 && sba::chain_supported(p);
+  return L.one_kernel && chain_of(L, p) != Layout::kNone;
+}
+
+// The backward on row tiles, in the launches that the layout asks for: each has queues of its own, what is handed over takes turns.
+hipError_t launch_row_tiles(const sba::BwdParams& whole, const Layout& L, bool f16, hipStream_t stream) {
+  const int64_t launches = L.row_launches(whole.num_heads);
+  for (int64_t i = 0; i < launches; i++) {
+    sba::BwdParams p = whole;
+    const int64_t h0 = i * L.row_group;
+    p.num_heads = (int32_t)(whole.num_heads - h0 < L.row_group ? whole.num_heads - h0 : L.row_group);
+    for (sba::TensorRef* t : {&p.q, &p.k, &p.v, &p.d_o, &p.dq, &p.dk, &p.dv}) t->ptr = (char*)t->ptr + h0 * t->sh * 2;
+    if (p.d_rem.ptr) p.d_rem.ptr = (char*)p.d_rem.ptr + h0 * p.d_rem.sh * 2;
+    if (p.row_stat) p.row_stat += h0 * p.stat_sh;
+    p.carry += h0 * p.carry_head_stride;
+    p.chain_c += 8 * i;
+    p.chain_head_xcc += 8 * i;
+    p.chain_flags += h0 * p.chain_tile_cap * 8;
+    const hipError_t e = sba::launch_bwd_row(p, f16, (int)L.max_k_tiles, stream);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 // One pass of the backward over the heads `a` describes (all of them, or one group of a larger call: `stat_heads` is
 // the head count of the caller's row_stat array, `first`/`last` say which trace events this pass records).  `sched`: the
 // schedule a forward left (the workspace is then the rest), or NULL to run the
 // scheduler here.
-int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* sched = nullptr) {
+int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* sched = nullptr, bool row_tiles = false) {
   Layout L;
-  int st = plan(a, &L);
+  int st = plan(a, &L, row_tiles);
   if (st != SBA_OK) return st;
   const bool fixed = a->cu_seqlens == nullptr;
   const size_t es = elem_size(a->dtype);
@@ -487,13 +583,15 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* 
   p.max_tiles = (int32_t)L.max_q_tiles;
   p.total_tokens = a->total_tokens;
   p.load = bwd_load(a);
+  p.wide_rows = bwd_wide_rows(a);
   p.split = split_keys(a, L, stat_heads, p.load);
   // One kernel (the key tiles of a sequence hand C and partial dQ to each other) where it applies, else dQ then dK/dV.
-  const bool chain = bwd_is_chained(a, L);
-  if (chain) {
-    p.chain_c = (uint32_t*)(ws + L.off_chain_c);
-    p.chain_flags = (int32_t*)(ws + L.off_chain_flags);
-    p.chain_head_xcc = (int32_t*)(ws + L.off_chain_xcc);
+  const Layout::Chain chain = a->dtype == SBA_F32 ? Layout::kNone : chain_of(L, p);
+  char* const cleared = L.one_kernel ? ws : rest;
+  if (chain != Layout::kNone) {
+    p.chain_c = (uint32_t*)(cleared + L.off_chain_c);
+    p.chain_flags = (int32_t*)(cleared + L.off_chain_flags);
+    p.chain_head_xcc = (int32_t*)(cleared + L.off_chain_xcc);
     p.chain_dq = (float*)(rest + L.off_prefix);
     p.status = (int32_t*)(ws + L.off_counts) + sba::kCountStatus;
     p.chain_rows = L.chain_rows;
@@ -501,7 +599,7 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* 
     p.chain_tile_cap = (int32_t)L.max_k_tiles;
   }
   // The key-tile list is built for the dK/dV kernel that will run.
-  const int key_tile = a->dtype == SBA_F32 ? kBlockK : sba::dkv_key_tile(p);
+  const int key_tile = a->dtype == SBA_F32 ? kBlockK : key_tile_of(L, p);
   if (!sched) {
     const sba::SchedParams sp = sched_params(a, ws, L, true, true, key_tile);
     if (sba::launch_sched(sp, clear_wgs(sp), stream) != hipSuccess) return SBA_ERR_LAUNCH;
@@ -534,9 +632,15 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* 
                                           : sba::launch_fwd_carry_only(f, a->dtype == SBA_F16, (int)L.max_q_tiles, stream)) != hipSuccess)
       return SBA_ERR_LAUNCH;
   }
-  if (chain) {
+  if (chain != Layout::kNone) {
+    if (!L.one_kernel && sba::launch_row_clear((uint32_t*)(cleared + L.off_chain_zero), (int64_t)L.chain_zero_bytes, stream) != hipSuccess)
+      return SBA_ERR_LAUNCH;
     if (ev && last && hipEventRecord(ev[1], stream) != hipSuccess) return SBA_ERR_LAUNCH;
-    if (sba::launch_bwd_chain(p, a->dtype == SBA_F16, (int)L.max_k_tiles, stream) != hipSuccess) return SBA_ERR_LAUNCH;
+    if (chain == Layout::kRowTiles) {
+      if (launch_row_tiles(p, L, a->dtype == SBA_F16, stream) != hipSuccess) return SBA_ERR_LAUNCH;
+    } else if (sba::launch_bwd_chain(p, a->dtype == SBA_F16, (int)L.max_k_tiles, stream) != hipSuccess) {
+      return SBA_ERR_LAUNCH;
+    }
     if (ev && last && hipEventRecord(ev[2], stream) != hipSuccess) return SBA_ERR_LAUNCH;
     return SBA_OK;
   }
@@ -561,7 +665,7 @@ int sba_bwd_kernels(const SbaArgs* a) {
   Layout L;
   const int st = plan(a, &L);
   if (st != SBA_OK) return st;
-  return bwd_is_chained(a, L) ? 1 : 2;
+  return bwd_is_one_kernel(a, L) ? 1 : 2;
 }
 
 int sba_bwd(const SbaArgs* a) {
@@ -584,7 +688,7 @@ int sba_bwd(const SbaArgs* a) {
   if (L.split_heads > 0 && a->workspace_bytes >= L.bwd_bytes) {
     SbaArgs c = heads_from(0, L.split_heads);
     Layout L8;
-    if (plan(&c, &L8) == SBA_OK && bwd_is_chained(&c, L8)) {      // (the tensors and the device allow the one kernel)
+    if (plan(&c, &L8) == SBA_OK && bwd_is_one_kernel(&c, L8)) {      // (the tensors and the device allow the one kernel)
       if ((st = bwd_pass(&c, a->num_heads, true, false)) != SBA_OK) return st;
       c = heads_from(L.split_heads, a->num_heads - L.split_heads);
       c.backward_kernels = 1;
@@ -595,25 +699,36 @@ int sba_bwd(const SbaArgs* a) {
   // A workspace smaller than the whole call needs: the heads are independent, so they go through in groups of as many
   // as fit (the per-head planes dominate the workspace), one group after the other on the stream.
   SbaArgs c = *a;
-  int64_t lo = 0, hi = a->num_heads;           // largest head count whose layout fits: plan() grows with num_heads
-  while (lo < hi) {
-    c.num_heads = (int32_t)((lo + hi + 1) / 2);
-    if (plan(&c, &L) == SBA_OK && L.pass_bytes <= a->workspace_bytes) lo = c.num_heads; else hi = c.num_heads - 1;
+  int32_t kernels = a->backward_kernels;
+  // The largest head count whose layout fits: plan() grows with num_heads.
+  auto largest = [&](bool row_tiles) {
+    int64_t lo = 0, hi = a->num_heads;
+    while (lo < hi) {
+      c.num_heads = (int32_t)((lo + hi + 1) / 2);
+      if (plan(&c, &L, row_tiles) == SBA_OK && L.pass_bytes <= a->workspace_bytes) lo = c.num_heads; else hi = c.num_heads - 1;
+    }
+    return lo;
+  };
+  const Layout::Chain whole = L.chain;
+  int64_t lo = whole == Layout::kRowTiles ? largest(true) : 0;
+  const bool row_tiles = lo > 0;
+  if (!row_tiles) {      // (a call that would not run either of the chained backwards runs the two kernels in groups too)
+    if (whole != Layout::kKeyTiles) kernels = c.backward_kernels = 1;
+    lo = largest(false);
   }
   if (lo < 1) return SBA_ERR_WORKSPACE;
   const int64_t passes = cdiv(a->num_heads, lo), group = cdiv(a->num_heads, passes);
   // The one-kernel backward's layout is the larger one and is only laid out for head counts it applies to, so a group
   // size below `lo` need not fit although `lo` does: every pass then takes the two-kernel backward, whose layout grows
   // with the head count and therefore fits.
-  int32_t kernels = a->backward_kernels;
   for (int64_t heads : {group, a->num_heads % group}) {
     c.num_heads = (int32_t)heads;
-    if (heads > 0 && (plan(&c, &L) != SBA_OK || L.pass_bytes > a->workspace_bytes)) kernels = 1;
+    if (heads > 0 && !row_tiles && (plan(&c, &L) != SBA_OK || L.pass_bytes > a->workspace_bytes)) kernels = 1;
   }
   for (int64_t h0 = 0; h0 < a->num_heads; h0 += group) {
     c = heads_from(h0, a->num_heads - h0 < group ? a->num_heads - h0 : group);
     c.backward_kernels = kernels;
-    if ((st = bwd_pass(&c, a->num_heads, h0 == 0, h0 + group >= a->num_heads)) != SBA_OK) return st;
+    if ((st = bwd_pass(&c, a->num_heads, h0 == 0, h0 + group >= a->num_heads, nullptr, row_tiles)) != SBA_OK) return st;
   }
   return SBA_OK;
 }
@@ -626,7 +741,7 @@ int prepared_bytes(const SbaArgs* a, Prepared* out) {
   Layout L;
   const int st = plan(a, &L);
   if (st != SBA_OK) return st;
-  *out = Prepared{L.sched_bytes, L.rest_bytes, L.carry_bytes, L.chain_zero_bytes > 0};
+  *out = Prepared{L.sched_bytes, L.rest_bytes, L.carry_bytes, L.one_kernel};
   return SBA_OK;
 }
 
@@ -638,8 +753,11 @@ bool prepared_fits(const SbaArgs* a) {
   BwdParams p{};
   p.head_dim = a->head_dim;
   p.load = bwd_load(a);
+  p.wide_rows = bwd_wide_rows(a);
+  p.num_heads = a->num_heads;
+  p.add_rem = a->add_remainder ? 1 : 0;
   p.split = split_keys(a, L, a->num_heads, p.load);
-  return a->dtype == SBA_F32 || dkv_key_tile(p) == expected_key_tile(a, L);
+  return a->dtype == SBA_F32 || key_tile_of(L, p) == expected_key_tile(a, L);
 }
 
 int backward_prepared(const SbaArgs* a, void* sched) { return bwd_pass(a, a->num_heads, true, true, (char*)sched); }

@@ -1,0 +1,523 @@
+// Backward on row tiles: dq, dk and dv from ONE evaluation of S, dP and the tile math per visible (query, key) pair.
+//
+// One workgroup = 8 waves = one tile of 256 query rows of one (head, sequence), 32 rows per wave (lane l owns query l%32), which
+// sweeps the keys UPWARDS from key 0 to its diagonal in blocks of 32.  C, the prefix sum of g along a row, therefore stays in a
+// register, and dQ is accumulated in registers as in the dQ kernel (sba_bwd_dq.hip).  What crosses rows is dK and dV: every wave
+// leaves its P and dZ of the block in LDS, and each of the 8 waves contracts one 32 x 32 piece of {dV, dK} over the 256 rows, dO or Q
+// as stationary operands in registers.  The piece is added to what the row tile ABOVE left of it in memory and left for the row
+// tile below; the tile that holds the keys' own rows converts and stores the result.  So the row tiles of a (head, sequence) form
+// a chain: the last one (whose sweep is longest) starts, and a tile follows the one above it a block or two behind.  Each sum is
+// formed in one fixed order: the same bits every time, no atomics (the reference adds dK and dV tiles behind a spin lock:
+// stickbreaking_attention/sb_varlen/sb_varlen_bwd.py:11-53).
+//
+// Hand-over.  A wave issues its stores, waits for them (vmcnt) and then stores the number of key blocks that are complete into a flag of
+// its own; the same wave of the tile below reads flag and partial results with sc1 (served by the L2, never by the vector L1).  All
+// tiles of a (head, sequence) run on one XCD, i.e. on one L2: (head, sequence) belongs to one of 8 queues, a workgroup takes
+// tiles from queue blockIdx % 8 (workgroups are dealt to the XCDs in turn), and every workgroup checks its XCC id against the first
+// of its queue.  Progress: tiles are taken in list order, a tile waits only for one that was taken before it, so every wait ends;
+// the waits are bounded all the same.
+//
+// What bounds it: per 32 x 32 block and wave 40 MFMAs (1280 cycles), 320 vector-ALU instructions and 48 KB of LDS reads, two waves per
+// SIMD.  The waves of a SIMD (w and w + 4) are kept out of step: one contracts the block of the step before at the start of a
+// step, the other at its end (32 heads x 8 x 4096: 4970 -> 4660 us per training pass).  32 heads x 8 x 4096 x 128, one pass of
+// the backward: 4180 us with key tiles (sba_bwd_chain.hip), 3330 us here; 32768 tokens in 25 sequences of up to 4096, 32 heads: 2650 and
+// 2150.  Without the hand-over it would take 3130, without the tile math as well 2590: at 2.1 GHz, the clock that the power limit
+// leaves, and 2.0 for the products alone.  256 rows per tile, because the hand-over costs 8 bytes per pair / (rows / 256).
+#include "sba_device.hpp"
+#include "sba_host.hpp"
+#include "sba_params.hpp"
+
+#include <atomic>
+#include <type_traits>
+
+namespace sba {
+
+constexpr int kRowTile = kRowTileRows;      // query rows per workgroup
+constexpr int kRowWaves = 8, kRowThreads = 64 * kRowWaves;
+constexpr int kRowKeys = 32;                // keys per step
+
+struct RowLds {
+  static constexpr int kExch = 0;                      // 2 x {P, dZ} of a step: [row][32 keys], 16 KB each
+  static constexpr int kExchBuf = 32768, kExchMat = 16384;
+  static constexpr int kQ = 65536;                     // Q of the tile: 4 panels of [row][32 columns]
+  static constexpr int kPanel = kRowTile * 64;
+  static constexpr int kKv = 131072;                   // 2 x {K, V} of a step: 4 panels of [key][32 columns] each
+  static constexpr int kKvBuf = 16384, kKvMat = 8192, kKvPanel = kRowKeys * 64;
+  static constexpr int kBytes = 163840;
+};
+
+typedef __attribute__((address_space(3))) unsigned char lds_u8;
+
+template <typename V>
+__device__ __forceinline__ V lds_load(lds_u8* p) { return *reinterpret_cast<__attribute__((address_space(3))) V*>(p); }
+
+__device__ __forceinline__ u32x4 buffer_desc(const void* base, int bytes) {
+  const uint64_t a = (uint64_t)base;
+  return u32x4{(uint32_t)a, (uint32_t)(a >> 32) & 0xffffu, (uint32_t)bytes, 0x00020000u};
+}
+// The scalars of a vector-memory instruction must not have been written by a vector instruction (as a reloaded spill is) in the
+// five wait states before it.  The compiler sees to that for its own instructions, not for those in inline assembly: each of
+// these statements begins with its own five.
+//
+// 64 x 16 bytes from a buffer straight into LDS, lane i's to lds + 16 i; twice, kStep bytes apart there.
+template <int kStep>
+__device__ __forceinline__ void dma16x2(int lds, int voff, u32x4 desc, int soff0, int soff1) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds\n\t"
+               "s_mov_b32 m0, %5\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %4 offen lds"
+               ::"s"(lds), "v"(voff), "s"(desc), "s"(soff0), "s"(soff1), "s"(lds + kStep) : "memory");
+}
+template <int kLeft>
+__device__ __forceinline__ void vm_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLeft) : "memory"); }
+
+template <typename T>
+__device__ __forceinline__ typename Elem<T>::vec8 tr_pair(lds_u8* p0, lds_u8* p1) {
+  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+  typedef __attribute__((ext_vector_type(8))) short s16x8;
+  s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p0);
+  s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p1);
+  s16x8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  return __builtin_bit_cast(typename Elem<T>::vec8, v);
+}
+
+__device__ __forceinline__ void lds_put(lds_u8* p, u32x4 v) { *reinterpret_cast<__attribute__((address_space(3))) u32x4*>(p) = v; }
+// x ^ kBit, computed where it is used: kept over the loop it would cost a register the loop does not have.
+template <int kBit>
+__device__ __forceinline__ int flip(int x) {
+  int r;
+  asm volatile("v_xor_b32 %0, %1, %2" : "=v"(r) : "n"(kBit), "v"(x));
+  return r;
+}
+
+// The tile math of 32 rows x 32 keys (bwd_math_front / bwd_math_back) in two parts, so that dP need not be there for the first:
+// P, which leaves for LDS at once, and sigma and the products below each key for the second.
+template <typename T>
+struct RowMath {
+  float beta[16], pe[16], seed;
+  // s: base-2 logits, -inf where hidden.
+  __device__ __forceinline__ void weights(const f32x16& s, int half, float prod_in, lds_u8* p_out) {
+    float run = 1.f;
+#pragma unroll
+    for (int R = 15; R >= 0; --R) {
+      const float omb = fast_rcp(1.f + fast_exp2(s[R]));
+      beta[R] = 1.f - omb;
+      run *= omb;
+      pe[R] = run;
+    }
+    const float oth = other_half(run, half);
+    seed = half ? prod_in : prod_in * oth;
+    float above = seed;
+#pragma unroll
+    for (int i = 1; i >= 0; --i) {
+      float a[8];
+#pragma unroll
+      for (int r = 7; r >= 0; --r) {
+        const int R = 8 * i + r;
+        a[r] = beta[R] * above;
+        above = pe[R] * seed;
+        pe[R] = above;
+      }
+      lds_put(i ? (lds_u8*)(uintptr_t)((int)(uintptr_t)p_out ^ 16) : p_out, u32x4{pack2<T>(a[0], a[1]), pack2<T>(a[2], a[3]), pack2<T>(a[4], a[5]), pack2<T>(a[6], a[7])});
+    }
+  }
+  __device__ __forceinline__ void gradients(const f32x16& dp, int half, float drem, float& prefix, u32x4 (&dz)[2]) {
+    float u[16], D = drem;
+#pragma unroll
+    for (int R = 0; R < 16; R++) {
+      u[R] = dp[R] - D;
+      D = fmaf(beta[R], u[R], D);
+    }
+    const float tot = (D - drem) * seed, oth_g = other_half(tot, half);
+    const float below = prefix + (half ? oth_g : 0.f);
+    prefix += tot + oth_g;
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+      dz[i >> 2][i & 3] = pack2<T>(beta[2 * i] * fmaf(pe[2 * i], u[2 * i], -below), beta[2 * i + 1] * fmaf(pe[2 * i + 1], u[2 * i + 1], -below));
+  }
+};
+
+// The lane's number, computed where it is used (see flip).
+__device__ __forceinline__ int this_lane() {
+  int r;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(r));
+  return r;
+}
+
+// Until the tile above has passed on more than t key blocks: how many it has.
+__device__ __forceinline__ int wait_for(const int32_t* pred, int t, int32_t* status, int lane) {
+  int v = 0;
+#pragma unroll 1
+  for (int spins = 0; spins < (1 << 20); spins++) {
+    asm volatile("s_nop 4\n\tglobal_load_dword %0, %1, %2 sc1\n\ts_waitcnt vmcnt(0)" : "=v"(v) : "v"(0), "s"(pred) : "memory");
+    v = __builtin_amdgcn_readfirstlane(v);
+    if (v > t) return v;
+    __builtin_amdgcn_s_sleep(1);
+  }
+  if (lane == 0) atomicMax(status, kSchedChainTimeout);
+  return 0x7fffffff;      // no later wait of this tile
+}
+
+template <typename T, bool kAddRem>
+__global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
+  constexpr int DH = 128, kSteps = DH / 16, kDTiles = DH / 32;
+  typedef typename Elem<T>::vec8 vec8;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
+  lds_u8* const lds = (lds_u8*)lds_raw;
+  const int lds_base = __builtin_amdgcn_readfirstlane((int)(uintptr_t)lds);
+
+  const int n_tiles = p.counts[kCountK];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int half = lane >> 5, col = lane & 31;
+  const int ac = p.attend_current, H = p.num_heads;
+  const int queue = blockIdx.x & 7;
+  int32_t* const cursor = (int32_t*)p.chain_c + queue;
+
+  if (threadIdx.x == 0) {
+    const int xcc = (int)(__builtin_amdgcn_s_getreg((20) | (0 << 6) | ((4 - 1) << 11)) & 15) + 1;     // HW_REG_XCC_ID
+    const int old = atomicCAS(p.chain_head_xcc + queue, 0, xcc);
+    if (old != 0 && old != xcc) atomicMax(p.status, kSchedChainXcd);
+  }
+  // Rows of the packed token axis that belong to no sequence: zero gradients.
+  {
+    const int64_t covered = p.counts[kCountCovered];
+    if (covered < p.total_tokens) {
+      const int parts = ((int)gridDim.x + H - 1) / H;
+      const int64_t n = p.total_tokens - covered, per = (n + parts - 1) / parts;
+      for (int i = blockIdx.x; i < parts * H; i += gridDim.x) {
+        const int64_t a = covered + per * (i / H), b = a + per < p.total_tokens ? a + per : p.total_tokens;
+        if (a < b) {
+          zero_rows<T>(p.dq, i % H, a, b, DH);
+          zero_rows<T>(p.dk, i % H, a, b, DH);
+          zero_rows<T>(p.dv, i % H, a, b, DH);
+        }
+      }
+    }
+  }
+
+  // Where a lane reads and writes in the panels: 64-byte rows whose 16-byte chunks are XORed with (row >> 2) & 3.
+  const int sw = (col >> 2) & 3, s15 = lane & 15, g = (lane >> 4) & 1;
+  const int row_a = col * 64 + ((half ^ sw) << 4);                                            // row reads; odd steps: ^ 32
+  const int tr_chunk = 2 * g + ((s15 >> 1) & 1), tr_byte = 8 * (s15 & 1);
+  const int tr_e = (8 * half + (s15 >> 2)) * 64 + ((tr_chunk ^ (2 * half)) << 4) + tr_byte;   // 4 rows down; the next 4: (^ 16) + 256
+  const int tr_k = (4 * half + (s15 >> 2)) * 64 + ((tr_chunk ^ half) << 4) + tr_byte;         // ... in key order: (^ 32) + 512
+  const int wr_a = (32 * wave + col) * 64 + (((2 * half) ^ sw) << 4);                         // 8 of this lane's keys; the others: ^ 16
+
+  const bool out = wave >= 4;              // which result this wave contracts: dK, else dV
+  const int cp = wave & 3;                 // ... and which 32 columns of it
+  const int per_slot = (H + 7) >> 3;       // heads of a tile slot that a queue may hold
+
+  for (;;) {
+    if (threadIdx.x == 0) *reinterpret_cast<int*>(lds_raw) = atomicAdd(cursor, 1);
+    __syncthreads();
+    const int claim = __builtin_amdgcn_readfirstlane(*reinterpret_cast<int*>(lds_raw));
+    __syncthreads();
+    const int slot = claim / per_slot;
+    if (slot >= n_tiles) break;
+    Tile tile = p.k_tiles[slot];
+    const int L = __builtin_amdgcn_readfirstlane(tile.seq_len), seq_id = __builtin_amdgcn_readfirstlane(tile.seq_id);
+    const int head = ((queue - seq_id * H) & 7) + 8 * (claim - slot * per_slot);
+    if (head >= H) continue;
+    const int64_t tok0 = __builtin_amdgcn_readfirstlane(tile.seq_start);
+    const int64_t carry_base = (int64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)tile.carry_base) |
+                               (int64_t)__builtin_amdgcn_readfirstlane((int)(tile.carry_base >> 32)) << 32;
+    // The list holds the tiles first to last; they are taken last to first.
+    const int n_rt = (L + kRowTile - 1) / kRowTile;
+    const int I = n_rt - 1 - __builtin_amdgcn_readfirstlane(tile.origin) / kRowTile, q0 = I * kRowTile;
+    const bool has_pred = I < n_rt - 1;
+    const int n = (min(q0 + kRowTile, L) + kRowKeys - 1) / kRowKeys;      // key blocks of this tile
+    const int own = q0 / kRowKeys;                                        // the first of the tile's own rows' keys
+    const int w_hi = (min(kRowTile, L - q0) + 31) / 32;                   // waves with rows
+
+    const T* qb = (const T*)p.q.ptr + seq_id * p.q.sb + head * p.q.sh + tok0 * p.q.st;
+    const T* kb = (const T*)p.k.ptr + seq_id * p.k.sb + head * p.k.sh + tok0 * p.k.st;
+    const T* vb = (const T*)p.v.ptr + seq_id * p.v.sb + head * p.v.sh + tok0 * p.v.st;
+    const T* dob = (const T*)p.d_o.ptr + seq_id * p.d_o.sb + head * p.d_o.sh + tok0 * p.d_o.st;
+    const int q_st = (int)(p.q.st * 2), do_st = (int)(p.d_o.st * 2);
+    // K and V rows of key block t into stage t & 1: waves 0-3 bring a panel of K each, 4-7 one of V.
+    const int kv_st = (int)((out ? p.v.st : p.k.st) * 2);
+    const u32x4 kv_desc = buffer_desc(out ? vb : kb, (L - 1) * kv_st + 2 * DH);
+    const int kv_voff = mfma_row_to_key32(lane >> 2) * kv_st + cp * 64 + (((lane & 3) ^ ((lane >> 4) & 3)) << 4);
+    auto request_kv = [&](int t) {
+      const int soff = min(t, n - 1) * kRowKeys * kv_st;
+      dma16x2<1024>(lds_base + RowLds::kKv + (t & 1) * RowLds::kKvBuf + wave * 2048, kv_voff, kv_desc, soff, soff + 8 * kv_st);
+    };
+    // Q and dO of the tile; dO into the exchange buffers until its operands are in registers.
+    {
+      const u32x4 q_desc = buffer_desc(qb, (L - 1) * q_st + 2 * DH), do_desc = buffer_desc(dob, (L - 1) * do_st + 2 * DH);
+      const int chunk = ((lane & 3) ^ ((lane >> 4) & 3)) * 16;
+      const int q_voff = (lane >> 2) * q_st + chunk, do_voff = (lane >> 2) * do_st + chunk;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {      // panel i, rows 16 wave and 128 + 16 wave
+        const int row = q0 + 16 * wave, dst = lds_base + wave * 1024 + i * RowLds::kPanel;
+        dma16x2<8192>(dst + RowLds::kQ, q_voff, q_desc, row * q_st + 64 * i, (row + 128) * q_st + 64 * i);
+        dma16x2<8192>(dst + RowLds::kExch, do_voff, do_desc, row * do_st + 64 * i, (row + 128) * do_st + 64 * i);
+      }
+    }
+    request_kv(0);
+    const int w_first = q0 + 32 * wave, w_last = w_first + 31, qi = w_first + col;
+    const bool row_ok = qi < L;
+    float drem = 0.f;
+    if (row_ok && p.d_rem.ptr) drem = (float)((const T*)p.d_rem.ptr)[seq_id * p.d_rem.sb + head * p.d_rem.sh + (tok0 + qi) * p.d_rem.st];
+    // The forward's product above key block u for this lane's row (kept within what was recorded).
+    const int n_qt = (L + kBlockQ - 1) / kBlockQ;
+    const int last_seen = min(w_last, L - 1) - 1 + ac;                    // last key a row of this wave sees
+    const int u_last = w_first < L && last_seen > 0 ? last_seen / kRowKeys : 0;
+    const float* carry = p.carry + (int64_t)head * p.carry_head_stride + carry_base;
+    const int row_c = min(qi, L - 1);
+    auto product_at = [&](int t) {
+      const int u = min(t, u_last);
+      return carry + (carry_offset(u, n_qt) - kBlockQ * (u >> 2));
+    };
+    // What the row tiles of a (head, sequence) hand down: per key block and wave, the 32 x 32 partial result.
+    float* part = p.chain_dq + ((int64_t)head * p.chain_rows + ((int64_t)seq_id * p.chain_sb + tok0) * 9 / 256) * 8192 + wave * 1024;
+    int32_t* flag = p.chain_flags + ((int64_t)head * p.chain_tile_cap + slot) * 8 + wave;
+    const int32_t* pred = has_pred ? flag - 8 : flag;
+    const int lane16 = lane * 16;
+
+    vm_wait<0>();
+    __syncthreads();
+    vec8 dof[kSteps], wf[16];
+    {
+      lds_u8* rows = lds + RowLds::kExch + 32 * wave * 64;
+#pragma unroll
+      for (int kk = 0; kk < kSteps; kk++) dof[kk] = lds_load<vec8>(rows + ((kk & 1) ? row_a ^ 32 : row_a) + (kk >> 1) * RowLds::kPanel);
+      lds_u8* cols = lds + (out ? RowLds::kQ : RowLds::kExch) + cp * RowLds::kPanel;
+#pragma unroll
+      for (int c = 0; c < 16; c++) wf[c] = tr_pair<T>(cols + tr_e + 1024 * c, cols + (tr_e ^ 16) + 256 + 1024 * c);
+    }
+    if (kAddRem) {      // the forward wrote o + rem * v: the gradient reaching rem is d_rem + d_o . v_i
+      float dot = 0.f;
+      const RowSource<T> vsrc = make_row_source<T, kLoadAligned>(vb, p.v.st, L, DH);
+#pragma unroll
+      for (int kk = 0; kk < kSteps; kk++) {
+        const vec8 vf = as_vec8<T>(__builtin_amdgcn_raw_buffer_load_b128(vsrc.rsrc, chunk_offset<T, kLoadAligned>(vsrc, qi, 16 * kk + 8 * half), 0, 0));
+#pragma unroll
+        for (int t = 0; t < 8; t++) dot = fmaf((float)dof[kk][t], (float)vf[t], dot);
+      }
+      drem += dot + other_half(dot, half);
+    }
+    f32x16 dqacc[kDTiles];
+#pragma unroll
+    for (int dt = 0; dt < kDTiles; dt++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) dqacc[dt][r] = 0.f;
+    float prefix = 0.f;
+
+    const RowSink<T> sink = out ? make_row_sink<T>((T*)p.dk.ptr + seq_id * p.dk.sb + head * p.dk.sh + tok0 * p.dk.st, p.dk.st, L, DH)
+                                : make_row_sink<T>((T*)p.dv.ptr + seq_id * p.dv.sb + head * p.dv.sh + tok0 * p.dv.st, p.dv.st, L, DH);
+    float n_prod;
+    int seen_count = 0;      // key blocks the tile above has passed on, as last read
+    asm volatile("s_nop 4\n\tglobal_load_dword %0, %1, %2" : "=v"(n_prod) : "v"(row_c * 4), "s"(product_at(0)) : "memory");
+    asm volatile("s_waitcnt vmcnt(0)" : "+v"(n_prod)::"memory");
+
+    f32x4 c0 = {0.f, 0.f, 0.f, 0.f}, c1 = c0, c2 = c0, c3 = c0;      // what the tile above has passed on of the key block contracted next
+    auto contract = [&](int tc) {
+      f32x16 acc;
+#pragma unroll
+      for (int r = 0; r < 16; r++) acc[r] = 0.f;
+      lds_u8* ex = lds + RowLds::kExch + (tc & 1) * RowLds::kExchBuf + (out ? RowLds::kExchMat : 0);
+      lds_u8* e0 = ex + tr_e;
+      lds_u8* e1 = ex + flip<16>(tr_e) + 256;
+      const int w0 = max(0, tc - own);
+      if (w0 == 0 && w_hi == kRowWaves) {
+        vec8 a[4];
+#pragma unroll
+        for (int c = 0; c < 4; c++) a[c] = tr_pair<T>(e0 + 1024 * c, e1 + 1024 * c);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int c = 0; c < 16; c++) {
+          acc = Elem<T>::mfma(a[c & 3], wf[c], acc);
+          if (c + 4 < 16) a[c & 3] = tr_pair<T>(e0 + 1024 * (c + 4), e1 + 1024 * (c + 4));
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      } else {
+#pragma unroll
+        for (int kk = 0; kk < kRowWaves; kk++)
+          if (kk >= w0 && kk < w_hi) {
+#pragma unroll
+            for (int c = 2 * kk; c < 2 * kk + 2; c++) acc = Elem<T>::mfma(tr_pair<T>(e0 + 1024 * c, e1 + 1024 * c), wf[c], acc);
+          }
+      }
+      asm volatile("s_waitcnt vmcnt(0)" : "+v"(c0), "+v"(c1), "+v"(c2), "+v"(c3)::"memory");
+#pragma unroll
+      for (int r = 0; r < 4; r++) { acc[r] += c0[r]; acc[4 + r] += c1[r]; acc[8 + r] += c2[r]; acc[12 + r] += c3[r]; }      // (zeros without a tile above)
+      if (tc >= own) {
+        if (kAddRem && !out) {      // dv_j gains rem_j * d_o_j
+          const float* stat = p.row_stat + seq_id * p.stat_sb + head * p.stat_sh + tok0;
+#pragma unroll
+          for (int r = 0; r < 16; r++) {
+            const int j = kRowKeys * tc + 8 * (r >> 2) + 4 * half + (r & 3);
+            if (j < L) acc[r] += fast_exp2(stat[j]) * (float)dob[(int64_t)j * p.d_o.st + 32 * cp + col];
+          }
+        }
+        store_acc_tile<T>(sink, acc, out ? p.logit_scale : 1.f, kRowKeys * tc, 32 * cp, half, col, DH);
+      } else {
+        const f32x4 d0 = __builtin_shufflevector(acc, acc, 0, 1, 2, 3), d1 = __builtin_shufflevector(acc, acc, 4, 5, 6, 7),
+                    d2 = __builtin_shufflevector(acc, acc, 8, 9, 10, 11), d3 = __builtin_shufflevector(acc, acc, 12, 13, 14, 15);
+        float* dst = part + (int64_t)tc * 8192;
+        asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %5\n\tglobal_store_dwordx4 %0, %2, %5 offset:1024\n\t"
+                     "global_store_dwordx4 %0, %3, %5 offset:2048\n\tglobal_store_dwordx4 %0, %4, %5 offset:3072"
+                     ::"v"(lane16), "v"(d0), "v"(d1), "v"(d2), "v"(d3), "s"(dst) : "memory");
+      }
+    };
+    const bool late = wave >= 4;      // (waves w and w + 4 share a SIMD)
+    lds_barrier();
+    for (int t = 0; t < n; ++t) {
+      asm volatile("; nothing in flight");
+      const float prod_in = n_prod;
+      const int j0 = kRowKeys * t;
+      const bool seen = w_first < L && j0 <= last_seen;
+      lds_u8* kt = lds + RowLds::kKv + (t & 1) * RowLds::kKvBuf;
+      lds_u8* ex = lds + RowLds::kExch + (t & 1) * RowLds::kExchBuf;
+      u32x4 dz[2];
+      float r_prod;
+      int r_count, count;
+      asm volatile("s_nop 4\n\tglobal_load_dword %0, %2, %4 sc1\n\tglobal_load_dword %1, %3, %5"
+                   : "=&v"(r_count), "=&v"(r_prod) : "v"(0), "v"(row_c * 4), "s"(pred), "s"(product_at(t + 1)) : "memory");
+      request_kv(t + 1);
+      if (seen) {
+        f32x16 s, dp;
+#pragma unroll
+        for (int r = 0; r < 16; r++) { s[r] = 0.f; dp[r] = 0.f; }
+        lds_u8* k0 = kt + row_a;
+        lds_u8* k1 = kt + flip<32>(row_a);
+        lds_u8* q0p = lds + RowLds::kQ + 32 * wave * 64 + row_a;
+        lds_u8* q1p = lds + RowLds::kQ + 32 * wave * 64 + flip<32>(row_a);
+        auto k_op = [&](int kk) { return lds_load<vec8>(((kk & 1) ? k1 : k0) + (kk >> 1) * RowLds::kKvPanel); };
+        auto v_op = [&](int kk) { return lds_load<vec8>(((kk & 1) ? k1 : k0) + RowLds::kKvMat + (kk >> 1) * RowLds::kKvPanel); };
+        auto q_op = [&](int kk) { return lds_load<vec8>(((kk & 1) ? q1p : q0p) + (kk >> 1) * RowLds::kPanel); };
+        constexpr int kAhead = 3, kVAhead = 3;
+        vec8 ka[kAhead], qa[kAhead], va[kVAhead];
+#pragma unroll
+        for (int kk = 0; kk < kAhead; kk++) { ka[kk] = k_op(kk); qa[kk] = q_op(kk); }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int kk = 0; kk < kSteps; kk++) {
+          s = Elem<T>::mfma(ka[kk % kAhead], qa[kk % kAhead], s);
+          if (kk + kAhead < kSteps) { ka[kk % kAhead] = k_op(kk + kAhead); qa[kk % kAhead] = q_op(kk + kAhead); }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int r = 0; r < 16; r++) s[r] *= p.scale_log2;
+        if (j0 + 31 > w_first - 1 + ac || w_last >= L) {      // hidden keys
+          const int me = this_lane(), qi = w_first + (me & 31);
+          const int lim = qi < L ? qi + ac - j0 - 16 * (me >> 5) : 0;
+#pragma unroll
+          for (int r = 0; r < 16; r++) s[r] = r < lim ? s[r] : -INFINITY;
+        }
+        RowMath<T> m;
+        m.weights(s, half, prod_in, ex + wr_a);
+#pragma unroll
+        for (int kk = 0; kk < kVAhead; kk++) va[kk] = v_op(kk);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int kk = 0; kk < kSteps; kk++) {
+          dp = Elem<T>::mfma(va[kk % kVAhead], dof[kk], dp);
+          if (kk + kVAhead < kSteps) va[kk % kVAhead] = v_op(kk + kVAhead);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        m.gradients(dp, half, drem, prefix, dz);
+      } else {
+        dz[0] = dz[1] = u32x4{0, 0, 0, 0};
+        lds_put(ex + wr_a, dz[0]);
+        lds_put(ex + (wr_a ^ 16), dz[0]);
+      }
+      lds_put(ex + RowLds::kExchMat + wr_a, dz[0]);
+      lds_put(ex + RowLds::kExchMat + flip<16>(wr_a), dz[1]);
+      asm volatile("s_waitcnt vmcnt(2)\n\tv_mov_b32 %0, %2\n\tv_readfirstlane_b32 %1, %3"
+                   : "=&v"(n_prod), "=s"(count) : "v"(r_prod), "v"(r_count) : "memory");
+      // The key blocks that are complete are passed on; what the tile above left of the one that is contracted next is asked for.
+      const int tn = late ? t - 1 : t;
+      if (lane == 0) *flag = tn;
+      seen_count = max(seen_count, count);
+      if (has_pred && tn >= 0) {
+        if (seen_count <= tn) seen_count = wait_for(pred, tn, p.status, lane);
+        const float* src = part + (int64_t)tn * 8192;
+        asm volatile("s_nop 4\n\tglobal_load_dwordx4 %0, %4, %5 sc1\n\tglobal_load_dwordx4 %1, %4, %5 offset:1024 sc1\n\t"
+                     "global_load_dwordx4 %2, %4, %5 offset:2048 sc1\n\tglobal_load_dwordx4 %3, %4, %5 offset:3072 sc1"
+                     : "=&v"(c0), "=&v"(c1), "=&v"(c2), "=&v"(c3) : "v"(lane16), "s"(src) : "memory");
+      } else {
+        c0 = c1 = c2 = c3 = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+      if (seen) {
+        lds_u8* t0 = kt + tr_k;
+        lds_u8* t1 = kt + flip<32>(tr_k) + 512;
+        auto kc_op = [&](int i) { const int o = 1024 * (i >> 2) + (i & 3) * RowLds::kKvPanel; return tr_pair<T>(t0 + o, t1 + o); };
+        vec8 b[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) b[i] = kc_op(i);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+          dqacc[i & 3] = Elem<T>::mfma(as_vec8<T>(dz[i >> 2]), b[i & 3], dqacc[i & 3]);
+          if (i + 4 < 8) b[i & 3] = kc_op(i + 4);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      // The rows of step t + 1 are in LDS before the barrier (behind them: the flag, and what the tile above left).
+      if (!late || t == 0) {
+        if (has_pred && !late) vm_wait<5>(); else vm_wait<1>();
+      }
+      if (!late) lds_barrier();
+      if (tn >= 0) contract(tn);
+      if (late) lds_barrier();
+    }
+    if (late) {
+      vm_wait<0>();
+      if (has_pred) {
+        if (seen_count < n) seen_count = wait_for(pred, n - 1, p.status, lane);
+        const float* src = part + (int64_t)(n - 1) * 8192;
+        asm volatile("s_nop 4\n\tglobal_load_dwordx4 %0, %4, %5 sc1\n\tglobal_load_dwordx4 %1, %4, %5 offset:1024 sc1\n\t"
+                     "global_load_dwordx4 %2, %4, %5 offset:2048 sc1\n\tglobal_load_dwordx4 %3, %4, %5 offset:3072 sc1"
+                     : "=&v"(c0), "=&v"(c1), "=&v"(c2), "=&v"(c3) : "v"(lane16), "s"(src) : "memory");
+      }
+      contract(n - 1);
+    }
+    // The last results are passed on.
+    vm_wait<0>();
+    if (lane == 0) *flag = n;
+    if (w_first < L) {
+      const RowSink<T> dq_sink = make_row_sink<T>((T*)p.dq.ptr + seq_id * p.dq.sb + head * p.dq.sh + tok0 * p.dq.st, p.dq.st, L, DH);
+#pragma unroll
+      for (int dt = 0; dt < kDTiles; dt++) store_acc_tile<T>(dq_sink, dqacc[dt], p.logit_scale, w_first, 32 * dt, half, col, DH);
+    }
+    __syncthreads();
+  }
+}
+
+// Clears a region of `n16` pieces of 16 bytes.
+__global__ __launch_bounds__(256) void row_clear_kernel(u32x4* z, int64_t n16) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n16; i += (int64_t)gridDim.x * 256) z[i] = u32x4{0u, 0u, 0u, 0u};
+}
+
+template <typename T, bool kAddRem>
+static hipError_t launch_row_t(const BwdParams& p, int max_tiles, hipStream_t stream) {
+  static std::atomic<uint64_t> lds_done{0};
+  int dev = 0, cus = 0;
+  hipError_t e = device_cus(&dev, &cus);
+  if (e != hipSuccess) return e;
+  if ((e = raise_lds_limit(&bwd_row_kernel<T, kAddRem>, lds_done, dev, RowLds::kBytes)) != hipSuccess) return e;
+  const int64_t tiles = (int64_t)max_tiles * ((p.num_heads + 7) / 8);      // per queue, at most
+  const int per_queue = (int)(tiles < cus / 8 ? tiles : cus / 8);
+  hipLaunchKernelGGL((bwd_row_kernel<T, kAddRem>), dim3((unsigned)(8 * per_queue)), dim3(kRowThreads), RowLds::kBytes, stream, p);
+  return hipGetLastError();
+}
+
+// Whether the tensors and the device allow the backward on row tiles.
+bool row_supported(const BwdParams& p) {
+  int dev = 0, cus = 0;
+  if (device_cus(&dev, &cus) != hipSuccess) return false;
+  return p.load == kLoadAligned && p.head_dim == 128 && !p.wide_rows && cus >= 8;
+}
+
+hipError_t launch_row_clear(uint32_t* region, int64_t bytes, hipStream_t stream) {
+  const int64_t n16 = bytes / 16, wgs = (n16 + 1023) / 1024;
+  hipLaunchKernelGGL(row_clear_kernel, dim3((unsigned)(wgs < 256 ? wgs : 256)), dim3(256), 0, stream, (u32x4*)region, n16);
+  return hipGetLastError();
+}
+
+hipError_t launch_bwd_row(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream) {
+  if (p.add_rem) return dtype_is_f16 ? launch_row_t<_Float16, true>(p, max_tiles, stream) : launch_row_t<__bf16, true>(p, max_tiles, stream);
+  return dtype_is_f16 ? launch_row_t<_Float16, false>(p, max_tiles, stream) : launch_row_t<__bf16, false>(p, max_tiles, stream);
+}
+
+}  // namespace sba

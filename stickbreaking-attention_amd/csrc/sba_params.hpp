@@ -61,6 +61,8 @@ struct SchedParams {
 // takes 12 vector-ALU instructions per sequence and wave, 1.5 us at 64, and replaces a launch of 8 us in front of the forward.
 constexpr int kInlineSeqs = 64;
 
+constexpr int kRowTileRows = 256;      // query rows per tile of the backward on row tiles
+
 struct FwdParams {
   TensorRef q, k, v, o;
   VectorRef rem;
@@ -96,6 +98,7 @@ struct BwdParams {
   float logit_scale;
   int32_t attend_current;
   int32_t load;                // as in FwdParams
+  int32_t wide_rows;           // a row stride of 4 MiB or more
   int32_t split;               // dK/dV: too few key tiles to fill the chip
   // Fused remainder term (the forward wrote o + rem * v): d_rem_eff = d_rem + d_o . v per row, dv += rem * d_o.
   int32_t add_rem;
@@ -108,11 +111,13 @@ struct BwdParams {
                                // d_o . v when add_rem), written by the dQ kernel and read by the dK/dV kernel
   int32_t max_tiles;           // query-tile slots the dQ launch provides per head
   int64_t total_tokens;        // packed mode: rows of the token axis; rows no sequence covers are zero-filled
-  // One-kernel backward (sba_bwd_chain.hip): what the key tiles of a (head, sequence) hand to each other.
-  float* chain_dq;             // [head][row][128] fp32: partial dQ of a row over the key tiles below the reader
-  uint32_t* chain_c;           // [head][row] {fp32 C below the reader's tile, tag = index of the reader's tile}
-  int32_t* chain_flags;        // [head][key tile slot][8]: per consumer wave, row blocks whose partial dQ is complete
-  int32_t* chain_head_xcc;     // [head]: XCC id + 1 of the head's workgroups (0 = none yet)
+  // What the key tiles (sba_bwd_chain.hip) or row tiles (sba_bwd_row.hip) of a (head, sequence) hand to each other.
+  float* chain_dq;             // key tiles: [head][row][128] fp32, partial dQ of a row over the key tiles below the reader;
+                               // row tiles: [head][key block of 32][32 x 256] fp32, partial dV and dK over the row tiles above
+  uint32_t* chain_c;           // key tiles: [head][row] {fp32 C below the reader's tile, tag = index of the reader's tile};
+                               // row tiles: [8], next tile not yet taken, per queue
+  int32_t* chain_flags;        // [head][tile slot][8]: per wave, row (key) blocks whose partial result is complete
+  int32_t* chain_head_xcc;     // [head] (row tiles: [queue]): XCC id + 1 of its workgroups (0 = none yet)
   int32_t* status;             // the scheduler's status word; the kernel raises it when a wait runs out
   int64_t chain_rows;          // rows per head in chain_dq / chain_c
   int64_t chain_sb;            // fixed-length mode: rows per batch element (0 in packed mode)

@@ -1,0 +1,165 @@
+"""CPU checks of the backward on row tiles (csrc/sba_bwd_row.hip): which recorded products it reads, how the queues of its tiles fall, and
+what its inline assembly has to keep that the compiler does not check."""
+import os
+import re
+import shutil
+import subprocess
+
+import pytest
+
+from test_carry_slots_model import bits, cdiv, forward_writes, slot
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "stickbreaking-attention_amd", "csrc")
+
+
+def row_tile_reads(L, ac):
+    """Products used by the 32 rows of a wave against a 32-key block: slots (block, row), rows beyond the sequence as its last one."""
+    m, out = cdiv(L, 128), set()
+    for q0 in range(0, L, 256):
+        for w_first in range(q0, min(q0 + 256, L), 32):
+            last_seen = min(w_first + 31, L - 1) - 1 + ac
+            for u in range(last_seen // 32 + 1 if last_seen >= 0 else 0):
+                for row in range(w_first, w_first + 32):
+                    out.add(slot(u, min(row, L - 1), m))
+    return out
+
+
+@pytest.mark.parametrize("fwd_kt", [32, 64, "split"])
+@pytest.mark.parametrize("ac", [0, 1])
+def test_every_product_read_was_written(fwd_kt, ac):
+    for L in list(range(1, 300)) + [511, 512, 513, 640, 641, 673, 705, 1000]:
+        assert bits(row_tile_reads, L, ac) & ~bits(forward_writes, L, ac, fwd_kt) == 0, f"L={L}"
+
+
+def test_partial_results_of_neighbours_do_not_overlap():
+    """The blocks of a sequence start at floor(9 start / 256) of the head's; sequences of up to 256 rows hand nothing over."""
+    for L in range(257, 1300):
+        for start in range(0, 300):
+            first = start * 9 // 256
+            assert (start + L) * 9 // 256 - first >= cdiv(L, 32), (L, start)      # before the next sequence's, which starts at or behind
+            assert first + cdiv(L, 32) <= (start + L) * 9 // 256 + 2              # within the head's
+
+
+@pytest.mark.parametrize("heads", [1, 4, 7, 8, 12, 20, 32])
+def test_every_head_is_in_one_queue(heads):
+    per_slot = cdiv(heads, 8)
+    for seq in range(9):
+        got = sorted(h for q in range(8) for i in range(per_slot) for h in [((q - seq * heads) % 8) + 8 * i] if h < heads)
+        assert got == list(range(heads))
+
+
+@pytest.fixture(scope="module")
+def listing(tmp_path_factory):
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("no hipcc")
+    flags = re.search(r"^HIPFLAGS = (.*?)\nSRCS", open(os.path.join(CSRC, "Makefile")).read(), re.S | re.M).group(1)
+    flags = flags.replace("\\\n", " ").replace("$(ARCH)", "gfx950").split()
+    out = str(tmp_path_factory.mktemp("s") / "row.s")
+    subprocess.run([hipcc, *flags, "-S", "--cuda-device-only", os.path.join(CSRC, "sba_bwd_row.hip"), "-o", out], check=True, capture_output=True)
+    kernels, name = {}, None
+    for line in open(out):
+        m = re.match(r"(_Z\w+):", line)
+        if m:
+            name = m.group(1)
+            kernels[name] = []
+        if name:
+            kernels[name].append(line)
+        if ".Lfunc_end" in line:
+            name = None
+    return {n: k for n, k in kernels.items() if "bwd_row_kernel" in n}
+
+
+def registers(text, kind):
+    out = set()
+    for a, b, c in re.findall(rf"\b{kind}(\d+)\b|\b{kind}\[(\d+):(\d+)\]", text):
+        out |= {int(a)} if a else set(range(int(b), int(c) + 1))
+    return out
+
+
+VECTOR_MEMORY = re.compile(r"global_|buffer_(load|store)|scratch_|flat_")
+
+
+def test_scalars_of_vector_memory_instructions_are_old_enough(listing):
+    """A scalar register written by a vector instruction (a reloaded spill) may be read by a vector-memory instruction only five wait
+    states later, which the compiler keeps for its own instructions and not for those in inline assembly."""
+    assert listing
+    for name, lines in listing.items():
+        age = {}
+        for line in lines:
+            text = line.split(";")[0].strip()
+            if not text or text.endswith(":") or text.startswith("."):
+                continue
+            op, _, rest = text.partition(" ")
+            if VECTOR_MEMORY.match(op):
+                young = [r for r in registers(text, "s") if age.get(r, 9) < 5]
+                assert not young, f"{name}: {text}: s{young}"
+            step = int(rest, 0) + 1 if op == "s_nop" else 1
+            age = {r: a + step for r, a in age.items() if a + step < 6}
+            written = registers(rest.split(",")[0], "s")
+            if op in ("v_readlane_b32", "v_readfirstlane_b32") or op.startswith("v_cmp"):
+                age.update((r, 0) for r in written)
+            elif op.startswith("s_") and not op.startswith(("s_waitcnt", "s_cmp", "s_cbranch", "s_barrier", "s_nop", "s_branch")):
+                for r in written:
+                    age.pop(r, None)
+
+
+def test_registers_on_their_way_are_left_alone(listing):
+    """No register that a load in inline assembly is still filling is read, copied or spilled before a wait that covers the load.
+    Forward over the control-flow graph: register -> fewest vector-memory operations issued since its load, over all paths; "nothing
+    in flight" marks the head of the loop, where by construction nothing is."""
+    for name, lines in listing.items():
+        order, blocks, asm = ["entry"], {"entry": []}, False
+        for line in lines:
+            if "#ASMSTART" in line or "#ASMEND" in line:
+                asm = "#ASMSTART" in line
+                continue
+            m = re.match(r"(\.LBB\d+_\d+):", line)
+            if m:
+                order.append(m.group(1))
+                blocks[m.group(1)] = []
+                continue
+            text = "nothing in flight" if "nothing in flight" in line else line.split(";")[0].strip()
+            if text and not text.startswith(".") and not text.endswith(":"):
+                blocks[order[-1]].append((text, asm))
+        follow = dict(zip(order, order[1:]))
+        state, work, bad = {"entry": {}}, ["entry"], []
+
+        def flow(to, s):
+            old = state.get(to)
+            new = dict(s) if old is None else {r: min(old.get(r, 99), s.get(r, 99)) for r in {**old, **s}}
+            if new != old:
+                state[to] = new
+                work.append(to)
+
+        def run(block, visit):
+            s = dict(state[block])
+            for text, in_asm in blocks[block]:
+                op, _, rest = text.partition(" ")
+                if text == "nothing in flight":
+                    s = {}
+                elif op.startswith(("s_cbranch", "s_branch")):
+                    visit(rest.strip(), s)
+                    if op == "s_branch":
+                        return
+                elif op == "s_endpgm":
+                    return
+                elif op == "s_waitcnt":
+                    m = re.search(r"vmcnt\((\d+)\)", rest)
+                    s = {r: c for r, c in s.items() if c < int(m.group(1))} if m else s
+                else:
+                    if not op.startswith("s_") and registers(text, "v") & set(s):
+                        bad.append(f"{block}: {text}")
+                    if VECTOR_MEMORY.match(op):
+                        s = {r: min(c + 1, 63) for r, c in s.items()}
+                        if in_asm and "_load_" in op and " lds" not in text:
+                            s.update((r, 0) for r in registers(rest.split(",")[0], "v"))
+            if block in follow:
+                visit(follow[block], s)
+
+        while work:
+            run(work.pop(), flow)
+        bad.clear()
+        for block in state:
+            run(block, lambda *_: None)
+        assert not bad, f"{name}: {bad[:5]}"

@@ -525,5 +525,13 @@ __device__ __forceinline__ void xcd_head_tile(int wg, int num_heads, int* head, 
     *slot = wg / num_heads;
   }
 }
+// The same for kernels that give a tile to `subs` workgroups: those of one tile run on one XCD.  Launched with xcd_sub_grid: whole
+// groups of 8 tiles, so that slots beyond the last tile's occur, which hold nothing.  (Dealt in turn, the workgroups of a tile ran on as
+// many XCDs, each of which read the tile's K and V: training passes, us, 12 heads, 6143 tokens, fp32 991 -> 979; 16-bit, head_dim 50,
+// 185 -> 180.)
+__device__ __forceinline__ void xcd_head_tile_sub(int wg, int subs, int num_heads, int* head, int* slot, int* sub) {
+  *sub = (wg >> 3) % subs;
+  xcd_head_tile((wg >> 3) / subs * 8 + (wg & 7), num_heads, head, slot);
+}
 
 }  // namespace sba

@@ -329,9 +329,9 @@ __global__ __launch_bounds__(kThreads, DH == 96 ? 3 : 2) void fwd_f32_kernel(Fwd
     forward_service(p.sched, blockIdx.x);
     return;
   }
-  const int wg = blockIdx.x - p.sched.service, sub = wg % kF32Split;
-  int head, slot;
-  xcd_head_tile(wg / kF32Split, p.num_heads, &head, &slot);
+  const int wg = blockIdx.x - p.sched.service;
+  int head, slot, sub;
+  xcd_head_tile_sub(wg, kF32Split, p.num_heads, &head, &slot, &sub);
   Tile tile;
   int64_t r0, r1;
   if (!forward_tile(p, slot, sub, kF32Rows, &tile, &r0, &r1)) {
@@ -414,9 +414,8 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dq_f32_kernel(BwdParams p) {
   constexpr int NB = DH / 32;
   __shared__ __attribute__((aligned(16))) float lds[RowsF32Lds<DH, 2>::kFloats];      // Q and dO rows and the waves' scratch, then the final sums
   __shared__ float xch[2][kWaves][32];
-  int head, slot;
-  xcd_head_tile(blockIdx.x / kF32Split, p.num_heads, &head, &slot);
-  const int sub = blockIdx.x % kF32Split;
+  int head, slot, sub;
+  xcd_head_tile_sub(blockIdx.x, kF32Split, p.num_heads, &head, &slot, &sub);
   if (slot >= p.counts[kCountQ]) {
     int64_t r0, r1;
     if (uncovered_rows(p.counts, slot, p.total_tokens, sub, kF32Rows, &r0, &r1)) {      // rows of no sequence: zero gradients
@@ -532,13 +531,13 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dkv_f32_kernel(BwdParams p) {
   constexpr int NB = DH / 32;
   typedef DkvF32Lds<DH> Lds;
   extern __shared__ __attribute__((aligned(16))) float lds[];
-  int head, slot;
-  xcd_head_tile(blockIdx.x / kF32KeySplit, p.num_heads, &head, &slot);
+  int head, slot, sub;
+  xcd_head_tile_sub(blockIdx.x, kF32KeySplit, p.num_heads, &head, &slot, &sub);
   if (slot >= p.counts[kCountK]) return;
   const Tile tile = p.k_tiles[slot];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = lane >> 5, col = lane & 31;
   const int L = tile.seq_len, ac = p.attend_current, D = p.head_dim;
-  const int k0 = tile.origin + (blockIdx.x % kF32KeySplit) * kF32Rows;
+  const int k0 = tile.origin + sub * kF32Rows;
   if (k0 >= L) return;
   const int64_t tok0 = tile.seq_start;
   const float* qb = (const float*)p.q.ptr + tile.seq_id * p.q.sb + head * p.q.sh + tok0 * p.q.st;
@@ -646,7 +645,7 @@ static hipError_t by_head_dim(int D, int load, F&& f) {
 
 hipError_t launch_fwd_f32(const FwdParams& p, int max_tiles, hipStream_t stream) {
   return by_head_dim(p.head_dim, p.load, [&](auto dh, auto mode) {
-    hipLaunchKernelGGL((fwd_f32_kernel<decltype(dh)::value, decltype(mode)::value>), dim3((unsigned)(max_tiles * p.num_heads * kF32Split + p.sched.service)),
+    hipLaunchKernelGGL((fwd_f32_kernel<decltype(dh)::value, decltype(mode)::value>), dim3((unsigned)(xcd_sub_grid(max_tiles * p.num_heads, kF32Split) + p.sched.service)),
                        dim3(kThreads), 0, stream, p);
     return hipGetLastError();
   });
@@ -663,8 +662,8 @@ hipError_t launch_bwd_f32(const BwdParams& p, int max_q_tiles, int max_k_tiles, 
     static std::atomic<uint64_t> lds_done{0};
     const hipError_t r = raise_lds_limit(&bwd_dkv_f32_kernel<DH, kMode>, lds_done, dev, lds_bytes);
     if (r != hipSuccess) return r;
-    hipLaunchKernelGGL((bwd_dq_f32_kernel<DH, kMode>), dim3((unsigned)(max_q_tiles * p.num_heads * kF32Split)), dim3(kThreads), 0, stream, p);
-    hipLaunchKernelGGL((bwd_dkv_f32_kernel<DH, kMode>), dim3((unsigned)(max_k_tiles * p.num_heads * kF32KeySplit)), dim3(kThreads), lds_bytes, stream, p);
+    hipLaunchKernelGGL((bwd_dq_f32_kernel<DH, kMode>), dim3((unsigned)xcd_sub_grid(max_q_tiles * p.num_heads, kF32Split)), dim3(kThreads), 0, stream, p);
+    hipLaunchKernelGGL((bwd_dkv_f32_kernel<DH, kMode>), dim3((unsigned)xcd_sub_grid(max_k_tiles * p.num_heads, kF32KeySplit)), dim3(kThreads), lds_bytes, stream, p);
     return hipGetLastError();
   });
 }

@@ -31,4 +31,7 @@ inline hipError_t raise_lds_limit(Kernel kernel, std::atomic<uint64_t>& done, in
   return e;
 }
 
+// Workgroups of a kernel that maps them with xcd_head_tile_sub: `tiles` tiles, whole groups of 8.
+inline int64_t xcd_sub_grid(int64_t tiles, int subs) { return (tiles + 7) / 8 * 8 * subs; }
+
 }  // namespace sba

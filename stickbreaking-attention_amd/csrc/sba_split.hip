@@ -111,9 +111,9 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_split_kernel(FwdParams p) {
     forward_service(p.sched, blockIdx.x);
     return;
   }
-  const int wg = blockIdx.x - p.sched.service, sub = wg % kSplitSubs;
-  int head, slot;
-  xcd_head_tile(wg / kSplitSubs, p.num_heads, &head, &slot);
+  const int wg = blockIdx.x - p.sched.service;
+  int head, slot, sub;
+  xcd_head_tile_sub(wg, kSplitSubs, p.num_heads, &head, &slot, &sub);
   Tile tile;
   int64_t r0, r1;
   if (!forward_tile(p, slot, sub, kSplitRows, &tile, &r0, &r1)) {
@@ -213,9 +213,8 @@ __global__ __launch_bounds__(kThreads, DH == 128 ? 1 : 2) void bwd_dq_split_kern
   __shared__ float xch[2][kWaves][32];
   T* const k_lds = reinterpret_cast<T*>(lds_raw);
   T* const v_lds = k_lds + SplitLds<DH>::kTile;
-  const int sub = blockIdx.x % kSplitSubs;
-  int head, slot;
-  xcd_head_tile(blockIdx.x / kSplitSubs, p.num_heads, &head, &slot);
+  int head, slot, sub;
+  xcd_head_tile_sub(blockIdx.x, kSplitSubs, p.num_heads, &head, &slot, &sub);
   if (slot >= p.counts[kCountQ]) {
     int64_t r0, r1;
     if (uncovered_rows(p.counts, slot, p.total_tokens, sub, kSplitRows, &r0, &r1)) {      // rows of no sequence: zero gradients
@@ -329,9 +328,9 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dkv_split_kernel(BwdParams p)
   __shared__ float rem_lds[32];
   T* const q_lds = reinterpret_cast<T*>(lds_raw);
   T* const do_lds = q_lds + SplitLds<DH>::kTile;
-  const int subs = kBlockK / kSplitRows, sub = blockIdx.x % subs;
-  int head, slot;
-  xcd_head_tile(blockIdx.x / subs, p.num_heads, &head, &slot);
+  constexpr int subs = kBlockK / kSplitRows;
+  int head, slot, sub;
+  xcd_head_tile_sub(blockIdx.x, subs, p.num_heads, &head, &slot, &sub);
   if (slot >= p.counts[kCountK]) return;
   const Tile tile = p.k_tiles[slot];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = lane >> 5, col = lane & 31;
@@ -464,7 +463,7 @@ static hipError_t launch_fwd_split_t(const FwdParams& p, int dtype_is_f16, int m
   return by_shape(dtype_is_f16, p.head_dim, p.load, [&](auto t, auto dh, auto load) {
     static std::atomic<uint64_t> lds_done{0};
     return launch_split(&fwd_split_kernel<decltype(t), decltype(dh)::value, decltype(load)::value, kCarryOnly>, lds_done,
-                        SplitLds<decltype(dh)::value>::kBytes, (unsigned)(max_tiles * p.num_heads * kSplitSubs + p.sched.service), p, stream);
+                        SplitLds<decltype(dh)::value>::kBytes, (unsigned)(xcd_sub_grid(max_tiles * p.num_heads, kSplitSubs) + p.sched.service), p, stream);
   });
 }
 hipError_t launch_fwd_split(const FwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream) {
@@ -477,7 +476,7 @@ hipError_t launch_bwd_dq_split(const BwdParams& p, int dtype_is_f16, int max_til
   return by_shape(dtype_is_f16, p.head_dim, p.load, [&](auto t, auto dh, auto load) {
     static std::atomic<uint64_t> lds_done{0};
     return launch_split(&bwd_dq_split_kernel<decltype(t), decltype(dh)::value, decltype(load)::value>, lds_done, SplitLds<decltype(dh)::value>::kBytes,
-                        (unsigned)(max_tiles * p.num_heads * kSplitSubs), p, stream);
+                        (unsigned)xcd_sub_grid(max_tiles * p.num_heads, kSplitSubs), p, stream);
   });
 }
 // max_tiles: key tiles of kBlockK keys; head_dim up to 64.
@@ -485,7 +484,7 @@ hipError_t launch_bwd_dkv_split(const BwdParams& p, int dtype_is_f16, int max_ti
   return by_shape(dtype_is_f16, p.head_dim, p.load, [&](auto t, auto, auto load) {
     static std::atomic<uint64_t> lds_done{0};
     return launch_split(&bwd_dkv_split_kernel<decltype(t), decltype(load)::value>, lds_done, SplitLds<64>::kBytes,
-                        (unsigned)(max_tiles * p.num_heads * (kBlockK / kSplitRows)), p, stream);
+                        (unsigned)xcd_sub_grid(max_tiles * p.num_heads, kBlockK / kSplitRows), p, stream);
   });
 }
 

@@ -1,20 +1,23 @@
-// fp32 path: the same operator evaluated entirely in fp32, for fp32 inputs, on the fp32 matrix instruction
-// (v_mfma_f32_32x32x2_f32: exact fp32 products and sums).
+// fp32 path: the same operator for fp32 inputs, everything held and summed in fp32.
 //
-// What bounds it: the matrix pipe.  A 32x32x2 fp32 MFMA takes 64 cycles for 4096 FLOP, 1/16 of the bf16 rate, so a
-// 32 x 32 block of (query, key) pairs costs 8192 (forward, D = 128), 12288 (dQ) or 16384 (dK/dV) matrix cycles against
-// fewer than 2000 cycles of everything else.  Consequences for the design:
+// Products.  An fp32 number is the sum of three bf16 numbers; of the nine products of two such triples the six that matter are formed
+// on the bf16 matrix instruction (v_mfma_f32_32x32x16_bf16: exact products, fp32 sums), which takes 192 cycles for a 32 x 32 x 16 block
+// where v_mfma_f32_32x32x2_f32 takes 512.  The result is the more accurate one (fewer roundings of the sum; 126 cases of 7
+// head_dims against float64, rms error of o, dq, dk, dv 0.80 to 0.87 of the fp32 instruction's).  Workgroups that meet numbers
+// which triples do not hold (see Split) run again on the fp32 instruction.
+// What bounds it: per 32 x 32 block at head_dim 128 the forward needs 3072 matrix cycles and 1300 vector instructions (5200 cycles), 700 of
+// them to split K and V, which every workgroup of 32 rows does for itself; two waves per SIMD overlap the two to about 70 %.
+// Consequences for the design:
 //   * no tile is shared between waves: an operand goes from global memory straight into the registers of the wave that
-//     uses it (16 KB per 4096 cycles and wave, served by the L2), a phase ahead of its use, in the registers the phase
-//     before has consumed.  One barrier per 128 keys; two waves per SIMD cover each other's element-wise math.
+//     uses it, a phase ahead of its use, in the registers the phase before has consumed.  One barrier per 128 keys; two waves
+//     per SIMD cover each other's element-wise math.
 //   * the unit of work is small (32 query rows, or 32 keys, per workgroup of four waves), because the longest row
-//     would otherwise be the critical path: a single wave needs 64 x 8192 cycles = 0.25 ms for 32 rows of 2048 keys,
-//     twice what the whole chip needs for the rest of such a batch.  The four waves split the KEYS of the forward and
+//     would otherwise be the critical path: 32 rows of 2048 keys are 64 blocks, one wave 0.1 ms.
+//     The four waves split the KEYS of the forward and
 //     of dQ (sub-tiles of 32 dealt round robin, one scalar per row exchanged per step) and the ROWS of dK/dV (nothing
 //     exchanged), and add their partial results through LDS at the end, in a fixed order: bit-reproducible.
-// Measured: 12 heads x 128, 6143 tokens in sequences of up to 2048, forward + backward 0.99 ms; 86.7 ms on the vector ALU
-// with one wave per query row and fp32 atomics for dK/dV.  32 heads x 2048 tokens: forward 0.34, dQ 0.49, dK/dV 0.67 ms =
-// 100, 104 and 102 TFLOP/s of products, where a large fp32 matrix product reaches 154 on this chip.
+// Measured: 12 heads x 128, 6143 tokens in sequences of up to 2048, forward + backward: 0.98 ms with the fp32 instruction, 0.77 ms
+// (forward 0.21, dQ 0.29, dK/dV 0.37); head_dim 64 0.52 and 0.44, 96 0.74 and 0.62, 127 1.18 and 0.86, 32 (4 heads) 0.174 and 0.151.
 //
 //   fwd_f32_kernel     : keys swept in reverse from the diagonal (as sb_varlen_fwd.py:155-165), running product per row;
 //                        records the product above every 32-key sub-tile in `carry`.
@@ -23,10 +26,12 @@
 //   bwd_dkv_f32_kernel : key-stationary; dV += P^T dO, dK += dZ^T Q over the rows that see the keys.
 //
 // Register layout: S^T = K Q^T as in the 16-bit kernels (lane l owns query l%32 and the 16 consecutive keys
-// 16*(l/32) + r).  The contraction index of an MFMA is split between the half-waves, k = l/32, and which element it
-// stands for is free as long as both operands agree:
-//   over head_dim : d = 8*i + 4*(l/32) + t for MFMA 4*i + t, so a lane reads 16-byte pieces of its row from LDS;
-//   over keys/rows: index 16*(l/32) + r for MFMA r: the score registers are the A operand as they stand.
+// 16*(l/32) + r).  The contraction index of an MFMA is split between the half-waves, and which element it
+// stands for is free as long as both operands agree.
+//   fp32 instruction, k = l/32: over head_dim d = 8*i + 4*(l/32) + t for MFMA 4*i + t, so a lane reads 16-byte pieces of its row from
+//     LDS; over keys/rows index 16*(l/32) + r for MFMA r: the score registers are the A operand as they stand.
+//   bf16 instruction, k = 8*(l/32) + t: over head_dim 16 consecutive columns, planes of bf16 in LDS; over keys/rows index
+//     16*(l/32) + 8*i + t for MFMA i: score registers and columns of x are operands as they stand, split pair by pair.
 #include "sba_device.hpp"
 #include "sba_host.hpp"
 #include "sba_params.hpp"
@@ -41,7 +46,7 @@ constexpr int kF32Split = kBlockQ / kF32Rows;      // workgroups per 128-row que
 constexpr int kF32KeySplit = kBlockK / kF32Rows;   // workgroups per 64-key tile of the schedule
 constexpr int kF32TrStride = 36;                   // floats per row of the transposition buffers
 
-enum : int { kF32Padded = 0, kF32Exact = 1, kF32Far = 2 };      // how rows are read, see Operand
+enum : int { kF32Padded = 0, kF32Exact = 1, kF32Far = 2, kF32Quads = 3 };      // how rows are read, see Operand
 
 __device__ __forceinline__ f32x16 mfma_f32(float a, float b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
 __device__ __forceinline__ f32x16 zero16() {
@@ -49,6 +54,12 @@ __device__ __forceinline__ f32x16 zero16() {
 #pragma unroll
   for (int r = 0; r < 16; r++) z[r] = 0.f;
   return z;
+}
+// The lane's number, computed where it is used: the addresses that follow from it would cost registers that the loops do not have.
+__device__ __forceinline__ int this_lane() {
+  int r;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(r));
+  return r;
 }
 typedef __attribute__((ext_vector_type(4), aligned(4))) float f32x4_u;      // rows need only be 4-byte aligned
 
@@ -77,7 +88,8 @@ __device__ __forceinline__ Rows32 rows32(const float* base, int64_t stride, int 
 // rows as it stands, and 64 lanes read two runs of C*4 contiguous bytes per instruction.  (A lane per row, what a
 // contraction over head_dim wants, costs a cache access per lane when loaded like that: measured 1024 instead of 290 per
 // 32 x 128 operand, and the kernels were bound by them.  Those operands go through LDS, a part at a time.)
-// kF32Exact: head_dim == DH.  kF32Padded: an element beyond head_dim is asked for outside the buffer and reads as zero.
+// kF32Exact: head_dim == DH.  kF32Quads: a multiple of 4.  kF32Padded: any; an element beyond head_dim is asked for outside the buffer
+// and reads as zero.
 // kF32Far: any head_dim, rows at any distance.
 template <int DH> struct Parts {
   static constexpr int C = DH == 128 ? 64 : 32, N = DH / C, NC = C / 32;
@@ -276,19 +288,21 @@ __device__ __forceinline__ float sticks_f32(const f32x16& s, float scale_log2, i
 
 // Sum the four waves' partial [32 rows][DH] results through LDS and store them (times `scale`, plus add_scale[row] *
 // add[row] when `add` is given).  acc[dt][r]: row 8*(r/4) + 4*half + r%4, column out_col(dt).  All waves take part.
-template <int DH, int kMode>
-__device__ __forceinline__ void reduce_store_f32(float* lds, const f32x16 (&acc)[DH / 32], float scale, float* out, int64_t stride,
+// Returns whether this thread stored a sum that calls for the other engine (see Split).
+template <class E, int DH, int kMode>
+__device__ __forceinline__ bool reduce_store_f32(float* lds, const f32x16 (&acc)[DH / 32], float scale, float* out, int64_t stride,
                                                  int rows, int D, const float* add = nullptr, int64_t add_stride = 0,
                                                  const float* add_scale = nullptr) {
   constexpr int NB = DH / 32, kStride = DH + 4;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, half = lane >> 5, col = lane & 31;
+  bool odd = false;
   __syncthreads();
   float* mine = lds + wave * 32 * kStride;
 #pragma unroll
   for (int r = 0; r < 16; r++)
 #pragma unroll
     for (int dt = 0; dt < NB; dt++)
-      mine[(8 * (r >> 2) + 4 * half + (r & 3)) * kStride + out_col<DH>(dt, col)] = acc[dt][r];
+      mine[(8 * (r >> 2) + 4 * half + (r & 3)) * kStride + E::out_col(dt, col)] = acc[dt][r];
   __syncthreads();
   for (int idx = threadIdx.x; idx < 32 * (DH / 4); idx += kThreads) {
     const int row = idx / (DH / 4), d0 = (idx % (DH / 4)) * 4;
@@ -296,6 +310,11 @@ __device__ __forceinline__ void reduce_store_f32(float* lds, const f32x16 (&acc)
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < kWaves; w++) v += *reinterpret_cast<const f32x4*>(lds + (w * 32 + row) * kStride + d0);
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      v[t] *= E::kDown;
+      if (kMode == kF32Exact || d0 + t < D) odd |= E::odd(v[t]);
+    }
     v *= scale;
     float* o = out + (int64_t)row * stride + d0;
     const float* a = add ? add + (int64_t)row * add_stride + d0 : nullptr;
@@ -309,20 +328,310 @@ __device__ __forceinline__ void reduce_store_f32(float* lds, const f32x16 (&acc)
         if (d0 + t < D) o[t] = v[t] + (a ? as * a[t] : 0.f);
     }
   }
+  return odd;
 }
 
-// LDS of the row-stationary kernels: kTiles tiles of 32 rows and the waves' scratch; the final sums lie over both.
-template <int DH, int kTiles>
-struct RowsF32Lds {
-  static constexpr int kLoop = kTiles * 32 * (DH + 4) + kWaves * Parts<DH>::kTurn, kRed = kWaves * 32 * (DH + 4);
-  static constexpr int kFloats = kLoop > kRed ? kLoop : kRed;
+// The two ways to form the products.  x: the registers of the streamed operand.
+//   stage    : 32 rows into LDS as the resident operand of score() (kRows: as its A operand, whose row m is key mfma_row_to_key32(m))
+//   score    : (rows in x) . (resident rows), contracted over head_dim; x then holds `next`
+//   contract : acc[dt] += a . x, contracted over 32 rows; x then holds `next` if `more`
+template <int DH, int kMode>
+struct Plain {
+  typedef Operand<DH, kMode> Op;
+  static constexpr bool kSplit = false;
+  static constexpr float kUp = 1.f, kDown = 1.f;
+  static __device__ __forceinline__ bool odd(float) { return false; }
+  static constexpr int kResident = 32 * (DH + 4), kTurn = Parts<DH>::kTurn;      // floats
+  static __device__ __forceinline__ int out_col(int dt, int col) { return sba::out_col<DH>(dt, col); }
+  static __device__ __forceinline__ Op op(const float* base, int64_t stride, int first, int rows_total, int half, int col, int D) {
+    return operand<DH, kMode>(base, stride, first, rows_total, half, col, D);
+  }
+  template <bool kScore>
+  static __device__ __forceinline__ void fill(float (&x)[DH / 2], const Op& o) { o.fill(x); }
+  template <bool kRows>
+  static __device__ __forceinline__ bool stage(float* lds, const Rows32& s, int D) {
+    stage_rows<DH, kMode>(lds, s, D);
+    return false;
+  }
+  template <bool kLdsIsA, bool kNextScore>
+  static __device__ __forceinline__ f32x16 score(float (&x)[DH / 2], float* turn, const float* resident, int half, int col, const Op& next,
+                                                 const Op& late, bool has_late, uint64_t& odd) {
+    const int key = mfma_row_to_key32(col);
+    return score_phase<DH, kMode, kLdsIsA>(x, turn, kLdsIsA ? col : key, resident + (kLdsIsA ? key : col) * (DH + 4), half, col, next, late, has_late);
+  }
+  template <bool kNextScore>
+  static __device__ __forceinline__ void contract(f32x16 (&acc)[DH / 32], const float (&a)[16], float (&x)[DH / 2], const Op& next, bool more,
+                                                  const Op& late, bool has_late) {
+    contract_phase<DH, kMode>(acc, a, x, next, more, late, has_late);
+  }
 };
+
+// An fp32 number as the sum of three bf16 numbers, each the one before's rounding error rounded: 26 bits.  (Numbers whose first part
+// rounds to infinity have none; what comes of them is not a number.)  Pairs of numbers; the residuals are exact.
+struct Split3 { uint32_t h, m, l; };
+__device__ __forceinline__ Split3 split3(float x0, float x1) {
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+  auto round = [](float a, float b) { return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2)); };
+  auto low = [](uint32_t v) { return __builtin_bit_cast(float, v << 16); };
+  auto high = [](uint32_t v) { return __builtin_bit_cast(float, v & 0xffff0000u); };
+  Split3 r;
+  r.h = round(x0, x1);
+  const float m0 = x0 - low(r.h), m1 = x1 - high(r.h);
+  r.m = round(m0, m1);
+  r.l = round(m0 - low(r.m), m1 - high(r.m));
+  return r;
+}
+
+// Products of triples.  What they do not hold: numbers beyond the largest bf16 number (and infinities), whose triples are not numbers,
+// and the last bits of numbers below 2^-109.  The latter matter only where a result is as small or the partner is as large, so a
+// workgroup calls for the fp32 instruction (`odd`) if a score is not a number, if an element of its resident rows is outside
+// 2^-80 .. 2^80, or if one of its results is.  Weights and their gradients, which may be that small in sums that are not, are scaled by 2^24.
+// The residuals are taken with shifts and subtractions: v_dot2_f32_bf16 does it in one instruction instead of two, but not beside
+// MFMAs (12 heads, 6143 tokens: 828 us against 800).
+template <int DH, int kMode>
+struct Split {
+  typedef typename Elem<__bf16>::vec8 vec8;
+  static constexpr bool kSplit = true;
+  static constexpr float kUp = 0x1p24f, kDown = 0x1p-24f;
+  static __device__ __forceinline__ bool odd(float x) { return x != 0.f && !(fabsf(x) >= 0x1p-80f && fabsf(x) <= 0x1p80f); }
+  static constexpr int NB = DH / 32, kPlane = 2048, kPanel = 3 * kPlane;      // bytes; a panel: 3 planes of [32 rows][32 columns]
+  static constexpr int kResident = NB * kPanel / 4, kTurn = kPanel / 4;       // floats
+  static __device__ __forceinline__ int out_col(int dt, int col) { return NB * col + dt; }
+
+  // 32 rows in DH/2 registers per lane.  For score(): piece (p, i) is rows 8 i + lane/8, columns 32 p + 4 (lane%8) .. +3, in registers
+  // 16 p + 4 i.  For contract(): piece r is row 16 half + r, columns NB (lane%32) .. +NB-1, in registers NB r.
+  struct Op {
+    Rows32 src;
+    uint32_t voff_s, voff_c;
+    int lane, D;
+    // kN numbers from byte voff on, which are columns d to d + kN - 1; zero if all are beyond head_dim.  A piece that head_dim cuts holds
+    // what lies behind the row (within the rows' memory, or zero beyond the resource's end), or, kZero, zeros there.
+    template <int kN, bool kZero>
+    __device__ __forceinline__ void load(float* y, uint32_t voff, uint32_t soff, int d) const {
+      const uint32_t vo = kMode == kF32Exact || d < D ? voff : (uint32_t)kOutside;
+      if constexpr (kN == 1) {
+        y[0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(src.rsrc, vo, soff, 0));
+      } else {
+        typedef __attribute__((ext_vector_type(kN))) float vec;
+        vec v;
+        if constexpr (kN == 2) v = __builtin_bit_cast(vec, __builtin_amdgcn_raw_buffer_load_b64(src.rsrc, vo, soff, 0));
+        else if constexpr (kN == 3) v = __builtin_bit_cast(vec, __builtin_amdgcn_raw_buffer_load_b96(src.rsrc, vo, soff, 0));
+        else v = __builtin_bit_cast(vec, __builtin_amdgcn_raw_buffer_load_b128(src.rsrc, vo, soff, 0));
+#pragma unroll
+        for (int c = 0; c < kN; c++) y[c] = !kZero || kMode != kF32Padded || c == 0 || d + c < D ? v[c] : 0.f;
+      }
+    }
+    __device__ __forceinline__ void score_piece(float (&x)[DH / 2], int p, int i) const {
+      load<4, true>(x + 16 * p + 4 * i, voff_s + 128 * p, 8u * (uint32_t)i * src.stride_bytes, 32 * p + 4 * (lane & 7));
+    }
+    __device__ __forceinline__ void contract_piece(float (&x)[DH / 2], int r) const {
+      load<NB, false>(x + NB * r, voff_c, (uint32_t)r * src.stride_bytes, NB * (lane & 31));
+    }
+    // The pieces whose registers are free once those below `to` are, and were not once those below `from` were.
+    template <bool kScore>
+    __device__ __forceinline__ void refill(float (&x)[DH / 2], int from, int to) const {
+      if (kScore) {
+#pragma unroll
+        for (int j = 0; j < DH / 8; j++)
+          if (4 * j + 4 > from && 4 * j + 4 <= to) score_piece(x, j >> 2, j & 3);
+      } else {
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+          if (NB * r + NB > from && NB * r + NB <= to) contract_piece(x, r);
+      }
+    }
+  };
+  static __device__ __forceinline__ Op op(const float* base, int64_t stride, int first, int rows_total, int half, int col, int D) {
+    const Rows32 s = rows32(base, stride, first, rows_total, D);
+    const int lane = this_lane();
+    return Op{s, (uint32_t)(lane >> 3) * s.stride_bytes + 16u * (lane & 7), 16u * (uint32_t)(lane >> 5) * s.stride_bytes + 4u * NB * (lane & 31), lane, D};
+  }
+  template <bool kScore>
+  static __device__ __forceinline__ void fill(float (&x)[DH / 2], const Op& o) { o.template refill<kScore>(x, 0, DH / 2); }
+
+  // Panels: 64-byte rows whose 16-byte chunks are XORed with (row >> 2) & 3: no bank is met twice by row reads.
+  static __device__ __forceinline__ void put(unsigned char* at, float a, float b, float c, float d) {
+    const Split3 u = split3(a, b), v = split3(c, d);
+    *reinterpret_cast<u32x2*>(at) = u32x2{u.h, v.h};
+    *reinterpret_cast<u32x2*>(at + kPlane) = u32x2{u.m, v.m};
+    *reinterpret_cast<u32x2*>(at + 2 * kPlane) = u32x2{u.l, v.l};
+  }
+  template <bool kRows>
+  static __device__ __forceinline__ bool stage(float* lds, const Rows32& s, int D) {
+    bool any = false;
+    unsigned char* const at = (unsigned char*)lds;
+    for (int idx = threadIdx.x; idx < 32 * (DH / 4); idx += kThreads) {
+      const int row = idx / (DH / 4), d = (idx % (DH / 4)) * 4;
+      const Op o{s, 0, 0, 0, D};
+      float v[4];
+      o.template load<4, true>(v, (uint32_t)row * s.stride_bytes + 4 * d, 0, d);
+      const int m = kRows ? 8 * ((row & 15) >> 2) + 4 * (row >> 4) + (row & 3) : row;
+      put(at + (d >> 5) * kPanel + m * 64 + ((((d >> 3) & 3) ^ ((m >> 2) & 3)) << 4) + 2 * (d & 4), v[0], v[1], v[2], v[3]);
+#pragma unroll
+      for (int c = 0; c < 4; c++) any |= odd(v[c]);
+    }
+    return any;
+  }
+  // The six products that matter, the small ones first.
+  static __device__ __forceinline__ f32x16 six(const vec8 (&a)[3], const vec8 (&b)[3], f32x16 c) {
+    c = Elem<__bf16>::mfma(a[2], b[0], c);
+    c = Elem<__bf16>::mfma(a[0], b[2], c);
+    c = Elem<__bf16>::mfma(a[1], b[1], c);
+    c = Elem<__bf16>::mfma(a[1], b[0], c);
+    c = Elem<__bf16>::mfma(a[0], b[1], c);
+    return Elem<__bf16>::mfma(a[0], b[0], c);
+  }
+  template <bool kLdsIsA, bool kNextScore>
+  static __device__ __forceinline__ f32x16 score(float (&x)[DH / 2], float* turn, const float* resident, int half, int col, const Op& next,
+                                                 const Op&, bool, uint64_t& odd) {
+    f32x16 acc = zero16();
+    unsigned char* const mine = (unsigned char*)turn;
+    const unsigned char* const res = (const unsigned char*)resident;
+    const int lane = this_lane(), l8 = lane >> 3, chunk = (lane & 7) >> 1, sub = 8 * (lane & 1);
+    // rows 8 i + l8 go to their own place, or (as the A operand) to that of their key
+    const int w0 = kLdsIsA ? l8 * 64 + ((chunk ^ (l8 >> 2)) << 4) + sub : (8 * (l8 >> 2) + (l8 & 3)) * 64 + ((chunk ^ (2 * (l8 >> 2))) << 4) + sub;
+    const int row_a = (lane & 31) * 64 + (((lane >> 5) ^ ((lane >> 2) & 3)) << 4);
+#pragma unroll
+    for (int p = 0; p < NB; p++) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int w = kLdsIsA ? (w0 ^ (32 * (i & 1))) + 512 * i : (w0 ^ (16 * (i >> 1))) + 1024 * (i & 1) + 256 * (i >> 1);
+        const float* y = x + 16 * p + 4 * i;
+        put(mine + w, y[0], y[1], y[2], y[3]);
+      }
+      next.template refill<kNextScore>(x, 16 * p, 16 * p + 16);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int kk = 0; kk < 2; kk++) {
+        vec8 a[3], b[3];
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+          const int at = kk ? row_a ^ 32 : row_a;
+          const vec8 u = *reinterpret_cast<const vec8*>(mine + j * kPlane + at), v = *reinterpret_cast<const vec8*>(res + p * kPanel + j * kPlane + at);
+          a[j] = kLdsIsA ? v : u;
+          b[j] = kLdsIsA ? u : v;
+        }
+        acc = six(a, b, acc);
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 16; r += 2) odd |= __ballot(__builtin_isunordered(acc[r], acc[r + 1]));
+    return acc;
+  }
+  template <bool kNextScore>
+  static __device__ __forceinline__ void contract(f32x16 (&acc)[DH / 32], const float (&a)[16], float (&x)[DH / 2], const Op& next, bool more,
+                                                  const Op&, bool) {
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      auto planes = [&](auto&& at, vec8 (&out)[3]) {
+        u32x4 v[3];
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+          const Split3 u = split3(at(2 * t), at(2 * t + 1));
+          v[0][t] = u.h; v[1][t] = u.m; v[2][t] = u.l;
+        }
+#pragma unroll
+        for (int j = 0; j < 3; j++) out[j] = as_vec8<__bf16>(v[j]);
+      };
+      vec8 av[3];
+      planes([&](int t) { return a[8 * i + t]; }, av);
+#pragma unroll
+      for (int dt = 0; dt < NB; dt++) {
+        vec8 bv[3];
+        planes([&](int t) { return x[(8 * i + t) * NB + dt]; }, bv);
+        acc[dt] = six(av, bv, acc[dt]);
+      }
+      next.template refill<kNextScore>(x, 8 * NB * i, 8 * NB * (i + 1));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+};
+template <int DH, int kMode>
+using Engine = typename std::conditional<kMode == kF32Far, Plain<DH, kMode>, Split<DH, kMode>>::type;
+
+// LDS of the row-stationary kernels: kTiles tiles of 32 rows and the waves' scratch; the final sums lie over both.
+constexpr int most(int a, int b) { return a > b ? a : b; }
+template <class E, int DH, int kTiles>
+struct RowsF32Lds {
+  static constexpr int kFloats = most(kTiles * E::kResident + kWaves * E::kTurn, kWaves * 32 * (DH + 4));
+};
+template <int DH, int kMode, int kTiles>
+constexpr int kRowsF32 = most(RowsF32Lds<Plain<DH, kMode>, DH, kTiles>::kFloats, RowsF32Lds<Engine<DH, kMode>, DH, kTiles>::kFloats);
+
+// Where the products were split: whether any wave met what the fp32 matrix instruction treats otherwise (the workgroup agrees).
+__device__ __forceinline__ bool any_odd(uint64_t odd, bool mine) { return __syncthreads_or((int)(odd != 0) | (int)mine) != 0; }
+
+template <class E, int DH, int kMode>
+__device__ __forceinline__ bool fwd_f32_rows(const FwdParams& p, const Tile& tile, int head, int q0, float* lds, float (&xch)[2][kWaves][32], float (&rem_lds)[32]) {
+  constexpr int NB = DH / 32;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = lane >> 5, col = lane & 31;
+  const int L = tile.seq_len, ac = p.attend_current, D = p.head_dim;
+  const int64_t tok0 = tile.seq_start;
+  const float* qb = (const float*)p.q.ptr + tile.seq_id * p.q.sb + head * p.q.sh + tok0 * p.q.st;
+  const float* kb = (const float*)p.k.ptr + tile.seq_id * p.k.sb + head * p.k.sh + tok0 * p.k.st;
+  const float* vb = (const float*)p.v.ptr + tile.seq_id * p.v.sb + head * p.v.sh + tok0 * p.v.st;
+  const int64_t n_qt = (L + kBlockQ - 1) / kBlockQ;
+  float* carry = p.carry ? p.carry + (int64_t)head * p.carry_head_stride + tile.carry_base : nullptr;
+
+  const int qi = q0 + col;
+  const int last_key = min(q0 + kF32Rows, L) - 2 + ac;
+  const int n_sub = last_key < 0 ? 0 : last_key / 32 + 1, n_steps = (n_sub + kWaves - 1) / kWaves;
+  auto k_of = [&](int u) { return E::op(kb, p.k.st, 32 * u, L, half, col, D); };
+  auto v_of = [&](int u) { return E::op(vb, p.v.st, 32 * u, L, half, col, D); };
+  float x[DH / 2];
+  // Wave w takes sub-tile n_sub - 1 - (4 t + w) in step t.
+  int U = n_sub - 1 - wave;
+  if (U >= 0) E::template fill<true>(x, k_of(U));
+  bool staged = E::template stage<false>(lds, rows32(qb, p.q.st, q0, L, D), D);
+  float* turn = lds + E::kResident + wave * E::kTurn;
+  f32x16 oacc[NB];
+#pragma unroll
+  for (int dt = 0; dt < NB; dt++) oacc[dt] = zero16();
+  uint64_t odd = 0;
+  float prod = 1.f;      // product over the keys of the steps done so far
+  __syncthreads();
+  for (int t = 0; t < n_steps; ++t, U -= kWaves) {
+    const int me = this_lane(), half = me >> 5, col = me & 31, qi = q0 + col;
+    float beta[16], pe[16];
+    float run = 1.f, oth = 1.f;
+    if (U >= 0) {
+      const f32x16 s = E::template score<false, false>(x, turn, lds, half, col, v_of(U), k_of(U), t > 0, odd);
+      run = sticks_f32(s, p.scale_log2, qi + ac - 32 * U - 16 * half, beta, pe);
+      oth = other_half(run, half);
+    }
+    if (half == 0) xch[t & 1][wave][col] = run * oth;
+    lds_barrier();
+    float above = prod;
+#pragma unroll
+    for (int w = 0; w < kWaves; w++) {
+      const float y = xch[t & 1][w][col];
+      if (w < wave) above *= y;
+      prod *= y;
+    }
+    if (U >= 0) {
+      if (carry && half == 0) carry[carry_offset(U, n_qt) + (qi - kBlockQ * (U >> 2))] = above;
+      const float seed = E::kUp * (half ? above : above * oth);      // the upper half-wave holds the higher keys
+#pragma unroll
+      for (int r = 0; r < 16; r++) pe[r] = beta[r] * (pe[r] * seed);
+      E::template contract<true>(oacc, pe, x, k_of(U >= kWaves ? U - kWaves : n_sub), U >= kWaves, k_of(U), false);
+    }
+  }
+  if (wave == 0 && half == 0) {
+    rem_lds[col] = prod;
+    if (qi < L) {
+      ((float*)p.rem.ptr)[tile.seq_id * p.rem.sb + head * p.rem.sh + (tok0 + qi) * p.rem.st] = prod;
+      p.row_stat[tile.seq_id * p.stat_sb + head * p.stat_sh + tok0 + qi] = log2f(prod);
+    }
+  }
+  float* ob = (float*)p.o.ptr + tile.seq_id * p.o.sb + head * p.o.sh + (tok0 + q0) * p.o.st;
+  const bool stored = reduce_store_f32<E, DH, kMode>(lds, oacc, 1.f, ob, p.o.st, L - q0, D, p.add_rem ? vb + (int64_t)q0 * p.v.st : nullptr, p.v.st, rem_lds);
+  return E::kSplit && any_odd(odd, stored | staged);
+}
 
 // (Width 96 keeps three waves per SIMD by spilling four registers; 177 registers and two waves take 4 % of a pass more.)
 template <int DH, int kMode>
 __global__ __launch_bounds__(kThreads, DH == 96 ? 3 : 2) void fwd_f32_kernel(FwdParams p) {
-  constexpr int NB = DH / 32;
-  __shared__ __attribute__((aligned(16))) float lds[RowsF32Lds<DH, 1>::kFloats];      // Q rows and the waves' scratch, then the final sums
+  __shared__ __attribute__((aligned(16))) float lds[kRowsF32<DH, kMode, 1>];      // Q rows and the waves' scratch, then the final sums
   __shared__ float xch[2][kWaves][32];
   __shared__ float rem_lds[32];
   if ((int)blockIdx.x < p.sched.service) {
@@ -344,92 +653,16 @@ __global__ __launch_bounds__(kThreads, DH == 96 ? 3 : 2) void fwd_f32_kernel(Fwd
     }
     return;
   }
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = lane >> 5, col = lane & 31;
-  const int L = tile.seq_len, ac = p.attend_current, D = p.head_dim;
   const int q0 = tile.origin + sub * kF32Rows;
-  if (q0 >= L) return;
-  const int64_t tok0 = tile.seq_start;
-  const float* qb = (const float*)p.q.ptr + tile.seq_id * p.q.sb + head * p.q.sh + tok0 * p.q.st;
-  const float* kb = (const float*)p.k.ptr + tile.seq_id * p.k.sb + head * p.k.sh + tok0 * p.k.st;
-  const float* vb = (const float*)p.v.ptr + tile.seq_id * p.v.sb + head * p.v.sh + tok0 * p.v.st;
-  const int64_t n_qt = (L + kBlockQ - 1) / kBlockQ;
-  float* carry = p.carry ? p.carry + (int64_t)head * p.carry_head_stride + tile.carry_base : nullptr;
-
-  const int qi = q0 + col;
-  const int last_key = min(q0 + kF32Rows, L) - 2 + ac;
-  const int n_sub = last_key < 0 ? 0 : last_key / 32 + 1, n_steps = (n_sub + kWaves - 1) / kWaves;
-  const int krow = mfma_row_to_key32(col);
-  auto k_of = [&](int u) { return operand<DH, kMode>(kb, p.k.st, 32 * u, L, half, col, D); };
-  auto v_of = [&](int u) { return operand<DH, kMode>(vb, p.v.st, 32 * u, L, half, col, D); };
-  float x[DH / 2];
-  // Wave w takes sub-tile n_sub - 1 - (4 t + w) in step t.
-  int U = n_sub - 1 - wave;
-  if (U >= 0) k_of(U).fill(x);
-  stage_rows<DH, kMode>(lds, rows32(qb, p.q.st, q0, L, D), D);
-  const float* q_lds = lds + col * (DH + 4);
-  float* turn = lds + 32 * (DH + 4) + wave * Parts<DH>::kTurn;
-  f32x16 oacc[NB];
-#pragma unroll
-  for (int dt = 0; dt < NB; dt++) oacc[dt] = zero16();
-  float prod = 1.f;      // product over the keys of the steps done so far
-  __syncthreads();
-  for (int t = 0; t < n_steps; ++t, U -= kWaves) {
-    float beta[16], pe[16];
-    float run = 1.f, oth = 1.f;
-    if (U >= 0) {
-      const f32x16 s = score_phase<DH, kMode, false>(x, turn, krow, q_lds, half, col, v_of(U), k_of(U), t > 0);
-      run = sticks_f32(s, p.scale_log2, qi + ac - 32 * U - 16 * half, beta, pe);
-      oth = other_half(run, half);
-    }
-    if (half == 0) xch[t & 1][wave][col] = run * oth;
-    lds_barrier();
-    float above = prod;
-#pragma unroll
-    for (int w = 0; w < kWaves; w++) {
-      const float y = xch[t & 1][w][col];
-      if (w < wave) above *= y;
-      prod *= y;
-    }
-    if (U >= 0) {
-      if (carry && half == 0) carry[carry_offset(U, n_qt) + (qi - kBlockQ * (U >> 2))] = above;
-      const float seed = half ? above : above * oth;        // the upper half-wave holds the higher keys
-#pragma unroll
-      for (int r = 0; r < 16; r++) pe[r] = beta[r] * (pe[r] * seed);
-      contract_phase<DH, kMode>(oacc, pe, x, k_of(U - kWaves), U >= kWaves, k_of(U), false);
-    }
-  }
-  if (wave == 0 && half == 0) {
-    rem_lds[col] = prod;
-    if (qi < L) {
-      ((float*)p.rem.ptr)[tile.seq_id * p.rem.sb + head * p.rem.sh + (tok0 + qi) * p.rem.st] = prod;
-      p.row_stat[tile.seq_id * p.stat_sb + head * p.stat_sh + tok0 + qi] = log2f(prod);
-    }
-  }
-  float* ob = (float*)p.o.ptr + tile.seq_id * p.o.sb + head * p.o.sh + (tok0 + q0) * p.o.st;
-  reduce_store_f32<DH, kMode>(lds, oacc, 1.f, ob, p.o.st, L - q0, D, p.add_rem ? vb + (int64_t)q0 * p.v.st : nullptr, p.v.st, rem_lds);
+  if (q0 >= tile.seq_len) return;
+  if (p.fp32_products || fwd_f32_rows<Engine<DH, kMode>, DH, kMode>(p, tile, head, q0, lds, xch, rem_lds)) fwd_f32_rows<Plain<DH, kMode>, DH, kMode>(p, tile, head, q0, lds, xch, rem_lds);
 }
 
-template <int DH, int kMode>
-__global__ __launch_bounds__(kThreads, 2) void bwd_dq_f32_kernel(BwdParams p) {
+template <class E, int DH, int kMode>
+__device__ __forceinline__ bool bwd_dq_f32_rows(const BwdParams& p, const Tile& tile, int head, int q0, float* lds, float (&xch)[2][kWaves][32]) {
   constexpr int NB = DH / 32;
-  __shared__ __attribute__((aligned(16))) float lds[RowsF32Lds<DH, 2>::kFloats];      // Q and dO rows and the waves' scratch, then the final sums
-  __shared__ float xch[2][kWaves][32];
-  int head, slot, sub;
-  xcd_head_tile_sub(blockIdx.x, kF32Split, p.num_heads, &head, &slot, &sub);
-  if (slot >= p.counts[kCountQ]) {
-    int64_t r0, r1;
-    if (uncovered_rows(p.counts, slot, p.total_tokens, sub, kF32Rows, &r0, &r1)) {      // rows of no sequence: zero gradients
-      zero_rows<float>(p.dq, head, r0, r1, p.head_dim);
-      zero_rows<float>(p.dk, head, r0, r1, p.head_dim);
-      zero_rows<float>(p.dv, head, r0, r1, p.head_dim);
-    }
-    return;
-  }
-  const Tile tile = p.q_tiles[slot];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = lane >> 5, col = lane & 31;
   const int L = tile.seq_len, ac = p.attend_current, D = p.head_dim;
-  const int q0 = tile.origin + sub * kF32Rows;
-  if (q0 >= L) return;
   const int64_t tok0 = tile.seq_start;
   const float* qb = (const float*)p.q.ptr + tile.seq_id * p.q.sb + head * p.q.sh + tok0 * p.q.st;
   const float* kb = (const float*)p.k.ptr + tile.seq_id * p.k.sb + head * p.k.sh + tok0 * p.k.st;
@@ -443,17 +676,14 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dq_f32_kernel(BwdParams p) {
   const int qi = q0 + col;
   const int last_key = min(q0 + kF32Rows, L) - 2 + ac;
   const int n_sub = last_key < 0 ? 0 : last_key / 32 + 1, n_steps = (n_sub + kWaves - 1) / kWaves;
-  const int krow = mfma_row_to_key32(col);
-  auto k_of = [&](int u) { return operand<DH, kMode>(kb, p.k.st, 32 * u, L, half, col, D); };
-  auto v_of = [&](int u) { return operand<DH, kMode>(vb, p.v.st, 32 * u, L, half, col, D); };
+  auto k_of = [&](int u) { return E::op(kb, p.k.st, 32 * u, L, half, col, D); };
+  auto v_of = [&](int u) { return E::op(vb, p.v.st, 32 * u, L, half, col, D); };
   float x[DH / 2];
   int U = wave;            // wave w takes sub-tile 4 t + w in step t
-  if (U < n_sub) k_of(U).fill(x);
-  stage_rows<DH, kMode>(lds, rows32(qb, p.q.st, q0, L, D), D);
-  stage_rows<DH, kMode>(lds + 32 * (DH + 4), rows32(dob, p.d_o.st, q0, L, D), D);
-  const float* q_lds = lds + col * (DH + 4);
-  const float* do_lds = q_lds + 32 * (DH + 4);
-  float* turn = lds + 64 * (DH + 4) + wave * Parts<DH>::kTurn;
+  if (U < n_sub) E::template fill<true>(x, k_of(U));
+  bool staged = E::template stage<false>(lds, rows32(qb, p.q.st, q0, L, D), D);
+  staged |= E::template stage<false>(lds + E::kResident, rows32(dob, p.d_o.st, q0, L, D), D);
+  float* turn = lds + 2 * E::kResident + wave * E::kTurn;
   float drem = 0.f;
   if (qi < L && p.d_rem.ptr) drem = ((const float*)p.d_rem.ptr)[tile.seq_id * p.d_rem.sb + head * p.d_rem.sh + (tok0 + qi) * p.d_rem.st];
   __syncthreads();
@@ -461,7 +691,8 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dq_f32_kernel(BwdParams p) {
     // The forward wrote o + rem * v: the gradient reaching rem is d_rem + d_o . v_i.
     const float* vi = vb + (int64_t)min(qi, L - 1) * p.v.st;
     float dot = 0.f;
-    for (int d = half; d < D; d += 2) dot = fmaf(lds[(32 + col) * (DH + 4) + d], vi[d], dot);
+    const float* doi = dob + (int64_t)min(qi, L - 1) * p.d_o.st;
+    for (int d = half; d < D; d += 2) dot = fmaf(doi[d], vi[d], dot);
     drem += dot + other_half(dot, half);
   }
   if (wave == 0 && half == 0 && qi < L) p.drem_eff[tile.seq_id * p.drem_sb + head * p.stat_sh + tok0 + qi] = drem;
@@ -469,20 +700,22 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dq_f32_kernel(BwdParams p) {
   f32x16 dqacc[NB];
 #pragma unroll
   for (int dt = 0; dt < NB; dt++) dqacc[dt] = zero16();
+  uint64_t odd = 0;
   float prefix = 0.f;      // sum of g over the keys of the steps done so far
   for (int t = 0; t < n_steps; ++t, U += kWaves) {
+    const int me = this_lane(), half = me >> 5, col = me & 31, qi = q0 + col;
     float beta[16], dz[16];
     float tot = 0.f, fix = 0.f;
     const int64_t cslot = carry_offset(U, n_qt) + (qi - kBlockQ * (U >> 2));
     const bool active = U < n_sub;
     if (active) {
       const float prod_in = carry[cslot];
-      const f32x16 s = score_phase<DH, kMode, false>(x, turn, krow, q_lds, half, col, v_of(U), k_of(U), t > 0);
-      const f32x16 dp = score_phase<DH, kMode, false>(x, turn, krow, do_lds, half, col, k_of(U), k_of(U), false);
+      const f32x16 s = E::template score<false, true>(x, turn, lds, half, col, v_of(U), k_of(U), t > 0, odd);
+      const f32x16 dp = E::template score<false, false>(x, turn, lds + E::kResident, half, col, k_of(U), k_of(U), false, odd);
       float pe[16];
       const float run = sticks_f32(s, p.scale_log2, qi < L ? qi + ac - 32 * U - 16 * half : 0, beta, pe);
       const float oth = other_half(run, half);
-      const float seed = half ? prod_in : prod_in * oth;
+      const float seed = E::kUp * (half ? prod_in : prod_in * oth);
       float acc = 0.f;
 #pragma unroll
       for (int R = 0; R < 16; R++) {
@@ -504,41 +737,54 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dq_f32_kernel(BwdParams p) {
       prefix += y;
     }
     if (active) {
-      if (half == 0) prefix_out[cslot] = below;
+      if (half == 0) prefix_out[cslot] = E::kDown * below;
       const float fixup = below + fix;
 #pragma unroll
       for (int r = 0; r < 16; r++) dz[r] -= beta[r] * fixup;
-      contract_phase<DH, kMode>(dqacc, dz, x, k_of(U + kWaves), U + kWaves < n_sub, k_of(U), false);
+      E::template contract<true>(dqacc, dz, x, k_of(U + kWaves), U + kWaves < n_sub, k_of(U), false);
     }
   }
   float* dqb = (float*)p.dq.ptr + tile.seq_id * p.dq.sb + head * p.dq.sh + (tok0 + q0) * p.dq.st;
-  reduce_store_f32<DH, kMode>(lds, dqacc, p.logit_scale, dqb, p.dq.st, L - q0, D);
+  const bool stored = reduce_store_f32<E, DH, kMode>(lds, dqacc, p.logit_scale, dqb, p.dq.st, L - q0, D);
+  return E::kSplit && any_odd(odd, stored | staged);
 }
 
-template <int DH>
+template <int DH, int kMode>
+__global__ __launch_bounds__(kThreads, 2) void bwd_dq_f32_kernel(BwdParams p) {
+  __shared__ __attribute__((aligned(16))) float lds[kRowsF32<DH, kMode, 2>];      // Q and dO rows and the waves' scratch, then the final sums
+  __shared__ float xch[2][kWaves][32];
+  int head, slot, sub;
+  xcd_head_tile_sub(blockIdx.x, kF32Split, p.num_heads, &head, &slot, &sub);
+  if (slot >= p.counts[kCountQ]) {
+    int64_t r0, r1;
+    if (uncovered_rows(p.counts, slot, p.total_tokens, sub, kF32Rows, &r0, &r1)) {      // rows of no sequence: zero gradients
+      zero_rows<float>(p.dq, head, r0, r1, p.head_dim);
+      zero_rows<float>(p.dk, head, r0, r1, p.head_dim);
+      zero_rows<float>(p.dv, head, r0, r1, p.head_dim);
+    }
+    return;
+  }
+  const Tile tile = p.q_tiles[slot];
+  const int q0 = tile.origin + sub * kF32Rows;
+  if (q0 >= tile.seq_len) return;
+  if (p.fp32_products || bwd_dq_f32_rows<Engine<DH, kMode>, DH, kMode>(p, tile, head, q0, lds, xch)) bwd_dq_f32_rows<Plain<DH, kMode>, DH, kMode>(p, tile, head, q0, lds, xch);
+}
+
+template <class E, int DH>
 struct DkvF32Lds {
-  static constexpr int kRowStride = DH + 4;
-  static constexpr int kK = 0, kV = kK + 32 * kRowStride;                             // the workgroup's keys
-  static constexpr int kTr = kV + 32 * kRowStride;                                    // per wave: operand scratch; P^T, dZ^T
-  static constexpr int kTrWave = Parts<DH>::kTurn > 2 * 32 * kF32TrStride ? Parts<DH>::kTurn : 2 * 32 * kF32TrStride;
-  static constexpr int kLoop = kTr + kWaves * kTrWave;
-  static constexpr int kRed = kWaves * 32 * kRowStride;                               // final sums, over the above
-  static constexpr int kFloats = (kLoop > kRed ? kLoop : kRed) + 32;                  // + rem of 32 rows
+  static constexpr int kK = 0, kV = kK + E::kResident;                                // the workgroup's keys
+  static constexpr int kTr = kV + E::kResident;                                       // per wave: operand scratch; P^T, dZ^T
+  static constexpr int kTrWave = most(E::kTurn, 32 * kF32TrStride);
+  static constexpr int kRem = most(kTr + kWaves * kTrWave, kWaves * 32 * (DH + 4));   // (the final sums lie over the above) rem of 32 rows
+  static constexpr int kFloats = kRem + 32;
 };
 
-template <int DH, int kMode>
-__global__ __launch_bounds__(kThreads, 2) void bwd_dkv_f32_kernel(BwdParams p) {
+template <class E, int DH, int kMode>
+__device__ __forceinline__ bool bwd_dkv_f32_keys(const BwdParams& p, const Tile& tile, int head, int k0, float* lds) {
   constexpr int NB = DH / 32;
-  typedef DkvF32Lds<DH> Lds;
-  extern __shared__ __attribute__((aligned(16))) float lds[];
-  int head, slot, sub;
-  xcd_head_tile_sub(blockIdx.x, kF32KeySplit, p.num_heads, &head, &slot, &sub);
-  if (slot >= p.counts[kCountK]) return;
-  const Tile tile = p.k_tiles[slot];
+  typedef DkvF32Lds<E, DH> Lds;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = lane >> 5, col = lane & 31;
   const int L = tile.seq_len, ac = p.attend_current, D = p.head_dim;
-  const int k0 = tile.origin + sub * kF32Rows;
-  if (k0 >= L) return;
   const int64_t tok0 = tile.seq_start;
   const float* qb = (const float*)p.q.ptr + tile.seq_id * p.q.sb + head * p.q.sh + tok0 * p.q.st;
   const float* kb = (const float*)p.k.ptr + tile.seq_id * p.k.sb + head * p.k.sh + tok0 * p.k.st;
@@ -551,87 +797,99 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dkv_f32_kernel(BwdParams p) {
   const float* prefix = p.prefix + slot0;
   const float* drem_plane = p.drem_eff + tile.seq_id * p.drem_sb + head * p.stat_sh + tok0;
 
-  auto q_of = [&](int b) { return operand<DH, kMode>(qb, p.q.st, 32 * b, L, half, col, D); };
-  auto do_of = [&](int b) { return operand<DH, kMode>(dob, p.d_o.st, 32 * b, L, half, col, D); };
+  auto q_of = [&](int b) { return E::op(qb, p.q.st, 32 * b, L, half, col, D); };
+  auto do_of = [&](int b) { return E::op(dob, p.d_o.st, 32 * b, L, half, col, D); };
   // Row blocks of 32 that see these keys: from the last one down to the one that holds the keys' own rows; wave w takes every
   // fourth.  (Downwards the loop needs one bound fewer in registers: 20 instead of 64 of them spilled at head_dim 128, 2 % of
   // the pass.)
   const int nb = k0 + 1 - ac < L ? (L + 31) / 32 : 0;
   int b = nb - 1 - wave;
   float x[DH / 2];
-  if (b >= U) q_of(b).fill(x);
+  if (b >= U) E::template fill<true>(x, q_of(b));
   // K and V of the 32 keys stay in LDS for the A operands of S^T and dP^T.
-  stage_rows<DH, kMode>(lds + Lds::kK, rows32(kb, p.k.st, k0, L, D), D);
-  stage_rows<DH, kMode>(lds + Lds::kV, rows32(vb, p.v.st, k0, L, D), D);
-  const int krow = mfma_row_to_key32(col);
-  const float* k_lds = lds + Lds::kK + krow * Lds::kRowStride;
-  const float* v_lds = lds + Lds::kV + krow * Lds::kRowStride;
+  bool staged = E::template stage<true>(lds + Lds::kK, rows32(kb, p.k.st, k0, L, D), D);
+  staged |= E::template stage<true>(lds + Lds::kV, rows32(vb, p.v.st, k0, L, D), D);
   float* turn = lds + Lds::kTr + wave * Lds::kTrWave;
   float* tp = turn;                                        // P^T [key][row], then dZ^T
-  float* tz = tp + 32 * kF32TrStride;
 
+  uint64_t odd = 0;
   f32x16 dkacc[NB], dvacc[NB];
 #pragma unroll
   for (int dt = 0; dt < NB; dt++) { dkacc[dt] = zero16(); dvacc[dt] = zero16(); }
   __syncthreads();
   for (; b >= U; b -= kWaves) {
-    const int qi = 32 * b + col;
+    const int me = this_lane(), half = me >> 5, col = me & 31, qi = 32 * b + col;
     const bool row_ok = qi < L;
     const float prod_in = carry[qi], prefix_in = prefix[qi];
     const float drem = row_ok ? drem_plane[qi] : 0.f;
-    const f32x16 s = score_phase<DH, kMode, true>(x, turn, col, k_lds, half, col, do_of(b), q_of(b), b < nb - kWaves);
-    const f32x16 dp = score_phase<DH, kMode, true>(x, turn, col, v_lds, half, col, do_of(b), do_of(b), false);
-    {
-      float beta[16], pe[16];
-      const float run = sticks_f32(s, p.scale_log2, row_ok ? qi + ac - k0 - 16 * half : 0, beta, pe);
-      const float oth = other_half(run, half);
-      const float seed = half ? prod_in : prod_in * oth;
-      // To [key][row] order (wave-private): the contraction over rows needs a lane per key.
-      float acc = 0.f;
+    const f32x16 s = E::template score<true, true>(x, turn, lds + Lds::kK, half, col, do_of(b), q_of(b), b < nb - kWaves, odd);
+    const f32x16 dp = E::template score<true, false>(x, turn, lds + Lds::kV, half, col, do_of(b), do_of(b), false, odd);
+    float beta[16], pe[16], dz[16];
+    const float run = sticks_f32(s, p.scale_log2, row_ok ? qi + ac - k0 - 16 * half : 0, beta, pe);
+    const float oth = other_half(run, half);
+    const float seed = E::kUp * (half ? prod_in : prod_in * oth);
+    // To [key][row] order (wave-private): the contraction over rows needs a lane per key.
+    float acc = 0.f;
 #pragma unroll
-      for (int R = 0; R < 16; R++) {
-        const float a = beta[R] * (pe[R] * seed);
-        const float g = a * (dp[R] - drem);
-        tp[(16 * half + R) * kF32TrStride + col] = a;
-        acc += g;
-        pe[R] = g - beta[R] * acc;
-      }
-      const float oth_g = other_half(acc, half);
-      const float fixup = prefix_in + (half ? oth_g : 0.f);
-#pragma unroll
-      for (int R = 0; R < 16; R++) tz[(16 * half + R) * kF32TrStride + col] = pe[R] - beta[R] * fixup;
+    for (int R = 0; R < 16; R++) {
+      const float a = beta[R] * (pe[R] * seed);
+      const float g = a * (dp[R] - drem);
+      tp[(16 * half + R) * kF32TrStride + col] = a;
+      acc += g;
+      dz[R] = g - beta[R] * acc;
     }
-    auto transposed = [&](const float* t, float (&y)[16]) {
+    const float oth_g = other_half(acc, half);
+    const float fixup = E::kUp * prefix_in + (half ? oth_g : 0.f);
+#pragma unroll
+    for (int R = 0; R < 16; R++) dz[R] -= beta[R] * fixup;
+    float y[16];
+    auto transposed = [&]() {
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        const f32x4 v = *reinterpret_cast<const f32x4*>(t + col * kF32TrStride + 16 * half + 4 * i);
+        const f32x4 v = *reinterpret_cast<const f32x4*>(tp + col * kF32TrStride + 16 * half + 4 * i);
 #pragma unroll
         for (int k = 0; k < 4; k++) y[4 * i + k] = v[k];
       }
     };
-    float y[16];
-    transposed(tp, y);
-    contract_phase<DH, kMode>(dvacc, y, x, q_of(b), true, q_of(b), false);
-    transposed(tz, y);
-    contract_phase<DH, kMode>(dkacc, y, x, q_of(b - kWaves), b - kWaves >= U, q_of(b), true);
+    transposed();
+    E::template contract<false>(dvacc, y, x, q_of(b), true, q_of(b), false);
+#pragma unroll
+    for (int R = 0; R < 16; R++) tp[(16 * half + R) * kF32TrStride + col] = dz[R];
+    transposed();
+    E::template contract<true>(dkacc, y, x, q_of(b - kWaves >= U ? b - kWaves : nb), b - kWaves >= U, q_of(b), true);
   }
-  float* rem_lds = lds + Lds::kFloats - 32;
+  float* rem_lds = lds + Lds::kRem;
   if (p.add_rem && threadIdx.x < 32 && k0 + (int)threadIdx.x < L)      // the forward wrote o + rem * v: dv_i gains rem_i * d_o_i
     rem_lds[threadIdx.x] = exp2f(p.row_stat[tile.seq_id * p.stat_sb + head * p.stat_sh + tok0 + k0 + threadIdx.x]);
   float* dvb = (float*)p.dv.ptr + tile.seq_id * p.dv.sb + head * p.dv.sh + (tok0 + k0) * p.dv.st;
   float* dkb = (float*)p.dk.ptr + tile.seq_id * p.dk.sb + head * p.dk.sh + (tok0 + k0) * p.dk.st;
-  reduce_store_f32<DH, kMode>(lds, dvacc, 1.f, dvb, p.dv.st, L - k0, D, p.add_rem ? dob + (int64_t)k0 * p.d_o.st : nullptr,
+  bool stored = reduce_store_f32<E, DH, kMode>(lds, dvacc, 1.f, dvb, p.dv.st, L - k0, D, p.add_rem ? dob + (int64_t)k0 * p.d_o.st : nullptr,
                                p.d_o.st, rem_lds);
-  reduce_store_f32<DH, kMode>(lds, dkacc, p.logit_scale, dkb, p.dk.st, L - k0, D);
+  stored |= reduce_store_f32<E, DH, kMode>(lds, dkacc, p.logit_scale, dkb, p.dk.st, L - k0, D);
+  return E::kSplit && any_odd(odd, stored | staged);
+}
+
+template <int DH, int kMode>
+__global__ __launch_bounds__(kThreads, 2) void bwd_dkv_f32_kernel(BwdParams p) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  int head, slot, sub;
+  xcd_head_tile_sub(blockIdx.x, kF32KeySplit, p.num_heads, &head, &slot, &sub);
+  if (slot >= p.counts[kCountK]) return;
+  const Tile tile = p.k_tiles[slot];
+  const int k0 = tile.origin + sub * kF32Rows;
+  if (k0 >= tile.seq_len) return;
+  if (p.fp32_products || bwd_dkv_f32_keys<Engine<DH, kMode>, DH, kMode>(p, tile, head, k0, lds)) bwd_dkv_f32_keys<Plain<DH, kMode>, DH, kMode>(p, tile, head, k0, lds);
 }
 
 // head_dim is rounded up to a multiple of 32 (the matrix cycles go by that); the exact variants skip every test of a
-// column against head_dim and load 16 bytes where the others load 4.
+// column against head_dim, the ones for multiples of 4 those within a piece of 4 columns (training pass, 3 heads x 80: 285 us
+// instead of 430).
 template <int DH, typename F>
 static hipError_t by_mode(int D, int load, F&& f) {
   std::integral_constant<int, DH> dh;
   if (load == kLoadScalar) return f(dh, std::integral_constant<int, kF32Far>());
-  return D == DH ? f(dh, std::integral_constant<int, kF32Exact>()) : f(dh, std::integral_constant<int, kF32Padded>());
+  if (D == DH) return f(dh, std::integral_constant<int, kF32Exact>());
+  return D % 4 ? f(dh, std::integral_constant<int, kF32Padded>()) : f(dh, std::integral_constant<int, kF32Quads>());
 }
 template <typename F>
 static hipError_t by_head_dim(int D, int load, F&& f) {
@@ -642,8 +900,16 @@ static hipError_t by_head_dim(int D, int load, F&& f) {
     default: return by_mode<128>(D, load, f);
   }
 }
+// Whether a call has too few workgroups for split products: a step of a wave takes longer with them, and more code is fetched; they pay
+// where waves share the matrix pipe or sequences are long.  Split / fp32 products, us:
+//   head_dim  64   4 heads, 448 tokens in sequences of up to 256 (112 workgroups)  kernels 45.4 / 40.6
+//             64   1 head, 6143 tokens in sequences of up to 2048 (240)   196 / 208        128: 319 / 360
+//             32   1 head, the same                                       139 / 130        2 heads (16) 141 / 147, 4 heads 151 / 177
+static bool few_workgroups(int D, int64_t tiles) { return tiles * kF32Split <= (D <= 32 ? 256 : 128); }
 
-hipError_t launch_fwd_f32(const FwdParams& p, int max_tiles, hipStream_t stream) {
+hipError_t launch_fwd_f32(const FwdParams& call, int max_tiles, hipStream_t stream) {
+  FwdParams p = call;
+  p.fp32_products = few_workgroups(p.head_dim, (int64_t)max_tiles * p.num_heads);
   return by_head_dim(p.head_dim, p.load, [&](auto dh, auto mode) {
     hipLaunchKernelGGL((fwd_f32_kernel<decltype(dh)::value, decltype(mode)::value>), dim3((unsigned)(xcd_sub_grid(max_tiles * p.num_heads, kF32Split) + p.sched.service)),
                        dim3(kThreads), 0, stream, p);
@@ -651,14 +917,16 @@ hipError_t launch_fwd_f32(const FwdParams& p, int max_tiles, hipStream_t stream)
   });
 }
 
-hipError_t launch_bwd_f32(const BwdParams& p, int max_q_tiles, int max_k_tiles, hipStream_t stream) {
+hipError_t launch_bwd_f32(const BwdParams& call, int max_q_tiles, int max_k_tiles, hipStream_t stream) {
+  BwdParams p = call;
+  p.fp32_products = few_workgroups(p.head_dim, (int64_t)max_q_tiles * p.num_heads);
   int dev = 0, cus = 0;
   const hipError_t e = device_cus(&dev, &cus);
   if (e != hipSuccess) return e;
   return by_head_dim(p.head_dim, p.load, [&](auto dh, auto mode) {
     constexpr int DH = decltype(dh)::value;
     constexpr int kMode = decltype(mode)::value;
-    constexpr size_t lds_bytes = DkvF32Lds<DH>::kFloats * sizeof(float);
+    constexpr size_t lds_bytes = most(DkvF32Lds<Plain<DH, kMode>, DH>::kFloats, DkvF32Lds<Engine<DH, kMode>, DH>::kFloats) * sizeof(float);
     static std::atomic<uint64_t> lds_done{0};
     const hipError_t r = raise_lds_limit(&bwd_dkv_f32_kernel<DH, kMode>, lds_done, dev, lds_bytes);
     if (r != hipSuccess) return r;

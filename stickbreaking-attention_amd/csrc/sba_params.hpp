@@ -81,6 +81,7 @@ struct FwdParams {
   int32_t add_rem;             // write o + rem * v
   int32_t max_tiles;           // query-tile slots the launch provides per head (>= counts[kCountQ])
   int64_t total_tokens;        // packed mode: rows of the token axis; rows no sequence covers are zero-filled
+  int32_t fp32_products;       // fp32 path: products on the fp32 matrix instruction throughout
 };
 
 struct BwdParams {
@@ -122,6 +123,7 @@ struct BwdParams {
   int64_t chain_rows;          // rows per head in chain_dq / chain_c
   int64_t chain_sb;            // fixed-length mode: rows per batch element (0 in packed mode)
   int32_t chain_tile_cap;      // key-tile slots per head in chain_flags
+  int32_t fp32_products;       // as in FwdParams
 };
 
 // One sequence's token range from cu_seqlens (cumulative sequence ends, optionally preceded by a 0).  Returns false

@@ -1,0 +1,50 @@
+"""From 128 workgroups on the fp32 kernels form their products of bf16 triples, which hold 26 bits of a number between 2^-109 and the largest bf16 number;
+workgroups that meet others form them of fp32 numbers instead.  Tensors at both ends of fp32's range, alone and with a partner that brings
+the products back to the middle, against the float64 oracle, 1e-5 in norm: a gradient is a difference of prefix sums of up to 161 terms,
+161 x 2^-24 = 0.96e-5 at worst where nothing cancels (measured: up to 1.3e-6); a triple of a number of 2^-122 is 2^-12 off at worst.  An infinite key against a large one: the logit saturates for both."""
+import pytest
+import torch
+
+from oracle import sb_oracle as orc
+from test_gpu_parity import NAMES, run_varlen, small_case
+
+pytestmark = pytest.mark.gpu
+
+LENGTHS, HEADS = [1, 33, 64, 161], 8      # (7 tiles per head, 224 workgroups: more than 128, below which triples are not used)
+CASES = {      # exponents added to q, k, v, do, drem
+    "middle": (0, 0, 0, 0, 0),
+    "tiny-values": (0, 0, -122, 0, 0),
+    "tiny-gradients": (0, 0, 0, -122, -122),
+    "tiny-values-and-drem": (0, 0, -122, 0, -122),
+    "tiny-keys-huge-queries": (122, -122, 0, 0, 0),
+    "huge-keys-tiny-queries": (-122, 122, 0, 0, 0),
+    "huge-values-tiny-gradients": (0, 0, 122, -122, 0),
+}
+
+
+@pytest.mark.parametrize("label", CASES)
+@pytest.mark.parametrize("D", [36, 64, 127, 128])
+def test_ends_of_the_range(gpu_device, D, label):
+    host, _, cu = small_case(HEADS, D, LENGTHS, torch.float32, seed=D)
+    host = [t * 2.0 ** e for t, e in zip(host, CASES[label])]
+    dev = [t.to(gpu_device) for t in host]
+    outs = run_varlen(dev[0], dev[1], dev[2], cu.to(gpu_device), LENGTHS, False, False, dev[3], dev[4])
+    d = [t.double() for t in host]
+    ref = orc.varlen_stream(d[0], d[1], d[2], cu, do=d[3], drem=d[4], dtype=torch.float64)
+    for n, a, r in zip(NAMES, outs, ref):
+        rel = ((a.detach().double().cpu() - r).norm() / r.norm()).item()
+        print(f"{label} D={D} {n}: relative error {rel:.2e}", flush=True)
+        assert rel < 1e-5, f"{n}: {rel:.2e}"
+
+
+@pytest.mark.parametrize("D", [36, 128])
+def test_infinite_key(gpu_device, D):
+    host, _, cu = small_case(HEADS, D, LENGTHS, torch.float32, seed=D)
+    host[0][..., 0] = 1
+    got = []
+    for value in (float("inf"), 1e30):
+        host[1][:, 50, 0] = value
+        dev = [t.to(gpu_device) for t in host]
+        got.append(run_varlen(dev[0], dev[1], dev[2], cu.to(gpu_device), LENGTHS, False, False, dev[3], dev[4]))
+    for n, a, b in zip(NAMES[:2], *got):
+        assert torch.isfinite(a).all() and ((a - b).norm() / b.norm()).item() < 1e-5, n

@@ -58,17 +58,20 @@ struct Layout {
 
 constexpr int64_t kRowTilesFrom = 64 << 10;      // rows x heads from which the backward on row tiles runs (see plan)
 
-// Whether the 8 queues of the backward on row tiles, each fed to one XCD, hold about the same work: (head, sequence) goes to queue
-// (head + heads x sequence) % 8.  With a head count that is a multiple of 8 they do; else a queue may hold one head of a sequence more
-// than another, which evens out over the sequences if none is much longer than the rest.
-bool queues_even(int64_t heads, int64_t seqs, int64_t mean_len, int64_t max_len) {
+// Whether the 8 queues of the backward on row tiles, each fed to one XCD, hold about the same work, within 8/7 of the mean.  With a head
+// count that is a multiple of 8 they do; else a queue may hold one head of a sequence more than another, which evens out over the
+// sequences (row_queue) but for what the longest has more than the others: at most its share of all pairs, where the others are equal.
+bool queues_even(int64_t heads, int64_t seqs, int64_t tokens, int64_t max_len) {
   if ((heads & 7) == 0) return true;
   int64_t units[8] = {0}, most = 0;
   const int64_t n = seqs < 8 ? seqs : 8;      // (the pattern repeats)
-  for (int64_t s = 0; s < n; s++)
-    for (int64_t q = 0; q < 8; q++) units[(q + heads * s) & 7] += heads / 8 + (q < (heads & 7));
+  for (int64_t r = 0; r < n; r++)
+    for (int64_t h = 0; h < heads; h++) units[(sba::row_queue((int)r, (int)(heads & 7)) + h) & 7]++;
   for (int64_t u : units) most = u > most ? u : most;
-  return most * 7 <= heads * n && (max_len <= 2 * mean_len || cdiv(heads, 8) * 7 <= heads);      // within 8/7 of the mean
+  if (most * 7 > heads * n) return false;
+  if (max_len * seqs <= 2 * tokens) return true;
+  const double others = seqs > 1 ? (double)(tokens - max_len) / max_len : 0., longest = 1. / (1. + others * others / (double)(seqs > 1 ? seqs - 1 : 1));
+  return ((double)(8 * cdiv(heads, 8)) / (double)heads - 1.) * longest <= 1. / 7;
 }
 
 // `row_tiles`: a group of the heads of a call that runs the backward on row tiles, which the group then runs as well.
@@ -119,15 +122,20 @@ int plan(const SbaArgs* a, Layout* out, bool row_tiles = false) {
   // key tiles over the two kernels
   //   20 K .. 64 K, length x heads from 16 K on      0.79 .. 0.93        up to 256 tokens  0.91 .. 0.97
   //   < 20 K        1024 to 2048 tokens              1.10 .. 1.25        up to 256 tokens  0.93 .. 0.97
+  // At head_dim 64 (against the two kernels; the tiles' element-wise work bounds it, and rows that a tile does not fill cost more):
+  //   length     64           128          256          384          512          768, 1024    2048, 4096   8192, 16384
+  //   64 K       1.00         1.00         0.90 .. 1.00 1.03         0.84 .. 0.89 0.80 .. 0.84 0.83 .. 0.92 0.88 .. 1.00
+  //   128 .. 512 K 1.20 .. 1.47 1.05 .. 1.26 0.89 .. 1.01 1.02 .. 1.16 0.82 .. 0.99 0.78 .. 0.95 0.76 .. 0.89 0.68 .. 0.81
+  //   32 K       0.99         0.92 .. 1.00 1.00         0.97         0.99         1.02 .. 1.19 1.15 .. 1.48
   const int64_t mean_len = fixed ? T : T / B, rows_heads = rows * a->num_heads, mean_heads = mean_len * a->num_heads;
   const bool chain_shape = a->dtype != SBA_F32 && a->head_dim == 128 && (a->num_heads & 7) == 0 && !a->add_remainder;
   if (row_tiles) {
     L.chain = Layout::kRowTiles;
-  } else if (rows_heads >= kRowTilesFrom && a->dtype != SBA_F32 && a->head_dim == 128 && a->backward_kernels != 1 && (chain_shape || a->backward_kernels == 0)) {
+  } else if (rows_heads >= kRowTilesFrom && a->dtype != SBA_F32 && (a->head_dim == 128 || (a->head_dim == 64 && mean_len >= 512)) && a->backward_kernels != 1 && (chain_shape || a->backward_kernels == 0)) {
     // One kernel where its flags were cleared with the schedule ...
     L.one_kernel = chain_shape && (a->backward_kernels == 2 || (max_len <= 128 && mean_len > 96) ||
                                    (a->num_heads <= 32 && mean_heads >= 32 << 10 && max_len * a->num_heads <= 192 << 10));
-    if (L.one_kernel || queues_even(a->num_heads, B, mean_len, max_len)) L.chain = Layout::kRowTiles;
+    if (L.one_kernel || queues_even(a->num_heads, B, rows, max_len)) L.chain = Layout::kRowTiles;
   } else if (chain_shape && (a->backward_kernels == 2 ||
                              (a->backward_kernels == 0 &&
                               (max_len <= 256 || (a->num_heads <= 32 && rows_heads >= 20 << 10 && mean_heads >= 16 << 10))))) {
@@ -154,15 +162,16 @@ int plan(const SbaArgs* a, Layout* out, bool row_tiles = false) {
   if (L.chain == Layout::kRowTiles) {
     L.chain_rows = rows * 9 / 256 + 2;      // (key blocks of 32: every sequence that hands any over is longer than 256)
     L.row_group = a->num_heads;
+    const int64_t row_block = 2 * 32 * 4 * (int64_t)a->head_dim;      // bytes of a key block's dV and dK
     // What is handed over lies at its key blocks' places, also where most rows are in sequences that hand nothing over: 1152 bytes
     // per row and head.  The heads of such a batch go through in several launches, multiples of 8 (an equal share for each
     // queue), that keep this within 1.15 times the carry plane as long as each still fills the chip twice.
     if (mean_len < sba::kRowTileRows && max_len > sba::kRowTileRows) {
-      const int64_t least = align_up(cdiv(2 * kRowTilesFrom, rows), 8), fit = (int64_t)L.carry_bytes / 20 * 23 / (L.chain_rows * 32768) & ~7;
+      const int64_t least = align_up(cdiv(2 * kRowTilesFrom, rows), 8), fit = (int64_t)L.carry_bytes / 20 * 23 / (L.chain_rows * row_block) & ~7;
       const int64_t group = fit > least ? fit : least;
       if (group < a->num_heads) L.row_group = group;
     }
-    chain_bytes = (size_t)L.row_group * L.chain_rows * 32768;
+    chain_bytes = (size_t)L.row_group * L.chain_rows * row_block;
     if (L.one_kernel) row_region();
   }
   L.sched_bytes = off;

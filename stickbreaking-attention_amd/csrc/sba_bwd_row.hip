@@ -12,7 +12,7 @@
 //
 // Hand-over.  A wave issues its stores, waits for them (vmcnt) and then stores the number of key blocks that are complete into a flag of
 // its own; the same wave of the tile below reads flag and partial results with sc1 (served by the L2, never by the vector L1).  All
-// tiles of a (head, sequence) run on one XCD, i.e. on one L2: (head, sequence) belongs to one of 8 queues, a workgroup takes
+// tiles of a (head, sequence) run on one XCD, i.e. on one L2: (head, sequence) belongs to one of 8 queues (row_queue), a workgroup takes
 // tiles from queue blockIdx % 8 (workgroups are dealt to the XCDs in turn), and every workgroup checks its XCC id against the first
 // of its queue.  Progress: tiles are taken in list order, a tile waits only for one that was taken before it, so every wait ends;
 // the waits are bounded all the same.
@@ -23,6 +23,12 @@
 // the backward: 4180 us with key tiles (sba_bwd_chain.hip), 3330 us here; 32768 tokens in 25 sequences of up to 4096, 32 heads: 2650 and
 // 2150.  Without the hand-over it would take 3130, without the tile math as well 2590: at 2.1 GHz, the clock that the power limit
 // leaves, and 2.0 for the products alone.  256 rows per tile, because the hand-over costs 8 bytes per pair / (rows / 256).
+//
+// head_dim 64: half the products per pair and the same element-wise work, which bounds it (320 vector-ALU instructions against 20
+// MFMAs per block and wave).  A key block has four pieces of {dV, dK}, so a step is two blocks and a wave contracts a piece of one of
+// them; LDS holds four blocks, Q stays in registers.  (Steps of one block, contracted by every second wave in turn: the wave whose
+// turn it is arrives last at every barrier: 12 heads, 16384 tokens in 10 sequences of up to 3523, 474 us instead of 434.)  Training passes,
+// us, two kernels and here: 484 and 434; 16 heads x 4 x 4096 946 and 763; 8 heads x 8 x 1024 142 and 108.
 #include "sba_device.hpp"
 #include "sba_host.hpp"
 #include "sba_params.hpp"
@@ -36,14 +42,16 @@ constexpr int kRowTile = kRowTileRows;      // query rows per workgroup
 constexpr int kRowWaves = 8, kRowThreads = 64 * kRowWaves;
 constexpr int kRowKeys = 32;                // keys per step
 
+template <int DH>
 struct RowLds {
-  static constexpr int kExch = 0;                      // 2 x {P, dZ} of a step: [row][32 keys], 16 KB each
+  static constexpr int kBufs = DH == 128 ? 2 : 4;      // of the key blocks' buffers: two steps' worth
+  static constexpr int kExch = 0;                      // {P, dZ} of a block: [row][32 keys], 16 KB each
   static constexpr int kExchBuf = 32768, kExchMat = 16384;
-  static constexpr int kQ = 65536;                     // Q of the tile: 4 panels of [row][32 columns]
-  static constexpr int kPanel = kRowTile * 64;
-  static constexpr int kKv = 131072;                   // 2 x {K, V} of a step: 4 panels of [key][32 columns] each
-  static constexpr int kKvBuf = 16384, kKvMat = 8192, kKvPanel = kRowKeys * 64;
-  static constexpr int kBytes = 163840;
+  static constexpr int kQ = 65536;                     // Q of the tile: panels of [row][32 columns] (head_dim 64: until it is in registers)
+  static constexpr int kPanels = DH / 32, kPanel = kRowTile * 64;
+  static constexpr int kKv = 131072;                   // {K, V} of a block: panels of [key][32 columns] each
+  static constexpr int kKvPanel = kRowKeys * 64, kKvMat = kPanels * kKvPanel, kKvBuf = 2 * kKvMat;
+  static constexpr int kBytes = kKv + kBufs * kKvBuf;
 };
 
 typedef __attribute__((address_space(3))) unsigned char lds_u8;
@@ -156,9 +164,12 @@ __device__ __forceinline__ int wait_for(const int32_t* pred, int t, int32_t* sta
   return 0x7fffffff;      // no later wait of this tile
 }
 
-template <typename T, bool kAddRem>
+template <typename T, int DH, bool kAddRem>
 __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
-  constexpr int DH = 128, kSteps = DH / 16, kDTiles = DH / 32;
+  constexpr int kSteps = DH / 16, kDTiles = DH / 32;
+  constexpr bool kWide = DH == 128;        // a step is one key block, of which every wave contracts a piece; else two, of which it contracts one
+  constexpr int kPieces = DH / 16;         // 32 x 32 pieces of dV and dK per key block
+  typedef RowLds<DH> Lds;
   typedef typename Elem<T>::vec8 vec8;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   lds_u8* const lds = (lds_u8*)lds_raw;
@@ -201,10 +212,11 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
   const int tr_k = (4 * half + (s15 >> 2)) * 64 + ((tr_chunk ^ half) << 4) + tr_byte;         // ... in key order: (^ 32) + 512
   const int wr_a = (32 * wave + col) * 64 + (((2 * half) ^ sw) << 4);                         // 8 of this lane's keys; the others: ^ 16
 
-  const bool out = wave >= 4;              // which result this wave contracts: dK, else dV
-  const int cp = wave & 3;                 // ... and which 32 columns of it
+  const bool out = kWide ? wave >= 4 : (wave & 2) != 0;      // which result this wave contracts: dK, else dV
+  const int cp = kWide ? wave & 3 : wave & 1;           // ... and which 32 columns of it
   const int per_slot = (H + 7) >> 3;       // heads of a tile slot that a queue may hold
 
+  int rank = -1, ranked = -1;              // how many sequences the list begins up to slot `ranked`, less 1
   for (;;) {
     if (threadIdx.x == 0) *reinterpret_cast<int*>(lds_raw) = atomicAdd(cursor, 1);
     __syncthreads();
@@ -214,7 +226,11 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
     if (slot >= n_tiles) break;
     Tile tile = p.k_tiles[slot];
     const int L = __builtin_amdgcn_readfirstlane(tile.seq_len), seq_id = __builtin_amdgcn_readfirstlane(tile.seq_id);
-    const int head = ((queue - seq_id * H) & 7) + 8 * (claim - slot * per_slot);
+    if (H & 7) {
+      for (int first = ranked + 1; first <= slot; first += 64) rank += __builtin_popcountll(__ballot(first + lane <= slot && p.k_tiles[min(first + lane, slot)].origin == 0));
+      ranked = slot;
+    }
+    const int head = ((queue - row_queue(rank, H)) & 7) + 8 * (claim - slot * per_slot);
     if (head >= H) continue;
     const int64_t tok0 = __builtin_amdgcn_readfirstlane(tile.seq_start);
     const int64_t carry_base = (int64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)tile.carry_base) |
@@ -232,13 +248,17 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
     const T* vb = (const T*)p.v.ptr + seq_id * p.v.sb + head * p.v.sh + tok0 * p.v.st;
     const T* dob = (const T*)p.d_o.ptr + seq_id * p.d_o.sb + head * p.d_o.sh + tok0 * p.d_o.st;
     const int q_st = (int)(p.q.st * 2), do_st = (int)(p.d_o.st * 2);
-    // K and V rows of key block t into stage t & 1: waves 0-3 bring a panel of K each, 4-7 one of V.
-    const int kv_st = (int)((out ? p.v.st : p.k.st) * 2);
-    const u32x4 kv_desc = buffer_desc(out ? vb : kb, (L - 1) * kv_st + 2 * DH);
-    const int kv_voff = mfma_row_to_key32(lane >> 2) * kv_st + cp * 64 + (((lane & 3) ^ ((lane >> 4) & 3)) << 4);
+    // K and V rows of step t's key blocks: a wave brings a panel of one of them (waves 0-3: K, 4-7: V; head_dim 64: of the first block, of
+    // the second).
+    const int kv_panel = kWide ? cp : wave & 1, kv_sub = kWide ? 0 : wave >> 2;
+    const bool brings_v = kWide ? out : (wave & kDTiles) != 0;
+    const int kv_st = (int)((brings_v ? p.v.st : p.k.st) * 2);
+    const u32x4 kv_desc = buffer_desc(brings_v ? vb : kb, (L - 1) * kv_st + 2 * DH);
+    const int kv_voff = mfma_row_to_key32(lane >> 2) * kv_st + kv_panel * 64 + (((lane & 3) ^ ((lane >> 4) & 3)) << 4);
     auto request_kv = [&](int t) {
-      const int soff = min(t, n - 1) * kRowKeys * kv_st;
-      dma16x2<1024>(lds_base + RowLds::kKv + (t & 1) * RowLds::kKvBuf + wave * 2048, kv_voff, kv_desc, soff, soff + 8 * kv_st);
+      const int block = kWide ? t : 2 * t + kv_sub, soff = min(block, n - 1) * kRowKeys * kv_st;
+      const int dst = kWide ? (t & 1) * Lds::kKvBuf + wave * 2048 : (block & 3) * Lds::kKvBuf + (wave & 3) * 2048;
+      dma16x2<1024>(lds_base + Lds::kKv + dst, kv_voff, kv_desc, soff, soff + 8 * kv_st);
     };
     // Q and dO of the tile; dO into the exchange buffers until its operands are in registers.
     {
@@ -246,10 +266,10 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
       const int chunk = ((lane & 3) ^ ((lane >> 4) & 3)) * 16;
       const int q_voff = (lane >> 2) * q_st + chunk, do_voff = (lane >> 2) * do_st + chunk;
 #pragma unroll
-      for (int i = 0; i < 4; i++) {      // panel i, rows 16 wave and 128 + 16 wave
-        const int row = q0 + 16 * wave, dst = lds_base + wave * 1024 + i * RowLds::kPanel;
-        dma16x2<8192>(dst + RowLds::kQ, q_voff, q_desc, row * q_st + 64 * i, (row + 128) * q_st + 64 * i);
-        dma16x2<8192>(dst + RowLds::kExch, do_voff, do_desc, row * do_st + 64 * i, (row + 128) * do_st + 64 * i);
+      for (int i = 0; i < Lds::kPanels; i++) {      // panel i, rows 16 wave and 128 + 16 wave
+        const int row = q0 + 16 * wave, dst = lds_base + wave * 1024 + i * Lds::kPanel;
+        dma16x2<8192>(dst + Lds::kQ, q_voff, q_desc, row * q_st + 64 * i, (row + 128) * q_st + 64 * i);
+        dma16x2<8192>(dst + Lds::kExch, do_voff, do_desc, row * do_st + 64 * i, (row + 128) * do_st + 64 * i);
       }
     }
     request_kv(0);
@@ -268,19 +288,24 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
       return carry + (carry_offset(u, n_qt) - kBlockQ * (u >> 2));
     };
     // What the row tiles of a (head, sequence) hand down: per key block and wave, the 32 x 32 partial result.
-    float* part = p.chain_dq + ((int64_t)head * p.chain_rows + ((int64_t)seq_id * p.chain_sb + tok0) * 9 / 256) * 8192 + wave * 1024;
+    float* part = p.chain_dq + ((int64_t)head * p.chain_rows + ((int64_t)seq_id * p.chain_sb + tok0) * 9 / 256) * (kPieces * 1024) + (wave & (kPieces - 1)) * 1024;
     int32_t* flag = p.chain_flags + ((int64_t)head * p.chain_tile_cap + slot) * 8 + wave;
     const int32_t* pred = has_pred ? flag - 8 : flag;
     const int lane16 = lane * 16;
 
     vm_wait<0>();
     __syncthreads();
-    vec8 dof[kSteps], wf[16];
-    {
-      lds_u8* rows = lds + RowLds::kExch + 32 * wave * 64;
+    vec8 dof[kSteps], wf[16], qf[kWide ? 1 : kSteps];
+    if constexpr (!kWide) {      // (head_dim 128: read from LDS in every step)
+      lds_u8* rows = lds + Lds::kQ + 32 * wave * 64;
 #pragma unroll
-      for (int kk = 0; kk < kSteps; kk++) dof[kk] = lds_load<vec8>(rows + ((kk & 1) ? row_a ^ 32 : row_a) + (kk >> 1) * RowLds::kPanel);
-      lds_u8* cols = lds + (out ? RowLds::kQ : RowLds::kExch) + cp * RowLds::kPanel;
+      for (int kk = 0; kk < kSteps; kk++) qf[kk] = lds_load<vec8>(rows + ((kk & 1) ? row_a ^ 32 : row_a) + (kk >> 1) * Lds::kPanel);
+    }
+    {
+      lds_u8* rows = lds + Lds::kExch + 32 * wave * 64;
+#pragma unroll
+      for (int kk = 0; kk < kSteps; kk++) dof[kk] = lds_load<vec8>(rows + ((kk & 1) ? row_a ^ 32 : row_a) + (kk >> 1) * Lds::kPanel);
+      lds_u8* cols = lds + (out ? Lds::kQ : Lds::kExch) + cp * Lds::kPanel;
 #pragma unroll
       for (int c = 0; c < 16; c++) wf[c] = tr_pair<T>(cols + tr_e + 1024 * c, cols + (tr_e ^ 16) + 256 + 1024 * c);
     }
@@ -304,17 +329,18 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
 
     const RowSink<T> sink = out ? make_row_sink<T>((T*)p.dk.ptr + seq_id * p.dk.sb + head * p.dk.sh + tok0 * p.dk.st, p.dk.st, L, DH)
                                 : make_row_sink<T>((T*)p.dv.ptr + seq_id * p.dv.sb + head * p.dv.sh + tok0 * p.dv.st, p.dv.st, L, DH);
-    float n_prod;
+    float n_prod; float n_prod2;      // of the next step's key blocks
     int seen_count = 0;      // key blocks the tile above has passed on, as last read
     asm volatile("s_nop 4\n\tglobal_load_dword %0, %1, %2" : "=v"(n_prod) : "v"(row_c * 4), "s"(product_at(0)) : "memory");
-    asm volatile("s_waitcnt vmcnt(0)" : "+v"(n_prod)::"memory");
+    if constexpr (!kWide) asm volatile("s_nop 4\n\tglobal_load_dword %0, %1, %2" : "=v"(n_prod2) : "v"(row_c * 4), "s"(product_at(1)) : "memory");
+    if constexpr (kWide) asm volatile("s_waitcnt vmcnt(0)" : "+v"(n_prod)::"memory"); else asm volatile("s_waitcnt vmcnt(0)" : "+v"(n_prod), "+v"(n_prod2)::"memory");
 
     f32x4 c0 = {0.f, 0.f, 0.f, 0.f}, c1 = c0, c2 = c0, c3 = c0;      // what the tile above has passed on of the key block contracted next
     auto contract = [&](int tc) {
       f32x16 acc;
 #pragma unroll
       for (int r = 0; r < 16; r++) acc[r] = 0.f;
-      lds_u8* ex = lds + RowLds::kExch + (tc & 1) * RowLds::kExchBuf + (out ? RowLds::kExchMat : 0);
+      lds_u8* ex = lds + Lds::kExch + (tc & (Lds::kBufs - 1)) * Lds::kExchBuf + (out ? Lds::kExchMat : 0);
       lds_u8* e0 = ex + tr_e;
       lds_u8* e1 = ex + flip<16>(tr_e) + 256;
       const int w0 = max(0, tc - own);
@@ -353,38 +379,29 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
       } else {
         const f32x4 d0 = __builtin_shufflevector(acc, acc, 0, 1, 2, 3), d1 = __builtin_shufflevector(acc, acc, 4, 5, 6, 7),
                     d2 = __builtin_shufflevector(acc, acc, 8, 9, 10, 11), d3 = __builtin_shufflevector(acc, acc, 12, 13, 14, 15);
-        float* dst = part + (int64_t)tc * 8192;
+        float* dst = part + (int64_t)tc * (kPieces * 1024);
         asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %5\n\tglobal_store_dwordx4 %0, %2, %5 offset:1024\n\t"
                      "global_store_dwordx4 %0, %3, %5 offset:2048\n\tglobal_store_dwordx4 %0, %4, %5 offset:3072"
                      ::"v"(lane16), "v"(d0), "v"(d1), "v"(d2), "v"(d3), "s"(dst) : "memory");
       }
     };
     const bool late = wave >= 4;      // (waves w and w + 4 share a SIMD)
-    lds_barrier();
-    for (int t = 0; t < n; ++t) {
-      asm volatile("; nothing in flight");
-      const float prod_in = n_prod;
-      const int j0 = kRowKeys * t;
-      const bool seen = w_first < L && j0 <= last_seen;
-      lds_u8* kt = lds + RowLds::kKv + (t & 1) * RowLds::kKvBuf;
-      lds_u8* ex = lds + RowLds::kExch + (t & 1) * RowLds::kExchBuf;
-      u32x4 dz[2];
-      float r_prod;
-      int r_count, count;
-      asm volatile("s_nop 4\n\tglobal_load_dword %0, %2, %4 sc1\n\tglobal_load_dword %1, %3, %5"
-                   : "=&v"(r_count), "=&v"(r_prod) : "v"(0), "v"(row_c * 4), "s"(pred), "s"(product_at(t + 1)) : "memory");
-      request_kv(t + 1);
+    // Of a key block: P and dZ of this wave's rows, into LDS ...
+    auto front = [&](int j0, bool seen, lds_u8* kt, lds_u8* ex, float prod_in, u32x4 (&dz)[2]) {
       if (seen) {
         f32x16 s, dp;
 #pragma unroll
         for (int r = 0; r < 16; r++) { s[r] = 0.f; dp[r] = 0.f; }
         lds_u8* k0 = kt + row_a;
         lds_u8* k1 = kt + flip<32>(row_a);
-        lds_u8* q0p = lds + RowLds::kQ + 32 * wave * 64 + row_a;
-        lds_u8* q1p = lds + RowLds::kQ + 32 * wave * 64 + flip<32>(row_a);
-        auto k_op = [&](int kk) { return lds_load<vec8>(((kk & 1) ? k1 : k0) + (kk >> 1) * RowLds::kKvPanel); };
-        auto v_op = [&](int kk) { return lds_load<vec8>(((kk & 1) ? k1 : k0) + RowLds::kKvMat + (kk >> 1) * RowLds::kKvPanel); };
-        auto q_op = [&](int kk) { return lds_load<vec8>(((kk & 1) ? q1p : q0p) + (kk >> 1) * RowLds::kPanel); };
+        lds_u8* q0p = lds + Lds::kQ + 32 * wave * 64 + row_a;
+        lds_u8* q1p = lds + Lds::kQ + 32 * wave * 64 + flip<32>(row_a);
+        auto k_op = [&](int kk) { return lds_load<vec8>(((kk & 1) ? k1 : k0) + (kk >> 1) * Lds::kKvPanel); };
+        auto v_op = [&](int kk) { return lds_load<vec8>(((kk & 1) ? k1 : k0) + Lds::kKvMat + (kk >> 1) * Lds::kKvPanel); };
+        auto q_op = [&](int kk) {
+          if constexpr (kWide) return lds_load<vec8>(((kk & 1) ? q1p : q0p) + (kk >> 1) * Lds::kPanel);
+          else return qf[kk];
+        };
         constexpr int kAhead = 3, kVAhead = 3;
         vec8 ka[kAhead], qa[kAhead], va[kVAhead];
 #pragma unroll
@@ -421,56 +438,93 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
         lds_put(ex + wr_a, dz[0]);
         lds_put(ex + (wr_a ^ 16), dz[0]);
       }
-      lds_put(ex + RowLds::kExchMat + wr_a, dz[0]);
-      lds_put(ex + RowLds::kExchMat + flip<16>(wr_a), dz[1]);
-      asm volatile("s_waitcnt vmcnt(2)\n\tv_mov_b32 %0, %2\n\tv_readfirstlane_b32 %1, %3"
-                   : "=&v"(n_prod), "=s"(count) : "v"(r_prod), "v"(r_count) : "memory");
-      // The key blocks that are complete are passed on; what the tile above left of the one that is contracted next is asked for.
-      const int tn = late ? t - 1 : t;
-      if (lane == 0) *flag = tn;
-      seen_count = max(seen_count, count);
-      if (has_pred && tn >= 0) {
-        if (seen_count <= tn) seen_count = wait_for(pred, tn, p.status, lane);
-        const float* src = part + (int64_t)tn * 8192;
-        asm volatile("s_nop 4\n\tglobal_load_dwordx4 %0, %4, %5 sc1\n\tglobal_load_dwordx4 %1, %4, %5 offset:1024 sc1\n\t"
-                     "global_load_dwordx4 %2, %4, %5 offset:2048 sc1\n\tglobal_load_dwordx4 %3, %4, %5 offset:3072 sc1"
-                     : "=&v"(c0), "=&v"(c1), "=&v"(c2), "=&v"(c3) : "v"(lane16), "s"(src) : "memory");
-      } else {
-        c0 = c1 = c2 = c3 = f32x4{0.f, 0.f, 0.f, 0.f};
-      }
+      lds_put(ex + Lds::kExchMat + wr_a, dz[0]);
+      lds_put(ex + Lds::kExchMat + flip<16>(wr_a), dz[1]);
+    };
+    // ... and dQ += dZ K.
+    auto add_dq = [&](bool seen, lds_u8* kt, const u32x4 (&dz)[2]) {
       if (seen) {
         lds_u8* t0 = kt + tr_k;
         lds_u8* t1 = kt + flip<32>(tr_k) + 512;
-        auto kc_op = [&](int i) { const int o = 1024 * (i >> 2) + (i & 3) * RowLds::kKvPanel; return tr_pair<T>(t0 + o, t1 + o); };
+        auto kc_op = [&](int i) { const int o = 1024 * (i / kDTiles) + (i % kDTiles) * Lds::kKvPanel; return tr_pair<T>(t0 + o, t1 + o); };
         vec8 b[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) b[i] = kc_op(i);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-          dqacc[i & 3] = Elem<T>::mfma(as_vec8<T>(dz[i >> 2]), b[i & 3], dqacc[i & 3]);
-          if (i + 4 < 8) b[i & 3] = kc_op(i + 4);
+        for (int i = 0; i < 2 * kDTiles; i++) {
+          dqacc[i % kDTiles] = Elem<T>::mfma(as_vec8<T>(dz[i / kDTiles]), b[i & 3], dqacc[i % kDTiles]);
+          if (i + 4 < 2 * kDTiles) b[i & 3] = kc_op(i + 4);
           __builtin_amdgcn_sched_barrier(0);
         }
       }
+    };
+    // What the tile above left of block t is asked for, once it is there.
+    auto request_above = [&](int t) {
+      if (seen_count <= t) seen_count = wait_for(pred, t, p.status, lane);
+      const float* src = part + (int64_t)t * (kPieces * 1024);
+      asm volatile("s_nop 4\n\tglobal_load_dwordx4 %0, %4, %5 sc1\n\tglobal_load_dwordx4 %1, %4, %5 offset:1024 sc1\n\t"
+                   "global_load_dwordx4 %2, %4, %5 offset:2048 sc1\n\tglobal_load_dwordx4 %3, %4, %5 offset:3072 sc1"
+                   : "=&v"(c0), "=&v"(c1), "=&v"(c2), "=&v"(c3) : "v"(lane16), "s"(src) : "memory");
+    };
+    const int steps = kWide ? n : (n + 1) / 2;
+    // The block of step t that this wave contracts.
+    auto block_of = [&](int t) { return kWide ? t : 2 * t + (wave >> 2); };
+    lds_barrier();
+    for (int t = 0; t < steps; ++t) {
+      asm volatile("; nothing in flight");
+      const float prod_in = n_prod, prod_in2 = kWide ? 0.f : n_prod2;
+      const int first = kWide ? t : 2 * t, last = kWide ? t : 2 * t + 1;      // the step's key blocks
+      const bool seen = w_first < L && kRowKeys * last <= last_seen;
+      lds_u8* kt = lds + Lds::kKv + (last & (Lds::kBufs - 1)) * Lds::kKvBuf;
+      lds_u8* ex = lds + Lds::kExch + (last & (Lds::kBufs - 1)) * Lds::kExchBuf;
+      u32x4 dz[2];
+      float r_prod, r_prod2;
+      int r_count, count;
+      if constexpr (kWide) {
+        asm volatile("s_nop 4\n\tglobal_load_dword %0, %2, %4 sc1\n\tglobal_load_dword %1, %3, %5"
+                     : "=&v"(r_count), "=&v"(r_prod) : "v"(0), "v"(row_c * 4), "s"(pred), "s"(product_at(t + 1)) : "memory");
+      } else {
+        asm volatile("s_nop 4\n\tglobal_load_dword %0, %3, %5 sc1\n\tglobal_load_dword %1, %4, %6\n\tglobal_load_dword %2, %4, %7"
+                     : "=&v"(r_count), "=&v"(r_prod), "=&v"(r_prod2)
+                     : "v"(0), "v"(row_c * 4), "s"(pred), "s"(product_at(2 * t + 2)), "s"(product_at(2 * t + 3)) : "memory");
+      }
+      request_kv(t + 1);
+      if constexpr (kWide) {
+        front(kRowKeys * t, seen, kt, ex, prod_in, dz);
+        asm volatile("s_waitcnt vmcnt(2)\n\tv_mov_b32 %0, %2\n\tv_readfirstlane_b32 %1, %3"
+                     : "=&v"(n_prod), "=s"(count) : "v"(r_prod), "v"(r_count) : "memory");
+      } else {
+        const bool seen1 = w_first < L && kRowKeys * first <= last_seen;
+        front(kRowKeys * first, seen1, kt - Lds::kKvBuf, ex - Lds::kExchBuf, prod_in, dz);
+        add_dq(seen1, kt - Lds::kKvBuf, dz);
+        front(kRowKeys * last, seen, kt, ex, prod_in2, dz);
+        asm volatile("s_waitcnt vmcnt(2)\n\tv_mov_b32 %0, %3\n\tv_mov_b32 %1, %4\n\tv_readfirstlane_b32 %2, %5"
+                     : "=&v"(n_prod), "=&v"(n_prod2), "=s"(count) : "v"(r_prod), "v"(r_prod2), "v"(r_count) : "memory");
+      }
+      // The key blocks that are complete are passed on; what the tile above left of the one that is contracted next is asked for.
+      const int tn = late ? t - 1 : t, block = block_of(tn);
+      const bool any = tn >= 0 && (kWide || block < n);
+      if (lane == 0) *flag = kWide ? block : block - 1;      // (the one before was this wave's last)
+      seen_count = max(seen_count, count);
+      if (has_pred && any) request_above(block);
+      else c0 = c1 = c2 = c3 = f32x4{0.f, 0.f, 0.f, 0.f};
+      add_dq(seen, kt, dz);
       // The rows of step t + 1 are in LDS before the barrier (behind them: the flag, and what the tile above left).
-      if (!late || t == 0) {
-        if (has_pred && !late) vm_wait<5>(); else vm_wait<1>();
+      if (!late || !any) {
+        if (has_pred && any) vm_wait<5>(); else vm_wait<1>();
       }
       if (!late) lds_barrier();
-      if (tn >= 0) contract(tn);
+      if (any) contract(block);
       if (late) lds_barrier();
     }
     if (late) {
       vm_wait<0>();
-      if (has_pred) {
-        if (seen_count < n) seen_count = wait_for(pred, n - 1, p.status, lane);
-        const float* src = part + (int64_t)(n - 1) * 8192;
-        asm volatile("s_nop 4\n\tglobal_load_dwordx4 %0, %4, %5 sc1\n\tglobal_load_dwordx4 %1, %4, %5 offset:1024 sc1\n\t"
-                     "global_load_dwordx4 %2, %4, %5 offset:2048 sc1\n\tglobal_load_dwordx4 %3, %4, %5 offset:3072 sc1"
-                     : "=&v"(c0), "=&v"(c1), "=&v"(c2), "=&v"(c3) : "v"(lane16), "s"(src) : "memory");
+      const int block = block_of(steps - 1);
+      if (kWide || block < n) {
+        if (has_pred) request_above(block);
+        contract(block);
       }
-      contract(n - 1);
     }
     // The last results are passed on.
     vm_wait<0>();
@@ -489,16 +543,16 @@ __global__ __launch_bounds__(256) void row_clear_kernel(u32x4* z, int64_t n16) {
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n16; i += (int64_t)gridDim.x * 256) z[i] = u32x4{0u, 0u, 0u, 0u};
 }
 
-template <typename T, bool kAddRem>
+template <typename T, int DH, bool kAddRem>
 static hipError_t launch_row_t(const BwdParams& p, int max_tiles, hipStream_t stream) {
   static std::atomic<uint64_t> lds_done{0};
   int dev = 0, cus = 0;
   hipError_t e = device_cus(&dev, &cus);
   if (e != hipSuccess) return e;
-  if ((e = raise_lds_limit(&bwd_row_kernel<T, kAddRem>, lds_done, dev, RowLds::kBytes)) != hipSuccess) return e;
+  if ((e = raise_lds_limit(&bwd_row_kernel<T, DH, kAddRem>, lds_done, dev, RowLds<DH>::kBytes)) != hipSuccess) return e;
   const int64_t tiles = (int64_t)max_tiles * ((p.num_heads + 7) / 8);      // per queue, at most
   const int per_queue = (int)(tiles < cus / 8 ? tiles : cus / 8);
-  hipLaunchKernelGGL((bwd_row_kernel<T, kAddRem>), dim3((unsigned)(8 * per_queue)), dim3(kRowThreads), RowLds::kBytes, stream, p);
+  hipLaunchKernelGGL((bwd_row_kernel<T, DH, kAddRem>), dim3((unsigned)(8 * per_queue)), dim3(kRowThreads), RowLds<DH>::kBytes, stream, p);
   return hipGetLastError();
 }
 
@@ -506,7 +560,7 @@ static hipError_t launch_row_t(const BwdParams& p, int max_tiles, hipStream_t st
 bool row_supported(const BwdParams& p) {
   int dev = 0, cus = 0;
   if (device_cus(&dev, &cus) != hipSuccess) return false;
-  return p.load == kLoadAligned && p.head_dim == 128 && !p.wide_rows && cus >= 8;
+  return p.load == kLoadAligned && (p.head_dim == 64 || p.head_dim == 128) && !p.wide_rows && cus >= 8;
 }
 
 hipError_t launch_row_clear(uint32_t* region, int64_t bytes, hipStream_t stream) {
@@ -515,9 +569,13 @@ hipError_t launch_row_clear(uint32_t* region, int64_t bytes, hipStream_t stream)
   return hipGetLastError();
 }
 
+template <int DH>
+static hipError_t launch_row_dim(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream) {
+  if (p.add_rem) return dtype_is_f16 ? launch_row_t<_Float16, DH, true>(p, max_tiles, stream) : launch_row_t<__bf16, DH, true>(p, max_tiles, stream);
+  return dtype_is_f16 ? launch_row_t<_Float16, DH, false>(p, max_tiles, stream) : launch_row_t<__bf16, DH, false>(p, max_tiles, stream);
+}
 hipError_t launch_bwd_row(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream) {
-  if (p.add_rem) return dtype_is_f16 ? launch_row_t<_Float16, true>(p, max_tiles, stream) : launch_row_t<__bf16, true>(p, max_tiles, stream);
-  return dtype_is_f16 ? launch_row_t<_Float16, false>(p, max_tiles, stream) : launch_row_t<__bf16, false>(p, max_tiles, stream);
+  return p.head_dim == 128 ? launch_row_dim<128>(p, dtype_is_f16, max_tiles, stream) : launch_row_dim<64>(p, dtype_is_f16, max_tiles, stream);
 }
 
 }  // namespace sba

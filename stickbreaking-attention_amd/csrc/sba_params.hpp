@@ -62,6 +62,9 @@ struct SchedParams {
 constexpr int kInlineSeqs = 64;
 
 constexpr int kRowTileRows = 256;      // query rows per tile of the backward on row tiles
+// Its queue, of 8, for head 0 of the sequence with this rank (the list holds the longest first); head h's is (this + h) % 8.  If the heads do
+// not fill the queues evenly, the fuller ones are others for the next sequence, in an order that goes forth and back (a Gray code).
+__host__ __device__ inline int row_queue(int rank, int heads) { return heads & 7 ? ((rank ^ rank >> 1) * (heads & 7)) & 7 : 0; }
 
 struct FwdParams {
   TensorRef q, k, v, o;

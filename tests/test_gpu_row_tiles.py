@@ -1,4 +1,4 @@
-"""GPU tests of the backward on row tiles (csrc/sba_bwd_row.hip), which runs from 64 K rows x heads on at head_dim 128: many heads over
+"""GPU tests of the backward on row tiles (csrc/sba_bwd_row.hip), which runs from 64 K rows x heads on at head_dim 64 and 128: many heads over
 few rows, so that the edges of its tiles (256 rows, 32 per wave), key blocks (32) and queues are reached with an oracle in reach.
 
 Against the float64 oracle on some heads (the bar of test_gpu_parity.py), against the dQ and dK/dV kernels on all (two orders of
@@ -52,13 +52,14 @@ def gradients(native, mode, dev, cu, lengths, c):
 
 
 @pytest.mark.parametrize("label,H,lengths,c", CASES, ids=[c[0] for c in CASES])
-def test_against_oracle_and_two_kernels(gpu_device, label, H, lengths, c):
+@pytest.mark.parametrize("D", [128, 64])
+def test_against_oracle_and_two_kernels(gpu_device, D, label, H, lengths, c):
     from stickbreaking_attention import _native
 
     dtype, T, pad = c.get("dtype", torch.bfloat16), sum(lengths), c.get("pad", 0)
     assert T * H >= 64 << 10      # (fewer do not reach the kernel)
     g = torch.Generator().manual_seed(len(label) + H)
-    q, k, v, do = (torch.randn(H, T + pad, 128, generator=g) for _ in range(4))
+    q, k, v, do = (torch.randn(H, T + pad, D, generator=g) for _ in range(4))
     q, k = q * c.get("qk_std", 1.0), k * c.get("qk_std", 1.0)
     host = [t.to(dtype) for t in (q, k, v, do, torch.randn(H, T + pad, generator=g))]
     dev = [t.transpose(0, 1).contiguous().to(gpu_device).transpose(0, 1) if c.get("token_major") and t.dim() == 3 else t.to(gpu_device) for t in host]

@@ -42,10 +42,15 @@ def test_partial_results_of_neighbours_do_not_overlap():
 
 @pytest.mark.parametrize("heads", [1, 4, 7, 8, 12, 20, 32])
 def test_every_head_is_in_one_queue(heads):
-    per_slot = cdiv(heads, 8)
-    for seq in range(9):
-        got = sorted(h for q in range(8) for i in range(per_slot) for h in [((q - seq * heads) % 8) + 8 * i] if h < heads)
-        assert got == list(range(heads))
+    """... of every sequence, and 8 sequences in a row fill the queues alike."""
+    per_slot, units = cdiv(heads, 8), [0] * 8
+    for rank in range(16):
+        first = (rank ^ rank >> 1) * heads      # (Gray code)
+        by_queue = [[h for i in range(per_slot) for h in [((q - first) % 8) + 8 * i] if h < heads] for q in range(8)]
+        assert sorted(sum(by_queue, [])) == list(range(heads))
+        units = [u + len(b) for u, b in zip(units, by_queue)]
+        if rank % 8 == 7:
+            assert max(units) - min(units) <= heads % 8, (rank, units)
 
 
 @pytest.fixture(scope="module")

@@ -13,10 +13,57 @@
 // log A = x - softplus2(x) + cumsum(-softplus2) needs three.  The product can only underflow where A itself is
 // below 2^-126, and row_stat = log2(prod) is taken once per row at the end.
 #include "sba_device.hpp"
+#include "sba_dma.hpp"
 #include "sba_params.hpp"
 #include "sba_sched.hpp"
 
 namespace sba {
+
+// What a wave's rows come to: o (and the remainder's share of it), rem, row_stat.  oacc[dt][r]: query row 8*(r/4) + 4*half + r%4 of this
+// wave, column 32*dt + col; prod: the remainder of row w_first + col.
+template <typename T, int DH, int kLoad>
+__device__ __forceinline__ void store_rows(const FwdParams& p, const Tile& tile, int head, int w_first, int half, int col, const T* vb,
+                                           const f32x16 (&oacc)[DH / 32], float prod) {
+  constexpr bool kFast = kLoad != kLoadScalar;
+  constexpr int kDTiles = DH / 32;
+  const int L = tile.seq_len, D = p.head_dim, qi = w_first + col;
+  T* ob = (T*)p.o.ptr + tile.seq_id * p.o.sb + head * p.o.sh + (int64_t)tile.seq_start * p.o.st;
+  if (p.add_rem) {
+    // o + rem * v (the step callers of the reference apply to its outputs, tests/test_varlen.py:103): the row's
+    // remainder is held by the lane whose query it is.
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const int lr = 8 * (r >> 2) + 4 * half + (r & 3);
+      const int row = w_first + lr;
+      const float rem_row = __shfl(prod, lr);
+#pragma unroll
+      for (int dt = 0; dt < kDTiles; dt++) {
+        const int d = 32 * dt + col;
+        if (row < L && d < D)
+          ob[(int64_t)row * p.o.st + d] = (T)(oacc[dt][r] + rem_row * (float)vb[(int64_t)row * p.v.st + d]);
+      }
+    }
+  } else if (kFast) {
+    const RowSink<T> sink = make_row_sink<T>(ob, p.o.st, L, D);
+#pragma unroll
+    for (int dt = 0; dt < kDTiles; dt++) store_acc_tile<T>(sink, oacc[dt], 1.f, w_first, 32 * dt, half, col, kLoad == kLoadPadded ? D : DH);
+  } else {
+#pragma unroll
+    for (int dt = 0; dt < kDTiles; dt++) {
+      const int d = 32 * dt + col;
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        const int row = w_first + 8 * (r >> 2) + 4 * half + (r & 3);
+        if (row < L && d < D) ob[(int64_t)row * p.o.st + d] = (T)oacc[dt][r];
+      }
+    }
+  }
+  if (half == 0 && qi < L) {
+    T* rb = (T*)p.rem.ptr + tile.seq_id * p.rem.sb + head * p.rem.sh + (int64_t)(tile.seq_start + qi) * p.rem.st;
+    *rb = (T)prod;
+    p.row_stat[tile.seq_id * p.stat_sb + head * p.stat_sh + tile.seq_start + qi] = fast_log2(prod);
+  }
+}
 
 // kCarryOnly: only the products of (1 - sigma) above every sub-tile are rebuilt (into `carry`), for a backward whose
 // forward did not keep them: no V, no P V, no outputs.
@@ -173,50 +220,147 @@ __global__ __launch_bounds__(kThreads, kMinWaves) void fwd_kernel(FwdParams p) {
   }
 
   if (kCarryOnly) return;
-  // Epilogue.  oacc[dt][r]: query row 8*(r/4) + 4*half + r%4 of this wave, column 32*dt + col.
-  T* ob = (T*)p.o.ptr + tile.seq_id * p.o.sb + head * p.o.sh + (int64_t)tile.seq_start * p.o.st;
-  if (p.add_rem) {
-    // o + rem * v (the step callers of the reference apply to its outputs, tests/test_varlen.py:103): the row's
-    // remainder is held by the lane whose query it is.
-#pragma unroll
-    for (int r = 0; r < 16; r++) {
-      const int lr = 8 * (r >> 2) + 4 * half + (r & 3);
-      const int row = w_first + lr;
-      const float rem_row = __shfl(prod, lr);
-#pragma unroll
-      for (int dt = 0; dt < kDTiles; dt++) {
-        const int d = 32 * dt + col;
-        if (row < L && d < D)
-          ob[(int64_t)row * p.o.st + d] = (T)(oacc[dt][r] + rem_row * (float)vb[(int64_t)row * p.v.st + d]);
+  store_rows<T, DH, kLoad>(p, tile, head, w_first, half, col, vb, oacc, prod);
+}
+
+// The same for aligned rows of 128 elements (kLoadAligned): key tiles of 32 keys come straight into LDS, one ahead of the tile that is
+// worked on, in two buffers: no registers, no LDS writes and one barrier per tile instead of two.
+// What bounds it: per 32 x 32 block 119 vector-ALU instructions (620 cycles) and 16 MFMAs (512 cycles), at three waves per SIMD, which
+// keep one of the two pipes busy 96 % of the time and both 23 %; and the power limit (1.9 GHz).  32 heads x 8 x 4096: 1140 us with tiles
+// through registers, 1100 here.  (head_dim 64 keeps its tiles of 64 keys: 107 us for 12 heads, 16384 tokens, against 112.)
+template <typename T>
+__global__ __launch_bounds__(kThreads, 3) void fwd_dma_kernel(FwdParams p) {
+  typedef typename Elem<T>::vec8 vec8;
+  constexpr int DH = 128, KT = 32, kSteps = DH / 16, kDTiles = DH / 32;
+  constexpr int kPanel = KT * 64, kMat = kDTiles * kPanel, kBuf = 2 * kMat;      // bytes
+  __shared__ __attribute__((aligned(16))) unsigned char lds_raw[2 * kBuf];
+  lds_u8* const lds = (lds_u8*)lds_raw;
+  const int lds_base = __builtin_amdgcn_readfirstlane((int)(uintptr_t)lds);
+
+  if ((int)blockIdx.x < p.sched.service) {
+    forward_service(p.sched, blockIdx.x);
+    return;
+  }
+  int head, slot;
+  xcd_head_tile(blockIdx.x - p.sched.service, p.num_heads, &head, &slot);
+  Tile tile;
+  int64_t r0, r1;
+  if (!forward_tile(p, slot, 0, kBlockQ, &tile, &r0, &r1)) {
+    if (r0 < r1) {      // rows of no sequence: o = rem = 0
+      zero_rows<T>(p.o, head, r0, r1, p.head_dim);
+      for (int64_t r = r0 + threadIdx.x; r < r1; r += kThreads) {
+        ((T*)p.rem.ptr)[head * p.rem.sh + r * p.rem.st] = (T)0;
+        p.row_stat[head * p.stat_sh + r] = 0.f;
       }
     }
-  } else if (kFast) {
-    const RowSink<T> sink = make_row_sink<T>(ob, p.o.st, L, D);
+    return;
+  }
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = lane >> 5, col = lane & 31;
+  const int L = tile.seq_len, q0 = tile.origin, ac = p.attend_current;
+  const T* qb = (const T*)p.q.ptr + tile.seq_id * p.q.sb + head * p.q.sh + (int64_t)tile.seq_start * p.q.st;
+  const T* kb = (const T*)p.k.ptr + tile.seq_id * p.k.sb + head * p.k.sh + (int64_t)tile.seq_start * p.k.st;
+  const T* vb = (const T*)p.v.ptr + tile.seq_id * p.v.sb + head * p.v.sh + (int64_t)tile.seq_start * p.v.st;
+
+  const int last_row = min(q0 + kBlockQ, L) - 1;
+  const int last_key = last_row - 1 + ac;                    // last key any row of this tile can see
+  const int n_kt = last_key < 0 ? 0 : last_key / KT + 1;
+  const int w_first = q0 + wave * 32, w_last = w_first + 31, qi = w_first + col;
+
+  // Tile jt into buffer jt & 1: waves 0 and 1 bring two panels of K each, 2 and 3 of V.  Row m is key mfma_row_to_key32(m): the MFMA's output row.
+  const bool brings_v = wave >= 2;
+  const int panel0 = 2 * (wave & 1), kv_st = (int)((brings_v ? p.v.st : p.k.st) * 2);
+  const u32x4 desc = buffer_desc(brings_v ? vb : kb, (L - 1) * kv_st + 2 * DH);
+  const int voff = mfma_row_to_key32(lane >> 2) * kv_st + panel0 * 64 + (((lane & 3) ^ ((lane >> 4) & 3)) << 4);
+  auto request = [&](int jt) {
+    const int soff = jt * KT * kv_st, dst = lds_base + (jt & 1) * kBuf + wave * (2 * kPanel);
 #pragma unroll
-    for (int dt = 0; dt < kDTiles; dt++) store_acc_tile<T>(sink, oacc[dt], 1.f, w_first, 32 * dt, half, col, kLoad == kLoadPadded ? D : DH);
-  } else {
+    for (int i = 0; i < 2; i++) dma16x2<1024>(dst + i * kPanel, voff, desc, soff + 64 * i, soff + 64 * i + 8 * kv_st);
+  };
+  if (n_kt > 0) request(n_kt - 1);
+  vec8 qf[kSteps];
+  load_operand<T, kLoadAligned>(qf, make_row_source<T, kLoadAligned>(qb, p.q.st, L, DH), qi, half);
+
+  f32x16 oacc[kDTiles];
 #pragma unroll
-    for (int dt = 0; dt < kDTiles; dt++) {
-      const int d = 32 * dt + col;
+  for (int dt = 0; dt < kDTiles; dt++)
 #pragma unroll
-      for (int r = 0; r < 16; r++) {
-        const int row = w_first + 8 * (r >> 2) + 4 * half + (r & 3);
-        if (row < L && d < D) ob[(int64_t)row * p.o.st + d] = (T)oacc[dt][r];
+    for (int r = 0; r < 16; r++) oacc[dt][r] = 0.f;
+  float prod = 1.f;    // prod over the keys already swept of (1 - sigma): both half-waves hold the same value
+  const int64_t n_qt = (L + kBlockQ - 1) / kBlockQ;
+  float* carry = p.carry ? p.carry + (int64_t)head * p.carry_head_stride + tile.carry_base : nullptr;
+  // Slots of sub-tile u: a uniform base and this lane's row within the tile.  The products are read per 64 keys by backward kernels
+  // that sweep as many at a time: a sweep that ends on the lower half also records the (empty) product above the upper half.
+  const uint32_t lrow = wave * 32 + col;
+  auto carry_row = [&](int u) { return carry + carry_offset(u, n_qt) + (q0 - kBlockQ * (u >> 2)); };
+  if (carry && half == 0 && (n_kt & 1)) carry_row(n_kt)[lrow] = 1.f;
+  const int s15 = lane & 15, g = (lane >> 4) & 1;
+  const int row_a = col * 64 + ((half ^ ((col >> 2) & 3)) << 4);                                                   // odd steps: ^ 32
+  const int tr_k = (4 * half + (s15 >> 2)) * 64 + (((2 * g + ((s15 >> 1) & 1)) ^ half) << 4) + 8 * (s15 & 1);      // the next 4 rows: (^ 32) + 512
+  vm_wait<0>();
+  lds_barrier();
+  for (int jt = n_kt - 1; jt >= 0; --jt) {
+    const int j0 = jt * KT;
+    if (jt > 0) request(jt - 1);
+    if (carry && half == 0) carry_row(jt)[lrow] = prod;       // for the backward: the product over the keys between this tile and the row
+    if (j0 <= w_last - 1 + ac) {                              // (else nothing visible to this wave yet)
+      const bool diagonal = (j0 + KT - 1) > (w_first - 1 + ac);
+      lds_u8* kt = lds + (jt & 1) * kBuf;
+      // The two MFMA phases of a step run at raised wave priority, the element-wise math at the default: a wave whose
+      // next MFMA is ready then gets the issue port ahead of the other waves' vector-ALU streams.
+      __builtin_amdgcn_s_setprio(3);
+      f32x16 s[1];
+#pragma unroll
+      for (int r = 0; r < 16; r++) s[0][r] = 0.f;
+      lds_u8* k0 = kt + row_a;
+      lds_u8* k1 = kt + (row_a ^ 32);
+      auto k_op = [&](int kk) { return lds_load<vec8>(((kk & 1) ? k1 : k0) + (kk >> 1) * kPanel); };
+      vec8 a[4];
+#pragma unroll
+      for (int kk = 0; kk < 4; kk++) a[kk] = k_op(kk);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int kk = 0; kk < kSteps; kk++) {
+        s[0] = Elem<T>::mfma(a[kk & 3], qf[kk], s[0]);
+        if (kk + 4 < kSteps) a[kk & 3] = k_op(kk + 4);
+        __builtin_amdgcn_sched_barrier(0);
       }
+      __builtin_amdgcn_s_setprio(0);
+      Weights<16> w;
+      const int lim = qi + ac - j0 - 16 * half;               // key R is visible iff R < lim
+      if (diagonal) w.template front<true>(s, p.scale_log2, lim); else w.template front<false>(s, p.scale_log2, lim);
+      const float run = w.run;
+      const float oth = other_half(run, half);
+      const float seed = half ? prod : prod * oth;            // the upper half-wave holds the higher keys, which come first in the sweep
+      prod = (prod * oth) * run;
+      w.back(seed);
+      __builtin_amdgcn_s_setprio(3);
+      lds_u8* t0 = kt + kMat + tr_k;
+      lds_u8* t1 = kt + kMat + (tr_k ^ 32) + 512;
+#pragma unroll
+      for (int c = 0; c < 2; c++) {
+        u32x4 av;
+#pragma unroll
+        for (int i = 0; i < 4; i++) av[i] = pack2<T>(w.t[8 * c + 2 * i], w.t[8 * c + 2 * i + 1]);
+#pragma unroll
+        for (int dt = 0; dt < kDTiles; dt++)
+          oacc[dt] = Elem<T>::mfma(as_vec8<T>(av), tr_pair<T>(t0 + 1024 * c + dt * kPanel, t1 + 1024 * c + dt * kPanel), oacc[dt]);
+      }
+      __builtin_amdgcn_s_setprio(0);
+    }
+    if (jt > 0) {      // the next tile is in LDS (the product just recorded may still be on its way), and this one has been read
+      if (carry) vm_wait<1>(); else vm_wait<0>();
+      lds_barrier();
     }
   }
-  if (half == 0 && qi < L) {
-    T* rb = (T*)p.rem.ptr + tile.seq_id * p.rem.sb + head * p.rem.sh + (int64_t)(tile.seq_start + qi) * p.rem.st;
-    *rb = (T)prod;
-    p.row_stat[tile.seq_id * p.stat_sb + head * p.stat_sh + tile.seq_start + qi] = fast_log2(prod);
-  }
+  store_rows<T, DH, kLoadAligned>(p, tile, head, w_first, half, col, vb, oacc, prod);
 }
 
 template <typename T, bool kCarryOnly>
 static hipError_t launch_fwd_t(const FwdParams& p, int max_tiles, hipStream_t stream) {
   const dim3 grid((unsigned)(max_tiles * p.num_heads + p.sched.service)), block(kThreads);
   if (p.load == kLoadAligned) {
-    if (p.head_dim == 128) hipLaunchKernelGGL((fwd_kernel<T, 128, kLoadAligned, 32, 3, kCarryOnly>), grid, block, 0, stream, p);
+    if (p.head_dim == 128 && !kCarryOnly) hipLaunchKernelGGL((fwd_dma_kernel<T>), grid, block, 0, stream, p);
+    else if (p.head_dim == 128) hipLaunchKernelGGL((fwd_kernel<T, 128, kLoadAligned, 32, 3, true>), grid, block, 0, stream, p);
     else hipLaunchKernelGGL((fwd_kernel<T, 64, kLoadAligned, 64, 2, kCarryOnly>), grid, block, 0, stream, p);
   } else if (p.load == kLoadPadded) {
     if (p.head_dim > 64) hipLaunchKernelGGL((fwd_kernel<T, 128, kLoadPadded, 32, 3, kCarryOnly>), grid, block, 0, stream, p);

@@ -46,7 +46,7 @@ extern "C" {
 #define SBA_SCHED_OK 0
 #define SBA_SCHED_BAD_CU_SEQLENS 1
 #define SBA_SCHED_CARRY_TOO_SMALL 2
-#define SBA_CHAIN_TIMEOUT 3        /* one-kernel backward: a workgroup gave up waiting for the key tile below its own */
+#define SBA_CHAIN_TIMEOUT 3        /* one-kernel backward: a workgroup gave up waiting for the tile before its own */
 #define SBA_CHAIN_XCD_MISMATCH 4   /* one-kernel backward: the workgroups of a head did not share an XCD */
 
 /* Size of the static device scratch behind sba_fwd_static. */

@@ -65,13 +65,13 @@ POISON = os.environ.get("SBA_DEBUG_POISON", "0") == "1"
 # and raise on a schedule the device refused.  Without it a bad ``cu_seqlens`` that only exists on the device yields
 # all-zero outputs and gradients and no error.
 DEBUG_CHECK = os.environ.get("SBA_DEBUG_CHECK", "0") == "1"
-# SbaArgs.backward_kernels: 0 = the library chooses, 1 = dQ then dK/dV, 2 = one chained kernel where it applies.
+# SbaArgs.backward_kernels: 0 = the library chooses, 1 = dQ then dK/dV, 2 = one kernel where it applies.
 BACKWARD_KERNELS = int(os.environ.get("SBA_BACKWARD_KERNELS", "0"))
-# Attention kernels the last traced backward ran: 1 (chained) or 2 (set when TRACE_EVENTS is).
+# Kernels the last traced backward ran behind its schedule, 1 or 2 (set when TRACE_EVENTS is).
 LAST_BWD_KERNELS = 0
 _STATUS_TEXT = {1: "cu_seqlens is not a non-decreasing sequence within [0, total_tokens] (or its leading entry is not 0)",
                 2: "the carry buffer is too small for these sequence lengths (max_seqlens understated?)",
-                3: "one-kernel backward: a workgroup gave up waiting for the key tile below its own",
+                3: "one-kernel backward: a workgroup gave up waiting for the tile before its own",
                 4: "one-kernel backward: the workgroups of a head did not share an XCD"}
 
 

@@ -91,3 +91,14 @@ def test_against_oracle_and_two_kernels(gpu_device, D, label, H, lengths, c):
         ulp = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10
         excess = (x - y).abs() - 2 * torch.maximum(torch.full_like(y, 2e-2), y.abs() * ulp)
         assert excess.max().item() <= 0, f"{label}: {name} against the two kernels, {excess.max().item():.3e} beyond twice the bound"
+
+
+@pytest.mark.parametrize("save_carry", [True, False])
+@pytest.mark.parametrize("case", [(32, 128, [1300, 2100], torch.bfloat16), (64, 64, [1100], torch.bfloat16), (20, 64, [1200, 1700, 3400], torch.float16)],
+                         ids=["cleared-with-the-schedule", "head-dim-64", "ranked-queues"])
+def test_both_passes_in_a_graph(gpu_device, monkeypatch, case, save_carry):
+    """Queues and counters are cleared anew by every replay: against the same calls made eagerly, bit for bit."""
+    import test_gpu_prepared_schedule as prepared
+
+    monkeypatch.setitem(prepared.CASES, "row tiles", case)
+    prepared.test_both_passes_in_a_graph(gpu_device, monkeypatch, "row tiles", save_carry)

@@ -628,7 +628,8 @@ __device__ __forceinline__ bool fwd_f32_rows(const FwdParams& p, const Tile& til
   return E::kSplit && any_odd(odd, stored | staged);
 }
 
-// (Width 96 keeps three waves per SIMD by spilling four registers; 177 registers and two waves take 4 % of a pass more.)
+// (Width 96 keeps three waves per SIMD by spilling up to 29 registers: forward, 12 heads x 80 148 us, with two waves 167; x 96 165 and 167;
+// padded pieces, x 95 165 and 172, but 4 heads 85 and 77.)
 template <int DH, int kMode>
 __global__ __launch_bounds__(kThreads, DH == 96 ? 3 : 2) void fwd_f32_kernel(FwdParams p) {
   __shared__ __attribute__((aligned(16))) float lds[kRowsF32<DH, kMode, 1>];      // Q rows and the waves' scratch, then the final sums

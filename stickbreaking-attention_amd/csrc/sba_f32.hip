@@ -2,9 +2,12 @@
 //
 // Products.  An fp32 number is the sum of three bf16 numbers; of the nine products of two such triples the six that matter are formed
 // on the bf16 matrix instruction (v_mfma_f32_32x32x16_bf16: exact products, fp32 sums), which takes 192 cycles for a 32 x 32 x 16 block
-// where v_mfma_f32_32x32x2_f32 takes 512.  The result is the more accurate one (fewer roundings of the sum; 126 cases of 7
-// head_dims against float64, rms error of o, dq, dk, dv 0.80 to 0.87 of the fp32 instruction's).  Workgroups that meet numbers
-// which triples do not hold (see Split) run again on the fp32 instruction.
+// where v_mfma_f32_32x32x2_f32 takes 512.  A sum of three terms or more is the more accurate one (fewer roundings; rms error of a sum of
+// positive products, in 2^-24, triples and fp32 instruction: 0.58 and 0.43 for 1 term, 0.53 and 0.50 for 2, 0.50 and 0.55 for 3, 0.46 and
+// 0.78 for 8, 2.3 and 2.9 for 128).  Fewer terms stay with the fp32 instruction: the first 32 rows of a sequence in the forward and in dQ, its
+// keys that fewer than 32 rows behind their block see in dK/dV, and head_dims 1 and 2.  Against float64, 8 heads, 6 sequences of up to
+// 500 tokens, head_dims 16 to 128, three kinds of values: rms error of o, dq, dk, dv 0.80 to 0.93 of the fp32 instruction's.  Workgroups
+// that meet numbers which triples do not hold (see Split) run again on the fp32 instruction.
 // What bounds it: per 32 x 32 block at head_dim 128 the forward needs 3072 matrix cycles and 1300 vector instructions (5200 cycles), 700 of
 // them to split K and V, which every workgroup of 32 rows does for itself; two waves per SIMD overlap the two to about 70 %.
 // Consequences for the design:
@@ -472,7 +475,7 @@ struct Split {
     }
     return any;
   }
-  // The six products that matter, the small ones first.
+  // The six products that matter, the small ones first.  (m x l twice and l x l are left out, 2^-25 of the product at most.)
   static __device__ __forceinline__ f32x16 six(const vec8 (&a)[3], const vec8 (&b)[3], f32x16 c) {
     c = Elem<__bf16>::mfma(a[2], b[0], c);
     c = Elem<__bf16>::mfma(a[0], b[2], c);
@@ -656,7 +659,7 @@ __global__ __launch_bounds__(kThreads, DH == 96 ? 3 : 2) void fwd_f32_kernel(Fwd
   }
   const int q0 = tile.origin + sub * kF32Rows;
   if (q0 >= tile.seq_len) return;
-  if (p.fp32_products || fwd_f32_rows<Engine<DH, kMode>, DH, kMode>(p, tile, head, q0, lds, xch, rem_lds)) fwd_f32_rows<Plain<DH, kMode>, DH, kMode>(p, tile, head, q0, lds, xch, rem_lds);
+  if (p.fp32_products || q0 == 0 || fwd_f32_rows<Engine<DH, kMode>, DH, kMode>(p, tile, head, q0, lds, xch, rem_lds)) fwd_f32_rows<Plain<DH, kMode>, DH, kMode>(p, tile, head, q0, lds, xch, rem_lds);
 }
 
 template <class E, int DH, int kMode>
@@ -768,7 +771,7 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dq_f32_kernel(BwdParams p) {
   const Tile tile = p.q_tiles[slot];
   const int q0 = tile.origin + sub * kF32Rows;
   if (q0 >= tile.seq_len) return;
-  if (p.fp32_products || bwd_dq_f32_rows<Engine<DH, kMode>, DH, kMode>(p, tile, head, q0, lds, xch)) bwd_dq_f32_rows<Plain<DH, kMode>, DH, kMode>(p, tile, head, q0, lds, xch);
+  if (p.fp32_products || q0 == 0 || bwd_dq_f32_rows<Engine<DH, kMode>, DH, kMode>(p, tile, head, q0, lds, xch)) bwd_dq_f32_rows<Plain<DH, kMode>, DH, kMode>(p, tile, head, q0, lds, xch);
 }
 
 template <class E, int DH>
@@ -879,7 +882,7 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dkv_f32_kernel(BwdParams p) {
   const Tile tile = p.k_tiles[slot];
   const int k0 = tile.origin + sub * kF32Rows;
   if (k0 >= tile.seq_len) return;
-  if (p.fp32_products || bwd_dkv_f32_keys<Engine<DH, kMode>, DH, kMode>(p, tile, head, k0, lds)) bwd_dkv_f32_keys<Plain<DH, kMode>, DH, kMode>(p, tile, head, k0, lds);
+  if (p.fp32_products || k0 + 2 * kF32Rows > tile.seq_len || bwd_dkv_f32_keys<Engine<DH, kMode>, DH, kMode>(p, tile, head, k0, lds)) bwd_dkv_f32_keys<Plain<DH, kMode>, DH, kMode>(p, tile, head, k0, lds);
 }
 
 // head_dim is rounded up to a multiple of 32 (the matrix cycles go by that); the exact variants skip every test of a
@@ -906,7 +909,7 @@ static hipError_t by_head_dim(int D, int load, F&& f) {
 //   head_dim  64   4 heads, 448 tokens in sequences of up to 256 (112 workgroups)  kernels 45.4 / 40.6
 //             64   1 head, 6143 tokens in sequences of up to 2048 (240)   196 / 208        128: 319 / 360
 //             32   1 head, the same                                       139 / 130        2 heads (16) 141 / 147, 4 heads 151 / 177
-static bool few_workgroups(int D, int64_t tiles) { return tiles * kF32Split <= (D <= 32 ? 256 : 128); }
+static bool few_workgroups(int D, int64_t tiles) { return tiles * kF32Split <= (D <= 32 ? 256 : 128) || D <= 2; }
 
 hipError_t launch_fwd_f32(const FwdParams& call, int max_tiles, hipStream_t stream) {
   FwdParams p = call;

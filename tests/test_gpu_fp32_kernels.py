@@ -33,6 +33,44 @@ def test_fp32_tile_edges_against_oracle(gpu_device, D, qk_std, attend_current, a
         assert torch.equal(a, b), f"{n}: two runs differ"
 
 
+@pytest.mark.parametrize("D", [20, 64, 96, 128])
+def test_single_products_are_rounded_once(gpu_device, D):
+    """Sequences of two tokens: every contraction over keys or rows has one term.  Column 0 of q, k, v and d_o is 1, so column 0 of an
+    output is the other factor, and the rest are its products rounded to fp32: within 2^-24 of them."""
+    H, n = 8, 40      # (1312 workgroups: products of triples elsewhere)
+    (q, k, v, do, drem), _, cu = small_case(H, D, [2] * n, torch.float32, seed=D)
+    for t in (q, k, v, do):
+        t[..., 0] = 1
+    dev = [t.to(gpu_device) for t in (q, k, v, do, drem)]
+    got = dict(zip(NAMES, run_varlen(dev[0], dev[1], dev[2], cu.to(gpu_device), [2] * n, False, False, dev[3], dev[4], scale=1.0)))
+    for name, vec, row, other in (("o", v, 1, 0), ("dq", k, 1, 0), ("dk", q, 0, 1), ("dv", do, 0, 1)):
+        out = got[name].detach().double().cpu()[:, row::2]
+        exact = out[..., :1] * vec.double()[:, other::2]
+        worst = ((out - exact).abs() * 2.0 ** 24 - exact.abs()).max().item()
+        print(f"D={D} {name}: {worst:.2e}", flush=True)
+        assert worst <= 0, name
+
+
+@pytest.mark.parametrize("values", ["normal", "slow"])
+@pytest.mark.parametrize("D", [3, 16, 64, 128])
+def test_triples_are_no_less_accurate_than_fp32_products(gpu_device, D, values):
+    """Eight heads together form their products of triples, two at a time (52 workgroups) of fp32 numbers: the error against float64, in
+    norm, may not be larger than 1.02 times theirs (a rms over 8 x 1200 rows x D numbers is known to about 1 %; measured: 0.80 to 0.97)."""
+    lengths, H = [40, 97, 33, 65, 129, 50, 71, 200, 300, 215], 8
+    (q, k, v, do, drem), _, cu = small_case(H, D, lengths, torch.float32, seed=D)
+    if values == "slow":
+        q, k, v = 0.25 * (q + 1), 0.25 * (k - 1), 0.25 * v
+    dev = [t.to(gpu_device) for t in (q, k, v, do, drem)]
+    run = lambda h: run_varlen(*(t[h] for t in dev[:3]), cu.to(gpu_device), lengths, False, False, dev[3][h], dev[4][h])
+    triples = run(slice(0, H))
+    parts = [run(slice(h, h + 2)) for h in range(0, H, 2)]
+    ref = orc.varlen_stream(*(t.double() for t in (q, k, v)), cu, do=do.double(), drem=drem.double(), dtype=torch.float64)
+    for i, n in enumerate(NAMES):
+        a, b = ((t.detach().double().cpu() - ref[i]).norm().item() for t in (triples[i], torch.cat([p[i] for p in parts])))
+        print(f"D={D} {values} {n}: error of triples / of fp32 products {a / b:.3f}", flush=True)
+        assert a <= 1.02 * b, n
+
+
 @pytest.mark.parametrize("D", [64, 128])
 def test_odds_below_the_smallest_normal_number(gpu_device, D):
     """Logits of -92 to -86, odds of 2^-133 to 2^-124.  A logit in octaves has an error of up to 2^-17.9 (133 octaves, two

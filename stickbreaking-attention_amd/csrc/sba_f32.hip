@@ -315,8 +315,8 @@ __device__ __forceinline__ bool reduce_store_f32(float* lds, const f32x16 (&acc)
     for (int w = 0; w < kWaves; w++) v += *reinterpret_cast<const f32x4*>(lds + (w * 32 + row) * kStride + d0);
 #pragma unroll
     for (int t = 0; t < 4; t++) {
-      v[t] *= E::kDown;
-      if (kMode == kF32Exact || d0 + t < D) odd |= E::odd(v[t]);
+      if (kMode == kF32Exact || d0 + t < D) odd |= E::odd_sum(v[t]);
+      v[t] *= E::kDown * E::kDown;
     }
     v *= scale;
     float* o = out + (int64_t)row * stride + d0;
@@ -336,14 +336,14 @@ __device__ __forceinline__ bool reduce_store_f32(float* lds, const f32x16 (&acc)
 
 // The two ways to form the products.  x: the registers of the streamed operand.
 //   stage    : 32 rows into LDS as the resident operand of score() (kRows: as its A operand, whose row m is key mfma_row_to_key32(m))
-//   score    : (rows in x) . (resident rows), contracted over head_dim; x then holds `next`
-//   contract : acc[dt] += a . x, contracted over 32 rows; x then holds `next` if `more`
+//   score    : (rows in x) . (resident rows), contracted over head_dim (kGrad: dP, times 1 / kDown); x then holds `next`
+//   contract : acc[dt] += a . x, contracted over 32 rows, a times 1 / kDown, the result times 1 / kDown^2; x then holds `next` if `more`
 template <int DH, int kMode>
 struct Plain {
   typedef Operand<DH, kMode> Op;
   static constexpr bool kSplit = false;
   static constexpr float kUp = 1.f, kDown = 1.f;
-  static __device__ __forceinline__ bool odd(float) { return false; }
+  static __device__ __forceinline__ bool odd_sum(float) { return false; }
   static constexpr int kResident = 32 * (DH + 4), kTurn = Parts<DH>::kTurn;      // floats
   static __device__ __forceinline__ int out_col(int dt, int col) { return sba::out_col<DH>(dt, col); }
   static __device__ __forceinline__ Op op(const float* base, int64_t stride, int first, int rows_total, int half, int col, int D) {
@@ -356,7 +356,7 @@ struct Plain {
     stage_rows<DH, kMode>(lds, s, D);
     return false;
   }
-  template <bool kLdsIsA, bool kNextScore>
+  template <bool kLdsIsA, bool kNextScore, bool kGrad>
   static __device__ __forceinline__ f32x16 score(float (&x)[DH / 2], float* turn, const float* resident, int half, int col, const Op& next,
                                                  const Op& late, bool has_late, uint64_t& odd) {
     const int key = mfma_row_to_key32(col);
@@ -386,9 +386,15 @@ __device__ __forceinline__ Split3 split3(float x0, float x1) {
 }
 
 // Products of triples.  What they do not hold: numbers beyond the largest bf16 number (and infinities), whose triples are not numbers,
-// and the last bits of numbers below 2^-109.  The latter matter only where a result is as small or the partner is as large, so a
-// workgroup calls for the fp32 instruction (`odd`) if a score is not a number, if an element of its resident rows is outside
-// 2^-80 .. 2^80, or if one of its results is.  Weights and their gradients, which may be that small in sums that are not, are scaled by 2^24.
+// and the last bits of numbers below 2^-102, whose last parts would be no normal numbers.
+//   Resident rows (Q, dO; K, V): a workgroup calls for the fp32 instruction (`odd`) if an element is outside 2^-80 .. 2^80.
+//   Streamed rows: the operand of dP and those of the contractions are scaled by 2^24 before they are split (kUp), and so are the weights
+//     and their gradients they are contracted with: no fp32 number loses a bit.  dP and the results are scaled back.  What is too large
+//     for that makes infinities or no numbers, in results that rows or keys of the workgroup store: they call for the fp32 instruction.
+//   The operand of the logits is not scaled: a part lost there is below 2^-126, times 2^80 of the resident row and 128 columns 2^-39,
+//     times the logit scale (at most 2^10 here, see fp32_products_only) nothing that a logit's effect could show.  Logits that are no
+//     numbers call for the fp32 instruction, infinite ones saturate as they do there.
+// Cost of the scaling: 12 heads x 128, 6143 tokens, forward 230 -> 230 us, dQ 315 -> 323, dK/dV 402 -> 408.
 // The residuals are taken with shifts and subtractions: v_dot2_f32_bf16 does it in one instruction instead of two, but not beside
 // MFMAs (12 heads, 6143 tokens: 828 us against 800).
 template <int DH, int kMode>
@@ -397,6 +403,7 @@ struct Split {
   static constexpr bool kSplit = true;
   static constexpr float kUp = 0x1p24f, kDown = 0x1p-24f;
   static __device__ __forceinline__ bool odd(float x) { return x != 0.f && !(fabsf(x) >= 0x1p-80f && fabsf(x) <= 0x1p80f); }
+  static __device__ __forceinline__ bool odd_sum(float x) { return !(fabsf(x) < INFINITY); }
   static constexpr int NB = DH / 32, kPlane = 2048, kPanel = 3 * kPlane;      // bytes; a panel: 3 planes of [32 rows][32 columns]
   static constexpr int kResident = NB * kPanel / 4, kTurn = kPanel / 4;       // floats
   static __device__ __forceinline__ int out_col(int dt, int col) { return NB * col + dt; }
@@ -453,8 +460,8 @@ struct Split {
   static __device__ __forceinline__ void fill(float (&x)[DH / 2], const Op& o) { o.template refill<kScore>(x, 0, DH / 2); }
 
   // Panels: 64-byte rows whose 16-byte chunks are XORed with (row >> 2) & 3: no bank is met twice by row reads.
-  static __device__ __forceinline__ void put(unsigned char* at, float a, float b, float c, float d) {
-    const Split3 u = split3(a, b), v = split3(c, d);
+  static __device__ __forceinline__ void put(unsigned char* at, float a, float b, float c, float d, float up = 1.f) {
+    const Split3 u = split3(up * a, up * b), v = split3(up * c, up * d);
     *reinterpret_cast<u32x2*>(at) = u32x2{u.h, v.h};
     *reinterpret_cast<u32x2*>(at + kPlane) = u32x2{u.m, v.m};
     *reinterpret_cast<u32x2*>(at + 2 * kPlane) = u32x2{u.l, v.l};
@@ -484,7 +491,7 @@ struct Split {
     c = Elem<__bf16>::mfma(a[0], b[1], c);
     return Elem<__bf16>::mfma(a[0], b[0], c);
   }
-  template <bool kLdsIsA, bool kNextScore>
+  template <bool kLdsIsA, bool kNextScore, bool kGrad>
   static __device__ __forceinline__ f32x16 score(float (&x)[DH / 2], float* turn, const float* resident, int half, int col, const Op& next,
                                                  const Op&, bool, uint64_t& odd) {
     f32x16 acc = zero16();
@@ -500,7 +507,7 @@ struct Split {
       for (int i = 0; i < 4; i++) {
         const int w = kLdsIsA ? (w0 ^ (32 * (i & 1))) + 512 * i : (w0 ^ (16 * (i >> 1))) + 1024 * (i & 1) + 256 * (i >> 1);
         const float* y = x + 16 * p + 4 * i;
-        put(mine + w, y[0], y[1], y[2], y[3]);
+        put(mine + w, y[0], y[1], y[2], y[3], kGrad ? kUp : 1.f);
       }
       next.template refill<kNextScore>(x, 16 * p, 16 * p + 16);
       __builtin_amdgcn_sched_barrier(0);
@@ -517,8 +524,10 @@ struct Split {
         acc = six(a, b, acc);
       }
     }
+    if (!kGrad) {      // (dP that is not a number makes results that are none)
 #pragma unroll
-    for (int r = 0; r < 16; r += 2) odd |= __ballot(__builtin_isunordered(acc[r], acc[r + 1]));
+      for (int r = 0; r < 16; r += 2) odd |= __ballot(__builtin_isunordered(acc[r], acc[r + 1]));
+    }
     return acc;
   }
   template <bool kNextScore>
@@ -541,7 +550,7 @@ struct Split {
 #pragma unroll
       for (int dt = 0; dt < NB; dt++) {
         vec8 bv[3];
-        planes([&](int t) { return x[(8 * i + t) * NB + dt]; }, bv);
+        planes([&](int t) { return kUp * x[(8 * i + t) * NB + dt]; }, bv);
         acc[dt] = six(av, bv, acc[dt]);
       }
       next.template refill<kNextScore>(x, 8 * NB * i, 8 * NB * (i + 1));
@@ -598,7 +607,7 @@ __device__ __forceinline__ bool fwd_f32_rows(const FwdParams& p, const Tile& til
     float beta[16], pe[16];
     float run = 1.f, oth = 1.f;
     if (U >= 0) {
-      const f32x16 s = E::template score<false, false>(x, turn, lds, half, col, v_of(U), k_of(U), t > 0, odd);
+      const f32x16 s = E::template score<false, false, false>(x, turn, lds, half, col, v_of(U), k_of(U), t > 0, odd);
       run = sticks_f32(s, p.scale_log2, qi + ac - 32 * U - 16 * half, beta, pe);
       oth = other_half(run, half);
     }
@@ -714,8 +723,8 @@ __device__ __forceinline__ bool bwd_dq_f32_rows(const BwdParams& p, const Tile& 
     const bool active = U < n_sub;
     if (active) {
       const float prod_in = carry[cslot];
-      const f32x16 s = E::template score<false, true>(x, turn, lds, half, col, v_of(U), k_of(U), t > 0, odd);
-      const f32x16 dp = E::template score<false, false>(x, turn, lds + E::kResident, half, col, k_of(U), k_of(U), false, odd);
+      const f32x16 s = E::template score<false, true, false>(x, turn, lds, half, col, v_of(U), k_of(U), t > 0, odd);
+      const f32x16 dp = E::template score<false, false, true>(x, turn, lds + E::kResident, half, col, k_of(U), k_of(U), false, odd);
       float pe[16];
       const float run = sticks_f32(s, p.scale_log2, qi < L ? qi + ac - 32 * U - 16 * half : 0, beta, pe);
       const float oth = other_half(run, half);
@@ -723,7 +732,7 @@ __device__ __forceinline__ bool bwd_dq_f32_rows(const BwdParams& p, const Tile& 
       float acc = 0.f;
 #pragma unroll
       for (int R = 0; R < 16; R++) {
-        const float g = beta[R] * (pe[R] * seed) * (dp[R] - drem);
+        const float g = beta[R] * (pe[R] * seed) * fmaf(dp[R], E::kDown, -drem);
         acc += g;
         dz[R] = g - beta[R] * acc;
       }
@@ -826,8 +835,8 @@ __device__ __forceinline__ bool bwd_dkv_f32_keys(const BwdParams& p, const Tile&
     const bool row_ok = qi < L;
     const float prod_in = carry[qi], prefix_in = prefix[qi];
     const float drem = row_ok ? drem_plane[qi] : 0.f;
-    const f32x16 s = E::template score<true, true>(x, turn, lds + Lds::kK, half, col, do_of(b), q_of(b), b < nb - kWaves, odd);
-    const f32x16 dp = E::template score<true, false>(x, turn, lds + Lds::kV, half, col, do_of(b), do_of(b), false, odd);
+    const f32x16 s = E::template score<true, true, false>(x, turn, lds + Lds::kK, half, col, do_of(b), q_of(b), b < nb - kWaves, odd);
+    const f32x16 dp = E::template score<true, false, true>(x, turn, lds + Lds::kV, half, col, do_of(b), do_of(b), false, odd);
     float beta[16], pe[16], dz[16];
     const float run = sticks_f32(s, p.scale_log2, row_ok ? qi + ac - k0 - 16 * half : 0, beta, pe);
     const float oth = other_half(run, half);
@@ -837,7 +846,7 @@ __device__ __forceinline__ bool bwd_dkv_f32_keys(const BwdParams& p, const Tile&
 #pragma unroll
     for (int R = 0; R < 16; R++) {
       const float a = beta[R] * (pe[R] * seed);
-      const float g = a * (dp[R] - drem);
+      const float g = a * fmaf(dp[R], E::kDown, -drem);
       tp[(16 * half + R) * kF32TrStride + col] = a;
       acc += g;
       dz[R] = g - beta[R] * acc;
@@ -909,11 +918,13 @@ static hipError_t by_head_dim(int D, int load, F&& f) {
 //   head_dim  64   4 heads, 448 tokens in sequences of up to 256 (112 workgroups)  kernels 45.4 / 40.6
 //             64   1 head, 6143 tokens in sequences of up to 2048 (240)   196 / 208        128: 319 / 360
 //             32   1 head, the same                                       139 / 130        2 heads (16) 141 / 147, 4 heads 151 / 177
-static bool few_workgroups(int D, int64_t tiles) { return tiles * kF32Split <= (D <= 32 ? 256 : 128) || D <= 2; }
+static bool few_workgroups(int D, int64_t tiles) { return tiles * kF32Split <= (D <= 32 ? 256 : 128); }
+// ... or sums over head_dim that are too short for them, or a logit scale at which the parts that their logits lack would count (see Split).
+static bool fp32_products_only(int D, int64_t tiles, float scale_log2) { return few_workgroups(D, tiles) || D <= 2 || !(fabsf(scale_log2) <= 1024.f); }
 
 hipError_t launch_fwd_f32(const FwdParams& call, int max_tiles, hipStream_t stream) {
   FwdParams p = call;
-  p.fp32_products = few_workgroups(p.head_dim, (int64_t)max_tiles * p.num_heads);
+  p.fp32_products = fp32_products_only(p.head_dim, (int64_t)max_tiles * p.num_heads, p.scale_log2);
   return by_head_dim(p.head_dim, p.load, [&](auto dh, auto mode) {
     hipLaunchKernelGGL((fwd_f32_kernel<decltype(dh)::value, decltype(mode)::value>), dim3((unsigned)(xcd_sub_grid(max_tiles * p.num_heads, kF32Split) + p.sched.service)),
                        dim3(kThreads), 0, stream, p);
@@ -923,7 +934,7 @@ hipError_t launch_fwd_f32(const FwdParams& call, int max_tiles, hipStream_t stre
 
 hipError_t launch_bwd_f32(const BwdParams& call, int max_q_tiles, int max_k_tiles, hipStream_t stream) {
   BwdParams p = call;
-  p.fp32_products = few_workgroups(p.head_dim, (int64_t)max_q_tiles * p.num_heads);
+  p.fp32_products = fp32_products_only(p.head_dim, (int64_t)max_q_tiles * p.num_heads, p.scale_log2);
   int dev = 0, cus = 0;
   const hipError_t e = device_cus(&dev, &cus);
   if (e != hipSuccess) return e;

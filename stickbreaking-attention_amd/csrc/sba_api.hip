@@ -24,7 +24,7 @@ hipError_t launch_fwd_split_carry_only(const FwdParams& p, int dtype_is_f16, int
 hipError_t launch_bwd_dq_split(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
 hipError_t launch_bwd_dkv_split(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
 hipError_t launch_fwd_f32(const FwdParams& p, int max_tiles, hipStream_t stream);
-hipError_t launch_bwd_f32(const BwdParams& p, int max_q_tiles, int max_k_tiles, hipStream_t stream);
+hipError_t launch_bwd_f32(const BwdParams& p, int64_t heads, int max_q_tiles, int max_k_tiles, hipStream_t stream);
 }  // namespace sba
 
 namespace {
@@ -616,7 +616,7 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* 
   hipEvent_t* ev = (hipEvent_t*)a->trace_events;
   if (ev && first && hipEventRecord(ev[0], stream) != hipSuccess) return SBA_ERR_LAUNCH;
   if (a->dtype == SBA_F32) {
-    if (sba::launch_bwd_f32(p, (int)L.max_q_tiles, (int)L.max_k_tiles, stream) != hipSuccess) return SBA_ERR_LAUNCH;
+    if (sba::launch_bwd_f32(p, stat_heads, (int)L.max_q_tiles, (int)L.max_k_tiles, stream) != hipSuccess) return SBA_ERR_LAUNCH;
     if (ev && last && (hipEventRecord(ev[1], stream) != hipSuccess || hipEventRecord(ev[2], stream) != hipSuccess)) return SBA_ERR_LAUNCH;
     return SBA_OK;
   }

@@ -932,9 +932,10 @@ hipError_t launch_fwd_f32(const FwdParams& call, int max_tiles, hipStream_t stre
   });
 }
 
-hipError_t launch_bwd_f32(const BwdParams& call, int max_q_tiles, int max_k_tiles, hipStream_t stream) {
+// `heads`: of the caller's call, also where the backward takes them through in groups: the groups then give the bits of one pass.
+hipError_t launch_bwd_f32(const BwdParams& call, int64_t heads, int max_q_tiles, int max_k_tiles, hipStream_t stream) {
   BwdParams p = call;
-  p.fp32_products = fp32_products_only(p.head_dim, (int64_t)max_q_tiles * p.num_heads, p.scale_log2);
+  p.fp32_products = fp32_products_only(p.head_dim, max_q_tiles * heads, p.scale_log2);
   int dev = 0, cus = 0;
   const hipError_t e = device_cus(&dev, &cus);
   if (e != hipSuccess) return e;

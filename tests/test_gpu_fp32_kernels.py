@@ -71,6 +71,24 @@ def test_triples_are_no_less_accurate_than_fp32_products(gpu_device, D, values):
         assert a <= 1.02 * b, n
 
 
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_head_groups_give_the_bits_of_one_pass(gpu_device, D):
+    """A call whose workgroups are enough for products of triples, under workspace limits that leave each group of heads fewer."""
+    from stickbreaking_attention import _native
+
+    lengths, H = [200, 33, 1, 385], 10      # (320 workgroups; one head at a time: 32)
+    host, dev, cu = small_case(H, D, lengths, torch.float32, seed=D)
+    run = lambda: run_varlen(*dev[:3], cu.to(gpu_device), lengths, False, False, dev[3], dev[4])
+    whole = run()
+    try:
+        for limit in (1, 1 << 21, 1 << 22):
+            _native.set_backward_workspace_limit(limit)
+            for n, a, b in zip(NAMES, run(), whole):
+                assert torch.equal(a, b), f"{n}, limit {limit}"
+    finally:
+        _native.set_backward_workspace_limit(None)
+
+
 @pytest.mark.parametrize("D", [64, 128])
 def test_odds_below_the_smallest_normal_number(gpu_device, D):
     """Logits of -92 to -86, odds of 2^-133 to 2^-124.  A logit in octaves has an error of up to 2^-17.9 (133 octaves, two

@@ -160,7 +160,12 @@ typedef struct SbaArgs {
                                   through the one kernel, the remaining heads through the two, one pass after the other
                                   (with trace_events, [1] and [2] then bracket the last pass's kernels only).  Must be the
                                   same in sba_workspace_bytes and sba_bwd. */
-  int32_t reserved0;
+  int32_t row_blocks;          /* What the backward on row tiles hands from tile to tile, per head, in key blocks of 32: 8 * the sum
+                                  over all sequences longer than 256 tokens of ceil(length / 256), or more.  0: sized from the bound
+                                  9/256 * total_tokens, which is many times the need of one long sequence among short ones;
+                                  a caller that knows the lengths on the host passes the sum (1 if there is no such sequence).
+                                  Checked on the device like carry_slots.  Must be the same in the forward, the backward and
+                                  sba_workspace_bytes.  Ignored in fixed-length mode. */
 } SbaArgs;
 
 /* What the device scheduler will derive from cu_seqlens, computed on the host from a host copy. */

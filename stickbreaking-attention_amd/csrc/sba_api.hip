@@ -48,6 +48,7 @@ struct Layout {
   Chain chain;
   bool one_kernel;                          // what has to be cleared is cleared with the schedule (else by a kernel in front)
   int64_t chain_rows;                       // rows per head (key tiles), key blocks per head (row tiles)
+  bool rows_by_slot;                        // see BwdParams::chain_by_slot; chain_rows is then checked on the device
   size_t off_chain_zero, chain_zero_bytes;  // {C, tag} per row or the queues, the flags and the XCC ids: cleared for every call
   size_t off_chain_c, off_chain_flags, off_chain_xcc;
   int64_t row_group;                        // row tiles: heads per launch (see plan), of which there are row_launches(heads)
@@ -74,13 +75,14 @@ bool queues_even(int64_t heads, int64_t seqs, int64_t tokens, int64_t max_len) {
   return ((double)(8 * cdiv(heads, 8)) / (double)heads - 1.) * longest <= 1. / 7;
 }
 
-// `row_tiles`: a group of the heads of a call that runs the backward on row tiles, which the group then runs as well.
+// `row_tiles`: a group of the heads of a call that runs the backward on row tiles, which the group then runs as well (and nothing else:
+// there is no room for the two kernels' planes).
 int plan(const SbaArgs* a, Layout* out, bool row_tiles = false) {
   if (a->num_heads <= 0 || a->num_seqs <= 0 || a->total_tokens <= 0) return SBA_ERR_SHAPE;
   if (a->head_dim < 1 || a->head_dim > 128) return SBA_ERR_HEAD_DIM;
   if (a->dtype != SBA_BF16 && a->dtype != SBA_F16 && a->dtype != SBA_F32) return SBA_ERR_DTYPE;
   if (a->total_tokens > (int64_t)1 << 30) return SBA_ERR_SHAPE;
-  if ((a->recompute_carry != 0 && a->recompute_carry != 1) || a->carry_slots < 0) return SBA_ERR_SHAPE;
+  if ((a->recompute_carry != 0 && a->recompute_carry != 1) || a->carry_slots < 0 || a->row_blocks < 0) return SBA_ERR_SHAPE;
   if (a->backward_kernels < 0 || a->backward_kernels > 2) return SBA_ERR_SHAPE;
   if (a->recompute_carry && a->dtype == SBA_F32) return SBA_ERR_DTYPE;      // the fp32 path always keeps its products
   Layout L{};
@@ -160,15 +162,16 @@ int plan(const SbaArgs* a, Layout* out, bool row_tiles = false) {
     L.chain_zero_bytes = off - L.off_chain_zero;
   };
   if (L.chain == Layout::kRowTiles) {
-    L.chain_rows = rows * 9 / 256 + 2;      // (key blocks of 32: every sequence that hands any over is longer than 256)
+    // Key blocks of 32 per head.  (Unknown lengths: every sequence that hands any over is longer than 256.)
+    L.rows_by_slot = fixed || a->row_blocks > 0;
+    L.chain_rows = fixed ? B * sba::row_blocks(T) : a->row_blocks > 0 ? a->row_blocks : rows * 9 / 256 + 2;
     L.row_group = a->num_heads;
     const int64_t row_block = 2 * 32 * 4 * (int64_t)a->head_dim;      // bytes of a key block's dV and dK
-    // What is handed over lies at its key blocks' places, also where most rows are in sequences that hand nothing over: 1152 bytes
-    // per row and head.  The heads of such a batch go through in several launches, multiples of 8 (an equal share for each
-    // queue), that keep this within 1.15 times the carry plane as long as each still fills the chip twice.
+    // Where most sequences hand nothing over, the heads go through in several launches, multiples of 8 (an equal share for each
+    // queue) that still fill the chip twice: what is handed over takes its turns in the same memory (2048 short sequences and one of 16384,
+    // 32 heads, 8 at a time: 11570 -> 10760 to 10990 us).
     if (mean_len < sba::kRowTileRows && max_len > sba::kRowTileRows) {
-      const int64_t least = align_up(cdiv(2 * kRowTilesFrom, rows), 8), fit = (int64_t)L.carry_bytes / 20 * 23 / (L.chain_rows * row_block) & ~7;
-      const int64_t group = fit > least ? fit : least;
+      const int64_t group = align_up(cdiv(2 * kRowTilesFrom, rows), 8);
       if (group < a->num_heads) L.row_group = group;
     }
     chain_bytes = (size_t)L.row_group * L.chain_rows * row_block;
@@ -176,7 +179,7 @@ int plan(const SbaArgs* a, Layout* out, bool row_tiles = false) {
   }
   L.sched_bytes = off;
   off = 0;
-  L.off_prefix = off;      off += L.carry_bytes > chain_bytes ? L.carry_bytes : chain_bytes;
+  L.off_prefix = off;      off += L.carry_bytes > chain_bytes && !row_tiles ? L.carry_bytes : align_up(chain_bytes, 256);
   // d_rem + d_o . v per row (fp32), used when the remainder term is fused
   L.off_drem = off;        off = align_up(off + (size_t)a->num_heads * (size_t)T * (fixed ? (size_t)B : 1) * sizeof(float), 256);
   // the forward's products, rebuilt inside the backward when the caller did not keep them
@@ -302,6 +305,7 @@ sba::SchedParams sched_params(const SbaArgs* a, char* ws, const Layout& L, bool 
   sp.fixed_len = (int32_t)a->total_tokens;
   sp.total_tokens = a->total_tokens;
   sp.carry_capacity = L.carry_slots_per_head;
+  sp.row_capacity = for_backward && L.chain == Layout::kRowTiles && L.rows_by_slot && a->cu_seqlens && key_tile == sba::kRowTileRows ? L.chain_rows : -1;
   sp.want_key_tiles = for_backward ? 1 : 0;
   sp.want_carry_base = want_carry_base ? 1 : 0;
   sp.q_tiles = (sba::Tile*)(ws + L.off_q_tiles);
@@ -510,15 +514,117 @@ namespace {
 
 int bwd_load(const SbaArgs* a) { return row_load(a, {&a->q, &a->k, &a->v, &a->d_o, &a->dq, &a->dk, &a->dv}); }
 bool bwd_wide_rows(const SbaArgs* a) { return wide_rows({&a->q, &a->k, &a->v, &a->d_o, &a->dq, &a->dk, &a->dv}); }
-// Whether one pass over the heads `a` describes runs one kernel.
-bool bwd_is_one_kernel(const SbaArgs* a, const Layout& L) {
+// Which backward one pass over the heads `a` describes runs, and whether that is one kernel.
+Layout::Chain form_of(const SbaArgs* a, const Layout& L) {
+  if (a->dtype == SBA_F32) return Layout::kNone;
   sba::BwdParams p{};
   p.load = bwd_load(a);
   p.wide_rows = bwd_wide_rows(a);
   p.head_dim = a->head_dim;
   p.num_heads = a->num_heads;
   p.add_rem = a->add_remainder ? 1 : 0;
-  return L.one_kernel && chain_of(L, p) != Layout::kNone;
+  return chain_of(L, p);
+}
+bool bwd_is_one_kernel(const SbaArgs* a, const Layout& L) { return L.one_kernel && form_of(a, L) != Layout::kNone; }
+
+// The heads of a call from h0 on, as a call of their own.
+SbaArgs heads_from(const SbaArgs* a, int64_t h0, int64_t count) {
+  SbaArgs c = *a;
+  const int64_t es = (int64_t)elem_size(a->dtype);
+  Layout L;
+  c.num_heads = (int32_t)count;
+  for (SbaTensor* t : {&c.q, &c.k, &c.v, &c.d_o, &c.dq, &c.dk, &c.dv})
+    if (t->ptr) t->ptr = (char*)t->ptr + h0 * t->stride_head * es;
+  if (c.d_rem.ptr) c.d_rem.ptr = (char*)c.d_rem.ptr + h0 * c.d_rem.stride_head * es;
+  if (c.carry && plan(a, &L) == SBA_OK) c.carry += h0 * L.carry_slots_per_head;      // slots per head do not depend on the head count
+  if (c.row_stat) c.row_stat += h0 * a->total_tokens;
+  return c;
+}
+
+// How sba_bwd takes a call through: passes of `group` heads, one after the other on the stream, and a last one of those that are left.
+struct Route {
+  int64_t group;
+  int32_t kernels, tail_kernels;            // SbaArgs.backward_kernels of a pass
+  bool row_tiles, tail_row_tiles;           // a group of a call that runs the backward on row tiles, which the group then runs as well
+};
+
+// `group` heads on row tiles: enough tiles for the chip, spread over its XCDs (as for a call of its own, see plan).
+bool row_group(const SbaArgs* a, int64_t group) {
+  const int64_t rows = a->cu_seqlens ? a->total_tokens : a->num_seqs * a->total_tokens;
+  const int64_t longest = a->max_seqlen > 0 && a->max_seqlen < a->total_tokens ? a->max_seqlen : a->total_tokens;
+  return rows * group >= kRowTilesFrom && queues_even(group, a->num_seqs, rows, longest);
+}
+
+int route_of(const SbaArgs* a, Route* out) {
+  Layout L;
+  const int st = plan(a, &L);
+  if (st != SBA_OK) return st;
+  Route r{a->num_heads, a->backward_kernels, a->backward_kernels, false, false};
+  if (L.split_heads > 0 && a->workspace_bytes >= L.bwd_bytes) {
+    const SbaArgs c = heads_from(a, 0, L.split_heads);
+    Layout L8;
+    if (plan(&c, &L8) == SBA_OK && bwd_is_one_kernel(&c, L8)) {      // (the tensors and the device allow the one kernel)
+      *out = Route{L.split_heads, a->backward_kernels, 1, false, false};
+      return SBA_OK;
+    }
+  }
+  if (a->workspace_bytes >= L.pass_bytes || a->num_heads == 1) {
+    *out = r;
+    return SBA_OK;
+  }
+  // A workspace smaller than the whole call needs: the heads are independent, so they go through in groups of as many
+  // as fit (the per-head planes dominate the workspace).
+  SbaArgs c = *a;
+  auto fits = [&](int64_t heads, bool row_tiles) {
+    Layout G;
+    c.num_heads = (int32_t)heads;
+    return plan(&c, &G, row_tiles) == SBA_OK && G.pass_bytes <= a->workspace_bytes;
+  };
+  // The largest head count whose layout fits: plan() grows with num_heads.
+  auto largest = [&](bool row_tiles) {
+    int64_t lo = 0, hi = a->num_heads;
+    while (lo < hi) {
+      const int64_t mid = (lo + hi + 1) / 2;
+      if (fits(mid, row_tiles)) lo = mid; else hi = mid - 1;
+    }
+    return lo;
+  };
+  if (form_of(a, L) == Layout::kRowTiles) {
+    // Groups of one sequence's few heads would leave XCDs without work (8 heads x 65536, one at a time: 32 of 256 compute units), groups of few
+    // rows most of them: such groups run the two kernels, which use all of them.
+    // Equal groups if they suit, else the largest with a remainder that suits too, else the largest, its remainder on the two kernels.
+    const int64_t most = largest(true);
+    auto rest_suits = [&](int64_t group) { return a->num_heads % group == 0 || row_group(a, a->num_heads % group); };
+    auto rest_fits = [&](int64_t group) {
+      c.backward_kernels = 1;
+      const bool ok = rest_suits(group) || fits(a->num_heads % group, false);
+      c.backward_kernels = a->backward_kernels;
+      return ok;
+    };
+    int64_t group = most > 0 ? cdiv(a->num_heads, cdiv(a->num_heads, most)) : 0;
+    if (group > 0 && !(row_group(a, group) && rest_suits(group))) {
+      for (group = most; group > 0 && !(row_group(a, group) && rest_suits(group));) group--;
+      if (group == 0)
+        for (group = most; group > 0 && !(row_group(a, group) && rest_fits(group));) group--;
+    }
+    if (group > 0) {
+      *out = Route{group, a->backward_kernels, rest_suits(group) ? a->backward_kernels : 1, true, rest_suits(group)};
+      return SBA_OK;
+    }
+  }
+  // (a call that would not run either of the chained backwards runs the two kernels in groups too)
+  if (L.chain != Layout::kKeyTiles) r.kernels = c.backward_kernels = 1;
+  const int64_t lo = largest(false);
+  if (lo < 1) return SBA_ERR_WORKSPACE;
+  r.group = cdiv(a->num_heads, cdiv(a->num_heads, lo));
+  // The one-kernel backward's layout is the larger one and is only laid out for head counts it applies to, so a group
+  // size below `lo` need not fit although `lo` does: every pass then takes the two-kernel backward, whose layout grows
+  // with the head count and therefore fits.
+  const int64_t tail = a->num_heads % r.group;
+  if (!fits(r.group, false) || (tail > 0 && !fits(tail, false))) r.kernels = 1;
+  r.tail_kernels = r.kernels;
+  *out = r;
+  return SBA_OK;
 }
 
 // The backward on row tiles, in the launches that the layout asks for: each has queues of its own, what is handed over takes turns.
@@ -596,6 +702,7 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* 
   p.split = split_keys(a, L, stat_heads, p.load);
   // One kernel (the key tiles of a sequence hand C and partial dQ to each other) where it applies, else dQ then dK/dV.
   const Layout::Chain chain = a->dtype == SBA_F32 ? Layout::kNone : chain_of(L, p);
+  if (row_tiles && chain != Layout::kRowTiles) return SBA_ERR_WORKSPACE;      // (route_of asked)
   char* const cleared = L.one_kernel ? ws : rest;
   if (chain != Layout::kNone) {
     p.chain_c = (uint32_t*)(cleared + L.off_chain_c);
@@ -604,6 +711,7 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* 
     p.chain_dq = (float*)(rest + L.off_prefix);
     p.status = (int32_t*)(ws + L.off_counts) + sba::kCountStatus;
     p.chain_rows = L.chain_rows;
+    p.chain_by_slot = L.rows_by_slot ? 1 : 0;
     p.chain_sb = fixed ? a->total_tokens : 0;
     p.chain_tile_cap = (int32_t)L.max_k_tiles;
   }
@@ -679,65 +787,14 @@ int sba_bwd_kernels(const SbaArgs* a) {
 
 int sba_bwd(const SbaArgs* a) {
   if (!a) return SBA_ERR_NULL;
-  Layout L;
-  int st = plan(a, &L);
+  Route r;
+  int st = route_of(a, &r);
   if (st != SBA_OK) return st;
-  const size_t es = elem_size(a->dtype);
-  // the heads of a call from h0 on, as a call of their own
-  auto heads_from = [&](int64_t h0, int64_t count) {
-    SbaArgs c = *a;
-    c.num_heads = (int32_t)count;
-    for (SbaTensor* t : {&c.q, &c.k, &c.v, &c.d_o, &c.dq, &c.dk, &c.dv})
-      if (t->ptr) t->ptr = (char*)t->ptr + h0 * t->stride_head * (int64_t)es;
-    if (c.d_rem.ptr) c.d_rem.ptr = (char*)c.d_rem.ptr + h0 * c.d_rem.stride_head * (int64_t)es;
-    if (c.carry) c.carry += h0 * L.carry_slots_per_head;          // slots per head do not depend on the head count
-    if (c.row_stat) c.row_stat += h0 * a->total_tokens;
-    return c;
-  };
-  if (L.split_heads > 0 && a->workspace_bytes >= L.bwd_bytes) {
-    SbaArgs c = heads_from(0, L.split_heads);
-    Layout L8;
-    if (plan(&c, &L8) == SBA_OK && bwd_is_one_kernel(&c, L8)) {      // (the tensors and the device allow the one kernel)
-      if ((st = bwd_pass(&c, a->num_heads, true, false)) != SBA_OK) return st;
-      c = heads_from(L.split_heads, a->num_heads - L.split_heads);
-      c.backward_kernels = 1;
-      return bwd_pass(&c, a->num_heads, false, true);
-    }
-  }
-  if (a->workspace_bytes >= L.pass_bytes || a->num_heads == 1) return bwd_pass(a, a->num_heads, true, true);
-  // A workspace smaller than the whole call needs: the heads are independent, so they go through in groups of as many
-  // as fit (the per-head planes dominate the workspace), one group after the other on the stream.
-  SbaArgs c = *a;
-  int32_t kernels = a->backward_kernels;
-  // The largest head count whose layout fits: plan() grows with num_heads.
-  auto largest = [&](bool row_tiles) {
-    int64_t lo = 0, hi = a->num_heads;
-    while (lo < hi) {
-      c.num_heads = (int32_t)((lo + hi + 1) / 2);
-      if (plan(&c, &L, row_tiles) == SBA_OK && L.pass_bytes <= a->workspace_bytes) lo = c.num_heads; else hi = c.num_heads - 1;
-    }
-    return lo;
-  };
-  const Layout::Chain whole = L.chain;
-  int64_t lo = whole == Layout::kRowTiles ? largest(true) : 0;
-  const bool row_tiles = lo > 0;
-  if (!row_tiles) {      // (a call that would not run either of the chained backwards runs the two kernels in groups too)
-    if (whole != Layout::kKeyTiles) kernels = c.backward_kernels = 1;
-    lo = largest(false);
-  }
-  if (lo < 1) return SBA_ERR_WORKSPACE;
-  const int64_t passes = cdiv(a->num_heads, lo), group = cdiv(a->num_heads, passes);
-  // The one-kernel backward's layout is the larger one and is only laid out for head counts it applies to, so a group
-  // size below `lo` need not fit although `lo` does: every pass then takes the two-kernel backward, whose layout grows
-  // with the head count and therefore fits.
-  for (int64_t heads : {group, a->num_heads % group}) {
-    c.num_heads = (int32_t)heads;
-    if (heads > 0 && !row_tiles && (plan(&c, &L) != SBA_OK || L.pass_bytes > a->workspace_bytes)) kernels = 1;
-  }
-  for (int64_t h0 = 0; h0 < a->num_heads; h0 += group) {
-    c = heads_from(h0, a->num_heads - h0 < group ? a->num_heads - h0 : group);
-    c.backward_kernels = kernels;
-    if ((st = bwd_pass(&c, a->num_heads, h0 == 0, h0 + group >= a->num_heads, nullptr, row_tiles)) != SBA_OK) return st;
+  for (int64_t h0 = 0; h0 < a->num_heads; h0 += r.group) {
+    const bool tail = a->num_heads - h0 < r.group;
+    SbaArgs c = heads_from(a, h0, tail ? a->num_heads - h0 : r.group);
+    c.backward_kernels = tail ? r.tail_kernels : r.kernels;
+    if ((st = bwd_pass(&c, a->num_heads, h0 == 0, h0 + r.group >= a->num_heads, nullptr, tail ? r.tail_row_tiles : r.row_tiles)) != SBA_OK) return st;
   }
   return SBA_OK;
 }
@@ -767,6 +824,19 @@ bool prepared_fits(const SbaArgs* a) {
   p.add_rem = a->add_remainder ? 1 : 0;
   p.split = split_keys(a, L, a->num_heads, p.load);
   return a->dtype == SBA_F32 || key_tile_of(L, p) == expected_key_tile(a, L);
+}
+
+int backward_route(const SbaArgs* a, BackwardRoute* out) {
+  Route r;
+  Layout L;
+  const int st = route_of(a, &r);
+  if (st != SBA_OK) return st;
+  SbaArgs c = heads_from(a, 0, r.group);
+  c.backward_kernels = r.kernels;
+  if (plan(&c, &L, r.row_tiles) != SBA_OK) return SBA_ERR_SHAPE;
+  const Layout::Chain chain = form_of(&c, L);
+  *out = BackwardRoute{chain == Layout::kRowTiles ? kBwdRowTiles : chain == Layout::kKeyTiles ? kBwdKeyTiles : kBwdTwoKernels, (int32_t)r.group};
+  return SBA_OK;
 }
 
 int backward_prepared(const SbaArgs* a, void* sched) { return bwd_pass(a, a->num_heads, true, true, (char*)sched); }

@@ -283,8 +283,10 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
       const int u = min(t, u_last);
       return carry + (carry_offset(u, n_qt) - kBlockQ * (u >> 2));
     };
-    // What the row tiles of a (head, sequence) hand down: per key block and wave, the 32 x 32 partial result.
-    float* part = p.chain_dq + ((int64_t)head * p.chain_rows + ((int64_t)seq_id * p.chain_sb + tok0) * 9 / 256) * (kPieces * 1024) + (wave & (kPieces - 1)) * 1024;
+    // What the row tiles of a (head, sequence) hand down: per key block and wave, the 32 x 32 partial result.  (Sequences of more than one
+    // tile come first in the list, each with 8 key blocks per tile.)
+    const int64_t first_block = p.chain_by_slot ? (int64_t)(slot - __builtin_amdgcn_readfirstlane(tile.origin) / kRowTile) * (kRowTile / kRowKeys) : tok0 * 9 / 256;
+    float* part = p.chain_dq + ((int64_t)head * p.chain_rows + first_block) * (kPieces * 1024) + (wave & (kPieces - 1)) * 1024;
     int32_t* flag = p.chain_flags + ((int64_t)head * p.chain_tile_cap + slot) * 8 + wave;
     const int32_t* pred = has_pred ? flag - 8 : flag;
     const int lane16 = lane * 16;

@@ -1,5 +1,5 @@
 // What the torch host layer uses of libsba.so besides the C ABI: a forward that prepares the schedule of the backward that
-// follows it (tile lists, cursors, cleared flags), so that the backward needs no scheduler launch of its own.
+// follows it (tile lists, cursors, cleared flags), so that the backward needs no scheduler launch of its own; and which backward a call runs.
 #pragma once
 #include "../../include/sba.h"
 
@@ -18,5 +18,13 @@ int forward_prepared(const SbaArgs* a);
 bool prepared_fits(const SbaArgs* a);
 // sba_bwd on that schedule, with the rest in a->workspace.  The schedule serves ONE backward: its cursors are used up.
 int backward_prepared(const SbaArgs* a, void* sched);
+
+// What sba_bwd would run for these arguments on the current device, with this workspace: the form of its first pass, and the heads that
+// pass takes (all, unless they go through in groups or are split between two forms).
+enum : int32_t { kBwdTwoKernels = 0, kBwdKeyTiles = 1, kBwdRowTiles = 2 };
+struct BackwardRoute {
+  int32_t form, heads;
+};
+int backward_route(const SbaArgs* a, BackwardRoute* out);
 
 }  // namespace sba

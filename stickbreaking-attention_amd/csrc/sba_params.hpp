@@ -43,6 +43,7 @@ struct SchedParams {
   int32_t fixed_len;       // L in fixed-length mode
   int64_t total_tokens;    // T: rows of the packed token axis (L in fixed-length mode)
   int64_t carry_capacity;  // carry slots reserved per head
+  int64_t row_capacity;    // key blocks reserved per head for what row tiles hand over (< 0: not to be checked)
   int32_t want_key_tiles;  // backward: also build the key-tile list
   int32_t want_carry_base; // also lay out the per-sequence carry offsets
   Tile* q_tiles;           // query tiles (kBlockQ rows), heaviest first
@@ -62,6 +63,8 @@ struct SchedParams {
 constexpr int kInlineSeqs = 64;
 
 constexpr int kRowTileRows = 256;      // query rows per tile of the backward on row tiles
+// Key blocks of 32 that the row tiles of a sequence hand over, rounded up to whole tiles (none if it is a single tile).
+__host__ __device__ inline int64_t row_blocks(int64_t len) { return len > kRowTileRows ? (len + kRowTileRows - 1) / kRowTileRows * (kRowTileRows / 32) : 0; }
 // Its queue, of 8, for head 0 of the sequence with this rank (the list holds the longest first); head h's is (this + h) % 8.  If the heads do
 // not fill the queues evenly, the fuller ones are others for the next sequence, in an order that goes forth and back (a Gray code).
 __host__ __device__ inline int row_queue(int rank, int heads) { return heads & 7 ? ((rank ^ rank >> 1) * (heads & 7)) & 7 : 0; }
@@ -123,7 +126,8 @@ struct BwdParams {
   int32_t* chain_flags;        // [head][tile slot][8]: per wave, row (key) blocks whose partial result is complete
   int32_t* chain_head_xcc;     // [head] (row tiles: [queue]): XCC id + 1 of its workgroups (0 = none yet)
   int32_t* status;             // the scheduler's status word; the kernel raises it when a wait runs out
-  int64_t chain_rows;          // rows per head in chain_dq / chain_c
+  int64_t chain_rows;          // rows (row tiles: key blocks) per head in chain_dq / chain_c
+  int32_t chain_by_slot;       // row tiles: a sequence's key blocks lie at 8 * its first slot of the list (else at 9/256 * its first token)
   int64_t chain_sb;            // fixed-length mode: rows per batch element (0 in packed mode)
   int32_t chain_tile_cap;      // key-tile slots per head in chain_flags
   int32_t fp32_products;       // as in FwdParams

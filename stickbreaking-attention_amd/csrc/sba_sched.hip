@@ -51,10 +51,11 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
   __shared__ int kbins[kBins];
   __shared__ int scratch[kSchedThreads];
   __shared__ long long carry_run;
+  __shared__ unsigned long long row_run;
   __shared__ int status;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = kSchedThreads / 64;
   for (int i = threadIdx.x; i < kBins; i += kSchedThreads) { qbins[i] = 0; kbins[i] = 0; }
-  if (threadIdx.x == 0) { carry_run = 0; status = kSchedOk; }
+  if (threadIdx.x == 0) { carry_run = 0; row_run = 0; status = kSchedOk; }
   __syncthreads();
 
   // Pass 1: tiles per length class (class = number of query tiles of the sequence, saturating).  Every entry of
@@ -67,7 +68,10 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
     const int cls = min(nq, kBins - 1);
     if (nq) atomicAdd(&qbins[cls], nq);
     if (nk && p.want_key_tiles) atomicAdd(&kbins[cls], nk);
+    if (p.row_capacity >= 0 && row_blocks(len) > 0) atomicAdd(&row_run, (unsigned long long)row_blocks(len));
   }
+  __syncthreads();
+  if (threadIdx.x == 0 && status == kSchedOk && p.row_capacity >= 0 && row_run > (unsigned long long)p.row_capacity) status = kSchedCarryOverflow;
   __syncthreads();
   if (status != kSchedOk) {      // uniform: nothing is scheduled, every output row is zero-filled as uncovered
     if (threadIdx.x == 0) { p.counts[kCountQ] = 0; p.counts[kCountK] = 0; p.counts[kCountStatus] = status; p.counts[kCountCovered] = 0; }

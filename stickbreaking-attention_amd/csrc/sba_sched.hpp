@@ -29,6 +29,11 @@ __device__ __forceinline__ SeqLanes load_lanes(const SchedParams& p) {
     for (int j = 0; j < p.num_seqs; j++) slots += carry_slots(__builtin_amdgcn_readlane(s.nq, j));
     if (slots > p.carry_capacity) s.status = kSchedCarryOverflow;
   }
+  if (s.status == kSchedOk && p.row_capacity >= 0) {
+    int64_t blocks = 0;
+    for (int j = 0; j < p.num_seqs; j++) blocks += row_blocks(__builtin_amdgcn_readlane(s.len, j));
+    if (blocks > p.row_capacity) s.status = kSchedCarryOverflow;
+  }
   return s;
 }
 // First slot of this lane's sequence in a list of `n` tiles per sequence: sequences with more query tiles first, then by

@@ -94,7 +94,7 @@ void check_status(const Tensor& ws, const char* what) {
 struct Call {
   Tensor cu;      // packed batches only
   bool fixed = false, leading_zero = false, attend_current = false, add_remainder = false;
-  int64_t max_seqlen = 0, carry_slots = 0, flags = 0;
+  int64_t max_seqlen = 0, carry_slots = 0, row_blocks = 0, flags = 0;
   double logit_scale = 0;
 };
 
@@ -110,6 +110,7 @@ SbaArgs base_args(const Call& c, const Tensor& q) {
     a.cu_is_int64 = c.cu.scalar_type() == at::kLong;
     a.cu_has_leading_zero = c.leading_zero;
     a.carry_slots = c.carry_slots;
+    a.row_blocks = (int32_t)c.row_blocks;
   }
   a.max_seqlen = c.max_seqlen;
   a.logit_scale = (float)c.logit_scale;
@@ -118,6 +119,22 @@ SbaArgs base_args(const Call& c, const Tensor& q) {
   a.backward_kernels = (int32_t)(c.flags >> kBackwardKernelsShift);
   a.stream = (void*)c10::hip::getCurrentHIPStream(q.device().index()).stream();
   return a;
+}
+
+// SbaArgs::row_blocks of these (valid) lengths.
+template <typename T>
+int64_t row_blocks_of(const T* ends, int64_t n, bool leading_zero) {
+  int64_t sum = 0, last = 0;
+  for (int64_t i = leading_zero ? 1 : 0; i < n; i++) {
+    const int64_t len = (int64_t)ends[i] - last;
+    if (len > 256) sum += (len + 255) / 256 * 8;
+    last = (int64_t)ends[i];
+  }
+  return std::max<int64_t>(sum, 1);
+}
+int64_t row_blocks(const Tensor& host, bool leading_zero) {
+  return host.scalar_type() == at::kLong ? row_blocks_of(host.const_data_ptr<int64_t>(), host.numel(), leading_zero)
+                                         : row_blocks_of(host.const_data_ptr<int32_t>(), host.numel(), leading_zero);
 }
 
 Tensor bytes(size_t n, const Tensor& like) { return at::empty({(int64_t)n}, like.options().dtype(at::kByte)); }
@@ -248,7 +265,8 @@ struct StickBreaking : torch::autograd::Function<StickBreaking> {
     ctx->save_for_backward({q, k, v, c.cu, out.state});
     ctx->saved_data["fresh"] = true;
     ctx->saved_data["call"] = c10::IValue(std::vector<int64_t>{c.fixed, c.leading_zero, c.attend_current, c.add_remainder,
-                                                               c.max_seqlen, c.carry_slots, c.flags, save_carry, out.kept_schedule});
+                                                               c.max_seqlen, c.carry_slots, c.flags, save_carry, out.kept_schedule,
+                                                               c.row_blocks});
     ctx->saved_data["scale"] = c.logit_scale;
     return {out.o, out.rem};
   }
@@ -257,7 +275,7 @@ struct StickBreaking : torch::autograd::Function<StickBreaking> {
     const std::vector<int64_t> n = ctx->saved_data["call"].toIntVector();
     Call c;
     c.fixed = n[0]; c.leading_zero = n[1]; c.attend_current = n[2]; c.add_remainder = n[3];
-    c.max_seqlen = n[4]; c.carry_slots = n[5]; c.flags = n[6];
+    c.max_seqlen = n[4]; c.carry_slots = n[5]; c.flags = n[6]; c.row_blocks = n[9];
     c.logit_scale = ctx->saved_data["scale"].toDouble();
     c.cu = s[3];
     c10::IValue& fresh = ctx->saved_data["fresh"];
@@ -362,6 +380,7 @@ std::optional<std::tuple<Tensor, Tensor>> varlen(py::handle hq, py::handle hk, p
     check(sba_plan_host(&a, host.const_data_ptr(), &plan), "sba_plan_host");
     TORCH_CHECK_VALUE(plan.status == 0, "cu_seqlens must be non-decreasing sequence ends within [0, total_tokens]");
     c.carry_slots = plan.carry_slots;
+    c.row_blocks = row_blocks(host, zero_start);
     c.max_seqlen = std::max(plan.longest, 1);
   }
   if (cu.device() != q.device()) cu = cu.to(q.device());
@@ -377,5 +396,11 @@ PYBIND11_MODULE(_sba_torch, m) {
   m.def("fixed", &fixed);
   m.def("varlen", &varlen);
   m.def("set_backward_workspace_limit", [](std::optional<int64_t> n) { g_bwd_limit.store(n ? std::max<int64_t>(*n, 0) : -1); });
+  // (form, heads of the first pass) of the backward that the SbaArgs at this address describe.
+  m.def("backward_route", [](uint64_t args) {
+    sba::BackwardRoute r{};
+    check(sba::backward_route((const SbaArgs*)(uintptr_t)args, &r), "backward_route");
+    return std::make_tuple(r.form, r.heads);
+  });
   m.def("version", &sba_version);
 }

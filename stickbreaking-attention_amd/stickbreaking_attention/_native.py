@@ -46,7 +46,7 @@ class SbaArgs(ctypes.Structure):
         ("workspace", ctypes.c_void_p), ("workspace_bytes", ctypes.c_size_t), ("stream", ctypes.c_void_p),
         ("trace_events", ctypes.POINTER(ctypes.c_void_p)),
         ("add_remainder", ctypes.c_int32), ("recompute_carry", ctypes.c_int32), ("carry_slots", ctypes.c_int64),
-        ("backward_kernels", ctypes.c_int32), ("reserved0", ctypes.c_int32),
+        ("backward_kernels", ctypes.c_int32), ("row_blocks", ctypes.c_int32),
     ]
 
 
@@ -278,7 +278,7 @@ _WS_BYTES = {}
 def _workspace_bytes(a: SbaArgs):
     """(forward workspace, backward workspace, carry) sizes in bytes for these arguments."""
     key = (a.dtype, a.num_heads, a.head_dim, a.num_seqs, a.total_tokens, a.max_seqlen, bool(a.cu_seqlens), a.cu_is_int64,
-           a.cu_has_leading_zero, a.attend_current, a.add_remainder, a.recompute_carry, a.carry_slots, a.backward_kernels)
+           a.cu_has_leading_zero, a.attend_current, a.add_remainder, a.recompute_carry, a.carry_slots, a.backward_kernels, a.row_blocks)
     got = _WS_BYTES.get(key)
     if got is None:
         f, b, c = ctypes.c_size_t(0), ctypes.c_size_t(0), ctypes.c_size_t(0)

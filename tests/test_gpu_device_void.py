@@ -135,3 +135,30 @@ def test_python_operators_raise_on_a_void_schedule(gpu_device):
     q, k, v = (t.requires_grad_() for t in _inputs(2, 4096, 64, torch.bfloat16, gpu_device))
     with pytest.raises(ValueError, match="carry"):
         sb_attn_varlen(q, k, v, cu, 64, zero_start=False, save_carry=False)      # void in the forward already
+
+
+@pytest.mark.parametrize("n", [1, 70], ids=["inline-scheduler", "scheduler-kernel"])
+def test_understated_row_blocks_void_the_backward(gpu_device, n):
+    """Row tiles hand over 8 key blocks per tile of 256 rows; a caller that reserves fewer gets zero gradients and a status."""
+    from stickbreaking_attention import _native as native
+
+    H, D, lengths = 16, 128, [4096] + [20] * n
+    T, need = sum(lengths), 8 * 16
+    q, k, v = _inputs(H, T, D, torch.bfloat16, gpu_device)
+    cu = torch.tensor(lengths).cumsum(0).int().to(gpu_device)
+    ret, status, _, carry = _forward(native, q, k, v, cu, 4096, 0, want_carry=True)
+    assert ret == 0 and status == 0
+    base_args = native._base_args
+    for blocks, expected in ((need, 0), (need - 1, CARRY_TOO_SMALL)):
+        def with_blocks(*args, **kw):
+            a = base_args(*args, **kw)
+            a.row_blocks = blocks
+            return a
+
+        native._base_args = with_blocks
+        try:
+            ret, status, grads = _backward(native, q, k, v, cu, 4096, 0, carry, 0)
+        finally:
+            native._base_args = base_args
+        assert ret == 0 and status == expected
+        assert all((t == 0).all() if expected else torch.isfinite(t.float()).all() and not (t == 0).all() for t in grads)

@@ -93,6 +93,26 @@ def test_against_oracle_and_two_kernels(gpu_device, D, label, H, lengths, c):
         assert excess.max().item() <= 0, f"{label}: {name} against the two kernels, {excess.max().item():.3e} beyond twice the bound"
 
 
+@pytest.mark.parametrize("H,lengths", [(80, [600, 33, 289, 256, 257]), (64, [1100, 300] + [35] * 50), (16, [40] * 40 + [2100, 700, 1300] + [40] * 40), (96, [255, 256, 64])],
+                         ids=["chain", "two-launches", "scheduler-kernel", "nothing-handed-over"])
+@pytest.mark.parametrize("D", [128, 64])
+def test_lengths_on_the_host_give_the_same_bits(gpu_device, D, H, lengths):
+    """With the lengths on the host, what the tiles hand over is laid out by their place in the list and takes as much memory as it needs."""
+    from stickbreaking_attention import _native
+
+    g = torch.Generator().manual_seed(H)
+    dev = [torch.randn(H, sum(lengths), D, generator=g).bfloat16().to(gpu_device) for _ in range(4)]
+    dev.append(torch.randn(H, sum(lengths), generator=g).bfloat16().to(gpu_device))
+    cu = torch.tensor(np.cumsum(lengths), dtype=torch.int32)
+    saved = (_native.BACKWARD_KERNELS, _native.POISON)
+    try:
+        _native.POISON = True
+        for got in zip(*(gradients(_native, 0, dev, t, lengths, {}) for t in (cu.to(gpu_device), cu, cu.long()))):
+            assert torch.isfinite(got[0].float()).all() and torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+    finally:
+        _native.BACKWARD_KERNELS, _native.POISON = saved
+
+
 @pytest.mark.parametrize("save_carry", [True, False])
 @pytest.mark.parametrize("case", [(32, 128, [1300, 2100], torch.bfloat16), (64, 64, [1100], torch.bfloat16), (20, 64, [1200, 1700, 3400], torch.float16)],
                          ids=["cleared-with-the-schedule", "head-dim-64", "ranked-queues"])

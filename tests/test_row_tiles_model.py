@@ -1,6 +1,7 @@
 """CPU checks of the backward on row tiles (csrc/sba_bwd_row.hip): which recorded products it reads, how the queues of its tiles fall, and
 what its inline assembly has to keep that the compiler does not check."""
 import os
+import random
 import re
 import shutil
 import subprocess
@@ -38,6 +39,21 @@ def test_partial_results_of_neighbours_do_not_overlap():
             first = start * 9 // 256
             assert (start + L) * 9 // 256 - first >= cdiv(L, 32), (L, start)      # before the next sequence's, which starts at or behind
             assert first + cdiv(L, 32) <= (start + L) * 9 // 256 + 2              # within the head's
+
+
+def test_places_by_slot_do_not_overlap():
+    """The list holds sequences with more query tiles of 128 rows first; one of more than 256 rows has 8 key blocks per row tile at 8 times
+    its first slot, all within SbaArgs.row_blocks."""
+    rng = random.Random(0)
+    for _ in range(300):
+        lengths = [rng.choice([0, 1, 255, 256, 257, 511, 512, 513, rng.randint(1, 3000)]) for _ in range(rng.randint(1, 40))]
+        total, slot0, end = sum(8 * cdiv(n, 256) for n in lengths if n > 256), 0, 0
+        for n in sorted(lengths, key=lambda n: -cdiv(n, 128)):
+            if n > 256:
+                assert 8 * slot0 >= end      # behind the one before
+                end = 8 * slot0 + cdiv(n, 256) * 8 - 8      # (its last tile's own rows are handed to none)
+                assert end <= total
+            slot0 += cdiv(n, 256)
 
 
 @pytest.mark.parametrize("heads", [1, 4, 7, 8, 12, 20, 32])

@@ -138,6 +138,27 @@ int64_t row_blocks(const Tensor& host, bool leading_zero) {
 }
 
 Tensor bytes(size_t n, const Tensor& like) { return at::empty({(int64_t)n}, like.options().dtype(at::kByte)); }
+// The backward's scratch: `n` bytes or, where memory is short, less, which takes the heads through in groups: what the dQ and dK/dV kernels
+// need (up to a fifth of what row tiles do), then half as much, down to what one head needs, the least that sba_bwd accepts.
+Tensor backward_bytes(const SbaArgs& a, size_t n, const Tensor& like) {
+  size_t two_kernels = 0, one_head = 0;
+  for (;;) {
+    try {
+      return bytes(n, like);
+    } catch (const c10::OutOfMemoryError&) {
+      if (one_head == 0) {
+        SbaArgs c = a;
+        c.backward_kernels = 1;
+        check(sba_workspace_bytes(&c, nullptr, &two_kernels, nullptr), "sba_workspace_bytes");
+        c = a;
+        c.num_heads = 1;
+        check(sba_workspace_bytes(&c, nullptr, &one_head, nullptr), "sba_workspace_bytes");
+      }
+      if (n <= one_head) throw;
+    }
+    n = std::max(one_head, two_kernels < n ? two_kernels : n / 2);
+  }
+}
 
 struct Outputs {
   Tensor o, rem;
@@ -236,8 +257,17 @@ variable_list run_backward(Call c, Tensor d_o, Tensor d_rem, Tensor q, Tensor k,
   // The forward's schedule serves one backward.  Under graph capture it may be replayed more often than the forward.
   const bool prepared = kept_schedule > 0 && fresh && limit < 0 && sba::prepared_fits(&a) &&
                         c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None;
-  size_t ws_bytes = size.rest;
-  if (!prepared) {
+  Tensor ws;
+  bool on_schedule = prepared;
+  if (prepared) {
+    try {
+      ws = bytes(size.rest, q);
+    } catch (const c10::OutOfMemoryError&) {
+      on_schedule = false;
+    }
+  }
+  if (!on_schedule) {
+    size_t ws_bytes = 0;
     check(sba_workspace_bytes(&a, nullptr, &ws_bytes, nullptr), "sba_workspace_bytes");
     if (limit >= 0 && ws_bytes > (size_t)limit) {
       SbaArgs one = a;                        // the smallest workspace the library accepts is the one of a single head
@@ -246,13 +276,13 @@ variable_list run_backward(Call c, Tensor d_o, Tensor d_rem, Tensor q, Tensor k,
       check(sba_workspace_bytes(&one, nullptr, &one_bytes, nullptr), "sba_workspace_bytes");
       ws_bytes = std::max((size_t)limit, one_bytes);
     }
+    ws = backward_bytes(a, ws_bytes, q);
   }
-  const Tensor ws = bytes(ws_bytes, q);
   if (c.flags & kPoison) poison(ws);
   a.workspace = ws.data_ptr();
-  a.workspace_bytes = ws_bytes;
-  check(prepared ? sba::backward_prepared(&a, base) : sba_bwd(&a), "sba_bwd");
-  if (c.flags & kDebugCheck) check_status(prepared ? state : ws, "sba_bwd");
+  a.workspace_bytes = ws.numel();
+  check(on_schedule ? sba::backward_prepared(&a, base) : sba_bwd(&a), "sba_bwd");
+  if (c.flags & kDebugCheck) check_status(on_schedule ? state : ws, "sba_bwd");
   return {dq, dk, dv};
 }
 

@@ -287,6 +287,24 @@ def _workspace_bytes(a: SbaArgs):
     return got
 
 
+def _backward_scratch(a: SbaArgs, nbytes: int, device) -> torch.Tensor:
+    """The backward's workspace or, where memory is short, a smaller one, which takes the heads through in groups: what the dQ and dK/dV
+    kernels need, then half as much, down to what one head needs, the least that the library accepts."""
+    while True:
+        try:
+            return torch.empty(nbytes, dtype=torch.uint8, device=device)
+        except torch.cuda.OutOfMemoryError:
+            kernels, heads = a.backward_kernels, a.num_heads
+            a.backward_kernels = 1
+            two_kernels = _workspace_bytes(a)[1]
+            a.backward_kernels, a.num_heads = kernels, 1
+            one_head = _workspace_bytes(a)[1]
+            a.num_heads = heads
+            if nbytes <= one_head:
+                raise
+            nbytes = max(one_head, two_kernels if two_kernels < nbytes else nbytes // 2)
+
+
 def _launch_fwd(q, k, v, cu_seqlens, cu_has_leading_zero, max_seqlen, carry_slots, logit_scale, attend_current, add_remainder,
                 o, rem, neg_log_acc, carry):
     fixed = cu_seqlens is None
@@ -336,8 +354,8 @@ def _launch_bwd(do, drem, q, k, v, carry, neg_log_acc, cu_seqlens, cu_has_leadin
             one_head = _workspace_bytes(a)[1]
             a.num_heads = heads
             nbytes = max(BWD_WORKSPACE_LIMIT, one_head)
-        ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
-        a.workspace, a.workspace_bytes = ws.data_ptr(), nbytes
+        ws = _backward_scratch(a, nbytes, q.device)
+        a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
         if POISON:
             _poison(ws)
         if TRACE_EVENTS is not None:

@@ -46,8 +46,9 @@ extern "C" {
 #define SBA_SCHED_OK 0
 #define SBA_SCHED_BAD_CU_SEQLENS 1
 #define SBA_SCHED_CARRY_TOO_SMALL 2
-#define SBA_CHAIN_TIMEOUT 3        /* one-kernel backward: a workgroup gave up waiting for the tile before its own */
-#define SBA_CHAIN_XCD_MISMATCH 4   /* one-kernel backward: the workgroups of a head did not share an XCD */
+#define SBA_CHAIN_TIMEOUT 3        /* a backward whose tiles hand partial sums to each other: a tile gave up waiting for the one before
+                                      its own.  The gradients that depend on it are NaN. */
+#define SBA_CHAIN_XCD_MISMATCH 4   /* not raised any more: workgroups that do not share the XCD of those before them leave them the tiles */
 
 /* Size of the static device scratch behind sba_fwd_static. */
 #define SBA_STATIC_SCRATCH_BYTES ((size_t)1 << 20)

@@ -651,8 +651,8 @@ hipError_t launch_row_tiles(const sba::BwdParams& whole, const Layout& L, bool f
 // One pass of the backward over the heads `a` describes (all of them, or one group of a larger call: `stat_heads` is
 // the head count of the caller's row_stat array, `first`/`last` say which trace events this pass records).  `sched`: the
 // schedule a forward left (the workspace is then the rest), or NULL to run the
-// scheduler here.
-int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* sched = nullptr, bool row_tiles = false) {
+// scheduler here.  `polls`: of a wait between tiles before it runs out (0: about half a second's).
+int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* sched = nullptr, bool row_tiles = false, int32_t polls = 0) {
   Layout L;
   int st = plan(a, &L, row_tiles);
   if (st != SBA_OK) return st;
@@ -711,6 +711,7 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* 
     p.chain_head_xcc = (int32_t*)(cleared + L.off_chain_xcc);
     p.chain_dq = (float*)(rest + L.off_prefix);
     p.status = (int32_t*)(ws + L.off_counts) + sba::kCountStatus;
+    p.wait_polls = polls > 0 ? polls : chain == Layout::kRowTiles ? 1 << 20 : 1 << 17;
     p.chain_rows = L.chain_rows;
     p.chain_by_slot = L.rows_by_slot ? 1 : 0;
     p.chain_sb = fixed ? a->total_tokens : 0;
@@ -839,6 +840,8 @@ int backward_route(const SbaArgs* a, BackwardRoute* out) {
   *out = BackwardRoute{chain == Layout::kRowTiles ? kBwdRowTiles : chain == Layout::kKeyTiles ? kBwdKeyTiles : kBwdTwoKernels, (int32_t)r.group};
   return SBA_OK;
 }
+
+int backward_with_polls(const SbaArgs* a, int32_t polls) { return bwd_pass(a, a->num_heads, true, true, nullptr, false, polls); }
 
 int backward_prepared(const SbaArgs* a, void* sched) { return bwd_pass(a, a->num_heads, true, true, (char*)sched); }
 

@@ -24,8 +24,9 @@
 //     loaded from the chain.
 // All workgroups of a head run on one XCD (workgroup ids are dealt round-robin to the XCDs), so the hand-over
 // needs L2 coherence only: ordinary stores, completed (s_waitcnt vmcnt(0)) before a flag store, and loads that
-// bypass the vector L1 (sc1).  Waits are bounded: a wait that runs out sets the status word and the kernel
-// finishes with wrong results rather than hanging.
+// bypass the vector L1 (sc1).  A workgroup that is not on the XCD of its head's first one leaves its tiles to those that are.  Waits are
+// bounded: a wait that runs out sets the status word, and what depends on it comes out as NaN (through the data, and for the partial
+// dQ, which the tile below may still overwrite, through its count as well).
 #include "sba_device.hpp"
 #include "sba_host.hpp"
 #include "sba_params.hpp"
@@ -39,7 +40,6 @@ constexpr int kChKeys = 128, kChRows = 32, kChThreads = 512;
 constexpr int kChQStages = 6, kChDoStages = 5;   // Q rows live from the request (3 slots ahead) to the dK/dQ contraction
                                                  // (2 slots behind), dO rows to the dV contraction (1 slot behind)
 constexpr int kChMinSlots = 6;                   // slots per tile: the next tile is claimed late (see below)
-constexpr int kChSpinLimit = 1 << 17;
 
 struct ChLds {   // byte offsets into the dynamic LDS segment
   static constexpr int kRowBytes = lds_stride<128>() * 2;            // 304: padded row of 128 16-bit elements
@@ -168,11 +168,11 @@ __global__ __launch_bounds__(kChThreads) void bwd_chain_kernel(BwdParams p) {
   float* tot_lds = reinterpret_cast<float*>(lds_raw + ChLds::kTot);
 
   // All workgroups of a head must share an XCD (the hand-over relies on one L2): the first to arrive records its
-  // XCC id for the head, the others compare.
+  // XCC id for the head, and one that is elsewhere takes no tile.
   if (threadIdx.x == 0) {
     const int xcc = (int)(__builtin_amdgcn_s_getreg((20) | (0 << 6) | ((4 - 1) << 11)) & 15) + 1;     // HW_REG_XCC_ID
     const int old = atomicCAS(p.chain_head_xcc + head, 0, xcc);
-    if (old != 0 && old != xcc) atomicMax(p.status, kSchedChainXcd);
+    next_lds[8] = old != 0 && old != xcc ? 0x7fffffff : 0;
   }
   // Rows of the packed token axis that belong to no sequence: zero gradients (the reference allocates zeros).
   {
@@ -190,7 +190,7 @@ __global__ __launch_bounds__(kChThreads) void bwd_chain_kernel(BwdParams p) {
   // The first tile.  Tiles are taken from the head's cursor when a workgroup needs one, never ahead of time: the
   // chain wants the tiles of a sequence STARTED in key order, and the workgroups become free in that order only
   // if each takes its next tile late.
-  if (threadIdx.x == 0) next_lds[8] = atomicAdd(p.head_queue + head, 1);
+  if (threadIdx.x == 0 && next_lds[8] == 0) next_lds[8] = atomicAdd(p.head_queue + head, 1);
   __syncthreads();
   int slot_idx = next_lds[8];
   if (slot_idx >= n_tiles) return;
@@ -437,10 +437,11 @@ __global__ __launch_bounds__(kChThreads) void bwd_chain_kernel(BwdParams p) {
               cin = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(crs, qi * 8, 0, kAuxSc1));
               ok = !row_ok || (cin[1] == (uint32_t)J);
               if (__all(ok)) break;
-              if (++spins > kChSpinLimit || ((spins & 255) == 0 && ch_load_flag(p.status) != 0)) { give_up(); break; }
+              if (++spins > p.wait_polls || ((spins & 255) == 0 && ch_load_flag(p.status) != 0)) { give_up(); break; }
               __builtin_amdgcn_s_sleep(1);
             }
           }
+          if (aborted) cin[0] = 0x7fc00000u;
         }
       }
       // K/V of the next tile into the same registers, once they have fed their last MFMAs of this tile; the next
@@ -629,10 +630,11 @@ __global__ __launch_bounds__(kChThreads) void bwd_chain_kernel(BwdParams p) {
             while (true) {
               flag_seen = ch_load_flag(pred_flag);
               if (flag_seen >= kz + 1) break;
-              if (++spins > kChSpinLimit || ((spins & 255) == 0 && ch_load_flag(p.status) != 0)) { give_up(); break; }
+              if (++spins > p.wait_polls || ((spins & 255) == 0 && ch_load_flag(p.status) != 0)) { give_up(); break; }
               __builtin_amdgcn_s_sleep(1);
             }
           }
+          if (flag_seen == kChainBroken) aborted = true;
           // (the loads that follow are issued after the count has been seen: the hardware issues this wave's loads in
           // program order)  The count for the slots to come travels with the partial sums.
           const int soff = qz0 * (DH * 4);
@@ -732,6 +734,9 @@ __global__ __launch_bounds__(kChThreads) void bwd_chain_kernel(BwdParams p) {
 #pragma unroll
               for (int b = 0; b < 4; b++) dq0[4 * a4 + b] += v[b];
             }
+            if (aborted)
+#pragma unroll
+              for (int r = 0; r < 16; r++) dq0[r] = NAN;
           }
           if (J > 0 && kz + 1 < n && !aborted) { ch_flag_request(flag_late, pred_flag); late_pending = true; }
           // dq0[4a + b]: row qz0 + col, column 32c + 8a + 4*half + b.
@@ -752,7 +757,7 @@ __global__ __launch_bounds__(kChThreads) void bwd_chain_kernel(BwdParams p) {
         }
         if (out == 0 && s >= 1 && s - 1 < n) bump(cd_stage, kChDoStages);
         if (do_dq) {
-          if (!final_rows) { pub_flag = my_flag; pub_count = kz + 1; }
+          if (!final_rows) { pub_flag = my_flag; pub_count = aborted ? kChainBroken : kz + 1; }
         }
         if (has_z) bump(cq_stage, kChQStages);
         lds_barrier();

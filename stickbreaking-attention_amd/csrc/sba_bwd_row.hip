@@ -14,8 +14,9 @@
 // its own; the same wave of the tile below reads flag and partial results with sc1 (served by the L2, never by the vector L1).  All
 // tiles of a (head, sequence) run on one XCD, i.e. on one L2: (head, sequence) belongs to one of 8 queues (row_queue), a workgroup takes
 // tiles from queue blockIdx % 8 (workgroups are dealt to the XCDs in turn), and every workgroup checks its XCC id against the first
-// of its queue.  Progress: tiles are taken in list order, a tile waits only for one that was taken before it, so every wait ends;
-// the waits are bounded all the same.
+// of its queue: one that is elsewhere leaves.  Progress: tiles are taken in list order, a tile waits only for one that was taken before
+// it, so every wait ends; the waits are bounded all the same.  A tile whose wait ran out passes on NaN and a count that says so
+// (kChainBroken; data alone would not do, the tile above may still overwrite it), and stores NaN: no wrong number leaves the kernel.
 //
 // What bounds it: per 32 x 32 block and wave 40 MFMAs (1280 cycles), 320 vector-ALU instructions and 48 KB of LDS reads, two waves per
 // SIMD.  The waves of a SIMD (w and w + 4) are kept out of step: one contracts the block of the step before at the start of a
@@ -147,17 +148,17 @@ __device__ __forceinline__ void add_rem_rows(f32x16& acc, const typename Elem<T>
 }
 
 // Until the tile above has passed on more than t key blocks: how many it has.
-__device__ __forceinline__ int wait_for(const int32_t* pred, int t, int32_t* status, int lane) {
+__device__ __forceinline__ int wait_for(const int32_t* pred, int t, int polls, int32_t* status, int lane) {
   int v = 0;
 #pragma unroll 1
-  for (int spins = 0; spins < (1 << 20); spins++) {
+  for (int spins = 0; spins < polls; spins++) {
     asm volatile("s_nop 4\n\tglobal_load_dword %0, %1, %2 sc1\n\ts_waitcnt vmcnt(0)" : "=v"(v) : "v"(0), "s"(pred) : "memory");
     v = __builtin_amdgcn_readfirstlane(v);
     if (v > t) return v;
     __builtin_amdgcn_s_sleep(1);
   }
   if (lane == 0) atomicMax(status, kSchedChainTimeout);
-  return 0x7fffffff;      // no later wait of this tile
+  return kChainBroken;      // no later wait of this tile
 }
 
 template <typename T, int DH, bool kAddRem>
@@ -181,7 +182,7 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
   if (threadIdx.x == 0) {
     const int xcc = (int)(__builtin_amdgcn_s_getreg((20) | (0 << 6) | ((4 - 1) << 11)) & 15) + 1;     // HW_REG_XCC_ID
     const int old = atomicCAS(p.chain_head_xcc + queue, 0, xcc);
-    if (old != 0 && old != xcc) atomicMax(p.status, kSchedChainXcd);
+    *reinterpret_cast<int*>(lds_raw) = old != 0 && old != xcc;
   }
   // Rows of the packed token axis that belong to no sequence: zero gradients.
   {
@@ -199,6 +200,11 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
       }
     }
   }
+
+  // A workgroup that is not on its queue's XCD leaves the tiles to those that are.
+  __syncthreads();
+  if (__builtin_amdgcn_readfirstlane(*reinterpret_cast<int*>(lds_raw))) return;
+  __syncthreads();
 
   // Where a lane reads and writes in the panels: 64-byte rows whose 16-byte chunks are XORed with (row >> 2) & 3.
   const int sw = (col >> 2) & 3, s15 = lane & 15, g = (lane >> 4) & 1;
@@ -362,6 +368,12 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
             for (int c = 2 * kk; c < 2 * kk + 2; c++) acc = Elem<T>::mfma(tr_pair<T>(e0 + 1024 * c, e1 + 1024 * c), wf[c], acc);
           }
       }
+      if (seen_count == kChainBroken) {      // (as a product: 16 registers set in a branch spilled 21 in the loop)
+        vec8 nans;
+#pragma unroll
+        for (int i = 0; i < 8; i++) nans[i] = (T)NAN;
+        acc = Elem<T>::mfma(nans, nans, acc);
+      }
       asm volatile("s_waitcnt vmcnt(0)" : "+v"(c0), "+v"(c1), "+v"(c2), "+v"(c3)::"memory");
 #pragma unroll
       for (int r = 0; r < 4; r++) { acc[r] += c0[r]; acc[4 + r] += c1[r]; acc[8 + r] += c2[r]; acc[12 + r] += c3[r]; }      // (zeros without a tile above)
@@ -456,7 +468,7 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
     };
     // What the tile above left of block t is asked for, once it is there.
     auto request_above = [&](int t) {
-      if (seen_count <= t) seen_count = wait_for(pred, t, p.status, lane);
+      if (seen_count <= t) seen_count = wait_for(pred, t, p.wait_polls, p.status, lane);
       const float* src = part + (int64_t)t * (kPieces * 1024);
       asm volatile("s_nop 4\n\tglobal_load_dwordx4 %0, %4, %5 sc1\n\tglobal_load_dwordx4 %1, %4, %5 offset:1024 sc1\n\t"
                    "global_load_dwordx4 %2, %4, %5 offset:2048 sc1\n\tglobal_load_dwordx4 %3, %4, %5 offset:3072 sc1"
@@ -500,7 +512,7 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
       // The key blocks that are complete are passed on; what the tile above left of the one that is contracted next is asked for.
       const int tn = late ? t - 1 : t, block = block_of(tn);
       const bool any = tn >= 0 && (kWide || block < n);
-      if (lane == 0) *flag = kWide ? block : block - 1;      // (the one before was this wave's last)
+      if (lane == 0) *flag = seen_count == kChainBroken ? kChainBroken : kWide ? block : block - 1;      // (the one before was this wave's last)
       seen_count = max(seen_count, count);
       if (has_pred && any) request_above(block);
       else c0 = c1 = c2 = c3 = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -523,7 +535,7 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
     }
     // The last results are passed on.
     vm_wait<0>();
-    if (lane == 0) *flag = n;
+    if (lane == 0) *flag = seen_count == kChainBroken ? kChainBroken : n;
     if (w_first < L) {
       const RowSink<T> dq_sink = make_row_sink<T>((T*)p.dq.ptr + seq_id * p.dq.sb + head * p.dq.sh + tok0 * p.dq.st, p.dq.st, L, DH);
 #pragma unroll

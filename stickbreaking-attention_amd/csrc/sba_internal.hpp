@@ -26,5 +26,7 @@ struct BackwardRoute {
   int32_t form, heads;
 };
 int backward_route(const SbaArgs* a, BackwardRoute* out);
+// One pass of sba_bwd whose tiles wait for each other for so many polls only (a workspace for all heads).
+int backward_with_polls(const SbaArgs* a, int32_t polls);
 
 }  // namespace sba

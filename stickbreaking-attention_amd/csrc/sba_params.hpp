@@ -31,10 +31,13 @@ struct Tile {
 //   kLoadScalar  : what is left (head_dim below 8, or a sequence whose rows span 2 GiB): element by element.
 enum : int { kLoadScalar = 0, kLoadAligned = 1, kLoadPadded = 2 };
 
+// A count of handed-over blocks that says: all of them, but what was handed over is not to be had (a wait ran out further up).
+constexpr int kChainBroken = 0x7fffffff;
+
 // Slots of the scheduler's `counts` array.
 enum : int { kCountQ = 0, kCountK = 1, kCountStatus = 2, kCountCovered = 3 };
 // Values of counts[kCountStatus].
-enum : int { kSchedOk = 0, kSchedBadCu = 1, kSchedCarryOverflow = 2, kSchedChainTimeout = 3, kSchedChainXcd = 4 };
+enum : int { kSchedOk = 0, kSchedBadCu = 1, kSchedCarryOverflow = 2, kSchedChainTimeout = 3 };
 
 struct SchedParams {
   const void* cu;          // NULL: fixed-length mode
@@ -124,8 +127,9 @@ struct BwdParams {
   uint32_t* chain_c;           // key tiles: [head][row] {fp32 C below the reader's tile, tag = index of the reader's tile};
                                // row tiles: [8], next tile not yet taken, per queue
   int32_t* chain_flags;        // [head][tile slot][8]: per wave, row (key) blocks whose partial result is complete
-  int32_t* chain_head_xcc;     // [head] (row tiles: [queue]): XCC id + 1 of its workgroups (0 = none yet)
+  int32_t* chain_head_xcc;     // [head] (row tiles: [queue]): XCC id + 1 of its first workgroup (0 = none yet); those on other XCDs leave
   int32_t* status;             // the scheduler's status word; the kernel raises it when a wait runs out
+  int32_t wait_polls;          // polls after which a wait runs out: what depends on it comes out as NaN
   int64_t chain_rows;          // rows (row tiles: key blocks) per head in chain_dq / chain_c
   int32_t chain_by_slot;       // row tiles: a sequence's key blocks lie at 8 * its first slot of the list (else at 9/256 * its first token)
   int64_t chain_sb;            // fixed-length mode: rows per batch element (0 in packed mode)

@@ -432,5 +432,6 @@ PYBIND11_MODULE(_sba_torch, m) {
     check(sba::backward_route((const SbaArgs*)(uintptr_t)args, &r), "backward_route");
     return std::make_tuple(r.form, r.heads);
   });
+  m.def("backward_with_polls", [](uint64_t args, int32_t polls) { check(sba::backward_with_polls((const SbaArgs*)(uintptr_t)args, polls), "sba_bwd"); });
   m.def("version", &sba_version);
 }

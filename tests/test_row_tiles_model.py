@@ -69,6 +69,28 @@ def test_every_head_is_in_one_queue(heads):
             assert max(units) - min(units) <= heads % 8, (rank, units)
 
 
+def test_tiles_of_a_queue_stay_on_one_xcd():
+    """Whatever XCDs the workgroups of a queue land on: those that are not where the first one is leave, the others take every tile, in list
+    order, so that a tile never waits for one that nobody has taken."""
+    rng = random.Random(0)
+    for _ in range(200):
+        workgroups = [rng.randint(1, 8) if rng.random() < 0.5 else 1 for _ in range(rng.randint(1, 32))]      # XCD + 1, in order of arrival
+        recorded, stay = 0, []
+        for xcd in workgroups:      # compare and swap
+            recorded = recorded or xcd
+            if xcd == recorded:
+                stay.append(xcd)
+        assert stay and set(stay) == {recorded}
+        cursor, taken = 0, []
+        busy = [0] * len(stay)
+        while cursor < 100:      # whoever is free takes the next one; tile t waits for t - 1, which was taken before it
+            w = min(range(len(stay)), key=lambda i: busy[i])
+            taken.append(cursor)
+            busy[w] += rng.randint(1, 9)
+            cursor += 1
+        assert taken == list(range(100))
+
+
 @pytest.fixture(scope="module")
 def listing(tmp_path_factory):
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"

@@ -278,10 +278,9 @@ def main():
     # (its own recompute of QK^T and dO V^T is not algorithmic work).
     # The chained backwards are ONE kernel with all 10 D pairs of the backward and no recompute of their own; what is timed
     # in front of it is then only what clears its flags (row tiles) and the kernel that rebuilds the forward's products.
-    rows_heads = inp["q"].numel() // D
-    row_tiles = D in (64, 128) and rows_heads >= 64 << 10 and _native.BACKWARD_KERNELS != 1 and (_native.LAST_BWD_KERNELS == 1 or k_dq < 0.4 * k_dkv)
-    if row_tiles or _native.LAST_BWD_KERNELS == 1:
-        kernels = {"fwd_kernel": (k_fwd, 4 * D * pairs), "bwd_row_kernel" if row_tiles else "bwd_chain_kernel": (k_dkv, 10 * D * pairs)}
+    chained = {_native.ROW_TILES: "bwd_row_kernel", _native.KEY_TILES: "bwd_chain_kernel"}.get(_native.LAST_BWD_FORM)
+    if chained:
+        kernels = {"fwd_kernel": (k_fwd, 4 * D * pairs), chained: (k_dkv, 10 * D * pairs)}
         if not save_carry:
             kernels["fwd_kernel(products only)"] = (k_dq, 2 * D * pairs)
     else:

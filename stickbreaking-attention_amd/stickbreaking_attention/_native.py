@@ -69,6 +69,9 @@ DEBUG_CHECK = os.environ.get("SBA_DEBUG_CHECK", "0") == "1"
 BACKWARD_KERNELS = int(os.environ.get("SBA_BACKWARD_KERNELS", "0"))
 # Kernels the last traced backward ran behind its schedule, 1 or 2 (set when TRACE_EVENTS is).
 LAST_BWD_KERNELS = 0
+# ... and which backward it was (of its first heads, where they are split between two).
+TWO_KERNELS, KEY_TILES, ROW_TILES = range(3)
+LAST_BWD_FORM = TWO_KERNELS
 _STATUS_TEXT = {1: "cu_seqlens is not a non-decreasing sequence within [0, total_tokens] (or its leading entry is not 0)",
                 2: "the carry buffer is too small for these sequence lengths (max_seqlens understated?)",
                 3: "one-kernel backward: a workgroup gave up waiting for the tile before its own",
@@ -359,8 +362,9 @@ def _launch_bwd(do, drem, q, k, v, carry, neg_log_acc, cu_seqlens, cu_has_leadin
         if POISON:
             _poison(ws)
         if TRACE_EVENTS is not None:
-            global LAST_BWD_KERNELS
+            global LAST_BWD_KERNELS, LAST_BWD_FORM
             LAST_BWD_KERNELS = lib().sba_bwd_kernels(ctypes.byref(a))
+            LAST_BWD_FORM = ext().backward_route(ctypes.addressof(a))[0]
         _check(lib().sba_bwd(ctypes.byref(a)), "sba_bwd")
         if DEBUG_CHECK:
             check_status(ws, "sba_bwd")

@@ -8,7 +8,7 @@ from stickbreaking_attention import _native
 
 pytestmark = pytest.mark.gpu
 
-TWO_KERNELS, KEY_TILES, ROW_TILES = range(3)
+TWO_KERNELS, KEY_TILES, ROW_TILES = _native.TWO_KERNELS, _native.KEY_TILES, _native.ROW_TILES
 
 
 def args(heads, dim, lengths, kernels=0, exact=False):

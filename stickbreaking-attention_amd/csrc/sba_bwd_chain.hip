@@ -295,7 +295,7 @@ __global__ __launch_bounds__(kChThreads) void bwd_chain_kernel(BwdParams p) {
       const float* c2 = p.carry + (int64_t)head * p.carry_head_stride + next_tile.carry_base + carry_offset(4 * f.J + g, n_qt) - (int64_t)kBlockQ * f.J;
       const int r = kChRows * (f.nb - 1 - k) + col;
       drem_r = (T)0.f;
-      if (p.d_rem.ptr && r < f.L)
+      if (p.d_rem.ptr && f.n > k && r < f.L)      // (a tile of one row block: r is negative for the second)
         drem_r = ((const T*)p.d_rem.ptr)[next_tile.seq_id * p.d_rem.sb + head * p.d_rem.sh + (f.tok0 + r) * p.d_rem.st];
       prod_r = f.n > k ? c2[r] : 1.f;
     };

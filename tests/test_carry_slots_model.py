@@ -212,3 +212,15 @@ def test_model_flags_a_skip_test_that_counts_rows_beyond_the_end(L, dq_kt, dkv):
     written_prefix = dq_prefix_writes(L, 0, dq_kt)
     assert not dkv_reads(L, 0, dkv, rows_beyond_end_count=True)[1] <= written_prefix
     assert dkv_reads(L, 0, dkv)[1] <= written_prefix
+
+
+def test_key_tiles_ask_for_no_row_outside_their_sequence():
+    """Key tiles (csrc/sba_bwd_chain.hip) fetch a row block's scalars ahead: blocks 0 and 1 of the next tile while the one before ends, block
+    s + 2 in slot s.  Block k is rows 32 (nb - 1 - k) on; a tile of one block has no block 1 (its rows would lie in front of the sequence)."""
+    for L in range(1, 700):
+        nb = cdiv(L, 32)
+        for J in range(cdiv(L, 128)):
+            n = nb - 4 * J
+            fetched = [k for k in (0, 1) if n > k] + [s + 2 for s in range(n) if s + 2 < n]
+            assert sorted(fetched) == list(range(n))
+            assert all(128 * J <= 32 * (nb - 1 - k) < L for k in fetched), (L, J)

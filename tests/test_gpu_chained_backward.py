@@ -157,6 +157,21 @@ def test_chained_backward_fixed_length(gpu_device, native_checked):
             tol_check(name, a[b], r, torch.bfloat16, f"chained fixed-length batch {b}")
 
 
+def test_tiny_sequences_and_a_gradient_at_the_start_of_its_memory(gpu_device, native_checked):
+    """Sequences of one row block, many to a workgroup, and d_rem at the first byte of a device allocation: nothing in front of it is asked
+    for (the prefetch of a tile's second row block, which such a tile has not, would lie 32 rows before its first)."""
+    lengths, H = [8, 3, 32, 1, 17, 31] * 60, 8
+    host, dev_t, cu = small_case(H, 128, lengths, torch.bfloat16, seed=79)
+    memory = torch.empty(32 << 20, dtype=torch.bfloat16, device=gpu_device)
+    first = memory[:dev_t[4].numel()].view(dev_t[4].shape)
+    first.copy_(dev_t[4])
+    assert sum(lengths) * H < 64 << 10      # (key tiles)
+    one = grads_varlen(native_checked, 2, [*dev_t[:4], first], cu, lengths, False)
+    ref = orc.varlen_stream(*host[:3], cu, do=host[3], drem=host[4], dtype=torch.float64, heads=[0, 7])
+    for name, a, r in zip(("dq", "dk", "dv"), one, ref[2:]):
+        tol_check(name, a[[0, 7]], r[[0, 7]], torch.bfloat16, "tiny sequences")
+
+
 def test_chained_backward_in_head_groups(gpu_device, native_checked):
     """A backward workspace too small for all heads: the heads go through in groups, each group a chained launch of its
     own (its own flags, tags and XCD map); same bits as the single launch."""

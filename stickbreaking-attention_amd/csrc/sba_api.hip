@@ -23,8 +23,8 @@ hipError_t launch_fwd_split(const FwdParams& p, int dtype_is_f16, int max_tiles,
 hipError_t launch_fwd_split_carry_only(const FwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
 hipError_t launch_bwd_dq_split(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
 hipError_t launch_bwd_dkv_split(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
-hipError_t launch_fwd_f32(const FwdParams& p, int max_tiles, hipStream_t stream);
-hipError_t launch_bwd_f32(const BwdParams& p, int64_t heads, int max_q_tiles, int max_k_tiles, hipStream_t stream);
+hipError_t launch_fwd_f32(const FwdParams& p, int64_t rows_heads, int64_t longest, int max_tiles, hipStream_t stream);
+hipError_t launch_bwd_f32(const BwdParams& p, int64_t rows_heads, int64_t longest, int max_q_tiles, int max_k_tiles, hipStream_t stream);
 }  // namespace sba
 
 namespace {
@@ -117,6 +117,8 @@ int plan(const SbaArgs* a, Layout* out, bool row_tiles = false) {
   // kernels, equal sequences of 32768 tokens in all:
   //   length     64           128          192, 256     384          512          768 .. 4096   8192, 16384
   //              0.98 .. 1.01 0.92 .. 0.96 0.80 .. 0.86 0.93 .. 0.96 0.82 .. 0.85 0.79 .. 0.85  0.77 .. 0.85    (8 to 32 heads)
+  //   and over the two kernels alone: 96 tokens 0.91 .. 0.92, 64 1.00, 48 1.06 .. 1.08, 32 0.98 .. 1.01, 24 1.00 .. 1.02, 16 1.03,
+  //   8 1.05, 8 to 64 1.01 .. 1.03: where no sequence has more than 64 the two kernels run.
   // A tile is 256 rows, so 64 K rows x heads give a tile to each compute unit.  Down there, by rows x heads:
   //   64 K       512 .. 1024 tokens 0.77 .. 0.96     2048 tokens 0.86 (4 sequences), 0.97 (2), 1.04 (1)
   //   32 K       512 tokens 0.82 .. 0.97             1024 tokens 0.97 (4 sequences), 1.22 (2 and 1)     2048 tokens 1.25
@@ -129,17 +131,20 @@ int plan(const SbaArgs* a, Layout* out, bool row_tiles = false) {
   //   64 K       1.00         1.00         0.90 .. 1.00 1.03         0.84 .. 0.89 0.80 .. 0.84 0.83 .. 0.92 0.88 .. 1.00
   //   128 .. 512 K 1.20 .. 1.47 1.05 .. 1.26 0.89 .. 1.01 1.02 .. 1.16 0.82 .. 0.99 0.78 .. 0.95 0.76 .. 0.89 0.68 .. 0.81
   //   32 K       0.99         0.92 .. 1.00 1.00         0.97         0.99         1.02 .. 1.19 1.15 .. 1.48
+  // and ragged ones with a mean of 512 to 1061, 7 to 24 heads: one of 16384 beside 260 or 40 tokens 0.78 .. 0.85, 4 of 4096 beside 300
+  // 0.86 .. 0.89, 3 of 5000 beside 64 0.81 .. 0.93, 8 of 2000 beside 20 0.86 .. 0.89, halves of 1000 and 24 0.78 .. 0.91, 12 of 1300 beside 8
+  // 0.88 .. 0.96.
   const int64_t mean_len = fixed ? T : T / B, rows_heads = rows * a->num_heads, mean_heads = mean_len * a->num_heads;
   const bool chain_shape = a->dtype != SBA_F32 && a->head_dim == 128 && (a->num_heads & 7) == 0 && !a->add_remainder;
   if (row_tiles) {
     L.chain = Layout::kRowTiles;
-  } else if (rows_heads >= kRowTilesFrom && a->dtype != SBA_F32 && (a->head_dim == 128 || (a->head_dim == 64 && mean_len >= 512)) && a->backward_kernels != 1 && (chain_shape || a->backward_kernels == 0)) {
+  } else if (rows_heads >= kRowTilesFrom && a->dtype != SBA_F32 && ((a->head_dim == 128 && max_len > 64) || (a->head_dim == 64 && mean_len >= 512)) && a->backward_kernels != 1 && (chain_shape || a->backward_kernels == 0)) {
     // One kernel where its flags were cleared with the schedule ...
     L.one_kernel = chain_shape && (a->backward_kernels == 2 || (max_len <= 128 && mean_len > 96) ||
                                    (a->num_heads <= 32 && mean_heads >= 32 << 10 && max_len * a->num_heads <= 192 << 10));
     if (L.one_kernel || queues_even(a->num_heads, B, rows, max_len)) L.chain = Layout::kRowTiles;
   } else if (chain_shape && (a->backward_kernels == 2 ||
-                             (a->backward_kernels == 0 &&
+                             (a->backward_kernels == 0 && rows_heads < kRowTilesFrom &&
                               (max_len <= 256 || (a->num_heads <= 32 && rows_heads >= 20 << 10 && mean_heads >= 16 << 10))))) {
     L.chain = Layout::kKeyTiles;
     L.one_kernel = true;
@@ -206,6 +211,10 @@ int plan(const SbaArgs* a, Layout* out, bool row_tiles = false) {
   *out = L;
   return SBA_OK;
 }
+
+// Rows per head, and the longest sequence as far as the caller says.
+int64_t rows_of(const SbaArgs* a) { return a->cu_seqlens ? a->total_tokens : a->num_seqs * a->total_tokens; }
+int64_t longest_of(const SbaArgs* a) { return a->max_seqlen > 0 && a->max_seqlen < a->total_tokens ? a->max_seqlen : a->total_tokens; }
 
 size_t elem_size(int dtype) { return dtype == SBA_F32 ? 4 : 2; }
 
@@ -484,7 +493,7 @@ int fwd_on(const SbaArgs* a, char* ws, size_t ws_bytes, bool ws_is_static, bool 
   p.load = row_load(a, {&a->q, &a->k, &a->v, &a->o});
   hipEvent_t* ev = (hipEvent_t*)a->trace_events;
   if (ev && hipEventRecord(ev[0], stream) != hipSuccess) return SBA_ERR_LAUNCH;
-  hipError_t e = (a->dtype == SBA_F32) ? sba::launch_fwd_f32(p, (int)L.max_q_tiles, stream)
+  hipError_t e = (a->dtype == SBA_F32) ? sba::launch_fwd_f32(p, rows_of(a) * a->num_heads, longest_of(a), (int)L.max_q_tiles, stream)
                  : few_tiles(a, a->num_heads, p.load) ? sba::launch_fwd_split(p, a->dtype == SBA_F16, (int)L.max_q_tiles, stream)
                                          : sba::launch_fwd(p, a->dtype == SBA_F16, (int)L.max_q_tiles, stream);
   if (e != hipSuccess) return SBA_ERR_LAUNCH;
@@ -551,9 +560,7 @@ struct Route {
 
 // `group` heads on row tiles: enough tiles for the chip, spread over its XCDs (as for a call of its own, see plan).
 bool row_group(const SbaArgs* a, int64_t group) {
-  const int64_t rows = a->cu_seqlens ? a->total_tokens : a->num_seqs * a->total_tokens;
-  const int64_t longest = a->max_seqlen > 0 && a->max_seqlen < a->total_tokens ? a->max_seqlen : a->total_tokens;
-  return rows * group >= kRowTilesFrom && queues_even(group, a->num_seqs, rows, longest);
+  return rows_of(a) * group >= kRowTilesFrom && queues_even(group, a->num_seqs, rows_of(a), longest_of(a));
 }
 
 int route_of(const SbaArgs* a, Route* out) {
@@ -726,7 +733,7 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* 
   hipEvent_t* ev = (hipEvent_t*)a->trace_events;
   if (ev && first && hipEventRecord(ev[0], stream) != hipSuccess) return SBA_ERR_LAUNCH;
   if (a->dtype == SBA_F32) {
-    if (sba::launch_bwd_f32(p, stat_heads, (int)L.max_q_tiles, (int)L.max_k_tiles, stream) != hipSuccess) return SBA_ERR_LAUNCH;
+    if (sba::launch_bwd_f32(p, rows_of(a) * stat_heads, longest_of(a), (int)L.max_q_tiles, (int)L.max_k_tiles, stream) != hipSuccess) return SBA_ERR_LAUNCH;
     if (ev && last && (hipEventRecord(ev[1], stream) != hipSuccess || hipEventRecord(ev[2], stream) != hipSuccess)) return SBA_ERR_LAUNCH;
     return SBA_OK;
   }

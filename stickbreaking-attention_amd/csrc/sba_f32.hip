@@ -914,17 +914,32 @@ static hipError_t by_head_dim(int D, int load, F&& f) {
   }
 }
 // Whether a call has too few workgroups for split products: a step of a wave takes longer with them, and more code is fetched; they pay
-// where waves share the matrix pipe or sequences are long.  Split / fp32 products, us:
-//   head_dim  64   4 heads, 448 tokens in sequences of up to 256 (112 workgroups)  kernels 45.4 / 40.6
-//             64   1 head, 6143 tokens in sequences of up to 2048 (240)   196 / 208        128: 319 / 360
-//             32   1 head, the same                                       139 / 130        2 heads (16) 141 / 147, 4 heads 151 / 177
-static bool few_workgroups(int D, int64_t tiles) { return tiles * kF32Split <= (D <= 32 ? 256 : 128); }
+// where two workgroups share a compute unit (one takes 32 rows: from 8192 rows x heads on) or, but for the narrowest, where sequences are
+// long.  The first 32 rows of a sequence do not use them, which moves the line for the shortest.  Split products over fp32 products,
+// the three kernels' time on 256 compute units, by rows x heads / 32:
+//   equal sequences of    128           256           512           2048          6143 tokens in 5 of 600 to 2048
+//   head_dim 32   to 256  1.10 .. 1.11  1.08 .. 1.09  1.08          1.05 .. 1.06  1.04
+//                 from 288 1.04 (384)   0.95 .. 0.99  0.98 .. 0.99  0.89 .. 0.94  0.84 .. 0.93
+//   64            to 256  1.12 .. 1.14  1.07 .. 1.09  0.99 .. 1.04  0.94 .. 0.97  0.94
+//                 from 288 1.05 (384)   0.95 .. 0.98  0.92          0.85 .. 0.86  0.82 .. 0.87
+//   96            to 256  1.16 .. 1.18  1.07 .. 1.12  0.99 .. 1.01  0.90 .. 0.95  0.91
+//                 from 288 1.10 (384)   0.93 .. 0.94  0.87 .. 0.90  0.85 .. 0.86  0.79 .. 0.84
+//   128           to 256  1.14 .. 1.17  1.07 .. 1.08  1.00 .. 1.02  0.93 .. 0.94  0.92
+//                 from 288 1.02 (384)   0.91 .. 0.94  0.86 .. 0.89  0.81 .. 0.84  0.78 .. 0.84
+//   (1024, 300 and 700 tokens: 0.94 .. 0.99 to 256, head_dim 32 1.06; 24 of 40 tokens: 0.96 .. 1.01 at 180.)
+static bool few_workgroups(int D, int64_t rows_heads, int64_t longest) {
+  return rows_heads <= 32 * (longest <= 128 ? 384 : 256) && (D <= 32 || longest < 1024);
+}
 // ... or sums over head_dim that are too short for them, or a logit scale at which the parts that their logits lack would count (see Split).
-static bool fp32_products_only(int D, int64_t tiles, float scale_log2) { return few_workgroups(D, tiles) || D <= 2 || !(fabsf(scale_log2) <= 1024.f); }
+static bool fp32_products_only(int D, int64_t rows_heads, int64_t longest, float scale_log2) {
+  return few_workgroups(D, rows_heads, longest) || D <= 2 || !(fabsf(scale_log2) <= 1024.f);
+}
 
-hipError_t launch_fwd_f32(const FwdParams& call, int max_tiles, hipStream_t stream) {
+// `rows_heads`, `longest`: of the caller's call, also where the backward takes its heads through in groups, which then give the bits of one
+// pass.
+hipError_t launch_fwd_f32(const FwdParams& call, int64_t rows_heads, int64_t longest, int max_tiles, hipStream_t stream) {
   FwdParams p = call;
-  p.fp32_products = fp32_products_only(p.head_dim, (int64_t)max_tiles * p.num_heads, p.scale_log2);
+  p.fp32_products = fp32_products_only(p.head_dim, rows_heads, longest, p.scale_log2);
   return by_head_dim(p.head_dim, p.load, [&](auto dh, auto mode) {
     hipLaunchKernelGGL((fwd_f32_kernel<decltype(dh)::value, decltype(mode)::value>), dim3((unsigned)(xcd_sub_grid(max_tiles * p.num_heads, kF32Split) + p.sched.service)),
                        dim3(kThreads), 0, stream, p);
@@ -932,10 +947,9 @@ hipError_t launch_fwd_f32(const FwdParams& call, int max_tiles, hipStream_t stre
   });
 }
 
-// `heads`: of the caller's call, also where the backward takes them through in groups: the groups then give the bits of one pass.
-hipError_t launch_bwd_f32(const BwdParams& call, int64_t heads, int max_q_tiles, int max_k_tiles, hipStream_t stream) {
+hipError_t launch_bwd_f32(const BwdParams& call, int64_t rows_heads, int64_t longest, int max_q_tiles, int max_k_tiles, hipStream_t stream) {
   BwdParams p = call;
-  p.fp32_products = fp32_products_only(p.head_dim, max_q_tiles * heads, p.scale_log2);
+  p.fp32_products = fp32_products_only(p.head_dim, rows_heads, longest, p.scale_log2);
   int dev = 0, cus = 0;
   const hipError_t e = device_cus(&dev, &cus);
   if (e != hipSuccess) return e;

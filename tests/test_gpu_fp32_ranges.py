@@ -1,4 +1,4 @@
-"""From 128 workgroups on the fp32 kernels form their products of bf16 triples.  Workgroups that meet numbers which triples do not hold form
+"""From 8192 rows x heads on the fp32 kernels form their products of bf16 triples.  Workgroups that meet numbers which triples do not hold form
 them of fp32 numbers instead.  Tensors at both ends of fp32's range, alone and with partners that bring the products back to the middle,
 against the float64 oracle, 1e-5 in norm: a gradient is a difference of prefix sums of up to 161 terms, 161 x 2^-24 = 0.96e-5 at worst
 where nothing cancels (measured: up to 1.3e-6).  An operand of 2^-122 whose last bits were lost (those below 2^-133) would be 2^-12 = 2.4e-4
@@ -11,7 +11,7 @@ from test_gpu_parity import NAMES, run_varlen, small_case
 
 pytestmark = pytest.mark.gpu
 
-LENGTHS, HEADS = [1, 33, 64, 161], 8      # (7 tiles per head, 224 workgroups: more than 128, below which triples are not used)
+LENGTHS, HEADS = [1, 33, 64, 161], 32      # (8288 rows x heads, more than which triples are used from)
 ZERO = -1000      # (2.0 ** ZERO is 0 in fp32)
 CASES = {      # exponents added to q, k, v, do, drem
     "middle": (0, 0, 0, 0, 0),

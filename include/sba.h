@@ -152,8 +152,9 @@ typedef struct SbaArgs {
                                   applies and no sequence is longer than 256 tokens, or at most 32 heads have
                                   (total_tokens / num_seqs) * num_heads >= 16 K and rows * heads >= 20 K.  From 64 K on the
                                   kernel on row tiles, with any head count whose heads and sequences spread over the 8 XCDs
-                                  within a seventh, and with add_remainder, also at head_dim 64 where sequences have 512
-                                  tokens or more on average: as the one kernel (head_dim 128) where no sequence is
+                                  within a seventh, and with add_remainder (the two kernels where no sequence has more
+                                  than 64 tokens), also at head_dim 64 where sequences have 512 tokens or more on average:
+                                  as the one kernel (head_dim 128) where no sequence is
                                   longer than 128 tokens and the mean is above 96, or at most 32 heads have (total_tokens /
                                   num_seqs) * num_heads >= 32 K and max_seqlen * num_heads <= 192 K, and else behind a
                                   kernel that clears what its tiles hand over.  Any other head count above 8 that is

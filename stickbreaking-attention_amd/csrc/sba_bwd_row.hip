@@ -21,12 +21,13 @@
 // What bounds it: per 32 x 32 block and wave 40 MFMAs (1280 cycles), 320 vector-ALU instructions and 48 KB of LDS reads, two waves per
 // SIMD.  The waves of a SIMD (w and w + 4) are kept out of step: one contracts the block of the step before at the start of a
 // step, the other at its end (32 heads x 8 x 4096: 4970 -> 4660 us per training pass).  32 heads x 8 x 4096 x 128, one pass of
-// the backward: 4180 us with key tiles (sba_bwd_chain.hip), 3330 us here; 32768 tokens in 25 sequences of up to 4096, 32 heads: 2650 and
-// 2150.  Without the hand-over it would take 3130, without the tile math as well 2590: at 2.1 GHz, the clock that the power limit
+// the backward: 4180 us with key tiles (sba_bwd_chain.hip), 3385 us here; 32768 tokens in 25 sequences of up to 4096, 32 heads: 2650 and
+// 2200.  Either pipe of a SIMD is busy 74 % of the time (62 % on the 25 sequences), both 8 % (6 %); waves wait 37 % (43 %) of theirs.  Without the hand-over it would take 3130, without the tile math as well 2590: at 2.1 GHz, the clock that the power limit
 // leaves, and 2.0 for the products alone.  256 rows per tile, because the hand-over costs 8 bytes per pair / (rows / 256).
 //
-// head_dim 64: half the products per pair and the same element-wise work, which bounds it (320 vector-ALU instructions against 20
-// MFMAs per block and wave).  A key block has four pieces of {dV, dK}, so a step is two blocks and a wave contracts a piece of one of
+// head_dim 64: half the products per pair and the same element-wise work (320 vector-ALU instructions against 20 MFMAs per block and
+// wave); vector ALU busy 45 %, either pipe 61 %, and waves wait 46 % of their time: two waves per SIMD that meet at two barriers per step
+// bound it.  A key block has four pieces of {dV, dK}, so a step is two blocks and a wave contracts a piece of one of
 // them; LDS holds four blocks, Q stays in registers.  (Steps of one block, contracted by every second wave in turn: the wave whose
 // turn it is arrives last at every barrier: 12 heads, 16384 tokens in 10 sequences of up to 3523, 474 us instead of 434.)  Training passes,
 // us, two kernels and here: 484 and 434; 16 heads x 4 x 4096 946 and 763; 8 heads x 8 x 1024 142 and 108.
@@ -147,8 +148,13 @@ __device__ __forceinline__ void add_rem_rows(f32x16& acc, const typename Elem<T>
     }
 }
 
-// Until the tile above has passed on more than t key blocks: how many it has.
-__device__ __forceinline__ int wait_for(const int32_t* pred, int t, int polls, int32_t* status, int lane) {
+// Until the tile above has passed on more than t key blocks: how many it has.  (What only a wait needs is read from the kernel's arguments
+// here and not kept in scalar registers, which the loop around it is short of.)
+__device__ __forceinline__ int wait_for(const int32_t* pred, int t, int lane) {
+  typedef const __attribute__((address_space(4))) BwdParams Args;
+  Args* args = (Args*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(args));
+  const int polls = args->wait_polls;
   int v = 0;
 #pragma unroll 1
   for (int spins = 0; spins < polls; spins++) {
@@ -157,7 +163,7 @@ __device__ __forceinline__ int wait_for(const int32_t* pred, int t, int polls, i
     if (v > t) return v;
     __builtin_amdgcn_s_sleep(1);
   }
-  if (lane == 0) atomicMax(status, kSchedChainTimeout);
+  if (lane == 0) atomicMax(args->status, kSchedChainTimeout);
   return kChainBroken;      // no later wait of this tile
 }
 
@@ -468,7 +474,7 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
     };
     // What the tile above left of block t is asked for, once it is there.
     auto request_above = [&](int t) {
-      if (seen_count <= t) seen_count = wait_for(pred, t, p.wait_polls, p.status, lane);
+      if (seen_count <= t) seen_count = wait_for(pred, t, lane);
       const float* src = part + (int64_t)t * (kPieces * 1024);
       asm volatile("s_nop 4\n\tglobal_load_dwordx4 %0, %4, %5 sc1\n\tglobal_load_dwordx4 %1, %4, %5 offset:1024 sc1\n\t"
                    "global_load_dwordx4 %2, %4, %5 offset:2048 sc1\n\tglobal_load_dwordx4 %3, %4, %5 offset:3072 sc1"

@@ -20,7 +20,7 @@
 //     of dQ (sub-tiles of 32 dealt round robin, one scalar per row exchanged per step) and the ROWS of dK/dV (nothing
 //     exchanged), and add their partial results through LDS at the end, in a fixed order: bit-reproducible.
 // Measured: 12 heads x 128, 6143 tokens in sequences of up to 2048, forward + backward: 1.01 ms with the fp32 instruction, 0.85 ms
-// with triples (forward 0.20, dQ 0.29, dK/dV 0.36); head_dim 64 0.53 and 0.45, 96 0.75 and 0.63, 127 1.20 and 0.95, 32 (4 heads) 0.175 and
+// with triples (forward 0.20, dQ 0.28, dK/dV 0.36); head_dim 64 0.53 and 0.45, 96 0.75 and 0.63, 127 1.20 and 0.95, 32 (4 heads) 0.175 and
 // 0.151.  All nine products but l x l, with the small ones in a sum of their own, would halve the errors and cost more than the gain: 1.09 ms.
 //
 //   fwd_f32_kernel     : keys swept in reverse from the diagonal (as sb_varlen_fwd.py:155-165), running product per row;

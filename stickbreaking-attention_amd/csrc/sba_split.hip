@@ -1,12 +1,17 @@
 // The 16-bit kernels for problems too small to fill the chip with workgroups of 128 query rows (or of a key tile).
 //
 // What bounds such a problem is the time one workgroup needs for its longest row: a wave takes ~0.5 us per 32 keys however
-// empty the chip is.  So a workgroup's four waves work on the SAME 32 query rows (forward, dQ) and split the keys of every
-// step of 128 -- wave w takes the sub-tile 32 w of it, one scalar per row and wave is exchanged through LDS -- or on the same
-// 32 keys (dK/dV) and split the rows, with nothing exchanged.  Four times the workgroups, a quarter of the steps each; the
-// partial sums of the waves are added through LDS at the end, in a fixed order.  The price is that K and V (Q and dO) are
-// staged per 32 rows instead of per 128, which is why these kernels stop paying once the chip is full (the rule stands with
-// the launches).
+// empty the chip is.  So a workgroup's four waves work on the SAME 32 query rows (forward, dQ) and split the keys, or on the same
+// 32 keys (dK/dV) and split the rows.  Four times the workgroups, a quarter of the steps each; the partial sums of the waves are
+// added through LDS at the end, in a fixed order.  The price is that K and V (Q and dO) are staged per 32 rows instead of per 128,
+// which is why these kernels stop paying once the chip is full (the rule stands with the launches).
+//
+// A wave stages the 32 keys (rows) it works on for itself, so nothing waits for another wave's loads.  Forward: a wave takes a
+// contiguous part of the keys and starts from a product of 1; what the waves above have left of the stick is multiplied on at the end (into
+// the sums, and into the recorded products).  dQ: C below a sub-tile is a sum with signs that is rounded with the weights, so the waves take
+// every fourth sub-tile and exchange one number per row and step, with one barrier.  dK/dV: nothing is exchanged.  Against staging together with
+// three barriers per step of 128 keys, us: forward, 1 head x 2048 tokens x 64 19.6 -> 16.2, 4096 36.2 -> 27.9; head_dim 50, 4096 53.6 -> 41.9; training
+// pass of 7 heads, 8191 tokens in 14 sequences of up to 1886, head_dim 50 180 -> 172, 64 135 -> 129.
 #include "sba_device.hpp"
 #include "sba_host.hpp"
 #include "sba_params.hpp"
@@ -67,10 +72,13 @@ __device__ __forceinline__ void reduce_store(float* lds, const f32x16 (&acc)[DH 
 }
 
 template <int DH> struct SplitLds {
-  static constexpr int kTile = kStep * lds_stride<DH>();                              // elements of one staged tensor
-  static constexpr size_t kStage = (size_t)2 * kTile * 2, kSums = (size_t)kWaves * 32 * (DH + 4) * 4;
+  static constexpr int kSub = 32 * lds_stride<DH>();                                  // elements of a wave's part of one staged tensor
+  static constexpr size_t kStage = (size_t)2 * kWaves * kSub * 2, kSums = (size_t)kWaves * 32 * (DH + 4) * 4;
   static constexpr size_t kBytes = kStage > kSums ? kStage : kSums;
 };
+
+// What the lanes of a wave hand each other through LDS of the wave's own needs no barrier, only the order of the accesses.
+__device__ __forceinline__ void wave_fence() { asm volatile("" ::: "memory"); }
 
 // S^T (or dP^T) of a 32-row operand in registers against the 32 rows `rows` of a staged tile.
 template <typename T, int DH>
@@ -103,10 +111,8 @@ __device__ __forceinline__ void contract32(f32x16 (&acc)[DH / 32], const uint32_
 template <typename T, int DH, int kLoad, bool kCarryOnly>
 __global__ __launch_bounds__(kThreads, 2) void fwd_split_kernel(FwdParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
-  __shared__ float xch[2][kWaves][32];
+  __shared__ __attribute__((aligned(16))) float xch[kWaves][32];
   __shared__ float rem_lds[32];
-  T* const k_lds = reinterpret_cast<T*>(lds_raw);
-  T* const v_lds = k_lds + SplitLds<DH>::kTile;
   if (!kCarryOnly && (int)blockIdx.x < p.sched.service) {
     forward_service(p.sched, blockIdx.x);
     return;
@@ -137,14 +143,22 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_split_kernel(FwdParams p) {
   const int qi = q0 + col;
   const int64_t n_qt = (L + kBlockQ - 1) / kBlockQ;
   float* carry = p.carry ? p.carry + (int64_t)head * p.carry_head_stride + tile.carry_base + sub * kSplitRows : nullptr;
-  const int last_key = min(q0 + kSplitRows, L) - 2 + ac, n_kt = last_key < 0 ? 0 : last_key / kStep + 1;
+  const int last_key = min(q0 + kSplitRows, L) - 2 + ac, n_sub = last_key < 0 ? 0 : last_key / 32 + 1;
   const int krow = mfma_row_to_key32(col);
+  auto carry_row = [&](int u) { return carry + carry_offset(u, n_qt) + (tile.origin - kBlockQ * (u >> 2)); };
+  // (Recorded in whole groups of four: the kernels that sweep 64 keys read the upper sub-tile of a pair.)
+  if (carry && wave == 0 && half == 0)
+    for (int u = n_sub; u & 3; u++) carry_row(u)[col] = 1.f;
 
+  // This wave's sub-tiles, the last wave's the uppermost: swept on their own, downwards from a product of 1.
+  const int per = (n_sub + kWaves - 1) / kWaves, top = n_sub - (kWaves - 1 - wave) * per, bottom = max(top - per, 0);
+  T* const k_lds = reinterpret_cast<T*>(lds_raw) + wave * (2 * SplitLds<DH>::kSub);
+  T* const v_lds = k_lds + SplitLds<DH>::kSub;
   const RowSource<T> ksrc = make_row_source<T, kLoad>(kb, p.k.st, L, D), vsrc = make_row_source<T, kLoad>(vb, p.v.st, L, D);
-  TileCopy<T, DH, kStep, kLoad> ck, cv;
-  if (n_kt > 0) {
-    ck.load(ksrc, (n_kt - 1) * kStep);
-    if (!kCarryOnly) cv.load(vsrc, (n_kt - 1) * kStep);
+  TileCopy<T, DH, 32, kLoad, 64> ck, cv;
+  if (top > 0) {
+    ck.load(ksrc, (top - 1) * 32);
+    if (!kCarryOnly) cv.load(vsrc, (top - 1) * 32);
   }
   typename Elem<T>::vec8 qf[DH / 16];
   load_operand<T, kLoad>(qf, make_row_source<T, kLoad>(qb, p.q.st, L, D), qi, half);
@@ -153,48 +167,62 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_split_kernel(FwdParams p) {
   for (int dt = 0; dt < DH / 32; dt++)
 #pragma unroll
     for (int r = 0; r < 16; r++) oacc[dt][r] = 0.f;
-  float prod = 1.f;      // product over the keys of the steps done so far
-  for (int jt = n_kt - 1; jt >= 0; --jt) {
-    const int u = 4 * jt + wave, j0 = 32 * u;                 // this wave's sub-tile
-    const bool active = j0 <= last_key;
-    lds_barrier();
+  float prod = 1.f;      // product over the keys of this wave's sub-tiles done so far
+  for (int u = top - 1; u >= bottom; --u) {
+    const int j0 = 32 * u;
     ck.store(k_lds);
     if (!kCarryOnly) cv.store(v_lds);
-    lds_barrier();
-    if (jt > 0) {
-      ck.load(ksrc, (jt - 1) * kStep);
-      if (!kCarryOnly) cv.load(vsrc, (jt - 1) * kStep);
+    wave_fence();
+    if (u > bottom) {
+      ck.load(ksrc, j0 - 32);
+      if (!kCarryOnly) cv.load(vsrc, j0 - 32);
     }
+    f32x16 s[1];
+    s[0] = scores32<T, DH>(k_lds, qf, krow, half);
     Weights<16> w;
-    w.run = 1.f;
-    float oth = 1.f;
-    if (active) {
-      f32x16 s[1];
-      s[0] = scores32<T, DH>(k_lds + 32 * wave * lds_stride<DH>(), qf, krow, half);
-      const int lim = qi + ac - j0 - 16 * half;
-      if (j0 + 31 > q0 - 1 + ac) w.template front<true>(s, p.scale_log2, lim); else w.template front<false>(s, p.scale_log2, lim);
-      oth = other_half(w.run, half);
-    }
-    if (half == 0) xch[jt & 1][wave][col] = w.run * oth;
-    lds_barrier();
-    float above = prod;
-#pragma unroll
-    for (int x = 0; x < kWaves; x++) {
-      const float y = xch[jt & 1][x][col];
-      if (x > wave) above *= y;
-      prod *= y;
-    }
-    // (every sub-tile of the step is recorded: the kernels that sweep 64 keys read the upper of a pair)
-    if (carry && half == 0) (carry + carry_offset(u, n_qt) + (tile.origin - kBlockQ * (u >> 2)))[col] = above;
-    if (!kCarryOnly && active) {
-      w.back(half ? above : above * oth);                     // the upper half-wave holds the higher keys
+    const int lim = qi + ac - j0 - 16 * half;
+    if (j0 + 31 > q0 - 1 + ac) w.template front<true>(s, p.scale_log2, lim); else w.template front<false>(s, p.scale_log2, lim);
+    const float oth = other_half(w.run, half);
+    if (carry && half == 0) carry_row(u)[col] = prod;
+    const float seed = half ? prod : prod * oth;              // the upper half-wave holds the higher keys
+    prod *= w.run * oth;
+    if (!kCarryOnly) {
+      w.back(seed);
       uint32_t pk[8];
 #pragma unroll
       for (int i = 0; i < 8; i++) pk[i] = pack2<T>(w.t[2 * i], w.t[2 * i + 1]);
-      contract32<T, DH>(oacc, pk, v_lds + 32 * wave * lds_stride<DH>(), half, lane);
+      contract32<T, DH>(oacc, pk, v_lds, half, lane);
     }
+    wave_fence();
+  }
+  // Below the sub-tiles of the waves above: their products come on top.
+  if (half == 0) xch[wave][col] = prod;
+  __syncthreads();
+  float above = 1.f;
+  prod = 1.f;
+#pragma unroll
+  for (int x = kWaves - 1; x >= 0; --x) {
+    if (x == wave) above = prod;
+    prod *= xch[x][col];
+  }
+  if (carry && half == 0 && wave < kWaves - 1) {
+#pragma unroll 4
+    for (int u = bottom; u < top; u++) carry_row(u)[col] *= above;
   }
   if (kCarryOnly) return;
+  if (wave < kWaves - 1) {
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+      f32x4 scale = {1.f, 1.f, 1.f, 1.f};      // of rows 8 g + 4 half ..
+#pragma unroll
+      for (int x = kWaves - 1; x > 0; --x)
+        if (x > wave) scale *= *reinterpret_cast<const f32x4*>(&xch[x][8 * g + 4 * half]);
+#pragma unroll
+      for (int dt = 0; dt < DH / 32; dt++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) oacc[dt][4 * g + r] *= scale[r];
+    }
+  }
   if (wave == 0 && half == 0) {
     rem_lds[col] = prod;
     if (qi < L) {
@@ -211,8 +239,6 @@ template <typename T, int DH, int kLoad>
 __global__ __launch_bounds__(kThreads, DH == 128 ? 1 : 2) void bwd_dq_split_kernel(BwdParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   __shared__ float xch[2][kWaves][32];
-  T* const k_lds = reinterpret_cast<T*>(lds_raw);
-  T* const v_lds = k_lds + SplitLds<DH>::kTile;
   int head, slot, sub;
   xcd_head_tile_sub(blockIdx.x, kSplitSubs, p.num_heads, &head, &slot, &sub);
   if (slot >= p.counts[kCountQ]) {
@@ -242,12 +268,14 @@ __global__ __launch_bounds__(kThreads, DH == 128 ? 1 : 2) void bwd_dq_split_kern
   const int64_t slot0 = (int64_t)head * p.carry_head_stride + tile.carry_base + sub * kSplitRows;
   auto slot_row = [&](int u) { return slot0 + carry_offset(u, n_qt) + (tile.origin - kBlockQ * (u >> 2)); };
 
+  T* const k_lds = reinterpret_cast<T*>(lds_raw) + wave * (2 * SplitLds<DH>::kSub);
+  T* const v_lds = k_lds + SplitLds<DH>::kSub;
   const RowSource<T> ksrc = make_row_source<T, kLoad>(kb, p.k.st, L, D), vsrc = make_row_source<T, kLoad>(vb, p.v.st, L, D);
-  TileCopy<T, DH, kStep, kLoad> ck, cv;
+  TileCopy<T, DH, 32, kLoad, 64> ck, cv;
   float n_prod = 1.f;      // the forward's product above this wave's sub-tile of the next step
   if (n_kt > 0) {
-    ck.load(ksrc, 0);
-    cv.load(vsrc, 0);
+    ck.load(ksrc, 32 * wave);
+    cv.load(vsrc, 32 * wave);
     if (32 * wave <= last_key) n_prod = (p.carry + slot_row(wave))[col];
   }
   typename Elem<T>::vec8 qf[DH / 16], dof[DH / 16];
@@ -277,22 +305,22 @@ __global__ __launch_bounds__(kThreads, DH == 128 ? 1 : 2) void bwd_dq_split_kern
   for (int jt = 0; jt < n_kt; ++jt) {
     const int u = 4 * jt + wave, j0 = 32 * u;                 // this wave's sub-tile
     const bool active = j0 <= last_key;
-    lds_barrier();
+    wave_fence();
     ck.store(k_lds);
     cv.store(v_lds);
-    lds_barrier();
+    wave_fence();
     const float prod_in = n_prod;
     if (jt + 1 < n_kt) {
-      ck.load(ksrc, (jt + 1) * kStep);
-      cv.load(vsrc, (jt + 1) * kStep);
+      ck.load(ksrc, j0 + kStep);
+      cv.load(vsrc, j0 + kStep);
       if (j0 + kStep <= last_key) n_prod = (p.carry + slot_row(u + 4))[col];
     }
     BwdMath<16> m;
     m.tot = m.oth_g = 0.f;
     if (active) {
       f32x16 s[1], dp[1];
-      s[0] = scores32<T, DH>(k_lds + 32 * wave * lds_stride<DH>(), qf, krow, half);
-      dp[0] = scores32<T, DH>(v_lds + 32 * wave * lds_stride<DH>(), dof, krow, half);
+      s[0] = scores32<T, DH>(k_lds, qf, krow, half);
+      dp[0] = scores32<T, DH>(v_lds, dof, krow, half);
       const int lim = row_ok ? qi + ac - j0 - 16 * half : 0;
       if (j0 + 31 > q0 - 1 + ac || q0 + 31 >= L) bwd_math_front<1, true, false>(m, s, dp, p.scale_log2, lim, half, drem, prod_in);
       else bwd_math_front<1, false, false>(m, s, dp, p.scale_log2, lim, half, drem, prod_in);
@@ -310,7 +338,7 @@ __global__ __launch_bounds__(kThreads, DH == 128 ? 1 : 2) void bwd_dq_split_kern
       if (half == 0) (p.prefix + slot_row(u))[col] = below;   // C just below the sub-tile, for the dK/dV kernel
       uint32_t pk[8], dzk[8];
       bwd_math_back<T, 16, false>(m, below + (half ? m.oth_g : 0.f), pk, dzk);
-      contract32<T, DH>(dqacc, dzk, k_lds + 32 * wave * lds_stride<DH>(), half, lane);
+      contract32<T, DH>(dqacc, dzk, k_lds, half, lane);
     }
   }
   T* dqb = (T*)p.dq.ptr + tile.seq_id * p.dq.sb + head * p.dq.sh + (tok0 + q0) * p.dq.st;
@@ -326,8 +354,6 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dkv_split_kernel(BwdParams p)
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   __shared__ __attribute__((aligned(16))) T pz_lds[kWaves][2][32 * kPzStride];
   __shared__ float rem_lds[32];
-  T* const q_lds = reinterpret_cast<T*>(lds_raw);
-  T* const do_lds = q_lds + SplitLds<DH>::kTile;
   constexpr int subs = kBlockK / kSplitRows;
   int head, slot, sub;
   xcd_head_tile_sub(blockIdx.x, subs, p.num_heads, &head, &slot, &sub);
@@ -349,24 +375,22 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dkv_split_kernel(BwdParams p)
   const float* prefix = p.prefix + slot0;
   const float* drem_plane = p.drem_eff + tile.seq_id * p.drem_sb + head * p.stat_sh + tok0;
   const int first_row = k0 + 1 - ac;                          // first row that sees key k0
-  const int t_begin = first_row < L ? first_row / kStep : 0, t_end = first_row < L ? (L + kStep - 1) / kStep : 0;
+  const int i_first = first_row / 32 + wave, i_end = first_row < L ? (L + 31) / 32 : 0;      // this wave's groups of 32 rows: every fourth
 
   const RowSource<T> qsrc = make_row_source<T, kLoad>(qb, p.q.st, L, D), dosrc = make_row_source<T, kLoad>(dob, p.d_o.st, L, D);
-  TileCopy<T, DH, kStep, kLoad> cq, cdo;
+  T* const q_lds = reinterpret_cast<T*>(lds_raw) + wave * (2 * SplitLds<DH>::kSub);
+  T* const do_lds = q_lds + SplitLds<DH>::kSub;
+  TileCopy<T, DH, 32, kLoad, 64> cq, cdo;
   float n_prod = 1.f, n_prefix = 0.f, n_drem = 0.f;
-  auto fetch_row_scalars = [&](int t) {                       // of this wave's rows of step t, where any was recorded
-    const int w_first = kStep * t + 32 * wave, qi = w_first + col;
-    if (w_first < L && k0 <= min(w_first + 31, L - 1) - 1 + ac) {
-      n_prod = carry[qi];
-      n_prefix = prefix[qi];
-      n_drem = qi < L ? drem_plane[qi] : 0.f;
-    }
+  auto fetch_rows = [&](int i) {
+    const int qi = 32 * i + col;
+    cq.load(qsrc, 32 * i);
+    cdo.load(dosrc, 32 * i);
+    n_prod = carry[qi];
+    n_prefix = prefix[qi];
+    n_drem = qi < L ? drem_plane[qi] : 0.f;
   };
-  if (t_begin < t_end) {
-    cq.load(qsrc, t_begin * kStep);
-    cdo.load(dosrc, t_begin * kStep);
-    fetch_row_scalars(t_begin);
-  }
+  if (i_first < i_end) fetch_rows(i_first);
   const int key = k0 + mfma_row_to_key32(col);
   typename Elem<T>::vec8 kf[DH / 16], vf[DH / 16];
   load_operand<T, kLoad>(kf, make_row_source<T, kLoad>(kb, p.k.st, L, D), key, half);
@@ -376,32 +400,24 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dkv_split_kernel(BwdParams p)
   for (int dt = 0; dt < DH / 32; dt++)
 #pragma unroll
     for (int r = 0; r < 16; r++) { dkacc[dt][r] = 0.f; dvacc[dt][r] = 0.f; }
-  for (int t = t_begin; t < t_end; ++t) {
-    lds_barrier();
+  for (int i = i_first; i < i_end; i += kWaves) {
+    wave_fence();
     cq.store(q_lds);
     cdo.store(do_lds);
-    lds_barrier();
+    wave_fence();
     const float prod_in = n_prod, prefix_in = n_prefix, drem = n_drem;
-    if (t + 1 < t_end) {
-      cq.load(qsrc, (t + 1) * kStep);
-      cdo.load(dosrc, (t + 1) * kStep);
-      fetch_row_scalars(t + 1);
-    }
-    const int w_first = kStep * t + 32 * wave, w_last = w_first + 31, qi = w_first + col;
-    // No row of the sequence in this wave's block sees the keys (nothing is recorded for blocks beyond the sequence).
-    if (w_first >= L || k0 > min(w_last, L - 1) - 1 + ac) continue;
-    const T* q_rows = q_lds + 32 * wave * kStride;
-    const T* do_rows = do_lds + 32 * wave * kStride;
+    if (i + kWaves < i_end) fetch_rows(i + kWaves);
+    const int w_first = 32 * i, w_last = w_first + 31, qi = w_first + col;
     f32x16 s[1], dp[1];
 #pragma unroll
     for (int r = 0; r < 16; r++) { s[0][r] = 0.f; dp[0][r] = 0.f; }
     typename Elem<T>::vec8 b[DH / 16];
 #pragma unroll
-    for (int kk = 0; kk < DH / 16; kk++) b[kk] = lds_row8<T>(q_rows, kStride, col, 16 * kk + 8 * half);
+    for (int kk = 0; kk < DH / 16; kk++) b[kk] = lds_row8<T>(q_lds, kStride, col, 16 * kk + 8 * half);
 #pragma unroll
     for (int kk = 0; kk < DH / 16; kk++) s[0] = Elem<T>::mfma(kf[kk], b[kk], s[0]);
 #pragma unroll
-    for (int kk = 0; kk < DH / 16; kk++) b[kk] = lds_row8<T>(do_rows, kStride, col, 16 * kk + 8 * half);
+    for (int kk = 0; kk < DH / 16; kk++) b[kk] = lds_row8<T>(do_lds, kStride, col, 16 * kk + 8 * half);
 #pragma unroll
     for (int kk = 0; kk < DH / 16; kk++) dp[0] = Elem<T>::mfma(vf[kk], b[kk], dp[0]);
     uint32_t pk[8], dzk[8];
@@ -422,8 +438,8 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dkv_split_kernel(BwdParams p)
       const typename Elem<T>::vec8 ap = lds_col8<T>(p_rows, kPzStride, row0, 0, lane), az = lds_col8<T>(z_rows, kPzStride, row0, 0, lane);
 #pragma unroll
       for (int dt = 0; dt < DH / 32; dt++) {
-        dvacc[dt] = Elem<T>::mfma(ap, lds_col8<T>(do_rows, kStride, row0, 32 * dt, lane), dvacc[dt]);
-        dkacc[dt] = Elem<T>::mfma(az, lds_col8<T>(q_rows, kStride, row0, 32 * dt, lane), dkacc[dt]);
+        dvacc[dt] = Elem<T>::mfma(ap, lds_col8<T>(do_lds, kStride, row0, 32 * dt, lane), dvacc[dt]);
+        dkacc[dt] = Elem<T>::mfma(az, lds_col8<T>(q_lds, kStride, row0, 32 * dt, lane), dkacc[dt]);
       }
     }
   }

@@ -40,6 +40,29 @@ def test_lengths_around_the_steps(gpu_device, H, D, attend_current, add_remainde
         assert (a[:, T:] == 0).all(), f"{n}: rows no sequence covers must be zero"
 
 
+@pytest.mark.parametrize("H,D", [(2, 50), (2, 64), (1, 128)])
+@pytest.mark.parametrize("values", ["normal", "slow"])
+def test_waves_with_several_sub_tiles(gpu_device, H, D, values):
+    """Each wave of the forward sweeps a contiguous part of a row's keys, whose products are put on top of each other at the end: rows
+    whose sub-tiles do not divide by the waves, sticks that end within a part and sticks that last over all of them."""
+    lengths = [385, 513, 1000, 1441]
+    T = sum(lengths)
+    g = torch.Generator().manual_seed(H * D)
+    q, k, v, do = (torch.randn(H, T, D, generator=g) for _ in range(4))
+    if values == "slow":
+        q, k = 0.25 * (q + 1), 0.25 * (k - 1)
+    host = [t.bfloat16() for t in (q, k, v, do, torch.randn(H, T, generator=g))]
+    q, k, v, do, drem = (t.to(gpu_device) for t in host)
+    for t in (q, k, v):
+        t.requires_grad_()
+    cu = torch.tensor(np.cumsum(lengths), dtype=torch.int32)
+    o, rem = sb_attn_varlen(q, k, v, cu, max(lengths), zero_start=False)
+    got = (o, rem, *torch.autograd.grad([o, rem], [q, k, v], [do, drem]))
+    ref = orc.varlen_stream(*(t.double() for t in host[:3]), cu, do=host[3].double(), drem=host[4].double(), dtype=torch.float64)
+    for n, a, b in zip(NAMES, got, ref):
+        tol_check(n, a, b, torch.bfloat16, f"H={H} D={D} {values}")
+
+
 class Passing(TorchDispatchMode):
     def __torch_dispatch__(self, func, types, args=(), kwargs=None):
         return func(*args, **(kwargs or {}))

@@ -38,7 +38,7 @@ inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 struct Layout {
   int64_t max_q_tiles, max_k_tiles, carry_slots_per_head;
   // Offsets in the schedule, which a forward can prepare for the backward that follows it ...
-  size_t off_counts, off_q_tiles, off_k_tiles, off_carry_base, off_queue, sched_bytes;
+  size_t off_counts, off_q_tiles, off_k_tiles, off_carry_base, off_queue, off_turns, sched_bytes;
   // ... and in the rest of a backward's workspace, which starts behind it.
   size_t off_prefix, off_drem, off_carry, rest_bytes;
   size_t fwd_bytes, bwd_bytes, carry_bytes;
@@ -169,6 +169,7 @@ int plan(const SbaArgs* a, Layout* out, bool row_tiles = false) {
   if (L.chain == Layout::kRowTiles) {
     // Key blocks of 32 per head.  (Unknown lengths: every sequence that hands any over is longer than 256.)  One more than needed: heads
     // a power of two apart meet in the same cache sets (32 heads x 8 x 4096, one pass of the backward: 3405 us without it, 3385 with it).
+    L.off_turns = off;       off = align_up(off + (size_t)(fixed ? B * cdiv(T, sba::kRowTileRows) : cdiv(T, sba::kRowTileRows) + B) * sizeof(sba::Turn), 256);
     L.rows_by_slot = fixed || a->row_blocks > 0;
     L.chain_rows = fixed ? B * sba::row_blocks(T) + 1 : a->row_blocks > 0 ? (int64_t)a->row_blocks + 1 : rows * 9 / 256 + 2;
     L.row_group = a->num_heads;
@@ -300,6 +301,17 @@ int check_tensor(const SbaTensor& t, bool required, bool fixed) {
 sba::TensorRef ref(const SbaTensor& t, bool fixed) { return sba::TensorRef{t.ptr, fixed ? t.stride_batch : 0, t.stride_head, t.stride_token}; }
 sba::VectorRef vref(const SbaVector& t, bool fixed) { return sba::VectorRef{t.ptr, fixed ? t.stride_batch : 0, t.stride_head, t.stride_token}; }
 
+// Sequences whose row tiles take turns, by the heads of a launch: four (head, sequence) per queue, as far as there are any.  One after the
+// other, the last sequence's longest tile starts when all others are nearly done (12 heads x 4 x 8192: the fullest queue's last tile would
+// end 15 % behind the mean by the keys swept, 7 % when they take turns).  The more take turns, the fewer tiles of a (head, sequence) run at the
+// same time and find in the L2 what the tile above left.  Training passes, us, one after the other / two per queue / four / eight:
+// 12 heads x 4 x 8192 x 128 3356 / 3368 / 3255 / 3260; 16 heads, 16384 tokens in 14 sequences 870 / 867 / 857 / 855; 12 heads x 64, 16384 tokens in 10
+// 432 / 435 / 430 / 433; 32 heads x 8 x 4096 4465 / - / 4483 / 4560.
+int take_turns(int64_t heads) {
+  const int64_t n = 32 / heads;
+  return (int)(n < 1 ? 1 : n > sba::kMostTurns ? sba::kMostTurns : n);
+}
+
 // What the scheduler is asked for: always the query tiles; `for_backward`: the key tiles as well, the tile cursors at zero and
 // what the one-kernel backward needs cleared.
 sba::SchedParams sched_params(const SbaArgs* a, char* ws, const Layout& L, bool for_backward, bool want_carry_base, int key_tile) {
@@ -325,6 +337,11 @@ sba::SchedParams sched_params(const SbaArgs* a, char* ws, const Layout& L, bool 
   sp.head_queue = (int32_t*)(ws + L.off_queue);
   sp.num_heads = a->num_heads;
   sp.key_tile = key_tile;
+  sp.take_turns = 1;
+  if (for_backward && L.chain == Layout::kRowTiles && key_tile == sba::kRowTileRows) {
+    sp.k_turns = (sba::Turn*)(ws + L.off_turns);
+    sp.take_turns = take_turns(L.row_group);
+  }
   return sp;
 }
 
@@ -686,6 +703,7 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* 
   p.d_rem = vref(a->d_rem, fixed);
   p.q_tiles = (const sba::Tile*)(ws + L.off_q_tiles);
   p.k_tiles = (const sba::Tile*)(ws + L.off_k_tiles);
+  if (L.chain == Layout::kRowTiles) p.k_turns = (const sba::Turn*)(ws + L.off_turns);
   p.counts = (const int32_t*)(ws + L.off_counts);
   p.carry_base = (const int64_t*)(ws + L.off_carry_base);
   p.carry = a->recompute_carry ? (const float*)(rest + L.off_carry) : a->carry;

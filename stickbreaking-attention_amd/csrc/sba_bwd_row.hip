@@ -224,28 +224,24 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
   const int cp = kWide ? wave & 3 : wave & 1;           // ... and which 32 columns of it
   const int per_slot = (H + 7) >> 3;       // heads of a tile slot that a queue may hold
 
-  int rank = -1, ranked = -1;              // how many sequences the list begins up to slot `ranked`, less 1
   for (;;) {
     if (threadIdx.x == 0) *reinterpret_cast<int*>(lds_raw) = atomicAdd(cursor, 1);
     __syncthreads();
     const int claim = __builtin_amdgcn_readfirstlane(*reinterpret_cast<int*>(lds_raw));
     __syncthreads();
-    const int slot = claim / per_slot;
-    if (slot >= n_tiles) break;
-    Tile tile = p.k_tiles[slot];
+    const int place = claim / per_slot;
+    if (place >= n_tiles) break;
+    Tile tile = p.k_tiles[place];
+    const int first_slot = __builtin_amdgcn_readfirstlane(p.k_turns[place].first_slot), rank = __builtin_amdgcn_readfirstlane(p.k_turns[place].rank);
     const int L = __builtin_amdgcn_readfirstlane(tile.seq_len), seq_id = __builtin_amdgcn_readfirstlane(tile.seq_id);
-    if (H & 7) {
-      for (int first = ranked + 1; first <= slot; first += 64) rank += __builtin_popcountll(__ballot(first + lane <= slot && p.k_tiles[min(first + lane, slot)].origin == 0));
-      ranked = slot;
-    }
-    const int head = ((queue - row_queue(rank, H)) & 7) + 8 * (claim - slot * per_slot);
+    const int head = ((queue - row_queue(rank, H)) & 7) + 8 * (claim - place * per_slot);
     if (head >= H) continue;
     const int64_t tok0 = __builtin_amdgcn_readfirstlane(tile.seq_start);
     const int64_t carry_base = (int64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)tile.carry_base) |
                                (int64_t)__builtin_amdgcn_readfirstlane((int)(tile.carry_base >> 32)) << 32;
     // The list holds the tiles first to last; they are taken last to first.
     const int n_rt = (L + kRowTile - 1) / kRowTile;
-    const int I = n_rt - 1 - __builtin_amdgcn_readfirstlane(tile.origin) / kRowTile, q0 = I * kRowTile;
+    const int nth = __builtin_amdgcn_readfirstlane(tile.origin) / kRowTile, I = n_rt - 1 - nth, q0 = I * kRowTile, slot = first_slot + nth;
     const bool has_pred = I < n_rt - 1;
     const int n = (min(q0 + kRowTile, L) + kRowKeys - 1) / kRowKeys;      // key blocks of this tile
     const int own = q0 / kRowKeys;                                        // the first of the tile's own rows' keys
@@ -296,8 +292,8 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
       return carry + (carry_offset(u, n_qt) - kBlockQ * (u >> 2));
     };
     // What the row tiles of a (head, sequence) hand down: per key block and wave, the 32 x 32 partial result.  (Sequences of more than one
-    // tile come first in the list, each with 8 key blocks per tile.)
-    const int64_t first_block = p.chain_by_slot ? (int64_t)(slot - __builtin_amdgcn_readfirstlane(tile.origin) / kRowTile) * (kRowTile / kRowKeys) : tok0 * 9 / 256;
+    // tile have the first slots, each with 8 key blocks per tile.)
+    const int64_t first_block = p.chain_by_slot ? (int64_t)first_slot * (kRowTile / kRowKeys) : tok0 * 9 / 256;
     float* part = p.chain_dq + ((int64_t)head * p.chain_rows + first_block) * (kPieces * 1024) + (wave & (kPieces - 1)) * 1024;
     int32_t* flag = p.chain_flags + ((int64_t)head * p.chain_tile_cap + slot) * 8 + wave;
     const int32_t* pred = has_pred ? flag - 8 : flag;
@@ -393,8 +389,9 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
         const f32x4 d0 = __builtin_shufflevector(acc, acc, 0, 1, 2, 3), d1 = __builtin_shufflevector(acc, acc, 4, 5, 6, 7),
                     d2 = __builtin_shufflevector(acc, acc, 8, 9, 10, 11), d3 = __builtin_shufflevector(acc, acc, 12, 13, 14, 15);
         float* dst = part + (int64_t)tc * (kPieces * 1024);
+        // (A store's data is read a wait state after it was issued, which the compiler does not keep for assembly either.)
         asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %5\n\tglobal_store_dwordx4 %0, %2, %5 offset:1024\n\t"
-                     "global_store_dwordx4 %0, %3, %5 offset:2048\n\tglobal_store_dwordx4 %0, %4, %5 offset:3072"
+                     "global_store_dwordx4 %0, %3, %5 offset:2048\n\tglobal_store_dwordx4 %0, %4, %5 offset:3072\n\ts_nop 0"
                      ::"v"(lane16), "v"(d0), "v"(d1), "v"(d2), "v"(d3), "s"(dst) : "memory");
       }
     };

@@ -21,6 +21,11 @@ struct Tile {
   int32_t seq_id;      // sequence index; selects the batch stride in fixed-length mode
   int64_t carry_base;  // first carry slot of the sequence within a head's plane (0 when no carries are laid out)
 };
+// What a row tile (backward on row tiles) has to know of a list in which its sequence's tiles need not follow each other.
+struct Turn {
+  int32_t first_slot;  // of its sequence, in a list that held each sequence's tiles together: number in place of a slot
+  int32_t rank;        // sequences before this one in that list
+};
 
 // How the 16-bit kernels read rows of head_dim elements, by what the tensors allow:
 //   kLoadAligned : head_dim is the kernel's width (64 or 128) and every row starts on a 16-byte boundary: 16-byte loads.
@@ -57,6 +62,8 @@ struct SchedParams {
   int32_t* head_queue;     // backward: per-head cursor into the key-tile list, reset to 0 here
   int32_t num_heads;
   int32_t key_tile;        // keys per key tile (a multiple of 32; what the dK/dV kernel that will run sweeps)
+  Turn* k_turns;           // row tiles: beside k_tiles (else NULL)
+  int32_t take_turns;      // row tiles: sequences whose tiles take turns in the list, up to kMostTurns (1: each sequence's follow each other)
   uint32_t* zero_fill;     // optional: 16-byte aligned region cleared by the launch (the one-kernel backward's flags
   int64_t zero_bytes;      // and tags start every call at zero), a multiple of 16 bytes
   int32_t service;         // workgroups at the head of a forward launch that schedule and clear (0: a scheduler launch did)
@@ -71,6 +78,11 @@ __host__ __device__ inline int64_t row_blocks(int64_t len) { return len > kRowTi
 // Its queue, of 8, for head 0 of the sequence with this rank (the list holds the longest first); head h's is (this + h) % 8.  If the heads do
 // not fill the queues evenly, the fuller ones are others for the next sequence, in an order that goes forth and back (a Gray code).
 __host__ __device__ inline int row_queue(int rank, int heads) { return heads & 7 ? ((rank ^ rank >> 1) * (heads & 7)) & 7 : 0; }
+
+// Sequences of a batch whose row tiles take turns, at most.  The tiles of a group of sequences come by the number of keys they sweep, those with
+// most first: tile t of n of the group's j-th sequence (the first has most tiles) is at place j + sum over the group of max(0, tiles - (n - t)),
+// and the tile above it, t - 1, at a lower one.  (The rule and what it gives stand with take_turns in sba_api.hip.)
+constexpr int kMostTurns = 8;
 
 struct FwdParams {
   TensorRef q, k, v, o;
@@ -98,6 +110,7 @@ struct BwdParams {
   VectorRef d_rem;
   const Tile* q_tiles;
   const Tile* k_tiles;
+  const Turn* k_turns;         // row tiles: beside k_tiles
   const int32_t* counts;
   const int64_t* carry_base;
   const float* carry;          // [head][slot]: the forward's running product per (row, 32-key sub-tile)

@@ -49,12 +49,13 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
   }
   __shared__ int qbins[kBins];
   __shared__ int kbins[kBins];
+  __shared__ int sbins[kBins];      // row tiles: sequences per length class
   __shared__ int scratch[kSchedThreads];
   __shared__ long long carry_run;
   __shared__ unsigned long long row_run;
   __shared__ int status;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = kSchedThreads / 64;
-  for (int i = threadIdx.x; i < kBins; i += kSchedThreads) { qbins[i] = 0; kbins[i] = 0; }
+  for (int i = threadIdx.x; i < kBins; i += kSchedThreads) { qbins[i] = 0; kbins[i] = 0; sbins[i] = 0; }
   if (threadIdx.x == 0) { carry_run = 0; row_run = 0; status = kSchedOk; }
   __syncthreads();
 
@@ -68,6 +69,7 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
     const int cls = min(nq, kBins - 1);
     if (nq) atomicAdd(&qbins[cls], nq);
     if (nk && p.want_key_tiles) atomicAdd(&kbins[cls], nk);
+    if (nk && p.k_turns) atomicAdd(&sbins[cls], 1);
     if (p.row_capacity >= 0 && row_blocks(len) > 0) atomicAdd(&row_run, (unsigned long long)row_blocks(len));
   }
   __syncthreads();
@@ -81,6 +83,7 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
   }
   descending_offsets(qbins, scratch);
   if (p.want_key_tiles) descending_offsets(kbins, scratch);
+  if (p.k_turns) descending_offsets(sbins, scratch);
 
   // Carry layout: exclusive prefix sum of carry_slots(M_s) over sequences (block-wide, chunked).
   if (p.want_carry_base) {
@@ -122,7 +125,7 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
   const int group = min(64, (p.num_seqs + nwaves - 1) / nwaves);
   for (int s0 = wave * group; s0 < p.num_seqs; s0 += nwaves * group) {
     const int s = s0 + lane;
-    int start = 0, len = 0, qbase = 0, kbase = 0;
+    int start = 0, len = 0, qbase = 0, kbase = 0, rank = 0;
     int64_t cbase = 0;
     const bool mine = lane < group && s < p.num_seqs;
     if (mine) {
@@ -133,20 +136,29 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
     const int cls = min(nq, kBins - 1);
     if (nq) qbase = atomicAdd(&qbins[cls], nq);
     if (nk) kbase = atomicAdd(&kbins[cls], nk);
+    if (nk && p.k_turns) rank = atomicAdd(&sbins[cls], 1);
     Tile d;
     d.seq_start = start; d.seq_len = len; d.seq_id = s; d.carry_base = cbase;
     if (nq <= kOwnTiles) {
       for (int t = 0; t < nq; t++) { d.origin = (nq - 1 - t) * kBlockQ; p.q_tiles[qbase + t] = d; }      // heaviest first: the last one
-      for (int t = 0; t < nk; t++) { d.origin = t * p.key_tile; p.k_tiles[kbase + t] = d; }             // ... and the first one
+      for (int t = 0; t < nk; t++) {                                                                     // ... and the first one
+        d.origin = t * p.key_tile;
+        p.k_tiles[kbase + t] = d;
+        if (p.k_turns) p.k_turns[kbase + t] = Turn{kbase, rank};
+      }
     }
     for (uint64_t left = __ballot(nq > kOwnTiles); left; left &= left - 1) {
       const int j = __builtin_ctzll(left);
-      const int nq_j = __shfl(nq, j), nk_j = __shfl(nk, j), qbase_j = __shfl(qbase, j), kbase_j = __shfl(kbase, j);
+      const int nq_j = __shfl(nq, j), nk_j = __shfl(nk, j), qbase_j = __shfl(qbase, j), kbase_j = __shfl(kbase, j), rank_j = __shfl(rank, j);
       Tile e;
       e.seq_start = __shfl(start, j); e.seq_len = __shfl(len, j); e.seq_id = __shfl(s, j);
       e.carry_base = (int64_t)(uint32_t)__shfl((int)cbase, j) | (int64_t)__shfl((int)(cbase >> 32), j) << 32;
       for (int t = lane; t < nq_j; t += 64) { e.origin = (nq_j - 1 - t) * kBlockQ; p.q_tiles[qbase_j + t] = e; }
-      for (int t = lane; t < nk_j; t += 64) { e.origin = t * p.key_tile; p.k_tiles[kbase_j + t] = e; }
+      for (int t = lane; t < nk_j; t += 64) {
+        e.origin = t * p.key_tile;
+        p.k_tiles[kbase_j + t] = e;
+        if (p.k_turns) p.k_turns[kbase_j + t] = Turn{kbase_j, rank_j};
+      }
     }
   }
   __syncthreads();

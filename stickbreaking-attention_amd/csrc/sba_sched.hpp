@@ -108,6 +108,7 @@ __device__ __forceinline__ void forward_service(const SchedParams& p, int wg) {
   if (p.want_key_tiles && ok) {
     const int nk = (s.len + p.key_tile - 1) / p.key_tile;
     if (p.cu == nullptr) total_k = nk * p.num_seqs; else first_k = lane_slot(p, s, nk, &total_k);
+    const int turns = p.take_turns;
     Tile t;
     t.seq_start = 0; t.seq_len = s.len;
     if (p.cu == nullptr) {
@@ -117,17 +118,45 @@ __device__ __forceinline__ void forward_service(const SchedParams& p, int wg) {
       }
       for (int i = threadIdx.x; i < total_k; i += blockDim.x) {
         t.seq_id = i / nk; t.origin = i % nk * p.key_tile; t.carry_base = t.seq_id * carry_slots(s.nq);
-        p.k_tiles[i] = t;
+        int place = i;
+        if (p.k_turns) {      // (sequences of equal length)
+          const int group = t.seq_id / turns * turns, members = min(turns, p.num_seqs - group);
+          place = group * nk + i % nk * members + (t.seq_id - group);
+          p.k_turns[place] = Turn{t.seq_id * nk, t.seq_id};
+        }
+        p.k_tiles[place] = t;
       }
       for (int i = threadIdx.x; i < p.num_seqs; i += blockDim.x) p.carry_base[i] = i * carry_slots(s.nq);
     } else {
       t.carry_base = 0;
+      int sequences, rank = 0;      // of this lane's sequence
+      if (p.k_turns) rank = lane_slot(p, s, nk > 0, &sequences);
       for (int seq = 0; seq < p.num_seqs; seq++) {
         const int nq = __builtin_amdgcn_readlane(s.nq, seq), n = __builtin_amdgcn_readlane(nk, seq);
         const int q0 = __builtin_amdgcn_readlane(first_q, seq), k0 = __builtin_amdgcn_readlane(first_k, seq);
         t.seq_start = __builtin_amdgcn_readlane(s.start, seq); t.seq_len = __builtin_amdgcn_readlane(s.len, seq); t.seq_id = seq;
         for (int i = threadIdx.x; i < nq; i += blockDim.x) { t.origin = (nq - 1 - i) * kBlockQ; p.q_tiles[q0 + i] = t; }
-        for (int i = threadIdx.x; i < n; i += blockDim.x) { t.origin = i * p.key_tile; p.k_tiles[k0 + i] = t; }
+        if (p.k_turns) {
+          // The group's sequences, by rank, and where the first one's tiles begin (an empty sequence is in none).
+          const int mine = __builtin_amdgcn_readlane(rank, seq), group = mine / turns * turns;
+          int tiles[kMostTurns], start = k0;
+#pragma unroll
+          for (int j = 0; j < kMostTurns; j++) {
+            const uint64_t at = __ballot(nk > 0 && j < turns && rank == group + j);
+            tiles[j] = at ? __builtin_amdgcn_readlane(nk, __builtin_ctzll(at)) : 0;
+            if (j == 0 && at) start = __builtin_amdgcn_readlane(first_k, __builtin_ctzll(at));
+          }
+          for (int i = threadIdx.x; i < n; i += blockDim.x) {
+            int place = start + (mine - group);
+#pragma unroll
+            for (int j = 0; j < kMostTurns; j++) place += max(0, tiles[j] - (n - i));
+            t.origin = i * p.key_tile;
+            p.k_tiles[place] = t;
+            p.k_turns[place] = Turn{k0, mine};
+          }
+        } else {
+          for (int i = threadIdx.x; i < n; i += blockDim.x) { t.origin = i * p.key_tile; p.k_tiles[k0 + i] = t; }
+        }
         if (threadIdx.x == 0) p.carry_base[seq] = t.carry_base;
         t.carry_base += carry_slots(nq);
       }

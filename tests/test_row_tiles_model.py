@@ -56,6 +56,35 @@ def test_places_by_slot_do_not_overlap():
             slot0 += cdiv(n, 256)
 
 
+@pytest.mark.parametrize("turns", [1, 2, 3, 5, 8])
+def test_tiles_that_take_turns(turns):
+    """Places in the list (forward_service in csrc/sba_sched.hpp): each is taken once, the tile above comes first, and in a group those with
+    most keys do."""
+    rng = random.Random(turns)
+    for _ in range(200):
+        lengths = [rng.choice([0, 1, 256, 257, 512, 513, rng.randint(1, 5000)]) for _ in range(rng.randint(1, 64))]
+        order = sorted(range(len(lengths)), key=lambda s: -cdiv(lengths[s], 128))
+        nk = [cdiv(lengths[s], 256) for s in order if lengths[s]]      # by rank
+        first = [sum(nk[:r]) for r in range(len(nk))]
+        at = {}
+        for rank, n in enumerate(nk):
+            group = rank // turns * turns
+            members = [nk[r] if r < min(group + turns, len(nk)) else 0 for r in range(group, group + 8)]
+            for t in range(n):
+                place = first[group] + (rank - group) + sum(max(0, m - (n - t)) for m in members)
+                assert place not in at
+                at[place] = (rank, t, n - t, group)
+        assert sorted(at) == list(range(sum(nk)))
+        where = {v[:2]: k for k, v in at.items()}
+        for (rank, t), k in where.items():
+            assert t == 0 or where[rank, t - 1] < k
+        for k in range(1, len(at)):
+            assert at[k][3] >= at[k - 1][3] and (at[k][3] > at[k - 1][3] or at[k][2] <= at[k - 1][2])
+    for seqs, n in ((1, 3), (4, 32), (9, 1), (17, 5)):      # equal lengths
+        places = sorted(s // turns * turns * n + t * min(turns, seqs - s // turns * turns) + s % turns for s in range(seqs) for t in range(n))
+        assert places == list(range(seqs * n))
+
+
 @pytest.mark.parametrize("heads", [1, 4, 7, 8, 12, 20, 32])
 def test_every_head_is_in_one_queue(heads):
     """... of every sequence, and 8 sequences in a row fill the queues alike."""
@@ -206,3 +235,19 @@ def test_registers_on_their_way_are_left_alone(listing):
         for block in state:
             run(block, lambda *_: None)
         assert not bad, f"{name}: {bad[:5]}"
+
+
+def test_stored_registers_outlive_their_store_by_a_wait_state(listing):
+    """The hardware reads the data of a store of more than 8 bytes a wait state after it was issued: a vector instruction that writes those
+    registers must not be the next one.  The compiler keeps this for its own stores and not for those in inline assembly."""
+    for name, lines in listing.items():
+        data = set()
+        for line in lines:
+            text = line.split(";")[0].strip()
+            if not text or text.endswith(":") or text.startswith("."):
+                continue
+            op, _, rest = text.partition(" ")
+            if op.startswith("v_") and not op.startswith(("v_cmp", "v_readlane", "v_readfirstlane")):
+                assert not registers(re.split(r",(?![^\[]*\])", rest)[0], "v") & data, f"{name}: {text}"
+            wide = re.match(r"(global|buffer|scratch)_store_dwordx[34]", op)
+            data = registers(re.split(r",(?![^\[]*\])", rest)[1 if op.startswith(("global", "scratch")) else 0], "v") if wide else set()

@@ -32,6 +32,24 @@ def test_every_product_read_was_written(fwd_kt, ac):
         assert bits(row_tile_reads, L, ac) & ~bits(forward_writes, L, ac, fwd_kt) == 0, f"L={L}"
 
 
+def test_tiles_are_laid_from_the_end():
+    """Row tiles of a sequence: every row, and every block of 32 keys, is in one; the keys a tile sweeps are those it, or the tiles below it,
+    own, and those it hands down belong to the tiles below; the tile above sweeps 8 blocks more."""
+    for L in range(1, 1400):
+        rows, blocks, above = [], [], None
+        for nth in range(cdiv(L, 256)):
+            q_end = cdiv(L, 32) * 32 - 256 * nth
+            q0 = max(q_end - 256, 0)
+            n, own, waves = q_end // 32, q0 // 32, (q_end - q0) // 32
+            assert q_end > q0 and 1 <= waves <= 8 and n == own + waves and (waves == 8 or own == 0)
+            assert above is None or above[0] == n + 8 and above[1] == n      # what the tile above hands down are this tile's blocks
+            above = n, own
+            rows += [r for w in range(waves) for r in range(q0 + 32 * w, min(q0 + 32 * w + 32, L))]
+            blocks += range(own, n)
+            assert all(q0 + 32 * w < L for w in range(waves))
+        assert above[1] == 0 and sorted(rows) == list(range(L)) and sorted(blocks) == list(range(cdiv(L, 32)))
+
+
 def test_partial_results_of_neighbours_do_not_overlap():
     """The blocks of a sequence start at floor(9 start / 256) of the head's; sequences of up to 256 rows hand nothing over."""
     for L in range(257, 1300):

@@ -399,8 +399,8 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
       }
     };
     const bool late = wave >= 4;      // (waves w and w + 4 share a SIMD)
-    // Of a key block: P and dZ of this wave's rows, into LDS ...
-    auto front = [&](int j0, bool seen, lds_u8* kt, lds_u8* ex, float prod_in, u32x4 (&dz)[2]) {
+    // Of a key block: P and dZ of this wave's rows, into LDS (`behind_weights` is done behind the first of them) ...
+    auto front = [&](int j0, bool seen, lds_u8* kt, lds_u8* ex, float prod_in, u32x4 (&dz)[2], auto behind_weights) {
       if (seen) {
         f32x16 s, dp;
 #pragma unroll
@@ -436,6 +436,7 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
         }
         RowMath<T> m;
         m.weights(s, half, prod_in, ex + wr_a);
+        behind_weights();
 #pragma unroll
         for (int kk = 0; kk < kVAhead; kk++) va[kk] = v_op(kk);
         __builtin_amdgcn_sched_barrier(0);
@@ -447,6 +448,8 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
         }
         m.gradients(dp, half, drem, prefix, dz);
       } else {
+        behind_weights();
+        vm_wait<0>();
         dz[0] = dz[1] = u32x4{0, 0, 0, 0};
         lds_put(ex + wr_a, dz[0]);
         lds_put(ex + (wr_a ^ 16), dz[0]);
@@ -498,27 +501,36 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
         asm volatile("s_nop 4\n\tglobal_load_dword %0, %2, %4 sc1\n\tglobal_load_dword %1, %3, %5"
                      : "=&v"(r_count), "=&v"(r_prod) : "v"(0), "v"(row_c * 4), "s"(pred), "s"(product_at(t + 1)) : "memory");
       } else {
-        asm volatile("s_nop 4\n\tglobal_load_dword %0, %3, %5 sc1\n\tglobal_load_dword %1, %4, %6\n\tglobal_load_dword %2, %4, %7"
-                     : "=&v"(r_count), "=&v"(r_prod), "=&v"(r_prod2)
-                     : "v"(0), "v"(row_c * 4), "s"(pred), "s"(product_at(2 * t + 2)), "s"(product_at(2 * t + 3)) : "memory");
+        asm volatile("s_nop 4\n\tglobal_load_dword %0, %2, %3\n\tglobal_load_dword %1, %2, %4"
+                     : "=&v"(r_prod), "=&v"(r_prod2)
+                     : "v"(row_c * 4), "s"(product_at(2 * t + 2)), "s"(product_at(2 * t + 3)) : "memory");
       }
       request_kv(t + 1);
+      const int tn = late ? t - 1 : t, block = block_of(tn);      // contracted in this step
+      const bool any = tn >= 0 && (kWide || block < n);
+      // The key blocks that are complete are passed on: the stores of the last one left before this step's four loads and have arrived when the
+      // first weights are there.  (Passed on at the end of the step, and the count of the tile above read at the start of it, that count was one too
+      // small in 6 steps of 10 at head_dim 64, 1 to 2 of 10 at 128, and a wave spent 800 to 2300 cycles reading it again.  Training passes,
+      // us before / after: 12 heads x 64, 16384 tokens in 10 sequences 415 / 405; 32 heads x 8 x 4096 x 128 4366 / 4298; 12 x 4 x 8192 x 128 3132 / 3106.)
+      auto pass_on = [&] {
+        vm_wait<4>();
+        if (lane == 0) *flag = seen_count == kChainBroken ? kChainBroken : kWide ? block : block - 1;      // (the one before was this wave's last)
+      };
       if constexpr (kWide) {
-        front(kRowKeys * t, seen, kt, ex, prod_in, dz);
+        front(kRowKeys * t, seen, kt, ex, prod_in, dz, pass_on);
         asm volatile("s_waitcnt vmcnt(2)\n\tv_mov_b32 %0, %2\n\tv_readfirstlane_b32 %1, %3"
                      : "=&v"(n_prod), "=s"(count) : "v"(r_prod), "v"(r_count) : "memory");
       } else {
         const bool seen1 = has_rows && kRowKeys * first <= last_seen;
-        front(kRowKeys * first, seen1, kt - Lds::kKvBuf, ex - Lds::kExchBuf, prod_in, dz);
+        front(kRowKeys * first, seen1, kt - Lds::kKvBuf, ex - Lds::kExchBuf, prod_in, dz, pass_on);
         add_dq(seen1, kt - Lds::kKvBuf, dz);
-        front(kRowKeys * last, seen, kt, ex, prod_in2, dz);
-        asm volatile("s_waitcnt vmcnt(2)\n\tv_mov_b32 %0, %3\n\tv_mov_b32 %1, %4\n\tv_readfirstlane_b32 %2, %5"
+        front(kRowKeys * last, seen, kt, ex, prod_in2, dz, [&] {      // (at head_dim 128 K and V would be waited for as well: 0 to +2 %)
+          asm volatile("s_nop 4\n\tglobal_load_dword %0, %1, %2 sc1" : "=&v"(r_count) : "v"(0), "s"(pred) : "memory");
+        });
+        asm volatile("s_waitcnt vmcnt(0)\n\tv_mov_b32 %0, %3\n\tv_mov_b32 %1, %4\n\tv_readfirstlane_b32 %2, %5"
                      : "=&v"(n_prod), "=&v"(n_prod2), "=s"(count) : "v"(r_prod), "v"(r_prod2), "v"(r_count) : "memory");
       }
-      // The key blocks that are complete are passed on; what the tile above left of the one that is contracted next is asked for.
-      const int tn = late ? t - 1 : t, block = block_of(tn);
-      const bool any = tn >= 0 && (kWide || block < n);
-      if (lane == 0) *flag = seen_count == kChainBroken ? kChainBroken : kWide ? block : block - 1;      // (the one before was this wave's last)
+      // What the tile above left of the block that is contracted next is asked for.
       seen_count = max(seen_count, count);
       if (has_pred && any) request_above(block);
       else c0 = c1 = c2 = c3 = f32x4{0.f, 0.f, 0.f, 0.f};

@@ -161,7 +161,7 @@ int plan(const SbaArgs* a, Layout* out, bool row_tiles = false) {
   // Row tiles: the region that is cleared lies in the schedule, or (two kernels) in the rest.
   auto row_region = [&]() {
     L.off_chain_zero = off;
-    L.off_chain_c = off;      off = align_up(off + L.row_launches(a->num_heads) * 32, 256);      // the queues
+    L.off_chain_c = off;      off = align_up(off + L.row_launches(a->num_heads) * 64, 256);      // the queues, two lists each
     L.off_chain_xcc = off;    off = align_up(off + L.row_launches(a->num_heads) * 32, 256);
     L.off_chain_flags = off;  off = align_up(off + (size_t)a->num_heads * L.max_k_tiles * 32, 256);
     L.chain_zero_bytes = off - L.off_chain_zero;
@@ -663,7 +663,7 @@ hipError_t launch_row_tiles(const sba::BwdParams& whole, const Layout& L, bool f
     if (p.d_rem.ptr) p.d_rem.ptr = (char*)p.d_rem.ptr + h0 * p.d_rem.sh * 2;
     if (p.row_stat) p.row_stat += h0 * p.stat_sh;
     p.carry += h0 * p.carry_head_stride;
-    p.chain_c += 8 * i;
+    p.chain_c += 16 * i;
     p.chain_head_xcc += 8 * i;
     p.chain_flags += h0 * p.chain_tile_cap * 8;
     const hipError_t e = sba::launch_bwd_row(p, f16, (int)L.max_k_tiles, stream);

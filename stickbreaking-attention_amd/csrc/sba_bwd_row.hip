@@ -14,7 +14,7 @@
 // its own; the same wave of the tile below reads flag and partial results with sc1 (served by the L2, never by the vector L1).  All
 // tiles of a (head, sequence) run on one XCD, i.e. on one L2: (head, sequence) belongs to one of 8 queues (row_queue), a workgroup takes
 // tiles from queue blockIdx % 8 (workgroups are dealt to the XCDs in turn), and every workgroup checks its XCC id against the first
-// of its queue: one that is elsewhere leaves.  Progress: tiles are taken in list order, a tile waits only for one that was taken before
+// of its queue: one that is elsewhere leaves.  Progress: the tiles of chains are taken in list order, a tile waits only for one that was taken before
 // it, so every wait ends; the waits are bounded all the same.  A tile whose wait ran out passes on NaN and a count that says so
 // (kChainBroken; data alone would not do, the tile above may still overwrite it), and stores NaN: no wrong number leaves the kernel.
 //
@@ -223,14 +223,43 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
   const bool out = kWide ? wave >= 4 : (wave & 2) != 0;      // which result this wave contracts: dK, else dV
   const int cp = kWide ? wave & 3 : wave & 1;           // ... and which 32 columns of it
   const int per_slot = (H + 7) >> 3;       // heads of a tile slot that a queue may hold
+  // A queue has two lists: the tiles of chains, taken in order, and those that are their sequence's only one (no tile waits for them).  The latter
+  // wait for memory most of their time, so workgroups according to their share of the work begin with them while the others compute, and go over
+  // to the other list when theirs is used up.  If that share is none, one list holds all.  32 heads x 128, one sequence of 16384 tokens and 2048
+  // of up to 64, us per training pass, by workgroups (of 32) that begin with the short ones: none (all of them last) 11000, 4 10980, 6 10650, 8 (their
+  // share) 10370, 10 10760.
+  int chained, all;      // claims that chains have, and all (read again for each tile: the loop is short of scalar registers)
+  auto read_lists = [&] {
+    typedef const __attribute__((address_space(4))) BwdParams Args;
+    Args* args = (Args*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));
+    const int32_t* counts = args->counts;
+    const int n = counts[kCountK], slots = (args->num_heads + 7) >> 3, wgs = gridDim.x >> 3;
+    const int begin_apart = wgs * counts[kCountApart] + 512 >> 10;
+    all = __builtin_amdgcn_readfirstlane(n * slots);
+    chained = begin_apart > 0 ? __builtin_amdgcn_readfirstlane(min(max(counts[kCountChained], 0), n) * slots) : all;
+    return (int)(blockIdx.x >> 3) >= wgs - begin_apart;
+  };
+  bool apart = read_lists() && chained < all;
 
   for (;;) {
-    if (threadIdx.x == 0) *reinterpret_cast<int*>(lds_raw) = atomicAdd(cursor, 1);
+    if (threadIdx.x == 0) {
+      int c = atomicAdd(cursor + (apart ? 8 : 0), 1) + (apart ? chained : 0);
+      if (c >= (apart ? all : chained)) {      // that list is used up
+        c = all;
+        if (apart ? chained > 0 : chained < all) {
+          c = atomicAdd(cursor + (apart ? 0 : 8), 1) + (apart ? 0 : chained);
+          if (c >= (apart ? chained : all)) c = all;
+        }
+      }
+      *reinterpret_cast<int*>(lds_raw) = c;
+    }
     __syncthreads();
     const int claim = __builtin_amdgcn_readfirstlane(*reinterpret_cast<int*>(lds_raw));
     __syncthreads();
+    apart = claim >= chained;
+    if (claim >= all) break;
     const int place = claim / per_slot;
-    if (place >= n_tiles) break;
     Tile tile = p.k_tiles[place];
     const int first_slot = __builtin_amdgcn_readfirstlane(p.k_turns[place].first_slot), rank = __builtin_amdgcn_readfirstlane(p.k_turns[place].rank);
     const int L = __builtin_amdgcn_readfirstlane(tile.seq_len), seq_id = __builtin_amdgcn_readfirstlane(tile.seq_id);
@@ -559,6 +588,7 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
 #pragma unroll
       for (int dt = 0; dt < kDTiles; dt++) store_acc_tile<T>(dq_sink, dqacc[dt], p.logit_scale, w_first, 32 * dt, half, col, DH);
     }
+    read_lists();
     __syncthreads();
   }
 }

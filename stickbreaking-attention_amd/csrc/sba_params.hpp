@@ -40,7 +40,7 @@ enum : int { kLoadScalar = 0, kLoadAligned = 1, kLoadPadded = 2 };
 constexpr int kChainBroken = 0x7fffffff;
 
 // Slots of the scheduler's `counts` array.
-enum : int { kCountQ = 0, kCountK = 1, kCountStatus = 2, kCountCovered = 3 };
+enum : int { kCountQ = 0, kCountK = 1, kCountStatus = 2, kCountCovered = 3, kCountChained = 4, kCountApart = 5 };
 // Values of counts[kCountStatus].
 enum : int { kSchedOk = 0, kSchedBadCu = 1, kSchedCarryOverflow = 2, kSchedChainTimeout = 3 };
 
@@ -57,7 +57,9 @@ struct SchedParams {
   Tile* q_tiles;           // query tiles (kBlockQ rows), heaviest first
   Tile* k_tiles;           // key tiles (key_tile keys), heaviest first
   int32_t* counts;         // [kCountQ] query tiles, [kCountK] key tiles, [kCountStatus], [kCountCovered] = tokens
-                           // covered by sequences (rows at or beyond it belong to no sequence and are zero-filled)
+                           // covered by sequences (rows at or beyond it belong to no sequence and are zero-filled); row tiles:
+                           // [kCountChained] tiles at the head of the list, behind which every tile is its sequence's only one,
+                           // [kCountApart] the share of those in the work, in 1024ths
   int64_t* carry_base;     // per sequence: first carry slot of the sequence (per head)
   int32_t* head_queue;     // backward: per-head cursor into the key-tile list, reset to 0 here
   int32_t num_heads;
@@ -75,6 +77,13 @@ constexpr int kInlineSeqs = 64;
 constexpr int kRowTileRows = 256;      // query rows per tile of the backward on row tiles
 // Key blocks of 32 that the row tiles of a sequence hand over, rounded up to whole tiles (none if it is a single tile).
 __host__ __device__ inline int64_t row_blocks(int64_t len) { return len > kRowTileRows ? (len + kRowTileRows - 1) / kRowTileRows * (kRowTileRows / 32) : 0; }
+// What a sequence's row tiles cost, in key blocks swept: those up to each tile's diagonal, and one per tile for its rows.  (A tile costs 2 to 5 blocks
+// besides those, but one of a short sequence, with few waves at work, less per block: 64 tokens 2.9, 16384 tokens 265 per tile.)
+__host__ __device__ inline uint64_t row_work(int64_t len) {
+  const uint64_t tiles = (uint64_t)(len + kRowTileRows - 1) / kRowTileRows, blocks = (uint64_t)(len + 31) / 32;
+  return tiles * (blocks + 1) - tiles * (tiles - (tiles > 0)) / 2 * (kRowTileRows / 32);
+}
+__host__ __device__ inline int apart_share(uint64_t single, uint64_t chained) { return single ? (int)((double)single / (double)(single + chained) * 1024.) : 0; }
 // Its queue, of 8, for head 0 of the sequence with this rank (the list holds the longest first); head h's is (this + h) % 8.  If the heads do
 // not fill the queues evenly, the fuller ones are others for the next sequence, in an order that goes forth and back (a Gray code).
 __host__ __device__ inline int row_queue(int rank, int heads) { return heads & 7 ? ((rank ^ rank >> 1) * (heads & 7)) & 7 : 0; }
@@ -138,7 +147,7 @@ struct BwdParams {
   float* chain_dq;             // key tiles: [head][row][128] fp32, partial dQ of a row over the key tiles below the reader;
                                // row tiles: [head][key block of 32][32 x 256] fp32, partial dV and dK over the row tiles above
   uint32_t* chain_c;           // key tiles: [head][row] {fp32 C below the reader's tile, tag = index of the reader's tile};
-                               // row tiles: [8], next tile not yet taken, per queue
+                               // row tiles: [2][8], next tile not yet taken, per list and queue
   int32_t* chain_flags;        // [head][tile slot][8]: per wave, row (key) blocks whose partial result is complete
   int32_t* chain_head_xcc;     // [head] (row tiles: [queue]): XCC id + 1 of its first workgroup (0 = none yet); those on other XCDs leave
   int32_t* status;             // the scheduler's status word; the kernel raises it when a wait runs out

@@ -52,11 +52,11 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
   __shared__ int sbins[kBins];      // row tiles: sequences per length class
   __shared__ int scratch[kSchedThreads];
   __shared__ long long carry_run;
-  __shared__ unsigned long long row_run;
+  __shared__ unsigned long long row_run, work[2];      // work: of the sequences of one row tile, and of more
   __shared__ int status;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = kSchedThreads / 64;
   for (int i = threadIdx.x; i < kBins; i += kSchedThreads) { qbins[i] = 0; kbins[i] = 0; sbins[i] = 0; }
-  if (threadIdx.x == 0) { carry_run = 0; row_run = 0; status = kSchedOk; }
+  if (threadIdx.x == 0) { carry_run = 0; row_run = 0; work[0] = work[1] = 0; status = kSchedOk; }
   __syncthreads();
 
   // Pass 1: tiles per length class (class = number of query tiles of the sequence, saturating).  Every entry of
@@ -69,7 +69,10 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
     const int cls = min(nq, kBins - 1);
     if (nq) atomicAdd(&qbins[cls], nq);
     if (nk && p.want_key_tiles) atomicAdd(&kbins[cls], nk);
-    if (nk && p.k_turns) atomicAdd(&sbins[cls], 1);
+    if (nk && p.k_turns) {
+      atomicAdd(&sbins[cls], 1);
+      atomicAdd(&work[nk > 1], (unsigned long long)row_work(len));
+    }
     if (p.row_capacity >= 0 && row_blocks(len) > 0) atomicAdd(&row_run, (unsigned long long)row_blocks(len));
   }
   __syncthreads();
@@ -84,6 +87,10 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
   descending_offsets(qbins, scratch);
   if (p.want_key_tiles) descending_offsets(kbins, scratch);
   if (p.k_turns) descending_offsets(sbins, scratch);
+  if (p.k_turns && threadIdx.x == 0) {      // (behind the classes of more than two query tiles)
+    p.counts[kCountChained] = kbins[kRowTileRows / kBlockQ];
+    p.counts[kCountApart] = apart_share(work[0], work[1]);
+  }
 
   // Carry layout: exclusive prefix sum of carry_slots(M_s) over sequences (block-wide, chunked).
   if (p.want_carry_base) {

@@ -95,7 +95,7 @@ __device__ __forceinline__ void forward_service(const SchedParams& p, int wg) {
     return;
   }
   SeqLanes s{0, p.fixed_len, (p.fixed_len + kBlockQ - 1) / kBlockQ, kSchedOk};
-  int total_q, total_k = 0, first_q = 0, first_k = 0;
+  int total_q, total_k = 0, first_q = 0, first_k = 0, chained = 0, apart = 0;
   int64_t covered = p.total_tokens;
   if (p.cu == nullptr) {
     total_q = s.nq * p.num_seqs;
@@ -108,6 +108,7 @@ __device__ __forceinline__ void forward_service(const SchedParams& p, int wg) {
   if (p.want_key_tiles && ok) {
     const int nk = (s.len + p.key_tile - 1) / p.key_tile;
     if (p.cu == nullptr) total_k = nk * p.num_seqs; else first_k = lane_slot(p, s, nk, &total_k);
+    if (p.cu == nullptr) chained = nk > 1 ? total_k : 0;
     const int turns = p.take_turns;
     Tile t;
     t.seq_start = 0; t.seq_len = s.len;
@@ -130,7 +131,17 @@ __device__ __forceinline__ void forward_service(const SchedParams& p, int wg) {
     } else {
       t.carry_base = 0;
       int sequences, rank = 0;      // of this lane's sequence
-      if (p.k_turns) rank = lane_slot(p, s, nk > 0, &sequences);
+      if (p.k_turns) {
+        rank = lane_slot(p, s, nk > 0, &sequences);
+        const int groups = (__builtin_popcountll(__ballot(nk > 1)) + turns - 1) / turns;      // with a sequence of several tiles
+        uint64_t work[2] = {0, 0};
+        for (int seq = 0; seq < p.num_seqs; seq++) {
+          const int n = __builtin_amdgcn_readlane(nk, seq);
+          if (__builtin_amdgcn_readlane(rank, seq) < groups * turns) chained += n;
+          work[n > 1] += row_work(__builtin_amdgcn_readlane(s.len, seq));
+        }
+        apart = apart_share(work[0], work[1]);
+      }
       for (int seq = 0; seq < p.num_seqs; seq++) {
         const int nq = __builtin_amdgcn_readlane(s.nq, seq), n = __builtin_amdgcn_readlane(nk, seq);
         const int q0 = __builtin_amdgcn_readlane(first_q, seq), k0 = __builtin_amdgcn_readlane(first_k, seq);
@@ -169,6 +180,8 @@ __device__ __forceinline__ void forward_service(const SchedParams& p, int wg) {
     p.counts[kCountK] = total_k;
     p.counts[kCountStatus] = s.status;
     p.counts[kCountCovered] = ok ? (int32_t)covered : 0;
+    p.counts[kCountChained] = chained;
+    p.counts[kCountApart] = apart;
   }
 }
 

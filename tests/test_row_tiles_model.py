@@ -138,6 +138,49 @@ def test_tiles_of_a_queue_stay_on_one_xcd():
         assert taken == list(range(100))
 
 
+def row_work(length):
+    tiles, blocks = cdiv(length, 256), cdiv(length, 32)
+    return tiles * (blocks + 1) - tiles * (tiles - (tiles > 0)) // 2 * 8
+
+
+def test_work_of_a_sequence():
+    for length in range(0, 3000):
+        assert row_work(length) == sum(cdiv(length, 32) - 8 * nth + 1 for nth in range(cdiv(length, 256))), length
+
+
+@pytest.mark.parametrize("wgs", [1, 2, 5, 32])
+def test_two_lists_of_a_queue(wgs):
+    """Each workgroup begins with one list and goes over to the other: every claim below `all` is handed out once, those of the chains in order."""
+    rng = random.Random(wgs)
+    for _ in range(200):
+        chained, single = rng.choice([0, 1, 7, 40]), rng.choice([0, 1, 9, 300])
+        both, begin_apart = chained + single, (wgs * rng.randrange(0, 1025) + 512) >> 10
+        if not begin_apart:
+            chained = both      # one list holds all
+        cursor, out = [0, 0], []
+        apart = [i >= wgs - begin_apart and chained < both for i in range(wgs)]
+        running = set(range(wgs))
+        while running:
+            i = rng.choice(sorted(running))
+            first = apart[i]
+            c = cursor[first] + (chained if first else 0)
+            cursor[first] += 1
+            if c >= (both if first else chained):
+                c = both
+                if chained > 0 if first else chained < both:
+                    c = cursor[not first] + (0 if first else chained)
+                    cursor[not first] += 1
+                    if c >= (chained if first else both):
+                        c = both
+            apart[i] = c >= chained
+            if c >= both:
+                running.discard(i)
+            else:
+                out.append(c)
+        assert sorted(out) == list(range(both))
+        assert [c for c in out if c < chained] == list(range(chained))
+
+
 @pytest.fixture(scope="module")
 def listing(tmp_path_factory):
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"

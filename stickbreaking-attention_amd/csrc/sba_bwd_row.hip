@@ -227,10 +227,8 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
   const int cp = kWide ? wave & 3 : wave & 1;           // ... and which 32 columns of it
   const int per_slot = (H + 7) >> 3;       // heads of a tile slot that a queue may hold
   // A queue has two lists: the tiles of chains, taken in order, and those that are their sequence's only one (no tile waits for them).  The latter
-  // wait for memory most of their time, so workgroups according to their share of the work begin with them while the others compute, and go over
-  // to the other list when theirs is used up.  If that share is none, one list holds all.  32 heads x 128, one sequence of 16384 tokens and 2048
-  // of up to 64, us per training pass, by workgroups (of 32) that begin with the short ones: none (all of them last) 11000, 4 10980, 6 10650, 8 (their
-  // share) 10370, 10 10760.
+  // wait for memory most of their time, so some workgroups (apart_share in sba_params.hpp) begin with them while the others compute, and go over
+  // to the other list when theirs is used up.  If none do, one list holds all.
   int chained, all;      // claims that chains have, and all (read again for each tile: the loop is short of scalar registers)
   auto read_lists = [&] {
     typedef const __attribute__((address_space(4))) BwdParams Args;
@@ -238,7 +236,7 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
     asm volatile("" : "+s"(args));
     const int32_t* counts = args->counts;
     const int n = counts[kCountK], slots = (args->num_heads + 7) >> 3, wgs = gridDim.x >> 3;
-    const int begin_apart = wgs * counts[kCountApart] + 512 >> 10;
+    const int begin_apart = apart_workgroups(wgs, counts[kCountApart]);
     all = __builtin_amdgcn_readfirstlane(n * slots);
     chained = begin_apart > 0 ? __builtin_amdgcn_readfirstlane(min(max(counts[kCountChained], 0), n) * slots) : all;
     return (int)(blockIdx.x >> 3) >= wgs - begin_apart;

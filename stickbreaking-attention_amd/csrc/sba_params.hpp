@@ -59,7 +59,7 @@ struct SchedParams {
   int32_t* counts;         // [kCountQ] query tiles, [kCountK] key tiles, [kCountStatus], [kCountCovered] = tokens
                            // covered by sequences (rows at or beyond it belong to no sequence and are zero-filled); row tiles:
                            // [kCountChained] tiles at the head of the list, behind which every tile is its sequence's only one,
-                           // [kCountApart] the share of those in the work, in 1024ths
+                           // [kCountApart] what says how many workgroups begin with those (apart_share)
   int64_t* carry_base;     // per sequence: first carry slot of the sequence (per head)
   int32_t* head_queue;     // backward: per-head cursor into the key-tile list, reset to 0 here
   int32_t num_heads;
@@ -83,7 +83,32 @@ __host__ __device__ inline uint64_t row_work(int64_t len) {
   const uint64_t tiles = (uint64_t)(len + kRowTileRows - 1) / kRowTileRows, blocks = (uint64_t)(len + 31) / 32;
   return tiles * (blocks + 1) - tiles * (tiles - (tiles > 0)) / 2 * (kRowTileRows / 32);
 }
-__host__ __device__ inline int apart_share(uint64_t single, uint64_t chained) { return single ? (int)((double)single / (double)(single + chained) * 1024.) : 0; }
+// Workgroups of a queue that begin with the sequences of one tile: those tiles' share of the work, to the nearest, where it is at least a fifth and
+// the longest sequence alone is two thirds, all other chains a sixteenth (`share`, in 1024ths, else 0: one list, longest first).  The chain then has
+// most workgroups all the time, and when the short tiles are used up the shortest of its own are left.  Where the chains are less, or
+// several, long sweeps start when all else is done and run on alone; and a share of a few workgroups is too coarse.  Training passes at head_dim 128, us, one
+// list / two by the share:
+//    of 32 workgroups        8 heads                 16                32
+//     8   one of 16384 beside 2048 of up to 64   2670 / 2613   5318 / 5183   10970 / 10481
+//     9   one of 16384 beside 2048 of 64         2822 / 2797
+//    10   one of 14182 beside 1564 of 72         2336 / 2320
+//     9   one of 13000 beside 2000 of 30         1887 / 1858                  7394 /  7345
+//     9   one of 12881 beside  819 of 119        1827 / 1846
+//    12   one of 11000 beside 1500 of 64         1603 / 1577                  6177 /  6152
+//    10   one of  9942 beside  419 of 163        1263 / 1244
+// and where there is one list
+//    32   one of  1024 beside 2048 of 64          949 / 1022   1895 / 2052
+//    31   one of  2048 beside 2048 of 64          951 /  989   1875 /  1955
+//    24   three of 1500 beside 300 of 100         301 /  329    589 /  645    1162 /  1271
+//    10   four of 5000 beside 1000 of 40         1247 / 1268   2445 / 2490    4800 /  4905
+//     4   one of 14267 beside  299 of 112        1768 / 1824
+//     4   one of 11452 beside  143 of 254        1288 / 1316
+//    19   one of  8192 beside 2048 of 64         1408 / 1402
+__host__ __device__ inline int apart_share(uint64_t single, uint64_t chained, uint64_t longest) {
+  const uint64_t all = single + chained;
+  return single && 5 * single >= all && 3 * longest >= 2 * all && 16 * chained <= 16 * longest + all ? (int)((double)single / (double)all * 1024.) : 0;
+}
+__host__ __device__ inline int apart_workgroups(int wgs, int share) { return (wgs * share + 512) >> 10; }
 // Its queue, of 8, for head 0 of the sequence with this rank (the list holds the longest first); head h's is (this + h) % 8.  If the heads do
 // not fill the queues evenly, the fuller ones are others for the next sequence, in an order that goes forth and back (a Gray code).
 __host__ __device__ inline int row_queue(int rank, int heads) { return heads & 7 ? ((rank ^ rank >> 1) * (heads & 7)) & 7 : 0; }

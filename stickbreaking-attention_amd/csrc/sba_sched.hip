@@ -53,10 +53,10 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
   __shared__ int scratch[kSchedThreads];
   __shared__ long long carry_run;
   __shared__ unsigned long long row_run, work[2];      // work: of the sequences of one row tile, and of more
-  __shared__ int status;
+  __shared__ int status, longest;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = kSchedThreads / 64;
   for (int i = threadIdx.x; i < kBins; i += kSchedThreads) { qbins[i] = 0; kbins[i] = 0; sbins[i] = 0; }
-  if (threadIdx.x == 0) { carry_run = 0; row_run = 0; work[0] = work[1] = 0; status = kSchedOk; }
+  if (threadIdx.x == 0) { carry_run = 0; row_run = 0; work[0] = work[1] = 0; longest = 0; status = kSchedOk; }
   __syncthreads();
 
   // Pass 1: tiles per length class (class = number of query tiles of the sequence, saturating).  Every entry of
@@ -72,6 +72,7 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
     if (nk && p.k_turns) {
       atomicAdd(&sbins[cls], 1);
       atomicAdd(&work[nk > 1], (unsigned long long)row_work(len));
+      atomicMax(&longest, len);
     }
     if (p.row_capacity >= 0 && row_blocks(len) > 0) atomicAdd(&row_run, (unsigned long long)row_blocks(len));
   }
@@ -89,7 +90,7 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
   if (p.k_turns) descending_offsets(sbins, scratch);
   if (p.k_turns && threadIdx.x == 0) {      // (behind the classes of more than two query tiles)
     p.counts[kCountChained] = kbins[kRowTileRows / kBlockQ];
-    p.counts[kCountApart] = apart_share(work[0], work[1]);
+    p.counts[kCountApart] = apart_share(work[0], work[1], row_work(longest));
   }
 
   // Carry layout: exclusive prefix sum of carry_slots(M_s) over sequences (block-wide, chunked).

@@ -134,13 +134,15 @@ __device__ __forceinline__ void forward_service(const SchedParams& p, int wg) {
       if (p.k_turns) {
         rank = lane_slot(p, s, nk > 0, &sequences);
         const int groups = (__builtin_popcountll(__ballot(nk > 1)) + turns - 1) / turns;      // with a sequence of several tiles
-        uint64_t work[2] = {0, 0};
+        uint64_t work[2] = {0, 0}, longest = 0;
         for (int seq = 0; seq < p.num_seqs; seq++) {
           const int n = __builtin_amdgcn_readlane(nk, seq);
           if (__builtin_amdgcn_readlane(rank, seq) < groups * turns) chained += n;
-          work[n > 1] += row_work(__builtin_amdgcn_readlane(s.len, seq));
+          const uint64_t of_seq = row_work(__builtin_amdgcn_readlane(s.len, seq));
+          work[n > 1] += of_seq;
+          longest = of_seq > longest ? of_seq : longest;
         }
-        apart = apart_share(work[0], work[1]);
+        apart = apart_share(work[0], work[1], longest);
       }
       for (int seq = 0; seq < p.num_seqs; seq++) {
         const int nq = __builtin_amdgcn_readlane(s.nq, seq), n = __builtin_amdgcn_readlane(nk, seq);

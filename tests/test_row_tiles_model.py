@@ -1,5 +1,7 @@
 """CPU checks of the backward on row tiles (csrc/sba_bwd_row.hip): which recorded products it reads, how the queues of its tiles fall, and
 what its inline assembly has to keep that the compiler does not check."""
+import ctypes
+import heapq
 import os
 import random
 import re
@@ -138,14 +140,69 @@ def test_tiles_of_a_queue_stay_on_one_xcd():
         assert taken == list(range(100))
 
 
-def row_work(length):
-    tiles, blocks = cdiv(length, 256), cdiv(length, 32)
-    return tiles * (blocks + 1) - tiles * (tiles - (tiles > 0)) // 2 * 8
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    """The functions of csrc/sba_params.hpp that say how much work a sequence is and how many workgroups begin with sequences of one tile."""
+    cxx = shutil.which("g++")
+    if not cxx:
+        pytest.skip("no g++")
+    folder = tmp_path_factory.mktemp("rules")
+    (folder / "rules.cpp").write_text("""#include "sba_params.hpp"
+extern "C" uint64_t work(int64_t len) { return sba::row_work(len); }
+extern "C" int apart(int wgs, uint64_t single, uint64_t chained, uint64_t longest) {
+  return sba::apart_workgroups(wgs, sba::apart_share(single, chained, longest));
+}
+""")
+    subprocess.run([cxx, "-std=c++17", "-O1", "-shared", "-fPIC", "-D__host__=", "-D__device__=", "-I", CSRC, str(folder / "rules.cpp"), "-o",
+                    str(folder / "rules.so")], check=True, capture_output=True)
+    lib = ctypes.CDLL(str(folder / "rules.so"))
+    lib.work.restype, lib.work.argtypes = ctypes.c_uint64, [ctypes.c_int64]
+    lib.apart.argtypes = [ctypes.c_int] + 3 * [ctypes.c_uint64]
+    return lib
 
 
-def test_work_of_a_sequence():
+def test_work_of_a_sequence(rules):
     for length in range(0, 3000):
-        assert row_work(length) == sum(cdiv(length, 32) - 8 * nth + 1 for nth in range(cdiv(length, 256))), length
+        assert rules.work(length) == sum(cdiv(length, 32) - 8 * nth + 1 for nth in range(cdiv(length, 256))), length
+
+
+def time_of(wgs, chains, singles, begin_apart):
+    """A queue's time until its last tile is done: `begin_apart` workgroups begin with `singles`, all go over to the other list."""
+    lists = [list(chains) + (list(singles) if not begin_apart else []), [] if not begin_apart else list(singles)]
+    at, free = [0, 0], [(0., i, i >= wgs - begin_apart) for i in range(wgs)]
+    heapq.heapify(free)
+    end = 0.
+    while free:
+        now, i, which = heapq.heappop(free)
+        end = max(end, now)
+        which = which if at[which] < len(lists[which]) else not which
+        if at[which] < len(lists[which]):
+            heapq.heappush(free, (now + lists[which][at[which]], i, which))
+            at[which] += 1
+    return end
+
+
+@pytest.mark.parametrize("chain_cost", [0.9, 1.0, 1.1])
+@pytest.mark.parametrize("wgs", [8, 32])
+def test_sequences_of_one_tile_do_not_hold_up_the_chains(rules, wgs, chain_cost):
+    """The time of a queue with two lists is that of one list, longest first, or up to a seventh more (the tiles of one chain over 20-odd
+    workgroups; what runs better side by side, and at the clock that idle workgroups leave, is not in here), whatever there is beside many short
+    sequences, and also if the tiles of chains take 10 % more or less than the rule believes."""
+    rng = random.Random(wgs)
+    batches = [([1024], 2048, 64), ([2048], 2048, 64), ([600], 1000, 64), ([1500] * 3, 300, 100), ([16384], 2048, 32), ([16384], 2048, 64),
+               ([12000], 150, 250), ([700] * 8, 500, 60), ([5000] * 4, 1000, 40), ([8192], 300, 64), ([4096, 3000], 200, 100)]
+    batches += [([rng.randint(257, rng.choice([1000, 16384])) for _ in range(rng.choice([1, 1, 2, 5]))], rng.randint(1, 2500), rng.randint(1, 256)) for _ in range(400)]
+    two = 0
+    for long, n, short in batches:
+        single, chained = n * rules.work(short), sum(rules.work(x) for x in long)
+        begin_apart = rules.apart(wgs, single, chained, max(rules.work(x) for x in long))
+        assert 0 <= begin_apart <= wgs // 2
+        two += begin_apart > 0
+        chains = [chain_cost * (cdiv(x, 32) - 8 * nth + 1) for x in sorted(long, reverse=True) for nth in range(cdiv(x, 256))]
+        singles = [cdiv(short, 32) + 1] * n
+        one = time_of(wgs, chains, singles, 0)
+        assert time_of(wgs, chains, singles, begin_apart) <= 8 / 7 * one, (long, n, short, begin_apart)
+    assert two >= 10      # (and the rule does choose two lists)
 
 
 @pytest.mark.parametrize("wgs", [1, 2, 5, 32])

@@ -150,13 +150,14 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_split_kernel(FwdParams p) {
   if (carry && wave == 0 && half == 0)
     for (int u = n_sub; u & 3; u++) carry_row(u)[col] = 1.f;
 
-  // This wave's sub-tiles, the last wave's the uppermost: swept on their own, downwards from a product of 1.
-  const int per = (n_sub + kWaves - 1) / kWaves, top = n_sub - (kWaves - 1 - wave) * per, bottom = max(top - per, 0);
+  // This wave's sub-tiles, the last wave's the uppermost: swept on their own, downwards from a product of 1.  The parts are cut by where the rows
+  // lie and not by how many the sequence has (of which one less may see a key of the last sub-tile), so that no row's bits depend on the next.
+  const int q_sub = q0 / 32, per = q_sub / kWaves + 1, end = q_sub + 1 - (kWaves - 1 - wave) * per, top = min(end, n_sub), bottom = max(end - per, 0);
   T* const k_lds = reinterpret_cast<T*>(lds_raw) + wave * (2 * SplitLds<DH>::kSub);
   T* const v_lds = k_lds + SplitLds<DH>::kSub;
   const RowSource<T> ksrc = make_row_source<T, kLoad>(kb, p.k.st, L, D), vsrc = make_row_source<T, kLoad>(vb, p.v.st, L, D);
   TileCopy<T, DH, 32, kLoad, 64> ck, cv;
-  if (top > 0) {
+  if (top > bottom) {
     ck.load(ksrc, (top - 1) * 32);
     if (!kCarryOnly) cv.load(vsrc, (top - 1) * 32);
   }

@@ -50,3 +50,25 @@ def test_a_rows_bits_depend_on_no_other_row(gpu_device, H, D):
     for n, a, b in zip(("o", "rem", "dq"), run(q), run(saturated)):
         assert torch.equal(a[:, others], b[:, others]), n
         assert not torch.equal(a[:, odd], b[:, odd]), n
+
+
+@pytest.mark.parametrize("attend_current", [False, True])
+@pytest.mark.parametrize("D", [50, 64, 128])
+@pytest.mark.parametrize("H", [2, 1000])
+def test_a_rows_bits_do_not_depend_on_the_rows_behind_it(gpu_device, H, D, attend_current):
+    """Sequences that end just behind, just before and well behind a multiple of 32 and 128 rows: the rows they have in common, in the kernels
+    that split the keys over the waves (few heads) and those that do not."""
+    most, outs = 700, {}
+    g = torch.Generator(device=gpu_device).manual_seed(D)
+    q, k, v, do = (torch.randn(H, most, D, generator=g, device=gpu_device).bfloat16() for _ in range(4))
+    q, k = 0.25 * q + 0.8, 0.25 * k - 0.8      # (sticks that last for hundreds of keys)
+    for T in (33, 129, 130, 160, 161, 257, 289, 290, 385, 386, 513, 514, 641, 642, most):
+        x = [t[:, :T].contiguous().requires_grad_() for t in (q, k, v)]
+        cu = torch.tensor([T], dtype=torch.int32, device=gpu_device)
+        o, rem = sb_attn_varlen(*x, cu, T, zero_start=False, attend_current=attend_current)
+        outs[T] = dict(o=o.detach(), rem=rem.detach())
+        if H == 2:
+            outs[T]["dq"] = torch.autograd.grad(o, x[0], do[:, :T])[0]
+    for T, got in outs.items():
+        for n, a in got.items():
+            assert torch.equal(a, outs[most][n][:, :T]), f"{n}, {T} rows"

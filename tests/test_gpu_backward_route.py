@@ -25,6 +25,15 @@ def route(a, workspace):
     return _native.ext().backward_route(ctypes.addressof(a))
 
 
+def runs_on_row_tiles(heads, dim, lengths, fixed=False, lengths_known=False, add_remainder=False):
+    """Whether a call's backward does, for tests that mean to reach it (16-bit data, aligned rows)."""
+    a = args(heads, dim, lengths, exact=lengths_known)
+    a.add_remainder = int(add_remainder)
+    if fixed:
+        a.cu_seqlens, a.total_tokens, a.row_blocks = None, lengths[0], 0
+    return route(a, 1 << 40) == (ROW_TILES, heads)
+
+
 LONG, RAGGED, EQUAL = [65536], [16384] + [31] * 600, [4096] * 16
 
 

@@ -248,27 +248,29 @@ int row_load(const SbaArgs* a, const SbaTensor* const (&tensors)[N]) {
 // Whether a call is too small to fill the chip with tiles of 128 query rows (and key tiles): its kernels then split the keys
 // (rows) of a workgroup's rows (keys) over the waves.  By rows times heads, at which the time of the longest row in an unsplit
 // workgroup (a third of which remains when it is split) meets the throughput of the split kernels, which stage K and V four
-// times as often.  Measured on 256 compute units, split / unsplit us:
+// times as often.  Measured on 256 compute units, split / unsplit us (row tiles or key tiles, which split nothing, run the other backwards):
 //   rows x heads          8 K         16 K        32 K        64 K
-//   head_dim 64   fwd   23.5 / 43.8  24.8 / 44.4  30 / 46    52 / 50     (2048 tokens; 8192: 83 / 162 up to 16 K, 162 / 176 at 64 K)
-//                 dQ    28.8 / 61    29.9 / 62    43 / 63    78 / 69
-//   head_dim 128  fwd   34.7 / 61    39 / 62      60 / 64   112 / 73     (8192: 128 / 230, 131 / 236, 189 / 238, 325 / 262)
-//                 dQ    39 / 79      47 / 80      91 / 84   185 / 94
+//   head_dim 64   fwd   21.0 / 43.3  22.8 / 43.1  30 / 46    53 / 48     (2048 tokens; 8192: 72 / 156, 81 / 157, 88 / 157, 153 / 166)
+//                 dQ    26.4 / 62    28.8 / 61    41 / 63                (87 / 226, 95 / 228, 122 / 229)
+//   head_dim 128  fwd   28.8 / 57    34 / 58      51 / 60    92 / 65     (107 / 212, 120 / 214, 149 / 214, 272 / 231)
+//                 dQ    35.6 / 79    43 / 80                             (125 / 302, 145 / 304, 269 / 304)
 // An unsplit workgroup's longest row costs what it does however many rows there are, so the line rises with the longest sequence; the
 // tiles of long sequences run first, so short ones beside them fill the gaps, and rows count for less the shorter the mean is.
 // Training passes, split / unsplit us, by rows x heads:
-//   head_dim 128   2 x  768   15 K  78 /  85   18 K  86 /  92   22 K 103 /  96      (line at 19 K)
-//                  4 x 1024   16 K  96 / 105   20 K 122 / 119   24 K 132 / 125      (21 K)
-//                  1 x 1740   19 K 149 / 171   24 K 161 / 178   31 K 190 / 185      (27 K)
-//                  2 x 2900   17 K 212 / 263   28 K 297 / 306   34 K 324 / 318      (30 K)
-//    7 of 222 to 1568 (mean 699)   33 K 169 / 171   5 of 568 down (mean 417)   18 K  84 /  77      (29 K; 19 K)
-//   head_dim 64    4 x  768   27 K  76 /  78   36 K  82 /  81   45 K  99 /  95      (32 K)
-//                  8 x 1024   32 K 101 /  98   40 K 118 / 112   48 K 129 / 117      (36 K)
-//                  1 x 2900   34 K 160 / 218   42 K 206 / 236   51 K 224 / 248      (60 K)
-//                 12 x 2900   34 K 223 / 245   68 K 344 / 325                       (60 K)
-//   28 of 1660 down (mean 473)     65 K 160 / 155  51 of 1324 down (mean 320)  48 K 125 / 125      (56 K; 50 K)
-// Over 877 batches of 1 to 146 sequences of up to 8000 tokens (equal, uniform, log-normal, one long among short ones) and
-// head_dims 50 to 128, the rule loses 0.3 % against the faster kind of each batch, 14 % at most.
+//   head_dim 128   2 x  768   16 K  76 /  85   20 K  85 /  90   22 K  93 /  93      (line at 19 K)
+//                  4 x 1024   16 K  89 / 103   20 K 113 / 117   24 K 126 / 122      (21 K)
+//                  1 x 1740   19 K 135 / 168   25 K 163 / 177   34 K 197 / 186      (27 K)
+//                  2 x 2900   17 K 187 / 256   28 K 270 / 301   40 K 340 / 316      (30 K)
+//    7 of 222 to 1568 (mean 699)   33 K 154 / 165   38 K 161 / 168   5 of 568 down (mean 417)   18 K  75 /  78   22 K 84 / 77   (29 K; 19 K)
+//   head_dim 64    4 x  768   33 K  76 /  76   39 K  82 /  80   45 K  89 /  89      (32 K)
+//                  8 x 1024   32 K  93 /  92   40 K 107 / 104   48 K 119 / 109      (36 K)
+//                  1 x 2900   37 K 162 / 213   48 K 204 / 229   65 K 243 / 235      (60 K)
+//                 12 x 2900   34 K 197 / 232   68 K 263 / 256                       (60 K)
+//   head_dim 50    4 x  768   33 K  83 /  85   39 K  92 /  92   45 K 102 / 104      (32 K)
+// The lines lie where the kernels crossed when the waves of a workgroup staged together and synchronised three times per step.  Over 877 batches
+// of 1 to 146 sequences of up to 8000 tokens (equal, uniform, log-normal, one long among short ones) and head_dims 50 to 128, the rule
+// then lost 0.3 % against the faster kind of each batch, 14 % at most.  Since a wave stages for itself they cross up to a third higher above
+// head_dim 64, and long sequences lose by the cap (7 of 222 to 1568, 33 K: 7 %; 4 heads x 8192 x 128: forward 135 / 209, training pass 631 / 747).
 // `heads` is the head count of the caller's call, also where the backward takes them through in groups: the groups then run the
 // kernels, and give the bits, of one pass, and products are rebuilt by the kernel whose forward would have kept them.
 bool few_tiles(const SbaArgs* a, int64_t heads, int load) {
@@ -280,8 +282,9 @@ bool few_tiles(const SbaArgs* a, int64_t heads, int load) {
   if (rows >= 2 * cap) return false;
   return rows * (mean + 3 * longest) < 4 * longest * (line < cap ? line : cap);
 }
-// The same for dK/dV: below, head_dim up to 64 splits the rows over the waves (130 K rows x heads: 542 / 565 us at 8192
-// tokens), wider ones take key tiles of 64 instead of 128 (64 K: 113 / 119 at 2048, 354 / 410 at 8192; 130 K: 672 / 657).
+// The same for dK/dV: below, head_dim up to 64 splits the rows over the waves (64 K rows x heads: 73 / 85 us at 2048 tokens, 232 / 314 at 8192; 100 K:
+// 112 / 98 and 338 / 323; 130 K: 155 / 126 and 440 / 423), wider ones take key tiles of 64 instead of 128 (64 K: 113 / 119 at 2048, 354 / 410 at
+// 8192; 130 K: 672 / 657).
 bool few_key_tiles(const SbaArgs* a, int64_t heads, int load) {
   if (a->dtype == SBA_F32 || load == sba::kLoadScalar) return false;
   return a->total_tokens * (a->cu_seqlens ? 1 : a->num_seqs) * heads < 100 << 10;
@@ -306,7 +309,8 @@ sba::VectorRef vref(const SbaVector& t, bool fixed) { return sba::VectorRef{t.pt
 // end 15 % behind the mean by the keys swept, 7 % when they take turns).  The more take turns, the fewer tiles of a (head, sequence) run at the
 // same time and find in the L2 what the tile above left.  Training passes, us, one after the other / two per queue / four / eight:
 // 12 heads x 4 x 8192 x 128 3356 / 3368 / 3255 / 3260; 16 heads, 16384 tokens in 14 sequences 870 / 867 / 857 / 855; 12 heads x 64, 16384 tokens in 10
-// 432 / 435 / 430 / 433; 32 heads x 8 x 4096 4465 / - / 4483 / 4560.
+// 432 / 435 / 430 / 433; 32 heads x 8 x 4096 4465 / - / 4483 / 4560.  (Where a forward prepares the schedule, of up to 64 sequences or of equal ones.  The
+// scheduler kernel, which lists the others and those of a backward that has to schedule for itself, keeps each sequence's tiles together.)
 int take_turns(int64_t heads) {
   const int64_t n = 32 / heads;
   return (int)(n < 1 ? 1 : n > sba::kMostTurns ? sba::kMostTurns : n);

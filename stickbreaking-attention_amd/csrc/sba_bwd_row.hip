@@ -151,12 +151,17 @@ __device__ __forceinline__ void add_rem_rows(f32x16& acc, const typename Elem<T>
     }
 }
 
-// Until the tile above has passed on more than t key blocks: how many it has.  (What only a wait needs is read from the kernel's arguments
-// here and not kept in scalar registers, which the loop around it is short of.)
-__device__ __forceinline__ int wait_for(const int32_t* pred, int t, int lane) {
-  typedef const __attribute__((address_space(4))) BwdParams Args;
+// The kernel's arguments, read where they are needed and not kept in scalar registers, which the loop is short of.
+typedef const __attribute__((address_space(4))) BwdParams Args;
+__device__ __forceinline__ Args* kernel_args() {
   Args* args = (Args*)__builtin_amdgcn_kernarg_segment_ptr();
   asm volatile("" : "+s"(args));
+  return args;
+}
+
+// Until the tile above has passed on more than t key blocks: how many it has.
+__device__ __forceinline__ int wait_for(const int32_t* pred, int t, int lane) {
+  Args* args = kernel_args();
   const int polls = args->wait_polls;
   int v = 0;
 #pragma unroll 1
@@ -181,7 +186,6 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
   lds_u8* const lds = (lds_u8*)lds_raw;
   const int lds_base = __builtin_amdgcn_readfirstlane((int)(uintptr_t)lds);
 
-  const int n_tiles = p.counts[kCountK];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int half = lane >> 5, col = lane & 31;
   const int ac = p.attend_current, H = p.num_heads;
@@ -229,11 +233,9 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
   // A queue has two lists: the tiles of chains, taken in order, and those that are their sequence's only one (no tile waits for them).  The latter
   // wait for memory most of their time, so some workgroups (apart_share in sba_params.hpp) begin with them while the others compute, and go over
   // to the other list when theirs is used up.  If none do, one list holds all.
-  int chained, all;      // claims that chains have, and all (read again for each tile: the loop is short of scalar registers)
+  int chained, all;      // claims that chains have, and all (read again for each tile)
   auto read_lists = [&] {
-    typedef const __attribute__((address_space(4))) BwdParams Args;
-    Args* args = (Args*)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(args));
+    Args* args = kernel_args();
     const int32_t* counts = args->counts;
     const int n = counts[kCountK], slots = (args->num_heads + 7) >> 3, wgs = gridDim.x >> 3;
     const int begin_apart = apart_workgroups(wgs, counts[kCountApart]);
@@ -548,6 +550,8 @@ __global__ __launch_bounds__(kRowThreads, 2) void bwd_row_kernel(BwdParams p) {
       };
       if constexpr (kWide) {
         front(kRowKeys * t, seen, kt, ex, prod_in, dz, pass_on);
+        // (In flight: count, product, K and V in two parts, the flag.  3 would do and measured the same, 32 heads x 8 x 4096 4279 us either way;
+        // 2 does not count on the flag.)
         asm volatile("s_waitcnt vmcnt(2)\n\tv_mov_b32 %0, %2\n\tv_readfirstlane_b32 %1, %3"
                      : "=&v"(n_prod), "=s"(count) : "v"(r_prod), "v"(r_count) : "memory");
       } else {

@@ -65,7 +65,8 @@ struct SchedParams {
   int32_t num_heads;
   int32_t key_tile;        // keys per key tile (a multiple of 32; what the dK/dV kernel that will run sweeps)
   Turn* k_turns;           // row tiles: beside k_tiles (else NULL)
-  int32_t take_turns;      // row tiles: sequences whose tiles take turns in the list, up to kMostTurns (1: each sequence's follow each other)
+  int32_t take_turns;      // row tiles: sequences whose tiles take turns in the list, up to kMostTurns (1, and in the scheduler kernel:
+                           // each sequence's follow each other)
   uint32_t* zero_fill;     // optional: 16-byte aligned region cleared by the launch (the one-kernel backward's flags
   int64_t zero_bytes;      // and tags start every call at zero), a multiple of 16 bytes
   int32_t service;         // workgroups at the head of a forward launch that schedule and clear (0: a scheduler launch did)

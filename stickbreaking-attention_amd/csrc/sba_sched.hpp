@@ -38,7 +38,7 @@ __device__ __forceinline__ SeqLanes load_lanes(const SchedParams& p) {
 }
 // First slot of this lane's sequence in a list of `n` tiles per sequence: sequences with more query tiles first, then by
 // index.  `total`: length of the list.
-__device__ __forceinline__ int lane_slot(const SchedParams& p, const SeqLanes& s, int n, int* total) {
+__device__ __forceinline__ int lane_slot(const SchedParams& p, const SeqLanes& s, int n, int* total = nullptr) {
   const int lane = threadIdx.x & 63;
   int before = 0, sum = 0;
   for (int j = 0; j < p.num_seqs; j++) {
@@ -46,7 +46,7 @@ __device__ __forceinline__ int lane_slot(const SchedParams& p, const SeqLanes& s
     before += qj > s.nq || (qj == s.nq && j < lane) ? nj : 0;
     sum += nj;
   }
-  *total = sum;
+  if (total) *total = sum;
   return before;
 }
 __device__ __forceinline__ int64_t lane_carry_base(const SeqLanes& s, int seq) {
@@ -130,9 +130,9 @@ __device__ __forceinline__ void forward_service(const SchedParams& p, int wg) {
       for (int i = threadIdx.x; i < p.num_seqs; i += blockDim.x) p.carry_base[i] = i * carry_slots(s.nq);
     } else {
       t.carry_base = 0;
-      int sequences, rank = 0;      // of this lane's sequence
+      int rank = 0;      // of this lane's sequence
       if (p.k_turns) {
-        rank = lane_slot(p, s, nk > 0, &sequences);
+        rank = lane_slot(p, s, nk > 0);
         const int groups = (__builtin_popcountll(__ballot(nk > 1)) + turns - 1) / turns;      // with a sequence of several tiles
         uint64_t work[2] = {0, 0}, longest = 0;
         for (int seq = 0; seq < p.num_seqs; seq++) {

@@ -346,8 +346,8 @@ __global__ __launch_bounds__(kThreads, DH == 128 ? 1 : 2) void bwd_dq_split_kern
   reduce_store<T, DH, kLoad>(reinterpret_cast<float*>(lds_raw), dqacc, p.logit_scale, dqb, p.dq.st, L - q0, D);
 }
 
-// dK/dV, head_dim up to 64: 32 keys per workgroup, K and V stationary in registers, the rows that see them swept by steps of
-// 128, wave w on rows 32 w of a step.
+// dK/dV, head_dim up to 64: 32 keys per workgroup, K and V stationary in registers.  Wave w takes every fourth group of 32 rows from the
+// w-th on, counted from the group of the first row that sees the keys.
 constexpr int kPzStride = 40;      // elements per row of a wave's P and dZ scratch
 template <typename T, int kLoad>
 __global__ __launch_bounds__(kThreads, 2) void bwd_dkv_split_kernel(BwdParams p) {

@@ -29,7 +29,7 @@ sys.path.insert(0, os.path.join(ROOT, "stickbreaking-attention_amd"))
 MFMA_BF16_PEAK = 2.5e15          # MI355X dense bf16 MFMA peak, FLOP/s
 
 # HBM bytes per launch (fetch + write) of each kernel cannot be read from inside this script (hardware counters need
-# rocprofv3): they are measured by the two `rocprofv3 --pmc` runs whose summary is profiles/c3_varlen_hbm_traffic_pmc.txt
+# rocprofv3): they are measured by the two `rocprofv3 --pmc` runs whose summary is profiles/hbm_traffic_pmc.txt
 # and kept, with the commit they were measured at, in the JSON file beside that summary.  `roofline.traffic` reports
 # the figure for the dominant kernel of the workload it was measured on, null otherwise.
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic.json")

@@ -21,15 +21,15 @@
 // What bounds it: per 32 x 32 block and wave 40 MFMAs (1280 cycles), 320 vector-ALU instructions and 48 KB of LDS reads, two waves per
 // SIMD.  The waves of a SIMD (w and w + 4) are kept out of step: one contracts the block of the step before at the start of a
 // step, the other at its end (32 heads x 8 x 4096: 4970 -> 4660 us per training pass).  32 heads x 8 x 4096 x 128, one pass of
-// the backward: 4180 us with key tiles (sba_bwd_chain.hip), 3200 us here; 32768 tokens in 25 sequences of up to 4096, 32 heads: 2650 and
-// 1900.  A step takes 5800 cycles.  Either pipe of a SIMD is busy three quarters of the time (63 % on the 25 sequences), both 6 to 8 %; waves wait 35 % (43 %) of
+// the backward: 4180 us with key tiles (sba_bwd_chain.hip), 3330 us here; 32768 tokens in 25 sequences of up to 4096, 32 heads: 2650 and
+// 2000.  A step takes 5800 cycles.  Either pipe of a SIMD is busy 78 % of the time (69 % on the 25 sequences), both 7 to 9 %; waves wait 35 % (39 %) of
 // theirs.  Without the hand-over it would take 3130 of 3300, without the tile math as well 2590: at 2.1 GHz, the clock that the power limit
 // leaves, and 2.0 for the products alone.  256 rows per tile, because the hand-over costs 8 bytes per pair / (rows / 256).  The next tile of a workgroup
 // costs 27000 cycles (17.8 tiles of 34 steps each on the 25 sequences): 11000 to 17000 for its Q and dO, behind the other workgroups' traffic, 3000
 // for dQ, 2300 for its place in the list.
 //
 // head_dim 64: half the products per pair and the same element-wise work (320 vector-ALU instructions against 20 MFMAs per block and
-// wave); vector ALU busy 45 %, either pipe 61 %, and waves wait 46 % of their time: two waves per SIMD that meet at two barriers per step
+// wave); vector ALU busy 51 %, either pipe 69 %, and waves wait 40 % of their time: two waves per SIMD that meet at two barriers per step
 // bound it.  A key block has four pieces of {dV, dK}, so a step is two blocks and a wave contracts a piece of one of
 // them; LDS holds four blocks, Q stays in registers.  (Steps of one block, contracted by every second wave in turn: the wave whose
 // turn it is arrives last at every barrier: 12 heads, 16384 tokens in 10 sequences of up to 3523, 474 us instead of 434.)  Training passes,

@@ -15,7 +15,7 @@ for p in (ROOT, PKG_PARENT):
 
 
 def pytest_configure(config):
-    config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu on the GPU box)")
+    config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu)")
 
 
 @pytest.fixture(scope="session")

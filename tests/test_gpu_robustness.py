@@ -260,7 +260,7 @@ def test_torch_compile_against_oracle(gpu_device, backend):
         loss, o, rem = compiled(q, k, v, dev[3], dev[4])
         loss.backward()
         torch.cuda.synchronize()
-    except Exception as e:       # code generation needs a working compiler toolchain on the box
+    except Exception as e:       # code generation needs a working compiler toolchain
         if backend == "inductor":
             pytest.skip(f"inductor backend unavailable here: {type(e).__name__}: {str(e)[:200]}")
         raise

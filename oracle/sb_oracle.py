@@ -1,7 +1,7 @@
 """CPU oracle for stick-breaking attention.  TEST INFRASTRUCTURE ONLY.
 
 Nothing that ships may import this module: only ``tests/``, ``__graft_entry__.smoke()`` and
-the ``cpu_baseline`` leg of ``bench.py`` use it, and only as the checker or as the timed CPU
+the ``cpu_baseline`` leg of ``bench.py`` use it, and only as the oracle of tests or as the timed CPU
 baseline -- never as a compute path of the product.
 
 What it restates (citations are into the reference repository):

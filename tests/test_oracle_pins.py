@@ -257,7 +257,7 @@ def test_remainder_term_gradients_match_autograd():
 
 @pytest.mark.parametrize("attend_current", [False, True])
 def test_fixed_stream_matches_brute_force_and_packed_view(attend_current):
-    """`fixed_stream` is the checker of every fixed-length GPU test: its (B, H, L, D) slicing is pinned against the
+    """`fixed_stream` is the oracle of every fixed-length GPU test: its (B, H, L, D) slicing is pinned against the
     scalar product-form loops on a tiny case (forward) with finite differences of those loops (gradients), and on a
     larger case against `varlen_stream` on the same data packed as B sequences, and against autograd through the
     dense restatement.  A transposed batch/head index, a dropped drem or a wrong scale default fails one of them."""
@@ -360,7 +360,7 @@ def test_rounding_floor_of_saturating_logits_sits_at_the_parity_bound():
 
 @pytest.mark.parametrize("attend_current", [False, True])
 def test_rowblocked_stream_matches_unblocked(attend_current):
-    """`stream_rowblocked` (the checker of the 64K-token GPU test) against the unblocked streaming form, which the tests
+    """`stream_rowblocked` (the oracle of the 64K-token GPU test) against the unblocked streaming form, which the tests
     above pin: block sizes that do and do not divide the length, a block larger than the sequence, length 1."""
     torch.manual_seed(31)
     for L, block in ((97, 32), (64, 64), (50, 512), (1, 4), (130, 7)):

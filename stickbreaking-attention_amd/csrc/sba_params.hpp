@@ -72,7 +72,7 @@ struct SchedParams {
   int32_t service;         // workgroups at the head of a forward launch that schedule and clear (0: a scheduler launch did)
 };
 // Most sequences of a packed batch whose tiles the forward's workgroups derive themselves (one lane each).  The derivation
-// takes 12 vector-ALU instructions per sequence and wave, 1.5 us at 64, and replaces a launch of 8 us in front of the forward.
+// takes 5 instructions per sequence and wave behind a scan of the lanes, and replaces a launch of 8 us in front of the forward.
 constexpr int kInlineSeqs = 64;
 
 constexpr int kRowTileRows = 256;      // query rows per tile of the backward on row tiles

@@ -12,47 +12,67 @@ __device__ __forceinline__ bool seq_bounds(const SchedParams& p, int s, int* sta
   return seq_span(p.cu, p.cu_is_int64, p.cu_has_leading_zero, s, p.total_tokens, start, len);
 }
 
+// Sums over the lanes up to and including this one, and the greatest over a wave; exchanges between lanes are DPP moves (no LDS).
+template <int kCtrl, int kRows>
+__device__ __forceinline__ uint64_t dpp_or_0(uint64_t x) {
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)x, kCtrl, kRows, 0xf, false), hi = __builtin_amdgcn_update_dpp(0, (int)(x >> 32), kCtrl, kRows, 0xf, false);
+  return (uint64_t)(uint32_t)lo | (uint64_t)(uint32_t)hi << 32;
+}
+template <int kCtrl, int kRows>
+__device__ __forceinline__ int dpp_or_0(int x) { return __builtin_amdgcn_update_dpp(0, x, kCtrl, kRows, 0xf, false); }
+template <typename V>
+__device__ __forceinline__ V sum_up_to_lane(V x) {
+  x += dpp_or_0<0x111, 0xf>(x);      // row_shr 1, 2, 4, 8: within 16 lanes
+  x += dpp_or_0<0x112, 0xf>(x);
+  x += dpp_or_0<0x114, 0xf>(x);
+  x += dpp_or_0<0x118, 0xf>(x);
+  x += dpp_or_0<0x142, 0xa>(x);      // row_bcast 15 into rows 1 and 3, 31 into rows 2 and 3
+  x += dpp_or_0<0x143, 0xc>(x);
+  return x;
+}
+__device__ __forceinline__ uint64_t read_lane(uint64_t x, int lane) {
+  return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)x, lane) | (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(x >> 32), lane) << 32;
+}
+__device__ __forceinline__ uint64_t wave_sum(uint64_t x) { return read_lane(sum_up_to_lane(x), 63); }
+__device__ __forceinline__ uint64_t wave_max(uint64_t x) {
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) {
+    const uint64_t y = __shfl_xor((unsigned long long)x, d);
+    x = y > x ? y : x;
+  }
+  return x;
+}
+
 // A batch of at most kInlineSeqs sequences (or of equal ones) held by one wave, a sequence per lane.
 struct SeqLanes {
   int start, len, nq;      // this lane's sequence, and its query tiles (0 beyond the last sequence)
   int status;              // kSchedOk, or why nothing is scheduled (uniform)
+  int64_t carry_base;      // of this lane's sequence: the carry slots of those in front of it
 };
 __device__ __forceinline__ SeqLanes load_lanes(const SchedParams& p) {
-  SeqLanes s{0, 0, 0, kSchedOk};
+  SeqLanes s{0, 0, 0, kSchedOk, 0};
   const int lane = threadIdx.x & 63;
   bool ok = true;
   if (lane < p.num_seqs) ok = seq_bounds(p, lane, &s.start, &s.len);
   s.nq = (s.len + kBlockQ - 1) / kBlockQ;
   if (__any(!ok)) s.status = kSchedBadCu;
-  if (s.status == kSchedOk && p.want_carry_base) {
-    int64_t slots = 0;
-    for (int j = 0; j < p.num_seqs; j++) slots += carry_slots(__builtin_amdgcn_readlane(s.nq, j));
-    if (slots > p.carry_capacity) s.status = kSchedCarryOverflow;
-  }
-  if (s.status == kSchedOk && p.row_capacity >= 0) {
-    int64_t blocks = 0;
-    for (int j = 0; j < p.num_seqs; j++) blocks += row_blocks(__builtin_amdgcn_readlane(s.len, j));
-    if (blocks > p.row_capacity) s.status = kSchedCarryOverflow;
-  }
+  const uint64_t slots = carry_slots(s.nq), upto = sum_up_to_lane(slots);
+  s.carry_base = (int64_t)(upto - slots);
+  if (s.status == kSchedOk && p.want_carry_base && (int64_t)read_lane(upto, 63) > p.carry_capacity) s.status = kSchedCarryOverflow;
+  if (s.status == kSchedOk && p.row_capacity >= 0 && (int64_t)wave_sum(row_blocks(s.len)) > p.row_capacity) s.status = kSchedCarryOverflow;
   return s;
 }
 // First slot of this lane's sequence in a list of `n` tiles per sequence: sequences with more query tiles first, then by
 // index.  `total`: length of the list.
 __device__ __forceinline__ int lane_slot(const SchedParams& p, const SeqLanes& s, int n, int* total = nullptr) {
-  const int lane = threadIdx.x & 63;
-  int before = 0, sum = 0;
+  const int key = s.nq << 6 | (63 - (threadIdx.x & 63));      // (a sequence has less than 2^25 tiles)
+  int before = 0;
   for (int j = 0; j < p.num_seqs; j++) {
-    const int qj = __builtin_amdgcn_readlane(s.nq, j), nj = __builtin_amdgcn_readlane(n, j);
-    before += qj > s.nq || (qj == s.nq && j < lane) ? nj : 0;
-    sum += nj;
+    const int kj = __builtin_amdgcn_readlane(key, j), nj = __builtin_amdgcn_readlane(n, j);
+    before += kj > key ? nj : 0;
   }
-  if (total) *total = sum;
+  if (total) *total = __builtin_amdgcn_readlane(sum_up_to_lane(n), 63);
   return before;
-}
-__device__ __forceinline__ int64_t lane_carry_base(const SeqLanes& s, int seq) {
-  int64_t base = 0;
-  for (int j = 0; j < seq; j++) base += carry_slots(__builtin_amdgcn_readlane(s.nq, j));
-  return base;
 }
 
 // The query tile in `slot`, derived by every wave for itself.  Returns false when the slot holds none: *covered then says from
@@ -80,8 +100,71 @@ __device__ __forceinline__ bool inline_q_tile(const SchedParams& p, int slot, Ti
   t->seq_len = __builtin_amdgcn_readlane(s.len, seq);
   t->seq_id = seq;
   t->origin = (__builtin_amdgcn_readlane(s.nq, seq) - 1 - (slot - __builtin_amdgcn_readlane(first, seq))) * kBlockQ;
-  t->carry_base = p.want_carry_base ? lane_carry_base(s, seq) : 0;
+  t->carry_base = p.want_carry_base ? (int64_t)read_lane(s.carry_base, seq) : 0;
   return true;
+}
+
+// The tile lists of a batch held by the lanes.  A wave of the workgroup lists every fourth sequence: a lane the tiles of its own one where they are
+// few, the wave together those of a longer one.  (One sequence after the other, by the whole workgroup, took 0.6 us each, which was most of a
+// training forward of up to 64 short sequences: forward kernel, 7 heads x 64, 64 sequences of 32 / 64 / 128 tokens 49 / 39 / 39 us, then, the sums of
+// load_lanes by scans instead of loops as well, 23 / 10 / 13.)
+constexpr int kLaneTiles = 4;      // query tiles of a sequence that a lane lists
+__device__ __forceinline__ void list_lanes(const SchedParams& p, const SeqLanes& s, int first_q, int first_k, int nk, int* chained, int* apart) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6, turns = p.take_turns;
+  if (wave == 0 && lane < p.num_seqs) p.carry_base[lane] = s.carry_base;
+
+  // Row tiles: the group of sequences this lane's one takes turns with: its rank, where the group's first tiles begin, how many tiles they have.
+  int rank = 0, start = 0, tiles[kMostTurns] = {};
+  if (p.k_turns) {
+    rank = lane_slot(p, s, nk > 0);
+    const uint64_t here = __ballot(nk > 0);
+    // (Empty sequences, which are in no group, come behind the others: every lane has a rank of its own.)
+    const int place = nk > 0 ? rank : __builtin_popcountll(here) + __builtin_popcountll(~here & ((1ull << lane) - 1));
+    const int nk_at = __builtin_amdgcn_ds_permute(place * 4, nk), first_at = __builtin_amdgcn_ds_permute(place * 4, first_k);      // by rank
+    const int group = rank / turns * turns;
+    start = __shfl(first_at, group & 63);
+#pragma unroll
+    for (int j = 0; j < kMostTurns; j++) {
+      const int n = __shfl(nk_at, (group + j) & 63);
+      tiles[j] = j < turns && group + j < 64 ? n : 0;
+    }
+    const int in_groups = (__builtin_popcountll(__ballot(nk > 1)) + turns - 1) / turns * turns;      // ranks of groups with a sequence of several tiles
+    const uint64_t work = row_work(s.len);
+    *chained = (int)wave_sum(nk > 0 && rank < in_groups ? nk : 0);
+    *apart = apart_share(wave_sum(nk > 1 ? 0 : work), wave_sum(nk > 1 ? work : 0), wave_max(work));
+  }
+
+  auto list_keys = [&](Tile t, int i, int n, int k0, int mine, int from, const int (&of)[kMostTurns]) {
+    t.origin = i * p.key_tile;
+    int place = k0 + i;
+    if (p.k_turns) {
+      place = from + mine % turns;
+#pragma unroll
+      for (int j = 0; j < kMostTurns; j++) place += max(0, of[j] - (n - i));
+      p.k_turns[place] = Turn{k0, mine};
+    }
+    p.k_tiles[place] = t;
+  };
+  const bool listed_here = lane % waves == wave && s.nq > 0;
+  if (listed_here && s.nq <= kLaneTiles) {
+    Tile t;
+    t.seq_start = s.start; t.seq_len = s.len; t.seq_id = lane; t.carry_base = s.carry_base;
+    for (int i = 0; i < s.nq; i++) { t.origin = (s.nq - 1 - i) * kBlockQ; p.q_tiles[first_q + i] = t; }
+    for (int i = 0; i < nk; i++) list_keys(t, i, nk, first_k, rank, start, tiles);
+  }
+  for (uint64_t left = __ballot(listed_here && s.nq > kLaneTiles); left; left &= left - 1) {
+    const int seq = __builtin_ctzll(left);
+    const int nq = __builtin_amdgcn_readlane(s.nq, seq), n = __builtin_amdgcn_readlane(nk, seq), q0 = __builtin_amdgcn_readlane(first_q, seq),
+              k0 = __builtin_amdgcn_readlane(first_k, seq), mine = __builtin_amdgcn_readlane(rank, seq), from = __builtin_amdgcn_readlane(start, seq);
+    int of[kMostTurns];
+#pragma unroll
+    for (int j = 0; j < kMostTurns; j++) of[j] = __builtin_amdgcn_readlane(tiles[j], seq);
+    Tile t;
+    t.seq_start = __builtin_amdgcn_readlane(s.start, seq); t.seq_len = __builtin_amdgcn_readlane(s.len, seq); t.seq_id = seq;
+    t.carry_base = (int64_t)read_lane(s.carry_base, seq);
+    for (int i = lane; i < nq; i += 64) { t.origin = (nq - 1 - i) * kBlockQ; p.q_tiles[q0 + i] = t; }
+    for (int i = lane; i < n; i += 64) list_keys(t, i, n, k0, mine, from, of);
+  }
 }
 
 // The first `p.service` workgroups of a forward launch: number 0 leaves the status word and, when a backward will follow, that
@@ -94,7 +177,7 @@ __device__ __forceinline__ void forward_service(const SchedParams& p, int wg) {
     for (int64_t i = a + threadIdx.x; i < b; i += blockDim.x) z[i] = u32x4{0u, 0u, 0u, 0u};
     return;
   }
-  SeqLanes s{0, p.fixed_len, (p.fixed_len + kBlockQ - 1) / kBlockQ, kSchedOk};
+  SeqLanes s{0, p.fixed_len, (p.fixed_len + kBlockQ - 1) / kBlockQ, kSchedOk, 0};
   int total_q, total_k = 0, first_q = 0, first_k = 0, chained = 0, apart = 0;
   int64_t covered = p.total_tokens;
   if (p.cu == nullptr) {
@@ -129,50 +212,7 @@ __device__ __forceinline__ void forward_service(const SchedParams& p, int wg) {
       }
       for (int i = threadIdx.x; i < p.num_seqs; i += blockDim.x) p.carry_base[i] = i * carry_slots(s.nq);
     } else {
-      t.carry_base = 0;
-      int rank = 0;      // of this lane's sequence
-      if (p.k_turns) {
-        rank = lane_slot(p, s, nk > 0);
-        const int groups = (__builtin_popcountll(__ballot(nk > 1)) + turns - 1) / turns;      // with a sequence of several tiles
-        uint64_t work[2] = {0, 0}, longest = 0;
-        for (int seq = 0; seq < p.num_seqs; seq++) {
-          const int n = __builtin_amdgcn_readlane(nk, seq);
-          if (__builtin_amdgcn_readlane(rank, seq) < groups * turns) chained += n;
-          const uint64_t of_seq = row_work(__builtin_amdgcn_readlane(s.len, seq));
-          work[n > 1] += of_seq;
-          longest = of_seq > longest ? of_seq : longest;
-        }
-        apart = apart_share(work[0], work[1], longest);
-      }
-      for (int seq = 0; seq < p.num_seqs; seq++) {
-        const int nq = __builtin_amdgcn_readlane(s.nq, seq), n = __builtin_amdgcn_readlane(nk, seq);
-        const int q0 = __builtin_amdgcn_readlane(first_q, seq), k0 = __builtin_amdgcn_readlane(first_k, seq);
-        t.seq_start = __builtin_amdgcn_readlane(s.start, seq); t.seq_len = __builtin_amdgcn_readlane(s.len, seq); t.seq_id = seq;
-        for (int i = threadIdx.x; i < nq; i += blockDim.x) { t.origin = (nq - 1 - i) * kBlockQ; p.q_tiles[q0 + i] = t; }
-        if (p.k_turns) {
-          // The group's sequences, by rank, and where the first one's tiles begin (an empty sequence is in none).
-          const int mine = __builtin_amdgcn_readlane(rank, seq), group = mine / turns * turns;
-          int tiles[kMostTurns], start = k0;
-#pragma unroll
-          for (int j = 0; j < kMostTurns; j++) {
-            const uint64_t at = __ballot(nk > 0 && j < turns && rank == group + j);
-            tiles[j] = at ? __builtin_amdgcn_readlane(nk, __builtin_ctzll(at)) : 0;
-            if (j == 0 && at) start = __builtin_amdgcn_readlane(first_k, __builtin_ctzll(at));
-          }
-          for (int i = threadIdx.x; i < n; i += blockDim.x) {
-            int place = start + (mine - group);
-#pragma unroll
-            for (int j = 0; j < kMostTurns; j++) place += max(0, tiles[j] - (n - i));
-            t.origin = i * p.key_tile;
-            p.k_tiles[place] = t;
-            p.k_turns[place] = Turn{k0, mine};
-          }
-        } else {
-          for (int i = threadIdx.x; i < n; i += blockDim.x) { t.origin = i * p.key_tile; p.k_tiles[k0 + i] = t; }
-        }
-        if (threadIdx.x == 0) p.carry_base[seq] = t.carry_base;
-        t.carry_base += carry_slots(nq);
-      }
+      list_lanes(p, s, first_q, first_k, nk, &chained, &apart);
     }
   }
   if (p.want_key_tiles)

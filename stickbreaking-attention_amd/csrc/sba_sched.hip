@@ -17,28 +17,30 @@ namespace sba {
 constexpr int kBins = 4096;          // sequence length classes (query tiles per sequence, saturating)
 constexpr int kSchedThreads = 1024;
 
-// Exclusive prefix sum over bins taken from the heaviest bin downwards; bins[] becomes the start offsets.
-__device__ void descending_offsets(int* bins, int* scratch) {
-  constexpr int kPer = kBins / kSchedThreads;
-  const int t = threadIdx.x;
-  // thread t owns bins (kBins-1 - kPer*t) down to (kBins-1 - kPer*t - kPer + 1)
-  int local[kPer], sum = 0;
+constexpr int kSchedWaves = kSchedThreads / 64;
+
+// What the waves in front of this one, and all of them, hold of `n` values per thread; upto[i]: in, a value, out, its sum over the wave's lanes up
+// to this one.  `parts` must not be in use; one barrier.
+template <int kN, typename V>
+__device__ __forceinline__ void block_sums(V (&upto)[kN], V (&before)[kN], V (&all)[kN], V (*parts)[kSchedWaves]) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 #pragma unroll
-  for (int i = 0; i < kPer; i++) { local[i] = bins[kBins - 1 - (kPer * t + i)]; sum += local[i]; }
-  scratch[t] = sum;
-  __syncthreads();
-  for (int d = 1; d < kSchedThreads; d <<= 1) {
-    const int v = (t >= d) ? scratch[t - d] : 0;
-    __syncthreads();
-    scratch[t] += v;
-    __syncthreads();
+  for (int i = 0; i < kN; i++) {
+    upto[i] = sum_up_to_lane(upto[i]);
+    if (lane == 63) parts[i][wave] = upto[i];
   }
-  int base = scratch[t] - sum;
-#pragma unroll
-  for (int i = 0; i < kPer; i++) { bins[kBins - 1 - (kPer * t + i)] = base; base += local[i]; }
   __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kN; i++) {
+    const V of_waves = sum_up_to_lane(lane < kSchedWaves ? parts[i][lane] : (V)0);
+    before[i] = wave > 0 ? read_lane(of_waves, wave - 1) : (V)0;
+    all[i] = read_lane(of_waves, kSchedWaves - 1);
+  }
 }
 
+// What bounds it is the length of its chain of steps (one workgroup): sums are formed by scans over the lanes and one exchange between the waves, and
+// what all lanes of a wave add to one counter the wave adds up first.  (With sums over LDS, ten barriers each, and a counter for every
+// lane, us: 2049 sequences 20, now 11; 600 12 and 7; 100 10 and 6.)
 __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
   if (blockIdx.x > 0) {      // helper workgroups: clear the region the launch was asked to clear
     const int64_t n16 = p.zero_bytes / 16, per = (n16 + gridDim.x - 2) / (gridDim.x - 1);
@@ -47,82 +49,92 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
     for (int64_t i = a + threadIdx.x; i < b; i += kSchedThreads) z[i] = u32x4{0u, 0u, 0u, 0u};
     return;
   }
-  __shared__ int qbins[kBins];
-  __shared__ int kbins[kBins];
-  __shared__ int sbins[kBins];      // row tiles: sequences per length class
-  __shared__ int scratch[kSchedThreads];
-  __shared__ long long carry_run;
+  __shared__ int bins[3][kBins];      // query tiles, key tiles and (row tiles) sequences of a length class, then where each class begins
+  int (&qbins)[kBins] = bins[0], (&kbins)[kBins] = bins[1], (&sbins)[kBins] = bins[2];
+  __shared__ uint64_t parts[2][1][kSchedWaves];
+  __shared__ int bin_parts[3][kSchedWaves];
   __shared__ unsigned long long row_run, work[2];      // work: of the sequences of one row tile, and of more
   __shared__ int status, longest;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = kSchedThreads / 64;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = kSchedWaves;
   for (int i = threadIdx.x; i < kBins; i += kSchedThreads) { qbins[i] = 0; kbins[i] = 0; sbins[i] = 0; }
-  if (threadIdx.x == 0) { carry_run = 0; row_run = 0; work[0] = work[1] = 0; longest = 0; status = kSchedOk; }
+  if (threadIdx.x == 0) { row_run = 0; work[0] = work[1] = 0; longest = 0; status = kSchedOk; }
   __syncthreads();
 
-  // Pass 1: tiles per length class (class = number of query tiles of the sequence, saturating).  Every entry of
-  // cu_seqlens is checked here; the checks are local (each end against its predecessor and the token count), and
-  // together they bound the tile counts and carry slots by what the caller's buffers were sized for.
-  for (int s = threadIdx.x; s < p.num_seqs; s += kSchedThreads) {
-    int start, len;
-    if (!seq_bounds(p, s, &start, &len)) status = kSchedBadCu;
+  // Pass 1: tiles per length class (class = number of query tiles of the sequence, saturating), and the layout of the carries: a sum over the
+  // sequences in front.  Every entry of cu_seqlens is checked here; the checks are local (each end against its predecessor and the token
+  // count), and together they bound the tile counts and carry slots by what the caller's buffers were sized for.  What all lanes of a wave
+  // add to is added up by the wave first.
+  uint64_t carry_run = 0;
+  for (int s0 = 0; s0 < p.num_seqs; s0 += kSchedThreads) {
+    const int s = s0 + threadIdx.x;
+    int start = 0, len = 0;
+    if (s < p.num_seqs && !seq_bounds(p, s, &start, &len)) status = kSchedBadCu;
     const int nq = (len + kBlockQ - 1) / kBlockQ, nk = (len + p.key_tile - 1) / p.key_tile;
     const int cls = min(nq, kBins - 1);
-    if (nq) atomicAdd(&qbins[cls], nq);
-    if (nk && p.want_key_tiles) atomicAdd(&kbins[cls], nk);
-    if (nk && p.k_turns) {
-      atomicAdd(&sbins[cls], 1);
-      atomicAdd(&work[nk > 1], (unsigned long long)row_work(len));
+    // (Most sequences of a large batch are of one class.)
+    const int first_cls = __builtin_amdgcn_readfirstlane(cls);
+    if (first_cls > 0 && __all(cls == first_cls)) {
+      const int of_q = read_lane(sum_up_to_lane(nq), 63), of_k = read_lane(sum_up_to_lane(nk), 63);
+      if (lane == 0) {
+        atomicAdd(&qbins[cls], of_q);
+        if (p.want_key_tiles) atomicAdd(&kbins[cls], of_k);
+        if (p.k_turns) atomicAdd(&sbins[cls], 64);
+      }
+    } else if (nq) {
+      atomicAdd(&qbins[cls], nq);
+      if (p.want_key_tiles) atomicAdd(&kbins[cls], nk);
+      if (p.k_turns) atomicAdd(&sbins[cls], 1);
+    }
+    if (p.k_turns) {
+      const uint64_t mine = row_work(len), of_wave[2] = {wave_sum(nk > 1 ? 0 : mine), wave_sum(nk > 1 ? mine : 0)};
+      if (lane < 2 && of_wave[lane]) atomicAdd(&work[lane], (unsigned long long)of_wave[lane]);
       atomicMax(&longest, len);
     }
-    if (p.row_capacity >= 0 && row_blocks(len) > 0) atomicAdd(&row_run, (unsigned long long)row_blocks(len));
+    if (p.row_capacity >= 0) {
+      const uint64_t blocks = wave_sum(row_blocks(len));
+      if (lane == 0 && blocks) atomicAdd(&row_run, (unsigned long long)blocks);
+    }
+    if (p.want_carry_base) {
+      const uint64_t mine = carry_slots(nq);
+      uint64_t upto[1] = {mine}, before[1], all[1];
+      block_sums(upto, before, all, parts[(s0 / kSchedThreads) & 1]);
+      if (s < p.num_seqs) p.carry_base[s] = (int64_t)(carry_run + before[0] + upto[0] - mine);
+      carry_run += all[0];
+    }
   }
   __syncthreads();
-  if (threadIdx.x == 0 && status == kSchedOk && p.row_capacity >= 0 && row_run > (unsigned long long)p.row_capacity) status = kSchedCarryOverflow;
-  __syncthreads();
-  if (status != kSchedOk) {      // uniform: nothing is scheduled, every output row is zero-filled as uncovered
-    if (threadIdx.x == 0) { p.counts[kCountQ] = 0; p.counts[kCountK] = 0; p.counts[kCountStatus] = status; p.counts[kCountCovered] = 0; }
+  int verdict = status;
+  if (verdict == kSchedOk && p.row_capacity >= 0 && row_run > (unsigned long long)p.row_capacity) verdict = kSchedCarryOverflow;
+  if (verdict == kSchedOk && p.want_carry_base && (int64_t)carry_run > p.carry_capacity) verdict = kSchedCarryOverflow;      // the caller's max_seqlen (or slot count) was too small
+  if (verdict != kSchedOk) {      // uniform: nothing is scheduled, every output row is zero-filled as uncovered
+    if (threadIdx.x == 0) { p.counts[kCountQ] = 0; p.counts[kCountK] = 0; p.counts[kCountStatus] = verdict; p.counts[kCountCovered] = 0; }
     if (p.want_key_tiles)
       for (int h = threadIdx.x; h < p.num_heads; h += kSchedThreads) p.head_queue[h] = 0;
     return;
   }
-  descending_offsets(qbins, scratch);
-  if (p.want_key_tiles) descending_offsets(kbins, scratch);
-  if (p.k_turns) descending_offsets(sbins, scratch);
+  // Where each class begins: sums over the classes from the heaviest down.  Thread t owns bins kBins - 1 - kPer t down to kBins - kPer (t + 1).
+  {
+    constexpr int kPer = kBins / kSchedThreads;
+    int local[3][kPer], upto[3], before[3], all[3];
+#pragma unroll
+    for (int b = 0; b < 3; b++) {
+      upto[b] = 0;
+#pragma unroll
+      for (int i = 0; i < kPer; i++) { local[b][i] = bins[b][kBins - 1 - (kPer * threadIdx.x + i)]; upto[b] += local[b][i]; }
+    }
+    const int mine[3] = {upto[0], upto[1], upto[2]};
+    block_sums(upto, before, all, bin_parts);
+#pragma unroll
+    for (int b = 0; b < 3; b++) {
+      int base = before[b] + upto[b] - mine[b];
+#pragma unroll
+      for (int i = 0; i < kPer; i++) { bins[b][kBins - 1 - (kPer * threadIdx.x + i)] = base; base += local[b][i]; }
+    }
+  }
+  __syncthreads();
   if (p.k_turns && threadIdx.x == 0) {      // (behind the classes of more than two query tiles)
     p.counts[kCountChained] = kbins[kRowTileRows / kBlockQ];
     p.counts[kCountApart] = apart_share(work[0], work[1], row_work(longest));
-  }
-
-  // Carry layout: exclusive prefix sum of carry_slots(M_s) over sequences (block-wide, chunked).
-  if (p.want_carry_base) {
-    for (int s0 = 0; s0 < p.num_seqs; s0 += kSchedThreads) {
-      const int s = s0 + threadIdx.x;
-      int start = 0, len = 0;
-      if (s < p.num_seqs) seq_bounds(p, s, &start, &len);
-      const long long mine = carry_slots((len + kBlockQ - 1) / kBlockQ);
-      // inclusive scan of `mine` through 64-bit shuffles would need two passes; sequences per chunk are
-      // few enough for a shared-memory Hillis-Steele scan on the low/high words kept as long long.
-      __shared__ long long sc[kSchedThreads];
-      sc[threadIdx.x] = mine;
-      __syncthreads();
-      for (int d = 1; d < kSchedThreads; d <<= 1) {
-        const long long v = (threadIdx.x >= d) ? sc[threadIdx.x - d] : 0;
-        __syncthreads();
-        sc[threadIdx.x] += v;
-        __syncthreads();
-      }
-      const long long base = carry_run;
-      if (s < p.num_seqs) p.carry_base[s] = base + sc[threadIdx.x] - mine;
-      __syncthreads();
-      if (threadIdx.x == kSchedThreads - 1) carry_run = base + sc[threadIdx.x];
-      __syncthreads();
-    }
-    if (carry_run > p.carry_capacity) {      // uniform: the caller's max_seqlen (or slot count) was too small
-      if (threadIdx.x == 0) { p.counts[kCountQ] = 0; p.counts[kCountK] = 0; p.counts[kCountStatus] = kSchedCarryOverflow; p.counts[kCountCovered] = 0; }
-      if (p.want_key_tiles)
-        for (int h = threadIdx.x; h < p.num_heads; h += kSchedThreads) p.head_queue[h] = 0;
-      return;
-    }
   }
   __syncthreads();
 
@@ -142,9 +154,22 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
     }
     const int nq = (len + kBlockQ - 1) / kBlockQ, nk = p.want_key_tiles ? (len + p.key_tile - 1) / p.key_tile : 0;
     const int cls = min(nq, kBins - 1);
-    if (nq) qbase = atomicAdd(&qbins[cls], nq);
-    if (nk) kbase = atomicAdd(&kbins[cls], nk);
-    if (nk && p.k_turns) rank = atomicAdd(&sbins[cls], 1);
+    const int first_cls = __builtin_amdgcn_readfirstlane(cls);
+    if (first_cls > 0 && __all(cls == first_cls)) {      // a place for all of them
+      const int upto_q = sum_up_to_lane(nq), upto_k = sum_up_to_lane(nk);
+      if (lane == 0) {
+        qbase = atomicAdd(&qbins[cls], read_lane(upto_q, 63));
+        if (p.want_key_tiles) kbase = atomicAdd(&kbins[cls], read_lane(upto_k, 63));
+        if (p.k_turns) rank = atomicAdd(&sbins[cls], 64);
+      }
+      qbase = __builtin_amdgcn_readfirstlane(qbase) + upto_q - nq;
+      kbase = __builtin_amdgcn_readfirstlane(kbase) + upto_k - nk;
+      rank = __builtin_amdgcn_readfirstlane(rank) + lane;
+    } else {
+      if (nq) qbase = atomicAdd(&qbins[cls], nq);
+      if (nk) kbase = atomicAdd(&kbins[cls], nk);
+      if (nk && p.k_turns) rank = atomicAdd(&sbins[cls], 1);
+    }
     Tile d;
     d.seq_start = start; d.seq_len = len; d.seq_id = s; d.carry_base = cbase;
     if (nq <= kOwnTiles) {

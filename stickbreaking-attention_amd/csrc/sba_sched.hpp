@@ -30,8 +30,10 @@ __device__ __forceinline__ V sum_up_to_lane(V x) {
   x += dpp_or_0<0x143, 0xc>(x);
   return x;
 }
-__device__ __forceinline__ uint64_t read_lane(uint64_t x, int lane) {
-  return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)x, lane) | (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(x >> 32), lane) << 32;
+template <typename V>
+__device__ __forceinline__ V read_lane(V x, int lane) {
+  if constexpr (sizeof(V) == 4) return __builtin_amdgcn_readlane(x, lane);
+  else return (V)((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)x, lane) | (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(x >> 32), lane) << 32);
 }
 __device__ __forceinline__ uint64_t wave_sum(uint64_t x) { return read_lane(sum_up_to_lane(x), 63); }
 __device__ __forceinline__ uint64_t wave_max(uint64_t x) {
@@ -100,7 +102,7 @@ __device__ __forceinline__ bool inline_q_tile(const SchedParams& p, int slot, Ti
   t->seq_len = __builtin_amdgcn_readlane(s.len, seq);
   t->seq_id = seq;
   t->origin = (__builtin_amdgcn_readlane(s.nq, seq) - 1 - (slot - __builtin_amdgcn_readlane(first, seq))) * kBlockQ;
-  t->carry_base = p.want_carry_base ? (int64_t)read_lane(s.carry_base, seq) : 0;
+  t->carry_base = p.want_carry_base ? read_lane(s.carry_base, seq) : 0;
   return true;
 }
 
@@ -161,7 +163,7 @@ __device__ __forceinline__ void list_lanes(const SchedParams& p, const SeqLanes&
     for (int j = 0; j < kMostTurns; j++) of[j] = __builtin_amdgcn_readlane(tiles[j], seq);
     Tile t;
     t.seq_start = __builtin_amdgcn_readlane(s.start, seq); t.seq_len = __builtin_amdgcn_readlane(s.len, seq); t.seq_id = seq;
-    t.carry_base = (int64_t)read_lane(s.carry_base, seq);
+    t.carry_base = read_lane(s.carry_base, seq);
     for (int i = lane; i < nq; i += 64) { t.origin = (nq - 1 - i) * kBlockQ; p.q_tiles[q0 + i] = t; }
     for (int i = lane; i < n; i += 64) list_keys(t, i, n, k0, mine, from, of);
   }

@@ -80,7 +80,7 @@ __global__ __launch_bounds__(kThreads, KT == 32 ? 2 : 1) void bwd_dq_kernel(BwdP
   const int last_key = last_row - 1 + ac;
   const int n_kt = last_key < 0 ? 0 : last_key / KT + 1;
   const int w_first = q0 + wave * 32, w_last = w_first + 31;
-  const int64_t n_qt = (L + kBlockQ - 1) / kBlockQ;
+  const int n_qt = (L + kBlockQ - 1) / kBlockQ;
   const int64_t slot0 = (int64_t)head * p.carry_head_stride + tile.carry_base;
   const float* carry = p.carry + slot0;
   float* prefix_out = p.prefix + slot0;
@@ -91,11 +91,11 @@ __global__ __launch_bounds__(kThreads, KT == 32 ? 2 : 1) void bwd_dq_kernel(BwdP
 #pragma unroll
     for (int r = 0; r < 16; r++) dqacc[dt][r] = 0.f;
 
-  // Slots of sub-tile u in either plane: a uniform offset, then this lane's row within the tile.
-  auto slot_row = [&](int u) { return carry_offset(u, n_qt) + (q0 - kBlockQ * (u >> 2)); };
+  // Slots of a sub-tile in either plane: a uniform offset, of the lower sub-tile of the tile, then this lane's row within the tile.
+  int64_t slot_row = q0;
   const uint32_t lrow = wave * 32 + col;
   // The forward's product above the next key tile (above its upper sub-tile), fetched one tile ahead.
-  auto product_above = [&](int t) { return (carry + slot_row(NT == 2 ? 2 * t + 1 : t))[lrow]; };
+  auto product_above = [&](int u_lo) { return (carry + slot_row + (NT == 2 ? carry_step(u_lo, n_qt) : 0))[lrow]; };
   float n_prod = 1.f;
   const RowSource<T> ksrc = make_row_source<T, kLoad>(kb, p.k.st, L, D), vsrc = make_row_source<T, kLoad>(vb, p.v.st, L, D);
   TileCopy<T, DH, KT, kLoad> ck, cv;
@@ -111,17 +111,20 @@ __global__ __launch_bounds__(kThreads, KT == 32 ? 2 : 1) void bwd_dq_kernel(BwdP
     cv.store(v_lds);
     __syncthreads();
     const float prod_in = n_prod;
+    // For the key-stationary kernel: C just below each 32-key sub-tile, for every row of the tile.
+    const int u_lo = NT * jt;
+    float* const row_lo = prefix_out + slot_row;
+    float* const row_hi = row_lo + carry_step(u_lo, n_qt);
+    slot_row += carry_step(u_lo, n_qt) + (NT == 2 ? carry_step(u_lo + 1, n_qt) : 0);
     if (jt + 1 < n_kt) {
       const int jn = j0 + KT;
       ck.load(ksrc, jn);
       cv.load(vsrc, jn);
-      n_prod = product_above(jt + 1);
+      n_prod = product_above(NT * jt + NT);
     }
-    // For the key-stationary kernel: C just below each 32-key sub-tile, for every row of the tile.
-    const int u_lo = NT == 2 ? 2 * jt : jt;
-    if (half == 0) (prefix_out + slot_row(u_lo))[lrow] = prefix;
+    if (half == 0) row_lo[lrow] = prefix;
     if (j0 > w_last - 1 + ac) {
-      if (NT == 2 && half == 0) (prefix_out + slot_row(u_lo + 1))[lrow] = prefix;
+      if (NT == 2 && half == 0) row_hi[lrow] = prefix;
       continue;
     }
     const bool diagonal = (j0 + KT - 1) > (w_first - 1 + ac) || w_last >= L;
@@ -175,7 +178,7 @@ __global__ __launch_bounds__(kThreads, KT == 32 ? 2 : 1) void bwd_dq_kernel(BwdP
       bwd_tile_math<T, NT, false>(s, dp, p.scale_log2, diagonal, lim, half, drem, prod_in, prefix, pk, dzk, prod_lower,
                            prefix_upper, prefix);
     }
-    if (NT == 2 && half == 0) (prefix_out + slot_row(u_lo + 1))[lrow] = prefix_upper;
+    if (NT == 2 && half == 0) row_hi[lrow] = prefix_upper;
 
     // dQ += dZ K: A = dZ from registers, B = K gathered down the keys.
 #pragma unroll

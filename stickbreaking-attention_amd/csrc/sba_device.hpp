@@ -203,6 +203,15 @@ __device__ __forceinline__ void load_operand(typename Elem<T>::vec8 (&x)[kSteps]
   }
 }
 
+// An operand (or a number) that was requested in front of a loop, waited for here.  Left to its first use, the wait stands inside the loop, where it
+// is one for the loop's own requests as well, issued just before, in every round.
+template <typename V, int kSteps>
+__device__ __forceinline__ void settle(V (&x)[kSteps]) {
+#pragma unroll
+  for (int kk = 0; kk < kSteps; kk++) asm volatile("" : "+v"(x[kk]));
+}
+__device__ __forceinline__ void settle(float& x) { asm volatile("" : "+v"(x)); }
+
 // Cooperative global -> register -> LDS copy of a [kRows x DH] tile of 16-bit elements, 16 bytes per access.
 // Rows beyond the source and columns at or beyond head_dim are zero-filled.
 template <typename T, int DH, int kRows, int kLoad, int kNumThreads = kThreads>
@@ -279,22 +288,28 @@ struct Weights {
       const float x = s[R >> 4][R & 15] * scale_log2;
       t[R] = fast_exp2(!kDiagonal || R < lim ? x : -INFINITY);
     }
-    float most = 0.f;      // (a sum, so that a NaN of inf * 0 shows)
+    float of_group[N / kGroup];
 #pragma unroll
     for (int g = 0; g < N / kGroup; g++) {
       float prod_g = 1.f + t[kGroup * g];
 #pragma unroll
       for (int i = 1; i < kGroup; i++) prod_g = fmaf(prod_g, t[kGroup * g + i], prod_g);
-      below[g] = prod_g;
-      most += prod_g;
+      of_group[g] = prod_g;
     }
-    mine = most < 0x1p100f;
-    tame = !__any(!mine);
     run = 1.f;
 #pragma unroll
     for (int g = N / kGroup - 1; g >= 0; --g) {
-      run *= fast_rcp(below[g]);
+      run *= fast_rcp(of_group[g]);
       below[g] = run;
+    }
+    // Where all keys together take less than 98 octaves no group takes 100: one comparison answers for most waves.
+    mine = tame = true;
+    if (__any(!(run > 0x1p-98f))) {
+      float most = 0.f;      // (a sum, so that a NaN of inf * 0 shows)
+#pragma unroll
+      for (int g = 0; g < N / kGroup; g++) most += of_group[g];
+      mine = most < 0x1p100f;
+      tame = !__any(!mine);
     }
     if (!tame && !mine) {
       run = 1.f;

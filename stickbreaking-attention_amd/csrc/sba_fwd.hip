@@ -142,7 +142,7 @@ __global__ __launch_bounds__(kThreads, kMinWaves) void fwd_kernel(FwdParams p) {
 #pragma unroll
     for (int r = 0; r < 16; r++) oacc[dt][r] = 0.f;
   float prod = 1.f;    // prod over the keys already swept of (1 - sigma): both half-waves hold the same value
-  const int64_t n_qt = (L + kBlockQ - 1) / kBlockQ;
+  const int n_qt = (L + kBlockQ - 1) / kBlockQ;
   float* carry = p.carry ? p.carry + (int64_t)head * p.carry_head_stride + tile.carry_base : nullptr;
 
   const RowSource<T> ksrc = make_row_source<T, kLoad>(kb, p.k.st, L, D), vsrc = make_row_source<T, kLoad>(vb, p.v.st, L, D);
@@ -158,6 +158,7 @@ __global__ __launch_bounds__(kThreads, kMinWaves) void fwd_kernel(FwdParams p) {
   const uint32_t lrow = wave * 32 + col;
   auto carry_row = [&](int u) { return carry + carry_offset(u, n_qt) + (q0 - kBlockQ * (u >> 2)); };
   if (NT == 1 && carry && half == 0 && (n_kt & 1)) carry_row(n_kt)[lrow] = 1.f;
+  float* row_hi = carry_row(NT * n_kt - 1);                      // of the sub-tile at the upper edge of the tile
   for (int jt = n_kt - 1; jt >= 0; --jt) {
     const int j0 = jt * KT;
     __syncthreads();
@@ -171,10 +172,12 @@ __global__ __launch_bounds__(kThreads, kMinWaves) void fwd_kernel(FwdParams p) {
     }
     // For the backward: the product over the keys between the upper 32-key sub-tile and the row, for every row
     // of the tile (the lower sub-tile's value follows once this tile's upper half is known).
-    const int u_hi = NT == 2 ? 2 * jt + 1 : jt;                // sub-tile at the upper edge of this tile
-    if (carry && half == 0) carry_row(u_hi)[lrow] = prod;
+    const int u_hi = NT * jt + NT - 1;                         // sub-tile at the upper edge of this tile
+    float* const row_lo = NT == 2 ? row_hi - carry_step(u_hi - 1, n_qt) : row_hi;
+    if (carry && half == 0) row_hi[lrow] = prod;
+    row_hi = row_lo - carry_step(NT * jt - 1, n_qt);           // (for the next tile, if there is one)
     if (j0 > w_last - 1 + ac) {                               // nothing visible to this wave yet
-      if (NT == 2 && carry && half == 0) carry_row(u_hi - 1)[lrow] = prod;
+      if (NT == 2 && carry && half == 0) row_lo[lrow] = prod;
       continue;
     }
     const bool diagonal = (j0 + KT - 1) > (w_first - 1 + ac);
@@ -220,7 +223,7 @@ __global__ __launch_bounds__(kThreads, kMinWaves) void fwd_kernel(FwdParams p) {
     const float oth = other_half(run, half);
     // The upper half-wave holds the higher keys, which come first in the sweep.
     const float seed = half ? prod : prod * oth;
-    if (NT == 2 && carry && half == 0) carry_row(u_hi - 1)[lrow] = seed;   // product above the lower sub-tile
+    if (NT == 2 && carry && half == 0) row_lo[lrow] = seed;   // product above the lower sub-tile
     prod = (prod * oth) * run;
     if (kCarryOnly) continue;
     w.back(seed);
@@ -308,13 +311,14 @@ __global__ __launch_bounds__(kThreads, 3) void fwd_dma_kernel(FwdParams p) {
 #pragma unroll
     for (int r = 0; r < 16; r++) oacc[dt][r] = 0.f;
   float prod = 1.f;    // prod over the keys already swept of (1 - sigma): both half-waves hold the same value
-  const int64_t n_qt = (L + kBlockQ - 1) / kBlockQ;
+  const int n_qt = (L + kBlockQ - 1) / kBlockQ;
   float* carry = p.carry ? p.carry + (int64_t)head * p.carry_head_stride + tile.carry_base : nullptr;
   // Slots of sub-tile u: a uniform base and this lane's row within the tile.  The products are read per 64 keys by backward kernels
   // that sweep as many at a time: a sweep that ends on the lower half also records the (empty) product above the upper half.
   const uint32_t lrow = wave * 32 + col;
   auto carry_row = [&](int u) { return carry + carry_offset(u, n_qt) + (q0 - kBlockQ * (u >> 2)); };
   if (carry && half == 0 && (n_kt & 1)) carry_row(n_kt)[lrow] = 1.f;
+  float* row = carry_row(n_kt - 1);
   const int s15 = lane & 15, g = (lane >> 4) & 1;
   const int row_a = col * 64 + ((half ^ ((col >> 2) & 3)) << 4);                                                   // odd steps: ^ 32
   const int tr_k = (4 * half + (s15 >> 2)) * 64 + (((2 * g + ((s15 >> 1) & 1)) ^ half) << 4) + 8 * (s15 & 1);      // the next 4 rows: (^ 32) + 512
@@ -323,7 +327,8 @@ __global__ __launch_bounds__(kThreads, 3) void fwd_dma_kernel(FwdParams p) {
   for (int jt = n_kt - 1; jt >= 0; --jt) {
     const int j0 = jt * KT;
     if (jt > 0) request(jt - 1);
-    if (carry && half == 0) carry_row(jt)[lrow] = prod;       // for the backward: the product over the keys between this tile and the row
+    if (carry && half == 0) row[lrow] = prod;                 // for the backward: the product over the keys between this tile and the row
+    row -= carry_step(jt - 1, n_qt);
     if (j0 <= w_last - 1 + ac) {                              // (else nothing visible to this wave yet)
       const bool diagonal = (j0 + KT - 1) > (w_first - 1 + ac);
       lds_u8* kt = lds + (jt & 1) * kBuf;

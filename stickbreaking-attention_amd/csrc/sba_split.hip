@@ -141,7 +141,7 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_split_kernel(FwdParams p) {
   const T* kb = (const T*)p.k.ptr + tile.seq_id * p.k.sb + head * p.k.sh + tok0 * p.k.st;
   const T* vb = (const T*)p.v.ptr + tile.seq_id * p.v.sb + head * p.v.sh + tok0 * p.v.st;
   const int qi = q0 + col;
-  const int64_t n_qt = (L + kBlockQ - 1) / kBlockQ;
+  const int n_qt = (L + kBlockQ - 1) / kBlockQ;
   float* carry = p.carry ? p.carry + (int64_t)head * p.carry_head_stride + tile.carry_base + sub * kSplitRows : nullptr;
   const int last_key = min(q0 + kSplitRows, L) - 2 + ac, n_sub = last_key < 0 ? 0 : last_key / 32 + 1;
   const int krow = mfma_row_to_key32(col);
@@ -169,6 +169,9 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_split_kernel(FwdParams p) {
 #pragma unroll
     for (int r = 0; r < 16; r++) oacc[dt][r] = 0.f;
   float prod = 1.f;      // product over the keys of this wave's sub-tiles done so far
+  settle(qf);
+  float* const lowest_row = carry_row(bottom);
+  float* row = carry_row(top - 1);
   for (int u = top - 1; u >= bottom; --u) {
     const int j0 = 32 * u;
     ck.store(k_lds);
@@ -184,7 +187,8 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_split_kernel(FwdParams p) {
     const int lim = qi + ac - j0 - 16 * half;
     if (j0 + 31 > q0 - 1 + ac) w.template front<true>(s, p.scale_log2, lim); else w.template front<false>(s, p.scale_log2, lim);
     const float oth = other_half(w.run, half);
-    if (carry && half == 0) carry_row(u)[col] = prod;
+    if (carry && half == 0) row[col] = prod;
+    row -= carry_step(u - 1, n_qt);
     const float seed = half ? prod : prod * oth;              // the upper half-wave holds the higher keys
     prod *= w.run * oth;
     if (!kCarryOnly) {
@@ -207,8 +211,25 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_split_kernel(FwdParams p) {
     prod *= xch[x][col];
   }
   if (carry && half == 0 && wave < kWaves - 1) {
-#pragma unroll 4
-    for (int u = bottom; u < top; u++) carry_row(u)[col] *= above;
+    // (Four under way at a time: one after the other, 15 sub-tiles took as many latencies.)
+    row = lowest_row;
+    int u = bottom;
+    for (; u + 4 <= top; u += 4) {
+      float* at[4];
+      float x[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        at[i] = row;
+        x[i] = row[col];
+        row += carry_step(u + i, n_qt);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; i++) at[i][col] = x[i] * above;
+    }
+    for (; u < top; u++) {
+      row[col] *= above;
+      row += carry_step(u, n_qt);
+    }
   }
   if (kCarryOnly) return;
   if (wave < kWaves - 1) {
@@ -265,9 +286,8 @@ __global__ __launch_bounds__(kThreads, DH == 128 ? 1 : 2) void bwd_dq_split_kern
   const bool row_ok = qi < L;
   const int last_key = min(q0 + kSplitRows, L) - 2 + ac, n_kt = last_key < 0 ? 0 : last_key / kStep + 1;
   const int krow = mfma_row_to_key32(col);
-  const int64_t n_qt = (L + kBlockQ - 1) / kBlockQ;
-  const int64_t slot0 = (int64_t)head * p.carry_head_stride + tile.carry_base + sub * kSplitRows;
-  auto slot_row = [&](int u) { return slot0 + carry_offset(u, n_qt) + (tile.origin - kBlockQ * (u >> 2)); };
+  const int n_qt = (L + kBlockQ - 1) / kBlockQ;
+  int64_t slot_row = (int64_t)head * p.carry_head_stride + tile.carry_base + sub * kSplitRows + carry_offset(wave, n_qt) + tile.origin;      // of this wave's sub-tile
 
   T* const k_lds = reinterpret_cast<T*>(lds_raw) + wave * (2 * SplitLds<DH>::kSub);
   T* const v_lds = k_lds + SplitLds<DH>::kSub;
@@ -277,7 +297,7 @@ __global__ __launch_bounds__(kThreads, DH == 128 ? 1 : 2) void bwd_dq_split_kern
   if (n_kt > 0) {
     ck.load(ksrc, 32 * wave);
     cv.load(vsrc, 32 * wave);
-    if (32 * wave <= last_key) n_prod = (p.carry + slot_row(wave))[col];
+    if (32 * wave <= last_key) n_prod = (p.carry + slot_row)[col];
   }
   typename Elem<T>::vec8 qf[DH / 16], dof[DH / 16];
   load_operand<T, kLoad>(qf, make_row_source<T, kLoad>(qb, p.q.st, L, D), qi, half);
@@ -303,6 +323,9 @@ __global__ __launch_bounds__(kThreads, DH == 128 ? 1 : 2) void bwd_dq_split_kern
 #pragma unroll
     for (int r = 0; r < 16; r++) dqacc[dt][r] = 0.f;
   float prefix = 0.f;      // sum of g over the keys of the steps done so far
+  settle(qf);
+  settle(dof);
+  settle(drem);
   for (int jt = 0; jt < n_kt; ++jt) {
     const int u = 4 * jt + wave, j0 = 32 * u;                 // this wave's sub-tile
     const bool active = j0 <= last_key;
@@ -311,10 +334,12 @@ __global__ __launch_bounds__(kThreads, DH == 128 ? 1 : 2) void bwd_dq_split_kern
     cv.store(v_lds);
     wave_fence();
     const float prod_in = n_prod;
+    float* const prefix_row = p.prefix + slot_row;
+    slot_row += carry_step4(u, n_qt);
     if (jt + 1 < n_kt) {
       ck.load(ksrc, j0 + kStep);
       cv.load(vsrc, j0 + kStep);
-      if (j0 + kStep <= last_key) n_prod = (p.carry + slot_row(u + 4))[col];
+      if (j0 + kStep <= last_key) n_prod = (p.carry + slot_row)[col];
     }
     BwdMath<16> m;
     m.tot = m.oth_g = 0.f;
@@ -336,7 +361,7 @@ __global__ __launch_bounds__(kThreads, DH == 128 ? 1 : 2) void bwd_dq_split_kern
       prefix += y;
     }
     if (active) {
-      if (half == 0) (p.prefix + slot_row(u))[col] = below;   // C just below the sub-tile, for the dK/dV kernel
+      if (half == 0) prefix_row[col] = below;                 // C just below the sub-tile, for the dK/dV kernel
       uint32_t pk[8], dzk[8];
       bwd_math_back<T, 16, false>(m, below + (half ? m.oth_g : 0.f), pk, dzk);
       contract32<T, DH>(dqacc, dzk, k_lds, half, lane);
@@ -401,6 +426,8 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dkv_split_kernel(BwdParams p)
   for (int dt = 0; dt < DH / 32; dt++)
 #pragma unroll
     for (int r = 0; r < 16; r++) { dkacc[dt][r] = 0.f; dvacc[dt][r] = 0.f; }
+  settle(kf);
+  settle(vf);
   for (int i = i_first; i < i_end; i += kWaves) {
     wave_fence();
     cq.store(q_lds);

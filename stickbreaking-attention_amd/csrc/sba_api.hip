@@ -125,7 +125,8 @@ int plan(const SbaArgs* a, Layout* out, bool row_tiles = false) {
   // where a tile's sweep over its keys is the time of the call, and key tiles of 128 keys are the better ones of long sequences:
   // key tiles over the two kernels
   //   20 K .. 64 K, length x heads from 16 K on      0.79 .. 0.93        up to 256 tokens  0.91 .. 0.97
-  //   < 20 K        1024 to 2048 tokens              1.10 .. 1.25        up to 256 tokens  0.93 .. 0.97
+  //   < 20 K        1024 to 2048 tokens              1.10 .. 1.25        up to 256 tokens  0.92 .. 1.20, one launch for two
+  //   12 K .. 64 K  up to 64 tokens                  1.07 .. 1.26
   // At head_dim 64 (against the two kernels; the tiles' element-wise work bounds it, and rows that a tile does not fill cost more):
   //   length     64           128          256          384          512          768, 1024    2048, 4096   8192, 16384
   //   64 K       1.00         1.00         0.90 .. 1.00 1.03         0.84 .. 0.89 0.80 .. 0.84 0.83 .. 0.92 0.88 .. 1.00
@@ -145,7 +146,8 @@ int plan(const SbaArgs* a, Layout* out, bool row_tiles = false) {
     if (L.one_kernel || queues_even(a->num_heads, B, rows, max_len)) L.chain = Layout::kRowTiles;
   } else if (chain_shape && (a->backward_kernels == 2 ||
                              (a->backward_kernels == 0 && rows_heads < kRowTilesFrom &&
-                              (max_len <= 256 || (a->num_heads <= 32 && rows_heads >= 20 << 10 && mean_heads >= 16 << 10))))) {
+                              ((max_len <= 256 && (mean_len > 64 || rows_heads < 12 << 10)) ||
+                               (a->num_heads <= 32 && rows_heads >= 20 << 10 && mean_heads >= 16 << 10))))) {
     L.chain = Layout::kKeyTiles;
     L.one_kernel = true;
   }
@@ -245,49 +247,61 @@ int row_load(const SbaArgs* a, const SbaTensor* const (&tensors)[N]) {
   }
   return load;
 }
-// Whether a call is too small to fill the chip with tiles of 128 query rows (and key tiles): its kernels then split the keys
-// (rows) of a workgroup's rows (keys) over the waves.  By rows times heads, at which the time of the longest row in an unsplit
-// workgroup (a third of which remains when it is split) meets the throughput of the split kernels, which stage K and V four
-// times as often.  Measured on 256 compute units, split / unsplit us (row tiles or key tiles, which split nothing, run the other backwards):
-//   rows x heads          8 K         16 K        32 K        64 K
-//   head_dim 64   fwd   21.0 / 43.3  22.8 / 43.1  30 / 46    53 / 48     (2048 tokens; 8192: 72 / 156, 81 / 157, 88 / 157, 153 / 166)
-//                 dQ    26.4 / 62    28.8 / 61    41 / 63                (87 / 226, 95 / 228, 122 / 229)
-//   head_dim 128  fwd   28.8 / 57    34 / 58      51 / 60    92 / 65     (107 / 212, 120 / 214, 149 / 214, 272 / 231)
-//                 dQ    35.6 / 79    43 / 80                             (125 / 302, 145 / 304, 269 / 304)
-// An unsplit workgroup's longest row costs what it does however many rows there are, so the line rises with the longest sequence; the
-// tiles of long sequences run first, so short ones beside them fill the gaps, and rows count for less the shorter the mean is.
-// Training passes, split / unsplit us, by rows x heads:
-//   head_dim 128   2 x  768   16 K  76 /  85   20 K  85 /  90   22 K  93 /  93      (line at 19 K)
-//                  4 x 1024   16 K  89 / 103   20 K 113 / 117   24 K 126 / 122      (21 K)
-//                  1 x 1740   19 K 135 / 168   25 K 163 / 177   34 K 197 / 186      (27 K)
-//                  2 x 2900   17 K 187 / 256   28 K 270 / 301   40 K 340 / 316      (30 K)
-//    7 of 222 to 1568 (mean 699)   33 K 154 / 165   38 K 161 / 168   5 of 568 down (mean 417)   18 K  75 /  78   22 K 84 / 77   (29 K; 19 K)
-//   head_dim 64    4 x  768   33 K  76 /  76   39 K  82 /  80   45 K  89 /  89      (32 K)
-//                  8 x 1024   32 K  93 /  92   40 K 107 / 104   48 K 119 / 109      (36 K)
-//                  1 x 2900   37 K 162 / 213   48 K 204 / 229   65 K 243 / 235      (60 K)
-//                 12 x 2900   34 K 197 / 232   68 K 263 / 256                       (60 K)
-//   head_dim 50    4 x  768   33 K  83 /  85   39 K  92 /  92   45 K 102 / 104      (32 K)
-// The lines lie where the kernels crossed when the waves of a workgroup staged together and synchronised three times per step.  Over 877 batches
-// of 1 to 146 sequences of up to 8000 tokens (equal, uniform, log-normal, one long among short ones) and head_dims 50 to 128, the rule
-// then lost 0.3 % against the faster kind of each batch, 14 % at most.  Since a wave stages for itself they cross up to a third higher above
-// head_dim 64, and long sequences lose by the cap (7 of 222 to 1568, 33 K: 7 %; 4 heads x 8192 x 128: forward 135 / 209, training pass 631 / 747).
+// Whether a call is too small to fill the chip with tiles of 128 query rows (or key tiles): its kernels then split the keys (rows) of a
+// workgroup's rows (keys) over the waves.  An unsplit workgroup's longest row costs what it does however many rows there are, about a third of
+// which remains when it is split; split kernels stage K and V four times as often, and launch four times the workgroups, of which a
+// short sequence's rows fill one.  So the line, in rows x heads, rises with the longest sequence up to a cap, a sequence counts as 32 rows more
+// than it has, rows count for less the shorter the mean is (tiles of long sequences run first, short ones beside them fill the gaps), and
+// sequences of up to 64 tokens, whose rows see two sub-tiles, are split only where one has the chip to itself (0.5 us either way), so that it
+// keeps its rows' bits when it grows.  Split / unsplit, us, training calls on 256 compute units:
+//   rows x heads         16 K             32 K             64 K         128 K
+//   head_dim 64   fwd    12.6 / 14.4      20.4 / 16.1      39 / 22     54 / 34    512 tokens
+//                        23.0 / 40.3      36.8 / 41.1      57 / 51     92 / 84   2048
+//                        56.6 / 145       84.6 / 146      137 / 178              8192
+//                 dQ     13.2 / 18.5      22.3 / 19.4                             512
+//                        31.0 / 57.7      51.0 / 59.2                            2048
+//                        82.0 / 217      114  / 218      251 / 340 (head_dim 50) 8192
+//                 dK/dV  14.3 / 24.0 (50)                 54 / 37 (50)            512
+//                        38.4 / 82.9 (50) 62.6 / 104 (48 K)  111 / 115 (50)      2048
+//   head_dim 128  fwd    18.4 / 19.0      30.0 / 21.1      67 / 29                512
+//                        37.0 / 55.2      59.2 / 56.8     101 / 73               2048
+//                        91.7 / 200      132  / 204                              8192
+//                 dQ     25.1 / 23.4      43.1 / 25.4                             512
+//                        43.7 / 73.3      98.6 / 76.2                            2048
+//                        130  / 275      258  / 280                              8192
+//   and of short sequences, head_dim 64, fwd / dQ: 64 of 32 tokens, 4 heads 16.2 / 8.3, 13.1 / 5.2; 200 of 64, 4 heads 22.4 / 10.2, 36.9 / 12.6;
+//   64 of 192, 1 head 10.0 / 10.6; one of 3000 and 3 of 300, 7 heads 28.8 / 56.5, 38.5 / 85.1.
+// The lines lose 0.2 % on average and 14 to 22 % at most against the better kernel of each of 500 batches (1 to 400 equal, uniform, log-normal
+// sequences, or one long among short ones, of up to 8192 tokens; 1 to 200 K rows x heads; head_dims 50 to 128).  A line by rows x heads and the
+// longest sequence alone, drawn when the kernels were slower, lost 9 to 17 %, mostly on short sequences.
 // `heads` is the head count of the caller's call, also where the backward takes them through in groups: the groups then run the
 // kernels, and give the bits, of one pass, and products are rebuilt by the kernel whose forward would have kept them.
-bool few_tiles(const SbaArgs* a, int64_t heads, int load) {
-  if (a->dtype == SBA_F32 || load == sba::kLoadScalar) return false;
-  const int64_t seq_rows = a->total_tokens * (a->cu_seqlens ? 1 : a->num_seqs), rows = seq_rows * heads;
+bool below_line(const SbaArgs* a, int64_t heads, int64_t base, int64_t slope, int64_t cap) {
+  const int64_t tokens = a->total_tokens * (a->cu_seqlens ? 1 : a->num_seqs), mean = tokens / a->num_seqs;
   const int64_t longest = a->max_seqlen > 0 && a->max_seqlen < a->total_tokens ? a->max_seqlen : a->total_tokens;
-  const int64_t mean = a->cu_seqlens ? a->total_tokens / a->num_seqs : a->total_tokens;
-  const int64_t cap = a->head_dim > 64 ? 30 << 10 : 60 << 10, line = a->head_dim > 64 ? (13 << 10) + 8 * longest : (20 << 10) + 16 * longest;
-  if (rows >= 2 * cap) return false;
-  return rows * (mean + 3 * longest) < 4 * longest * (line < cap ? line : cap);
+  const int64_t line = base + slope * longest;
+  if (longest <= 64) return longest > 32 && heads * (int64_t)a->num_seqs < 8;
+  return heads * (tokens + 32 * (int64_t)a->num_seqs) * (mean + 2 * longest) < 3 * longest * (line < cap ? line : cap);
 }
-// The same for dK/dV: below, head_dim up to 64 splits the rows over the waves (64 K rows x heads: 73 / 85 us at 2048 tokens, 232 / 314 at 8192; 100 K:
-// 112 / 98 and 338 / 323; 130 K: 155 / 126 and 440 / 423), wider ones take key tiles of 64 instead of 128 (64 K: 113 / 119 at 2048, 354 / 410 at
-// 8192; 130 K: 672 / 657).
+bool few_tiles_fwd(const SbaArgs* a, int64_t heads, int load) {
+  if (a->dtype == SBA_F32 || load == sba::kLoadScalar) return false;
+  return a->head_dim > 64 ? below_line(a, heads, 10 << 10, 19, 48 << 10) : below_line(a, heads, 13 << 10, 25, 65 << 10);
+}
+bool few_tiles_dq(const SbaArgs* a, int64_t heads, int load) {
+  if (a->dtype == SBA_F32 || load == sba::kLoadScalar) return false;
+  return a->head_dim > 64 ? below_line(a, heads, 9 << 10, 6, 48 << 10) : below_line(a, heads, 19 << 10, 18, 80 << 10);
+}
+// The same for dK/dV: below, head_dim up to 64 splits the rows over the waves, wider ones take key tiles of 64 instead of 128.  These are also the
+// better ones of short sequences, however many: 64 keys / 128 keys, us, 256 K to 512 K rows x heads,
+//   tokens          20            64            256           512           1024          4096
+//   head_dim 80     269 / 576     160 / 330     222 / 270     174 / 199     484 / 501     797 / 750
+//            105    341 / 632     252 / 395     330 / 334     232 / 228     638 / 587     983 / 821
+//            128    271 / 291     389 / 411 (1 M)
 bool few_key_tiles(const SbaArgs* a, int64_t heads, int load) {
   if (a->dtype == SBA_F32 || load == sba::kLoadScalar) return false;
-  return a->total_tokens * (a->cu_seqlens ? 1 : a->num_seqs) * heads < 100 << 10;
+  if (a->head_dim <= 64) return below_line(a, heads, 10 << 10, 60, 153 << 10);
+  const int64_t tokens = a->total_tokens * (a->cu_seqlens ? 1 : a->num_seqs);
+  return tokens * heads < 100 << 10 || tokens / a->num_seqs < (a->head_dim & 7 ? 400 : 1100);
 }
 // Row strides from 4 MiB on: the offsets of a row tile's rows beyond the sequence would not stay within 32 bits.
 template <size_t N>
@@ -515,7 +529,7 @@ int fwd_on(const SbaArgs* a, char* ws, size_t ws_bytes, bool ws_is_static, bool 
   hipEvent_t* ev = (hipEvent_t*)a->trace_events;
   if (ev && hipEventRecord(ev[0], stream) != hipSuccess) return SBA_ERR_LAUNCH;
   hipError_t e = (a->dtype == SBA_F32) ? sba::launch_fwd_f32(p, rows_of(a) * a->num_heads, longest_of(a), (int)L.max_q_tiles, stream)
-                 : few_tiles(a, a->num_heads, p.load) ? sba::launch_fwd_split(p, a->dtype == SBA_F16, (int)L.max_q_tiles, stream)
+                 : few_tiles_fwd(a, a->num_heads, p.load) ? sba::launch_fwd_split(p, a->dtype == SBA_F16, (int)L.max_q_tiles, stream)
                                          : sba::launch_fwd(p, a->dtype == SBA_F16, (int)L.max_q_tiles, stream);
   if (e != hipSuccess) return SBA_ERR_LAUNCH;
   if (ev && hipEventRecord(ev[1], stream) != hipSuccess) return SBA_ERR_LAUNCH;
@@ -776,7 +790,7 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* 
     f.max_tiles = (int32_t)L.max_q_tiles;
     f.total_tokens = a->total_tokens;
     f.load = row_load(a, {&a->q, &a->k});
-    if ((few_tiles(a, stat_heads, f.load) ? sba::launch_fwd_split_carry_only(f, a->dtype == SBA_F16, (int)L.max_q_tiles, stream)
+    if ((few_tiles_fwd(a, stat_heads, f.load) ? sba::launch_fwd_split_carry_only(f, a->dtype == SBA_F16, (int)L.max_q_tiles, stream)
                                           : sba::launch_fwd_carry_only(f, a->dtype == SBA_F16, (int)L.max_q_tiles, stream)) != hipSuccess)
       return SBA_ERR_LAUNCH;
   }
@@ -793,7 +807,7 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* 
     return SBA_OK;
   }
   const bool f16 = a->dtype == SBA_F16;
-  if ((few_tiles(a, stat_heads, p.load) ? sba::launch_bwd_dq_split(p, f16, (int)L.max_q_tiles, stream) : sba::launch_bwd_dq(p, f16, (int)L.max_q_tiles, stream)) != hipSuccess)
+  if ((few_tiles_dq(a, stat_heads, p.load) ? sba::launch_bwd_dq_split(p, f16, (int)L.max_q_tiles, stream) : sba::launch_bwd_dq(p, f16, (int)L.max_q_tiles, stream)) != hipSuccess)
     return SBA_ERR_LAUNCH;
   if (ev && last && hipEventRecord(ev[1], stream) != hipSuccess) return SBA_ERR_LAUNCH;
   if ((p.split && a->head_dim <= 64 ? sba::launch_bwd_dkv_split(p, f16, (int)L.max_k_tiles, stream)

@@ -211,8 +211,8 @@ __host__ __device__ inline int64_t carry_offset(int64_t U, int64_t M) {
 }
 // From a row's slot in sub-tile U to its slot in sub-tile U + 1 (or U + 4): a sweep steps from one to the next without the above, which is 20 scalar
 // instructions.
-__host__ __device__ inline int carry_step(int U, int M) { return 128 * (M - (U >> 2) - ((U & 3) == 3)); }
-__host__ __device__ inline int carry_step4(int U, int M) { return 128 * (4 * (M - (U >> 2)) - (U & 3) - 1); }
+__host__ __device__ inline int carry_step(int U, int M) { return 128 * (M - ((U + 1) >> 2)); }
+__host__ __device__ inline int carry_step4(int U, int M) { return 128 * (4 * M - U - 1); }
 __host__ __device__ inline int64_t carry_slots(int64_t M) { return 256 * M * (M + 1); }   // carry_offset(4M, M)
 
 }  // namespace sba

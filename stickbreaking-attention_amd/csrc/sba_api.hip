@@ -23,6 +23,7 @@ hipError_t launch_fwd_split(const FwdParams& p, int dtype_is_f16, int max_tiles,
 hipError_t launch_fwd_split_carry_only(const FwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
 hipError_t launch_bwd_dq_split(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
 hipError_t launch_bwd_dkv_split(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
+hipError_t launch_bwd_tiny(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
 hipError_t launch_fwd_f32(const FwdParams& p, int64_t rows_heads, int64_t longest, int max_tiles, hipStream_t stream);
 hipError_t launch_bwd_f32(const BwdParams& p, int64_t rows_heads, int64_t longest, int max_q_tiles, int max_k_tiles, hipStream_t stream);
 }  // namespace sba
@@ -73,6 +74,18 @@ bool queues_even(int64_t heads, int64_t seqs, int64_t tokens, int64_t max_len) {
   if (max_len * seqs <= 2 * tokens) return true;
   const double others = seqs > 1 ? (double)(tokens - max_len) / max_len : 0., longest = 1. / (1. + others * others / (double)(seqs > 1 ? seqs - 1 : 1));
   return ((double)(8 * cdiv(heads, 8)) / (double)heads - 1.) * longest <= 1. / 7;
+}
+
+// Which sequences the backward of those of up to kTinyRows tokens takes (`load`: as rows can be read): all, where there are no others, and those
+// there are, beside longer ones, where there may be many.  Backward, us, the other kernels / with it: 32 heads, 2048 of 1 to 64 tokens (and one of
+// 64), head_dim 128 2138 / 919, 64 1060 / 468; 1000 of those, 80 1050 / 447; 8 heads, 1000 of up to 64 and one of 300, 64 134 / 63, 128 296 / 47;
+// 32 heads, 2048 of up to 64 beside one of 16384 8070 / 7160; 8 heads, 300 uniform in 1 to 200 130 / 121, log-normal around 55 (80 .. 99 on average)
+// 0.75 .. 1.0 of the time, none of them tiny (65 to 128) 0.94 .. 1.0.  Up to 64 sequences lose (1.0 .. 1.5): one more launch, little to gain.
+int tiny_of(const SbaArgs* a, int load) {
+  if (a->dtype == SBA_F32 || load == sba::kLoadScalar || a->backward_kernels == 2) return sba::kTinyNone;
+  const int64_t longest = a->max_seqlen > 0 && a->max_seqlen < a->total_tokens ? a->max_seqlen : a->total_tokens;
+  if (longest <= sba::kTinyRows) return sba::kTinyAll;
+  return a->cu_seqlens && a->num_seqs > sba::kInlineSeqs && a->total_tokens / a->num_seqs < 128 ? sba::kTinyApart : sba::kTinyNone;
 }
 
 // `row_tiles`: a group of the heads of a call that runs the backward on row tiles, which the group then runs as well (and nothing else:
@@ -180,7 +193,8 @@ int plan(const SbaArgs* a, Layout* out, bool row_tiles = false) {
     // queue) that still fill the chip twice: what is handed over takes its turns in the same memory (2048 short sequences and one of 16384,
     // 32 heads, 8 at a time: 11570 -> 10760 to 10990 us).
     if (mean_len < sba::kRowTileRows && max_len > sba::kRowTileRows) {
-      const int64_t group = align_up(cdiv(2 * kRowTilesFrom, rows), 8);
+      const bool apart = tiny_of(a, sba::kLoadAligned) == sba::kTinyApart;      // (the longest is then what surely is here)
+      const int64_t group = align_up(cdiv(2 * kRowTilesFrom, apart ? max_len : rows), 8);
       if (group < a->num_heads) L.row_group = group;
     }
     chain_bytes = (size_t)L.row_group * L.chain_rows * row_block;
@@ -398,6 +412,8 @@ int expected_key_tile(const SbaArgs* a, const Layout& L) {
   p.split = split_keys(a, L, a->num_heads, p.load);
   return key_tile_of(L, p);
 }
+// ... and whether it will take tiny sequences by themselves.
+int expected_tiny(const SbaArgs* a) { return tiny_of(a, row_load(a, {&a->q, &a->k, &a->v})); }
 
 }  // namespace
 
@@ -503,6 +519,7 @@ int fwd_on(const SbaArgs* a, char* ws, size_t ws_bytes, bool ws_is_static, bool 
   // will rebuild them: both passes then agree on whether the schedule stands.
   sba::FwdParams p{};
   p.sched = sched_params(a, ws, L, for_backward, a->carry != nullptr || a->recompute_carry, for_backward ? expected_key_tile(a, L) : kBlockK);
+  if (for_backward) p.sched.tiny = expected_tiny(a);
   if (fixed || a->num_seqs <= sba::kInlineSeqs) {
     p.sched.service = 1 + clear_wgs(p.sched);
   } else {
@@ -744,6 +761,7 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* 
   p.load = bwd_load(a);
   p.wide_rows = bwd_wide_rows(a);
   p.split = split_keys(a, L, stat_heads, p.load);
+  p.tiny = tiny_of(a, p.load);
   // One kernel (the key tiles of a sequence hand C and partial dQ to each other) where it applies, else dQ then dK/dV.
   const Layout::Chain chain = a->dtype == SBA_F32 ? Layout::kNone : chain_of(L, p);
   if (row_tiles && chain != Layout::kRowTiles) return SBA_ERR_WORKSPACE;      // (route_of asked)
@@ -763,7 +781,8 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* 
   // The key-tile list is built for the dK/dV kernel that will run.
   const int key_tile = a->dtype == SBA_F32 ? kBlockK : key_tile_of(L, p);
   if (!sched) {
-    const sba::SchedParams sp = sched_params(a, ws, L, true, true, key_tile);
+    sba::SchedParams sp = sched_params(a, ws, L, true, true, key_tile);
+    sp.tiny = p.tiny;
     if (sba::launch_sched(sp, clear_wgs(sp), stream) != hipSuccess) return SBA_ERR_LAUNCH;
   }
   hipEvent_t* ev = (hipEvent_t*)a->trace_events;
@@ -793,6 +812,13 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* 
     if ((few_tiles_fwd(a, stat_heads, f.load) ? sba::launch_fwd_split_carry_only(f, a->dtype == SBA_F16, (int)L.max_q_tiles, stream)
                                           : sba::launch_fwd_carry_only(f, a->dtype == SBA_F16, (int)L.max_q_tiles, stream)) != hipSuccess)
       return SBA_ERR_LAUNCH;
+  }
+  if (p.tiny != sba::kTinyNone) {
+    if (sba::launch_bwd_tiny(p, a->dtype == SBA_F16, (int)L.max_q_tiles, stream) != hipSuccess) return SBA_ERR_LAUNCH;
+    if (p.tiny == sba::kTinyAll) {
+      if (ev && last && (hipEventRecord(ev[1], stream) != hipSuccess || hipEventRecord(ev[2], stream) != hipSuccess)) return SBA_ERR_LAUNCH;
+      return SBA_OK;
+    }
   }
   if (chain != Layout::kNone) {
     if (!L.one_kernel && sba::launch_row_clear((uint32_t*)(cleared + L.off_chain_zero), (int64_t)L.chain_zero_bytes, stream) != hipSuccess)
@@ -868,7 +894,7 @@ bool prepared_fits(const SbaArgs* a) {
   p.num_heads = a->num_heads;
   p.add_rem = a->add_remainder ? 1 : 0;
   p.split = split_keys(a, L, a->num_heads, p.load);
-  return a->dtype == SBA_F32 || key_tile_of(L, p) == expected_key_tile(a, L);
+  return a->dtype == SBA_F32 || (key_tile_of(L, p) == expected_key_tile(a, L) && tiny_of(a, p.load) == expected_tiny(a));
 }
 
 int backward_route(const SbaArgs* a, BackwardRoute* out) {

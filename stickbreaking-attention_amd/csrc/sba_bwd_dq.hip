@@ -44,6 +44,7 @@ __global__ __launch_bounds__(kThreads, KT == 32 ? 2 : 1) void bwd_dq_kernel(BwdP
     return;
   }
   const Tile tile = p.q_tiles[slot];
+  if (p.tiny && tile.seq_len <= kTinyRows) return;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, half = lane >> 5, col = lane & 31;
   const int L = tile.seq_len, q0 = tile.origin, ac = p.attend_current, D = p.head_dim;
   const int64_t tok0 = tile.seq_start;

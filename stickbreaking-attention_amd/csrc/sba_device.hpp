@@ -482,13 +482,12 @@ __device__ __forceinline__ void store_acc_tile(const RowSink<T>& sink, const f32
   }
 }
 
-// The same tile through a wave-private LDS scratch of 32 x lds_stride<32>() elements, so that it leaves as two
+// The same tile through a wave-private LDS scratch of 32 x kStride elements, so that it leaves as two
 // 16-byte stores per lane instead of sixteen 2-byte ones: each lane writes its column's 4-key groups transposed
 // ([column][row] layout, 8 bytes per write), and the transpose read hands every lane 8 consecutive columns of one row.
-template <typename T>
+template <typename T, int kStride = lds_stride<32>()>
 __device__ __forceinline__ void store_acc_tile_wide(const RowSink<T>& sink, const f32x16& acc, float scale, int row0, int col0,
                                                     int half, int col, int lane, T* scratch) {
-  constexpr int kStride = lds_stride<32>();
 #pragma unroll
   for (int g = 0; g < 4; g++) {
     uint32_t lo = pack2<T>(acc[4 * g] * scale, acc[4 * g + 1] * scale), hi = pack2<T>(acc[4 * g + 2] * scale, acc[4 * g + 3] * scale);

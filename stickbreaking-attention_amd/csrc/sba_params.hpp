@@ -64,6 +64,7 @@ struct SchedParams {
   int32_t* head_queue;     // backward: per-head cursor into the key-tile list, reset to 0 here
   int32_t num_heads;
   int32_t key_tile;        // keys per key tile (a multiple of 32; what the dK/dV kernel that will run sweeps)
+  int32_t tiny;            // not kTinyNone: sequences of up to kTinyRows tokens get no key tiles
   Turn* k_turns;           // row tiles: beside k_tiles (else NULL)
   int32_t take_turns;      // row tiles: sequences whose tiles take turns in the list, up to kMostTurns (1, and in the scheduler kernel:
                            // each sequence's follow each other)
@@ -74,6 +75,11 @@ struct SchedParams {
 // Most sequences of a packed batch whose tiles the forward's workgroups derive themselves (one lane each).  The derivation
 // takes 5 instructions per sequence and wave behind a scan of the lanes, and replaces a launch of 8 us in front of the forward.
 constexpr int kInlineSeqs = 64;
+
+// Sequences of up to kTinyRows tokens have a backward of their own (sba_bwd_tiny.hip): none of a call, all, or those there are, beside the
+// kernels of the longer ones, which then have no key tiles of them.
+constexpr int kTinyRows = 64;
+enum : int { kTinyNone = 0, kTinyAll = 1, kTinyApart = 2 };
 
 constexpr int kRowTileRows = 256;      // query rows per tile of the backward on row tiles
 // Key blocks of 32 that the row tiles of a sequence hand over, rounded up to whole tiles (none if it is a single tile).
@@ -158,6 +164,7 @@ struct BwdParams {
   int32_t load;                // as in FwdParams
   int32_t wide_rows;           // a row stride of 4 MiB or more
   int32_t split;               // dK/dV: too few key tiles to fill the chip
+  int32_t tiny;                // kTinyNone, kTinyAll or kTinyApart
   // Fused remainder term (the forward wrote o + rem * v): d_rem_eff = d_rem + d_o . v per row, dv += rem * d_o.
   int32_t add_rem;
   const float* row_stat;       // log2(rem), fp32 [batch][head][token]

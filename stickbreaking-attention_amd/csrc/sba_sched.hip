@@ -69,26 +69,27 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
     const int s = s0 + threadIdx.x;
     int start = 0, len = 0;
     if (s < p.num_seqs && !seq_bounds(p, s, &start, &len)) status = kSchedBadCu;
-    const int nq = (len + kBlockQ - 1) / kBlockQ, nk = (len + p.key_tile - 1) / p.key_tile;
+    const int nq = (len + kBlockQ - 1) / kBlockQ, nk = key_tiles(p, len);
     const int cls = min(nq, kBins - 1);
     // (Most sequences of a large batch are of one class.)
+    const uint64_t with_keys = __ballot(nk > 0);
     const int first_cls = __builtin_amdgcn_readfirstlane(cls);
     if (first_cls > 0 && __all(cls == first_cls)) {
       const int of_q = read_lane(sum_up_to_lane(nq), 63), of_k = read_lane(sum_up_to_lane(nk), 63);
       if (lane == 0) {
         atomicAdd(&qbins[cls], of_q);
         if (p.want_key_tiles) atomicAdd(&kbins[cls], of_k);
-        if (p.k_turns) atomicAdd(&sbins[cls], 64);
+        if (p.k_turns) atomicAdd(&sbins[cls], __builtin_popcountll(with_keys));
       }
     } else if (nq) {
       atomicAdd(&qbins[cls], nq);
       if (p.want_key_tiles) atomicAdd(&kbins[cls], nk);
-      if (p.k_turns) atomicAdd(&sbins[cls], 1);
+      if (nk && p.k_turns) atomicAdd(&sbins[cls], 1);
     }
     if (p.k_turns) {
-      const uint64_t mine = row_work(len), of_wave[2] = {wave_sum(nk > 1 ? 0 : mine), wave_sum(nk > 1 ? mine : 0)};
+      const uint64_t mine = nk ? row_work(len) : 0, of_wave[2] = {wave_sum(nk > 1 ? 0 : mine), wave_sum(nk > 1 ? mine : 0)};
       if (lane < 2 && of_wave[lane]) atomicAdd(&work[lane], (unsigned long long)of_wave[lane]);
-      atomicMax(&longest, len);
+      if (nk) atomicMax(&longest, len);
     }
     if (p.row_capacity >= 0) {
       const uint64_t blocks = wave_sum(row_blocks(len));
@@ -152,19 +153,20 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
       seq_bounds(p, s, &start, &len);
       if (p.want_carry_base) cbase = p.carry_base[s];      // written above by this workgroup
     }
-    const int nq = (len + kBlockQ - 1) / kBlockQ, nk = p.want_key_tiles ? (len + p.key_tile - 1) / p.key_tile : 0;
+    const int nq = (len + kBlockQ - 1) / kBlockQ, nk = p.want_key_tiles ? key_tiles(p, len) : 0;
     const int cls = min(nq, kBins - 1);
     const int first_cls = __builtin_amdgcn_readfirstlane(cls);
     if (first_cls > 0 && __all(cls == first_cls)) {      // a place for all of them
       const int upto_q = sum_up_to_lane(nq), upto_k = sum_up_to_lane(nk);
+      const uint64_t with_keys = __ballot(nk > 0);
       if (lane == 0) {
         qbase = atomicAdd(&qbins[cls], read_lane(upto_q, 63));
         if (p.want_key_tiles) kbase = atomicAdd(&kbins[cls], read_lane(upto_k, 63));
-        if (p.k_turns) rank = atomicAdd(&sbins[cls], 64);
+        if (p.k_turns) rank = atomicAdd(&sbins[cls], __builtin_popcountll(with_keys));
       }
       qbase = __builtin_amdgcn_readfirstlane(qbase) + upto_q - nq;
       kbase = __builtin_amdgcn_readfirstlane(kbase) + upto_k - nk;
-      rank = __builtin_amdgcn_readfirstlane(rank) + lane;
+      rank = __builtin_amdgcn_readfirstlane(rank) + __builtin_popcountll(with_keys & ((1ull << lane) - 1));
     } else {
       if (nq) qbase = atomicAdd(&qbins[cls], nq);
       if (nk) kbase = atomicAdd(&kbins[cls], nk);

@@ -45,6 +45,8 @@ __device__ __forceinline__ uint64_t wave_max(uint64_t x) {
   return x;
 }
 
+__device__ __forceinline__ int key_tiles(const SchedParams& p, int len) { return p.tiny && len <= kTinyRows ? 0 : (len + p.key_tile - 1) / p.key_tile; }
+
 // A batch of at most kInlineSeqs sequences (or of equal ones) held by one wave, a sequence per lane.
 struct SeqLanes {
   int start, len, nq;      // this lane's sequence, and its query tiles (0 beyond the last sequence)
@@ -131,7 +133,7 @@ __device__ __forceinline__ void list_lanes(const SchedParams& p, const SeqLanes&
       tiles[j] = j < turns && group + j < 64 ? n : 0;
     }
     const int in_groups = (__builtin_popcountll(__ballot(nk > 1)) + turns - 1) / turns * turns;      // ranks of groups with a sequence of several tiles
-    const uint64_t work = row_work(s.len);
+    const uint64_t work = nk > 0 ? row_work(s.len) : 0;
     *chained = (int)wave_sum(nk > 0 && rank < in_groups ? nk : 0);
     *apart = apart_share(wave_sum(nk > 1 ? 0 : work), wave_sum(nk > 1 ? work : 0), wave_max(work));
   }
@@ -191,7 +193,7 @@ __device__ __forceinline__ void forward_service(const SchedParams& p, int wg) {
   }
   const bool ok = s.status == kSchedOk;
   if (p.want_key_tiles && ok) {
-    const int nk = (s.len + p.key_tile - 1) / p.key_tile;
+    const int nk = key_tiles(p, s.len);
     if (p.cu == nullptr) total_k = nk * p.num_seqs; else first_k = lane_slot(p, s, nk, &total_k);
     if (p.cu == nullptr) chained = nk > 1 ? total_k : 0;
     const int turns = p.take_turns;

@@ -273,6 +273,7 @@ __global__ __launch_bounds__(kThreads, DH == 128 ? 1 : 2) void bwd_dq_split_kern
     return;
   }
   const Tile tile = p.q_tiles[slot];
+  if (p.tiny && tile.seq_len <= kTinyRows) return;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = lane >> 5, col = lane & 31;
   const int L = tile.seq_len, ac = p.attend_current, D = kLoad == kLoadPadded ? p.head_dim : DH;
   const int q0 = tile.origin + sub * kSplitRows;

@@ -751,7 +751,7 @@ __global__ __launch_bounds__(kChThreads) void bwd_chain_kernel(BwdParams p) {
 #pragma unroll
             for (int a4 = 0; a4 < 4; a4++) {
               const f32x4 v = {dq0[4 * a4], dq0[4 * a4 + 1], dq0[4 * a4 + 2], dq0[4 * a4 + 3]};
-              __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), dqc_rs, dqc_voff + 32 * a4, qz0 * (DH * 4), 0);
+              store_16_bytes(__builtin_bit_cast(u32x4, v), dqc_rs, dqc_voff + 32 * a4, qz0 * (DH * 4));
             }
           }
         }

@@ -76,16 +76,18 @@ bool queues_even(int64_t heads, int64_t seqs, int64_t tokens, int64_t max_len) {
   return ((double)(8 * cdiv(heads, 8)) / (double)heads - 1.) * longest <= 1. / 7;
 }
 
-// Which sequences the backward of those of up to kTinyRows tokens takes (`load`: as rows can be read): all, where there are no others, and those
+// Which sequences the backward of those of up to kTinyRows tokens takes (`heads`: of the whole call, `load`: as rows can be read): all, where there are no others, and those
 // there are, beside longer ones, where there may be many.  Backward, us, the other kernels / with it: 32 heads, 2048 of 1 to 64 tokens (and one of
 // 64), head_dim 128 2138 / 919, 64 1060 / 468; 1000 of those, 80 1050 / 447; 8 heads, 1000 of up to 64 and one of 300, 64 134 / 63, 128 296 / 47;
 // 32 heads, 2048 of up to 64 beside one of 16384 8070 / 7160; 8 heads, 300 uniform in 1 to 200 130 / 121, log-normal around 55 (80 .. 99 on average)
-// 0.75 .. 1.0 of the time, none of them tiny (65 to 128) 0.94 .. 1.0.  Up to 64 sequences lose (1.0 .. 1.5): one more launch, little to gain.
-int tiny_of(const SbaArgs* a, int load) {
+// 0.75 .. 1.0 of the time, none of them tiny (65 to 128) 0.94 .. 1.0.  Up to 64 sequences lose (1.0 .. 1.5) and so do 242 with 2 heads (1.03): one
+// more launch, little to gain.
+int tiny_of(const SbaArgs* a, int64_t heads, int load) {
   if (a->dtype == SBA_F32 || load == sba::kLoadScalar || a->backward_kernels == 2) return sba::kTinyNone;
   const int64_t longest = a->max_seqlen > 0 && a->max_seqlen < a->total_tokens ? a->max_seqlen : a->total_tokens;
   if (longest <= sba::kTinyRows) return sba::kTinyAll;
-  return a->cu_seqlens && a->num_seqs > sba::kInlineSeqs && a->total_tokens / a->num_seqs < 128 ? sba::kTinyApart : sba::kTinyNone;
+  return a->cu_seqlens && a->num_seqs > sba::kInlineSeqs && a->num_seqs * heads >= 1024 && a->total_tokens / a->num_seqs < 128 ?
+             sba::kTinyApart : sba::kTinyNone;
 }
 
 // `row_tiles`: a group of the heads of a call that runs the backward on row tiles, which the group then runs as well (and nothing else:
@@ -193,7 +195,7 @@ int plan(const SbaArgs* a, Layout* out, bool row_tiles = false) {
     // queue) that still fill the chip twice: what is handed over takes its turns in the same memory (2048 short sequences and one of 16384,
     // 32 heads, 8 at a time: 11570 -> 10760 to 10990 us).
     if (mean_len < sba::kRowTileRows && max_len > sba::kRowTileRows) {
-      const bool apart = tiny_of(a, sba::kLoadAligned) == sba::kTinyApart;      // (the longest is then what surely is here)
+      const bool apart = tiny_of(a, a->num_heads, sba::kLoadAligned) == sba::kTinyApart;      // (the longest is then what surely is here)
       const int64_t group = align_up(cdiv(2 * kRowTilesFrom, apart ? max_len : rows), 8);
       if (group < a->num_heads) L.row_group = group;
     }
@@ -413,7 +415,7 @@ int expected_key_tile(const SbaArgs* a, const Layout& L) {
   return key_tile_of(L, p);
 }
 // ... and whether it will take tiny sequences by themselves.
-int expected_tiny(const SbaArgs* a) { return tiny_of(a, row_load(a, {&a->q, &a->k, &a->v})); }
+int expected_tiny(const SbaArgs* a) { return tiny_of(a, a->num_heads, row_load(a, {&a->q, &a->k, &a->v})); }
 
 }  // namespace
 
@@ -761,7 +763,7 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* 
   p.load = bwd_load(a);
   p.wide_rows = bwd_wide_rows(a);
   p.split = split_keys(a, L, stat_heads, p.load);
-  p.tiny = tiny_of(a, p.load);
+  p.tiny = tiny_of(a, stat_heads, p.load);
   // One kernel (the key tiles of a sequence hand C and partial dQ to each other) where it applies, else dQ then dK/dV.
   const Layout::Chain chain = a->dtype == SBA_F32 ? Layout::kNone : chain_of(L, p);
   if (row_tiles && chain != Layout::kRowTiles) return SBA_ERR_WORKSPACE;      // (route_of asked)
@@ -894,7 +896,7 @@ bool prepared_fits(const SbaArgs* a) {
   p.num_heads = a->num_heads;
   p.add_rem = a->add_remainder ? 1 : 0;
   p.split = split_keys(a, L, a->num_heads, p.load);
-  return a->dtype == SBA_F32 || (key_tile_of(L, p) == expected_key_tile(a, L) && tiny_of(a, p.load) == expected_tiny(a));
+  return a->dtype == SBA_F32 || (key_tile_of(L, p) == expected_key_tile(a, L) && tiny_of(a, a->num_heads, p.load) == expected_tiny(a));
 }
 
 int backward_route(const SbaArgs* a, BackwardRoute* out) {

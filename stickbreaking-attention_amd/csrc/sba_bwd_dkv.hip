@@ -323,15 +323,10 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dkv5_kernel(BwdParams p) {
   }
   if (k0 >= L) return;
   if (p.add_rem) {      // the forward wrote o + rem * v: dv_j gains rem_j * d_o_j
-    const float* stat = p.row_stat + tile.seq_id * p.stat_sb + head * p.stat_sh + tok0;
+    const float rem = k0 + col < L ? fast_exp2(p.row_stat[tile.seq_id * p.stat_sb + head * p.stat_sh + tok0 + k0 + col]) : 0.f;
+    const RowSource<T> rows = make_row_source<T, kLoad>(dob, p.d_o.st, L, D);
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-      const int j = k0 + 8 * (r >> 2) + 4 * half + (r & 3);
-      const float rem = j < L ? fast_exp2(stat[j]) : 0.f;
-#pragma unroll
-      for (int dt = 0; dt < kDTiles; dt++)
-        if (j < L && 32 * dt + col < D) dvacc[dt][r] += rem * (float)dob[(int64_t)j * p.d_o.st + 32 * dt + col];
-    }
+    for (int dt = 0; dt < kDTiles; dt++) add_scaled_rows<T>(dvacc[dt], rows, rem, k0, 32 * dt, half, col, D);
   }
   const RowSink<T> dk_sink = make_row_sink<T>((T*)p.dk.ptr + tile.seq_id * p.dk.sb + head * p.dk.sh + tok0 * p.dk.st, p.dk.st, L, D);
   const RowSink<T> dv_sink = make_row_sink<T>((T*)p.dv.ptr + tile.seq_id * p.dv.sb + head * p.dv.sh + tok0 * p.dv.st, p.dv.st, L, D);
@@ -389,6 +384,7 @@ __global__ __launch_bounds__(kDkv3Threads) void bwd_dkv3_kernel(BwdParams p) {
   const bool producer = threadIdx.x < 256;
   const int half = lane >> 5, col = lane & 31;
   const int ac = p.attend_current, D = kLoad == kLoadPadded ? p.head_dim : DH;
+  const int own = ac | p.add_rem;      // whether the sweep begins with the tile's own rows even where they do not attend to themselves
   // The `wph` workgroups of a head start with the head's first wph tiles (the list is heaviest first) and then take
   // the next tile from a per-head cursor whenever they finish one, so the load balances itself.  The cursor is read
   // a tile ahead: thread 0 takes the slot after next before a tile's start-up barrier and publishes it through LDS.
@@ -404,7 +400,7 @@ __global__ __launch_bounds__(kDkv3Threads) void bwd_dkv3_kernel(BwdParams p) {
   }
   int* next_slot_lds = reinterpret_cast<int*>(lds_raw + (size_t)Lds::kElems * sizeof(T));
   auto first_row_block = [&](const Tile& tl) {               // first 64-row step that sees the tile's first key
-    const int first_row = tl.origin + 1 - ac;
+    const int first_row = tl.origin + 1 - own;
     return first_row < tl.seq_len ? (first_row / kDkvRows) * kDkvRows : tl.seq_len;
   };
   // The tile record of the next round is fetched a round ahead; the consumers also request the first query rows
@@ -441,7 +437,7 @@ __global__ __launch_bounds__(kDkv3Threads) void bwd_dkv3_kernel(BwdParams p) {
   const int64_t tok0 = tile.seq_start;
   const int jt = j0 / kBlockK;
 
-  const int first_row = j0 + 1 - ac;                         // first row that sees key j0
+  const int first_row = j0 + 1 - own;                        // first row that sees key j0
   const int n_qt = (L + kBlockQ - 1) / kBlockQ;
   const int row_begin = first_row < L ? (first_row / kDkvRows) * kDkvRows : L;
   const int n_steps = (L - row_begin + kDkvRows - 1) / kDkvRows;
@@ -556,20 +552,6 @@ __global__ __launch_bounds__(kDkv3Threads) void bwd_dkv3_kernel(BwdParams p) {
       const int64_t tl_tok0 = tl.seq_start;
       T* dkb = (T*)p.dk.ptr + tl.seq_id * p.dk.sb + head * p.dk.sh + tl_tok0 * p.dk.st;
       T* dvb = (T*)p.dv.ptr + tl.seq_id * p.dv.sb + head * p.dv.sh + tl_tok0 * p.dv.st;
-      if (p.add_rem) {
-        // the remainder term o += rem * v contributes rem_j * d_o_j to dv_j
-        const T* dob = (const T*)p.d_o.ptr + tl.seq_id * p.d_o.sb + head * p.d_o.sh + tl_tok0 * p.d_o.st;
-        const int d = 32 * ct + col;
-#pragma unroll
-        for (int mt = 0; mt < kMT; mt++)
-#pragma unroll
-          for (int r = 0; r < 16; r++) {
-            const int key = tl_j0 + 32 * mt + 8 * (r >> 2) + 4 * half + (r & 3);
-            if (key < tl_len && d < D)
-              dvacc[mt][r] += fast_exp2(p.row_stat[tl.seq_id * p.stat_sb + head * p.stat_sh + tl_tok0 + key]) *
-                              (float)dob[(int64_t)key * p.d_o.st + d];
-          }
-      }
       const RowSink<T> dk_sink = make_row_sink<T>(dkb, p.dk.st, tl_len, D), dv_sink = make_row_sink<T>(dvb, p.dv.st, tl_len, D);
       // Wave-private transposition scratch in the third Q/dO buffer: free during a tile's first step and after the
       // last one.
@@ -585,7 +567,7 @@ __global__ __launch_bounds__(kDkv3Threads) void bwd_dkv3_kernel(BwdParams p) {
   const int L = tile.seq_len, j0 = tile.origin;
   const int64_t tok0 = tile.seq_start;
 
-  const int first_row = j0 + 1 - ac;                         // first row that sees key j0
+  const int first_row = j0 + 1 - own;                        // first row that sees key j0
   const int row_begin = first_row < L ? (first_row / kDkvRows) * kDkvRows : L;
   const int n_steps = (L - row_begin + kDkvRows - 1) / kDkvRows;
 
@@ -619,6 +601,8 @@ __global__ __launch_bounds__(kDkv3Threads) void bwd_dkv3_kernel(BwdParams p) {
         }
       }
     };
+    // The forward wrote o + rem * v: dv_j gains rem_j * d_o_j, and the first step's rows are the tile's own.
+    const float stat = p.add_rem && j0 + lane < L ? p.row_stat[tile.seq_id * p.stat_sb + head * p.stat_sh + tok0 + j0 + lane] : -INFINITY;
     // Step 0: nothing to contract yet, so the previous tile's results leave now.
     stage_step(0);
     if (pending) store_results(done_tile);
@@ -626,6 +610,11 @@ __global__ __launch_bounds__(kDkv3Threads) void bwd_dkv3_kernel(BwdParams p) {
     for (int b = 0; b < kMT; b++)
 #pragma unroll
       for (int r = 0; r < 16; r++) { dkacc[b][r] = 0.f; dvacc[b][r] = 0.f; }
+    if (p.add_rem) {
+#pragma unroll
+      for (int mt = 0; mt < kMT; mt++)
+        add_scaled_rows<T>(dvacc[mt], lds + Lds::kQ + Lds::kQdoTile + 32 * mt * kRowStride + 32 * ct, kRowStride, fast_exp2(stat), 32 * mt, half, col);
+    }
     __syncthreads();
     for (int t = 1; t <= n_steps; ++t) {
       stage_step(t);
@@ -726,6 +715,7 @@ __global__ __launch_bounds__(kDkv4Threads) void bwd_dkv4_kernel(BwdParams p) {
   const bool producer = threadIdx.x < 256;
   const int half = lane >> 5, col = lane & 31;
   const int ac = p.attend_current, D = kLoad == kLoadPadded ? p.head_dim : DH;
+  const int own = ac | p.add_rem;      // whether the sweep begins with the tile's own rows even where they do not attend to themselves
   const int wph = p.wgs_per_head;
   int head, w;
   if ((p.num_heads & 7) == 0) {
@@ -738,7 +728,7 @@ __global__ __launch_bounds__(kDkv4Threads) void bwd_dkv4_kernel(BwdParams p) {
   }
   int* next_slot_lds = reinterpret_cast<int*>(lds_raw + (size_t)Lds::kElems * sizeof(T));
   auto first_row_block = [&](const Tile& tl) {               // first 32-row step that sees the tile's first key
-    const int first_row = tl.origin + 1 - ac;
+    const int first_row = tl.origin + 1 - own;
     return first_row < tl.seq_len ? (first_row / kRows) * kRows : tl.seq_len;
   };
   Tile next_tile = p.k_tiles[w < n_tiles ? w : 0];
@@ -763,7 +753,7 @@ __global__ __launch_bounds__(kDkv4Threads) void bwd_dkv4_kernel(BwdParams p) {
       const int L = tile.seq_len, j0 = tile.origin;
       const int64_t tok0 = tile.seq_start;
       const int jt = j0 / kDkv4Keys;
-      const int first_row = j0 + 1 - ac;                     // first row that sees key j0
+      const int first_row = j0 + 1 - own;                     // first row that sees key j0
       const int n_qt = (L + kBlockQ - 1) / kBlockQ;
       const int row_begin = first_row < L ? (first_row / kRows) * kRows : L;
       const int n_steps = (L - row_begin + kRows - 1) / kRows;
@@ -940,23 +930,6 @@ __global__ __launch_bounds__(kDkv4Threads) void bwd_dkv4_kernel(BwdParams p) {
       T* outb = out ? (T*)p.dk.ptr + tl.seq_id * p.dk.sb + head * p.dk.sh + tl_tok0 * p.dk.st
                     : (T*)p.dv.ptr + tl.seq_id * p.dv.sb + head * p.dv.sh + tl_tok0 * p.dv.st;
       const int64_t out_st = out ? p.dk.st : p.dv.st;
-      if (p.add_rem && out == 0) {
-        // the remainder term o += rem * v contributes rem_j * d_o_j to dv_j
-        const T* dob = (const T*)p.d_o.ptr + tl.seq_id * p.d_o.sb + head * p.d_o.sh + tl_tok0 * p.d_o.st;
-#pragma unroll
-        for (int m = 0; m < 4; m++)
-#pragma unroll
-          for (int r = 0; r < 16; r++) {
-            const int key = tl_j0 + 32 * m + 8 * (r >> 2) + 4 * half + (r & 3);
-            if (key < tl_len) {
-              const float rem = fast_exp2(p.row_stat[tl.seq_id * p.stat_sb + head * p.stat_sh + tl_tok0 + key]);
-#pragma unroll
-              for (int n = 0; n < kCT; n++)
-                if (32 * (kCT * cp + n) + col < D)
-                  acc[m][n][r] += rem * (float)dob[(int64_t)key * p.d_o.st + 32 * (kCT * cp + n) + col];
-            }
-          }
-      }
       const RowSink<T> sink = make_row_sink<T>(outb, out_st, tl_len, D);
       const float scale = out ? p.logit_scale : 1.f;
       T* scratch = lds + Lds::kScratch + wave * (32 * lds_stride<32>());
@@ -970,7 +943,7 @@ __global__ __launch_bounds__(kDkv4Threads) void bwd_dkv4_kernel(BwdParams p) {
       const Tile tile = next_tile;
       const int L = tile.seq_len, j0 = tile.origin;
       const int64_t tok0 = tile.seq_start;
-      const int first_row = j0 + 1 - ac;
+      const int first_row = j0 + 1 - own;
       const int row_begin = first_row < L ? (first_row / kRows) * kRows : L;
       const int n_steps = (L - row_begin + kRows - 1) / kRows;
       const T* qb = (const T*)p.q.ptr + tile.seq_id * p.q.sb + head * p.q.sh + tok0 * p.q.st;
@@ -994,6 +967,14 @@ __global__ __launch_bounds__(kDkv4Threads) void bwd_dkv4_kernel(BwdParams p) {
       slot = *next_slot_lds;                                 // the tile after this one
       const bool have_next = slot < n_tiles;
       if (have_next) next_tile = p.k_tiles[slot];
+      // The forward wrote o + rem * v: dv_j gains rem_j * d_o_j, and the first four steps' rows are the tile's own.
+      const int rem_steps = p.add_rem && !out ? 4 : 0;
+      float stat[2];
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        const int key = j0 + 64 * i + lane;
+        stat[i] = rem_steps && key < L ? p.row_stat[tile.seq_id * p.stat_sb + head * p.stat_sh + tok0 + key] : -INFINITY;
+      }
       // Step 0: nothing to contract yet, so the previous tile's results leave now.
       if (pending) store_results(done_tile);
       stage_rows(2);
@@ -1026,6 +1007,14 @@ __global__ __launch_bounds__(kDkv4Threads) void bwd_dkv4_kernel(BwdParams p) {
           for (int m = 0; m < 4; m++)
 #pragma unroll
             for (int n = 0; n < kCT; n++) acc[m][n] = Elem<T>::mfma(aw[m], br[n], acc[m][n]);
+        }
+        if (u < rem_steps) {
+          const float rem = fast_exp2(u < 2 ? stat[0] : stat[1]);
+#pragma unroll
+          for (int m = 0; m < 4; m++)
+            if (u == m)
+#pragma unroll
+              for (int n = 0; n < kCT; n++) add_scaled_rows<T>(acc[m][n], do_lds + 32 * (kCT * cp + n), kRowStride, rem, 32 * (m & 1), half, col);
         }
         lds_barrier();
       }

@@ -242,7 +242,8 @@ int sba_fwd_static(const SbaArgs* args);
  * Workspace: bwd_bytes of sba_workspace_bytes runs all heads in one pass.  A smaller workspace is taken as a memory
  * limit: the heads are independent, so the call takes them through in groups of as many as fit, one group after
  * the other on the stream (bit-identical results as long as every pass takes the same form of the backward as
- * the single pass would -- see backward_kernels; equal to rounding otherwise).  The minimum is bwd_bytes of the
+ * the single pass would -- see backward_kernels; equal to rounding otherwise).  In fp32 a workspace a little smaller runs all heads
+ * without the planes of split operands, more slowly and with the same bits.  The minimum is bwd_bytes of the
  * same arguments with num_heads = 1; below that the call returns SBA_ERR_WORKSPACE before launching anything.
  * With several groups trace_events
  * bracket the whole call but only the last group's dQ / dK/dV split.
@@ -251,7 +252,8 @@ int sba_bwd(const SbaArgs* args);
 
 /*
  * How many kernels sba_bwd runs behind its schedule for these arguments on the current device when the workspace holds
- * all heads: 1 (see SbaArgs.backward_kernels) or 2 (dQ, then dK/dV; the clearing kernel, then the one on row tiles;
+ * all heads: 1 (see SbaArgs.backward_kernels) or 2 (dQ, then dK/dV, in fp32 each behind one that lays out its operands where sequences are long;
+ * the clearing kernel, then the one on row tiles;
  * also for a call whose heads are split between two forms); a negative SBA_ERR_* for arguments sba_bwd would refuse.
  * Launches nothing.  For callers that attribute the time between trace_events.
  * No counterpart in the reference (it always runs one kernel with atomics and locks, sb_varlen_bwd.py:541-640).

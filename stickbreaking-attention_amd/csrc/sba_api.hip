@@ -43,6 +43,7 @@ struct Layout {
   // ... and in the rest of a backward's workspace, which starts behind it.
   size_t off_prefix, off_drem, off_carry, rest_bytes;
   size_t fwd_bytes, bwd_bytes, carry_bytes;
+  size_t laid_bytes;                        // fp32: behind the rest, where the workspace has them (see laid_pieces)
   size_t pass_bytes;                        // what ONE pass over these heads needs (bwd_bytes: what sba_bwd wants, see split_heads)
   // The backwards in which tiles hand partial sums to each other; these share the prefix plane's region (only one backward runs).
   enum Chain { kNone, kKeyTiles, kRowTiles };
@@ -88,6 +89,23 @@ int tiny_of(const SbaArgs* a, int64_t heads, int load) {
   if (longest <= sba::kTinyRows) return sba::kTinyAll;
   return a->cu_seqlens && a->num_seqs > sba::kInlineSeqs && a->num_seqs * heads >= 1024 && a->total_tokens / a->num_seqs < 128 ?
              sba::kTinyApart : sba::kTinyNone;
+}
+
+// A piece of 32 rows in all planes: three numbers of 2 bytes per element.
+int64_t laid_piece_bytes(const SbaArgs* a) { return sba::kLaidPlanes * 32 * 6 * (int64_t)align_up(a->head_dim, 32); }
+// Pieces of 32 rows per head of the planes of split operands that the fp32 backward works from (0: it splits as it goes).  Laying them out costs
+// what 6 bytes per element and plane cost (12 heads x 128, 6143 tokens: 65 + 45 us), what it saves goes by the pairs, so the line is the mean length.
+// Training passes, laid out / split as it goes, by the bytes of the planes, 1 to 32 heads, head_dims 16 to 128:
+//   mean length     512           1024          2048          4096          8192
+//   to 256 MB       0.94 .. 1.06  0.84 .. 1.00  0.79 .. 0.93  0.74 .. 0.92  0.72 .. 0.91
+//   beyond          1.08 .. 1.16  0.98 .. 1.05  0.86 .. 0.96  0.83 .. 0.92  0.85 .. 0.94
+// and 6143 tokens in sequences of 83 to 2048 (mean 680, 226 MB) 1.04.  (Where both multiply fp32 numbers, see fp32_products_only, the planes are not
+// laid out.)
+int64_t laid_pieces(const SbaArgs* a) {
+  if (a->dtype != SBA_F32) return 0;
+  const int64_t T = a->total_tokens, B = a->num_seqs, mean = a->cu_seqlens ? T / B : T, pieces = a->cu_seqlens ? (T >> 5) + B + 1 : B * cdiv(T, 32);
+  const int64_t bytes = pieces * a->num_heads * laid_piece_bytes(a);
+  return mean >= (bytes <= (int64_t)256 << 20 ? 1024 : 2048) && bytes <= (int64_t)4 << 30 ? pieces : 0;
 }
 
 // `row_tiles`: a group of the heads of a call that runs the backward on row tiles, which the group then runs as well (and nothing else:
@@ -211,7 +229,9 @@ int plan(const SbaArgs* a, Layout* out, bool row_tiles = false) {
   L.off_carry = off;       if (a->recompute_carry) off += L.carry_bytes;
   if (L.chain == Layout::kRowTiles && !L.one_kernel) row_region();
   L.rest_bytes = off;
-  L.bwd_bytes = L.pass_bytes = L.sched_bytes + L.rest_bytes;
+  L.pass_bytes = L.sched_bytes + L.rest_bytes;
+  L.laid_bytes = (size_t)(laid_pieces(a) * a->num_heads * laid_piece_bytes(a));
+  L.bwd_bytes = L.pass_bytes + L.laid_bytes;
   // A head count that is not a multiple of 8 (the reference's own benchmarks use 12) cannot run the one-kernel backward,
   // whose workgroups of a head must share an XCD.  Left to choose, sba_bwd then takes the largest multiple of 8 through
   // it and the remaining heads through the two kernels, one pass after the other on the stream -- where that pays: two
@@ -790,6 +810,10 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* 
   hipEvent_t* ev = (hipEvent_t*)a->trace_events;
   if (ev && first && hipEventRecord(ev[0], stream) != hipSuccess) return SBA_ERR_LAUNCH;
   if (a->dtype == SBA_F32) {
+    if (L.laid_bytes > 0 && p.load != sba::kLoadScalar && a->workspace_bytes >= (sched ? 0 : L.sched_bytes) + L.rest_bytes + L.laid_bytes) {
+      const int64_t pieces = laid_pieces(a);
+      p.laid = sba::LaidPlanes{rest + L.rest_bytes, pieces, pieces * a->num_heads, fixed ? cdiv(a->total_tokens, 32) : 0};
+    }
     if (sba::launch_bwd_f32(p, rows_of(a) * stat_heads, longest_of(a), (int)L.max_q_tiles, (int)L.max_k_tiles, stream) != hipSuccess) return SBA_ERR_LAUNCH;
     if (ev && last && (hipEventRecord(ev[1], stream) != hipSuccess || hipEventRecord(ev[2], stream) != hipSuccess)) return SBA_ERR_LAUNCH;
     return SBA_OK;
@@ -880,7 +904,7 @@ int prepared_bytes(const SbaArgs* a, Prepared* out) {
   Layout L;
   const int st = plan(a, &L);
   if (st != SBA_OK) return st;
-  *out = Prepared{L.sched_bytes, L.rest_bytes, L.carry_bytes, L.one_kernel};
+  *out = Prepared{L.sched_bytes, L.rest_bytes + L.laid_bytes, L.carry_bytes, L.one_kernel};
   return SBA_OK;
 }
 

@@ -342,7 +342,8 @@ __device__ __forceinline__ bool reduce_store_f32(float* lds, const f32x16 (&acc)
 template <int DH, int kMode>
 struct Plain {
   typedef Operand<DH, kMode> Op;
-  static constexpr bool kSplit = false;
+  typedef float Stream[DH / 2];
+  static constexpr bool kSplit = false, kLaid = false;
   static constexpr float kUp = 1.f, kDown = 1.f;
   static __device__ __forceinline__ bool odd_sum(float) { return false; }
   static constexpr int kResident = 32 * (DH + 4), kTurn = Parts<DH>::kTurn;      // floats
@@ -401,7 +402,8 @@ __device__ __forceinline__ Split3 split3(float x0, float x1) {
 template <int DH, int kMode>
 struct Split {
   typedef typename Elem<__bf16>::vec8 vec8;
-  static constexpr bool kSplit = true;
+  typedef float Stream[DH / 2];
+  static constexpr bool kSplit = true, kLaid = false;
   static constexpr float kUp = 0x1p24f, kDown = 0x1p-24f;
   static __device__ __forceinline__ bool odd(float x) { return x != 0.f && !(fabsf(x) >= 0x1p-80f && fabsf(x) <= 0x1p80f); }
   static __device__ __forceinline__ bool odd_sum(float x) { return !(fabsf(x) < INFINITY); }
@@ -483,6 +485,36 @@ struct Split {
     }
     return any;
   }
+  // A wave's 32 x 32 piece p of 32 rows, in x as score_piece() loads it, into a panel of its own: rows 8 i + lane/8 go to their own place,
+  // or (as the A operand) to that of their key.
+  template <bool kLdsIsA>
+  static __device__ __forceinline__ int turn_place(int lane) {
+    const int l8 = lane >> 3, chunk = (lane & 7) >> 1, sub = 8 * (lane & 1);
+    return kLdsIsA ? l8 * 64 + ((chunk ^ (l8 >> 2)) << 4) + sub : (8 * (l8 >> 2) + (l8 & 3)) * 64 + ((chunk ^ (2 * (l8 >> 2))) << 4) + sub;
+  }
+  template <bool kLdsIsA>
+  static __device__ __forceinline__ void put_panel(unsigned char* mine, int w0, const float (&x)[DH / 2], int p, float up) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int w = kLdsIsA ? (w0 ^ (32 * (i & 1))) + 512 * i : (w0 ^ (16 * (i >> 1))) + 1024 * (i & 1) + 256 * (i >> 1);
+      const float* y = x + 16 * p + 4 * i;
+      put(mine + w, y[0], y[1], y[2], y[3], up);
+    }
+  }
+  // Where this lane's part of an operand over 16 columns starts in a panel (the other 16 columns: ^ 32).
+  static __device__ __forceinline__ int row_place(int lane) { return (lane & 31) * 64 + (((lane >> 5) ^ ((lane >> 2) & 3)) << 4); }
+  // 8 numbers as the three planes of an operand.
+  template <typename At>
+  static __device__ __forceinline__ void planes(At&& at, vec8 (&out)[3]) {
+    u32x4 v[3];
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      const Split3 u = split3(at(2 * t), at(2 * t + 1));
+      v[0][t] = u.h; v[1][t] = u.m; v[2][t] = u.l;
+    }
+#pragma unroll
+    for (int j = 0; j < 3; j++) out[j] = as_vec8<__bf16>(v[j]);
+  }
   // The six products that matter, the small ones first.  (m x l twice and l x l are left out, 2^-25 of the product at most.)
   static __device__ __forceinline__ f32x16 six(const vec8 (&a)[3], const vec8 (&b)[3], f32x16 c) {
     c = Elem<__bf16>::mfma(a[2], b[0], c);
@@ -498,18 +530,10 @@ struct Split {
     f32x16 acc = zero16();
     unsigned char* const mine = (unsigned char*)turn;
     const unsigned char* const res = (const unsigned char*)resident;
-    const int lane = this_lane(), l8 = lane >> 3, chunk = (lane & 7) >> 1, sub = 8 * (lane & 1);
-    // rows 8 i + l8 go to their own place, or (as the A operand) to that of their key
-    const int w0 = kLdsIsA ? l8 * 64 + ((chunk ^ (l8 >> 2)) << 4) + sub : (8 * (l8 >> 2) + (l8 & 3)) * 64 + ((chunk ^ (2 * (l8 >> 2))) << 4) + sub;
-    const int row_a = (lane & 31) * 64 + (((lane >> 5) ^ ((lane >> 2) & 3)) << 4);
+    const int lane = this_lane(), w0 = turn_place<kLdsIsA>(lane), row_a = row_place(lane);
 #pragma unroll
     for (int p = 0; p < NB; p++) {
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int w = kLdsIsA ? (w0 ^ (32 * (i & 1))) + 512 * i : (w0 ^ (16 * (i >> 1))) + 1024 * (i & 1) + 256 * (i >> 1);
-        const float* y = x + 16 * p + 4 * i;
-        put(mine + w, y[0], y[1], y[2], y[3], kGrad ? kUp : 1.f);
-      }
+      put_panel<kLdsIsA>(mine, w0, x, p, kGrad ? kUp : 1.f);
       next.template refill<kNextScore>(x, 16 * p, 16 * p + 16);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -536,16 +560,6 @@ struct Split {
                                                   const Op&, bool) {
 #pragma unroll
     for (int i = 0; i < 2; i++) {
-      auto planes = [&](auto&& at, vec8 (&out)[3]) {
-        u32x4 v[3];
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-          const Split3 u = split3(at(2 * t), at(2 * t + 1));
-          v[0][t] = u.h; v[1][t] = u.m; v[2][t] = u.l;
-        }
-#pragma unroll
-        for (int j = 0; j < 3; j++) out[j] = as_vec8<__bf16>(v[j]);
-      };
       vec8 av[3];
       planes([&](int t) { return a[8 * i + t]; }, av);
 #pragma unroll
@@ -559,8 +573,167 @@ struct Split {
     }
   }
 };
+
+// Products of triples whose streamed operand a kernel in front has split and laid out as the matrix instruction takes it (lay_f32_kernel): a
+// wave loads what it needs straight into operand registers, three planes of 1 KB per six products, kAhead operands ahead of their use.  The numbers
+// and the order of the sums are Split's, and so are the bits.
+// What it saves: a workgroup of 32 rows or keys splits every operand that streams past it for itself, which in dQ is 1180 of 1900 vector-ALU
+// instructions per 32 x 32 block (4608 matrix cycles) and in dK/dV 1540 of 2800 (6144), and turns those of the scores round through LDS.  What it costs: six
+// bytes per element from the L2 instead of four, and the planes (the line between the two stands with laid_pieces in sba_api.hip).  Long sequences
+// alone on the chip run at the rate of their instructions (one head x 8192 x 128: 10 us of a wave's 32 x 32 blocks in dQ and dK/dV together); many, where
+// a quarter of the reads miss the L2, wait for those: 12 heads x 128, 6143 tokens, dQ 297 -> 237 us, dK/dV 380 -> 290, laying out 45 + 65.  Two
+// operands ahead instead of four 260 and 319; the resident operand read from LDS one ahead 236 and 305; one workgroup per compute unit
+// 423 (dK/dV); raised wave priority in either phase no change.
+// Training passes, us: one head x 8192 x 128 1303 -> 939, 2 x 4096 x 50 445 -> 368, 8 x 4096 x 128 1160 -> 981, 32 heads x 16384 tokens of 2048 x 128
+// 9187 -> 8729.
 template <int DH, int kMode>
-using Engine = typename std::conditional<kMode == kF32Far, Plain<DH, kMode>, Split<DH, kMode>>::type;
+struct Laid : Split<DH, kMode> {
+  typedef Split<DH, kMode> S;
+  typedef typename S::vec8 vec8;
+  static constexpr bool kLaid = true;
+  static constexpr int NB = S::NB, kTurn = 0;
+  static constexpr int kOps = 2 * NB, kAhead = NB == 4 ? 4 : kOps < 6 ? kOps : 3;      // operands of a phase; a divisor of it
+  static constexpr int kOpBytes = 3 * 1024, kTile = kOps * kOpBytes;                   // of 32 rows
+  struct Op {
+    __amdgpu_buffer_rsrc_t score, contract;      // from the sequence's first 32 rows on
+    int at;                                      // byte of these 32 rows
+  };
+  struct Stream {
+    u32x4 ring[kAhead][3];
+    __amdgpu_buffer_rsrc_t rsrc;                 // of the phase under way
+    int at;
+    __device__ __forceinline__ void load(const __amdgpu_buffer_rsrc_t& r, int byte, int i) {
+      const int voff = this_lane() * 16;
+#pragma unroll
+      for (int j = 0; j < 3; j++) ring[i % kAhead][j] = __builtin_amdgcn_raw_buffer_load_b128(r, voff + 1024 * j, byte + i * kOpBytes, 0);
+    }
+    __device__ __forceinline__ void take(int i, vec8 (&v)[3]) const {
+#pragma unroll
+      for (int j = 0; j < 3; j++) v[j] = as_vec8<__bf16>(ring[i % kAhead][j]);
+    }
+  };
+  template <bool kScore>
+  static __device__ __forceinline__ void fill(Stream& x, const Op& o) {
+    x.rsrc = kScore ? o.score : o.contract;
+    x.at = o.at;
+#pragma unroll
+    for (int i = 0; i < kAhead; i++) x.load(x.rsrc, x.at, i);
+  }
+  // Operand i has been used: the one kAhead further on, of this phase or the next.
+  template <bool kNextScore>
+  static __device__ __forceinline__ void step(Stream& x, const Op& next, int i, bool more = true) {
+    if (i + kAhead < kOps) x.load(x.rsrc, x.at, i + kAhead);
+    else if (more) x.load(kNextScore ? next.score : next.contract, next.at, i + kAhead - kOps);
+    if (i + 1 == kOps) {
+      x.rsrc = kNextScore ? next.score : next.contract;
+      x.at = next.at;
+    }
+  }
+  template <bool kLdsIsA, bool kNextScore, bool kGrad>
+  static __device__ __forceinline__ f32x16 score(Stream& x, float*, const float* resident, int, int, const Op& next, const Op&, bool, uint64_t& odd) {
+    f32x16 acc = zero16();
+    const unsigned char* const res = (const unsigned char*)resident;
+    const int row_a = S::row_place(this_lane());
+#pragma unroll
+    for (int i = 0; i < kOps; i++) {
+      vec8 u[3], v[3];
+      x.take(i, u);
+#pragma unroll
+      for (int j = 0; j < 3; j++) v[j] = *reinterpret_cast<const vec8*>(res + (i >> 1) * S::kPanel + j * S::kPlane + (i & 1 ? row_a ^ 32 : row_a));
+      acc = kLdsIsA ? S::six(v, u, acc) : S::six(u, v, acc);
+      step<kNextScore>(x, next, i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (!kGrad) {
+#pragma unroll
+      for (int r = 0; r < 16; r += 2) odd |= __ballot(__builtin_isunordered(acc[r], acc[r + 1]));
+    }
+    return acc;
+  }
+  template <bool kNextScore>
+  static __device__ __forceinline__ void contract(f32x16 (&acc)[NB], const float (&a)[16], Stream& x, const Op& next, bool more, const Op&, bool) {
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      vec8 av[3];
+      S::planes([&](int t) { return a[8 * i + t]; }, av);
+#pragma unroll
+      for (int dt = 0; dt < NB; dt++) {
+        vec8 bv[3];
+        x.take(i * NB + dt, bv);
+        acc[dt] = S::six(av, bv, acc[dt]);
+        step<kNextScore>(x, next, i * NB + dt, more);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+};
+// The 32-row pieces of a head's sequences in such a plane: sequences one after the other, each from a piece of its own on (packed: what starts at
+// token t of the batch as its s-th sequence at piece t / 32 + s, which is beyond the last piece of the one before).
+__device__ __forceinline__ int64_t laid_piece(const LaidPlanes& l, const Tile& tile) {
+  return l.per_seq ? (int64_t)tile.seq_id * l.per_seq : (int64_t)(tile.seq_start >> 5) + tile.seq_id;
+}
+template <int DH, int kMode>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t laid_rows(const LaidPlanes& l, const Tile& tile, int head, int plane) {
+  constexpr int kTile = Laid<DH, kMode>::kTile;
+  const int64_t first = laid_piece(l, tile), left = min(l.pieces - first, (int64_t)(0x7fffffff / kTile));
+  return __builtin_amdgcn_make_buffer_rsrc(l.base + (plane * l.plane_pieces + head * l.pieces + first) * kTile, 0, (int)left * kTile, 0x00020000);
+}
+
+// Bound by memory: it reads 512 and writes up to 3 KB per row at head_dim 128 (12 heads, 6143 tokens: k and v 45 us, q and d_o 65, 4.6 TB/s).
+// 32 rows of q and d_o (kKeys: k and v) as operands: an MFMA operand is 64 lanes x 16 bytes, its three planes follow each other.  Planes: 0 and
+// 1 q (k) over its columns and over its rows, 2 d_o (v) over its columns, 3 d_o over its rows.  A wave per 32 rows and tensor.
+template <int DH, int kMode, bool kKeys>
+__global__ __launch_bounds__(kThreads, 2) void lay_f32_kernel(BwdParams p) {
+  typedef Split<DH, kMode> S;
+  typedef Laid<DH, kMode> Out;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[kWaves * S::kPanel];
+  int head, slot, second;
+  xcd_head_tile_sub(blockIdx.x, 2, p.num_heads, &head, &slot, &second);
+  if (slot >= p.counts[kCountQ]) return;
+  const Tile tile = p.q_tiles[slot];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = lane >> 5, col = lane & 31;
+  const int row0 = tile.origin + 32 * wave;
+  if (row0 >= tile.seq_len) return;
+  const TensorRef& t = kKeys ? (second ? p.v : p.k) : (second ? p.d_o : p.q);
+  const float* base = (const float*)t.ptr + tile.seq_id * t.sb + head * t.sh + (int64_t)tile.seq_start * t.st;
+  const typename S::Op o = S::op(base, t.st, row0, tile.seq_len, half, col, p.head_dim);
+  unsigned char* const mine = lds + wave * S::kPanel;
+  const int piece = (row0 >> 5) * Out::kTile;
+  auto put = [&](const __amdgpu_buffer_rsrc_t& out, int op, int j, u32x4 v) {
+    __builtin_amdgcn_raw_buffer_store_b128(v, out, lane * 16 + piece + op * Out::kOpBytes + 1024 * j, 0, 0);
+  };
+  float x[DH / 2];
+  S::template fill<true>(x, o);
+  {
+    const __amdgpu_buffer_rsrc_t out = laid_rows<DH, kMode>(p.laid, tile, head, second ? 2 : 0);
+    const int w0 = S::template turn_place<!kKeys>(lane), row_a = S::row_place(lane);
+#pragma unroll
+    for (int c = 0; c < S::NB; c++) {
+      S::template put_panel<!kKeys>(mine, w0, x, c, second ? S::kUp : 1.f);
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int kk = 0; kk < 2; kk++)
+#pragma unroll
+        for (int j = 0; j < 3; j++) put(out, 2 * c + kk, j, *reinterpret_cast<const u32x4*>(mine + j * S::kPlane + (kk ? row_a ^ 32 : row_a)));
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
+  if (kKeys && second) return;
+  S::template fill<false>(x, o);
+  const __amdgpu_buffer_rsrc_t out = laid_rows<DH, kMode>(p.laid, tile, head, second ? 3 : 1);
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int dt = 0; dt < S::NB; dt++) {
+      typename S::vec8 v[3];
+      S::planes([&](int t) { return S::kUp * x[(8 * i + t) * S::NB + dt]; }, v);
+#pragma unroll
+      for (int j = 0; j < 3; j++) put(out, i * S::NB + dt, j, __builtin_bit_cast(u32x4, v[j]));
+    }
+}
+
+template <int DH, int kMode, bool kLaid = false>
+using Engine = typename std::conditional<kMode == kF32Far, Plain<DH, kMode>, typename std::conditional<kLaid, Laid<DH, kMode>, Split<DH, kMode>>::type>::type;
 
 // LDS of the row-stationary kernels: kTiles tiles of 32 rows and the waves' scratch; the final sums lie over both.
 constexpr int most(int a, int b) { return a > b ? a : b; }
@@ -591,7 +764,7 @@ __device__ __forceinline__ bool fwd_f32_rows(const FwdParams& p, const Tile& til
   const int n_sub = last_key < 0 ? 0 : last_key / 32 + 1, n_steps = (n_sub + kWaves - 1) / kWaves;
   auto k_of = [&](int u) { return E::op(kb, p.k.st, 32 * u, L, half, col, D); };
   auto v_of = [&](int u) { return E::op(vb, p.v.st, 32 * u, L, half, col, D); };
-  float x[DH / 2];
+  typename E::Stream x;
   // Wave w takes sub-tile n_sub - 1 - (4 t + w) in step t.
   int U = n_sub - 1 - wave;
   if (U >= 0) E::template fill<true>(x, k_of(U));
@@ -672,6 +845,19 @@ __global__ __launch_bounds__(kThreads, DH == 96 ? 3 : 2) void fwd_f32_kernel(Fwd
   if (p.fp32_products || q0 == 0 || fwd_f32_rows<Engine<DH, kMode>, DH, kMode>(p, tile, head, q0, lds, xch, rem_lds)) fwd_f32_rows<Plain<DH, kMode>, DH, kMode>(p, tile, head, q0, lds, xch, rem_lds);
 }
 
+// What streams past a workgroup of the backward: the operand of 32 rows from 32 u on, as E takes it.
+template <class E, int DH, int kMode>
+__device__ __forceinline__ auto streamed(const LaidPlanes& laid, const Tile& tile, int head, int score, int contract, const float* base, int64_t stride,
+                                         int half, int col, int D) {
+  if constexpr (E::kLaid) {
+    const __amdgpu_buffer_rsrc_t s = laid_rows<DH, kMode>(laid, tile, head, score), c = laid_rows<DH, kMode>(laid, tile, head, contract);
+    return [=](int u) { return typename E::Op{s, c, u * E::kTile}; };
+  } else {
+    const int L = tile.seq_len;
+    return [=](int u) { return E::op(base, stride, 32 * u, L, half, col, D); };
+  }
+}
+
 template <class E, int DH, int kMode>
 __device__ __forceinline__ bool bwd_dq_f32_rows(const BwdParams& p, const Tile& tile, int head, int q0, float* lds, float (&xch)[2][kWaves][32]) {
   constexpr int NB = DH / 32;
@@ -690,9 +876,9 @@ __device__ __forceinline__ bool bwd_dq_f32_rows(const BwdParams& p, const Tile& 
   const int qi = q0 + col;
   const int last_key = min(q0 + kF32Rows, L) - 2 + ac;
   const int n_sub = last_key < 0 ? 0 : last_key / 32 + 1, n_steps = (n_sub + kWaves - 1) / kWaves;
-  auto k_of = [&](int u) { return E::op(kb, p.k.st, 32 * u, L, half, col, D); };
-  auto v_of = [&](int u) { return E::op(vb, p.v.st, 32 * u, L, half, col, D); };
-  float x[DH / 2];
+  const auto k_of = streamed<E, DH, kMode>(p.laid, tile, head, 0, 1, kb, p.k.st, half, col, D);
+  const auto v_of = streamed<E, DH, kMode>(p.laid, tile, head, 2, 2, vb, p.v.st, half, col, D);
+  typename E::Stream x;
   int U = wave;            // wave w takes sub-tile 4 t + w in step t
   if (U < n_sub) E::template fill<true>(x, k_of(U));
   bool staged = E::template stage<false>(lds, rows32(qb, p.q.st, q0, L, D), D);
@@ -763,7 +949,7 @@ __device__ __forceinline__ bool bwd_dq_f32_rows(const BwdParams& p, const Tile& 
   return E::kSplit && any_odd(odd, stored | staged);
 }
 
-template <int DH, int kMode>
+template <int DH, int kMode, bool kLaid>
 __global__ __launch_bounds__(kThreads, 2) void bwd_dq_f32_kernel(BwdParams p) {
   __shared__ __attribute__((aligned(16))) float lds[kRowsF32<DH, kMode, 2>];      // Q and dO rows and the waves' scratch, then the final sums
   __shared__ float xch[2][kWaves][32];
@@ -781,7 +967,7 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dq_f32_kernel(BwdParams p) {
   const Tile tile = p.q_tiles[slot];
   const int q0 = tile.origin + sub * kF32Rows;
   if (q0 >= tile.seq_len) return;
-  if (p.fp32_products || q0 == 0 || bwd_dq_f32_rows<Engine<DH, kMode>, DH, kMode>(p, tile, head, q0, lds, xch)) bwd_dq_f32_rows<Plain<DH, kMode>, DH, kMode>(p, tile, head, q0, lds, xch);
+  if (p.fp32_products || q0 == 0 || bwd_dq_f32_rows<Engine<DH, kMode, kLaid>, DH, kMode>(p, tile, head, q0, lds, xch)) bwd_dq_f32_rows<Plain<DH, kMode>, DH, kMode>(p, tile, head, q0, lds, xch);
 }
 
 template <class E, int DH>
@@ -811,14 +997,14 @@ __device__ __forceinline__ bool bwd_dkv_f32_keys(const BwdParams& p, const Tile&
   const float* prefix = p.prefix + slot0;
   const float* drem_plane = p.drem_eff + tile.seq_id * p.drem_sb + head * p.stat_sh + tok0;
 
-  auto q_of = [&](int b) { return E::op(qb, p.q.st, 32 * b, L, half, col, D); };
-  auto do_of = [&](int b) { return E::op(dob, p.d_o.st, 32 * b, L, half, col, D); };
+  const auto q_of = streamed<E, DH, kMode>(p.laid, tile, head, 0, 1, qb, p.q.st, half, col, D);
+  const auto do_of = streamed<E, DH, kMode>(p.laid, tile, head, 2, 3, dob, p.d_o.st, half, col, D);
   // Row blocks of 32 that see these keys: from the last one down to the one that holds the keys' own rows; wave w takes every
   // fourth.  (Downwards the loop needs one bound fewer in registers: 20 instead of 64 of them spilled at head_dim 128, 2 % of
   // the pass.)
   const int nb = k0 + 1 - ac < L ? (L + 31) / 32 : 0;
   int b = nb - 1 - wave;
-  float x[DH / 2];
+  typename E::Stream x;
   if (b >= U) E::template fill<true>(x, q_of(b));
   // K and V of the 32 keys stay in LDS for the A operands of S^T and dP^T.
   bool staged = E::template stage<true>(lds + Lds::kK, rows32(kb, p.k.st, k0, L, D), D);
@@ -883,7 +1069,7 @@ __device__ __forceinline__ bool bwd_dkv_f32_keys(const BwdParams& p, const Tile&
   return E::kSplit && any_odd(odd, stored | staged);
 }
 
-template <int DH, int kMode>
+template <int DH, int kMode, bool kLaid>
 __global__ __launch_bounds__(kThreads, 2) void bwd_dkv_f32_kernel(BwdParams p) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   int head, slot, sub;
@@ -892,7 +1078,7 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_dkv_f32_kernel(BwdParams p) {
   const Tile tile = p.k_tiles[slot];
   const int k0 = tile.origin + sub * kF32Rows;
   if (k0 >= tile.seq_len) return;
-  if (p.fp32_products || k0 + 2 * kF32Rows > tile.seq_len || bwd_dkv_f32_keys<Engine<DH, kMode>, DH, kMode>(p, tile, head, k0, lds)) bwd_dkv_f32_keys<Plain<DH, kMode>, DH, kMode>(p, tile, head, k0, lds);
+  if (p.fp32_products || k0 + 2 * kF32Rows > tile.seq_len || bwd_dkv_f32_keys<Engine<DH, kMode, kLaid>, DH, kMode>(p, tile, head, k0, lds)) bwd_dkv_f32_keys<Plain<DH, kMode>, DH, kMode>(p, tile, head, k0, lds);
 }
 
 // head_dim is rounded up to a multiple of 32 (the matrix cycles go by that); the exact variants skip every test of a
@@ -958,11 +1144,25 @@ hipError_t launch_bwd_f32(const BwdParams& call, int64_t rows_heads, int64_t lon
     constexpr int DH = decltype(dh)::value;
     constexpr int kMode = decltype(mode)::value;
     constexpr size_t lds_bytes = most(DkvF32Lds<Plain<DH, kMode>, DH>::kFloats, DkvF32Lds<Engine<DH, kMode>, DH>::kFloats) * sizeof(float);
+    const dim3 grid_q((unsigned)xcd_sub_grid(max_q_tiles * p.num_heads, kF32Split)), grid_k((unsigned)xcd_sub_grid(max_k_tiles * p.num_heads, kF32KeySplit)), block(kThreads);
+    if constexpr (kMode != kF32Far) {
+      if (p.laid.base && !p.fp32_products) {
+        static std::atomic<uint64_t> laid_lds_done{0};
+        const hipError_t r = raise_lds_limit(&bwd_dkv_f32_kernel<DH, kMode, true>, laid_lds_done, dev, lds_bytes);
+        if (r != hipSuccess) return r;
+        const dim3 grid((unsigned)xcd_sub_grid(max_q_tiles * p.num_heads, 2));
+        hipLaunchKernelGGL((lay_f32_kernel<DH, kMode, true>), grid, block, 0, stream, p);
+        hipLaunchKernelGGL((bwd_dq_f32_kernel<DH, kMode, true>), grid_q, block, 0, stream, p);
+        hipLaunchKernelGGL((lay_f32_kernel<DH, kMode, false>), grid, block, 0, stream, p);
+        hipLaunchKernelGGL((bwd_dkv_f32_kernel<DH, kMode, true>), grid_k, block, lds_bytes, stream, p);
+        return hipGetLastError();
+      }
+    }
     static std::atomic<uint64_t> lds_done{0};
-    const hipError_t r = raise_lds_limit(&bwd_dkv_f32_kernel<DH, kMode>, lds_done, dev, lds_bytes);
+    const hipError_t r = raise_lds_limit(&bwd_dkv_f32_kernel<DH, kMode, false>, lds_done, dev, lds_bytes);
     if (r != hipSuccess) return r;
-    hipLaunchKernelGGL((bwd_dq_f32_kernel<DH, kMode>), dim3((unsigned)xcd_sub_grid(max_q_tiles * p.num_heads, kF32Split)), dim3(kThreads), 0, stream, p);
-    hipLaunchKernelGGL((bwd_dkv_f32_kernel<DH, kMode>), dim3((unsigned)xcd_sub_grid(max_k_tiles * p.num_heads, kF32KeySplit)), dim3(kThreads), lds_bytes, stream, p);
+    hipLaunchKernelGGL((bwd_dq_f32_kernel<DH, kMode, false>), grid_q, block, 0, stream, p);
+    hipLaunchKernelGGL((bwd_dkv_f32_kernel<DH, kMode, false>), grid_k, block, lds_bytes, stream, p);
     return hipGetLastError();
   });
 }

@@ -146,6 +146,15 @@ struct FwdParams {
   int32_t fp32_products;       // fp32 path: products on the fp32 matrix instruction throughout
 };
 
+// fp32 backward: operands split and laid out by a kernel in front (sba_f32.hip), [plane][head][piece of 32 rows].
+struct LaidPlanes {
+  char* base;                  // NULL: none
+  int64_t pieces;              // per head and plane
+  int64_t plane_pieces;        // per plane
+  int64_t per_seq;             // fixed-length mode: pieces per sequence (else 0)
+};
+constexpr int kLaidPlanes = 4;
+
 struct BwdParams {
   TensorRef q, k, v, d_o, dq, dk, dv;
   VectorRef d_rem;
@@ -190,6 +199,7 @@ struct BwdParams {
   int64_t chain_sb;            // fixed-length mode: rows per batch element (0 in packed mode)
   int32_t chain_tile_cap;      // key-tile slots per head in chain_flags
   int32_t fp32_products;       // as in FwdParams
+  LaidPlanes laid;             // fp32
 };
 
 // One sequence's token range from cu_seqlens (cumulative sequence ends, optionally preceded by a 0).  Returns false

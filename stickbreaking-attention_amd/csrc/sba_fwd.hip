@@ -382,12 +382,96 @@ __global__ __launch_bounds__(kThreads, 3) void fwd_dma_kernel(FwdParams p) {
   store_rows<T, DH, kLoadAligned>(p, tile, head, w_first, half, col, vb, oacc, prod);
 }
 
+// The products of fwd_dma_kernel rebuilt from q and k alone, bit for bit: 64 keys per barrier, K tiles straight into LDS one step ahead, and
+// registers for five waves per SIMD, where the general kernel without V takes three, two barriers per 32 keys and LDS writes.  Bound by vector-ALU
+// issue: 20 transcendentals at 16 cycles and 60 other instructions per 32 x 32 block beside 256 matrix cycles.  16 heads, 16384 tokens 102 -> 96 us.
+template <typename T>
+__global__ __launch_bounds__(kThreads, 4) void fwd_dma_carry_kernel(FwdParams p) {
+  typedef typename Elem<T>::vec8 vec8;
+  constexpr int DH = 128, kSteps = DH / 16, kPanel = 32 * 64, kMat = DH / 32 * kPanel, kBuf = 2 * kMat;      // bytes
+  __shared__ __attribute__((aligned(16))) unsigned char lds_raw[2 * kBuf];
+  lds_u8* const lds = (lds_u8*)lds_raw;
+  const int lds_base = __builtin_amdgcn_readfirstlane((int)(uintptr_t)lds);
+  int head, slot;
+  xcd_head_tile(blockIdx.x, p.num_heads, &head, &slot);
+  Tile tile;
+  int64_t r0, r1;
+  if (!forward_tile(p, slot, 0, kBlockQ, &tile, &r0, &r1)) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = lane >> 5, col = lane & 31;
+  const int L = tile.seq_len, q0 = tile.origin, ac = p.attend_current;
+  const T* qb = (const T*)p.q.ptr + tile.seq_id * p.q.sb + head * p.q.sh + (int64_t)tile.seq_start * p.q.st;
+  const T* kb = (const T*)p.k.ptr + tile.seq_id * p.k.sb + head * p.k.sh + (int64_t)tile.seq_start * p.k.st;
+  const int last_key = min(q0 + kBlockQ, L) - 2 + ac;        // last key any row of this tile can see
+  const int n_kt = last_key < 0 ? 0 : last_key / 32 + 1, n_pt = (n_kt + 1) >> 1;
+  if (n_pt == 0) return;
+  const int w_first = q0 + wave * 32, w_last = w_first + 31, qi = w_first + col;
+
+  // Keys 64 pt .. into buffer pt & 1: a wave brings one panel of either half.  Row m is key mfma_row_to_key32(m): the MFMA's output row.
+  const int k_st = (int)(p.k.st * 2);
+  const u32x4 desc = buffer_desc(kb, (L - 1) * k_st + 2 * DH);
+  const int voff = mfma_row_to_key32(lane >> 2) * k_st + 64 * wave + (((lane & 3) ^ ((lane >> 4) & 3)) << 4);
+  auto request = [&](int pt) {
+    const int dst = lds_base + (pt & 1) * kBuf + wave * kPanel;
+#pragma unroll
+    for (int i = 0; i < 2; i++) dma16x2<1024>(dst + i * kMat, voff, desc, (64 * pt + 32 * i) * k_st, (64 * pt + 32 * i + 8) * k_st);
+  };
+  request(n_pt - 1);
+  vec8 qf[kSteps];
+  load_operand<T, kLoadAligned>(qf, make_row_source<T, kLoadAligned>(qb, p.q.st, L, DH), qi, half);
+  float prod = 1.f;    // prod over the keys already swept of (1 - sigma): both half-waves hold the same value
+  const int n_qt = (L + kBlockQ - 1) / kBlockQ;
+  // (A last pair whose upper half no row sees: its product is the empty one, which the backward kernels that sweep 64 keys read.)
+  const uint32_t lrow = wave * 32 + col;
+  const int top = 2 * n_pt - 1;
+  float* row = p.carry + (int64_t)head * p.carry_head_stride + tile.carry_base + carry_offset(top, n_qt) + (q0 - kBlockQ * (top >> 2));
+  const int row_a = col * 64 + ((half ^ ((col >> 2) & 3)) << 4);      // odd steps: ^ 32
+  vm_wait<0>();
+  lds_barrier();
+  for (int pt = n_pt - 1; pt >= 0; --pt) {
+    if (pt > 0) request(pt - 1);
+#pragma unroll
+    for (int i = 1; i >= 0; --i) {
+      const int jt = 2 * pt + i, j0 = 32 * jt;
+      if (half == 0) row[lrow] = prod;
+      row -= carry_step(jt - 1, n_qt);
+      if (j0 > w_last - 1 + ac) continue;                     // nothing visible to this wave yet
+      const bool diagonal = (j0 + 31) > (w_first - 1 + ac);
+      __builtin_amdgcn_s_setprio(3);
+      f32x16 s[1];
+#pragma unroll
+      for (int r = 0; r < 16; r++) s[0][r] = 0.f;
+      lds_u8* k0 = lds + (pt & 1) * kBuf + i * kMat + row_a;
+      lds_u8* k1 = lds + (pt & 1) * kBuf + i * kMat + (row_a ^ 32);
+      auto k_op = [&](int kk) { return lds_load<vec8>(((kk & 1) ? k1 : k0) + (kk >> 1) * kPanel); };
+      vec8 a[4];
+#pragma unroll
+      for (int kk = 0; kk < 4; kk++) a[kk] = k_op(kk);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int kk = 0; kk < kSteps; kk++) {
+        s[0] = Elem<T>::mfma(a[kk & 3], qf[kk], s[0]);
+        if (kk + 4 < kSteps) a[kk & 3] = k_op(kk + 4);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      __builtin_amdgcn_s_setprio(0);
+      Weights<16> w;
+      const int lim = qi + ac - j0 - 16 * half;               // key R is visible iff R < lim
+      if (diagonal) w.template front<true>(s, p.scale_log2, lim); else w.template front<false>(s, p.scale_log2, lim);
+      prod = (prod * other_half(w.run, half)) * w.run;
+    }
+    if (pt > 0) {      // the next keys are in LDS (the two products just recorded may still be on their way), and these have been read
+      vm_wait<2>();
+      lds_barrier();
+    }
+  }
+}
+
 template <typename T, bool kCarryOnly>
 static hipError_t launch_fwd_t(const FwdParams& p, int max_tiles, hipStream_t stream) {
   const dim3 grid((unsigned)(max_tiles * p.num_heads + p.sched.service)), block(kThreads);
   if (p.load == kLoadAligned) {
     if (p.head_dim == 128 && !kCarryOnly) hipLaunchKernelGGL((fwd_dma_kernel<T>), grid, block, 0, stream, p);
-    else if (p.head_dim == 128) hipLaunchKernelGGL((fwd_kernel<T, 128, kLoadAligned, 32, 3, true>), grid, block, 0, stream, p);
+    else if (p.head_dim == 128) hipLaunchKernelGGL((fwd_dma_carry_kernel<T>), grid, block, 0, stream, p);
     else hipLaunchKernelGGL((fwd_kernel<T, 64, kLoadAligned, 64, 2, kCarryOnly>), grid, block, 0, stream, p);
   } else if (p.load == kLoadPadded) {
     if (p.head_dim > 64) hipLaunchKernelGGL((fwd_kernel<T, 128, kLoadPadded, 32, 3, kCarryOnly>), grid, block, 0, stream, p);

@@ -26,7 +26,9 @@ __device__ __forceinline__ void store_rows(const FwdParams& p, const Tile& tile,
                                            const f32x16 (&oacc)[DH / 32], float prod) {
   constexpr bool kFast = kLoad != kLoadScalar;
   // (Reading v a row at a time, a tile's 16 latencies took a tenth of the forward with the remainder: 211 us instead of 190, 16 heads x 128,
-  // 16384 tokens; 122 and 111 us, 12 heads x 64.  For padded rows it spills in the loop: 187 us instead of 165, 12 heads x 96.)
+  // 16384 tokens; 122 and 111 us, 12 heads x 64.  Padded rows, 4 at a time over all columns, since 16 spill in the loop (187 us instead of 165, 12 heads x
+  // 96): 12 heads, 20 x 500 tokens, head_dim 50 46 -> 39, 80 61 -> 50, 127 88 -> 67; 4 heads x 80, 8 x 52 13.8 -> 9.1; without the remainder, which pays
+  // for one spilled register, 1.00 on average, up to 1.04 at 127.)
   constexpr bool kBatched = kLoad == kLoadAligned;
   constexpr int kDTiles = DH / 32;
   const int L = tile.seq_len, D = p.head_dim, qi = w_first + col;
@@ -51,6 +53,27 @@ __device__ __forceinline__ void store_rows(const FwdParams& p, const Tile& tile,
         for (int r = 0; r < 16; r++) acc[r] += rem_row[r] * (float)__builtin_bit_cast(T, v[r]);
         store_acc_tile<T>(sink, acc, 1.f, w_first, 32 * dt, half, col, DH);
       }
+    } else if (kFast) {      // 4 rows
+      const RowSink<T> sink = make_row_sink<T>(ob, p.o.st, L, D);
+      const RowSource<T> vsrc = make_row_source<T, kLoad>(vb, p.v.st, L, D);
+      const int voff = 4 * half * vsrc.stride_bytes + col * (int)sizeof(T), sbase = __builtin_amdgcn_readfirstlane(w_first * vsrc.stride_bytes);
+      f32x16 acc[kDTiles];
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        uint16_t v[4][kDTiles];
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+          for (int dt = 0; dt < kDTiles; dt++) v[r][dt] = __builtin_amdgcn_raw_buffer_load_b16(vsrc.rsrc, voff, sbase + (8 * g + r) * vsrc.stride_bytes + 64 * dt, 0);
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const float rem_row = __shfl(prod, 8 * g + 4 * half + r);
+#pragma unroll
+          for (int dt = 0; dt < kDTiles; dt++) acc[dt][4 * g + r] = oacc[dt][4 * g + r] + rem_row * (float)__builtin_bit_cast(T, v[r][dt]);
+        }
+      }
+#pragma unroll
+      for (int dt = 0; dt < kDTiles; dt++) store_acc_tile<T>(sink, acc[dt], 1.f, w_first, 32 * dt, half, col, D);
     } else {
 #pragma unroll
       for (int r = 0; r < 16; r++) {

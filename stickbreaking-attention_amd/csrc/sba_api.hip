@@ -287,9 +287,9 @@ int row_load(const SbaArgs* a, const SbaTensor* const (&tensors)[N]) {
 // workgroup's rows (keys) over the waves.  An unsplit workgroup's longest row costs what it does however many rows there are, about a third of
 // which remains when it is split; split kernels stage K and V four times as often, and launch four times the workgroups, of which a
 // short sequence's rows fill one.  So the line, in rows x heads, rises with the longest sequence up to a cap, a sequence counts as 32 rows more
-// than it has, rows count for less the shorter the mean is (tiles of long sequences run first, short ones beside them fill the gaps), and
-// sequences of up to 64 tokens, whose rows see two sub-tiles, are split only where one has the chip to itself (0.5 us either way), so that it
-// keeps its rows' bits when it grows.  Split / unsplit, us, training calls on 256 compute units:
+// than it has, and rows count for less the shorter the mean is (tiles of long sequences run first, short ones beside them fill the gaps).
+// The two kinds round a row's weights at different places, and the line has no step in it, so that a prompt keeps its rows' bits while it
+// grows on one side of it, from the first token on.  Split / unsplit, us, training calls on 256 compute units:
 //   rows x heads         16 K             32 K             64 K         128 K
 //   head_dim 64   fwd    12.6 / 14.4      20.4 / 16.1      39 / 22     54 / 34    512 tokens
 //                        23.0 / 40.3      36.8 / 41.1      57 / 51     92 / 84   2048
@@ -316,7 +316,6 @@ bool below_line(const SbaArgs* a, int64_t heads, int64_t base, int64_t slope, in
   const int64_t tokens = a->total_tokens * (a->cu_seqlens ? 1 : a->num_seqs), mean = tokens / a->num_seqs;
   const int64_t longest = a->max_seqlen > 0 && a->max_seqlen < a->total_tokens ? a->max_seqlen : a->total_tokens;
   const int64_t line = base + slope * longest;
-  if (longest <= 64) return longest > 32 && heads * (int64_t)a->num_seqs < 8;
   return heads * (tokens + 32 * (int64_t)a->num_seqs) * (mean + 2 * longest) < 3 * longest * (line < cap ? line : cap);
 }
 bool few_tiles_fwd(const SbaArgs* a, int64_t heads, int load) {

@@ -4,7 +4,7 @@ import pytest
 import torch
 
 from oracle import sb_oracle as orc
-from stickbreaking_attention import sb_attn_varlen
+from stickbreaking_attention import sb_attn, sb_attn_varlen
 from test_gpu_parity import NAMES, run_varlen, tol_check
 
 pytestmark = pytest.mark.gpu
@@ -72,3 +72,16 @@ def test_a_rows_bits_do_not_depend_on_the_rows_behind_it(gpu_device, H, D, atten
     for T, got in outs.items():
         for n, a in got.items():
             assert torch.equal(a, outs[most][n][:, :T]), f"{n}, {T} rows"
+
+
+@pytest.mark.parametrize("attend_current", [False, True])
+@pytest.mark.parametrize("D", [50, 64, 128])
+@pytest.mark.parametrize("H,count", [(1, 1), (12, 1), (100, 1), (1000, 1), (4, 3)])
+def test_a_short_prompts_bits_stay_when_it_grows(gpu_device, H, count, D, attend_current):
+    """Prompts that grow from one and two sub-tiles of keys to three, at head counts on both sides of the line between the kernels."""
+    g = torch.Generator(device=gpu_device).manual_seed(D)
+    q, k, v = (torch.randn(count, H, 70, D, generator=g, device=gpu_device).bfloat16() for _ in range(3))
+    outs = {T: sb_attn(*(t[:, :, :T] for t in (q, k, v)), attend_current=attend_current) for T in (1, 31, 32, 33, 63, 64, 65, 70)}
+    for T, got in outs.items():
+        for n, a, b in zip(("o", "rem"), got, outs[70]):
+            assert torch.equal(a, b[:, :, :T]), f"{n}, {T} rows"

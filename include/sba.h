@@ -23,7 +23,8 @@
  *     share a workspace must be ordered on one stream.
  *   - cu_seqlens is read on the device, so a bad one cannot be reported by the return value.  The
  *     scheduler checks every entry (non-decreasing, within [0, total_tokens], a leading entry equal
- *     to 0) and that the carry buffer is large enough for the actual lengths; on failure it schedules
+ *     to 0), that the carry buffer is large enough for the actual lengths and, where max_seqlen promises sequences of
+ *     at most 64 tokens (see there), that there is no longer one; on failure it schedules
  *     nothing, all outputs of the call are zero-filled, and the int32 at SBA_STATUS_OFFSET of the
  *     workspace holds SBA_SCHED_BAD_CU_SEQLENS or SBA_SCHED_CARRY_TOO_SMALL (0 otherwise) once the
  *     stream has run.  Rows of the packed token axis at or beyond the last cu_seqlens entry belong to
@@ -93,7 +94,10 @@ typedef struct SbaArgs {
   int64_t total_tokens;        /* T (varlen) or L (fixed) */
   int64_t max_seqlen;          /* upper bound on the longest sequence; <= 0 means "unknown" (T is assumed).  Sizes scratch and takes
                                   part in the choice of the kernels, which an overstated bound may make the slower ones: a
-                                  caller with the lengths on the host passes SbaPlan.longest.  The same in both passes. */
+                                  caller with the lengths on the host passes SbaPlan.longest.  The same in both passes.
+                                  Packed mode, 16-bit, head_dim >= 8: from 1 to 64 it selects a backward that takes no longer sequence.
+                                  One of more than 64 tokens then voids the backward, and with it a forward that keeps
+                                  products or is told of a backward (recompute_carry), as SBA_SCHED_CARRY_TOO_SMALL. */
   float logit_scale;           /* z = logit_scale * q.k  (the operator's inv_temp) */
   int32_t attend_current;      /* 0: keys j < i are visible; 1: keys j <= i */
 
@@ -135,7 +139,7 @@ typedef struct SbaArgs {
                                   as in the reference (q, k, v and, with add_remainder, row_stat), at the price of one more
                                   kernel in the backward.  Must be the same in sba_workspace_bytes and sba_bwd.  16-bit
                                   dtypes only.  In sba_fwd (with carry = NULL) it makes the forward's scheduler check the
-                                  carry capacity exactly as the backward's will, so that an understated max_seqlen or
+                                  carry capacity (and max_seqlen) exactly as the backward's will, so that an understated max_seqlen or
                                   carry_slots voids both passes and not the backward alone. */
   int64_t carry_slots;         /* fp32 slots of `carry` (and of the backward's prefix plane) per head.  0: sized from
                                   the bound total_tokens * max_seqlen / 64 (packed mode), which is several times the

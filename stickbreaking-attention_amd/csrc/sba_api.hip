@@ -77,6 +77,16 @@ bool queues_even(int64_t heads, int64_t seqs, int64_t tokens, int64_t max_len) {
   return ((double)(8 * cdiv(heads, 8)) / (double)heads - 1.) * longest <= 1. / 7;
 }
 
+// What the caller says no sequence has more rows than.
+int64_t claimed_rows(const SbaArgs* a) {
+  return a->cu_seqlens && a->max_seqlen > 0 && a->max_seqlen < a->total_tokens ? a->max_seqlen : a->total_tokens;
+}
+// What a schedule holds the caller to: a backward of tiny sequences alone leaves a longer one's gradients unwritten, and a forward that it follows
+// is void as well.  By what both passes are told alike, and not by whether that backward will run (strides and backward_kernels have their say in it).
+int32_t most_rows_of(const SbaArgs* a) {
+  return a->dtype != SBA_F32 && a->head_dim >= 8 && claimed_rows(a) <= sba::kTinyRows ? sba::kTinyRows : 0x7fffffff;
+}
+
 // Which sequences the backward of those of up to kTinyRows tokens takes (`heads`: of the whole call, `load`: as rows can be read): all, where there are no others, and those
 // there are, beside longer ones, where there may be many.  Backward, us, the other kernels / with it: 32 heads, 2048 of 1 to 64 tokens (and one of
 // 64), head_dim 128 2138 / 919, 64 1060 / 468; 1000 of those, 80 1050 / 447; 8 heads, 1000 of up to 64 and one of 300, 64 134 / 63, 128 296 / 47;
@@ -85,8 +95,7 @@ bool queues_even(int64_t heads, int64_t seqs, int64_t tokens, int64_t max_len) {
 // more launch, little to gain.
 int tiny_of(const SbaArgs* a, int64_t heads, int load) {
   if (a->dtype == SBA_F32 || load == sba::kLoadScalar || a->backward_kernels == 2) return sba::kTinyNone;
-  const int64_t longest = a->max_seqlen > 0 && a->max_seqlen < a->total_tokens ? a->max_seqlen : a->total_tokens;
-  if (longest <= sba::kTinyRows) return sba::kTinyAll;
+  if (claimed_rows(a) <= sba::kTinyRows) return sba::kTinyAll;
   return a->cu_seqlens && a->num_seqs > sba::kInlineSeqs && a->num_seqs * heads >= 1024 && a->total_tokens / a->num_seqs < 128 ?
              sba::kTinyApart : sba::kTinyNone;
 }
@@ -380,6 +389,7 @@ sba::SchedParams sched_params(const SbaArgs* a, char* ws, const Layout& L, bool 
   sp.fixed_len = (int32_t)a->total_tokens;
   sp.total_tokens = a->total_tokens;
   sp.carry_capacity = L.carry_slots_per_head;
+  sp.most_rows = for_backward ? most_rows_of(a) : 0x7fffffff;
   sp.row_capacity = for_backward && L.chain == Layout::kRowTiles && L.rows_by_slot && a->cu_seqlens && key_tile == sba::kRowTileRows ? a->row_blocks : -1;
   sp.want_key_tiles = for_backward ? 1 : 0;
   sp.want_carry_base = want_carry_base ? 1 : 0;
@@ -520,8 +530,8 @@ int static_scratch(char** out) {
 }
 
 // The forward on a given workspace (the caller's, or the library's static scratch).  `for_backward`: the workspace holds
-// sched_bytes and keeps the schedule of the backward that will follow.
-int fwd_on(const SbaArgs* a, char* ws, size_t ws_bytes, bool ws_is_static, bool for_backward) {
+// sched_bytes and keeps the schedule of the backward that will follow.  `alone`: none will follow, whatever the arguments keep for one.
+int fwd_on(const SbaArgs* a, char* ws, size_t ws_bytes, bool ws_is_static, bool for_backward, bool alone = false) {
   Layout L;
   int st = plan(a, &L);
   if (st != SBA_OK) return st;
@@ -536,10 +546,11 @@ int fwd_on(const SbaArgs* a, char* ws, size_t ws_bytes, bool ws_is_static, bool 
   if (ws_is_static && ws_bytes < L.fwd_bytes) return SBA_ERR_TOO_LARGE;
   if (!ws || ((uintptr_t)ws & 255) || ws_bytes < (for_backward ? L.sched_bytes : L.fwd_bytes)) return SBA_ERR_WORKSPACE;
   hipStream_t stream = (hipStream_t)a->stream;
-  // The carry offsets are laid out (and the capacity checked) when products are recorded, and also when the backward
+  // The carry offsets are laid out (and the capacity and the lengths checked) when products are recorded, and also when the backward
   // will rebuild them: both passes then agree on whether the schedule stands.
   sba::FwdParams p{};
   p.sched = sched_params(a, ws, L, for_backward, a->carry != nullptr || a->recompute_carry, for_backward ? expected_key_tile(a, L) : kBlockK);
+  if (p.sched.want_carry_base && !alone) p.sched.most_rows = most_rows_of(a);
   if (for_backward) p.sched.tiny = expected_tiny(a);
   if (fixed || a->num_seqs <= sba::kInlineSeqs) {
     p.sched.service = 1 + clear_wgs(p.sched);
@@ -908,6 +919,7 @@ int prepared_bytes(const SbaArgs* a, Prepared* out) {
 }
 
 int forward_prepared(const SbaArgs* a) { return fwd_on(a, (char*)a->workspace, a->workspace_bytes, false, true); }
+int forward_alone(const SbaArgs* a) { return fwd_on(a, (char*)a->workspace, a->workspace_bytes, false, false, true); }
 
 bool prepared_fits(const SbaArgs* a) {
   Layout L;

@@ -14,6 +14,8 @@ struct Prepared {
 int prepared_bytes(const SbaArgs* a, Prepared* out);
 // sba_fwd with the schedule in a->workspace (`schedule` bytes of it).
 int forward_prepared(const SbaArgs* a);
+// sba_fwd for a call that no backward follows: a max_seqlen below the longest sequence then voids it only where the carry capacity does.
+int forward_alone(const SbaArgs* a);
 // Whether the backward these arguments describe can run on the schedule its forward prepared.
 bool prepared_fits(const SbaArgs* a);
 // sba_bwd on that schedule, with the rest in a->workspace.  The schedule serves ONE backward: its cursors are used up.

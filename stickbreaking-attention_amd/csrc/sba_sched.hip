@@ -54,10 +54,10 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
   __shared__ uint64_t parts[2][1][kSchedWaves];
   __shared__ int bin_parts[3][kSchedWaves];
   __shared__ unsigned long long row_run, work[2];      // work: of the sequences of one row tile, and of more
-  __shared__ int status, longest;
+  __shared__ int status, longest, too_long;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = kSchedWaves;
   for (int i = threadIdx.x; i < kBins; i += kSchedThreads) { qbins[i] = 0; kbins[i] = 0; sbins[i] = 0; }
-  if (threadIdx.x == 0) { row_run = 0; work[0] = work[1] = 0; longest = 0; status = kSchedOk; }
+  if (threadIdx.x == 0) { row_run = 0; work[0] = work[1] = 0; longest = too_long = 0; status = kSchedOk; }
   __syncthreads();
 
   // Pass 1: tiles per length class (class = number of query tiles of the sequence, saturating), and the layout of the carries: a sum over the
@@ -69,6 +69,7 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
     const int s = s0 + threadIdx.x;
     int start = 0, len = 0;
     if (s < p.num_seqs && !seq_bounds(p, s, &start, &len)) status = kSchedBadCu;
+    if (len > p.most_rows) too_long = 1;
     const int nq = (len + kBlockQ - 1) / kBlockQ, nk = key_tiles(p, len);
     const int cls = min(nq, kBins - 1);
     // (Most sequences of a large batch are of one class.)
@@ -105,6 +106,7 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
   }
   __syncthreads();
   int verdict = status;
+  if (verdict == kSchedOk && too_long) verdict = kSchedCarryOverflow;
   if (verdict == kSchedOk && p.row_capacity >= 0 && row_run > (unsigned long long)p.row_capacity) verdict = kSchedCarryOverflow;
   if (verdict == kSchedOk && p.want_carry_base && (int64_t)carry_run > p.carry_capacity) verdict = kSchedCarryOverflow;      // the caller's max_seqlen (or slot count) was too small
   if (verdict != kSchedOk) {      // uniform: nothing is scheduled, every output row is zero-filled as uncovered

@@ -63,6 +63,7 @@ __device__ __forceinline__ SeqLanes load_lanes(const SchedParams& p) {
   const uint64_t slots = carry_slots(s.nq), upto = sum_up_to_lane(slots);
   s.carry_base = (int64_t)(upto - slots);
   if (s.status == kSchedOk && p.want_carry_base && (int64_t)read_lane(upto, 63) > p.carry_capacity) s.status = kSchedCarryOverflow;
+  if (s.status == kSchedOk && __any(s.len > p.most_rows)) s.status = kSchedCarryOverflow;
   if (s.status == kSchedOk && p.row_capacity >= 0 && (int64_t)wave_sum(row_blocks(s.len)) > p.row_capacity) s.status = kSchedCarryOverflow;
   return s;
 }

@@ -210,7 +210,7 @@ Outputs run_forward(const Call& c, const Tensor& q, const Tensor& k, const Tenso
   a.carry = want_carry ? (float*)(state + kept) : nullptr;
   a.workspace = prepare ? state : other;
   a.workspace_bytes = sched;
-  check(prepare ? sba::forward_prepared(&a) : sba_fwd(&a), "sba_fwd");
+  check(prepare ? sba::forward_prepared(&a) : for_backward ? sba_fwd(&a) : sba::forward_alone(&a), "sba_fwd");
   if (c.flags & kDebugCheck) check_status(prepare ? out.state : scratch, "sba_fwd");
   return out;
 }

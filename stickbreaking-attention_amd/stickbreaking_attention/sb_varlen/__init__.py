@@ -55,7 +55,8 @@ def sb_attn_varlen(q, k, v, cu_seqlens, max_seqlens=None, inv_temp=None, zero_st
 
     A ``cu_seqlens`` that exists only on the device (a GPU tensor with ``zero_start=False``, or any call under
     ``torch.compile``) cannot be validated on the host.  The scheduler kernel validates it instead, and also checks
-    that the sequences fit the scratch sized from ``max_seqlens``; when either check fails it schedules NOTHING:
+    that the sequences fit the scratch sized from ``max_seqlens`` and, in training calls that promise at most 64 tokens, that none
+    is longer; when a check fails it schedules NOTHING:
     ``o``, ``rem`` and all gradients come back as zeros and no error is raised (the reference reads the same entries
     unchecked and would run out of bounds, sb_varlen_fwd.py:283-288).  Set ``SBA_DEBUG_CHECK=1`` to have every launch
     followed by a read of the scheduler's status word (one synchronisation per call) and a ``ValueError`` that says

@@ -196,7 +196,7 @@ const char* sba_strerror(int status);
  * Buffer sizes in bytes: the forward's workspace (tile schedule), the backward's workspace (tile
  * schedules plus the per-(row, key tile) prefix sums that let its two lock-free kernels agree) and the
  * `carry` buffer that travels from the forward to the backward.  Any output pointer may be NULL.
- * Uses dtype, head_dim, num_heads, num_seqs, total_tokens, max_seqlen and cu_seqlens (NULL or not).
+ * Uses dtype, head_dim, num_heads, num_seqs, total_tokens, max_seqlen, cu_seqlens (NULL or not), carry_slots, row_blocks and the flags.
  */
 int sba_workspace_bytes(const SbaArgs* args, size_t* fwd_bytes, size_t* bwd_bytes, size_t* carry_bytes);
 
@@ -246,9 +246,11 @@ int sba_fwd_static(const SbaArgs* args);
  * Workspace: bwd_bytes of sba_workspace_bytes runs all heads in one pass.  A smaller workspace is taken as a memory
  * limit: the heads are independent, so the call takes them through in groups of as many as fit, one group after
  * the other on the stream (bit-identical results as long as every pass takes the same form of the backward as
- * the single pass would -- see backward_kernels; equal to rounding otherwise).  In fp32 a workspace a little smaller runs all heads
- * without the planes of split operands, more slowly and with the same bits.  The minimum is bwd_bytes of the
+ * the single pass would -- see backward_kernels; equal to rounding otherwise).  The minimum is bwd_bytes of the
  * same arguments with num_heads = 1; below that the call returns SBA_ERR_WORKSPACE before launching anything.
+ * In fp32 bwd_bytes holds planes of split operands where sequences are long (24 bytes per element), which a pass does without where its
+ * workspace has no room for them: more slowly, with the same bits.  bwd_bytes with backward_kernels = 1 is without them, for all
+ * heads and (the minimum) for one; sba_bwd takes such a workspace whatever its own backward_kernels is.
  * With several groups trace_events
  * bracket the whole call but only the last group's dQ / dK/dV split.
  */

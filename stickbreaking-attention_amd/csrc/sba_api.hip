@@ -77,6 +77,10 @@ bool queues_even(int64_t heads, int64_t seqs, int64_t tokens, int64_t max_len) {
   return ((double)(8 * cdiv(heads, 8)) / (double)heads - 1.) * longest <= 1. / 7;
 }
 
+// Rows per head, and the longest sequence as far as the caller says.
+int64_t rows_of(const SbaArgs* a) { return a->cu_seqlens ? a->total_tokens : a->num_seqs * a->total_tokens; }
+int64_t longest_of(const SbaArgs* a) { return a->max_seqlen > 0 && a->max_seqlen < a->total_tokens ? a->max_seqlen : a->total_tokens; }
+
 // What the caller says no sequence has more rows than.
 int64_t claimed_rows(const SbaArgs* a) {
   return a->cu_seqlens && a->max_seqlen > 0 && a->max_seqlen < a->total_tokens ? a->max_seqlen : a->total_tokens;
@@ -240,7 +244,7 @@ int plan(const SbaArgs* a, Layout* out, bool row_tiles = false) {
   L.rest_bytes = off;
   L.pass_bytes = L.sched_bytes + L.rest_bytes;
   L.laid_bytes = (size_t)(laid_pieces(a) * a->num_heads * laid_piece_bytes(a));
-  L.bwd_bytes = L.pass_bytes + L.laid_bytes;
+  L.bwd_bytes = L.pass_bytes + (a->backward_kernels == 1 ? 0 : L.laid_bytes);
   // A head count that is not a multiple of 8 (the reference's own benchmarks use 12) cannot run the one-kernel backward,
   // whose workgroups of a head must share an XCD.  Left to choose, sba_bwd then takes the largest multiple of 8 through
   // it and the remaining heads through the two kernels, one pass after the other on the stream -- where that pays: two
@@ -259,10 +263,6 @@ int plan(const SbaArgs* a, Layout* out, bool row_tiles = false) {
   *out = L;
   return SBA_OK;
 }
-
-// Rows per head, and the longest sequence as far as the caller says.
-int64_t rows_of(const SbaArgs* a) { return a->cu_seqlens ? a->total_tokens : a->num_seqs * a->total_tokens; }
-int64_t longest_of(const SbaArgs* a) { return a->max_seqlen > 0 && a->max_seqlen < a->total_tokens ? a->max_seqlen : a->total_tokens; }
 
 size_t elem_size(int dtype) { return dtype == SBA_F32 ? 4 : 2; }
 
@@ -914,7 +914,7 @@ int prepared_bytes(const SbaArgs* a, Prepared* out) {
   Layout L;
   const int st = plan(a, &L);
   if (st != SBA_OK) return st;
-  *out = Prepared{L.sched_bytes, L.rest_bytes + L.laid_bytes, L.carry_bytes, L.one_kernel};
+  *out = Prepared{L.sched_bytes, L.rest_bytes, L.laid_bytes, L.carry_bytes, L.one_kernel};
   return SBA_OK;
 }
 

@@ -5,10 +5,10 @@
 
 namespace sba {
 
-// Sizes: of the schedule, of the backward's workspace besides it, and of `carry`; whether the schedule has parts per row and
-// head (and not only per tile).
+// Sizes: of the schedule, of the backward's workspace besides it, of what makes it faster behind that, and of `carry`; whether the schedule
+// has parts per row and head (and not only per tile).
 struct Prepared {
-  size_t schedule, rest, carry;
+  size_t schedule, rest, laid, carry;
   bool row_parts;
 };
 int prepared_bytes(const SbaArgs* a, Prepared* out);

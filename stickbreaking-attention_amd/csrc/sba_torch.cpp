@@ -138,25 +138,32 @@ int64_t row_blocks(const Tensor& host, bool leading_zero) {
 }
 
 Tensor bytes(size_t n, const Tensor& like) { return at::empty({(int64_t)n}, like.options().dtype(at::kByte)); }
-// The backward's scratch: `n` bytes or, where memory is short, less, which takes the heads through in groups: what the dQ and dK/dV kernels
-// need (up to a fifth of what row tiles do), then half as much, down to what one head needs, the least that sba_bwd accepts.
+// The least workspace that sba_bwd accepts for these arguments: one head's, in fp32 without the planes of split operands.
+size_t least_bytes(const SbaArgs& a) {
+  SbaArgs c = a;
+  c.num_heads = 1;
+  if (c.dtype == SBA_F32) c.backward_kernels = 1;
+  size_t n = 0;
+  check(sba_workspace_bytes(&c, nullptr, &n, nullptr), "sba_workspace_bytes");
+  return n;
+}
+// The backward's scratch: `n` bytes or, where memory is short, less: what the dQ and dK/dV kernels need (in fp32 without those planes; of what row
+// tiles need up to a fifth), then half as much, which takes the heads through in groups, down to the least there can be.
 Tensor backward_bytes(const SbaArgs& a, size_t n, const Tensor& like) {
-  size_t two_kernels = 0, one_head = 0;
+  size_t two_kernels = 0, least = 0;
   for (;;) {
     try {
       return bytes(n, like);
     } catch (const c10::OutOfMemoryError&) {
-      if (one_head == 0) {
+      if (least == 0) {
         SbaArgs c = a;
         c.backward_kernels = 1;
         check(sba_workspace_bytes(&c, nullptr, &two_kernels, nullptr), "sba_workspace_bytes");
-        c = a;
-        c.num_heads = 1;
-        check(sba_workspace_bytes(&c, nullptr, &one_head, nullptr), "sba_workspace_bytes");
+        least = least_bytes(a);
       }
-      if (n <= one_head) throw;
+      if (n <= least) throw;
     }
-    n = std::max(one_head, two_kernels < n ? two_kernels : n / 2);
+    n = std::max(least, two_kernels < n ? two_kernels : n / 2);
   }
 }
 
@@ -261,21 +268,22 @@ variable_list run_backward(Call c, Tensor d_o, Tensor d_rem, Tensor q, Tensor k,
   bool on_schedule = prepared;
   if (prepared) {
     try {
-      ws = bytes(size.rest, q);
+      ws = bytes(size.rest + size.laid, q);
     } catch (const c10::OutOfMemoryError&) {
       on_schedule = false;
+    }
+    if (!on_schedule && size.laid > 0) {
+      try {
+        ws = bytes(size.rest, q);
+        on_schedule = true;
+      } catch (const c10::OutOfMemoryError&) {
+      }
     }
   }
   if (!on_schedule) {
     size_t ws_bytes = 0;
     check(sba_workspace_bytes(&a, nullptr, &ws_bytes, nullptr), "sba_workspace_bytes");
-    if (limit >= 0 && ws_bytes > (size_t)limit) {
-      SbaArgs one = a;                        // the smallest workspace the library accepts is the one of a single head
-      one.num_heads = 1;
-      size_t one_bytes = 0;
-      check(sba_workspace_bytes(&one, nullptr, &one_bytes, nullptr), "sba_workspace_bytes");
-      ws_bytes = std::max((size_t)limit, one_bytes);
-    }
+    if (limit >= 0 && ws_bytes > (size_t)limit) ws_bytes = std::max((size_t)limit, least_bytes(a));
     ws = backward_bytes(a, ws_bytes, q);
   }
   if (c.flags & kPoison) poison(ws);

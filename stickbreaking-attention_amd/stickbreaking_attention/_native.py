@@ -290,22 +290,31 @@ def _workspace_bytes(a: SbaArgs):
     return got
 
 
+def _least_bytes(a: SbaArgs) -> int:
+    """The least workspace that the library's backward accepts: one head's, in fp32 without the planes of split operands."""
+    kernels, heads = a.backward_kernels, a.num_heads
+    a.num_heads = 1
+    if a.dtype == SBA_F32:
+        a.backward_kernels = 1
+    least = _workspace_bytes(a)[1]
+    a.backward_kernels, a.num_heads = kernels, heads
+    return least
+
+
 def _backward_scratch(a: SbaArgs, nbytes: int, device) -> torch.Tensor:
-    """The backward's workspace or, where memory is short, a smaller one, which takes the heads through in groups: what the dQ and dK/dV
-    kernels need, then half as much, down to what one head needs, the least that the library accepts."""
+    """The backward's workspace or, where memory is short, a smaller one: what the dQ and dK/dV kernels need (in fp32 without those planes),
+    then half as much, which takes the heads through in groups, down to the least there can be."""
     while True:
         try:
             return torch.empty(nbytes, dtype=torch.uint8, device=device)
         except torch.cuda.OutOfMemoryError:
-            kernels, heads = a.backward_kernels, a.num_heads
-            a.backward_kernels = 1
+            kernels, a.backward_kernels = a.backward_kernels, 1
             two_kernels = _workspace_bytes(a)[1]
-            a.backward_kernels, a.num_heads = kernels, 1
-            one_head = _workspace_bytes(a)[1]
-            a.num_heads = heads
-            if nbytes <= one_head:
+            a.backward_kernels = kernels
+            least = _least_bytes(a)
+            if nbytes <= least:
                 raise
-            nbytes = max(one_head, two_kernels if two_kernels < nbytes else nbytes // 2)
+            nbytes = max(least, two_kernels if two_kernels < nbytes else nbytes // 2)
 
 
 def _launch_fwd(q, k, v, cu_seqlens, cu_has_leading_zero, max_seqlen, carry_slots, logit_scale, attend_current, add_remainder,
@@ -352,11 +361,7 @@ def _launch_bwd(do, drem, q, k, v, carry, neg_log_acc, cu_seqlens, cu_has_leadin
             a.recompute_carry = 1        # the forward kept no products: rebuild them in the backward's workspace
         nbytes = _workspace_bytes(a)[1]
         if BWD_WORKSPACE_LIMIT is not None and nbytes > BWD_WORKSPACE_LIMIT:
-            # the smallest workspace the library accepts is the one of a single head
-            heads, a.num_heads = a.num_heads, 1
-            one_head = _workspace_bytes(a)[1]
-            a.num_heads = heads
-            nbytes = max(BWD_WORKSPACE_LIMIT, one_head)
+            nbytes = max(BWD_WORKSPACE_LIMIT, _least_bytes(a))
         ws = _backward_scratch(a, nbytes, q.device)
         a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
         if POISON:

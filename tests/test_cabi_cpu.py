@@ -245,3 +245,19 @@ def test_workload_generators():
             assert len(lengths) == count
     assert max(bench.lengths_for("c3")) <= 8192 and bench.lengths_for("c5")[-1] == 16384
     assert bench.visible_pairs([4096] * 8, 32) == 8 * 32 * 4096 * 4095 // 2 == 2146959360
+
+
+def test_planes_of_split_operands_are_not_part_of_the_least_workspace(native):
+    """fp32, long sequences: ``backward_kernels = 1`` reports what sba_bwd does without them, for all heads and for one; what is left over is what
+    the planes take: 24 bytes per element of 32 rows at a time, head_dim rounded up to 32."""
+    def backward(H, D, T, B, max_seqlen, kernels, varlen=True):
+        a = _args(native, H, D, T, B, varlen, max_seqlen, dtype=native.SBA_F32)
+        a.backward_kernels = kernels
+        return native._workspace_bytes(a)[1]
+
+    for H, D, T, B, max_seqlen in ((1, 128, 8192, 1, 8192), (3, 50, 3203, 3, 1153), (5, 32, 20480, 2, 20001), (1, 64, 2048, 1, 2048)):
+        planes = (T // 32 + B + 1) * H * 32 * 24 * (-(-D // 32) * 32)
+        assert backward(H, D, T, B, max_seqlen, 0) - backward(H, D, T, B, max_seqlen, 1) == planes
+        a = _args(native, H, D, T, B, max_seqlen=max_seqlen, dtype=native.SBA_F32)
+        assert native._least_bytes(a) == backward(1, D, T, B, max_seqlen, 1) and (a.num_heads, a.backward_kernels) == (H, 0)
+    assert backward(2, 64, 1025, 3, 0, 0, varlen=False) - backward(2, 64, 1025, 3, 0, 1, varlen=False) == 3 * 33 * 2 * 32 * 24 * 64

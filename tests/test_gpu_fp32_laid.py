@@ -1,20 +1,21 @@
 """The fp32 backward whose streamed operands a kernel in front has split and laid out (sequences of 1024 tokens or more on average): against the
-float64 oracle, and the same bits as where the workspace has no room for that."""
+float64 oracle, and the same bits as where the workspace has no room for that, of which it then takes no more than it is left."""
 import pytest
 import torch
 
 from oracle import sb_oracle as orc
-from stickbreaking_attention import _native
+from stickbreaking_attention import _native, sb_attn_varlen
 from test_gpu_parity import NAMES, run_varlen, small_case
 
 pytestmark = pytest.mark.gpu
 
 
-def backward_bytes(D, H, lengths):
+def backward_bytes(D, H, lengths, planes=True):
     a = _native.SbaArgs()
     a.dtype, a.head_dim, a.num_heads, a.num_seqs = _native.SBA_F32, D, H, len(lengths)
     a.total_tokens, a.max_seqlen, a.cu_seqlens = sum(lengths), max(lengths), 256      # (not read: packed sequences)
-    return _native._workspace_bytes(a)[1]
+    of_planes = (sum(lengths) // 32 + len(lengths) + 1) * H * 32 * 24 * (-(-D // 32) * 32)
+    return _native._workspace_bytes(a)[1] - (0 if planes else of_planes)
 
 
 @pytest.mark.parametrize("lengths,attend_current,add_remainder,token_major", [([1056, 1153, 994], False, False, False),
@@ -48,3 +49,71 @@ def test_against_oracle_and_without_room(gpu_device, D, lengths, attend_current,
         print(f"D={D} {n}: relative error {rel.item():.2e}", flush=True)
         assert rel < 1e-5, f"{n}: {rel.item():.2e}"      # (fp32 sums over up to 2271 terms: sqrt(2271) 2^-24 = 3e-6)
         assert torch.equal(a, b), f"{n}: laid out and not differ"
+
+
+def long_case(device, H, D, lengths):
+    g = torch.Generator(device=device).manual_seed(D)
+    q, k, v, do = (torch.randn(H, sum(lengths), D, generator=g, device=device) for _ in range(4))
+    for t in (q, k, v):
+        t.requires_grad_()
+    o, rem = sb_attn_varlen(q, k, v, torch.tensor(lengths).cumsum(0).int().to(device), max(lengths), zero_start=False)
+    return lambda: torch.autograd.grad(o, [q, k, v], do, retain_graph=True)
+
+
+def peak_of(backward, results):
+    """What a backward takes besides its results."""
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    grads = backward()
+    torch.cuda.synchronize()
+    return grads, torch.cuda.max_memory_allocated() - before - results
+
+
+@pytest.mark.parametrize("host_layer", [True, False])
+def test_a_limit_below_what_one_head_asks_for_is_kept(gpu_device, monkeypatch, host_layer):
+    if not host_layer:
+        monkeypatch.setattr(_native, "use_ext", lambda: False)
+    H, D, lengths = 2, 128, [4096]
+    backward = long_case(gpu_device, H, D, lengths)
+    whole = backward()
+    limit = backward_bytes(D, 1, lengths, planes=False) + (1 << 20)
+    assert limit + (8 << 20) < backward_bytes(D, 1, lengths)
+    _native.set_backward_workspace_limit(limit)
+    try:
+        grads, peak = peak_of(backward, 3 * H * sum(lengths) * D * 4)
+    finally:
+        _native.set_backward_workspace_limit(None)
+    slack = 64 << 10      # (the rows' zero gradients of rem, blocks rounded up)
+    assert peak <= limit + slack
+    for n, x, y in zip(NAMES[2:], whole, grads):
+        assert torch.equal(x, y), n
+
+
+@pytest.mark.parametrize("host_layer", [True, False])
+@pytest.mark.parametrize("H,lengths", [(1, [24576]), (4, [8192, 8192])])
+def test_little_memory_left(gpu_device, monkeypatch, H, lengths, host_layer):
+    """Room for all heads, one or several, without planes only: they run in one pass."""
+    if not host_layer:
+        monkeypatch.setattr(_native, "use_ext", lambda: False)
+    D, device = 128, torch.cuda.current_device()
+    whole = [t.cpu() for t in long_case(gpu_device, H, D, lengths)()]
+    backward = long_case(gpu_device, H, D, lengths)
+    results = 3 * H * sum(lengths) * D * 4
+    least, most = backward_bytes(D, H, lengths, planes=False), backward_bytes(D, H, lengths)
+    left = least + (6 << 20)
+    assert left + (32 << 20) < most
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(device).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + results + left) / total)
+    try:
+        for scheduled in ("by the forward", "by the backward"):
+            grads, peak = peak_of(backward, results)
+            assert 0.9 * least < peak < most, scheduled      # (not a group of heads)
+            for n, x, y in zip(NAMES[2:], whole, grads):
+                assert torch.equal(x, y.cpu()), f"{n}, scheduled {scheduled}"
+            del grads, y
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)

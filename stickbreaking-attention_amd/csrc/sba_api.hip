@@ -26,6 +26,7 @@ hipError_t launch_bwd_dkv_split(const BwdParams& p, int dtype_is_f16, int max_ti
 hipError_t launch_bwd_tiny(const BwdParams& p, int dtype_is_f16, int max_tiles, hipStream_t stream);
 hipError_t launch_fwd_f32(const FwdParams& p, int64_t rows_heads, int64_t longest, int max_tiles, hipStream_t stream);
 hipError_t launch_bwd_f32(const BwdParams& p, int64_t rows_heads, int64_t longest, int max_q_tiles, int max_k_tiles, hipStream_t stream);
+bool fp32_products_only(int D, int64_t rows_heads, int64_t longest, float scale_log2);
 }  // namespace sba
 
 namespace {
@@ -112,10 +113,10 @@ int64_t laid_piece_bytes(const SbaArgs* a) { return sba::kLaidPlanes * 32 * 6 * 
 //   mean length     512           1024          2048          4096          8192
 //   to 256 MB       0.94 .. 1.06  0.84 .. 1.00  0.79 .. 0.93  0.74 .. 0.92  0.72 .. 0.91
 //   beyond          1.08 .. 1.16  0.98 .. 1.05  0.86 .. 0.96  0.83 .. 0.92  0.85 .. 0.94
-// and 6143 tokens in sequences of 83 to 2048 (mean 680, 226 MB) 1.04.  (Where both multiply fp32 numbers, see fp32_products_only, the planes are not
-// laid out.)
+// and 6143 tokens in sequences of 83 to 2048 (mean 680, 226 MB) 1.04.  None where the shape already says that the products are
+// of fp32 numbers.  (Sizes go by shapes and flags alone: a logit scale beyond 709 and rows 64 MiB apart leave the planes unused.)
 int64_t laid_pieces(const SbaArgs* a) {
-  if (a->dtype != SBA_F32) return 0;
+  if (a->dtype != SBA_F32 || sba::fp32_products_only(a->head_dim, rows_of(a) * a->num_heads, longest_of(a), 1.f)) return 0;
   const int64_t T = a->total_tokens, B = a->num_seqs, mean = a->cu_seqlens ? T / B : T, pieces = a->cu_seqlens ? (T >> 5) + B + 1 : B * cdiv(T, 32);
   const int64_t bytes = pieces * a->num_heads * laid_piece_bytes(a);
   return mean >= (bytes <= (int64_t)256 << 20 ? 1024 : 2048) && bytes <= (int64_t)4 << 30 ? pieces : 0;

@@ -1118,7 +1118,7 @@ static bool few_workgroups(int D, int64_t rows_heads, int64_t longest) {
   return rows_heads <= 32 * (longest <= 128 ? 384 : 256) && (D <= 32 || longest < 1024);
 }
 // ... or sums over head_dim that are too short for them, or a logit scale at which the parts that their logits lack would count (see Split).
-static bool fp32_products_only(int D, int64_t rows_heads, int64_t longest, float scale_log2) {
+bool fp32_products_only(int D, int64_t rows_heads, int64_t longest, float scale_log2) {
   return few_workgroups(D, rows_heads, longest) || D <= 2 || !(fabsf(scale_log2) <= 1024.f);
 }
 

@@ -261,3 +261,6 @@ def test_planes_of_split_operands_are_not_part_of_the_least_workspace(native):
         a = _args(native, H, D, T, B, max_seqlen=max_seqlen, dtype=native.SBA_F32)
         assert native._least_bytes(a) == backward(1, D, T, B, max_seqlen, 1) and (a.num_heads, a.backward_kernels) == (H, 0)
     assert backward(2, 64, 1025, 3, 0, 0, varlen=False) - backward(2, 64, 1025, 3, 0, 1, varlen=False) == 3 * 33 * 2 * 32 * 24 * 64
+    # fp32 products whatever the workspace: nothing is asked for
+    for H, D, T in ((1, 32, 2048), (8, 2, 8192)):
+        assert backward(H, D, T, 1, T, 0) == backward(H, D, T, 1, T, 1)

@@ -127,7 +127,10 @@ typedef struct SbaArgs {
   void** trace_events;         /* optional (NULL = off): hipEvent_t handles the library records on `stream` so a
                                   caller can time the kernels separately.  sba_fwd records [0] before and [1] after
                                   the attention kernel (the scheduler kernel runs before [0]); sba_bwd records [0]
-                                  before the dQ kernel, [1] between the dQ and dK/dV kernels and [2] after. */
+                                  before its first kernel behind the schedule, [1] between the dQ and dK/dV kernels (or in front of
+                                  the kernel on key or row tiles) and [2] after: what runs in front of those, the kernel that
+                                  rebuilds the products, the one of tiny sequences and one that clears, is timed between [0] and [1].
+                                  Where one pass is tiny sequences only, or fp32, [1] and [2] are both after. */
   int32_t add_remainder;       /* 1: the forward writes o + rem * v instead of o, the step every caller of the
                                   reference applies to its outputs (tests/test_varlen.py:103, tests/test_attn.py:67).
                                   The backward then takes d_o as the gradient of that sum and d_rem as the
@@ -147,17 +150,20 @@ typedef struct SbaArgs {
                                   SbaPlan.carry_slots from sba_plan_host for the exact size.  Must be the same in the
                                   forward, the backward and sba_workspace_bytes.  Ignored in fixed-length mode, whose
                                   exact count follows from the shape. */
-  int32_t backward_kernels;    /* How sba_bwd computes dq, dk, dv.  1: a dQ kernel and a dK/dV kernel.  2: where it applies
+  int32_t backward_kernels;    /* How sba_bwd computes dq, dk, dv.  1: a dQ kernel and a dK/dV kernel (tiny sequences: as with 0).  2: where it applies
                                   (head_dim 128, 16-bit, 16-byte aligned rows, a head count that is a multiple of 8, no
                                   add_remainder) ONE kernel in which the tiles of a sequence hand partial sums to each
                                   other through the L2: key tiles (partial dQ) below 64 K rows * heads, row tiles (partial
                                   dK and dV) from there on; the two kernels otherwise.
-                                  0: what was measured to be the fastest.  Below 64 K rows * heads the one kernel where it
-                                  applies and no sequence is longer than 256 tokens, or at most 32 heads have
+                                  0: what was measured to be the fastest.  Sequences of up to 64 tokens (16-bit, head_dim >= 8) have a
+                                  kernel of their own, which forms all three gradients at once: alone where max_seqlen says that
+                                  there are no others, and in front of the others' kernels in packed batches of more than 64 sequences
+                                  and 1024 sequences * heads with fewer than 128 tokens on average.  The others: below 64 K rows * heads
+                                  the one kernel where it applies and no sequence is longer than 256 tokens (and the mean is
+                                  above 64, or there are fewer than 12 K rows * heads), or at most 32 heads have
                                   (total_tokens / num_seqs) * num_heads >= 16 K and rows * heads >= 20 K.  From 64 K on the
                                   kernel on row tiles, with any head count whose heads and sequences spread over the 8 XCDs
-                                  within a seventh, and with add_remainder (the two kernels where no sequence has more
-                                  than 64 tokens), also at head_dim 64 where sequences have 512 tokens or more on average:
+                                  within a seventh, and with add_remainder, also at head_dim 64 where sequences have 512 tokens or more on average:
                                   as the one kernel (head_dim 128) where no sequence is
                                   longer than 128 tokens and the mean is above 96, or at most 32 heads have (total_tokens /
                                   num_seqs) * num_heads >= 32 K and max_seqlen * num_heads <= 192 K, and else behind a
@@ -258,9 +264,10 @@ int sba_bwd(const SbaArgs* args);
 
 /*
  * How many kernels sba_bwd runs behind its schedule for these arguments on the current device when the workspace holds
- * all heads: 1 (see SbaArgs.backward_kernels) or 2 (dQ, then dK/dV, in fp32 each behind one that lays out its operands where sequences are long;
- * the clearing kernel, then the one on row tiles;
- * also for a call whose heads are split between two forms); a negative SBA_ERR_* for arguments sba_bwd would refuse.
+ * all heads: 1 (see SbaArgs.backward_kernels; also where all sequences are tiny) or 2 (dQ, then dK/dV, in fp32 each behind one that lays out
+ * its operands where sequences are long; the clearing kernel, then the one on row tiles; also for a call whose heads are split between two
+ * forms), and one more where tiny sequences are taken apart from the others (the kernel that rebuilds products is not counted); a negative
+ * SBA_ERR_* for arguments sba_bwd would refuse.
  * Launches nothing.  For callers that attribute the time between trace_events.
  * No counterpart in the reference (it always runs one kernel with atomics and locks, sb_varlen_bwd.py:541-640).
  */

@@ -890,7 +890,8 @@ int sba_bwd_kernels(const SbaArgs* a) {
   Layout L;
   const int st = plan(a, &L);
   if (st != SBA_OK) return st;
-  return bwd_is_one_kernel(a, L) ? 1 : 2;
+  const int tiny = tiny_of(a, a->num_heads, bwd_load(a));
+  return tiny == sba::kTinyAll ? 1 : (bwd_is_one_kernel(a, L) ? 1 : 2) + (tiny == sba::kTinyApart ? 1 : 0);
 }
 
 int sba_bwd(const SbaArgs* a) {
@@ -944,7 +945,7 @@ int backward_route(const SbaArgs* a, BackwardRoute* out) {
   c.backward_kernels = r.kernels;
   if (plan(&c, &L, r.row_tiles) != SBA_OK) return SBA_ERR_SHAPE;
   const Layout::Chain chain = form_of(&c, L);
-  *out = BackwardRoute{chain == Layout::kRowTiles ? kBwdRowTiles : chain == Layout::kKeyTiles ? kBwdKeyTiles : kBwdTwoKernels, (int32_t)r.group};
+  *out = BackwardRoute{tiny_of(a, a->num_heads, bwd_load(a)) == sba::kTinyAll ? kBwdTiny : chain == Layout::kRowTiles ? kBwdRowTiles : chain == Layout::kKeyTiles ? kBwdKeyTiles : kBwdTwoKernels, (int32_t)r.group};
   return SBA_OK;
 }
 

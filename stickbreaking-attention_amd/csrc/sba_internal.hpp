@@ -21,9 +21,9 @@ bool prepared_fits(const SbaArgs* a);
 // sba_bwd on that schedule, with the rest in a->workspace.  The schedule serves ONE backward: its cursors are used up.
 int backward_prepared(const SbaArgs* a, void* sched);
 
-// What sba_bwd would run for these arguments on the current device, with this workspace: the form of its first pass, and the heads that
-// pass takes (all, unless they go through in groups or are split between two forms).
-enum : int32_t { kBwdTwoKernels = 0, kBwdKeyTiles = 1, kBwdRowTiles = 2 };
+// What sba_bwd would run for these arguments on the current device, with this workspace: the form of its first pass (of its longer sequences,
+// where those of up to 64 tokens are taken apart from them), and the heads that pass takes (all, unless they go through in groups or are split between two forms).
+enum : int32_t { kBwdTwoKernels = 0, kBwdKeyTiles = 1, kBwdRowTiles = 2, kBwdTiny = 3 };
 struct BackwardRoute {
   int32_t form, heads;
 };

@@ -67,10 +67,10 @@ POISON = os.environ.get("SBA_DEBUG_POISON", "0") == "1"
 DEBUG_CHECK = os.environ.get("SBA_DEBUG_CHECK", "0") == "1"
 # SbaArgs.backward_kernels: 0 = the library chooses, 1 = dQ then dK/dV, 2 = one kernel where it applies.
 BACKWARD_KERNELS = int(os.environ.get("SBA_BACKWARD_KERNELS", "0"))
-# Kernels the last traced backward ran behind its schedule, 1 or 2 (set when TRACE_EVENTS is).
+# Kernels the last traced backward ran behind its schedule, 1 to 3 (sba_bwd_kernels; set when TRACE_EVENTS is).
 LAST_BWD_KERNELS = 0
-# ... and which backward it was (of its first heads, where they are split between two).
-TWO_KERNELS, KEY_TILES, ROW_TILES = range(3)
+# ... and which backward it was (of its first heads, where they are split between two, and of its sequences of more than 64 tokens, if any).
+TWO_KERNELS, KEY_TILES, ROW_TILES, TINY = range(4)
 LAST_BWD_FORM = TWO_KERNELS
 _STATUS_TEXT = {1: "cu_seqlens is not a non-decreasing sequence within [0, total_tokens] (or its leading entry is not 0)",
                 2: "the carry buffer is too small for these sequence lengths (max_seqlens understated?)",

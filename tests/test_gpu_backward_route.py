@@ -61,3 +61,16 @@ def test_other_forms(gpu_device):
     for a, expected in ((args(32, 128, [1024] * 32, kernels=1), (TWO_KERNELS, 32)), (args(8, 128, [2048, 2048]), (KEY_TILES, 8)),
                         (args(12, 64, [200] * 8), (TWO_KERNELS, 12)), (args(12, 128, [12288]), (ROW_TILES, 8))):      # (8 + 4)
         assert route(a, 1 << 40) == expected
+
+
+@pytest.mark.parametrize("a,form,count", [
+    (args(12, 64, [64, 3, 50]), _native.TINY, 1), (args(8, 128, [64] * 4), _native.TINY, 1), (args(12, 50, [64, 3], kernels=1), _native.TINY, 1),
+    (args(8, 128, [64] * 4, kernels=2), KEY_TILES, 1),                                    # (which takes no tiny ones apart)
+    (args(12, 7, [64, 3]), TWO_KERNELS, 2), (args(12, 64, [65, 3]), TWO_KERNELS, 2),
+    (args(32, 64, [20] * 300 + [70]), TWO_KERNELS, 3),
+    (args(16, 128, [8] * 70 + [200]), KEY_TILES, 2),                                      # apart from key tiles, under 12 K rows x heads
+    (args(32, 128, [20] * 300 + [4000]), ROW_TILES, 3),                                   # (the clearing kernel is one)
+    (args(32, 128, [20] * 300 + [4000], kernels=1), TWO_KERNELS, 3)])
+def test_tiny_sequences_are_reported(gpu_device, a, form, count):
+    assert route(a, 1 << 40) == (form, a.num_heads)
+    assert _native.lib().sba_bwd_kernels(ctypes.byref(a)) == count

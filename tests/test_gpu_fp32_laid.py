@@ -4,7 +4,7 @@ import pytest
 import torch
 
 from oracle import sb_oracle as orc
-from stickbreaking_attention import _native, sb_attn_varlen
+from stickbreaking_attention import _native, sb_attn, sb_attn_varlen
 from test_gpu_parity import NAMES, run_varlen, small_case
 
 pytestmark = pytest.mark.gpu
@@ -51,6 +51,38 @@ def test_against_oracle_and_without_room(gpu_device, D, lengths, attend_current,
         assert torch.equal(a, b), f"{n}: laid out and not differ"
 
 
+@pytest.mark.parametrize("D", [50, 128])
+@pytest.mark.parametrize("L", [1024, 1057])
+def test_of_one_length(gpu_device, L, D):
+    B, H = 3, 3
+    g = torch.Generator().manual_seed(L + D)
+    host = [torch.randn(B, H, L, D, generator=g) for _ in range(4)] + [torch.randn(B, H, L, generator=g)]
+    q, k, v, do, drem = (t.to(gpu_device) for t in host)
+    for t in (q, k, v):
+        t.requires_grad_()
+
+    def run():
+        o, rem = sb_attn(q, k, v)
+        return (o, rem, *torch.autograd.grad([o, rem], [q, k, v], [do, drem]))
+
+    outs = run()
+    a = _native.SbaArgs()
+    a.dtype, a.head_dim, a.num_heads, a.num_seqs, a.total_tokens, a.max_seqlen = _native.SBA_F32, D, H, B, L, L
+    _native.set_backward_workspace_limit(_native._workspace_bytes(a)[1] - 1)
+    try:
+        without = run()
+    finally:
+        _native.set_backward_workspace_limit(None)
+    cu = torch.tensor([L], dtype=torch.int32)
+    for b in range(B):
+        d = [t[b].double() for t in host]
+        ref = orc.varlen_stream(*d[:3], cu, do=d[3], drem=d[4], dtype=torch.float64)
+        for n, x, r in zip(NAMES, outs, ref):
+            assert (x[b].detach().double().cpu() - r).norm() / r.norm() < 1e-5, n      # (as above)
+    for n, x, y in zip(NAMES, outs, without):
+        assert torch.equal(x, y), f"{n}: laid out and not differ"
+
+
 def long_case(device, H, D, lengths):
     g = torch.Generator(device=device).manual_seed(D)
     q, k, v, do = (torch.randn(H, sum(lengths), D, generator=g, device=device) for _ in range(4))
@@ -69,6 +101,22 @@ def peak_of(backward, results):
     grads = backward()
     torch.cuda.synchronize()
     return grads, torch.cuda.max_memory_allocated() - before - results
+
+
+def test_groups_of_heads_with_planes(gpu_device):
+    """A workspace that holds three of five heads with their planes, and not all of them without."""
+    H, D, lengths = 5, 32, [20001, 479]
+    backward = long_case(gpu_device, H, D, lengths)
+    whole = backward()
+    limit = backward_bytes(D, H, lengths, planes=False) - 1
+    assert backward_bytes(D, 3, lengths) <= limit and backward_bytes(D, 3, lengths) > backward_bytes(D, 3, lengths, planes=False)
+    _native.set_backward_workspace_limit(limit)
+    try:
+        in_groups = backward()
+    finally:
+        _native.set_backward_workspace_limit(None)
+    for n, x, y in zip(NAMES[2:], whole, in_groups):
+        assert torch.equal(x, y), n
 
 
 @pytest.mark.parametrize("host_layer", [True, False])

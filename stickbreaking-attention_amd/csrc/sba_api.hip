@@ -376,8 +376,8 @@ int take_turns(int64_t heads) {
 }
 
 // What the scheduler is asked for: always the query tiles; `for_backward`: the key tiles as well, the tile cursors at zero and
-// what the one-kernel backward needs cleared.
-sba::SchedParams sched_params(const SbaArgs* a, char* ws, const Layout& L, bool for_backward, bool want_carry_base, int key_tile) {
+// what the one-kernel backward needs cleared; `carry_rows` as in SchedParams.
+sba::SchedParams sched_params(const SbaArgs* a, char* ws, const Layout& L, bool for_backward, int32_t carry_rows, int key_tile) {
   sba::SchedParams sp{};
   if (for_backward && L.one_kernel) {
     sp.zero_fill = (uint32_t*)(ws + L.off_chain_zero);
@@ -390,10 +390,9 @@ sba::SchedParams sched_params(const SbaArgs* a, char* ws, const Layout& L, bool 
   sp.fixed_len = (int32_t)a->total_tokens;
   sp.total_tokens = a->total_tokens;
   sp.carry_capacity = L.carry_slots_per_head;
-  sp.most_rows = for_backward ? most_rows_of(a) : 0x7fffffff;
   sp.row_capacity = for_backward && L.chain == Layout::kRowTiles && L.rows_by_slot && a->cu_seqlens && key_tile == sba::kRowTileRows ? a->row_blocks : -1;
   sp.want_key_tiles = for_backward ? 1 : 0;
-  sp.want_carry_base = want_carry_base ? 1 : 0;
+  sp.carry_rows = carry_rows;
   sp.q_tiles = (sba::Tile*)(ws + L.off_q_tiles);
   sp.k_tiles = (sba::Tile*)(ws + L.off_k_tiles);
   sp.counts = (int32_t*)(ws + L.off_counts);
@@ -550,8 +549,8 @@ int fwd_on(const SbaArgs* a, char* ws, size_t ws_bytes, bool ws_is_static, bool 
   // The carry offsets are laid out (and the capacity and the lengths checked) when products are recorded, and also when the backward
   // will rebuild them: both passes then agree on whether the schedule stands.
   sba::FwdParams p{};
-  p.sched = sched_params(a, ws, L, for_backward, a->carry != nullptr || a->recompute_carry, for_backward ? expected_key_tile(a, L) : kBlockK);
-  if (p.sched.want_carry_base && !alone) p.sched.most_rows = most_rows_of(a);
+  p.sched = sched_params(a, ws, L, for_backward, !a->carry && !a->recompute_carry ? 0 : alone ? 0x7fffffff : most_rows_of(a),
+                         for_backward ? expected_key_tile(a, L) : kBlockK);
   if (for_backward) p.sched.tiny = expected_tiny(a);
   if (fixed || a->num_seqs <= sba::kInlineSeqs) {
     p.sched.service = 1 + clear_wgs(p.sched);
@@ -814,7 +813,7 @@ int bwd_pass(const SbaArgs* a, int64_t stat_heads, bool first, bool last, char* 
   // The key-tile list is built for the dK/dV kernel that will run.
   const int key_tile = a->dtype == SBA_F32 ? kBlockK : key_tile_of(L, p);
   if (!sched) {
-    sba::SchedParams sp = sched_params(a, ws, L, true, true, key_tile);
+    sba::SchedParams sp = sched_params(a, ws, L, true, most_rows_of(a), key_tile);
     sp.tiny = p.tiny;
     if (sba::launch_sched(sp, clear_wgs(sp), stream) != hipSuccess) return SBA_ERR_LAUNCH;
   }

@@ -52,9 +52,8 @@ struct SchedParams {
   int64_t total_tokens;    // T: rows of the packed token axis (L in fixed-length mode)
   int64_t carry_capacity;  // carry slots reserved per head
   int64_t row_capacity;    // key blocks reserved per head for what row tiles hand over (< 0: not to be checked)
-  int32_t most_rows;       // a longer sequence voids the schedule: the backward would be one that takes no other (kTinyAll)
   int32_t want_key_tiles;  // backward: also build the key-tile list
-  int32_t want_carry_base; // also lay out the per-sequence carry offsets
+  int32_t carry_rows;      // > 0: also lay out the per-sequence carry offsets; a sequence with more rows than this voids the schedule
   Tile* q_tiles;           // query tiles (kBlockQ rows), heaviest first
   Tile* k_tiles;           // key tiles (key_tile keys), heaviest first
   int32_t* counts;         // [kCountQ] query tiles, [kCountK] key tiles, [kCountStatus], [kCountCovered] = tokens

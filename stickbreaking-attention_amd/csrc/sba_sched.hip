@@ -54,10 +54,10 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
   __shared__ uint64_t parts[2][1][kSchedWaves];
   __shared__ int bin_parts[3][kSchedWaves];
   __shared__ unsigned long long row_run, work[2];      // work: of the sequences of one row tile, and of more
-  __shared__ int status, longest, too_long;
+  __shared__ int status, longest;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = kSchedWaves;
   for (int i = threadIdx.x; i < kBins; i += kSchedThreads) { qbins[i] = 0; kbins[i] = 0; sbins[i] = 0; }
-  if (threadIdx.x == 0) { row_run = 0; work[0] = work[1] = 0; longest = too_long = 0; status = kSchedOk; }
+  if (threadIdx.x == 0) { row_run = 0; work[0] = work[1] = 0; longest = 0; status = kSchedOk; }
   __syncthreads();
 
   // Pass 1: tiles per length class (class = number of query tiles of the sequence, saturating), and the layout of the carries: a sum over the
@@ -69,7 +69,6 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
     const int s = s0 + threadIdx.x;
     int start = 0, len = 0;
     if (s < p.num_seqs && !seq_bounds(p, s, &start, &len)) status = kSchedBadCu;
-    if (len > p.most_rows) too_long = 1;
     const int nq = (len + kBlockQ - 1) / kBlockQ, nk = key_tiles(p, len);
     const int cls = min(nq, kBins - 1);
     // (Most sequences of a large batch are of one class.)
@@ -96,8 +95,8 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
       const uint64_t blocks = wave_sum(row_blocks(len));
       if (lane == 0 && blocks) atomicAdd(&row_run, (unsigned long long)blocks);
     }
-    if (p.want_carry_base) {
-      const uint64_t mine = carry_slots(nq);
+    if (p.carry_rows) {
+      const uint64_t mine = slots_of(p, len, nq);
       uint64_t upto[1] = {mine}, before[1], all[1];
       block_sums(upto, before, all, parts[(s0 / kSchedThreads) & 1]);
       if (s < p.num_seqs) p.carry_base[s] = (int64_t)(carry_run + before[0] + upto[0] - mine);
@@ -106,9 +105,8 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
   }
   __syncthreads();
   int verdict = status;
-  if (verdict == kSchedOk && too_long) verdict = kSchedCarryOverflow;
   if (verdict == kSchedOk && p.row_capacity >= 0 && row_run > (unsigned long long)p.row_capacity) verdict = kSchedCarryOverflow;
-  if (verdict == kSchedOk && p.want_carry_base && (int64_t)carry_run > p.carry_capacity) verdict = kSchedCarryOverflow;      // the caller's max_seqlen (or slot count) was too small
+  if (verdict == kSchedOk && p.carry_rows && (int64_t)carry_run > p.carry_capacity) verdict = kSchedCarryOverflow;      // the caller's max_seqlen (or slot count) was too small
   if (verdict != kSchedOk) {      // uniform: nothing is scheduled, every output row is zero-filled as uncovered
     if (threadIdx.x == 0) { p.counts[kCountQ] = 0; p.counts[kCountK] = 0; p.counts[kCountStatus] = verdict; p.counts[kCountCovered] = 0; }
     if (p.want_key_tiles)
@@ -153,7 +151,7 @@ __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
     const bool mine = lane < group && s < p.num_seqs;
     if (mine) {
       seq_bounds(p, s, &start, &len);
-      if (p.want_carry_base) cbase = p.carry_base[s];      // written above by this workgroup
+      if (p.carry_rows) cbase = p.carry_base[s];      // written above by this workgroup
     }
     const int nq = (len + kBlockQ - 1) / kBlockQ, nk = p.want_key_tiles ? key_tiles(p, len) : 0;
     const int cls = min(nq, kBins - 1);

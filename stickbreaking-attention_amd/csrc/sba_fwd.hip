@@ -273,8 +273,8 @@ __global__ __launch_bounds__(kThreads, kMinWaves) void fwd_kernel(FwdParams p) {
 
 // The same for aligned rows of 128 elements (kLoadAligned): key tiles of 32 keys come straight into LDS, one ahead of the tile that is
 // worked on, in two buffers: no registers, no LDS writes and one barrier per tile instead of two.
-// What bounds it: per 32 x 32 block 119 vector-ALU instructions (620 cycles) and 16 MFMAs (512 cycles), at three waves per SIMD, which
-// keep one of the two pipes busy 93 % of the time and both 21 % (32 heads x 8 x 4096; 84 and 16 % on 25 sequences of up to 4096, whose
+// What bounds it: per 32 x 32 block 113 vector-ALU instructions (600 cycles) and 16 MFMAs (512 cycles), at three waves per SIMD, which
+// keep one of the two pipes busy 94 % of the time and both 21 % (32 heads x 8 x 4096; 87 and 18 % on 25 sequences of up to 4096, whose
 // diagonal tiles and ends weigh more); and the power limit (1.9 GHz).  32 heads x 8 x 4096: 1140 us with tiles through registers, 1100 here.  (head_dim 64 keeps its tiles of 64 keys: 107 us for 12 heads, 16384 tokens, against 112.)
 template <typename T>
 __global__ __launch_bounds__(kThreads, 3) void fwd_dma_kernel(FwdParams p) {

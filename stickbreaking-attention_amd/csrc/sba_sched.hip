@@ -39,8 +39,9 @@ __device__ __forceinline__ void block_sums(V (&upto)[kN], V (&before)[kN], V (&a
 }
 
 // What bounds it is the length of its chain of steps (one workgroup): sums are formed by scans over the lanes and one exchange between the waves, and
-// what all lanes of a wave add to one counter the wave adds up first.  (With sums over LDS, ten barriers each, and a counter for every
-// lane, us: 2049 sequences 20, now 11; 600 12 and 7; 100 10 and 6.)
+// what all lanes of a wave add to one counter the wave adds up first.  (Training calls with one
+// sequence of 4096 tokens, all others of up to 64, us, with sums over LDS, ten barriers each, and a counter for every lane / now: 2049 sequences 29.5 / 14.5;
+// 600 16.9 / 8.3; 100 10.5 / 6.8.)
 __global__ __launch_bounds__(kSchedThreads) void sched_kernel(SchedParams p) {
   if (blockIdx.x > 0) {      // helper workgroups: clear the region the launch was asked to clear
     const int64_t n16 = p.zero_bytes / 16, per = (n16 + gridDim.x - 2) / (gridDim.x - 1);
